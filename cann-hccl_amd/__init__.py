@@ -9,11 +9,14 @@ The package directory name contains a hyphen; load it with `load_package()` from
 __graft_entry__.py, or via importlib from its path.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import json
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libhccl.so")
+RANKS_PATH = os.path.join(_HERE, "lib", "_hccl_ranks.so")
 
 # HcclResult (include/hccl/hccl_types.h)
 HCCL_SUCCESS, HCCL_E_PARA, HCCL_E_PTR, HCCL_E_MEMORY, HCCL_E_INTERNAL, HCCL_E_NOT_SUPPORT = 0, 1, 2, 3, 4, 5
@@ -125,12 +128,11 @@ _lib = None
 
 def lib():
     """Loads lib/libhccl.so; raises if it has not been built (there is no fallback path)."""
-    global _lib
+    global _lib, _call
     if _lib is not None:
         return _lib
-    if not os.path.exists(LIB_PATH):
+    if not os.path.exists(LIB_PATH) or not os.path.exists(RANKS_PATH):
         # nothing built yet (a fresh checkout): build once, in tree; a built library is never rebuilt from here
-        import importlib.util
         spec = importlib.util.spec_from_file_location("cann_hccl_amd_build", os.path.join(os.path.dirname(__file__), "build.py"))
         builder = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(builder)
@@ -138,7 +140,7 @@ def lib():
             builder.build()
         except Exception as e:   # noqa: BLE001
             raise RuntimeError("libhccl.so is not built and building it failed (needs hipcc): %s" % e)
-    if not os.path.exists(LIB_PATH):
+    if not os.path.exists(LIB_PATH) or not os.path.exists(RANKS_PATH):
         raise RuntimeError("libhccl.so is not built: run `python cann-hccl_amd/build.py` (needs hipcc)")
     # Streams and device pointers handed to the library must belong to the HIP runtime the library
     # itself uses.  PyTorch ships its own libamdhip64 (same soname): when it is loaded first the
@@ -189,8 +191,26 @@ def lib():
     L.HcclAmdGetLastOpInfo.argtypes = [vp, ctypes.POINTER(HcclAmdOpInfo)]
     L.HcclAmdDescribePlan.argtypes = [i32, i32, u32, u64, i32, u64, u64, u64, ctypes.POINTER(u64), ctypes.c_char_p,
                                       ctypes.c_size_t, ctypes.POINTER(ctypes.c_size_t)]
+    loader = importlib.machinery.ExtensionFileLoader("_hccl_ranks", RANKS_PATH)
+    ranks = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_hccl_ranks", RANKS_PATH, loader=loader))
+    loader.exec_module(ranks)
+    _call = ranks.call
     _lib = L
     return L
+
+
+# One collective on every rank: the loop over the ranks in native code (csrc/pyranks.cc).  The kinds are that file's.
+# Returns the first failing call's code, 0, or -1 where it does not know an argument's type and has called nothing.
+(_ALL_REDUCE, _REDUCE_SCATTER, _REDUCE_SCATTER_NO_ALLOC, _ALL_GATHER, _ALL_TO_ALL, _BROADCAST, _REDUCE, _SCATTER,
+ _ALL_TO_ALL_V) = range(9)
+
+
+def _load_and_call(*args):
+    lib()
+    return _call(*args)
+
+
+_call = _load_and_call
 
 
 class HcclError(RuntimeError):
@@ -229,29 +249,49 @@ def last_op_info(comm):
 
 def all_reduce(comms, sends, recvs, count, dtype, op, stream):
     """One HcclAllReduce call per rank (pointers are ints); the last call issues the work."""
-    for c, s, r in zip(comms, sends, recvs):
-        _check("HcclAllReduce", lib().HcclAllReduce(s, r, count, dtype, op, c, stream))
+    code = _call(_ALL_REDUCE, comms, sends, recvs, count, dtype, op, 0, stream, None)
+    if code == -1:
+        for c, s, r in zip(comms, sends, recvs):
+            _check("HcclAllReduce", lib().HcclAllReduce(s, r, count, dtype, op, c, stream))
+    else:
+        _check("HcclAllReduce", code)
 
 
 def reduce_scatter(comms, sends, recvs, recv_count, dtype, op, stream):
-    for c, s, r in zip(comms, sends, recvs):
-        _check("HcclReduceScatter", lib().HcclReduceScatter(s, r, recv_count, dtype, op, c, stream))
+    code = _call(_REDUCE_SCATTER, comms, sends, recvs, recv_count, dtype, op, 0, stream, None)
+    if code == -1:
+        for c, s, r in zip(comms, sends, recvs):
+            _check("HcclReduceScatter", lib().HcclReduceScatter(s, r, recv_count, dtype, op, c, stream))
+    else:
+        _check("HcclReduceScatter", code)
 
 
 def reduce_scatter_no_alloc(comms, sends, recvs, recv_count, dtype, op, stream):
     """HcclAmdReduceScatterNoAlloc on every rank: the reduce-scatter out of the fixed device workspace."""
-    for c, s, r in zip(comms, sends, recvs):
-        _check("HcclAmdReduceScatterNoAlloc", lib().HcclAmdReduceScatterNoAlloc(s, r, recv_count, dtype, op, c, stream))
+    code = _call(_REDUCE_SCATTER_NO_ALLOC, comms, sends, recvs, recv_count, dtype, op, 0, stream, None)
+    if code == -1:
+        for c, s, r in zip(comms, sends, recvs):
+            _check("HcclAmdReduceScatterNoAlloc", lib().HcclAmdReduceScatterNoAlloc(s, r, recv_count, dtype, op, c, stream))
+    else:
+        _check("HcclAmdReduceScatterNoAlloc", code)
 
 
 def all_gather(comms, sends, recvs, send_count, dtype, stream):
-    for c, s, r in zip(comms, sends, recvs):
-        _check("HcclAllGather", lib().HcclAllGather(s, r, send_count, dtype, c, stream))
+    code = _call(_ALL_GATHER, comms, sends, recvs, send_count, dtype, 0, 0, stream, None)
+    if code == -1:
+        for c, s, r in zip(comms, sends, recvs):
+            _check("HcclAllGather", lib().HcclAllGather(s, r, send_count, dtype, c, stream))
+    else:
+        _check("HcclAllGather", code)
 
 
 def all_to_all(comms, sends, recvs, count, dtype, stream):
-    for c, s, r in zip(comms, sends, recvs):
-        _check("HcclAlltoAll", lib().HcclAlltoAll(s, count, dtype, r, count, dtype, c, stream))
+    code = _call(_ALL_TO_ALL, comms, sends, recvs, count, dtype, 0, 0, stream, None)
+    if code == -1:
+        for c, s, r in zip(comms, sends, recvs):
+            _check("HcclAlltoAll", lib().HcclAlltoAll(s, count, dtype, r, count, dtype, c, stream))
+    else:
+        _check("HcclAlltoAll", code)
 
 
 def all_to_all_vc(comms, sends, recvs, matrix, dtype, stream):
@@ -279,19 +319,31 @@ def all_gather_v(comms, sends, recvs, counts, displs, dtype, stream):
 
 
 def broadcast(comms, bufs, count, dtype, root, stream):
-    for c, b in zip(comms, bufs):
-        _check("HcclBroadcast", lib().HcclBroadcast(b, count, dtype, root, c, stream))
+    code = _call(_BROADCAST, comms, bufs, bufs, count, dtype, 0, root, stream, None)
+    if code == -1:
+        for c, b in zip(comms, bufs):
+            _check("HcclBroadcast", lib().HcclBroadcast(b, count, dtype, root, c, stream))
+    else:
+        _check("HcclBroadcast", code)
 
 
 def reduce(comms, sends, recvs, count, dtype, op, root, stream):
-    for c, s, r in zip(comms, sends, recvs):
-        _check("HcclReduce", lib().HcclReduce(s, r, count, dtype, op, root, c, stream))
+    code = _call(_REDUCE, comms, sends, recvs, count, dtype, op, root, stream, None)
+    if code == -1:
+        for c, s, r in zip(comms, sends, recvs):
+            _check("HcclReduce", lib().HcclReduce(s, r, count, dtype, op, root, c, stream))
+    else:
+        _check("HcclReduce", code)
 
 
 def scatter(comms, sends, recvs, recv_count, dtype, root, stream):
     """sends[r] may be None / 0 for ranks other than the root."""
-    for c, s, r in zip(comms, sends, recvs):
-        _check("HcclScatter", lib().HcclScatter(s, r, recv_count, dtype, root, c, stream))
+    code = _call(_SCATTER, comms, sends, recvs, recv_count, dtype, 0, root, stream, None)
+    if code == -1:
+        for c, s, r in zip(comms, sends, recvs):
+            _check("HcclScatter", lib().HcclScatter(s, r, recv_count, dtype, root, c, stream))
+    else:
+        _check("HcclScatter", code)
 
 
 def send(comm, buf, count, dtype, dest, stream):
@@ -335,7 +387,7 @@ def a2av_tables(send_counts, sdispls, recv_counts, rdispls):
         keep = [np.ascontiguousarray(t, dtype=np.uint64) for t in (send_counts, sdispls, recv_counts, rdispls)]
         base = [t.ctypes.data for t in keep]
         out = _A2avTables([b + r * p * 8 for b in base] for r in range(p))
-        out.keep = keep
+        out.keep = tuple(keep)
         return out
     return [[(ctypes.c_uint64 * p)(*[int(x) for x in t[r]]) for t in (send_counts, sdispls, recv_counts, rdispls)]
             for r in range(p)]
@@ -343,12 +395,17 @@ def a2av_tables(send_counts, sdispls, recv_counts, rdispls):
 
 def all_to_all_v(comms, sends, send_counts, sdispls, recvs, recv_counts, rdispls, dtype, stream, tables=None):
     """counts / displs: per rank, sequences of p integers (elements); or pass tables=a2av_tables(...)."""
-    if tables is None:
-        tables = a2av_tables(send_counts, sdispls, recv_counts, rdispls)
-    fn = lib().HcclAlltoAllV
-    for r, c in enumerate(comms):
-        t = tables[r]
-        _check("HcclAlltoAllV", fn(sends[r], t[0], t[1], dtype, recvs[r], t[2], t[3], dtype, c, stream))
+    plain = (send_counts, sdispls, recv_counts, rdispls) if tables is None else getattr(tables, "keep", None)
+    code = _call(_ALL_TO_ALL_V, comms, sends, recvs, 0, dtype, 0, 0, stream, plain)
+    if code == -1:
+        if tables is None:
+            tables = a2av_tables(send_counts, sdispls, recv_counts, rdispls)
+        fn = lib().HcclAlltoAllV
+        for r, c in enumerate(comms):
+            t = tables[r]
+            _check("HcclAlltoAllV", fn(sends[r], t[0], t[1], dtype, recvs[r], t[2], t[3], dtype, c, stream))
+    else:
+        _check("HcclAlltoAllV", code)
 
 
 def describe_plan(coll, algo, p, count, dtype, ccl_bytes=200 << 20, align=128, in_place_mask=0, tables=None):

@@ -8,6 +8,7 @@ kernel translation units (one per element type plus the byte-copy variants) comp
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -16,6 +17,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libhccl.so")
+RANKS = os.path.join(LIBDIR, "_hccl_ranks.so")
 ABI_CALLER = os.path.join(LIBDIR, "abi_caller")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -74,9 +76,20 @@ def build(force=False, jobs=None):
                 sys.stderr.write(out + "\n")
     if force or tasks or _newer(LIB, objs):
         _run([HIPCC, "-shared", "-fPIC", "--offload-arch=gfx950", "-o", LIB] + objs + ["-lpthread"])
+    build_ranks(force)
     build_abi_caller(force)
     build_threads_latency(force)
     return LIB
+
+
+def build_ranks(force=False):
+    """The Python mirror's loop over the ranks (csrc/pyranks.cc), a CPython extension linked against the library."""
+    src = os.path.join(CSRC, "pyranks.cc")
+    if force or _newer(RANKS, [src, LIB]):
+        _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-I", os.path.join(ROOT, "include"),
+              "-I", sysconfig.get_paths()["include"], src, "-o", RANKS, "-L", LIBDIR, "-lhccl", "-Wl,-rpath,$ORIGIN",
+              "-Wl,--allow-shlib-undefined"])
+    return RANKS
 
 
 def build_abi_caller(force=False, include_dirs=None, out=None):

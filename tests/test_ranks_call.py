@@ -1,0 +1,89 @@
+"""The Python mirror's native loop over the ranks: what it recognises, what it leaves to ctypes, and that both ways the
+library sees the same arguments (told apart by its return codes; no GPU needed: without one a complete collective ends with
+HCCL_E_RUNTIME)."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from hccl_loader import load
+
+H = load()
+P = 4
+
+
+@pytest.fixture
+def comms():
+    c = H.comm_init_all(P)
+    yield c
+    H.comm_destroy(c)
+
+
+def _code(fn, *args, **kw):
+    try:
+        fn(*args, **kw)
+    except H.HcclError as e:
+        return e.code
+    return 0
+
+
+ISSUED = 0 if torch.cuda.is_available() else H.HCCL_E_RUNTIME
+
+
+@pytest.mark.parametrize("form", [list, tuple, lambda x: iter(list(x)), lambda x: [ctypes.c_void_p(v) for v in x]])
+def test_sequences_and_pointer_types(comms, form):
+    if torch.cuda.is_available():
+        pytest.skip("host pointers: only where no collective is issued")
+    ptrs = [0x100000 * (r + 1) for r in range(P)]
+    for fn in (H.all_reduce, H.reduce_scatter):
+        assert _code(fn, comms, form(ptrs), form([p + 0x80000 for p in ptrs]), 16, H.HCCL_DATA_TYPE_FP32, 0, 1) == ISSUED
+        # a null pointer of the second rank: its call fails, the first rank has arrived and is still waiting
+        assert _code(fn, comms, [ptrs[0], None, ptrs[2], ptrs[3]], ptrs, 16, H.HCCL_DATA_TYPE_FP32, 0, 1) == H.HCCL_E_PTR
+        assert _code(fn, comms, ptrs, ptrs, 16, H.HCCL_DATA_TYPE_FP32, 0, 1) == H.HCCL_E_AGAIN
+        # the others join what the first rank started
+        assert _code(fn, comms[1:], ptrs[1:], ptrs[1:], 16, H.HCCL_DATA_TYPE_FP32, 0, 1) == ISSUED
+
+
+def test_every_kind_reaches_its_call(comms):
+    a = [0x100000 * (r + 1) for r in range(P)]
+    none = [None] * P
+    dt = H.HCCL_DATA_TYPE_FP32
+    calls = [(H.all_reduce, (none, a, 8, dt, 0, 1)), (H.reduce_scatter, (none, a, 8, dt, 0, 1)), (H.reduce_scatter_no_alloc, (none, a, 8, dt, 0, 1)),
+             (H.all_gather, (none, a, 8, dt, 1)), (H.all_to_all, (none, a, 8, dt, 1)), (H.broadcast, (none, 8, dt, 0, 1)),
+             (H.reduce, (none, a, 8, dt, 0, 0, 1)), (H.scatter, (a, none, 8, dt, 0, 1))]
+    for fn, args in calls:
+        with pytest.raises(H.HcclError) as e:
+            fn(comms, *args)
+        assert e.value.code == H.HCCL_E_PTR and ("Hccl" + "".join(w.title() for w in fn.__name__.split("_"))
+                                                 .replace("AllToAll", "AlltoAll").replace("ReduceScatterNoAlloc", "AmdReduceScatterNoAlloc")) in str(e.value)
+
+
+@pytest.mark.parametrize("kind", ["uint64", "int64", "lists", "transposed", "tables", "ctypes tables"])
+def test_all_to_all_v_tables(comms, kind):
+    if torch.cuda.is_available():
+        pytest.skip("host pointers: only where no collective is issued")
+    rng = np.random.default_rng(3)
+    cnt = rng.integers(0, 9, (P, P)).astype(np.int64)
+    back = np.ascontiguousarray(cnt.T)
+    dis, rdis = np.cumsum(cnt, axis=1) - cnt, np.cumsum(back, axis=1) - back
+    ptrs = [0x100000 * (r + 1) for r in range(P)]
+
+    def run(c, b):
+        t = [c, dis, b, rdis]
+        kw = {}
+        if kind == "uint64":
+            t = [x.astype(np.uint64) for x in t]
+        elif kind == "lists":
+            t = [x.tolist() for x in t]
+        elif kind == "transposed":
+            t = [np.asfortranarray(x.astype(np.uint64)) for x in t]
+        elif kind != "int64":
+            kw["tables"] = H.a2av_tables(*([x.tolist() for x in t] if kind == "ctypes tables" else t))
+            t = [None] * 4
+        return _code(H.all_to_all_v, comms, ptrs, t[0], t[1], [p + 0x80000 for p in ptrs], t[2], t[3], H.HCCL_DATA_TYPE_INT32, 1, **kw)
+
+    assert run(cnt, back) == ISSUED
+    wrong = back.copy()
+    wrong[2, 1] += 1                    # rank 2 expects one more from rank 1 than it sends
+    assert run(cnt, wrong) == H.HCCL_E_PARA

@@ -938,10 +938,8 @@ Algo Level1Algo(const Group *g)
     return (n >= 8 || (n > 1 && (n & (n - 1)) == 0)) ? ALGO_RHD : ALGO_RING;
 }
 
-HcclResult Prepare(Group *g, int algo, std::unique_ptr<Prepared> *out, bool noAlloc, hipStream_t stream)
+PlanRequest MakeRequest(const Group *g, int algo)
 {
-    std::unique_ptr<Prepared> pp(new Prepared());
-    const bool reduceColl = g->ctx->sig.coll == COLL_ALLREDUCE || g->ctx->sig.coll == COLL_REDUCESCATTER || g->ctx->sig.coll == COLL_REDUCE;
     PlanRequest rq;
     rq.coll = CollKind(g->ctx->sig.coll);
     rq.algo = Algo(algo);
@@ -1044,29 +1042,63 @@ HcclResult Prepare(Group *g, int algo, std::unique_ptr<Prepared> *out, bool noAl
         rq.recvCounts = g->ctx->recvCounts;
         rq.rdispls = g->ctx->rdispls;
     }
+    return rq;
+}
+
+bool ReduceColl(int coll) { return coll == COLL_ALLREDUCE || coll == COLL_REDUCESCATTER || coll == COLL_REDUCE; }
+
+// Buffers of different ranks must not overlap where one of them is written (HCCL_E_PARA); a send buffer that
+// overlaps a receive buffer other than as an exact in-place pair is staged through scratch (*needStage).
+HcclResult CheckOverlap(const Group *g, const Plan &plan, bool *needStage)
+{
+    *needStage = false;
+    for (uint32_t i = 0; i < g->p; i++) {
+        const char *ri = static_cast<const char *>(g->ctx->recv[i]);
+        for (uint32_t j = 0; j < g->p; j++) {
+            const char *rj = static_cast<const char *>(g->ctx->recv[j]);
+            const char *sj = static_cast<const char *>(g->ctx->send[j]);
+            if (i != j && RangesOverlap(ri, plan.recvBytes[i], rj, plan.recvBytes[j])) {
+                HCCL_LOG_ERROR("%s: receive buffers of rank %u and rank %u overlap", CollName(g->ctx->sig.coll), i, j);
+                return HCCL_E_PARA;
+            }
+            if (RangesOverlap(ri, plan.recvBytes[i], sj, plan.sendBytes[j])) {
+                bool exact = (i == j) && ri == sj && (g->ctx->sig.coll == COLL_ALLREDUCE || g->ctx->sig.coll == COLL_BROADCAST);
+                *needStage = *needStage || !exact;
+            }
+        }
+    }
+    return HCCL_SUCCESS;
+}
+
+OpInfo MakeInfo(const Group *g, int algo, const Plan &plan, bool fused)
+{
+    OpInfo info;
+    info.coll = g->ctx->sig.coll;
+    info.algo = algo;
+    info.fused = fused ? 1 : 0;
+    info.bytesRead = fused ? plan.fusedRead : plan.stepRead;
+    info.bytesWritten = fused ? plan.fusedWritten : plan.stepWritten;
+    info.stepRead = plan.stepRead;
+    info.stepWritten = plan.stepWritten;
+    info.scratchBytes = fused ? 0 : plan.scratchBytes;
+    return info;
+}
+
+HcclResult Prepare(Group *g, int algo, std::unique_ptr<Prepared> *out, bool noAlloc, hipStream_t stream)
+{
+    std::unique_ptr<Prepared> pp(new Prepared());
+    const bool reduceColl = ReduceColl(g->ctx->sig.coll);
+    PlanRequest rq = MakeRequest(g, algo);
     std::string err;
     int rc = CachedPlan(g, rq, &pp->plan, &err);
     if (rc != 0) {
         HCCL_LOG_ERROR("%s: planning failed: %s", CollName(g->ctx->sig.coll), err.c_str());
         return rc == 1 ? HCCL_E_PARA : HCCL_E_INTERNAL;
     }
-    // Buffers of different ranks must not overlap where one of them is written; a send buffer that
-    // overlaps a receive buffer other than as an exact in-place pair is staged through scratch.
     bool needStage = false;
-    for (uint32_t i = 0; i < g->p; i++) {
-        const char *ri = static_cast<const char *>(g->ctx->recv[i]);
-        for (uint32_t j = 0; j < g->p; j++) {
-            const char *rj = static_cast<const char *>(g->ctx->recv[j]);
-            const char *sj = static_cast<const char *>(g->ctx->send[j]);
-            if (i != j && RangesOverlap(ri, pp->plan->recvBytes[i], rj, pp->plan->recvBytes[j])) {
-                HCCL_LOG_ERROR("%s: receive buffers of rank %u and rank %u overlap", CollName(g->ctx->sig.coll), i, j);
-                return HCCL_E_PARA;
-            }
-            if (RangesOverlap(ri, pp->plan->recvBytes[i], sj, pp->plan->sendBytes[j])) {
-                bool exact = (i == j) && ri == sj && (g->ctx->sig.coll == COLL_ALLREDUCE || g->ctx->sig.coll == COLL_BROADCAST);
-                needStage = needStage || !exact;
-            }
-        }
+    HcclResult overlap = CheckOverlap(g, *pp->plan, &needStage);
+    if (overlap != HCCL_SUCCESS) {
+        return overlap;
     }
     if (needStage) {
         rq.stageInput = true;
@@ -1108,23 +1140,114 @@ HcclResult Prepare(Group *g, int algo, std::unique_ptr<Prepared> *out, bool noAl
     }
     // The graph of a plan with several launches is built when the collective comes back a second time
     // (IssueCollective): a caller that brings fresh buffers every time pays for tables, not for a graph.
-    OpInfo &info = pp->info;
-    info.coll = g->ctx->sig.coll;
-    info.algo = algo;
-    info.fused = pp->fused ? 1 : 0;
-    info.graph = 0;
-    info.launches = uint32_t(pp->launches.size());
-    info.teamLaunches = 0;
+    pp->info = MakeInfo(g, algo, *pp->plan, pp->fused);
+    pp->info.launches = uint32_t(pp->launches.size());
     for (const LaunchRec &l : pp->launches) {
-        info.teamLaunches += l.team ? 1u : 0u;
+        pp->info.teamLaunches += l.team ? 1u : 0u;
     }
-    info.bytesRead = pp->fused ? pp->plan->fusedRead : pp->plan->stepRead;
-    info.bytesWritten = pp->fused ? pp->plan->fusedWritten : pp->plan->stepWritten;
-    info.stepRead = pp->plan->stepRead;
-    info.stepWritten = pp->plan->stepWritten;
-    info.scratchBytes = pp->fused ? 0 : pp->plan->scratchBytes;
     *out = std::move(pp);
     return HCCL_SUCCESS;
+}
+
+// What a prepared collective still needs before it can be launched on `ls`: its tables uploaded, its graph.
+HcclResult ReadyToLaunch(Group *g, Prepared *pp, hipStream_t ls, bool hit, bool *viaGraph)
+{
+    // A caller may be capturing this stream into a graph of its own.  A graph launched into a
+    // capturing stream is not recorded there (the caller's graph came out empty and replays did
+    // nothing), so the kernels are then launched one by one and become nodes of the caller's graph.
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    HIP_OK(hipStreamIsCapturing(ls, &capture));
+    const bool capturing = capture != hipStreamCaptureStatusNone;
+    if (!pp->uploadComplete) {
+        // The tables were written by launches on the stream of the call that prepared them, and nothing says yet
+        // that those have run.  Outside a capture: ask, and order this stream behind them if need be.  Under
+        // capture events of work outside the capture may not be touched and the caller's graph may be replayed
+        // on any stream later, so the same upload launches are recorded in front of the collective's kernels:
+        // every replay rewrites the same bytes.
+        if (capturing) {
+            HIP_OK(UploadThroughKernelArgs(pp->devTables, pp->hostTables.data(), pp->hostTables.size(), ls));
+        } else if (hipEventQuery(pp->uploaded) == hipSuccess) {
+            pp->uploadComplete = true;
+            std::vector<uint8_t>().swap(pp->hostTables);
+        } else {
+            (void)hipGetLastError();
+            if (ls != pp->uploadStream) {
+                HIP_OK(hipStreamWaitEvent(ls, pp->uploaded, 0));
+            }
+        }
+    }
+    if (capturing && !pp->pinned && !g->ctx->sig.noAlloc) {
+        // The caller's graph keeps pointers to this collective's tables and, step by step, to the group's
+        // scratch buffers: from now on neither is freed or handed out again while the group lives.
+        pp->pinned = true;
+        g->arena.Pin(pp->tableChunk);
+        if (pp->info.scratchBytes > 0) {
+            g->pinnedScratchUsers++;
+        }
+    }
+    // A graph launch costs about 33 us of host time plus 2 us per node, a direct launch 3.3 us (measured: 2 launches
+    // 38 us through a graph against 16 us, 14 launches 39 against 43, 64 launches 159 against 230): a graph pays
+    // from a dozen launches on.
+    if (!capturing && !g->ctx->sig.noAlloc && g->cfg.graph && pp->launches.size() >= kGraphMinLaunches && pp->exec == nullptr &&
+        pp->uses >= 1) {
+        // second use of the same collective on the same buffers: from now on it is replayed from a graph
+        HcclResult r = BuildGraph(pp);
+        if (r != HCCL_SUCCESS) {
+            return r;
+        }
+    }
+    pp->uses++;
+    *viaGraph = pp->exec != nullptr && !capturing;
+    g->lastInfo = pp->info;
+    g->lastInfo.cacheHit = hit ? 1 : 0;
+    g->lastInfo.graph = *viaGraph ? 1 : 0;
+    return HCCL_SUCCESS;
+}
+
+// The launch of a small collective whose descriptors ride in its arguments, nullptr where the call does not go out
+// that way.  Kept per request and settings; the buffers are this call's.
+DirectLaunch *FindDirect(Group *g, int algo)
+{
+    const OpSig &sig = g->ctx->sig;
+    const GroupConfig &cfg = g->cfg;
+    if (sig.noAlloc || sig.variable || sig.coll == COLL_ALLTOALLV || !cfg.fuse || cfg.team == 1 || cfg.blocksPerCu != 0 ||
+        cfg.launchCapMiB >= 0 || cfg.fusedStores >= 0) {
+        return nullptr;
+    }
+    uint64_t inPlace = 0;
+    for (uint32_t r = 0; r < g->p; r++) {
+        inPlace |= uint64_t(g->ctx->send[r] == g->ctx->recv[r] ? 1 : 0) << r;
+    }
+    const uint64_t head[8] = {uint64_t(sig.coll) | (uint64_t(algo) << 8) | (uint64_t(sig.dtype) << 16) | (uint64_t(sig.op) << 24) | (uint64_t(sig.root) << 32) |
+            (uint64_t(sig.peer) << 48), sig.count, inPlace, cfg.cclBytes, cfg.align,
+        uint64_t(cfg.servers) | (uint64_t(uint32_t(cfg.algo + 1)) << 16) | (uint64_t(cfg.level0Rings) << 32) | (uint64_t(cfg.deterministic) << 48),
+        cfg.nicMask, g->p};
+    std::string key(reinterpret_cast<const char *>(head), sizeof(head));
+    auto it = g->direct.find(key);
+    if (it == g->direct.end()) {
+        if (g->direct.size() >= 256) {
+            g->direct.clear();
+        }
+        DirectLaunch d;
+        std::string err;
+        if (CachedPlan(g, MakeRequest(g, algo), &d.plan, &err) != 0) {
+            return nullptr;             // the general path reports it
+        }
+        if (BuildDirect(*d.plan, ReduceColl(sig.coll), sig.dtype, sig.op, &d)) {
+            d.info = MakeInfo(g, algo, *d.plan, true);
+            d.info.launches = 1;
+        } else {
+            d = DirectLaunch();
+        }
+        it = g->direct.emplace(std::move(key), std::move(d)).first;
+    }
+    DirectLaunch *d = &it->second;
+    bool needStage = false;
+    if (d->func == nullptr || CheckOverlap(g, *d->plan, &needStage) != HCCL_SUCCESS || needStage) {
+        return nullptr;
+    }
+    d->info.cacheHit = FillBases(d, g->ctx->send, g->ctx->recv) ? 1 : 0;
+    return d;
 }
 
 }  // namespace
@@ -1238,6 +1361,7 @@ HcclResult IssueCollective(Group *g, uint32_t launcher)
         (g->ctx->sig.coll == COLL_ALLREDUCE || g->ctx->sig.coll == COLL_REDUCESCATTER || g->ctx->sig.coll == COLL_REDUCE)) {
         algo = ALGO_MESH_ATOMIC;
     }
+    DirectLaunch *direct = FindDirect(g, algo);
     Prepared *pp = nullptr;
     std::unique_ptr<Prepared> uncached;   // the collective of a call that allocates nothing: built, launched, dropped
     bool hit = false;
@@ -1256,9 +1380,10 @@ HcclResult IssueCollective(Group *g, uint32_t launcher)
         }
         pp = uncached.get();
     }
-    std::string key = pp ? std::string() : CacheKey(g, algo);
-    auto it = pp ? g->cache.end() : g->cache.find(key);
-    if (pp != nullptr) {
+    const bool looked = pp != nullptr || direct != nullptr;
+    std::string key = looked ? std::string() : CacheKey(g, algo);
+    auto it = looked ? g->cache.end() : g->cache.find(key);
+    if (looked) {
         // issued below
     } else if (it != g->cache.end() && (it->second->scratchGen == g->scratchGen || it->second->info.scratchBytes == 0)) {
         // (an entry that points into scratch buffers the group has since outgrown is stale)
@@ -1310,55 +1435,15 @@ HcclResult IssueCollective(Group *g, uint32_t launcher)
         g->cache[key] = std::move(fresh);
     }
     hipStream_t ls = g->ctx->streams[launcher];
-    // A caller may be capturing this stream into a graph of its own.  A graph launched into a
-    // capturing stream is not recorded there (the caller's graph came out empty and replays did
-    // nothing), so the kernels are then launched one by one and become nodes of the caller's graph.
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    HIP_OK(hipStreamIsCapturing(ls, &capture));
-    const bool capturing = capture != hipStreamCaptureStatusNone;
-    if (!pp->uploadComplete) {
-        // The tables were written by launches on the stream of the call that prepared them, and nothing says yet
-        // that those have run.  Outside a capture: ask, and order this stream behind them if need be.  Under
-        // capture events of work outside the capture may not be touched and the caller's graph may be replayed
-        // on any stream later, so the same upload launches are recorded in front of the collective's kernels:
-        // every replay rewrites the same bytes.
-        if (capturing) {
-            HIP_OK(UploadThroughKernelArgs(pp->devTables, pp->hostTables.data(), pp->hostTables.size(), ls));
-        } else if (hipEventQuery(pp->uploaded) == hipSuccess) {
-            pp->uploadComplete = true;
-            std::vector<uint8_t>().swap(pp->hostTables);
-        } else {
-            (void)hipGetLastError();
-            if (ls != pp->uploadStream) {
-                HIP_OK(hipStreamWaitEvent(ls, pp->uploaded, 0));
-            }
+    bool viaGraph = false;
+    if (direct != nullptr) {
+        g->lastInfo = direct->info;
+    } else {
+        HcclResult ready = ReadyToLaunch(g, pp, ls, hit, &viaGraph);
+        if (ready != HCCL_SUCCESS) {
+            return ready;
         }
     }
-    if (capturing && !pp->pinned && !g->ctx->sig.noAlloc) {
-        // The caller's graph keeps pointers to this collective's tables and, step by step, to the group's
-        // scratch buffers: from now on neither is freed or handed out again while the group lives.
-        pp->pinned = true;
-        g->arena.Pin(pp->tableChunk);
-        if (pp->info.scratchBytes > 0) {
-            g->pinnedScratchUsers++;
-        }
-    }
-    // A graph launch costs about 33 us of host time plus 2 us per node, a direct launch 3.3 us (measured: 2 launches
-    // 38 us through a graph against 16 us, 14 launches 39 against 43, 64 launches 159 against 230): a graph pays
-    // from a dozen launches on.
-    if (!capturing && !g->ctx->sig.noAlloc && g->cfg.graph && pp->launches.size() >= kGraphMinLaunches && pp->exec == nullptr &&
-        pp->uses >= 1) {
-        // second use of the same collective on the same buffers: from now on it is replayed from a graph
-        r = BuildGraph(pp);
-        if (r != HCCL_SUCCESS) {
-            return r;
-        }
-    }
-    pp->uses++;
-    const bool viaGraph = pp->exec != nullptr && !capturing;
-    g->lastInfo = pp->info;
-    g->lastInfo.cacheHit = hit ? 1 : 0;
-    g->lastInfo.graph = viaGraph ? 1 : 0;
 
     // Order the launch after everything queued so far on the other ranks' streams, and order those
     // streams after the collective.  Ranks that share the launcher's stream need nothing.
@@ -1384,7 +1469,10 @@ HcclResult IssueCollective(Group *g, uint32_t launcher)
         }
         others = true;
     }
-    if (viaGraph) {
+    if (direct != nullptr) {
+        void *args[1] = {direct->image.data()};
+        HIP_OK(hipLaunchKernel(direct->func, dim3(direct->gridX, direct->gridY, 1), dim3(kBlockThreads, 1, 1), args, 0, ls));
+    } else if (viaGraph) {
         HIP_OK(hipGraphLaunch(pp->exec, ls));
     } else {
         for (LaunchRec &l : pp->launches) {

@@ -72,8 +72,9 @@ constexpr uint32_t kGatherMaxBytes = 8192;
 enum KernelKind : int {
     KK_STEP = 0, KK_CHAIN = 1, KK_TREE = 2, KK_STACK = 3,
     KK_TEAM_CHAIN = 4, KK_TEAM_TREE = 5, KK_TEAM_STACK = 6,   // team forms of the fused kernels, see below
-    KK_COUNT = 7,
-    KK_GATHER = 7                                              // copy kernel table only
+    KK_DIRECT = 7, KK_DIRECT_WIDE = 8,                         // small collectives, see below
+    KK_COUNT = 9,
+    KK_GATHER = 9                                              // copy kernel table only
 };
 
 // Team form of a fused kernel: the workgroups of one XCD read their tiles together, park the results in LDS, and write
@@ -102,6 +103,35 @@ struct TeamRegion {
 };
 inline uint32_t TeamBlockWords(uint32_t nregions) { return kTeamHeaderWords + 2u * nregions + kTeamXcds * (nregions + 1u); }
 
+// Small collectives (kernels_direct.h): the whole description of a launch rides in its kernel arguments.  All sources of
+// an item lie at the same offset of their buffers and all destinations at the same offset of theirs.
+constexpr uint32_t kDirectChunk = kBlockThreads * 16;    // bytes of an item per workgroup
+enum DirectKind : uint32_t { DIRECT_CHAIN = 0, DIRECT_TREE = 1, DIRECT_STACK = 2 };
+
+// CAP = 8: up to 8 sources and destinations per item; CAP = 32: up to 32 (no stack programs).
+template <uint32_t CAP> struct DirectItem {
+    uint32_t bytes;
+    uint32_t srcOff, dstOff;
+    uint32_t nsrc, ndst;
+    uint32_t kind;
+    uint32_t nleaf;          // tree: number of leaves
+    uint32_t accLeft;        // chain: bit j as in FusedDesc::accLeftMask
+    uint32_t second;         // tree: bit i = leaf i is src[i] (+) src[kDirectSecond + i]
+    uint32_t src[CAP > 8 ? 8 : 4];     // base indexes, a byte each.  chain: sources; tree: first sources of the leaves, their
+                                       // second ones (repeating the first where there is none) from kDirectSecond on;
+                                       // stack: sources, the last one repeated up to 8
+    uint32_t dst[CAP / 4];             // base indexes of the destinations, 0 behind the last one
+    uint32_t ops[CAP > 8 ? 1 : 4];     // stack: a halfword per source
+};
+template <uint32_t CAP> constexpr uint32_t kDirectSecond = CAP > 8 ? 16 : 8;
+template <uint32_t CAP> constexpr uint32_t kDirectItems = CAP > 8 ? 32 : 16;
+template <uint32_t CAP> constexpr uint32_t kDirectBases = CAP > 8 ? 64 : 16;
+template <uint32_t CAP> struct DirectArgs {
+    uint64_t base[kDirectBases<CAP>];
+    DirectItem<CAP> item[kDirectItems<CAP>];
+};
+static_assert(sizeof(DirectArgs<32>) <= 4096, "kernel arguments");
+
 // Kernel entry for (data type, reduce op, kind); nullptr if the combination is not built.
 // Signatures:
 //   KK_STEP            (const StepDesc *steps, uint32_t nsteps, uint32_t nwhole, uint32_t ntiles, uint32_t flags)
@@ -110,11 +140,14 @@ inline uint32_t TeamBlockWords(uint32_t nregions) { return kTeamHeaderWords + 2u
 //                      (const FusedDesc *items, uint32_t nitems, uint32_t ntiles,
 //                       const void *const *srcPool, void *const *dstPool, uint32_t tilesPerItem)
 //   KK_TEAM_*          the same and (uint32_t *teamBlock)
+//   KK_DIRECT / KK_DIRECT_WIDE   (DirectArgs<8> / DirectArgs<32>), grid (1 + chunks of the longest item, items): blockIdx.x == 0
+//                      is for the bytes behind an item's last whole vector
 const void *LookupKernel(int hcclDataType, int hcclReduceOp, KernelKind kind);
 
 //   KK_GATHER          (const SegDesc *segs, uint32_t nsegs, uint32_t unused, const void *unused, void *unused)
 //                      copy kernel table only
-// Byte-wise variants for pure data movement (all-gather, all-to-all-v): KK_STEP, KK_CHAIN, KK_TEAM_CHAIN and KK_GATHER.
+// Byte-wise variants for pure data movement (all-gather, all-to-all-v): KK_STEP, KK_CHAIN, KK_TEAM_CHAIN, KK_GATHER,
+// KK_DIRECT and KK_DIRECT_WIDE.
 const void *LookupCopyKernel(KernelKind kind);
 
 }  // namespace hcclamd

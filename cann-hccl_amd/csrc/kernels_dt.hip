@@ -1,5 +1,6 @@
 // Instantiates the kernels for one HcclDataType (selected with -DHCCL_DT=<enum value>), so that the
 // twelve element types build in parallel, plus the byte-wise copy variants (-DHCCL_DT=255).
+#include "kernels_direct.h"
 #include "kernels_team.h"
 
 namespace hcclamd {
@@ -52,11 +53,13 @@ using DT = uint8_t;
 
 #if HCCL_DT == 255
 // pure data movement: the step kernel's copy path and the copy kernel
-extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[4] = {
+extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[6] = {
     reinterpret_cast<const void *>(&StepKernel<DT, ROP_SUM>),
     reinterpret_cast<const void *>(&CopyKernel<0>),
     reinterpret_cast<const void *>(&GatherKernel<0>),
     reinterpret_cast<const void *>(&TeamCopyKernel<0>),
+    reinterpret_cast<const void *>(&DirectCopyKernel<8>),
+    reinterpret_cast<const void *>(&DirectCopyKernel<32>),
 };
 #else
 #define HCCL_ROW(OP)                                                     \
@@ -68,6 +71,8 @@ extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[4] = {
         reinterpret_cast<const void *>(&TeamChainKernel<DT, OP>),        \
         reinterpret_cast<const void *>(&TeamTreeKernel<DT, OP>),         \
         reinterpret_cast<const void *>(&TeamStackKernel<DT, OP>),        \
+        reinterpret_cast<const void *>(&DirectKernel<DT, OP, 8>),        \
+        reinterpret_cast<const void *>(&DirectKernel<DT, OP, 32>),       \
     }
 extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[4][KK_COUNT] = {
     HCCL_ROW(ROP_SUM), HCCL_ROW(ROP_PROD), HCCL_ROW(ROP_MAX), HCCL_ROW(ROP_MIN),

@@ -107,6 +107,22 @@ struct Prepared {
     ~Prepared();
 };
 
+// One launch whose descriptors ride in its arguments (small collectives, kernels_direct.h).  It belongs to a request, not to
+// buffers: the base pointers are filled in by every call.
+struct DirectLaunch {
+    std::shared_ptr<const Plan> plan;
+    const void *func = nullptr;       // nullptr: this request does not go out this way
+    uint32_t gridX = 0, gridY = 0;
+    std::vector<std::pair<uint32_t, uint8_t>> bases;   // (rank, buffer) of every base pointer
+    std::vector<uint8_t> image;                        // the kernel's arguments, a DirectArgs
+    OpInfo info;
+};
+
+// The launch of `plan`; false (func == nullptr) where it is not small or does not fit.
+bool BuildDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaunch *d);
+// Puts the ranks' pointers in; true if they were there already (the previous call's).
+bool FillBases(DirectLaunch *d, const std::vector<void *> &send, const std::vector<void *> &recv);
+
 struct OpSig {
     int coll = -1;
     uint64_t count = 0;
@@ -209,6 +225,7 @@ struct Group {
     uint64_t scratchBytes = 0;
     uint64_t scratchGen = 0;
     std::unordered_map<std::string, std::unique_ptr<Prepared>> cache;   // keyed by request, settings and buffer addresses
+    std::unordered_map<std::string, DirectLaunch> direct;   // small collectives, keyed by request and settings
     TableArena arena;
     std::unordered_map<std::string, std::shared_ptr<const Plan>> planCache;   // keyed by the plan request
     std::unordered_map<std::string, std::vector<TemplateSlot>> planTemplates;   // keyed by the request without its count

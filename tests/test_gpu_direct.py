@@ -1,0 +1,126 @@
+"""Small collectives, whose descriptors ride in the kernel arguments (one launch, 4 KiB of an item per workgroup), against the
+CPU checker bit for bit: the edges of a workgroup's 4 KiB and of a 16-byte vector, every batch size of sources, trees and
+stack programs, buffers at any element boundary, in place, operand order on NaNs and signed zeros, new buffers on every call
+and replays of a caller's graph."""
+import numpy as np
+import pytest
+import torch
+
+import closed_forms as cf
+import gpu_harness as gh
+from closed_forms import BF16, FP16, FP32, INT8, INT64, MAX, MIN, PROD, SUM
+
+pytestmark = pytest.mark.gpu
+H = gh.H
+RING, MESH, RHD = 0, 1, 2
+
+
+def _ins(dt, p, n, seed, special=False):
+    rng = np.random.default_rng(seed)
+    ins = [cf.random_input(dt, n, rng) for _ in range(p)]
+    if special:
+        odd = np.array([np.nan, 0.0, -0.0, np.inf, -np.inf, 1.0], np.float32)
+        for x in ins:
+            at = rng.random(n) < 0.7
+            x[at] = cf.narrow(dt, odd[rng.integers(0, odd.size, int(at.sum()))])
+    return ins
+
+
+# ring: chains of 1 ... 32 sources (batches of 16, 8 and a rest); halving-doubling: trees of 2 ... 32 leaves with and
+# without second sources; several groups: stack programs
+@pytest.mark.parametrize("p,algo,servers", [(2, RING, 1), (3, RING, 1), (7, RING, 1), (8, RING, 1), (9, RING, 1), (15, RING, 1), (24, RING, 1),
+                                            (31, RING, 1), (32, RING, 1), (8, MESH, 1), (2, RHD, 1), (6, RHD, 1), (8, RHD, 1),
+                                            (13, RHD, 1), (24, RHD, 1), (32, RHD, 1), (8, RHD, 2), (8, RHD, 4), (6, RING, 3)])
+def test_all_reduce(orc, p, algo, servers):
+    g = gh.Group(p, algo=("ring", "mesh", "rhd")[algo], servers=servers, deterministic=1)
+    try:
+        for k, (dt, op, pad, in_place, special) in enumerate([(FP32, SUM, 0, False, False), (BF16, MAX, 2, True, True), (INT8, PROD, 3, False, False),
+                                                              (FP16, MIN, 16, False, True), (INT64, SUM, 8, True, False)]):
+            unit = H.DTYPE_SIZE[dt]
+            sizes = {1, 128 * p // unit + 1, (4096 * p) // unit, (4096 * p + 128) // unit - 1, (3 * 4096 + 128) * p // unit + 5, (1 << 20) // unit}
+            for n in sorted(sizes):
+                print("small all-reduce", p, algo, servers, "type", dt, "op", op, "n", n, "pad", pad, flush=True)
+                ins = _ins(dt, p, n, 31 * p + n % 1009 + k, special)
+                if servers > 1:
+                    want = orc.allreduce_two_level(ins, dt, op, servers, level1=algo)
+                else:
+                    want = orc.allreduce(ins, dt, op, algo=algo)
+                outs, keep = gh.all_reduce(g, ins, dt, op, in_place=in_place, pad=pad)
+                assert g.info()["launches"] <= 1 or servers > 1 or algo == MESH
+                for r in range(p):
+                    assert gh.same(dt, outs[r], want[r]), (dt, op, n, r)
+                    assert keep is None or np.array_equal(keep[r].view(np.uint8), ins[r].view(np.uint8))
+    finally:
+        g.close()
+
+
+@pytest.mark.parametrize("p", [2, 5, 8, 16, 32])
+def test_blocks(orc, p):
+    # reduce-scatter, all-gather, broadcast, reduce and send / receive: blocks that start at any byte
+    g = gh.Group(p)
+    try:
+        for dt, op, pad in ((INT8, SUM, 0), (BF16, SUM, 2), (FP32, MAX, 4)):
+            unit = H.DTYPE_SIZE[dt]
+            for n in (1, 15, 17, 4096 // unit - 1, 4096 // unit + 1, 20011 // unit):
+                print("small blocks", p, "type", dt, "n", n, flush=True)
+                ins = _ins(dt, p, n * p, 77 * p + n)
+                want = orc.reducescatter(ins, dt, op)
+                outs, _ = gh.reduce_scatter(g, ins, dt, op, pad=pad)
+                for r in range(p):
+                    assert gh.same(dt, outs[r], want[r]), ("reduce-scatter", dt, n, r)
+                parts = [x[:n] for x in ins]
+                outs = gh.all_gather(g, parts, dt, pad=pad)
+                for r in range(p):
+                    assert np.array_equal(outs[r].view(np.uint8), np.concatenate(parts).view(np.uint8)), ("all-gather", dt, n, r)
+                root = n % p
+                bufs = [gh.to_dev(x, pad) for x in parts]
+                dst = [gh.empty_dev(n * unit, pad) for _ in range(p)]
+                torch.cuda.synchronize()
+                H.reduce(g.comms, [t.data_ptr() for t in bufs], [t.data_ptr() for t in dst], n, dt, op, root, g.stream_ptr)
+                H.send(g.comms[0], bufs[0].data_ptr(), n, dt, p - 1, g.stream_ptr)
+                spare = gh.empty_dev(n * unit, pad)
+                H.recv(g.comms[p - 1], spare.data_ptr(), n, dt, 0, g.stream_ptr)
+                H.broadcast(g.comms, [t.data_ptr() for t in bufs], n, dt, root, g.stream_ptr)
+                g.stream.synchronize()
+                assert gh.same(dt, gh.to_host(dst[root], dt), orc.reduce_to_root(parts, dt, op, root)), ("reduce", dt, n)
+                assert np.array_equal(gh.to_host(spare, dt).view(np.uint8), parts[0].view(np.uint8)), ("send / receive", dt, n)
+                for r in range(p):
+                    assert np.array_equal(gh.to_host(bufs[r], dt).view(np.uint8), parts[root].view(np.uint8)), ("broadcast", dt, n, r)
+    finally:
+        g.close()
+
+
+def test_new_buffers_and_graph_replay(orc):
+    p, n = 8, 3001
+    g = gh.Group(p)
+    try:
+        ins = _ins(FP32, p, n, 5)
+        want = orc.allreduce(ins, FP32, SUM)
+        base = [gh.to_dev(x) for x in ins]
+        sets = [([t.clone() for t in base], [torch.zeros_like(t) for t in base]) for _ in range(20)]
+        torch.cuda.synchronize()
+        hits = []
+        for s, r in sets + sets[-1:]:
+            H.all_reduce(g.comms, [t.data_ptr() for t in s], [t.data_ptr() for t in r], n, FP32, SUM, g.stream_ptr)
+            hits.append(g.info()["cacheHit"])
+        assert hits == [0] * 20 + [1]
+        s, r = sets[3]
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.stream(g.stream):
+            graph.capture_begin()
+            H.all_reduce(g.comms, [t.data_ptr() for t in s], [t.data_ptr() for t in r], n, FP32, SUM, g.stream_ptr)
+            graph.capture_end()
+        for replay in range(3):
+            for t in r:
+                t.zero_()
+            H.all_reduce(g.comms, [t.data_ptr() for t in sets[7][0]], [t.data_ptr() for t in sets[7][1]], n, FP32, SUM, g.stream_ptr)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            for k in range(p):
+                assert np.array_equal(gh.to_host(r[k], FP32), want[k]), (replay, k)
+        for _, r in sets:
+            for k in range(p):
+                assert np.array_equal(gh.to_host(r[k], FP32), want[k])
+    finally:
+        g.close()

@@ -636,8 +636,16 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                 dsts.clear();
                 addrs.clear();
                 for (const Ref &d : it.dst) {
-                    dsts.push_back(b.Ptr(d));
+                    char *t = b.Ptr(d);
+                    if (!reduceColl && t == b.Ptr(it.src[0])) {
+                        pp->inPlaceBytes += it.bytes;     // a block gathered in place is where it belongs already
+                        continue;
+                    }
+                    dsts.push_back(t);
                     addrs.push_back(reinterpret_cast<uintptr_t>(dsts.back()));
+                }
+                if (dsts.empty()) {
+                    continue;
                 }
                 uint32_t streams = uint32_t(dsts.size());
                 for (size_t k = 0; k < it.src.size(); k++) {
@@ -1049,9 +1057,13 @@ bool ReduceColl(int coll) { return coll == COLL_ALLREDUCE || coll == COLL_REDUCE
 
 // Buffers of different ranks must not overlap where one of them is written (HCCL_E_PARA); a send buffer that
 // overlaps a receive buffer other than as an exact in-place pair is staged through scratch (*needStage).
-HcclResult CheckOverlap(const Group *g, const Plan &plan, bool *needStage)
+// An all-gather in place -- rank r sends its own block of its receive buffer -- is none of that for the fused form, in
+// which nothing but that block's item touches the block (*gatherInPlace); step by step, other blocks pass through it.
+HcclResult CheckOverlap(const Group *g, const Plan &plan, bool *needStage, bool *gatherInPlace)
 {
-    *needStage = false;
+    *needStage = *gatherInPlace = false;
+    const OpSig &sig = g->ctx->sig;
+    const uint64_t unit = DtypeSize(sig.dtype);
     for (uint32_t i = 0; i < g->p; i++) {
         const char *ri = static_cast<const char *>(g->ctx->recv[i]);
         for (uint32_t j = 0; j < g->p; j++) {
@@ -1062,8 +1074,10 @@ HcclResult CheckOverlap(const Group *g, const Plan &plan, bool *needStage)
                 return HCCL_E_PARA;
             }
             if (RangesOverlap(ri, plan.recvBytes[i], sj, plan.sendBytes[j])) {
-                bool exact = (i == j) && ri == sj && (g->ctx->sig.coll == COLL_ALLREDUCE || g->ctx->sig.coll == COLL_BROADCAST);
-                *needStage = *needStage || !exact;
+                bool exact = (i == j) && ri == sj && (sig.coll == COLL_ALLREDUCE || sig.coll == COLL_BROADCAST);
+                bool ownBlock = (i == j) && sig.coll == COLL_ALLGATHER && sj == ri + (sig.variable ? g->ctx->vDispls[i] : i * sig.count) * unit;
+                *gatherInPlace = *gatherInPlace || ownBlock;
+                *needStage = *needStage || !(exact || ownBlock);
             }
         }
     }
@@ -1095,11 +1109,12 @@ HcclResult Prepare(Group *g, int algo, std::unique_ptr<Prepared> *out, bool noAl
         HCCL_LOG_ERROR("%s: planning failed: %s", CollName(g->ctx->sig.coll), err.c_str());
         return rc == 1 ? HCCL_E_PARA : HCCL_E_INTERNAL;
     }
-    bool needStage = false;
-    HcclResult overlap = CheckOverlap(g, *pp->plan, &needStage);
+    bool needStage = false, gatherInPlace = false;
+    HcclResult overlap = CheckOverlap(g, *pp->plan, &needStage, &gatherInPlace);
     if (overlap != HCCL_SUCCESS) {
         return overlap;
     }
+    needStage = needStage || (gatherInPlace && !(g->cfg.fuse && pp->plan->fusedOk));
     if (needStage) {
         rq.stageInput = true;
         rq.alias.assign(g->p, 0);
@@ -1142,6 +1157,7 @@ HcclResult Prepare(Group *g, int algo, std::unique_ptr<Prepared> *out, bool noAl
     // (IssueCollective): a caller that brings fresh buffers every time pays for tables, not for a graph.
     pp->info = MakeInfo(g, algo, *pp->plan, pp->fused);
     pp->info.launches = uint32_t(pp->launches.size());
+    pp->info.bytesWritten -= pp->inPlaceBytes;
     for (const LaunchRec &l : pp->launches) {
         pp->info.teamLaunches += l.team ? 1u : 0u;
     }
@@ -1242,8 +1258,8 @@ DirectLaunch *FindDirect(Group *g, int algo)
         it = g->direct.emplace(std::move(key), std::move(d)).first;
     }
     DirectLaunch *d = &it->second;
-    bool needStage = false;
-    if (d->func == nullptr || CheckOverlap(g, *d->plan, &needStage) != HCCL_SUCCESS || needStage) {
+    bool needStage = false, gatherInPlace = false;   // (a gathered block stored onto itself: by the lane that has read it)
+    if (d->func == nullptr || CheckOverlap(g, *d->plan, &needStage, &gatherInPlace) != HCCL_SUCCESS || needStage) {
         return nullptr;
     }
     d->info.cacheHit = FillBases(d, g->ctx->send, g->ctx->recv) ? 1 : 0;

@@ -87,6 +87,7 @@ struct OpInfo {
 struct Prepared {
     std::shared_ptr<const Plan> plan;   // shared with the group's plan cache (plans do not depend on addresses)
     bool fused = false;
+    uint64_t inPlaceBytes = 0;        // fused: bytes of the plan that lie where they belong (an all-gather in place)
     void *devTables = nullptr;        // inside the group's table arena
     uint32_t tableChunk = 0;          // the arena chunk they came from
     std::vector<LaunchRec> launches;

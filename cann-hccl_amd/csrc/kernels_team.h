@@ -9,7 +9,7 @@
 //   read phase   every workgroup evaluates up to kTeamTiles tiles (every 32nd tile of the team's region, so an XCD
 //                works on one contiguous stretch of the tile space) and parks the results in LDS.  A round of whole
 //                tiles of one item is read with all its loads issued together (a copy) or source by source with the
-//                partial results in LDS (a chain), see Round() below
+//                partial results in LDS (a chain; a chain of chains), see Round() below
 //   barrier      among the team's workgroups only; the other XCDs run on, in whatever phase they are
 //   write phase  every workgroup writes its parked tiles to their destinations, destination by destination
 // Workgroup b belongs to XCD b % 8 (workgroups are dealt to the XCDs round robin).  If they are not, or if the team is
@@ -202,16 +202,16 @@ __device__ __forceinline__ void TeamBody(const FusedDesc *__restrict__ items, ui
                 d = items[idx];
                 dEnd = d.tile0 + uint32_t((d.bytes + kTileBytes - 1) / kTileBytes);
                 const uint32_t lastTile = first + (n - 1) * teamSize;
-                bySource = d.mode == ACC_VEC16 && d.nsrc >= Eval::kRoundMinSrc && lastTile < dEnd &&
+                bySource = d.mode == ACC_VEC16 && Eval::RoundFits(d) && lastTile < dEnd &&
                     uint64_t(lastTile - d.tile0 + 1) * kTileBytes <= d.bytes;
             }
             if (bySource) {
                 const uint64_t off = uint64_t(first - d.tile0) * kTileBytes;
                 const uint64_t stride = uint64_t(teamSize) * kTileBytes;
                 if (n == kTeamTiles) {
-                    Eval::template Round<kTeamTiles>(d, srcPool + d.srcBase, off, stride, park, slots + round, &seen);
+                    Eval::template Round<kTeamTiles>(d, srcPool + d.srcBase, extra, off, stride, park, slots + round, &seen);
                 } else {
-                    Eval::template Round<kTeamTiles / 2>(d, srcPool + d.srcBase, off, stride, park, slots + round, &seen);
+                    Eval::template Round<kTeamTiles / 2>(d, srcPool + d.srcBase, extra, off, stride, park, slots + round, &seen);
                 }
                 maxDst = d.ndst;
                 if (threadIdx.x < n) {
@@ -299,20 +299,9 @@ __device__ __forceinline__ void TeamBody(const FusedDesc *__restrict__ items, ui
 template <typename T> struct ReadsBySource { static constexpr bool value = true; };
 template <> struct ReadsBySource<Bf16Bits> { static constexpr bool value = false; };
 
-template <typename T, int OP> struct TeamChainEval {
-    static constexpr bool kBySource = ReadsBySource<T>::value;
-    static constexpr uint32_t kRoundMinSrc = 2;
-    // A whole round at once: N whole tiles of one item, `stride` bytes apart from `off` on.  The team reads source by
-    // source -- at any moment its loads go to one stretch of N x 32 tiles of one buffer instead of 32 tiles of each of
-    // the item's buffers -- and the partial results rest in LDS, folded in the chain's order, so the bits are those of
-    // the tile-by-tile evaluation.  Two register sets of N x 4 vectors: while one source is folded, the next one's
-    // loads are in flight, and the one after that is requested as soon as the fold has freed its set (8 ranks x
-    // 256 MiB, stand-alone: 691 us this way, 770 us with one set, 705 us tile by tile).
-    // Straight-line code for a source count fixed at compile time, in which every wait is for exactly the loads it
-    // needs, measured the same and takes three times as long to build.
-    // `peek` is looked at (thread 0, into *seen) once the last loads are on their way.
+// One register set: N whole tiles of one source, `stride` bytes apart.
     template <uint32_t N>
-    static __device__ __forceinline__ void LoadSet(V4 (&v)[N][kVecPerLane], const void *base, uint64_t off, uint64_t stride)
+    __device__ __forceinline__ void TeamLoadSet(V4 (&v)[N][kVecPerLane], const void *base, uint64_t off, uint64_t stride)
     {
         const char *s = static_cast<const char *>(base) + off;
 #pragma unroll
@@ -323,6 +312,19 @@ template <typename T, int OP> struct TeamChainEval {
             }
         }
     }
+
+template <typename T, int OP> struct TeamChainEval {
+    static constexpr bool kBySource = ReadsBySource<T>::value;
+    static __device__ __forceinline__ bool RoundFits(const FusedDesc &d) { return d.nsrc >= 2; }
+    // A whole round at once: N whole tiles of one item, `stride` bytes apart from `off` on.  The team reads source by
+    // source -- at any moment its loads go to one stretch of N x 32 tiles of one buffer instead of 32 tiles of each of
+    // the item's buffers -- and the partial results rest in LDS, folded in the chain's order, so the bits are those of
+    // the tile-by-tile evaluation.  Two register sets of N x 4 vectors: while one source is folded, the next one's
+    // loads are in flight, and the one after that is requested as soon as the fold has freed its set (8 ranks x
+    // 256 MiB, stand-alone: 691 us this way, 770 us with one set, 705 us tile by tile).
+    // Straight-line code for a source count fixed at compile time, in which every wait is for exactly the loads it
+    // needs, measured the same and takes three times as long to build.
+    // `peek` is looked at (thread 0, into *seen) once the last loads are on their way.
     // Source j into the partial results: source 0 starts them.  A tile's partial results are fetched from LDS together,
     // so that their latencies overlap.
     template <uint32_t N>
@@ -365,26 +367,26 @@ template <typename T, int OP> struct TeamChainEval {
         }
     }
     template <uint32_t N>
-    static __device__ __forceinline__ void Round(const FusedDesc &d, const void *const *__restrict__ src, uint64_t off,
+    static __device__ __forceinline__ void Round(const FusedDesc &d, const void *const *__restrict__ src, const void *, uint64_t off,
         uint64_t stride, LdsV4 *park, const uint32_t *peek, uint32_t *seen)
     {
         const uint32_t nsrc = d.nsrc;
         V4 va[N][kVecPerLane], vb[N][kVecPerLane];
-        LoadSet<N>(va, src[0], off, stride);
-        LoadSet<N>(vb, src[1], off, stride);
+        TeamLoadSet<N>(va, src[0], off, stride);
+        TeamLoadSet<N>(vb, src[1], off, stride);
         uint32_t j = 0;
 #pragma nounroll
         for (; j + 4 <= nsrc; j += 2) {
             FoldSet<N>(va, d, j, park);
-            LoadSet<N>(va, src[j + 2], off, stride);
+            TeamLoadSet<N>(va, src[j + 2], off, stride);
             FoldSet<N>(vb, d, j + 1, park);
-            LoadSet<N>(vb, src[j + 3], off, stride);
+            TeamLoadSet<N>(vb, src[j + 3], off, stride);
         }
         // two or three sources left, the first two of them loaded or on their way
         const bool three = nsrc - j == 3;
         FoldSet<N>(va, d, j, park);
         if (three) {
-            LoadSet<N>(va, src[j + 2], off, stride);
+            TeamLoadSet<N>(va, src[j + 2], off, stride);
         }
         if (threadIdx.x == 0) {
             *seen = TeamLoad(peek);
@@ -445,11 +447,11 @@ template <typename T, int OP> struct TeamChainEval {
 
 struct TeamCopyEval {
     static constexpr bool kBySource = true;
-    static constexpr uint32_t kRoundMinSrc = 1;
+    static __device__ __forceinline__ bool RoundFits(const FusedDesc &) { return true; }
     // A whole round at once (see TeamChainEval::Round): the loads of all N tiles are issued before the first of them is
     // parked, instead of tile after tile with an LDS write between them.
     template <uint32_t N>
-    static __device__ __forceinline__ void Round(const FusedDesc &, const void *const *__restrict__ src, uint64_t off,
+    static __device__ __forceinline__ void Round(const FusedDesc &, const void *const *__restrict__ src, const void *, uint64_t off,
         uint64_t stride, LdsV4 *park, const uint32_t *peek, uint32_t *seen)
     {
         const uint32_t tid = threadIdx.x;
@@ -527,7 +529,124 @@ template <typename T, int OP> struct TeamTreeEval {
 
 // extra = the launch's op words (they follow the item table)
 template <typename T, int OP> struct TeamStackEval {
-    static constexpr bool kBySource = false;
+    static constexpr bool kBySource = ReadsBySource<T>::value;
+    // A whole round source by source, as the chain's (TeamChainEval::Round), for expressions that never hold more than
+    // two partial results while a source is being read (a chain of chains: the two-level all-reduce): the lower one in
+    // LDS, the upper one in registers.  Three sets of eight tiles are more registers than a wave has, so the round goes
+    // in halves of four tiles, through one pipeline: the second half's first sources are requested while the first
+    // half's last ones are folded.  Measured (8 ranks, fp32 sum, us, tile by tile / this way): two servers of four, 64 MiB
+    // per rank 198.0 / 180.8 (5.4 / 5.9 TB/s), 256 MiB 745 - 755 / 721; the 8-rank ring's chain of 64 MiB takes 176.  What
+    // bounds it now is what bounds the chain, the write phase.
+    static __device__ __forceinline__ bool RoundFits(const FusedDesc &d) { return d.nsrc >= 2 && d.nleaf <= 3; }
+    static constexpr uint32_t kHalf = kTeamTiles / 2;
+    typedef V4 Set[kHalf][kVecPerLane];
+    static __device__ __forceinline__ void FoldUpper(Set &v, const Set &under, bool underLeft)
+    {
+#pragma unroll
+        for (uint32_t q = 0; q < kHalf; q++) {
+#pragma unroll
+            for (uint32_t u = 0; u < kVecPerLane; u++) {
+                v[q][u] = underLeft ? Combine16<T, OP>(under[q][u], v[q][u]) : Combine16<T, OP>(v[q][u], under[q][u]);
+            }
+        }
+    }
+    static __device__ __forceinline__ void FoldLower(Set &v, const LdsV4 *park, bool underLeft)
+    {
+#pragma unroll
+        for (uint32_t q = 0; q < kHalf; q++) {
+            V4 a[kVecPerLane];
+#pragma unroll
+            for (uint32_t u = 0; u < kVecPerLane; u++) {
+                a[u] = park[q * kTeamVecPerTile + u * kBlockThreads + threadIdx.x];
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kVecPerLane; u++) {
+                v[q][u] = underLeft ? Combine16<T, OP>(a[u], v[q][u]) : Combine16<T, OP>(v[q][u], a[u]);
+            }
+        }
+    }
+    // Pushes a source and folds as its op word says (`depth`: partial results held).
+    static __device__ __forceinline__ void Push(Set &v, uint32_t op, Set &upper, LdsV4 *park, uint32_t &depth)
+    {
+        uint32_t nfold = op & 7u, left = OrderMatters<T, OP>::value ? op >> 8 : ~0u;
+        if (depth == 2 && nfold != 0) {
+            if (left & 1u) {      // the same for the whole wave
+                FoldUpper(v, upper, true);
+            } else {
+                FoldUpper(v, upper, false);
+            }
+            left >>= 1;
+            nfold--;
+            depth = 1;
+        }
+        if (depth == 1 && nfold != 0) {
+            if (left & 1u) {
+                FoldLower(v, park, true);
+            } else {
+                FoldLower(v, park, false);
+            }
+            depth = 0;
+        }
+        if (depth == 0) {
+#pragma unroll
+            for (uint32_t q = 0; q < kHalf; q++) {
+#pragma unroll
+                for (uint32_t u = 0; u < kVecPerLane; u++) {
+                    park[q * kTeamVecPerTile + u * kBlockThreads + threadIdx.x] = v[q][u];
+                }
+            }
+        } else {
+#pragma unroll
+            for (uint32_t q = 0; q < kHalf; q++) {
+#pragma unroll
+                for (uint32_t u = 0; u < kVecPerLane; u++) {
+                    upper[q][u] = v[q][u];
+                }
+            }
+        }
+        depth++;
+    }
+    template <uint32_t N>
+    static __device__ __forceinline__ void Round(const FusedDesc &d, const void *const *__restrict__ src, const void *extra,
+        uint64_t off, uint64_t stride, LdsV4 *park, const uint32_t *peek, uint32_t *seen)
+    {
+        const uint32_t *ops = static_cast<const uint32_t *>(extra) + d.srcBase;
+        const uint32_t nsrc = d.nsrc, total = nsrc * (N / kHalf);
+        Set va, vb, upper;
+        uint32_t depth = 0;
+        auto load = [&](Set &v, uint32_t j) {
+            const uint32_t half = j >= nsrc ? 1u : 0u;
+            TeamLoadSet<kHalf>(v, src[j - half * nsrc], off + half * kHalf * stride, stride);
+        };
+        auto push = [&](Set &v, uint32_t j) {
+            const uint32_t half = j >= nsrc ? 1u : 0u;
+            depth = j == half * nsrc ? 0u : depth;
+            Push(v, ops[j - half * nsrc], upper, park + half * kHalf * kTeamVecPerTile, depth);
+        };
+        load(va, 0);
+        load(vb, 1);
+        uint32_t j = 0;
+#pragma nounroll
+        for (; j + 4 <= total; j += 2) {
+            push(va, j);
+            load(va, j + 2);
+            push(vb, j + 1);
+            load(vb, j + 3);
+        }
+        // two or three left, the first two of them loaded or on their way
+        const bool three = total - j == 3;
+        push(va, j);
+        if (three) {
+            load(va, j + 2);
+        }
+        if (threadIdx.x == 0) {
+            *seen = TeamLoad(peek);
+        }
+        push(vb, j + 1);
+        if (three) {
+            push(va, j + 2);
+        }
+    }
     __device__ __forceinline__ void SetItem(const FusedDesc &, const void *const *__restrict__) {}
     __device__ __forceinline__ void Vec(const FusedDesc &d, const void *const *__restrict__ srcPool, const void *extra,
         uint64_t off, uint32_t nvec, LdsV4 *park) const

@@ -297,6 +297,32 @@ template <uint32_t MODE> __device__ __forceinline__ V4 Load16(const void *base, 
         return V4{t.x, t.y, t.z, t.w};
     }
 }
+// 16 bytes at any address, fetched as whole words: the four words from the word boundary in front on, and the word that
+// holds the last bytes (for an address on a word boundary the fourth word again, so that nothing outside the words of
+// the 16 bytes is touched).  Vector(shift) puts them together, shift = address mod 4.
+// For 8-bit elements: a 128-bit load off a word boundary costs the vector memory unit more than the extra word does.
+// Reduce-scatter, int8, blocks of odd length, us, 128-bit loads / this way: 8 ranks x 3 000 017 sum 44.2 / 42.1 (blocks at
+// multiples of 64 bytes: 39.9), x 12 000 017 168.0 / 157.5; 16 ranks x 700 001 sum 47.1 / 43.1, max 55.6 / 47.2.  16-bit
+// elements gain nothing (bf16 sum 8 x 1 000 001 30.5 / 31.1, fp16 8 x 2 000 001 51.6 / 52.2) and keep the 128-bit loads.
+struct WordVec {
+    V4 v;
+    uint32_t last;
+    __device__ __forceinline__ void Load(const void *base, uint64_t byteOff, uint32_t shift)
+    {
+        typedef uint32_t HCCL_GLOBAL GlobalWord;
+        typedef uint32_t V4W __attribute__((ext_vector_type(4), aligned(4)));
+        typedef V4W HCCL_GLOBAL GlobalV4W;
+        const char *p = static_cast<const char *>(base) - shift + byteOff;
+        const V4W t = __builtin_nontemporal_load((const GlobalV4W *)p);
+        v = V4{t.x, t.y, t.z, t.w};
+        last = *(const GlobalWord *)(p + (shift != 0 ? 16 : 12));
+    }
+    __device__ __forceinline__ V4 Vector(uint32_t shift) const
+    {
+        return V4{__builtin_amdgcn_alignbyte(v.y, v.x, shift), __builtin_amdgcn_alignbyte(v.z, v.y, shift),
+            __builtin_amdgcn_alignbyte(v.w, v.z, shift), __builtin_amdgcn_alignbyte(last, v.w, shift)};
+    }
+};
 __device__ __forceinline__ void Store16(void *base, uint64_t byteOff, V4 v)
 {
     __builtin_nontemporal_store(v, (GlobalV4 *)(static_cast<char *>(base) + byteOff));
@@ -547,6 +573,7 @@ template <typename T, int OP, uint32_t MODE, bool FULL, bool ORDINARY = false, b
 __device__ __forceinline__ void ChainVecPass(const FusedDesc &d, const void *const *__restrict__ src,
     void *const *__restrict__ dst, uint64_t off, uint32_t vecBase, uint32_t nvec, LdsV4 *park = nullptr)
 {
+    constexpr bool kByWords = MODE == ACC_VEC16_ANY && sizeof(T) == 1 && !PARK;
     const uint32_t tid = threadIdx.x;
     uint64_t pos[kChainVec];
     bool live[kChainVec];
@@ -561,14 +588,21 @@ __device__ __forceinline__ void ChainVecPass(const FusedDesc &d, const void *con
     const uint32_t batched = ONE_BATCH ? 1u : nsrc;
     for (uint32_t j = 0; j < batched; j += kChainSrcBatch) {
         V4 v[kChainSrcBatch][kChainVec];
+        WordVec words[kChainSrcBatch][kChainVec];
+        uint32_t shift[kChainSrcBatch];
 #pragma unroll
         for (uint32_t jj = 0; jj < kChainSrcBatch; jj++) {
             if (j + jj < nsrc) {
                 const void *s = src[j + jj];
+                shift[jj] = uint32_t(reinterpret_cast<uintptr_t>(s)) & 3u;     // (positions are multiples of 16)
 #pragma unroll
                 for (uint32_t u = 0; u < kChainVec; u++) {
                     if (live[u]) {
-                        v[jj][u] = Load16<MODE>(s, pos[u]);
+                        if (kByWords) {
+                            words[jj][u].Load(s, pos[u], shift[jj]);
+                        } else {
+                            v[jj][u] = Load16<MODE>(s, pos[u]);
+                        }
                     }
                 }
             }
@@ -576,6 +610,12 @@ __device__ __forceinline__ void ChainVecPass(const FusedDesc &d, const void *con
 #pragma unroll
         for (uint32_t jj = 0; jj < kChainSrcBatch; jj++) {
             if (j + jj < nsrc) {
+                if (kByWords) {
+#pragma unroll
+                    for (uint32_t u = 0; u < kChainVec; u++) {
+                        v[jj][u] = words[jj][u].Vector(shift[jj]);
+                    }
+                }
                 if (j + jj == 0) {
 #pragma unroll
                     for (uint32_t u = 0; u < kChainVec; u++) {

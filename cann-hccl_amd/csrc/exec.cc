@@ -209,6 +209,10 @@ template <typename F> void SplitByAlignment(const std::vector<uintptr_t> &addrs,
 
 constexpr size_t kGraphMinLaunches = 12;   // fewer launches go out one by one
 constexpr uint32_t kTeamMinRounds = 2;     // the team kernels are chosen for launches of at least this many full rounds
+// The same for one source and many destinations.  8-rank all-gather, us, plain / team: blocks of 3 MiB (1536 tiles, less
+// than a round) 46.3 / 52.4, 4 MiB (2048) 63.4 / 58.9, 5 MiB 80.1 / 73.1, 6 MiB 92.8 / 85.8, 7.5 MiB 121.9 / 105.5; 16 ranks
+// 1.5 MiB (1536) 88.2 / 91.7, 2 MiB 116.2 / 111.5, 3 MiB 174.6 / 162.8.
+constexpr uint32_t kTeamMinRoundsCopy = 1;
 constexpr size_t kAsyncUploadBytes = 4 * kNoAllocUploadBytes;   // tables up to this size are uploaded by launches
 
 uint32_t TilesOf(uint64_t bytes) { return uint32_t((bytes + kTileBytes - 1) / kTileBytes); }
@@ -578,7 +582,7 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                                                               : std::max(1u, std::min(kTeamTiles, uint32_t(128.0 / std::max(1.0, widest))));
                     if (g->cfg.team < 0) {
                         team = bytes > 0 && storeStreams >= 4.0 * bytes && allStreams >= 8.0 * bytes &&
-                            tiles >= kTeamMinRounds * pl.rec.roundTiles * g->numCu;
+                            tiles >= (reduceColl ? kTeamMinRounds : kTeamMinRoundsCopy) * pl.rec.roundTiles * g->numCu;
                     }
                 }
                 if (team) {
@@ -602,7 +606,13 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                     }
                     for (uint32_t at = 0; at < tiles;) {
                         const uint32_t left = tiles - at;
-                        if (uint64_t(at) * 4 >= uint64_t(tiles) * 3) {
+                        if (tiles < 2 * pl.rec.roundTiles * g->numCu) {
+                            // Less than two full rounds: every team gets as much as the others in each, and the
+                            // odd tiles come last (all-gather of 8 x 6 MiB: 85.8 us, with the rule below 100.9).
+                            if (regions.size() % kTeamXcds == 0) {
+                                per = std::max(1u, std::min(per, left / g->numCu));
+                            }
+                        } else if (uint64_t(at) * 4 >= uint64_t(tiles) * 3) {
                             while (per > 1 && uint64_t(per) * perX * 8 > left) {
                                 per /= 2;
                             }

@@ -1,4 +1,4 @@
-"""The team form of the stack kernel on whole rounds (slices of 4 MiB and more), which it reads source by source: two
+"""The choice of the team form for all-gathers of one to two rounds, and the team form of the stack kernel on whole rounds (slices of 4 MiB and more), which it reads source by source: two
 halves of four tiles, one partial result in LDS and one in registers.  Against the CPU checker, bit for bit."""
 import numpy as np
 import pytest
@@ -40,5 +40,23 @@ def test_team_stack_whole_rounds(orc, dt, op, p, servers, special, extra):
                     assert np.array_equal(outs[r].view(np.uint32), want[r].view(np.uint32)), r
                 else:
                     assert gh.same(dt, outs[r], want[r]), r
+    finally:
+        g.close()
+
+
+@pytest.mark.parametrize("tiles,team", [(255, 0), (256, 1), (257, 1), (289, 1), (500, 1)])
+def test_allgather_of_one_to_two_rounds(tiles, team):
+    # `tiles` per rank; 8 x 256 tiles are a full round of 8 tiles on 256 compute units
+    p, n = 8, tiles * 16384
+    g = gh.Group(p)
+    try:
+        ins = [cf.random_input(INT8, n, np.random.default_rng(9600 + r)) for r in range(p)]
+        print("all-gather, tiles per rank", tiles, flush=True)
+        for rep in range(2):
+            outs = gh.all_gather(g, ins, INT8)
+            assert g.info()["teamLaunches"] == team
+            whole = np.concatenate(ins)
+            for r in range(p):
+                assert np.array_equal(outs[r], whole), r
     finally:
         g.close()

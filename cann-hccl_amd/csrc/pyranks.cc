@@ -8,10 +8,14 @@
 //
 // Whatever this loop does not recognise (other sequence or pointer types than lists or tuples of integers, None and
 // c_void_p) it leaves alone: call() then returns -1 before any call was made and the caller goes through ctypes.
+//
+// The functions are those of the library that the mirror has loaded, handed over by bind(): were this module linked
+// against the library, a libhccl.so elsewhere on the loader's search path could be taken for it.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
 #include <cstdint>
+#include <cstring>
 
 #include "hccl/hccl.h"
 #include "hccl/hccl_amd_ext.h"
@@ -22,6 +26,21 @@ enum Kind : long {
     ALL_REDUCE = 0, REDUCE_SCATTER, REDUCE_SCATTER_NO_ALLOC, ALL_GATHER, ALL_TO_ALL, BROADCAST, REDUCE, SCATTER, ALL_TO_ALL_V,
     KIND_COUNT
 };
+
+// in the order of Kind
+struct Functions {
+    decltype(&HcclAllReduce) allReduce;
+    decltype(&HcclReduceScatter) reduceScatter;
+    decltype(&HcclAmdReduceScatterNoAlloc) reduceScatterNoAlloc;
+    decltype(&HcclAllGather) allGather;
+    decltype(&HcclAlltoAll) allToAll;
+    decltype(&HcclBroadcast) broadcast;
+    decltype(&HcclReduce) reduce;
+    decltype(&HcclScatter) scatter;
+    decltype(&HcclAlltoAllV) allToAllV;
+};
+static_assert(sizeof(Functions) == KIND_COUNT * sizeof(void *), "one function per kind");
+Functions g_fn = {};
 
 constexpr Py_ssize_t kMostRanks = 64;
 PyObject *g_valueName = nullptr;      // "value"
@@ -100,7 +119,7 @@ struct Table {
 PyObject *Call(PyObject *, PyObject *const *args, Py_ssize_t nargs)
 {
     PyObject *const no = PyLong_FromLong(-1);
-    if (no == nullptr || nargs != 10 || !PyLong_CheckExact(args[0])) {
+    if (no == nullptr || nargs != 10 || g_fn.allReduce == nullptr || !PyLong_CheckExact(args[0])) {
         return no;
     }
     const long kind = PyLong_AsLong(args[0]);
@@ -148,16 +167,16 @@ PyObject *Call(PyObject *, PyObject *const *args, Py_ssize_t nargs)
     Py_BEGIN_ALLOW_THREADS
     for (Py_ssize_t r = 0; r < p && res == HCCL_SUCCESS; r++) {
         switch (kind) {
-            case ALL_REDUCE: res = HcclAllReduce(send[r], recv[r], count, dt, ro, comm[r], stream); break;
-            case REDUCE_SCATTER: res = HcclReduceScatter(send[r], recv[r], count, dt, ro, comm[r], stream); break;
-            case REDUCE_SCATTER_NO_ALLOC: res = HcclAmdReduceScatterNoAlloc(send[r], recv[r], count, dt, ro, comm[r], stream); break;
-            case ALL_GATHER: res = HcclAllGather(send[r], recv[r], count, dt, comm[r], stream); break;
-            case ALL_TO_ALL: res = HcclAlltoAll(send[r], count, dt, recv[r], count, dt, comm[r], stream); break;
-            case BROADCAST: res = HcclBroadcast(send[r], count, dt, rt, comm[r], stream); break;
-            case REDUCE: res = HcclReduce(send[r], recv[r], count, dt, ro, rt, comm[r], stream); break;
-            case SCATTER: res = HcclScatter(send[r], recv[r], count, dt, rt, comm[r], stream); break;
+            case ALL_REDUCE: res = g_fn.allReduce(send[r], recv[r], count, dt, ro, comm[r], stream); break;
+            case REDUCE_SCATTER: res = g_fn.reduceScatter(send[r], recv[r], count, dt, ro, comm[r], stream); break;
+            case REDUCE_SCATTER_NO_ALLOC: res = g_fn.reduceScatterNoAlloc(send[r], recv[r], count, dt, ro, comm[r], stream); break;
+            case ALL_GATHER: res = g_fn.allGather(send[r], recv[r], count, dt, comm[r], stream); break;
+            case ALL_TO_ALL: res = g_fn.allToAll(send[r], count, dt, recv[r], count, dt, comm[r], stream); break;
+            case BROADCAST: res = g_fn.broadcast(send[r], count, dt, rt, comm[r], stream); break;
+            case REDUCE: res = g_fn.reduce(send[r], recv[r], count, dt, ro, rt, comm[r], stream); break;
+            case SCATTER: res = g_fn.scatter(send[r], recv[r], count, dt, rt, comm[r], stream); break;
             default:
-                res = HcclAlltoAllV(send[r], t[0] + r * p, t[1] + r * p, dt, recv[r], t[2] + r * p, t[3] + r * p, dt, comm[r], stream);
+                res = g_fn.allToAllV(send[r], t[0] + r * p, t[1] + r * p, dt, recv[r], t[2] + r * p, t[3] + r * p, dt, comm[r], stream);
                 break;
         }
     }
@@ -165,8 +184,30 @@ PyObject *Call(PyObject *, PyObject *const *args, Py_ssize_t nargs)
     return PyLong_FromLong(static_cast<long>(res));
 }
 
+// bind(addresses): the library's functions, in the order of Kind, as integers.
+PyObject *Bind(PyObject *, PyObject *addresses)
+{
+    if (!PyTuple_CheckExact(addresses) || PyTuple_GET_SIZE(addresses) != KIND_COUNT) {
+        PyErr_SetString(PyExc_TypeError, "bind: a tuple of one address per collective");
+        return nullptr;
+    }
+    void *address[KIND_COUNT];
+    for (long k = 0; k < KIND_COUNT; k++) {
+        address[k] = PyLong_AsVoidPtr(PyTuple_GET_ITEM(addresses, k));
+        if (address[k] == nullptr) {
+            if (!PyErr_Occurred()) {
+                PyErr_SetString(PyExc_ValueError, "bind: null address");
+            }
+            return nullptr;
+        }
+    }
+    std::memcpy(&g_fn, address, sizeof(g_fn));
+    Py_RETURN_NONE;
+}
+
 PyMethodDef g_methods[] = {
     {"call", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(Call)), METH_FASTCALL, "one collective, called for every rank"},
+    {"bind", Bind, METH_O, "the functions that call() calls"},
     {nullptr, nullptr, 0, nullptr},
 };
 

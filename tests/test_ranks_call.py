@@ -2,6 +2,10 @@
 library sees the same arguments (told apart by its return codes; no GPU needed: without one a complete collective ends with
 HCCL_E_RUNTIME)."""
 import ctypes
+import os
+import shutil
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -87,3 +91,42 @@ def test_all_to_all_v_tables(comms, kind):
     wrong = back.copy()
     wrong[2, 1] += 1                    # rank 2 expects one more from rank 1 than it sends
     assert run(cnt, wrong) == H.HCCL_E_PARA
+
+
+# ---- start-up: in a process of its own, on a copy of the package beside a link to the built library ----------------
+
+START = """
+import importlib.util, sys
+spec = importlib.util.spec_from_file_location("mirror", sys.argv[1])
+H = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(H)
+comms = H.comm_init_all(2)
+try:
+    H.all_reduce(comms, [None, None], [4096, 8192], 8, H.HCCL_DATA_TYPE_FP32, 0, 1)
+except H.HcclError as e:
+    print("code", e.code)
+"""
+
+
+def _start(tmp_path, env):
+    package = os.path.dirname(os.path.dirname(H.LIB_PATH))
+    tree = tmp_path / "tree"
+    (tree / "lib").mkdir(parents=True)
+    shutil.copy(os.path.join(package, "__init__.py"), tree)
+    os.symlink(H.LIB_PATH, tree / "lib" / "libhccl.so")
+    os.symlink(H.RANKS_PATH, tree / "lib" / os.path.basename(H.RANKS_PATH))
+    r = subprocess.run([sys.executable, "-c", START, str(tree / "__init__.py")], env={**os.environ, **env}, stdout=subprocess.PIPE,
+                       stderr=subprocess.PIPE, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr
+    return r.stdout.strip()
+
+
+def test_the_library_called_is_the_one_loaded(tmp_path):
+    # another libhccl.so on the loader's search path, every function of which fails with 77
+    stub = tmp_path / "elsewhere"
+    stub.mkdir()
+    src = stub / "stub.cc"
+    src.write_text("".join('extern "C" int %s() { return 77; }\n' % name for name in H.EXPORTS))
+    subprocess.run(["g++", "-shared", "-fPIC", str(src), "-o", str(stub / "libhccl.so")], check=True)
+    path = str(stub) + os.pathsep + os.environ.get("LD_LIBRARY_PATH", "")
+    assert _start(tmp_path, {"LD_LIBRARY_PATH": path}) == "code %d" % H.HCCL_E_PTR

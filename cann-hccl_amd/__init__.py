@@ -16,7 +16,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libhccl.so")
-RANKS_PATH = os.path.join(_HERE, "lib", "_hccl_ranks.so")
+RANKS_PATH = os.path.join(_HERE, "lib", "_hccl_ranks" + importlib.machinery.EXTENSION_SUFFIXES[0])   # of this interpreter's ABI
 
 # HcclResult (include/hccl/hccl_types.h)
 HCCL_SUCCESS, HCCL_E_PARA, HCCL_E_PTR, HCCL_E_MEMORY, HCCL_E_INTERNAL, HCCL_E_NOT_SUPPORT = 0, 1, 2, 3, 4, 5
@@ -131,7 +131,7 @@ def lib():
     global _lib, _call
     if _lib is not None:
         return _lib
-    if not os.path.exists(LIB_PATH) or not os.path.exists(RANKS_PATH):
+    if not os.path.exists(LIB_PATH):
         # nothing built yet (a fresh checkout): build once, in tree; a built library is never rebuilt from here
         spec = importlib.util.spec_from_file_location("cann_hccl_amd_build", os.path.join(os.path.dirname(__file__), "build.py"))
         builder = importlib.util.module_from_spec(spec)
@@ -140,7 +140,7 @@ def lib():
             builder.build()
         except Exception as e:   # noqa: BLE001
             raise RuntimeError("libhccl.so is not built and building it failed (needs hipcc): %s" % e)
-    if not os.path.exists(LIB_PATH) or not os.path.exists(RANKS_PATH):
+    if not os.path.exists(LIB_PATH):
         raise RuntimeError("libhccl.so is not built: run `python cann-hccl_amd/build.py` (needs hipcc)")
     # Streams and device pointers handed to the library must belong to the HIP runtime the library
     # itself uses.  PyTorch ships its own libamdhip64 (same soname): when it is loaded first the
@@ -191,11 +191,7 @@ def lib():
     L.HcclAmdGetLastOpInfo.argtypes = [vp, ctypes.POINTER(HcclAmdOpInfo)]
     L.HcclAmdDescribePlan.argtypes = [i32, i32, u32, u64, i32, u64, u64, u64, ctypes.POINTER(u64), ctypes.c_char_p,
                                       ctypes.c_size_t, ctypes.POINTER(ctypes.c_size_t)]
-    loader = importlib.machinery.ExtensionFileLoader("_hccl_ranks", RANKS_PATH)
-    ranks = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_hccl_ranks", RANKS_PATH, loader=loader))
-    loader.exec_module(ranks)
-    ranks.bind(tuple(ctypes.cast(getattr(L, name), vp).value for name in _KINDS))
-    _call = ranks.call
+    _call = _native_call(L) or _through_ctypes
     _lib = L
     return L
 
@@ -206,6 +202,24 @@ _KINDS = ("HcclAllReduce", "HcclReduceScatter", "HcclAmdReduceScatterNoAlloc", "
           "HcclScatter", "HcclAlltoAllV")
 (_ALL_REDUCE, _REDUCE_SCATTER, _REDUCE_SCATTER_NO_ALLOC, _ALL_GATHER, _ALL_TO_ALL, _BROADCAST, _REDUCE, _SCATTER,
  _ALL_TO_ALL_V) = range(9)
+
+
+def _native_call(L):
+    """The native loop over L's functions; None where the extension is not there for this interpreter."""
+    if not os.path.exists(RANKS_PATH):
+        return None
+    loader = importlib.machinery.ExtensionFileLoader("_hccl_ranks", RANKS_PATH)
+    try:
+        ranks = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_hccl_ranks", RANKS_PATH, loader=loader))
+        loader.exec_module(ranks)
+    except ImportError:
+        return None
+    ranks.bind(tuple(ctypes.cast(getattr(L, name), ctypes.c_void_p).value for name in _KINDS))
+    return ranks.call
+
+
+def _through_ctypes(*args):
+    return -1
 
 
 def _load_and_call(*args):

@@ -17,7 +17,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libhccl.so")
-RANKS = os.path.join(LIBDIR, "_hccl_ranks.so")
+RANKS = os.path.join(LIBDIR, "_hccl_ranks" + sysconfig.get_config_var("EXT_SUFFIX"))   # of this interpreter's ABI
 ABI_CALLER = os.path.join(LIBDIR, "abi_caller")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -83,12 +83,17 @@ def build(force=False, jobs=None):
 
 
 def build_ranks(force=False):
-    """The Python mirror's loop over the ranks (csrc/pyranks.cc), a CPython extension.  It calls what the mirror
-    hands it and is linked against nothing."""
+    """The Python mirror's loop over the ranks (csrc/pyranks.cc), a CPython extension that calls what the mirror
+    hands it and is linked against nothing.  An accelerator only: where it cannot
+    be built (no headers of the interpreter, say) the mirror calls through ctypes."""
     src = os.path.join(CSRC, "pyranks.cc")
     if force or _newer(RANKS, [src]):
-        _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-I", os.path.join(ROOT, "include"),
-              "-I", sysconfig.get_paths()["include"], src, "-o", RANKS])
+        try:
+            _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-I", os.path.join(ROOT, "include"),
+                  "-I", sysconfig.get_paths()["include"], src, "-o", RANKS])
+        except (RuntimeError, OSError) as e:
+            sys.stderr.write("the loop over the ranks is not built, the Python mirror goes through ctypes: %s\n" % e)
+            return None
     return RANKS
 
 

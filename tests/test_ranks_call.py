@@ -104,21 +104,30 @@ comms = H.comm_init_all(2)
 try:
     H.all_reduce(comms, [None, None], [4096, 8192], 8, H.HCCL_DATA_TYPE_FP32, 0, 1)
 except H.HcclError as e:
-    print("code", e.code)
+    print("code", e.code, "native", int(H._call is not H._through_ctypes))
 """
 
 
-def _start(tmp_path, env):
+def _start(tmp_path, with_extension, env=None):
     package = os.path.dirname(os.path.dirname(H.LIB_PATH))
     tree = tmp_path / "tree"
     (tree / "lib").mkdir(parents=True)
     shutil.copy(os.path.join(package, "__init__.py"), tree)
     os.symlink(H.LIB_PATH, tree / "lib" / "libhccl.so")
-    os.symlink(H.RANKS_PATH, tree / "lib" / os.path.basename(H.RANKS_PATH))
-    r = subprocess.run([sys.executable, "-c", START, str(tree / "__init__.py")], env={**os.environ, **env}, stdout=subprocess.PIPE,
+    if with_extension == "broken":
+        (tree / "lib" / os.path.basename(H.RANKS_PATH)).write_bytes(b"not a library")
+    elif with_extension:
+        os.symlink(H.RANKS_PATH, tree / "lib" / os.path.basename(H.RANKS_PATH))
+    r = subprocess.run([sys.executable, "-c", START, str(tree / "__init__.py")], env={**os.environ, **(env or {})}, stdout=subprocess.PIPE,
                        stderr=subprocess.PIPE, text=True, timeout=300)
     assert r.returncode == 0, r.stderr
     return r.stdout.strip()
+
+
+@pytest.mark.parametrize("with_extension,native", [(True, 1), (False, 0), ("broken", 0)])
+def test_starts_without_the_extension(tmp_path, with_extension, native):
+    # a tree that was built with another interpreter, or without its headers, holds no extension for this one
+    assert _start(tmp_path, with_extension) == "code %d native %d" % (H.HCCL_E_PTR, native)
 
 
 def test_the_library_called_is_the_one_loaded(tmp_path):
@@ -129,4 +138,4 @@ def test_the_library_called_is_the_one_loaded(tmp_path):
     src.write_text("".join('extern "C" int %s() { return 77; }\n' % name for name in H.EXPORTS))
     subprocess.run(["g++", "-shared", "-fPIC", str(src), "-o", str(stub / "libhccl.so")], check=True)
     path = str(stub) + os.pathsep + os.environ.get("LD_LIBRARY_PATH", "")
-    assert _start(tmp_path, {"LD_LIBRARY_PATH": path}) == "code %d" % H.HCCL_E_PTR
+    assert _start(tmp_path, True, {"LD_LIBRARY_PATH": path}) == "code %d native 1" % H.HCCL_E_PTR

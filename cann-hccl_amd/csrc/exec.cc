@@ -1069,7 +1069,8 @@ bool ReduceColl(int coll) { return coll == COLL_ALLREDUCE || coll == COLL_REDUCE
 // overlaps a receive buffer other than as an exact in-place pair is staged through scratch (*needStage).
 // An all-gather in place -- rank r sends its own block of its receive buffer -- is none of that for the fused form, in
 // which nothing but that block's item touches the block (*gatherInPlace); step by step, other blocks pass through it.
-HcclResult CheckOverlap(const Group *g, const Plan &plan, bool *needStage, bool *gatherInPlace)
+HcclResult CheckOverlap(const Group *g, const std::vector<uint64_t> &sendBytes, const std::vector<uint64_t> &recvBytes, bool *needStage,
+    bool *gatherInPlace)
 {
     *needStage = *gatherInPlace = false;
     const OpSig &sig = g->ctx->sig;
@@ -1079,11 +1080,11 @@ HcclResult CheckOverlap(const Group *g, const Plan &plan, bool *needStage, bool 
         for (uint32_t j = 0; j < g->p; j++) {
             const char *rj = static_cast<const char *>(g->ctx->recv[j]);
             const char *sj = static_cast<const char *>(g->ctx->send[j]);
-            if (i != j && RangesOverlap(ri, plan.recvBytes[i], rj, plan.recvBytes[j])) {
+            if (i != j && RangesOverlap(ri, recvBytes[i], rj, recvBytes[j])) {
                 HCCL_LOG_ERROR("%s: receive buffers of rank %u and rank %u overlap", CollName(g->ctx->sig.coll), i, j);
                 return HCCL_E_PARA;
             }
-            if (RangesOverlap(ri, plan.recvBytes[i], sj, plan.sendBytes[j])) {
+            if (RangesOverlap(ri, recvBytes[i], sj, sendBytes[j])) {
                 bool exact = (i == j) && ri == sj && (sig.coll == COLL_ALLREDUCE || sig.coll == COLL_BROADCAST);
                 bool ownBlock = (i == j) && sig.coll == COLL_ALLGATHER && sj == ri + (sig.variable ? g->ctx->vDispls[i] : i * sig.count) * unit;
                 *gatherInPlace = *gatherInPlace || ownBlock;
@@ -1120,7 +1121,7 @@ HcclResult Prepare(Group *g, int algo, std::unique_ptr<Prepared> *out, bool noAl
         return rc == 1 ? HCCL_E_PARA : HCCL_E_INTERNAL;
     }
     bool needStage = false, gatherInPlace = false;
-    HcclResult overlap = CheckOverlap(g, *pp->plan, &needStage, &gatherInPlace);
+    HcclResult overlap = CheckOverlap(g, pp->plan->sendBytes, pp->plan->recvBytes, &needStage, &gatherInPlace);
     if (overlap != HCCL_SUCCESS) {
         return overlap;
     }
@@ -1237,7 +1238,7 @@ DirectLaunch *FindDirect(Group *g, int algo)
     const OpSig &sig = g->ctx->sig;
     const GroupConfig &cfg = g->cfg;
     if (sig.noAlloc || sig.variable || sig.coll == COLL_ALLTOALLV || !cfg.fuse || cfg.team == 1 || cfg.blocksPerCu != 0 ||
-        cfg.launchCapMiB >= 0 || cfg.fusedStores >= 0) {
+        cfg.launchCapMiB >= 0 || cfg.fusedStores >= 0 || !DirectFits(sig.coll, g->p, sig.count * DtypeSize(sig.dtype))) {
         return nullptr;
     }
     uint64_t inPlace = 0;
@@ -1251,16 +1252,17 @@ DirectLaunch *FindDirect(Group *g, int algo)
     std::string key(reinterpret_cast<const char *>(head), sizeof(head));
     auto it = g->direct.find(key);
     if (it == g->direct.end()) {
-        if (g->direct.size() >= 256) {
-            g->direct.clear();
+        if (g->direct.size() >= cfg.cacheEntries) {
+            g->direct.clear();          // as the prepared collectives: the table starts over
         }
         DirectLaunch d;
+        std::shared_ptr<const Plan> plan;
         std::string err;
-        if (CachedPlan(g, MakeRequest(g, algo), &d.plan, &err) != 0) {
+        if (CachedPlan(g, MakeRequest(g, algo), &plan, &err) != 0) {
             return nullptr;             // the general path reports it
         }
-        if (BuildDirect(*d.plan, ReduceColl(sig.coll), sig.dtype, sig.op, &d)) {
-            d.info = MakeInfo(g, algo, *d.plan, true);
+        if (BuildDirect(*plan, ReduceColl(sig.coll), sig.dtype, sig.op, &d)) {
+            d.info = MakeInfo(g, algo, *plan, true);
             d.info.launches = 1;
         } else {
             d = DirectLaunch();
@@ -1269,7 +1271,7 @@ DirectLaunch *FindDirect(Group *g, int algo)
     }
     DirectLaunch *d = &it->second;
     bool needStage = false, gatherInPlace = false;   // (a gathered block stored onto itself: by the lane that has read it)
-    if (d->func == nullptr || CheckOverlap(g, *d->plan, &needStage, &gatherInPlace) != HCCL_SUCCESS || needStage) {
+    if (d->func == nullptr || CheckOverlap(g, d->sendBytes, d->recvBytes, &needStage, &gatherInPlace) != HCCL_SUCCESS || needStage) {
         return nullptr;
     }
     d->info.cacheHit = FillBases(d, g->ctx->send, g->ctx->recv) ? 1 : 0;

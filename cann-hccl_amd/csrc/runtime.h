@@ -109,17 +109,19 @@ struct Prepared {
 };
 
 // One launch whose descriptors ride in its arguments (small collectives, kernels_direct.h).  It belongs to a request, not to
-// buffers: the base pointers are filled in by every call.
+// buffers: the base pointers are filled in by every call.  Of the plan only the buffers' lengths are kept.
 struct DirectLaunch {
-    std::shared_ptr<const Plan> plan;
     const void *func = nullptr;       // nullptr: this request does not go out this way
     uint32_t gridX = 0, gridY = 0;
     std::vector<std::pair<uint32_t, uint8_t>> bases;   // (rank, buffer) of every base pointer
     std::vector<uint8_t> image;                        // the kernel's arguments, a DirectArgs
+    std::vector<uint64_t> sendBytes, recvBytes;        // per rank, as the plan's
     OpInfo info;
 };
 
-// The launch of `plan`; false (func == nullptr) where it is not small or does not fit.
+// Whether a collective is small enough for this form, whatever its schedule (bytes: of the call's count).
+bool DirectFits(int coll, uint32_t p, uint64_t bytes);
+// The launch of `plan`; false (func == nullptr) where the kernels' records cannot hold it.
 bool BuildDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaunch *d);
 // Puts the ranks' pointers in; true if they were there already (the previous call's).
 bool FillBases(DirectLaunch *d, const std::vector<void *> &send, const std::vector<void *> &recv);
@@ -226,7 +228,7 @@ struct Group {
     uint64_t scratchBytes = 0;
     uint64_t scratchGen = 0;
     std::unordered_map<std::string, std::unique_ptr<Prepared>> cache;   // keyed by request, settings and buffer addresses
-    std::unordered_map<std::string, DirectLaunch> direct;   // small collectives, keyed by request and settings
+    std::unordered_map<std::string, DirectLaunch> direct;   // small collectives, keyed by request and settings; as many as `cache` holds
     TableArena arena;
     std::unordered_map<std::string, std::shared_ptr<const Plan>> planCache;   // keyed by the plan request
     std::unordered_map<std::string, std::vector<TemplateSlot>> planTemplates;   // keyed by the request without its count

@@ -9,6 +9,7 @@
 #pragma once
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <atomic>
 #include <condition_variable>
 #include <deque>
@@ -106,6 +107,23 @@ struct Prepared {
     bool pinned = false;
     OpInfo info;
     ~Prepared();
+};
+
+// Everything the launch of a small collective depends on besides the buffers: the request and the settings.
+struct DirectKey {
+    uint64_t w[8];
+    bool operator==(const DirectKey &o) const { return std::equal(w, w + 8, o.w); }
+};
+struct DirectKeyHash {
+    size_t operator()(const DirectKey &k) const
+    {
+        uint64_t h = 0;
+        for (uint64_t w : k.w) {
+            h = (h ^ w) * 0x9E3779B97F4A7C15ull;
+            h ^= h >> 32;
+        }
+        return size_t(h);
+    }
 };
 
 // One launch whose descriptors ride in its arguments (small collectives, kernels_direct.h).  It belongs to a request, not to
@@ -228,7 +246,7 @@ struct Group {
     uint64_t scratchBytes = 0;
     uint64_t scratchGen = 0;
     std::unordered_map<std::string, std::unique_ptr<Prepared>> cache;   // keyed by request, settings and buffer addresses
-    std::unordered_map<std::string, DirectLaunch> direct;   // small collectives, keyed by request and settings; as many as `cache` holds
+    std::unordered_map<DirectKey, DirectLaunch, DirectKeyHash> direct;   // small collectives, as many as `cache` holds
     TableArena arena;
     std::unordered_map<std::string, std::shared_ptr<const Plan>> planCache;   // keyed by the plan request
     std::unordered_map<std::string, std::vector<TemplateSlot>> planTemplates;   // keyed by the request without its count

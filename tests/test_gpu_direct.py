@@ -124,3 +124,41 @@ def test_new_buffers_and_graph_replay(orc):
                 assert np.array_equal(gh.to_host(r[k], FP32), want[k])
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("p", [4, 33])
+def test_overlapping_buffers_among_in_place_ranks(orc, p):
+    # some ranks in place, all else apart: one pass; a send buffer that reaches into another rank's receive buffer, or into its
+    # own at another offset: staged; two receive buffers that overlap: refused, and what is called next is not disturbed
+    n, dt = 1000, INT8
+    ins = _ins(dt, p, n, 11)
+    want = orc.allreduce(ins, dt, SUM)
+    g = gh.Group(p)
+    try:
+        for case in ("apart", "into another's", "into its own", "two receivers", "apart"):
+            pool = torch.zeros(2 * p * 4096, dtype=torch.uint8, device="cuda")
+            at = lambda k: pool[k * 4096:k * 4096 + n]  # noqa: E731
+            sends, recvs = [at(2 * r) for r in range(p)], [at(2 * r if r % 3 == 1 else 2 * r + 1) for r in range(p)]
+            if case == "into another's":
+                recvs[0] = pool[4 * 4096 + n - 1:4 * 4096 + n - 1 + n]      # the last byte of rank 2's send buffer
+            elif case == "into its own":
+                recvs[0] = pool[1:1 + n]
+            elif case == "two receivers":
+                recvs[0] = pool[5 * 4096 + n - 1:5 * 4096 + n - 1 + n]              # the last byte of rank 2's receive buffer
+            for r in range(p):
+                sends[r].copy_(torch.from_numpy(ins[r].view(np.uint8)))
+            torch.cuda.synchronize()
+            args = (g.comms, [t.data_ptr() for t in sends], [t.data_ptr() for t in recvs], n, dt, SUM, g.stream_ptr)
+            print("overlap", p, case, flush=True)
+            if case == "two receivers":
+                with pytest.raises(H.HcclError) as e:
+                    H.all_reduce(*args)
+                assert e.value.code == H.HCCL_E_PARA
+                continue
+            H.all_reduce(*args)
+            g.stream.synchronize()
+            assert g.info()["fused"] == (1 if case == "apart" else 0)
+            for r in range(p):
+                assert gh.same(dt, gh.to_host(recvs[r], dt), want[r]), (case, r)
+    finally:
+        g.close()

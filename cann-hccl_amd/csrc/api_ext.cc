@@ -130,6 +130,14 @@ HcclResult HcclAmdSetParam(HcclComm comm, const char *key, const char *value)
         } else {
             return HCCL_E_PARA;
         }
+    } else if (k == "direct") {
+        if (v == "auto") {
+            cfg.direct = true;
+        } else if (v == "0") {
+            cfg.direct = false;
+        } else {
+            return HCCL_E_PARA;
+        }
     } else if (k == "step_stores") {
         if (v == "auto") {
             cfg.stepStores = -1;
@@ -212,7 +220,7 @@ HcclResult HcclAmdGetLastOpInfo(HcclComm comm, HcclAmdOpInfo *info)
     info->schedWritten = o.stepWritten;
     info->scratchBytes = o.scratchBytes;
     info->teamLaunches = o.teamLaunches;
-    info->reserved = 0;
+    info->direct = o.direct;
     return HCCL_SUCCESS;
 }
 

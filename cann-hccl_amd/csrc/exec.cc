@@ -1268,7 +1268,7 @@ DirectLaunch *FindDirect(Group *g, int algo)
 {
     const OpSig &sig = g->ctx->sig;
     const GroupConfig &cfg = g->cfg;
-    if (sig.noAlloc || sig.variable || sig.coll == COLL_ALLTOALLV || !cfg.fuse || cfg.team == 1 || cfg.blocksPerCu != 0 ||
+    if (sig.noAlloc || sig.variable || sig.coll == COLL_ALLTOALLV || !cfg.fuse || !cfg.direct || cfg.team == 1 || cfg.blocksPerCu != 0 ||
         cfg.launchCapMiB >= 0 || cfg.fusedStores >= 0 || !DirectFits(sig.coll, g->p, sig.count * DtypeSize(sig.dtype))) {
         return nullptr;
     }
@@ -1294,6 +1294,7 @@ DirectLaunch *FindDirect(Group *g, int algo)
         if (BuildDirect(*plan, ReduceColl(sig.coll), sig.dtype, sig.op, &d)) {
             d.info = MakeInfo(g, algo, *plan, true);
             d.info.launches = 1;
+            d.info.direct = 1;
         } else {
             d = DirectLaunch();
         }

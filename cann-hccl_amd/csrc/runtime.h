@@ -51,6 +51,7 @@ struct GroupConfig {
     uint32_t teamTiles = 0;               // team kernels: tiles per workgroup and round, 0 = chosen per launch
     int team = -1;                        // team form of the fused kernels (an XCD's workgroups read together, then write together):
                                           // 1 wherever it can run, 0 never, -1 for large launches whose items touch many streams
+    bool direct = true;                   // small collectives go out as one launch whose descriptors ride in its arguments
     bool blockingArrive = false;          // ranks wait inside the call until the collective is issued
     uint32_t arriveTimeoutMs = 1800 * 1000;
 };
@@ -80,6 +81,7 @@ struct OpInfo {
     int coll = 0, algo = 0, fused = 0, graph = 0, cacheHit = 0;
     uint32_t launches = 0;
     uint32_t teamLaunches = 0;
+    uint32_t direct = 0;                          // 1: one launch whose descriptors ride in its arguments
     uint64_t bytesRead = 0, bytesWritten = 0;     // what the issued kernels move in HBM, all ranks
     uint64_t stepRead = 0, stepWritten = 0;       // the step-by-step schedule's figure
     uint64_t scratchBytes = 0;

@@ -62,6 +62,9 @@ extern "C" {
  *                                all-gather, broadcast); "1": wherever the device allows it; "0": never
  *   "team_tiles"    tiles of 16 KiB a workgroup of a team kernel takes per round, 1 ... 8 ("0", default: 8, fewer when an
  *                                item has more than 8 sources or destinations)
+ *   "direct"        "auto" | "0"   small collectives go out as one launch whose descriptors ride in its arguments ("auto",
+ *                                default: not with "fuse" = "0", "team" = "1" or any of "blocks_per_cu", "launch_cap_mib" and
+ *                                "fused_stores" set), or through descriptor tables as all others ("0")
  *   "cache_entries" how many prepared collectives (distinct sizes, buffers, settings) the group keeps (default 1024);
  *                   when full, the library waits for the device once and starts over
  *   "blocks_per_cu" launch width in workgroups per compute unit ("0": chosen per collective)
@@ -93,7 +96,7 @@ typedef struct HcclAmdOpInfoDef {
     uint64_t schedWritten;
     uint64_t scratchBytes;   /* per-rank scratch in use */
     uint32_t teamLaunches;   /* how many of the launches are team kernels (setting "team") */
-    uint32_t reserved;
+    uint32_t direct;         /* 1: one launch whose descriptors ride in its arguments (setting "direct") */
 } HcclAmdOpInfo;
 
 /* What the most recent collective of this communicator's group issued. */

@@ -6,6 +6,8 @@ import subprocess
 
 import pytest
 
+from hccl_loader import load
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
@@ -25,3 +27,16 @@ def test_the_arguments_are_the_plans_items(tmp_path):
     assert out.returncode == 0 and out.stdout.startswith("OK"), out.stdout
     # every kind of record was met, and every reason to go another way
     assert min(int(w) for w in out.stdout.split() if w.isdigit()) > 500, out.stdout
+
+
+def test_the_setting():
+    H = load()
+    comms = H.comm_init_all(2)
+    for v in ("0", "auto"):
+        H.set_param(comms[0], "direct", v)
+    for v in ("1", "2", "", "yes"):
+        with pytest.raises(H.HcclError) as e:
+            H.set_param(comms[0], "direct", v)
+        assert e.value.code == H.HCCL_E_PARA
+    assert H.last_op_info(comms[0])["direct"] == 0
+    H.comm_destroy(comms)

@@ -1,7 +1,7 @@
 """Small collectives, whose descriptors ride in the kernel arguments (one launch, 4 KiB of an item per workgroup), against the
 CPU checker bit for bit: the edges of a workgroup's 4 KiB and of a 16-byte vector, every batch size of sources, trees and
 stack programs, buffers at any element boundary, in place, operand order on NaNs and signed zeros, new buffers on every call
-and replays of a caller's graph."""
+and replays of a caller's graph.  Whether a call went that way is asserted for every one of them.  Whether a call went that way is asserted for every one of them."""
 import numpy as np
 import pytest
 import torch
@@ -26,30 +26,71 @@ def _ins(dt, p, n, seed, special=False):
     return ins
 
 
+def _fits(plan):
+    """Whether one launch's arguments hold the plan: items, sources and destinations per item, base pointers."""
+    def one(cap, items, bases):
+        seen = set()
+        for it in plan["fused"]:
+            src = [(k, r) for k, r in enumerate(it["src"]) if r]
+            tree, stack = it["kind"] == 2, it["kind"] == 3
+            if (it["nleaf"] if tree else len(src)) > cap or len(it["dst"]) > cap or (stack and cap > 8) or \
+                    (tree and it["nleaf"] > 2 * cap // (2 if cap <= 8 else 4) and any(k & 1 for k, _ in src)):
+                return False
+            if len({str(r[2:]) for _, r in src}) > 1 or len({str(r[2:]) for r in it["dst"]}) > 1:
+                return False
+            seen |= {tuple(r[:2]) for _, r in src} | {tuple(r[:2]) for r in it["dst"]}
+        return len(plan["fused"]) <= items and len(seen) <= bases
+    return plan["fusedOk"] and bool(plan["fused"]) and (one(8, 16, 16) or one(32, 32, 64))
+
+
+def _fits(plan):
+    """Whether one launch's arguments hold the plan: items, sources and destinations per item, base pointers."""
+    def one(cap, items, bases):
+        seen = set()
+        for it in plan["fused"]:
+            src = [(k, r) for k, r in enumerate(it["src"]) if r]
+            tree, stack = it["kind"] == 2, it["kind"] == 3
+            if (it["nleaf"] if tree else len(src)) > cap or len(it["dst"]) > cap or (stack and cap > 8) or \
+                    (tree and it["nleaf"] > min(cap, 16) and any(k & 1 for k, _ in src)):
+                return False
+            if len({r[2] for _, r in src}) > 1 or len({r[2] for r in it["dst"]}) > 1:
+                return False
+            seen |= {tuple(r[:2]) for _, r in src} | {tuple(r[:2]) for r in it["dst"]}
+        return len(plan["fused"]) <= items and len(seen) <= bases
+    return plan["fusedOk"] and bool(plan["fused"]) and (one(8, 16, 16) or one(32, 32, 64))
+
+
 # ring: chains of 1 ... 32 sources (batches of 16, 8 and a rest); halving-doubling: trees of 2 ... 32 leaves with and
-# without second sources; several groups: stack programs
-@pytest.mark.parametrize("p,algo,servers", [(2, RING, 1), (3, RING, 1), (7, RING, 1), (8, RING, 1), (9, RING, 1), (15, RING, 1), (24, RING, 1),
-                                            (31, RING, 1), (32, RING, 1), (8, MESH, 1), (2, RHD, 1), (6, RHD, 1), (8, RHD, 1),
-                                            (13, RHD, 1), (24, RHD, 1), (32, RHD, 1), (8, RHD, 2), (8, RHD, 4), (6, RING, 3)])
-def test_all_reduce(orc, p, algo, servers):
-    g = gh.Group(p, algo=("ring", "mesh", "rhd")[algo], servers=servers, deterministic=1)
+# without second sources; several groups: stack programs, with and without the piece cut (whose items do not always fit)
+@pytest.mark.parametrize("p,algo,servers,cut", [(2, RING, 1, 1), (3, RING, 1, 1), (7, RING, 1, 1), (8, RING, 1, 1), (9, RING, 1, 1), (15, RING, 1, 1),
+                                                (24, RING, 1, 1), (31, RING, 1, 1), (32, RING, 1, 1), (8, MESH, 1, 1), (2, RHD, 1, 1), (6, RHD, 1, 1),
+                                                (8, RHD, 1, 1), (13, RHD, 1, 1), (24, RHD, 1, 1), (32, RHD, 1, 1), (8, RHD, 2, 1), (8, RHD, 4, 1),
+                                                (6, RING, 3, 1), (8, RHD, 2, 0), (8, RING, 2, 0)])
+def test_all_reduce(orc, p, algo, servers, cut):
+    g = gh.Group(p, algo=("ring", "mesh", "rhd")[algo], servers=servers, deterministic=cut)
+    ways = []
     try:
         for k, (dt, op, pad, in_place, special) in enumerate([(FP32, SUM, 0, False, False), (BF16, MAX, 2, True, True), (INT8, PROD, 3, False, False),
                                                               (FP16, MIN, 16, False, True), (INT64, SUM, 8, True, False)]):
             unit = H.DTYPE_SIZE[dt]
-            sizes = {1, 128 * p // unit + 1, (4096 * p) // unit, (4096 * p + 128) // unit - 1, (3 * 4096 + 128) * p // unit + 5, (1 << 20) // unit}
+            sizes = {1, 128 * p // unit + 1, (4096 * p) // unit, (4096 * p + 128) // unit - 1, (3 * 4096 + 128) * p // unit + 5, (1 << 20) // unit, (1 << 20) // unit + 1}
+            uncut = int(not cut and dt != INT64 and op != PROD)
             for n in sorted(sizes):
                 print("small all-reduce", p, algo, servers, "type", dt, "op", op, "n", n, "pad", pad, flush=True)
                 ins = _ins(dt, p, n, 31 * p + n % 1009 + k, special)
                 if servers > 1:
-                    want = orc.allreduce_two_level(ins, dt, op, servers, level1=algo)
+                    want = orc.allreduce_two_level(ins, dt, op, servers, level1=algo, atomic=bool(uncut))
                 else:
                     want = orc.allreduce(ins, dt, op, algo=algo)
                 outs, keep = gh.all_reduce(g, ins, dt, op, in_place=in_place, pad=pad)
-                assert g.info()["launches"] <= 1 or servers > 1 or algo == MESH
+                word = algo | ((servers << 8 | uncut << 16) if servers > 1 else 0)
+                plan = H.describe_plan(H.COLL_ALLREDUCE, word, p, n, dt, in_place_mask=(1 << p) - 1 if in_place else 0)
+                ways.append(int(n * unit <= 1 << 20 and _fits(plan)))
+                assert g.info()["direct"] == ways[-1] and (ways[-1] == 0 or g.info()["launches"] == 1), (dt, op, n)
                 for r in range(p):
                     assert gh.same(dt, outs[r], want[r]), (dt, op, n, r)
                     assert keep is None or np.array_equal(keep[r].view(np.uint8), ins[r].view(np.uint8))
+        assert 0 in ways and 1 in ways
     finally:
         g.close()
 
@@ -66,10 +107,12 @@ def test_blocks(orc, p):
                 ins = _ins(dt, p, n * p, 77 * p + n)
                 want = orc.reducescatter(ins, dt, op)
                 outs, _ = gh.reduce_scatter(g, ins, dt, op, pad=pad)
+                assert g.info()["direct"] == 1
                 for r in range(p):
                     assert gh.same(dt, outs[r], want[r]), ("reduce-scatter", dt, n, r)
                 parts = [x[:n] for x in ins]
                 outs = gh.all_gather(g, parts, dt, pad=pad)
+                assert g.info()["direct"] == int(p * (p + 1) * n * unit <= 20 << 20)
                 for r in range(p):
                     assert np.array_equal(outs[r].view(np.uint8), np.concatenate(parts).view(np.uint8)), ("all-gather", dt, n, r)
                 root = n % p
@@ -77,10 +120,13 @@ def test_blocks(orc, p):
                 dst = [gh.empty_dev(n * unit, pad) for _ in range(p)]
                 torch.cuda.synchronize()
                 H.reduce(g.comms, [t.data_ptr() for t in bufs], [t.data_ptr() for t in dst], n, dt, op, root, g.stream_ptr)
+                assert g.info()["direct"] == 1
                 H.send(g.comms[0], bufs[0].data_ptr(), n, dt, p - 1, g.stream_ptr)
                 spare = gh.empty_dev(n * unit, pad)
                 H.recv(g.comms[p - 1], spare.data_ptr(), n, dt, 0, g.stream_ptr)
+                assert g.info()["direct"] == 1
                 H.broadcast(g.comms, [t.data_ptr() for t in bufs], n, dt, root, g.stream_ptr)
+                assert g.info()["direct"] == 1
                 g.stream.synchronize()
                 assert gh.same(dt, gh.to_host(dst[root], dt), orc.reduce_to_root(parts, dt, op, root)), ("reduce", dt, n)
                 assert np.array_equal(gh.to_host(spare, dt).view(np.uint8), parts[0].view(np.uint8)), ("send / receive", dt, n)
@@ -103,6 +149,7 @@ def test_new_buffers_and_graph_replay(orc):
         for s, r in sets + sets[-1:]:
             H.all_reduce(g.comms, [t.data_ptr() for t in s], [t.data_ptr() for t in r], n, FP32, SUM, g.stream_ptr)
             hits.append(g.info()["cacheHit"])
+            assert g.info()["direct"] == 1
         assert hits == [0] * 20 + [1]
         s, r = sets[3]
         graph = torch.cuda.CUDAGraph()

@@ -18,6 +18,15 @@ namespace {
 //     16 ranks 1 MiB 5.1 / 4.2, 2 MiB 6.7 / 6.8
 constexpr uint64_t kDirectMaxBytes = uint64_t(1) << 20;       // of a reduction's results
 constexpr uint64_t kDirectMaxToOne = uint64_t(4) << 20;       // the same where each has one destination
+// Blocks of whole 16-byte vectors of more than three sources, in types that combine in an instruction or two: the tile
+// kernels get ahead sooner there.  Tile kernels / this form, us, new data for every call, one destination per result:
+//   reduce-scatter, fp32: 4 ranks 2.5 MiB 5.1 / 5.1, 4 MiB 6.1 / 6.2; 16 ranks 2.5 MiB 10.4 / 9.7, 3 MiB 11.3 / 11.9;
+//     32 ranks 2.5 MiB 17.6 / 16.5, 4 MiB 23.5 / 24.8; int64 32 ranks 3 MiB 18.5 / 20.5
+//   reduce, fp32: 8 ranks 2.5 MiB 6.8 / 6.3, 4 MiB 8.5 / 8.8; 32 ranks 2.5 MiB 17.2 / 16.3, 4 MiB 22.8 / 25.4
+// Up to the larger limit this form stays ahead for bf16 and 8-bit elements (32 ranks, 4 MiB: bf16 27.6 / 25.1, int8 26.3 / 25.1)
+// and for ragged blocks, whose ends the tile kernels take element by element (fp32, 32 ranks, 4 MiB 62.9 / 27.6), and for three sources or fewer (3 ranks, 4 MiB 6.2 / 5.4).
+// Copies, also from one to one, are ahead up to their limit for 2 to 32 ranks (scatter of 10 MiB 6.4 / 6.0).
+constexpr uint64_t kDirectMaxToOneEven = uint64_t(5) << 19;
 constexpr uint64_t kDirectMaxTraffic = uint64_t(20) << 20;    // read and written by a collective that only moves data
 // The rule looks at the call alone: a collective that is too large is told apart before anything is looked up or planned
 // for it (with a look into the plan, a caller with more distinct requests than this form's table holds paid for a plan on
@@ -111,12 +120,14 @@ template <uint32_t CAP> bool FillDirect(const Plan &plan, DirectLaunch *d)
 
 }  // namespace
 
-bool DirectFits(int coll, uint32_t p, uint64_t bytes)
+bool DirectFits(int coll, uint32_t p, uint64_t bytes, int dtype)
 {
+    const bool even = bytes % 16 == 0 && p > 3 && dtype != HCCL_DATA_TYPE_INT8 && dtype != HCCL_DATA_TYPE_UINT8 && dtype != HCCL_DATA_TYPE_BFP16;
+    const uint64_t toOne = even ? kDirectMaxToOneEven : kDirectMaxToOne;
     switch (coll) {
-        case COLL_ALLREDUCE: return bytes <= (p > 1 ? kDirectMaxBytes : kDirectMaxToOne);
-        case COLL_REDUCESCATTER: return bytes <= kDirectMaxToOne / p;
-        case COLL_REDUCE: return bytes <= kDirectMaxToOne;
+        case COLL_ALLREDUCE: return bytes <= (p > 1 ? kDirectMaxBytes : toOne);
+        case COLL_REDUCESCATTER: return bytes <= toOne / p;
+        case COLL_REDUCE: return bytes <= toOne;
         case COLL_ALLGATHER: return bytes <= kDirectMaxTraffic / p / (p + 1);
         case COLL_BROADCAST: return bytes <= kDirectMaxTraffic / p;
         case COLL_SCATTER: return bytes <= kDirectMaxTraffic / p / 2;

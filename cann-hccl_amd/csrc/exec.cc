@@ -1269,7 +1269,7 @@ DirectLaunch *FindDirect(Group *g, int algo)
     const OpSig &sig = g->ctx->sig;
     const GroupConfig &cfg = g->cfg;
     if (sig.noAlloc || sig.variable || sig.coll == COLL_ALLTOALLV || !cfg.fuse || !cfg.direct || cfg.team == 1 || cfg.blocksPerCu != 0 ||
-        cfg.launchCapMiB >= 0 || cfg.fusedStores >= 0 || !DirectFits(sig.coll, g->p, sig.count * DtypeSize(sig.dtype))) {
+        cfg.launchCapMiB >= 0 || cfg.fusedStores >= 0 || !DirectFits(sig.coll, g->p, sig.count * DtypeSize(sig.dtype), sig.dtype)) {
         return nullptr;
     }
     uint64_t inPlace = 0;

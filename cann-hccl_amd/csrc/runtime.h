@@ -140,7 +140,7 @@ struct DirectLaunch {
 };
 
 // Whether a collective is small enough for this form, whatever its schedule (bytes: of the call's count).
-bool DirectFits(int coll, uint32_t p, uint64_t bytes);
+bool DirectFits(int coll, uint32_t p, uint64_t bytes, int dtype);
 // The launch of `plan`; false (func == nullptr) where the kernels' records cannot hold it.
 bool BuildDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaunch *d);
 // Puts the ranks' pointers in; true if they were there already (the previous call's).

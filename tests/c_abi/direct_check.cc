@@ -203,7 +203,8 @@ template <uint32_t CAP> bool Fits(const Plan &plan)
 int main(int argc, char **argv)
 {
     const long want = argc > 1 ? std::atol(argv[1]) : 3000;
-    const uint64_t limits[] = {uint64_t(1) << 20, uint64_t(4) << 20, uint64_t(20) << 20};    // results, results to one, traffic
+    // results, results to one destination each, the same of whole vectors, traffic
+    const uint64_t limits[] = {uint64_t(1) << 20, uint64_t(4) << 20, uint64_t(5) << 19, uint64_t(20) << 20};
     long narrow = 0, wide = 0, trees = 0, seconds = 0, stacks = 0, away = 0, large = 0, edges = 0;
     for (long n = 0; n < want;) {
         PlanRequest rq;
@@ -228,8 +229,9 @@ int main(int argc, char **argv)
                 rq.level0Rings = rq.p / s == 8 && Below(2) ? 4 : uint32_t(Below(2));
             }
         }
-        const uint32_t units[] = {1, 2, 4, 8};
-        rq.unit = units[Below(4)];
+        const int dtype = int(Below(12));
+        const uint32_t units[] = {1, 2, 4, 2, 4, 8, 8, 1, 2, 4, 8, 2};
+        rq.unit = units[dtype];
         rq.root = uint32_t(Below(rq.p));
         rq.peer = rq.coll == COLL_SENDRECV && rq.p > 1 ? (rq.root + 1 + uint32_t(Below(rq.p - 1))) % rq.p : 0;
         rq.alias.assign(rq.p, 0);
@@ -240,10 +242,15 @@ int main(int argc, char **argv)
         const uint64_t weight = rq.coll == COLL_ALLGATHER ? uint64_t(rq.p) * (rq.p + 1) : rq.coll == COLL_BROADCAST ? rq.p
             : rq.coll == COLL_SCATTER ? uint64_t(rq.p) * 2 : rq.coll == COLL_SENDRECV ? 2 : rq.coll == COLL_REDUCESCATTER ? rq.p : 1;
         const bool copies = rq.coll == COLL_ALLGATHER || rq.coll == COLL_BROADCAST || rq.coll == COLL_SCATTER || rq.coll == COLL_SENDRECV;
-        const uint64_t limit = copies ? limits[2] : (rq.coll == COLL_ALLREDUCE && rq.p > 1) ? limits[0] : limits[1];
+        const bool toOne = !copies && (rq.coll != COLL_ALLREDUCE || rq.p == 1);
+        uint64_t limit = copies ? limits[3] : toOne ? limits[1 + Below(2)] : limits[0];
         const uint64_t most = limit / weight / rq.unit;
         const bool edge = Below(4) == 0;
         rq.count = edge ? most + Below(2) : 1 + Below(Below(2) ? 500 : most);
+        if (toOne) {
+            const bool wide = dtype != HCCL_DATA_TYPE_INT8 && dtype != HCCL_DATA_TYPE_UINT8 && dtype != HCCL_DATA_TYPE_BFP16;
+            limit = limits[rq.count * rq.unit % 16 == 0 && rq.p > 3 && wide ? 2 : 1];
+        }
         Plan plan;
         std::string err;
         if (BuildPlan(rq, &plan, &err) != 0) {
@@ -251,7 +258,7 @@ int main(int argc, char **argv)
         }
         n++;
         const uint64_t bytes = rq.count * rq.unit;
-        const bool fits = DirectFits(rq.coll, rq.p, bytes);
+        const bool fits = DirectFits(rq.coll, rq.p, bytes, dtype);
         const bool reduceColl = !copies;
         if (plan.fusedOk) {
             uint64_t results = 0, traffic = 0;

@@ -8,7 +8,7 @@ import torch
 
 import closed_forms as cf
 import gpu_harness as gh
-from closed_forms import BF16, FP16, FP32, INT8, INT64, MAX, MIN, PROD, SUM
+from closed_forms import BF16, FP16, FP32, INT8, INT32, INT64, MAX, MIN, PROD, SUM
 
 pytestmark = pytest.mark.gpu
 H = gh.H
@@ -207,5 +207,72 @@ def test_overlapping_buffers_among_in_place_ranks(orc, p):
             assert g.info()["fused"] == (1 if case == "apart" else 0)
             for r in range(p):
                 assert gh.same(dt, gh.to_host(recvs[r], dt), want[r]), (case, r)
+    finally:
+        g.close()
+
+
+@pytest.mark.parametrize("p", [2, 8, 32])
+def test_size_limits(p):
+    # the largest of every collective that goes out this way, and one element more; integers, whose sums have no order
+    mib = 1 << 20
+    g = gh.Group(p)
+    try:
+        for dt in (INT8, INT32, INT64):
+            unit = H.DTYPE_SIZE[dt]
+            kind = {INT8: torch.int8, INT32: torch.int32, INT64: torch.int64}[dt]
+            even = 16 // unit
+            to_one = 4 * mib if p <= 3 or dt == INT8 else 5 * mib // 2
+            cases = [("reduce_scatter", to_one // p // unit // even * even, 1), ("reduce_scatter", to_one // p // unit // even * even + even, 0),
+                     ("reduce_scatter", 4 * mib // p // unit // even * even - 1, 1), ("reduce_scatter", 4 * mib // p // unit // even * even + 1, 0),
+                     ("reduce", to_one // unit, 1), ("reduce", to_one // unit + even, 0), ("reduce", 4 * mib // unit - 1, 1), ("reduce", 4 * mib // unit + 1, 0),
+                     ("all_gather", 20 * mib // p // (p + 1) // unit, 1), ("all_gather", 20 * mib // p // (p + 1) // unit + 1, 0),
+                     ("broadcast", 20 * mib // p // unit, 1), ("broadcast", 20 * mib // p // unit + 1, 0),
+                     ("scatter", 10 * mib // p // unit, 1), ("scatter", 10 * mib // p // unit + 1, 0),
+                     ("send", 10 * mib // unit, 1), ("send", 10 * mib // unit + 1, 0)]
+            for coll, n, direct in cases:
+                if p == 32 and coll == "reduce" and dt != INT32:
+                    continue
+                print("limit", p, coll, "type", dt, "n", n, flush=True)
+                gen = torch.Generator(device="cuda")
+                gen.manual_seed(n)
+                rand = lambda k: torch.randint(-100, 100, (k,), dtype=kind, device="cuda", generator=gen)  # noqa: E731
+                zero = lambda k: torch.zeros(k, dtype=kind, device="cuda")  # noqa: E731
+                ptr = lambda ts: [0 if t is None else t.data_ptr() for t in ts]  # noqa: E731
+                root = p - 1
+                if coll == "reduce_scatter":
+                    s, r = [rand(n * p) for _ in range(p)], [zero(n) for _ in range(p)]
+                    torch.cuda.synchronize()
+                    H.reduce_scatter(g.comms, ptr(s), ptr(r), n, dt, SUM, g.stream_ptr)
+                    want = list(sum(s[1:], s[0].clone()).split(n))
+                elif coll == "reduce":
+                    s, r = [rand(n) for _ in range(p)], [zero(n) for _ in range(p)]
+                    torch.cuda.synchronize()
+                    H.reduce(g.comms, ptr(s), ptr(r), n, dt, SUM, root, g.stream_ptr)
+                    r, want = [r[root]], [sum(s[1:], s[0].clone())]
+                elif coll == "all_gather":
+                    s, r = [rand(n) for _ in range(p)], [zero(n * p) for _ in range(p)]
+                    torch.cuda.synchronize()
+                    H.all_gather(g.comms, ptr(s), ptr(r), n, dt, g.stream_ptr)
+                    want = [torch.cat(s)] * p
+                elif coll == "broadcast":
+                    r = [rand(n) for _ in range(p)]
+                    want = [r[root].clone()] * p
+                    torch.cuda.synchronize()
+                    H.broadcast(g.comms, ptr(r), n, dt, root, g.stream_ptr)
+                elif coll == "scatter":
+                    s, r = [None] * root + [rand(n * p)], [zero(n) for _ in range(p)]
+                    torch.cuda.synchronize()
+                    H.scatter(g.comms, ptr(s), ptr(r), n, dt, root, g.stream_ptr)
+                    want = list(s[root].split(n))
+                else:
+                    s, r = [rand(n)], [zero(n)]
+                    torch.cuda.synchronize()
+                    H.send(g.comms[0], s[0].data_ptr(), n, dt, root, g.stream_ptr)
+                    H.recv(g.comms[root], r[0].data_ptr(), n, dt, 0, g.stream_ptr)
+                    want = s
+                g.stream.synchronize()
+                assert g.info()["direct"] == direct, (coll, n)
+                for a, b in zip(r, want):
+                    assert torch.equal(a, b), (coll, n)
     finally:
         g.close()

@@ -97,7 +97,7 @@ HcclResult EnsureDevice(Group *g, bool quiet)
     // the team kernels park their results in more LDS than a kernel gets without asking
     for (int dt = 0; dt <= 11; dt++) {
         for (int op = 0; op <= 3; op++) {
-            for (KernelKind kind : {KK_TEAM_CHAIN, KK_TEAM_TREE, KK_TEAM_STACK}) {
+            for (KernelKind kind : {KK_TEAM_CHAIN, KK_TEAM_TREE, KK_TEAM_STACK, KK_TEAM_STACK_TILES}) {
                 const void *f = LookupKernel(dt, op, kind);
                 if (f != nullptr) {
                     HIP_OK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, int(kTeamDynamicLds)));
@@ -599,6 +599,19 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                     // the more so since rounds of 8 and 4 whole tiles are read in one piece: with "fewer than 16"
                     // all-gather and broadcast took 2 % longer, the all-reduces 1 %).
                     const uint32_t perX = g->numCu / kTeamXcds;
+                    // Items well short of a region (the pieces of a cut schedule) leave few rounds of one item, and the 8-byte
+                    // types and 8-bit products run up to 4 % slower with those than tile by tile.  Two servers, us, with / without: 8 ranks x 64 MiB
+                    // (a third of the tiles in items of 171) maximum of int64 214.2 / 206.9, product of uint64 213.0 / 204.7, of fp64
+                    // 192.4 / 193.3, of int8 222.9 / 216.4; 16 ranks x 64 MiB (37 tiles) sum of int64 391.9 / 384.1.  From 192 tiles on it evens out, from
+                    // 235 they gain: 8 ranks x 88 MiB maximum of int64 271.3 / 276.4, x 96 MiB sum of int64 264.0 / 282.0.
+                    uint32_t inShort = 0;
+                    for (const FusedDesc &d : descs) {
+                        const uint32_t t = TilesOf(d.bytes);
+                        inShort += t < pl.rec.roundTiles * perX * 3 / 4 ? t : 0u;
+                    }
+                    if (kind == int(KK_STACK) && inShort > tiles / 4) {
+                        pl.rec.func = LookupKernel(dtype, op, KK_TEAM_STACK_TILES);
+                    }
                     std::vector<TeamRegion> regions;
                     uint32_t per = pl.rec.roundTiles;
                     while (per > 1 && uint64_t(per) * perX * kTeamXcds > tiles) {

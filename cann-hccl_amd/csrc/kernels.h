@@ -73,8 +73,9 @@ enum KernelKind : int {
     KK_STEP = 0, KK_CHAIN = 1, KK_TREE = 2, KK_STACK = 3,
     KK_TEAM_CHAIN = 4, KK_TEAM_TREE = 5, KK_TEAM_STACK = 6,   // team forms of the fused kernels, see below
     KK_DIRECT = 7, KK_DIRECT_WIDE = 8,                         // small collectives, see below
-    KK_COUNT = 9,
-    KK_GATHER = 9                                              // copy kernel table only
+    KK_TEAM_STACK_TILES = 9,                                   // the team's stack kernel without its rounds read source by source
+    KK_COUNT = 10,
+    KK_GATHER = 10                                             // copy kernel table only
 };
 
 // Team form of a fused kernel: the workgroups of one XCD read their tiles together, park the results in LDS, and write

@@ -70,9 +70,10 @@ extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[6] = {
         reinterpret_cast<const void *>(&StackKernel<DT, OP>),            \
         reinterpret_cast<const void *>(&TeamChainKernel<DT, OP>),        \
         reinterpret_cast<const void *>(&TeamTreeKernel<DT, OP>),         \
-        reinterpret_cast<const void *>(&TeamStackKernel<DT, OP>),        \
+        reinterpret_cast<const void *>(&TeamStackKernel<DT, OP, true>),  \
         reinterpret_cast<const void *>(&DirectKernel<DT, OP, 8>),        \
         reinterpret_cast<const void *>(&DirectKernel<DT, OP, 32>),       \
+        reinterpret_cast<const void *>(&TeamStackKernel<DT, OP, sizeof(DT) != 8 && (sizeof(DT) != 1 || OP != ROP_PROD)>),   \
     }
 extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[4][KK_COUNT] = {
     HCCL_ROW(ROP_SUM), HCCL_ROW(ROP_PROD), HCCL_ROW(ROP_MAX), HCCL_ROW(ROP_MIN),

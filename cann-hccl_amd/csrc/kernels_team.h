@@ -528,15 +528,18 @@ template <typename T, int OP> struct TeamTreeEval {
 };
 
 // extra = the launch's op words (they follow the item table)
-template <typename T, int OP> struct TeamStackEval {
-    static constexpr bool kBySource = ReadsBySource<T>::value;
+template <typename T, int OP, bool ROUNDS> struct TeamStackEval {
+    static constexpr bool kBySource = ROUNDS && ReadsBySource<T>::value;
     // A whole round source by source, as the chain's (TeamChainEval::Round), for expressions that never hold more than
     // two partial results while a source is being read (a chain of chains: the two-level all-reduce): the lower one in
     // LDS, the upper one in registers.  Three sets of eight tiles are more registers than a wave has, so the round goes
     // in halves of four tiles, through one pipeline: the second half's first sources are requested while the first
     // half's last ones are folded.  Measured (8 ranks, fp32 sum, us, tile by tile / this way): two servers of four, 64 MiB
     // per rank 198.0 / 180.8 (5.4 / 5.9 TB/s), 256 MiB 745 - 755 / 721; the 8-rank ring's chain of 64 MiB takes 176.  What
-    // bounds it now is what bounds the chain, the write phase.
+    // bounds it now is what bounds the chain, the write phase.  Without the piece cut all types but bf16 gain, 64 MiB: fp16
+    // 200.6 / 183.7, int8 209.5 / 186.8, int32 199.9 / 183.9, uint64 197.4 / 177.6, fp64 194.0 / 177.4, maximum of fp32 226.4 / 191.9.
+    // Its registers cost the tiles that are not read this way: 8-byte types and 8-bit products have a kernel without it
+    // (ROUNDS) for launches with few such rounds (exec.cc).
     static __device__ __forceinline__ bool RoundFits(const FusedDesc &d) { return d.nsrc >= 2 && d.nleaf <= 3; }
     static constexpr uint32_t kHalf = kTeamTiles / 2;
     typedef V4 Set[kHalf][kVecPerLane];
@@ -689,12 +692,12 @@ __global__ void __launch_bounds__(kBlockThreads) TeamTreeKernel(const FusedDesc 
     TeamBody<TeamTreeEval<T, OP>>(items, nitems, ntiles, srcPool, dstPool, tilesPerItem, teamCtr, nullptr);
 }
 
-template <typename T, int OP>
+template <typename T, int OP, bool ROUNDS>
 __global__ void __launch_bounds__(kBlockThreads) TeamStackKernel(const FusedDesc *__restrict__ items, uint32_t nitems,
     uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem,
     uint32_t *__restrict__ teamCtr)
 {
-    TeamBody<TeamStackEval<T, OP>>(items, nitems, ntiles, srcPool, dstPool, tilesPerItem, teamCtr, items + nitems);
+    TeamBody<TeamStackEval<T, OP, ROUNDS>>(items, nitems, ntiles, srcPool, dstPool, tilesPerItem, teamCtr, items + nitems);
 }
 
 }  // namespace hcclamd

@@ -5,7 +5,7 @@ import pytest
 
 import closed_forms as cf
 import gpu_harness as gh
-from closed_forms import BF16, FP16, FP32, INT8, INT64, MAX, MIN, PROD, SUM
+from closed_forms import BF16, FP16, FP32, FP64, INT8, INT64, MAX, MIN, PROD, SUM
 
 pytestmark = pytest.mark.gpu
 H = gh.H
@@ -40,6 +40,30 @@ def test_team_stack_whole_rounds(orc, dt, op, p, servers, special, extra):
                     assert np.array_equal(outs[r].view(np.uint32), want[r].view(np.uint32)), r
                 else:
                     assert gh.same(dt, outs[r], want[r]), r
+    finally:
+        g.close()
+
+
+# 8-byte elements and 8-bit products: where more than a quarter of the tiles lie in items shorter than three quarters of a region (8 tiles for each
+# of an XCD's 32 compute units) all are read tile by tile, else whole rounds source by source.  A slice goes in a third and two thirds.
+@pytest.mark.parametrize("dt,op", [(INT64, SUM), (FP64, MAX), (INT8, PROD)])
+@pytest.mark.parametrize("tiles,extra", [(95, 0), (191, 0), (192, 8), (257, 24)])
+def test_team_stack_of_short_and_long_items(orc, dt, op, tiles, extra):
+    p, servers = 8, 2
+    n = p * 3 * (tiles * 16384 + extra) // H.DTYPE_SIZE[dt]
+    plan = H.describe_plan(H.COLL_ALLREDUCE, RING | servers << 8, p, n, dt)
+    assert {it["kind"] for it in plan["fused"]} == {3}
+    print("team stack, short and long items", dt, op, tiles, extra, "items of", sorted({it["n"] for it in plan["fused"]}), flush=True)
+    rng = np.random.default_rng(9700 + tiles + dt)
+    ins = [cf.random_input(dt, n, rng) for _ in range(p)]
+    want = orc.allreduce_two_level([x.copy() for x in ins], dt, op, servers, level1=RING)
+    g = gh.Group(p, algo="ring", servers=servers, deterministic=1, team=1)
+    try:
+        for rep in range(2):
+            outs, _ = gh.all_reduce(g, ins, dt, op)
+            assert g.info()["teamLaunches"] >= 1
+            for r in range(p):
+                assert gh.same(dt, outs[r], want[r]), r
     finally:
         g.close()
 

@@ -22,11 +22,13 @@ def orc():
 # two and four servers, rounds of 8 and of 4 tiles, slices with a ragged end; max and min over NaNs and signed zeros, where a swapped operand changes the bits
 @pytest.mark.parametrize("dt,op,p,servers,special,extra", [
     (FP32, MAX, 8, 2, True, 0), (FP32, MIN, 8, 4, True, 0), (FP32, SUM, 8, 2, False, 4099), (FP16, SUM, 8, 4, False, 0), (INT8, SUM, 8, 2, False, 0),
-    (INT64, PROD, 6, 2, False, 0), (FP32, SUM, 6, 3, False, 0), (BF16, SUM, 8, 2, False, 0)])
+    (INT64, PROD, 9, 3, False, 0), (FP32, SUM, 10, 5, False, 0), (BF16, SUM, 8, 2, False, 0)])
 def test_team_stack_whole_rounds(orc, dt, op, p, servers, special, extra):
     n = (p * (4 << 20) + extra) // H.DTYPE_SIZE[dt]
     rng = np.random.default_rng(9400 + dt + servers)
     pool = np.array([0.0, -0.0, np.inf, -np.inf, np.nan, 1e-45, -1.0, 3.4e38], np.float32)
+    plan = H.describe_plan(H.COLL_ALLREDUCE, RING | servers << 8, p, n, dt)
+    assert {it["kind"] for it in plan["fused"]} == {3}
     print("team stack", dt, op, p, servers, special, extra, flush=True)
     ins = [rng.choice(pool, n).astype(np.float32) if special else cf.random_input(dt, n, rng) for _ in range(p)]
     want = orc.allreduce_two_level([x.copy() for x in ins], dt, op, servers, level1=RING)

@@ -299,7 +299,9 @@ template <uint32_t MODE> __device__ __forceinline__ V4 Load16(const void *base, 
 }
 // 16 bytes at any address, fetched as whole words: the four words from the word boundary in front on, and the word that
 // holds the last bytes (for an address on a word boundary the fourth word again, so that nothing outside the words of
-// the 16 bytes is touched).  Vector(shift) puts them together, shift = address mod 4.
+// the 16 bytes is touched; the words at a block's ends hold up to three bytes before and behind it, which may lie outside the
+// caller's buffer: they are read with their word, never past it, and dropped).  Vector(shift) puts them together, shift =
+// address mod 4.
 // For 8-bit elements: a 128-bit load off a word boundary costs the vector memory unit more than the extra word does.
 // Reduce-scatter, int8, blocks of odd length, us, 128-bit loads / this way: 8 ranks x 3 000 017 sum 44.2 / 42.1 (blocks at
 // multiples of 64 bytes: 39.9), x 12 000 017 168.0 / 157.5; 16 ranks x 700 001 sum 47.1 / 43.1, max 55.6 / 47.2.  16-bit

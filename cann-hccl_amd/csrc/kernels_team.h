@@ -300,31 +300,22 @@ template <typename T> struct ReadsBySource { static constexpr bool value = true;
 template <> struct ReadsBySource<Bf16Bits> { static constexpr bool value = false; };
 
 // One register set: N whole tiles of one source, `stride` bytes apart.
-    template <uint32_t N>
-    __device__ __forceinline__ void TeamLoadSet(V4 (&v)[N][kVecPerLane], const void *base, uint64_t off, uint64_t stride)
-    {
-        const char *s = static_cast<const char *>(base) + off;
+template <uint32_t N>
+__device__ __forceinline__ void TeamLoadSet(V4 (&v)[N][kVecPerLane], const void *base, uint64_t off, uint64_t stride)
+{
+    const char *s = static_cast<const char *>(base) + off;
 #pragma unroll
-        for (uint32_t q = 0; q < N; q++) {
+    for (uint32_t q = 0; q < N; q++) {
 #pragma unroll
-            for (uint32_t u = 0; u < kVecPerLane; u++) {
-                v[q][u] = Load16<ACC_VEC16>(s + q * stride + uint64_t(u) * kBlockThreads * 16, threadIdx.x * 16u);
-            }
+        for (uint32_t u = 0; u < kVecPerLane; u++) {
+            v[q][u] = Load16<ACC_VEC16>(s + q * stride + uint64_t(u) * kBlockThreads * 16, threadIdx.x * 16u);
         }
     }
+}
 
 template <typename T, int OP> struct TeamChainEval {
     static constexpr bool kBySource = ReadsBySource<T>::value;
     static __device__ __forceinline__ bool RoundFits(const FusedDesc &d) { return d.nsrc >= 2; }
-    // A whole round at once: N whole tiles of one item, `stride` bytes apart from `off` on.  The team reads source by
-    // source -- at any moment its loads go to one stretch of N x 32 tiles of one buffer instead of 32 tiles of each of
-    // the item's buffers -- and the partial results rest in LDS, folded in the chain's order, so the bits are those of
-    // the tile-by-tile evaluation.  Two register sets of N x 4 vectors: while one source is folded, the next one's
-    // loads are in flight, and the one after that is requested as soon as the fold has freed its set (8 ranks x
-    // 256 MiB, stand-alone: 691 us this way, 770 us with one set, 705 us tile by tile).
-    // Straight-line code for a source count fixed at compile time, in which every wait is for exactly the loads it
-    // needs, measured the same and takes three times as long to build.
-    // `peek` is looked at (thread 0, into *seen) once the last loads are on their way.
     // Source j into the partial results: source 0 starts them.  A tile's partial results are fetched from LDS together,
     // so that their latencies overlap.
     template <uint32_t N>
@@ -366,6 +357,15 @@ template <typename T, int OP> struct TeamChainEval {
             }
         }
     }
+    // A whole round at once: N whole tiles of one item, `stride` bytes apart from `off` on.  The team reads source by
+    // source -- at any moment its loads go to one stretch of N x 32 tiles of one buffer instead of 32 tiles of each of
+    // the item's buffers -- and the partial results rest in LDS, folded in the chain's order, so the bits are those of
+    // the tile-by-tile evaluation.  Two register sets of N x 4 vectors: while one source is folded, the next one's
+    // loads are in flight, and the one after that is requested as soon as the fold has freed its set (8 ranks x
+    // 256 MiB, stand-alone: 691 us this way, 770 us with one set, 705 us tile by tile).
+    // Straight-line code for a source count fixed at compile time, in which every wait is for exactly the loads it
+    // needs, measured the same and takes three times as long to build.
+    // `peek` is looked at (thread 0, into *seen) once the last loads are on their way.
     template <uint32_t N>
     static __device__ __forceinline__ void Round(const FusedDesc &d, const void *const *__restrict__ src, const void *, uint64_t off,
         uint64_t stride, LdsV4 *park, const uint32_t *peek, uint32_t *seen)

@@ -57,9 +57,9 @@ extern "C" {
  *                                or more destinations with more than 512 MB of output (all-gather, broadcast)
  *   "team"          "auto" | "0" | "1"   team form of the fused kernels: the workgroups of one XCD read their tiles together,
  *                                hold the results in LDS and write them together, which this memory system serves faster
- *                                than reads and writes interleaved; "auto" (default): for launches of at least four rounds
- *                                whose items write four or more destinations and touch eight or more buffers (all-reduce,
- *                                all-gather, broadcast); "1": wherever the device allows it; "0": never
+ *                                than reads and writes interleaved; "auto" (default): for launches of at least two full
+ *                                rounds, one where data is only moved, whose items write four or more destinations and touch
+ *                                eight or more buffers (all-reduce, all-gather, broadcast); "1": wherever the device allows it; "0": never
  *   "team_tiles"    tiles of 16 KiB a workgroup of a team kernel takes per round, 1 ... 8 ("0", default: 8, fewer when an
  *                                item has more than 8 sources or destinations)
  *   "direct"        "auto" | "0"   small collectives go out as one launch whose descriptors ride in its arguments ("auto",

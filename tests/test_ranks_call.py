@@ -139,3 +139,34 @@ def test_the_library_called_is_the_one_loaded(tmp_path):
     subprocess.run(["g++", "-shared", "-fPIC", str(src), "-o", str(stub / "libhccl.so")], check=True)
     path = str(stub) + os.pathsep + os.environ.get("LD_LIBRARY_PATH", "")
     assert _start(tmp_path, True, {"LD_LIBRARY_PATH": path}) == "code %d native 1" % H.HCCL_E_PTR
+
+
+# ---- which calls the native loop takes ------------------------------------------------------------------------------
+
+def test_what_the_native_loop_recognises(comms):
+    a = [0x100000 * (r + 1) for r in range(P)]
+    none = [None] * P
+    dt = H.HCCL_DATA_TYPE_FP32
+
+    def call(comms, sends, recvs, kind=H._ALL_REDUCE, count=8, stream=1, tables=None):
+        return H._call(kind, comms, sends, recvs, count, dt, 0, 0, stream, tables)
+
+    # (null send buffers: the first rank's call fails, so that nothing is left waiting)
+    for same in (list, tuple):
+        for recvs in (a, [ctypes.c_void_p(v) for v in a]):
+            assert call(same(comms), same(none), same(recvs)) == H.HCCL_E_PTR
+    assert call(comms, none, a, stream=ctypes.c_void_p(1)) == H.HCCL_E_PTR
+    for form in (iter, np.array, lambda x: dict(enumerate(x)), lambda x: [np.uint64(v) for v in x], lambda x: [ctypes.c_uint64(v) for v in x],
+                 lambda x: [float(v) for v in x]):
+        assert call(comms, none, form(a)) == -1, form
+    assert call(comms, none, a, count=8.0) == -1 and call(comms, none, a, stream="1") == -1
+    assert call([comms[0]] * 65, [None] * 65, [1] * 65) == -1
+
+    cnt = np.ones((P, P), np.uint64)
+    for good in (cnt, np.ascontiguousarray(cnt.T)):
+        assert call(comms, none, a, kind=H._ALL_TO_ALL_V, tables=[good] * 4) in (H.HCCL_E_PTR, H.HCCL_E_PARA)
+    for bad in (cnt.astype(np.int64), cnt.astype(np.uint32), cnt.astype(">u8"), np.ones((P, 2 * P), np.uint64)[:, ::2], np.ones((P, P + 1), np.uint64),
+                np.ones(P * P, np.uint64), cnt.tolist(), None):
+        assert call(comms, none, a, kind=H._ALL_TO_ALL_V, tables=(cnt, cnt, bad, cnt)) == -1, bad
+    assert call(comms, none, a, kind=H._ALL_TO_ALL_V, tables=(cnt, cnt, cnt)) == -1
+    assert call(comms, none, a, kind=H._ALL_TO_ALL_V) == -1

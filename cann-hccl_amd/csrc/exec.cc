@@ -173,34 +173,32 @@ struct Builder {
 
 // Cuts [0, bytes) into an element-wise head, a 16-byte vector body and an element-wise tail, given
 // the addresses involved (the first one is a destination; all are multiples of the element size).
-// The head brings the first destination to a 16-byte boundary; pointers that are then not on one
-// too are accessed with unaligned 128-bit loads and stores (ACC_VEC16_ANY).  emit(offset, bytes, mode).
-// A long body is cut once more so that its main part starts on a 128-byte boundary of the destination:
+// The head brings most of the pointers to a 16-byte boundary (of two equal groups the one with the first destination);
+// those that are then not on one too are accessed with unaligned 128-bit loads and stores (ACC_VEC16_ANY): a reduce-scatter
+// of odd blocks reads all its sources aligned and writes its one destination unaligned.  emit(offset, bytes, mode).
+// The head of a long stretch reaches to a 128-byte boundary of those pointers:
 // a wave stores 1 KiB at a time, and when those stores straddle memory lines every line is written in
 // two pieces (measured, 8-rank fp32 all-reduce of 256 MiB per rank with all buffers 16 bytes off a
 // 128-byte boundary: 0.97 ms fused against 0.76 ms aligned).
 template <typename F> void SplitByAlignment(const std::vector<uintptr_t> &addrs, uint64_t bytes, F emit)
 {
-    uintptr_t anchor = addrs[0];
-    bool co = true;
+    size_t count[16] = {0};
     for (uintptr_t a : addrs) {
-        co = co && ((a & 15) == (anchor & 15));
+        count[a & 15]++;
     }
-    uint64_t head = std::min<uint64_t>(bytes, (16 - (anchor & 15)) & 15);
-    uint64_t body = (bytes - head) & ~uint64_t(15);
-    uint64_t tail = bytes - head - body;
+    uintptr_t anchor = addrs[0];
+    for (uintptr_t a : addrs) {
+        anchor = count[a & 15] > count[anchor & 15] ? a : anchor;
+    }
+    const uint64_t align = bytes >= 4 * uint64_t(kTileBytes) + 128 ? 128 : 16;
+    const uint64_t head = std::min<uint64_t>(bytes, (align - (anchor & (align - 1))) & (align - 1));
+    const uint64_t body = (bytes - head) & ~uint64_t(15);
+    const uint64_t tail = bytes - head - body;
     if (head) {
         emit(uint64_t(0), head, uint32_t(ACC_ELEM));
     }
     if (body) {
-        const uint32_t mode = co ? ACC_VEC16 : ACC_VEC16_ANY;
-        const uint64_t lead = (128 - ((anchor + head) & 127)) & 127;     // a multiple of 16
-        if (lead != 0 && body >= 4 * uint64_t(kTileBytes)) {
-            emit(head, lead, mode);
-            emit(head + lead, body - lead, mode);
-        } else {
-            emit(head, body, mode);
-        }
+        emit(head, body, uint32_t(count[anchor & 15] == addrs.size() ? ACC_VEC16 : ACC_VEC16_ANY));
     }
     if (tail) {
         emit(head + body, tail, uint32_t(ACC_ELEM));
@@ -208,14 +206,58 @@ template <typename F> void SplitByAlignment(const std::vector<uintptr_t> &addrs,
 }
 
 constexpr size_t kGraphMinLaunches = 12;   // fewer launches go out one by one
-constexpr uint32_t kTeamMinRounds = 2;     // the team kernels are chosen for launches of at least this many full rounds
-// The same for one source and many destinations.  8-rank all-gather, us, plain / team: blocks of 3 MiB (1536 tiles, less
-// than a round) 46.3 / 52.4, 4 MiB (2048) 63.4 / 58.9, 5 MiB 80.1 / 73.1, 6 MiB 92.8 / 85.8, 7.5 MiB 121.9 / 105.5; 16 ranks
-// 1.5 MiB (1536) 88.2 / 91.7, 2 MiB 116.2 / 111.5, 3 MiB 174.6 / 162.8.
-constexpr uint32_t kTeamMinRoundsCopy = 1;
+// The team kernels are chosen for launches of at least this many halves of a round.  All-reduce, us, plain / team: 8 ranks,
+// fp32, 12 MiB (768 tiles) 36.0 / 36.6, 16 MiB (1024, half a round) 49.5 / 46.2, 24 MiB 72.4 / 68.2, 32 MiB 96.3 / 88.0, 48 MiB 145.4 /
+// 137.3; 32 ranks, bf16 halving-doubling (a round is 1024 tiles), 4 MiB (256) 45.3 / 46.6, 8 MiB (512) 95.1 / 87.8, 16 MiB 209 / 172.5.
+constexpr uint32_t kTeamMinHalfRounds = 1;
+// Items with fewer than 12 sources and destinations (4 ranks, fp32): 16 MiB 24.3 / 26.1, 32 MiB (a round) 48.0 / 47.4, 48 MiB 70.5 / 74.8,
+// 64 MiB 93.6 / 95.1, 128 MiB (4 rounds) 188.5 / 183.3.
+constexpr uint32_t kTeamMinHalfRoundsFew = 8;
+// One source and many destinations: 8-rank all-gather, blocks of 2 MiB (1024 tiles) 25.9 / 30.0, 4 MiB (2048, a round) 60.0 / 54.2,
+// 8 MiB 122.9 / 105.4; 16 ranks 1 MiB (1024) 54.8 / 53.4, 2 MiB 121.2 / 100.9.
+constexpr uint32_t kTeamMinHalfRoundsCopy = 2;
 constexpr size_t kAsyncUploadBytes = 4 * kNoAllocUploadBytes;   // tables up to this size are uploaded by launches
 
 uint32_t TilesOf(uint64_t bytes) { return uint32_t((bytes + kTileBytes - 1) / kTileBytes); }
+
+// The regions the teams of a launch draw (kernels_team.h): roundTiles tiles per workgroup; over the last quarter of the
+// tiles the size is halved whenever fewer than 8 regions of the current size are left.  The XCDs do not all move data at
+// the same rate, and with regions that get smaller towards the end they finish together (measured, 8 x 256 MiB fp32
+// all-reduce: 727 us with 64 equal regions dealt out in order, 714 us with the shrinking tail
+// drawn from the counter; shrinking earlier costs more than it brings, small regions run slower --
+// the more so since rounds of many whole tiles are read in one piece: with "fewer than 16"
+// all-gather and broadcast took 2 % longer, the all-reduces 1 %).
+// Less than two rounds: a full one and what is left dealt out evenly, or one round of what there is.  All-reduce of 8 ranks, fp32,
+// us, this way / two equal rounds / the rule above: 40 MiB 113.5 / 118.6 / 111.7, 48 MiB 136.6 / 140.2 / 147.4, 56 MiB 161.9 / 161.8 / 158.4;
+// all-gather 8 x 6 MiB 80.7 / - / 92.0.
+std::vector<TeamRegion> TeamRegions(uint32_t tiles, uint32_t ntiles, uint32_t roundTiles, uint32_t perTeam)
+{
+    std::vector<TeamRegion> regions;
+    const uint32_t round = roundTiles * perTeam * kTeamXcds;
+    uint32_t per = roundTiles;
+    for (uint32_t at = 0; at < tiles;) {
+        const uint32_t left = tiles - at;
+        if (ntiles < 2 * round) {
+            const uint32_t teamsLeft = kTeamXcds - uint32_t(regions.size()) % kTeamXcds;
+            const uint32_t n = std::min(roundTiles * perTeam, (left + teamsLeft - 1) / teamsLeft);
+            regions.push_back(TeamRegion{at, n});
+            at += n;
+            continue;
+        }
+        if (uint64_t(at) * 4 >= uint64_t(tiles) * 3) {
+            while (per > 1 && uint64_t(per) * perTeam * 8 > left) {
+                per /= 2;
+            }
+        }
+        const uint32_t n = std::min(left, per * perTeam);
+        regions.push_back(TeamRegion{at, n});
+        at += n;
+    }
+    while (regions.size() < kTeamXcds) {
+        regions.push_back(TeamRegion{tiles, 0});     // every team has a round (the items behind the whole tiles are handled there)
+    }
+    return regions;
+}
 
 struct PendingLaunch {
     LaunchRec rec;
@@ -449,19 +491,7 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
         // write-back stores.  Measured, 8-rank fp32 all-reduce replayed on the same buffers: write-back is
         // 5 % and 12 % faster at 16 and 32 MiB per rank (the output then stays in the 256 MB memory-side
         // cache), 20 % slower at 4 MiB and 7 % slower from 64 MiB per rank up.
-        // Pure data movement with one source and many destinations (all-gather, broadcast) is 4 - 5 % faster with
-        // write-back stores once the output is far larger than the memory-side cache (8 ranks: all-gather to
-        // 256 MiB per rank 473 us against 501 us, broadcast of 256 MiB 425 us against 447 us); one-to-one copies
-        // are not (uniform all-to-all 773 us against 752 us).
-        bool fusedOrdinary = g->cfg.fusedStores == 1;
-        if (g->cfg.fusedStores < 0 && !reduceColl) {
-            double written = 0, read = 0;
-            for (const FusedItem &it : pp->plan->fused) {
-                written += double(it.dst.size()) * double(it.bytes);
-                read += double(it.bytes);
-            }
-            fusedOrdinary = written >= 4.0 * read && written >= 2.0 * double(kMemorySideCacheBytes);
-        }
+        const bool fusedOrdinary = g->cfg.fusedStores == 1;
         // Pure data movement in many short segments (an all-to-all-v of a few hundred bytes per pair): those go to
         // the gather kernel, a wave per segment through LDS, instead of a tile, a table search and up to three
         // descriptors each (measured, 64 ranks, 4096 segments of 430 bytes on average: 32 us with the tile kernel).
@@ -515,44 +545,36 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
         // one launch per kernel kind present, or several under a launch cap: the items in their order, cut where the
         // bytes a launch moves (read and written) reach the cap
         for (int kind : {int(KK_CHAIN), int(KK_TREE), int(KK_STACK)}) {
-            std::vector<FusedDesc> descs;
+            std::vector<FusedDesc> descs;      // whole tiles
+            std::vector<FusedDesc> rests;      // what is left of a stretch behind them, and its element-wise ends: a tile each
             std::vector<const void *> srcPool;
             std::vector<uint32_t> opPool;      // stack items: one word per source-pool entry
             std::vector<void *> dstPool;
             uint32_t tiles = 0;
-            uint64_t traffic = 0;
+            uint64_t traffic = 0, written = 0;
             std::vector<char *> srcs, dsts;        // reused from item to item: an all-to-all-v has thousands
             std::vector<uintptr_t> addrs;
             const void *func = reduceColl ? LookupKernel(dtype, op, KernelKind(kind)) : LookupCopyKernel(KernelKind(kind));
             auto flush = [&]() {
-                if (descs.empty()) {
+                if (descs.empty() && rests.empty()) {
                     return;
                 }
                 PendingLaunch pl;
-                // the op words of the stack kernel sit right behind its item table
-                pl.tableAt = b.Reserve(descs.size() * sizeof(FusedDesc) + opPool.size() * sizeof(uint32_t));
-                std::memcpy(b.host.data() + pl.tableAt, descs.data(), descs.size() * sizeof(FusedDesc));
-                if (!opPool.empty()) {
-                    std::memcpy(b.host.data() + pl.tableAt + descs.size() * sizeof(FusedDesc), opPool.data(),
-                        opPool.size() * sizeof(uint32_t));
-                }
-                pl.srcAt = b.Reserve(srcPool.size() * sizeof(void *));
-                std::memcpy(b.host.data() + pl.srcAt, srcPool.data(), srcPool.size() * sizeof(void *));
-                pl.dstAt = b.Reserve(dstPool.size() * sizeof(void *));
-                std::memcpy(b.host.data() + pl.dstAt, dstPool.data(), dstPool.size() * sizeof(void *));
                 pl.rec.func = func;
                 pl.rec.nitems = uint32_t(descs.size());
-                pl.rec.ntiles = tiles;
+                pl.rec.nwhole = tiles;
+                pl.rec.ntiles = tiles + uint32_t(rests.size());
                 // equal slices (the usual collective): the kernels find a tile's item without searching the table
-                pl.rec.tilesPerItem = TilesOf(descs[0].bytes);
+                pl.rec.tilesPerItem = descs.empty() ? 0 : TilesOf(descs[0].bytes);
+                bool alike = !descs.empty() && kind == int(KK_CHAIN) && descs[0].nsrc >= 2;
                 for (size_t i = 0; i < descs.size(); i++) {
                     const uint32_t t = TilesOf(descs[i].bytes);
                     if (i + 1 < descs.size() ? t != pl.rec.tilesPerItem : t > pl.rec.tilesPerItem) {
                         pl.rec.tilesPerItem = 0;
-                        break;
                     }
+                    alike = alike && descs[i].nsrc == descs[0].nsrc;
                 }
-                pl.rec.grid = std::min(tiles, kind == int(KK_TREE) ? treeGrid : fusedGrid);
+                pl.rec.grid = std::min(pl.rec.ntiles, kind == int(KK_TREE) ? treeGrid : fusedGrid);
                 pl.rec.fusedArgs = true;
                 // Team form (kernels_team.h): pays when every workgroup has much to read or to write per tile and the
                 // launch runs for many rounds.  Measured on MI355X with streams of 256 MiB (sources : destinations,
@@ -581,8 +603,9 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                     pl.rec.roundTiles = g->cfg.teamTiles != 0 ? std::min(g->cfg.teamTiles, kTeamTiles)
                                                               : std::max(1u, std::min(kTeamTiles, uint32_t(128.0 / std::max(1.0, widest))));
                     if (g->cfg.team < 0) {
+                        const uint32_t halfRounds = !reduceColl ? kTeamMinHalfRoundsCopy : (allStreams < 12.0 * bytes ? kTeamMinHalfRoundsFew : kTeamMinHalfRounds);
                         team = bytes > 0 && storeStreams >= 4.0 * bytes && allStreams >= 8.0 * bytes &&
-                            tiles >= (reduceColl ? kTeamMinRounds : kTeamMinRoundsCopy) * pl.rec.roundTiles * g->numCu;
+                            2 * pl.rec.ntiles >= halfRounds * pl.rec.roundTiles * g->numCu;
                     }
                 }
                 if (team) {
@@ -590,14 +613,6 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                     pl.rec.team = true;
                     pl.rec.grid = g->numCu;
                     pl.rec.dynamicLds = kTeamDynamicLds;
-                    // The regions the teams draw: roundTiles tiles per workgroup (fewer when that would leave an XCD
-                    // without a region); over the last quarter of the tiles the size is halved whenever fewer than 8
-                    // regions of the current size are left.  The XCDs do not all move data at the same rate, and with
-                    // regions that get smaller towards the end they finish together (measured, 8 x 256 MiB fp32
-                    // all-reduce: 727 us with 64 equal regions dealt out in order, 714 us with the shrinking tail
-                    // drawn from the counter; shrinking earlier costs more than it brings, small regions run slower --
-                    // the more so since rounds of 8 and 4 whole tiles are read in one piece: with "fewer than 16"
-                    // all-gather and broadcast took 2 % longer, the all-reduces 1 %).
                     const uint32_t perX = g->numCu / kTeamXcds;
                     // Items well short of a region (the pieces of a cut schedule) leave few rounds of one item, and the 8-byte
                     // types and 8-bit products run up to 4 % slower with those than tile by tile.  Two servers, us, with / without: 8 ranks x 64 MiB
@@ -612,40 +627,47 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                     if (kind == int(KK_STACK) && inShort > tiles / 4) {
                         pl.rec.func = LookupKernel(dtype, op, KK_TEAM_STACK_TILES);
                     }
-                    std::vector<TeamRegion> regions;
-                    uint32_t per = pl.rec.roundTiles;
-                    while (per > 1 && uint64_t(per) * perX * kTeamXcds > tiles) {
-                        per /= 2;
-                    }
-                    for (uint32_t at = 0; at < tiles;) {
-                        const uint32_t left = tiles - at;
-                        if (tiles < 2 * pl.rec.roundTiles * g->numCu) {
-                            // Less than two full rounds: every team gets as much as the others in each, and the
-                            // odd tiles come last (all-gather of 8 x 6 MiB: 85.8 us, with the rule below 100.9).
-                            if (regions.size() % kTeamXcds == 0) {
-                                per = std::max(1u, std::min(per, left / g->numCu));
-                            }
-                        } else if (uint64_t(at) * 4 >= uint64_t(tiles) * 3) {
-                            while (per > 1 && uint64_t(per) * perX * 8 > left) {
-                                per /= 2;
-                            }
-                        }
-                        regions.push_back(TeamRegion{at, per});
-                        at += uint32_t(std::min<uint64_t>(left, uint64_t(per) * perX));
-                    }
+                    const std::vector<TeamRegion> regions = TeamRegions(tiles, pl.rec.ntiles, pl.rec.roundTiles, perX);
                     const uint32_t n = uint32_t(regions.size());
                     pl.ctrAt = b.Reserve(size_t(TeamBlockWords(n)) * 4);     // zero in the image, and zero again after every launch
                     uint32_t *block = reinterpret_cast<uint32_t *>(b.host.data() + pl.ctrAt);
                     block[kTeamRegionCount] = n;
                     std::memcpy(block + kTeamHeaderWords, regions.data(), regions.size() * sizeof(TeamRegion));
                 }
+                // Many sources into one destination, plain: the kernel that asks for less at a time, and stores written
+                // through (StorePolicy, kernels_impl.h).
+                const bool toOne = reduceColl && !team && written * 3 <= traffic;
+                const bool through = toOne && !fusedOrdinary && g->cfg.fusedStores < 0 && traffic <= 2 * kMemorySideCacheBytes;
+                if (toOne && kind == int(KK_CHAIN)) {
+                    pl.rec.func = LookupKernel(dtype, op, KK_CHAIN_SLOW);
+                }
+                const uint32_t flags = (fusedOrdinary ? kFusedOrdinaryStores : 0u) | (through ? kFusedThroughStores : 0u) | (alike ? kFusedAlike : 0u);
+                // the op words of the stack kernel sit right behind its item table
+                pl.tableAt = b.Reserve((descs.size() + rests.size()) * sizeof(FusedDesc) + opPool.size() * sizeof(uint32_t));
+                FusedDesc *table = reinterpret_cast<FusedDesc *>(b.host.data() + pl.tableAt);
+                for (size_t i = 0; i < rests.size(); i++) {
+                    rests[i].tile0 = tiles + uint32_t(i);
+                }
+                descs.insert(descs.end(), rests.begin(), rests.end());
+                for (FusedDesc &d : descs) {
+                    d.flags |= flags;
+                }
+                std::memcpy(table, descs.data(), descs.size() * sizeof(FusedDesc));
+                if (!opPool.empty()) {
+                    std::memcpy(table + descs.size(), opPool.data(), opPool.size() * sizeof(uint32_t));
+                }
+                pl.srcAt = b.Reserve((srcPool.size() + kPoolPad) * sizeof(void *));
+                std::memcpy(b.host.data() + pl.srcAt, srcPool.data(), srcPool.size() * sizeof(void *));
+                pl.dstAt = b.Reserve((dstPool.size() + kPoolPad) * sizeof(void *));
+                std::memcpy(b.host.data() + pl.dstAt, dstPool.data(), dstPool.size() * sizeof(void *));
                 pending.push_back(pl);
                 descs.clear();
+                rests.clear();
                 srcPool.clear();
                 opPool.clear();
                 dstPool.clear();
                 tiles = 0;
-                traffic = 0;
+                traffic = written = 0;
             };
             for (const FusedItem &it : pp->plan->fused) {
                 int want = it.kind == FK_TREE ? int(KK_TREE) : (it.kind == FK_STACK ? int(KK_STACK) : int(KK_CHAIN));
@@ -686,33 +708,48 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                 // an item that alone exceeds the cap goes in pieces of whole tiles
                 const uint64_t piece = capBytes == 0 ? ~uint64_t(0)
                                                      : std::max<uint64_t>(kTileBytes, capBytes / streams / kTileBytes * kTileBytes);
+                uint32_t flags = 0;
+                for (size_t k = 0; k < srcs.size(); k++) {
+                    flags |= kind == int(KK_TREE) && (k & 1u) != 0 && srcs[k] != nullptr ? kFusedPairs : 0u;
+                }
+                auto add = [&](std::vector<FusedDesc> &to, uint64_t off, uint64_t n, uint32_t mode) {
+                    FusedDesc d;
+                    std::memset(&d, 0, sizeof(d));
+                    d.bytes = n;
+                    d.accLeftMask = mask;
+                    d.tile0 = tiles;
+                    d.mode = mode;
+                    d.nsrc = uint32_t(srcs.size());
+                    d.ndst = uint32_t(dsts.size());
+                    d.srcBase = uint32_t(srcPool.size());
+                    d.dstBase = uint32_t(dstPool.size());
+                    d.nleaf = it.nleaf;
+                    d.flags = flags;
+                    for (size_t k = 0; k < srcs.size(); k++) {
+                        char *s = srcs[k] ? srcs[k] + off : nullptr;
+                        d.flags |= (reinterpret_cast<uintptr_t>(s) & 3u) != 0 ? kFusedWordSources : 0u;
+                        srcPool.push_back(s);
+                        if (kind == int(KK_STACK)) {
+                            opPool.push_back(k < it.ops.size() ? it.ops[k] : 0u);
+                        }
+                    }
+                    for (char *t : dsts) {
+                        dstPool.push_back(t + off);
+                    }
+                    traffic += n * streams;
+                    written += n * dsts.size();
+                    to.push_back(d);
+                };
                 SplitByAlignment(addrs, it.bytes, [&](uint64_t off0, uint64_t n0, uint32_t mode) {
                     for (uint64_t at = 0; at < n0; at += piece) {
-                        const uint64_t off = off0 + at, n = std::min(piece, n0 - at);
-                        FusedDesc d;
-                        std::memset(&d, 0, sizeof(d));
-                        d.bytes = n;
-                        d.accLeftMask = mask;
-                        d.tile0 = tiles;
-                        d.mode = mode;
-                        d.nsrc = uint32_t(srcs.size());
-                        d.ndst = uint32_t(dsts.size());
-                        d.srcBase = uint32_t(srcPool.size());
-                        d.dstBase = uint32_t(dstPool.size());
-                        d.nleaf = it.nleaf;
-                        d.flags = fusedOrdinary ? kFusedOrdinaryStores : 0u;
-                        for (size_t k = 0; k < srcs.size(); k++) {
-                            srcPool.push_back(srcs[k] ? srcs[k] + off : nullptr);
-                            if (kind == int(KK_STACK)) {
-                                opPool.push_back(k < it.ops.size() ? it.ops[k] : 0u);
-                            }
+                        const uint64_t n = std::min(piece, n0 - at), whole = mode != ACC_ELEM ? n / kTileBytes * kTileBytes : 0;
+                        if (whole != 0) {
+                            add(descs, off0 + at, whole, mode);
+                            tiles += uint32_t(whole / kTileBytes);
                         }
-                        for (char *t : dsts) {
-                            dstPool.push_back(t + off);
+                        if (n != whole) {
+                            add(rests, off0 + at + whole, n - whole, mode);
                         }
-                        tiles += TilesOf(n);
-                        traffic += n * streams;
-                        descs.push_back(d);
                         if (capBytes != 0 && traffic >= capBytes) {
                             flush();
                         }
@@ -796,11 +833,12 @@ void KernelArgs(LaunchRec &l, void **args)
     args[0] = &l.table;
     args[1] = &l.nitems;
     if (l.fusedArgs) {
-        args[2] = &l.ntiles;
-        args[3] = &l.srcPool;
-        args[4] = &l.dstPool;
-        args[5] = &l.tilesPerItem;
-        args[6] = &l.teamCtr;      // read by the team kernels only
+        args[2] = &l.nwhole;
+        args[3] = &l.ntiles;
+        args[4] = &l.srcPool;
+        args[5] = &l.dstPool;
+        args[6] = &l.tilesPerItem;
+        args[7] = &l.teamCtr;      // read by the team kernels only
     } else {
         args[2] = &l.nwhole;
         args[3] = &l.ntiles;
@@ -813,7 +851,7 @@ HcclResult BuildGraph(Prepared *pp)
     HIP_OK(hipGraphCreate(&pp->graph, 0));
     hipGraphNode_t prev = nullptr;
     for (LaunchRec &l : pp->launches) {
-        void *args[7];
+        void *args[8];
         KernelArgs(l, args);
         hipKernelNodeParams kp = {};
         kp.func = const_cast<void *>(l.func);
@@ -1548,7 +1586,7 @@ HcclResult IssueCollective(Group *g, uint32_t launcher)
         HIP_OK(hipGraphLaunch(pp->exec, ls));
     } else {
         for (LaunchRec &l : pp->launches) {
-            void *args[7];
+            void *args[8];
             KernelArgs(l, args);
             HIP_OK(hipLaunchKernel(l.func, dim3(l.grid, 1, 1), dim3(kBlockThreads, 1, 1), args, l.dynamicLds, ls));
         }

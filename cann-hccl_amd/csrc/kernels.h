@@ -16,8 +16,8 @@ constexpr uint32_t kBlockThreads = 256;
 // How a step's bytes may be accessed.
 enum AccessMode : uint32_t {
     ACC_VEC16 = 0,      // every pointer 16-byte aligned, byte count a multiple of 16
-    ACC_VEC16_ANY = 1,  // first destination 16-byte aligned, the other pointers at any element boundary; multiple of 16
-    ACC_ELEM = 2        // element by element (heads, tails, unaligned buffers)
+    ACC_VEC16_ANY = 1,  // multiple of 16, some pointers off a 16-byte boundary (at any element boundary)
+    ACC_ELEM = 2        // element by element (heads, tails)
 };
 
 // dst = a            when b == nullptr
@@ -52,8 +52,15 @@ struct FusedDesc {
     uint32_t flags;     // kFusedOrdinaryStores
 };
 
-// flags of a fused item
-constexpr uint32_t kFusedOrdinaryStores = 1u;  // whole passes of the chain kernel store write-back instead of non-temporal
+// flags of a fused item.  Stores: streamed past the caches unless one of the first two is set (StorePolicy, kernels_impl.h).
+constexpr uint32_t kFusedOrdinaryStores = 1u;  // write-back
+constexpr uint32_t kFusedThroughStores = 2u;   // written through to memory, without the non-temporal hint (plain kernels)
+constexpr uint32_t kFusedWordSources = 4u;     // 8-bit chains: a source starts off a 16-byte boundary
+constexpr uint32_t kFusedPairs = 8u;           // trees: some leaf has a second source
+constexpr uint32_t kFusedAlike = 16u;          // chains: all items of the launch have the same number of sources, two or more
+
+// What the tables of a launch keep behind their pointer pools, so that eight pointers can be fetched together.
+constexpr uint32_t kPoolPad = 8;
 
 // flags of the step kernel
 constexpr uint32_t kStepOrdinaryStores = 1u;   // write-back stores instead of non-temporal ones in the fast loop
@@ -74,8 +81,9 @@ enum KernelKind : int {
     KK_TEAM_CHAIN = 4, KK_TEAM_TREE = 5, KK_TEAM_STACK = 6,   // team forms of the fused kernels, see below
     KK_DIRECT = 7, KK_DIRECT_WIDE = 8,                         // small collectives, see below
     KK_TEAM_STACK_TILES = 9,                                   // the team's stack kernel without its rounds read source by source
-    KK_COUNT = 10,
-    KK_GATHER = 10                                             // copy kernel table only
+    KK_CHAIN_SLOW = 10,                                        // the chain kernel with two sources in flight
+    KK_COUNT = 11,
+    KK_GATHER = 11                                             // copy kernel table only
 };
 
 // Team form of a fused kernel: the workgroups of one XCD read their tiles together, park the results in LDS, and write
@@ -100,7 +108,7 @@ constexpr uint32_t kTeamHeaderWords = kTeamTicket + 4;
 constexpr uint32_t kTeamDynamicLds = kTeamTiles * kTileBytes;
 struct TeamRegion {
     uint32_t first;   // first tile
-    uint32_t per;     // tiles per workgroup, 1 ... kTeamTiles: workgroup i of the team takes [first + i * per, first + (i + 1) * per)
+    uint32_t count;   // tiles, at most kTeamTiles for each workgroup of a team
 };
 inline uint32_t TeamBlockWords(uint32_t nregions) { return kTeamHeaderWords + 2u * nregions + kTeamXcds * (nregions + 1u); }
 
@@ -137,15 +145,17 @@ static_assert(sizeof(DirectArgs<32>) <= 4096, "kernel arguments");
 // Signatures:
 //   KK_STEP            (const StepDesc *steps, uint32_t nsteps, uint32_t nwhole, uint32_t ntiles, uint32_t flags)
 //                      steps whose tiles are all whole and ACC_VEC16 come first: tiles [0, nwhole)
-//   KK_CHAIN / KK_TREE / KK_STACK
-//                      (const FusedDesc *items, uint32_t nitems, uint32_t ntiles,
+//   KK_CHAIN / KK_CHAIN_SLOW / KK_TREE / KK_STACK
+//                      (const FusedDesc *items, uint32_t nitems, uint32_t nwhole, uint32_t ntiles,
 //                       const void *const *srcPool, void *const *dstPool, uint32_t tilesPerItem)
+//                      tiles [0, nwhole) are the whole tiles of the first nitems items, each later tile is an item of its own;
+//                      tilesPerItem: tiles of each of the first nitems items (the last one at most as many), 0 = they differ
 //   KK_TEAM_*          the same and (uint32_t *teamBlock)
 //   KK_DIRECT / KK_DIRECT_WIDE   (DirectArgs<8> / DirectArgs<32>), grid (1 + chunks of the longest item, items): blockIdx.x == 0
 //                      is for the bytes behind an item's last whole vector
 const void *LookupKernel(int hcclDataType, int hcclReduceOp, KernelKind kind);
 
-//   KK_GATHER          (const SegDesc *segs, uint32_t nsegs, uint32_t unused, const void *unused, void *unused)
+//   KK_GATHER          (const SegDesc *segs, uint32_t nsegs)
 //                      copy kernel table only
 // Byte-wise variants for pure data movement (all-gather, all-to-all-v): KK_STEP, KK_CHAIN, KK_TEAM_CHAIN, KK_GATHER,
 // KK_DIRECT and KK_DIRECT_WIDE.

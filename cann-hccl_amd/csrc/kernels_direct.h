@@ -19,20 +19,6 @@
 
 namespace hcclamd {
 
-// What a lane works on: 16 bytes, or (behind the last whole vector of an item) one element.
-template <typename T, int OP> struct DirectVec {
-    typedef V4 Val;
-    static __device__ __forceinline__ Val Load(const void *p, uint32_t off) { return Load16<ACC_VEC16_ANY>(p, off); }
-    static __device__ __forceinline__ void Store(void *p, uint32_t off, Val v) { StoreAny16<ACC_VEC16_ANY>(p, off, v); }
-    static __device__ __forceinline__ Val Combine(Val a, Val b) { return Combine16<T, OP>(a, b); }
-};
-template <typename T, int OP> struct DirectElem {
-    typedef T Val;
-    static __device__ __forceinline__ Val Load(const void *p, uint32_t off) { return LoadElem<T>(p, off); }
-    static __device__ __forceinline__ void Store(void *p, uint32_t off, Val v) { StoreElem<T>(p, off, v); }
-    static __device__ __forceinline__ Val Combine(Val a, Val b) { return Elem<T, OP>::Apply(a, b); }
-};
-
 // The kernel arguments where they lie (constant memory): read through the parameter itself, the wide form is copied to
 // private memory first.
 #define HCCL_CONSTANT __attribute__((address_space(4)))
@@ -52,9 +38,6 @@ template <uint32_t CAP> struct DirectView {
     __device__ __forceinline__ uint64_t Dst(uint32_t k) const { return args->base[(it->dst[k >> 2] >> (8u * (k & 3u))) & 0xffu]; }
 };
 
-// Keeps the compiler from moving memory accesses over this point (it sinks loads to their first use otherwise).
-__device__ __forceinline__ void DirectPin() { asm volatile("" ::: "memory"); }
-
 // N sources from source j0 on into acc.
 template <typename L, typename T, int OP, uint32_t CAP, uint32_t N>
 __device__ __forceinline__ void DirectBatch(const DirectView<CAP> &view, uint32_t j0, uint32_t off,
@@ -70,7 +53,7 @@ __device__ __forceinline__ void DirectBatch(const DirectView<CAP> &view, uint32_
     for (uint32_t j = 0; j < N; j++) {
         v[j] = L::Load(reinterpret_cast<const void *>(p[j]), off);
     }
-    DirectPin();
+    PinAccesses();
     acc = j0 == 0 ? v[0] : ((OrderMatters<T, OP>::value && !((view.it->accLeft >> j0) & 1u)) ? L::Combine(v[0], acc) : L::Combine(acc, v[0]));
 #pragma unroll
     for (uint32_t j = 1; j < N; j++) {
@@ -127,7 +110,7 @@ __device__ __forceinline__ typename L::Val DirectLeaves(const DirectView<CAP> &v
         for (uint32_t i = 0; i < G; i++) {
             w[i] = L::Load(reinterpret_cast<const void *>(view.Src(kDirectSecond<CAP> + i0 + i)), off);
         }
-        DirectPin();
+        PinAccesses();
 #pragma unroll
         for (uint32_t i = 0; i < G; i++) {
             if ((view.it->second >> (i0 + i)) & 1u) {
@@ -135,7 +118,7 @@ __device__ __forceinline__ typename L::Val DirectLeaves(const DirectView<CAP> &v
             }
         }
     }
-    DirectPin();
+    PinAccesses();
 #pragma unroll
     for (uint32_t w = 1; w < G; w <<= 1) {
 #pragma unroll
@@ -178,7 +161,7 @@ __device__ __forceinline__ typename L::Val DirectStack(const DirectView<CAP> &vi
     for (uint32_t j = 0; j < 8; j++) {      // the list repeats its last source up to 8
         v[j] = L::Load(reinterpret_cast<const void *>(view.Src(j)), off);
     }
-    DirectPin();
+    PinAccesses();
     typename L::Val top = v[0], b0 = top, b1 = top, b2 = top, b3 = top, b4 = top, b5 = top, b6 = top;   // (b3 ... b6 only named)
     uint32_t depth = 0;
     const uint32_t nsrc = view.it->nsrc;
@@ -271,12 +254,12 @@ __global__ void __launch_bounds__(kBlockThreads) DirectKernel(const DirectArgs<C
     if (blockIdx.x != 0) {
         const uint32_t at = (blockIdx.x - 1) * kDirectChunk + threadIdx.x * 16u;
         if (at + 16u <= view.it->bytes) {
-            DirectLane<DirectVec<T, OP>, T, OP, CAP>(view, at);
+            DirectLane<VecLane<T, OP>, T, OP, CAP>(view, at);
         }
     } else {
         const uint32_t rest = view.it->bytes & 15u;
         if (threadIdx.x * uint32_t(sizeof(T)) < rest) {
-            DirectLane<DirectElem<T, OP>, T, OP, CAP>(view, view.it->bytes - rest + threadIdx.x * uint32_t(sizeof(T)));
+            DirectLane<ElemLane<T, OP>, T, OP, CAP>(view, view.it->bytes - rest + threadIdx.x * uint32_t(sizeof(T)));
         }
     }
 }
@@ -289,12 +272,12 @@ __global__ void __launch_bounds__(kBlockThreads) DirectCopyKernel(const DirectAr
     if (blockIdx.x != 0) {
         const uint32_t at = (blockIdx.x - 1) * kDirectChunk + threadIdx.x * 16u;
         if (at + 16u <= view.it->bytes) {
-            DirectMove<DirectVec<uint8_t, ROP_SUM>, CAP>(view, at);
+            DirectMove<VecLane<uint8_t, ROP_SUM>, CAP>(view, at);
         }
     } else {
         const uint32_t rest = view.it->bytes & 15u;
         if (threadIdx.x < rest) {
-            DirectMove<DirectElem<uint8_t, ROP_SUM>, CAP>(view, view.it->bytes - rest + threadIdx.x);
+            DirectMove<ElemLane<uint8_t, ROP_SUM>, CAP>(view, view.it->bytes - rest + threadIdx.x);
         }
     }
 }

@@ -65,7 +65,7 @@ extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[6] = {
 #define HCCL_ROW(OP)                                                     \
     {                                                                    \
         reinterpret_cast<const void *>(&StepKernel<DT, OP>),             \
-        reinterpret_cast<const void *>(&ChainKernel<DT, OP>),            \
+        reinterpret_cast<const void *>(&ChainKernel<DT, OP, false>),     \
         reinterpret_cast<const void *>(&TreeKernel<DT, OP>),             \
         reinterpret_cast<const void *>(&StackKernel<DT, OP>),            \
         reinterpret_cast<const void *>(&TeamChainKernel<DT, OP>),        \
@@ -74,6 +74,7 @@ extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[6] = {
         reinterpret_cast<const void *>(&DirectKernel<DT, OP, 8>),        \
         reinterpret_cast<const void *>(&DirectKernel<DT, OP, 32>),       \
         reinterpret_cast<const void *>(&TeamStackKernel<DT, OP, sizeof(DT) != 8 && (sizeof(DT) != 1 || OP != ROP_PROD)>),   \
+        reinterpret_cast<const void *>(&ChainKernel<DT, OP, true>),      \
     }
 extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[4][KK_COUNT] = {
     HCCL_ROW(ROP_SUM), HCCL_ROW(ROP_PROD), HCCL_ROW(ROP_MAX), HCCL_ROW(ROP_MIN),

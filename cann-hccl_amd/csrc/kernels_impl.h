@@ -330,6 +330,37 @@ __device__ __forceinline__ void Store16(void *base, uint64_t byteOff, V4 v)
     __builtin_nontemporal_store(v, (GlobalV4 *)(static_cast<char *>(base) + byteOff));
 }
 
+// 16 bytes at an address of any alignment, past the caches.
+__device__ __forceinline__ void StoreAny16(void *base, uint64_t pos, V4 v)
+{
+    V4U t = {v.x, v.y, v.z, v.w};
+    __builtin_nontemporal_store(t, (GlobalV4U *)(static_cast<char *>(base) + pos));
+}
+
+// Stores through a buffer descriptor: a choice of cache policies that plain stores do not have, one descriptor per
+// destination and tile instead of an address per lane and vector, and whatever lies at or behind its `bytes` is dropped.  The
+// address need not be aligned.  Policies, MI355X, plain streaming kernels, TB/s read and written (non-temporal alone /
+// ordinary / through / through + non-temporal):
+//   8 sources, 8 destinations of 4, 12, 24, 96 MiB   6.1 / 5.7 / 6.3 / 6.2   5.6 / - / 5.8 / 5.6   5.6 / 5.3 / 5.6 / 5.6   5.5 / 5.4 / 5.5 / 5.6
+//   1 source, 8 destinations of 4, 24, 96 MiB        5.2 / 4.8 / 6.1 / 5.9   5.4 / 5.1 / 5.5 / 5.5   5.2 / 5.1 / 5.3 / 5.2
+//   8 sources, 1 destination of 8, 32, 48, 96 MiB    6.1 / - / 6.2 / 6.1   6.3 / - / 6.5 / 6.1   6.3 / - / 6.5 / 6.2   6.1 / - / 6.1 / 6.1
+//   one to one, 32, 96 MiB                           5.3 / - / 5.9 / 5.5   6.0 / - / 6.2 / 6.1
+enum StorePolicy : uint32_t {
+    STORE_ORDINARY = 0,      // write-back
+    STORE_NT = 2,            // non-temporal
+    STORE_THROUGH = 16,      // past the L2 at once, kept in the memory-side cache
+    STORE_STREAMED = 18      // both
+};
+typedef __amdgpu_buffer_rsrc_t BufferRsrc;
+__device__ __forceinline__ BufferRsrc MakeBuffer(void *base, uint32_t bytes)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(base, 0, int(bytes), 0x00020000);
+}
+template <uint32_t POLICY> __device__ __forceinline__ void BufferStore16(BufferRsrc r, uint32_t pos, V4 v)
+{
+    __builtin_amdgcn_raw_buffer_store_b128(v, r, int(pos), 0, int(POLICY));
+}
+
 // Element-wise access to global memory (heads, tails, unaligned buffers).
 template <size_t N> struct ElemCarrier;
 template <> struct ElemCarrier<1> { typedef uint8_t type; };
@@ -539,9 +570,15 @@ __global__ void __launch_bounds__(kBlockThreads) StepKernel(const StepDesc *__re
     }
 }
 
-// ---- fused chain: read every source once, combine in schedule order, write every destination ----------
+// ---- fused kernels: what they share ---------------------------------------------------------------------
+// The tiles of a launch come in two parts.  Tiles [0, nwhole) are whole: they belong to the first nitems items, whose
+// byte counts are multiples of kTileBytes.  Every tile from nwhole on is an item of its own (item nitems + tile - nwhole):
+// what is left of a stretch behind its last whole tile, and its element-wise ends.  The loop over whole tiles has
+// nothing else in it: with the guarded paths in the same loop the compiler makes a tile's loads wait for each other and for
+// the stores of the tile before.  The pieces behind them go through the same straight-line code, all sources' loads in flight: one
+// after the other they were most of a ragged collective of a few MiB (all-reduce, 8 ranks, bf16, 2 MiB + 6 bytes per rank
+// 20.9 us, now 8.0; 32 ranks 77.6, now 27.9).
 constexpr uint32_t kChainVec = 4;      // vectors per lane per pass
-constexpr uint32_t kChainSrcBatch = 8; // sources whose loads are issued together
 
 // Operand order changes the bits only where the combine is not commutative bit for bit:
 // floating max / min (NaN and signed zero follow the selection rule).
@@ -551,201 +588,338 @@ template <int OP> struct OrderMatters<double, OP> { static constexpr bool value 
 template <int OP> struct OrderMatters<HalfBits, OP> { static constexpr bool value = (OP == ROP_MAX || OP == ROP_MIN); };
 template <int OP> struct OrderMatters<Bf16Bits, OP> { static constexpr bool value = (OP == ROP_MAX || OP == ROP_MIN); };
 
-template <uint32_t MODE, bool ORDINARY = false> __device__ __forceinline__ void StoreAny16(void *base, uint64_t pos, V4 v)
-{
-    if (MODE == ACC_VEC16) {
-        if (ORDINARY) {
-            *(GlobalV4 *)(static_cast<char *>(base) + pos) = v;
-        } else {
-            Store16(base, pos, v);
-        }
-    } else {
-        V4U t = {v.x, v.y, v.z, v.w};
-        __builtin_nontemporal_store(t, (GlobalV4U *)(static_cast<char *>(base) + pos));
+// What a lane works on: 16 bytes, or one element.  `base` is the same for the whole wave, `pos` a lane's offset from it.
+// What is loaded is a Raw; Value makes a Val of it.  Accesses are unaligned ones (the instruction is the same one), so one
+// form serves every alignment.
+template <typename T, int OP> struct VecLane {
+    typedef V4 Val;
+    typedef V4 Raw;
+    static __device__ __forceinline__ Raw Load(const void *base, uint32_t pos) { return Load16<ACC_VEC16_ANY>(base, pos); }
+    static __device__ __forceinline__ Val Value(const Raw &r, const void *) { return r; }
+    static __device__ __forceinline__ void Store(void *base, uint32_t pos, Val v) { StoreAny16(base, pos, v); }
+    static __device__ __forceinline__ Val Combine(Val a, Val b) { return Combine16<T, OP>(a, b); }
+};
+template <typename T, int OP> struct WordLane {
+    typedef V4 Val;
+    typedef WordVec Raw;
+    static __device__ __forceinline__ uint32_t Shift(const void *base) { return uint32_t(reinterpret_cast<uintptr_t>(base)) & 3u; }
+    static __device__ __forceinline__ Raw Load(const void *base, uint32_t pos)
+    {
+        Raw r;
+        r.Load(base, pos, Shift(base));
+        return r;
     }
-}
+    static __device__ __forceinline__ Val Value(const Raw &r, const void *base) { return r.Vector(Shift(base)); }
+    static __device__ __forceinline__ Val Combine(Val a, Val b) { return Combine16<T, OP>(a, b); }
+};
+template <typename T, int OP> struct ElemLane {
+    typedef T Val;
+    typedef T Raw;
+    static __device__ __forceinline__ Raw Load(const void *base, uint32_t pos) { return LoadElem<T>(base, pos); }
+    static __device__ __forceinline__ Val Value(const Raw &r, const void *) { return r; }
+    static __device__ __forceinline__ void Store(void *base, uint32_t pos, Val v) { StoreElem<T>(base, pos, v); }
+    static __device__ __forceinline__ Val Combine(Val a, Val b) { return Elem<T, OP>::Apply(a, b); }
+};
 
-// One pass over kChainVec * 256 vectors starting at vector vecBase of the tile.
-// FULL: every lane has all its vectors inside the tile (no per-lane guards).
-// PARK: the results are not stored to the destinations but left in LDS, vector i of the tile at park[i] (the team
-// kernels write them out later); dst is not used then.
-// ONE_BATCH: the item has at most kChainSrcBatch sources (the caller has checked), so `src` is only ever indexed with
-// constants: a caller that keeps the pointers in a local array then keeps them in registers from tile to tile.
-template <typename T, int OP, uint32_t MODE, bool FULL, bool ORDINARY = false, bool PARK = false, bool ONE_BATCH = false>
-__device__ __forceinline__ void ChainVecPass(const FusedDesc &d, const void *const *__restrict__ src,
-    void *const *__restrict__ dst, uint64_t off, uint32_t vecBase, uint32_t nvec, LdsV4 *park = nullptr)
+// Keeps the compiler from moving memory accesses over this point (it sinks loads to their first use otherwise).
+__device__ __forceinline__ void PinAccesses() { asm volatile("" ::: "memory"); }
+
+// U values per lane to nbytes at every destination (positions at or behind nbytes are dropped by the buffer range check).
+template <uint32_t POLICY, uint32_t U>
+__device__ __forceinline__ void StoreEach(void *const *__restrict__ dst, uint32_t ndst, uint64_t off, uint32_t nbytes,
+    const uint32_t (&pos)[U], const V4 (&v)[U])
 {
-    constexpr bool kByWords = MODE == ACC_VEC16_ANY && sizeof(T) == 1 && !PARK;
-    const uint32_t tid = threadIdx.x;
-    uint64_t pos[kChainVec];
-    bool live[kChainVec];
-#pragma unroll
-    for (uint32_t u = 0; u < kChainVec; u++) {
-        uint32_t i = vecBase + u * kBlockThreads + tid;
-        live[u] = FULL || i < nvec;
-        pos[u] = off + uint64_t(i) * 16;
-    }
-    V4 acc[kChainVec];
-    const uint32_t nsrc = d.nsrc;
-    const uint32_t batched = ONE_BATCH ? 1u : nsrc;
-    for (uint32_t j = 0; j < batched; j += kChainSrcBatch) {
-        V4 v[kChainSrcBatch][kChainVec];
-        WordVec words[kChainSrcBatch][kChainVec];
-        uint32_t shift[kChainSrcBatch];
-#pragma unroll
-        for (uint32_t jj = 0; jj < kChainSrcBatch; jj++) {
-            if (j + jj < nsrc) {
-                const void *s = src[j + jj];
-                shift[jj] = uint32_t(reinterpret_cast<uintptr_t>(s)) & 3u;     // (positions are multiples of 16)
-#pragma unroll
-                for (uint32_t u = 0; u < kChainVec; u++) {
-                    if (live[u]) {
-                        if (kByWords) {
-                            words[jj][u].Load(s, pos[u], shift[jj]);
-                        } else {
-                            v[jj][u] = Load16<MODE>(s, pos[u]);
-                        }
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (uint32_t jj = 0; jj < kChainSrcBatch; jj++) {
-            if (j + jj < nsrc) {
-                if (kByWords) {
-#pragma unroll
-                    for (uint32_t u = 0; u < kChainVec; u++) {
-                        v[jj][u] = words[jj][u].Vector(shift[jj]);
-                    }
-                }
-                if (j + jj == 0) {
-#pragma unroll
-                    for (uint32_t u = 0; u < kChainVec; u++) {
-                        acc[u] = v[0][u];
-                    }
-                } else {
-                    const bool accLeft = OrderMatters<T, OP>::value && ((d.accLeftMask >> (j + jj)) & 1ull);
-                    // the flag is the same for the whole wave: a branch, not both results and a select per element
-                    if (accLeft) {
-#pragma unroll
-                        for (uint32_t u = 0; u < kChainVec; u++) {
-                            if (live[u]) {
-                                acc[u] = Combine16<T, OP>(acc[u], v[jj][u]);
-                            }
-                        }
-                    } else {
-#pragma unroll
-                        for (uint32_t u = 0; u < kChainVec; u++) {
-                            if (live[u]) {
-                                acc[u] = Combine16<T, OP>(v[jj][u], acc[u]);
-                            }
-                        }
-                    }
-                }
-            }
-        }
-    }
-    if (PARK) {
-#pragma unroll
-        for (uint32_t u = 0; u < kChainVec; u++) {
-            if (live[u]) {
-                park[vecBase + u * kBlockThreads + tid] = acc[u];
-            }
-        }
-        return;
-    }
-    const uint32_t ndst = d.ndst;
     for (uint32_t k = 0; k < ndst; k++) {
-        void *o = dst[k];
+        const BufferRsrc r = MakeBuffer(static_cast<char *>(dst[k]) + off, nbytes);
 #pragma unroll
-        for (uint32_t u = 0; u < kChainVec; u++) {
-            if (live[u]) {
-                StoreAny16<MODE, ORDINARY>(o, pos[u], acc[u]);
-            }
+        for (uint32_t u = 0; u < U; u++) {
+            BufferStore16<POLICY>(r, pos[u], v[u]);
         }
     }
 }
-
-template <typename T, int OP>
-__device__ __forceinline__ void ChainElem(const FusedDesc &d, const void *const *__restrict__ src,
-    void *const *__restrict__ dst, uint64_t off, uint32_t n)
+template <uint32_t U>
+__device__ __forceinline__ void StoreByFlags(const FusedDesc &d, void *const *__restrict__ dst, uint64_t off, uint32_t nbytes,
+    const uint32_t (&pos)[U], const V4 (&v)[U])
 {
-    const uint32_t cnt = n / sizeof(T);
-    for (uint32_t i = threadIdx.x; i < cnt; i += kBlockThreads) {
-        const uint64_t at = off + uint64_t(i) * sizeof(T);
-        T acc = LoadElem<T>(src[0], at);
-        for (uint32_t j = 1; j < d.nsrc; j++) {
-            T v = LoadElem<T>(src[j], at);
-            acc = ((d.accLeftMask >> j) & 1ull) ? Elem<T, OP>::Apply(acc, v) : Elem<T, OP>::Apply(v, acc);
-        }
-        for (uint32_t k = 0; k < d.ndst; k++) {
-            StoreElem<T>(dst[k], at, acc);
-        }
+    if (d.flags & kFusedThroughStores) {
+        StoreEach<STORE_THROUGH>(dst, d.ndst, off, nbytes, pos, v);
+    } else if (d.flags & kFusedOrdinaryStores) {
+        StoreEach<STORE_ORDINARY>(dst, d.ndst, off, nbytes, pos, v);
+    } else {
+        StoreEach<STORE_NT>(dst, d.ndst, off, nbytes, pos, v);
     }
 }
 
-template <typename T, int OP>
-__global__ void __launch_bounds__(kBlockThreads) ChainKernel(const FusedDesc *__restrict__ items, uint32_t nitems,
-    uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem)
+// Positions of a lane's vectors in a tile, and where it reads: a lane behind the last vector of a piece that is no whole
+// tile reads that one again and drops the result.
+template <uint32_t U> __device__ __forceinline__ void TilePositions(uint32_t (&pos)[U])
+{
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) {
+        pos[u] = (u * kBlockThreads + threadIdx.x) * 16u;
+    }
+}
+template <uint32_t U> __device__ __forceinline__ void ReadPositions(const uint32_t (&pos)[U], uint32_t nbytes, uint32_t (&at)[U])
+{
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) {
+        at[u] = pos[u] < nbytes ? pos[u] : nbytes - 16u;
+    }
+}
+
+// Walks a launch's tiles with a grid stride: whole(d, ahead(d), off) for each whole tile, rest(d) for each item behind them.
+// A workgroup keeps its item while its tiles stay inside it; the next item, and what `ahead` fetches for it, is looked up
+// ahead of the current tile's loads, so that the chain of dependent loads (table, item, pointer) completes behind those.
+template <typename Ahead, typename Whole, typename Rest>
+__device__ __forceinline__ void WalkTiles(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole, uint32_t ntiles,
+    uint32_t tilesPerItem, Ahead ahead, Whole whole, Rest rest)
 {
     uint32_t tile = blockIdx.x;
-    if (tile >= ntiles) {
-        return;
-    }
-    // a workgroup keeps its item while its tiles stay inside it; the next item is looked up ahead of the current
-    // tile's loads (see the copy kernel)
-    FusedDesc d = items[ItemOfTile(items, nitems, tile, tilesPerItem)];
-    uint32_t dEnd = d.tile0 + uint32_t((d.bytes + kTileBytes - 1) / kTileBytes);
-    for (;;) {
-        const uint32_t next = tile + gridDim.x;
-        FusedDesc dn = d;
-        uint32_t dnEnd = dEnd;
-        if (next < ntiles && next >= dEnd) {
-            dn = items[ItemOfTile(items, nitems, next, tilesPerItem)];
-            dnEnd = dn.tile0 + uint32_t((dn.bytes + kTileBytes - 1) / kTileBytes);
+    if (tile < nwhole) {
+        FusedDesc d = items[ItemOfTile(items, nitems, tile, tilesPerItem)];
+        uint32_t dEnd = d.tile0 + uint32_t(d.bytes / kTileBytes);
+        auto a = ahead(d);
+        for (;;) {
+            const uint32_t next = tile + gridDim.x;
+            FusedDesc dn = d;
+            uint32_t dnEnd = dEnd;
+            auto an = a;
+            if (next < nwhole && next >= dEnd) {
+                dn = items[ItemOfTile(items, nitems, next, tilesPerItem)];
+                dnEnd = dn.tile0 + uint32_t(dn.bytes / kTileBytes);
+                an = ahead(dn);
+            }
+            whole(d, a, uint64_t(tile - d.tile0) * kTileBytes);
+            tile = next;
+            if (tile >= nwhole) {
+                break;
+            }
+            d = dn;
+            dEnd = dnEnd;
+            a = an;
         }
-        const uint64_t off = uint64_t(tile - d.tile0) * kTileBytes;
-        const uint64_t left = d.bytes - off;
-        const uint32_t n = left < kTileBytes ? uint32_t(left) : kTileBytes;
-        const void *const *src = srcPool + d.srcBase;
-        void *const *dst = dstPool + d.dstBase;
-        if (d.mode == ACC_ELEM) {
-            ChainElem<T, OP>(d, src, dst, off, n);
+    }
+    for (; tile < ntiles; tile += gridDim.x) {
+        const FusedDesc d = items[nitems + (tile - nwhole)];
+        rest(d);
+    }
+}
+
+// ---- fused chain: read every source once, combine in schedule order, write every destination ----------
+// Sources go in straight-line code, all loads of a step in front of its combines: a guard per source makes the compiler wait
+// for the loads issued so far at every guard, and a lane then has 8 loads in flight instead of 32.
+template <typename L, uint32_t N, uint32_t U>
+__device__ __forceinline__ void ChainLoad(const void *const *__restrict__ src, uint64_t off, const uint32_t (&at)[U], typename L::Raw (&v)[N][U])
+{
+#pragma unroll
+    for (uint32_t j = 0; j < N; j++) {
+        const char *s = static_cast<const char *>(src[j]) + off;
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) {
+            v[j][u] = L::Load(s, at[u]);
+        }
+    }
+    PinAccesses();
+}
+// Folds N sources into acc; FIRST: the first of them starts it.
+template <typename L, typename T, int OP, uint32_t N, uint32_t U, bool FIRST>
+__device__ __forceinline__ void ChainFold(const void *const *__restrict__ src, const typename L::Raw (&v)[N][U], uint64_t accLeft, typename L::Val (&acc)[U])
+{
+#pragma unroll
+    for (uint32_t j = 0; j < N; j++) {
+        if (FIRST && j == 0) {
+#pragma unroll
+            for (uint32_t u = 0; u < U; u++) {
+                acc[u] = L::Value(v[0][u], src[0]);
+            }
+        } else if (OrderMatters<T, OP>::value && ((accLeft >> j) & 1ull)) {
+            // the flag is the same for the whole wave: a branch, not both results and a select per element
+#pragma unroll
+            for (uint32_t u = 0; u < U; u++) {
+                acc[u] = L::Combine(acc[u], L::Value(v[j][u], src[j]));
+            }
         } else {
-            const uint32_t nvec = n >> 4;
-            constexpr uint32_t kPass = kChainVec * kBlockThreads;
-            uint32_t base = 0;
-            if (d.mode == ACC_VEC16) {
-                // the store kind is a compile-time property of the pass (a per-store choice at run time
-                // is merged by the compiler into one plain store)
-                if (d.flags & kFusedOrdinaryStores) {
-                    for (; base + kPass <= nvec; base += kPass) {
-                        ChainVecPass<T, OP, ACC_VEC16, true, true>(d, src, dst, off, base, nvec);
-                    }
-                } else {
-                    for (; base + kPass <= nvec; base += kPass) {
-                        ChainVecPass<T, OP, ACC_VEC16, true, false>(d, src, dst, off, base, nvec);
-                    }
-                }
-                if (base < nvec) {
-                    ChainVecPass<T, OP, ACC_VEC16, false>(d, src, dst, off, base, nvec);
-                }
-            } else {
-                for (; base + kPass <= nvec; base += kPass) {
-                    ChainVecPass<T, OP, ACC_VEC16_ANY, true>(d, src, dst, off, base, nvec);
-                }
-                if (base < nvec) {
-                    ChainVecPass<T, OP, ACC_VEC16_ANY, false>(d, src, dst, off, base, nvec);
-                }
+#pragma unroll
+            for (uint32_t u = 0; u < U; u++) {
+                acc[u] = L::Combine(L::Value(v[j][u], src[j]), acc[u]);
             }
         }
-        if (next >= ntiles) {
-            break;
-        }
-        tile = next;
-        d = dn;
-        dEnd = dnEnd;
     }
+}
+template <typename L, typename T, int OP, uint32_t N, uint32_t U, bool FIRST>
+__device__ __forceinline__ void ChainBatch(const void *const *__restrict__ src, uint64_t off, const uint32_t (&at)[U], uint64_t accLeft,
+    typename L::Val (&acc)[U])
+{
+    typename L::Raw v[N][U];
+    ChainLoad<L, N, U>(src, off, at, v);
+    ChainFold<L, T, OP, N, U, FIRST>(src, v, accLeft, acc);
+}
+
+// Makes what comes after it wait for these values.
+template <uint32_t U> __device__ __forceinline__ void HoldBack(V4 (&x)[U])
+{
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) {
+        asm volatile("" : "+v"(x[u])::"memory");
+    }
+}
+
+// The chain's value at U positions of a lane, `off` behind the item's pointers: up to 8 sources, all in flight together (src is
+// only indexed with constants: a caller may keep the pointers in registers).
+template <typename L, typename T, int OP, uint32_t U>
+__device__ __forceinline__ void ChainFew(uint32_t nsrc, uint64_t accLeft, const void *const *__restrict__ src, uint64_t off, const uint32_t (&at)[U],
+    typename L::Val (&acc)[U])
+{
+    switch (nsrc) {
+        case 1: ChainBatch<L, T, OP, 1, U, true>(src, off, at, accLeft, acc); break;
+        case 2: ChainBatch<L, T, OP, 2, U, true>(src, off, at, accLeft, acc); break;
+        case 3: ChainBatch<L, T, OP, 3, U, true>(src, off, at, accLeft, acc); break;
+        case 4: ChainBatch<L, T, OP, 4, U, true>(src, off, at, accLeft, acc); break;
+        case 5: ChainBatch<L, T, OP, 5, U, true>(src, off, at, accLeft, acc); break;
+        case 6: ChainBatch<L, T, OP, 6, U, true>(src, off, at, accLeft, acc); break;
+        case 7: ChainBatch<L, T, OP, 7, U, true>(src, off, at, accLeft, acc); break;
+        default: ChainBatch<L, T, OP, 8, U, true>(src, off, at, accLeft, acc); break;
+    }
+}
+// More than 8 sources: two sets of 4, one in flight while the other is folded.
+template <typename L, typename T, int OP, uint32_t U>
+__device__ __forceinline__ void ChainMany(uint32_t nsrc, uint64_t accLeft, const void *const *__restrict__ src, uint64_t off, const uint32_t (&at)[U],
+    typename L::Val (&acc)[U])
+{
+    constexpr uint32_t N = 4;
+    typename L::Raw va[N][U], vb[N][U];
+    ChainLoad<L, N, U>(src, off, at, va);
+    ChainLoad<L, N, U>(src + N, off, at, vb);
+    ChainFold<L, T, OP, N, U, true>(src, va, accLeft, acc);
+    uint32_t j = N;               // vb holds sources j ... j + N - 1
+#pragma nounroll
+    for (; j + 3 * N <= nsrc; j += 2 * N) {
+        ChainLoad<L, N, U>(src + j + N, off, at, va);
+        ChainFold<L, T, OP, N, U, false>(src + j, vb, accLeft >> j, acc);
+        ChainLoad<L, N, U>(src + j + 2 * N, off, at, vb);
+        ChainFold<L, T, OP, N, U, false>(src + j + N, va, accLeft >> (j + N), acc);
+    }
+    if (j + 2 * N <= nsrc) {
+        ChainLoad<L, N, U>(src + j + N, off, at, va);
+        ChainFold<L, T, OP, N, U, false>(src + j, vb, accLeft >> j, acc);
+        ChainFold<L, T, OP, N, U, false>(src + j + N, va, accLeft >> (j + N), acc);
+        j += 2 * N;
+    } else {
+        ChainFold<L, T, OP, N, U, false>(src + j, vb, accLeft >> j, acc);
+        j += N;
+    }
+    switch (nsrc - j) {
+        case 1: ChainBatch<L, T, OP, 1, U, false>(src + j, off, at, accLeft >> j, acc); break;
+        case 2: ChainBatch<L, T, OP, 2, U, false>(src + j, off, at, accLeft >> j, acc); break;
+        case 3: ChainBatch<L, T, OP, 3, U, false>(src + j, off, at, accLeft >> j, acc); break;
+        default: break;
+    }
+}
+template <typename L, typename T, int OP, uint32_t U>
+__device__ __forceinline__ void ChainValue(const FusedDesc &d, const void *const *__restrict__ src, uint64_t off, const uint32_t (&at)[U],
+    typename L::Val (&acc)[U])
+{
+    if (d.nsrc <= 8) {
+        ChainFew<L, T, OP, U>(d.nsrc, d.accLeftMask, src, off, at, acc);
+    } else {
+        ChainMany<L, T, OP, U>(d.nsrc, d.accLeftMask, src, off, at, acc);
+    }
+}
+// The same with two sources in flight at a time: a source is requested when the one two before it is folded.
+template <typename L, typename T, int OP, uint32_t U>
+__device__ __forceinline__ void ChainSlow(const FusedDesc &d, const void *const *__restrict__ src, uint64_t off, const uint32_t (&at)[U],
+    typename L::Val (&acc)[U])
+{
+    const uint32_t nsrc = d.nsrc;
+    const uint64_t accLeft = d.accLeftMask;
+    if (nsrc == 1) {
+        ChainBatch<L, T, OP, 1, U, true>(src, off, at, accLeft, acc);
+        return;
+    }
+    typename L::Raw va[1][U], vb[1][U];
+    ChainLoad<L, 1, U>(src, off, at, va);
+    ChainLoad<L, 1, U>(src + 1, off, at, vb);
+    ChainFold<L, T, OP, 1, U, true>(src, va, accLeft, acc);
+    HoldBack(acc);
+    uint32_t j = 1;               // vb holds source j
+#pragma nounroll
+    for (; j + 3 <= nsrc; j += 2) {
+        ChainLoad<L, 1, U>(src + j + 1, off, at, va);
+        ChainFold<L, T, OP, 1, U, false>(src + j, vb, accLeft >> j, acc);
+        HoldBack(acc);
+        ChainLoad<L, 1, U>(src + j + 2, off, at, vb);
+        ChainFold<L, T, OP, 1, U, false>(src + j + 1, va, accLeft >> (j + 1), acc);
+        HoldBack(acc);
+    }
+    if (j + 2 <= nsrc) {
+        ChainLoad<L, 1, U>(src + j + 1, off, at, va);
+        ChainFold<L, T, OP, 1, U, false>(src + j, vb, accLeft >> j, acc);
+        ChainFold<L, T, OP, 1, U, false>(src + j + 1, va, accLeft >> (j + 1), acc);
+    } else {
+        ChainFold<L, T, OP, 1, U, false>(src + j, vb, accLeft >> j, acc);
+    }
+}
+
+// U vectors per lane of a tile, or of a piece of `nbytes` (a multiple of 16).
+template <typename T, int OP, bool WHOLE, bool SLOW, uint32_t U>
+__device__ __forceinline__ void ChainTile(const FusedDesc &d, const void *const *__restrict__ src, void *const *__restrict__ dst, uint64_t off, uint32_t nbytes)
+{
+    typedef VecLane<T, OP> Vec;
+    typedef WordLane<T, OP> Words;
+    uint32_t pos[U], at[U];
+    V4 acc[U];
+    TilePositions(pos);
+    ReadPositions(pos, WHOLE ? kTileBytes : nbytes, at);
+    if (sizeof(T) == 1 && (d.flags & kFusedWordSources)) {
+        if (SLOW) {
+            ChainSlow<Words, T, OP, U>(d, src, off, at, acc);
+        } else {
+            ChainValue<Words, T, OP, U>(d, src, off, at, acc);
+        }
+    } else if (SLOW) {
+        ChainSlow<Vec, T, OP, U>(d, src, off, at, acc);
+    } else {
+        ChainValue<Vec, T, OP, U>(d, src, off, at, acc);
+    }
+    StoreByFlags(d, dst, off, WHOLE ? kTileBytes : nbytes, pos, acc);
+}
+
+// An item behind the whole tiles.
+template <typename T, int OP, bool SLOW = false>
+__device__ __forceinline__ void ChainRest(const FusedDesc &d, const void *const *__restrict__ src, void *const *__restrict__ dst)
+{
+    const uint32_t n = uint32_t(d.bytes);
+    if (d.mode != ACC_ELEM) {
+        if (n <= kBlockThreads * 16u) {
+            ChainTile<T, OP, false, false, 1>(d, src, dst, 0, n);
+        } else {
+            ChainTile<T, OP, false, SLOW, kChainVec>(d, src, dst, 0, n);
+        }
+    } else {
+        for (uint32_t i = threadIdx.x * uint32_t(sizeof(T)); i < n; i += kBlockThreads * uint32_t(sizeof(T))) {
+            const uint32_t at[1] = {i};
+            T acc[1];
+            ChainValue<ElemLane<T, OP>, T, OP, 1>(d, src, 0, at, acc);
+            for (uint32_t k = 0; k < d.ndst; k++) {
+                StoreElem<T>(dst[k], i, acc[0]);
+            }
+        }
+    }
+}
+
+// Two forms.  Measured, us, this kernel's loads guarded one by one (before) / all in flight / two sources in flight: all-reduce, 8
+// ranks, fp32, 2 MiB per rank 7.3 / 7.3 / 7.5, 6 MiB 20.1 / 17.5 / 18.9, 8 MiB 23.9 / 22.2 / 23.9; reduce-scatter, 8 ranks, fp32, blocks of 8 MiB
+// 97.0 / 101.0 / 98.6, 16 MiB 192.7 / 200.1 / 190.8; 16 ranks, bf16 maximum, 512 KiB 27.6 / 25.4 / 23.7, 16 MiB 777 / 767 / 755.
+// SLOW = false has all loads of a tile in flight, the shortest way through a tile, for results with several
+// destinations.  SLOW = true has two sources' in flight and 70 registers instead of 170: many sources into one destination
+// run better on more workgroups that ask for less each.
+template <typename T, int OP, bool SLOW>
+__global__ void __launch_bounds__(kBlockThreads) ChainKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole,
+    uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem)
+{
+    WalkTiles(items, nitems, nwhole, ntiles, tilesPerItem, [](const FusedDesc &) { return 0; },
+        [&](const FusedDesc &d, int, uint64_t off) { ChainTile<T, OP, true, SLOW, kChainVec>(d, srcPool + d.srcBase, dstPool + d.dstBase, off, kTileBytes); },
+        [&](const FusedDesc &d) { ChainRest<T, OP, SLOW>(d, srcPool + d.srcBase, dstPool + d.dstBase); });
 }
 
 // ---- pure data movement: one source, m destinations ------------------------------------------------------
@@ -753,37 +927,28 @@ __global__ void __launch_bounds__(kBlockThreads) ChainKernel(const FusedDesc *__
 // workgroups fit on a CU where the chain kernel fits two.  A copy keeps only 4 loads per lane in flight, and its
 // rate comes from how many waves do that at once (measured, 1 GiB copy: 5.1 TB/s through the chain kernel,
 // 6.3 TB/s for a plain copy kernel at full occupancy).
-template <uint32_t MODE, bool FULL, bool ORDINARY = false, bool PARK = false>
-__device__ __forceinline__ void CopyVecPass(const void *s, void *const *__restrict__ dst, uint32_t ndst, uint64_t off,
-    uint32_t vecBase, uint32_t nvec, LdsV4 *park = nullptr)
+typedef VecLane<uint8_t, ROP_SUM> MoveLane;
+
+template <bool WHOLE>
+__device__ __forceinline__ void CopyTile(const FusedDesc &d, const void *s, void *const *__restrict__ dst, uint64_t off, uint32_t nbytes)
 {
-    uint64_t pos[kChainVec];
-    bool live[kChainVec];
-    V4 v[kChainVec];
-#pragma unroll
-    for (uint32_t u = 0; u < kChainVec; u++) {
-        const uint32_t i = vecBase + u * kBlockThreads + threadIdx.x;
-        live[u] = FULL || i < nvec;
-        pos[u] = off + uint64_t(i) * 16;
-        if (live[u]) {
-            v[u] = Load16<MODE>(s, pos[u]);
-        }
-    }
-    if (PARK) {
-#pragma unroll
-        for (uint32_t u = 0; u < kChainVec; u++) {
-            if (live[u]) {
-                park[vecBase + u * kBlockThreads + threadIdx.x] = v[u];
-            }
-        }
-        return;
-    }
-    for (uint32_t k = 0; k < ndst; k++) {
-        void *o = dst[k];
-#pragma unroll
-        for (uint32_t u = 0; u < kChainVec; u++) {
-            if (live[u]) {
-                StoreAny16<MODE, ORDINARY>(o, pos[u], v[u]);
+    uint32_t pos[kChainVec], at[kChainVec];
+    V4 v[1][kChainVec];
+    TilePositions(pos);
+    ReadPositions(pos, WHOLE ? kTileBytes : nbytes, at);
+    ChainLoad<MoveLane, 1, kChainVec>(&s, off, at, v);
+    StoreByFlags(d, dst, off, WHOLE ? kTileBytes : nbytes, pos, v[0]);
+}
+__device__ __forceinline__ void CopyRest(const FusedDesc &d, const void *s, void *const *__restrict__ dst)
+{
+    const uint32_t n = uint32_t(d.bytes);
+    if (d.mode != ACC_ELEM) {
+        CopyTile<false>(d, s, dst, 0, n);
+    } else {
+        for (uint32_t i = threadIdx.x; i < n; i += kBlockThreads) {
+            const uint8_t b = LoadElem<uint8_t>(s, i);
+            for (uint32_t k = 0; k < d.ndst; k++) {
+                StoreElem<uint8_t>(dst[k], i, b);
             }
         }
     }
@@ -792,74 +957,12 @@ __device__ __forceinline__ void CopyVecPass(const void *s, void *const *__restri
 // Same arguments and tables as the chain kernel; every item has exactly one source.  (A template only so that the
 // definition may sit in this header; Variant is unused.)
 template <int Variant>
-__global__ void __launch_bounds__(kBlockThreads) CopyKernel(const FusedDesc *__restrict__ items, uint32_t nitems,
+__global__ void __launch_bounds__(kBlockThreads) CopyKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole,
     uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem)
 {
-    uint32_t tile = blockIdx.x;
-    if (tile >= ntiles) {
-        return;
-    }
-    // The item of a tile costs a chain of dependent loads (table, item, pointer).  A workgroup that stays inside one
-    // item from one tile to the next keeps what it has; when the next tile lies in another item, that item is looked
-    // up before the current tile's data is loaded, so that the chain completes behind those loads.
-    FusedDesc d = items[ItemOfTile(items, nitems, tile, tilesPerItem)];
-    const void *s = srcPool[d.srcBase];
-    uint32_t dEnd = d.tile0 + uint32_t((d.bytes + kTileBytes - 1) / kTileBytes);
-    for (;;) {
-        const uint32_t next = tile + gridDim.x;
-        FusedDesc dn = d;
-        const void *sn = s;
-        uint32_t dnEnd = dEnd;
-        if (next < ntiles && next >= dEnd) {
-            dn = items[ItemOfTile(items, nitems, next, tilesPerItem)];
-            sn = srcPool[dn.srcBase];
-            dnEnd = dn.tile0 + uint32_t((dn.bytes + kTileBytes - 1) / kTileBytes);
-        }
-        const uint64_t off = uint64_t(tile - d.tile0) * kTileBytes;
-        const uint64_t left = d.bytes - off;
-        const uint32_t n = left < kTileBytes ? uint32_t(left) : kTileBytes;
-        void *const *dst = dstPool + d.dstBase;
-        if (d.mode == ACC_ELEM) {
-            for (uint32_t i = threadIdx.x; i < n; i += kBlockThreads) {
-                const uint8_t b = LoadElem<uint8_t>(s, off + i);
-                for (uint32_t k = 0; k < d.ndst; k++) {
-                    StoreElem<uint8_t>(dst[k], off + i, b);
-                }
-            }
-        } else {
-            const uint32_t nvec = n >> 4;
-            constexpr uint32_t kPass = kChainVec * kBlockThreads;
-            uint32_t base = 0;
-            if (d.mode == ACC_VEC16) {
-                if (d.flags & kFusedOrdinaryStores) {
-                    for (; base + kPass <= nvec; base += kPass) {
-                        CopyVecPass<ACC_VEC16, true, true>(s, dst, d.ndst, off, base, nvec);
-                    }
-                } else {
-                    for (; base + kPass <= nvec; base += kPass) {
-                        CopyVecPass<ACC_VEC16, true>(s, dst, d.ndst, off, base, nvec);
-                    }
-                }
-                if (base < nvec) {
-                    CopyVecPass<ACC_VEC16, false>(s, dst, d.ndst, off, base, nvec);
-                }
-            } else {
-                for (; base + kPass <= nvec; base += kPass) {
-                    CopyVecPass<ACC_VEC16_ANY, true>(s, dst, d.ndst, off, base, nvec);
-                }
-                if (base < nvec) {
-                    CopyVecPass<ACC_VEC16_ANY, false>(s, dst, d.ndst, off, base, nvec);
-                }
-            }
-        }
-        if (next >= ntiles) {
-            break;
-        }
-        tile = next;
-        d = dn;
-        s = sn;
-        dEnd = dnEnd;
-    }
+    WalkTiles(items, nitems, nwhole, ntiles, tilesPerItem, [&](const FusedDesc &d) { return srcPool[d.srcBase]; },
+        [&](const FusedDesc &d, const void *s, uint64_t off) { CopyTile<true>(d, s, dstPool + d.dstBase, off, kTileBytes); },
+        [&](const FusedDesc &d) { CopyRest(d, srcPool[d.srcBase], dstPool + d.dstBase); });
 }
 
 // ---- small-segment gather: LDS staging ---------------------------------------------------------------------
@@ -875,8 +978,7 @@ __global__ void __launch_bounds__(kBlockThreads) CopyKernel(const FusedDesc *__r
 constexpr uint32_t kGatherLdsPerWave = kGatherMaxBytes + 32;
 
 template <int Variant>
-__global__ void __launch_bounds__(kBlockThreads) GatherKernel(const SegDesc *__restrict__ segs, uint32_t nsegs, uint32_t,
-    const void *const *__restrict__, void *const *__restrict__, uint32_t)
+__global__ void __launch_bounds__(kBlockThreads) GatherKernel(const SegDesc *__restrict__ segs, uint32_t nsegs)
 {
     __shared__ __attribute__((aligned(16))) uint8_t lds[(kBlockThreads / 64) * kGatherLdsPerWave];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
@@ -923,246 +1025,196 @@ __global__ void __launch_bounds__(kBlockThreads) GatherKernel(const SegDesc *__r
 }
 
 // ---- fused perfect tree (halving-doubling): leaves pairwise bottom-up ----------------------------------
-// v[i] = v[i] (+) v[i+w] for w = 1, 2, 4, ... is evaluated group by group: the first three levels
-// inside groups of 8 consecutive leaves (8 loads per vector in flight, one result kept per group), the
-// remaining levels over the group results.  Same association as the flat loop, a quarter of the
-// registers; a lane works on kTreeVec vectors at a time so that 16 loads are outstanding per group
-// (measured, 8-rank fp32 all-reduce of 32 MiB per rank: 124 us with one vector, 104 us with two).
+// v[i] = v[i] (+) v[i+w] for w = 1, 2, 4, ...  Same association as the flat loop, evaluated in groups of 8 leaves: a
+// group's leaves come in two sets of 4, and while one set is folded the other one's loads, then the next group's, are in
+// flight; the group results go through a binary counter.
 constexpr uint32_t kTreeGroup = 8;
-constexpr uint32_t kTreeMaxGroups = 4;   // up to 32 leaves
 
-constexpr uint32_t kTreeVecPlain = 2;    // vectors per lane per pass
-constexpr uint32_t kTreeVecTeam = 4;     // in the team kernels, which run one workgroup per CU: twice the loads in flight
-
-// Evaluates the tree for kTreeVec vectors of one lane (positions pos[u], skipped where !live[u]).
-// kTreeVec is kTreeVecPlain, or kTreeVecTeam when the results are parked (PARK).
-// G = leaves per group: 8 when the tree has 8 or more leaves, else the leaf count itself (1, 2, 4),
-// so that no group is ever partial and the loads of a group are issued back to back.
-template <typename T, int OP, uint32_t MODE, bool FULL, uint32_t G, uint32_t kTreeVec>
-__device__ __forceinline__ void TreeValue(const FusedDesc &d, const void *const *__restrict__ src,
-    const uint64_t (&pos)[kTreeVec], const bool (&live)[kTreeVec], V4 (&x)[kTreeVec])
+// N leaves from leaf 0 of `src` on (two pool entries each, the second one of a folded rank pair or null).
+template <typename L, uint32_t N, uint32_t U>
+__device__ __forceinline__ void TreeLoad(const void *const *__restrict__ src, uint64_t off, const uint32_t (&at)[U], typename L::Val (&v)[N][U])
 {
-    const uint32_t ngroups = d.nleaf / G;   // 1, 2 or 4
-    // Pending left operands of the upper levels (a binary counter over the groups seen so far).
-    V4 l0[kTreeVec], l1[kTreeVec];
 #pragma unroll
-    for (uint32_t u = 0; u < kTreeVec; u++) {
-        l0[u] = l1[u] = x[u] = V4{0, 0, 0, 0};
+    for (uint32_t i = 0; i < N; i++) {
+        const char *s = static_cast<const char *>(src[2 * i]) + off;
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) {
+            v[i][u] = L::Load(s, at[u]);
+        }
     }
-    // Kept as a loop on purpose: unrolled, the compiler hoists every group's loads to the top and
-    // the register count (and with it the number of resident waves) is back to the flat version's.
-#pragma nounroll
-    for (uint32_t gi = 0; gi < ngroups; gi++) {
-        const void *const *gs = src + 2 * gi * G;
-        V4 v[G][kTreeVec];
+    PinAccesses();
+}
+// The second sources of the leaves that have one: together where all of them do, the usual case.
+template <typename L, uint32_t N, uint32_t U>
+__device__ __forceinline__ void TreePairs(const void *const *__restrict__ src, uint64_t off, const uint32_t (&at)[U], typename L::Val (&v)[N][U])
+{
+    bool all = true;
 #pragma unroll
-        for (uint32_t i = 0; i < G; i++) {
-            const void *s = gs[2 * i];
+    for (uint32_t i = 0; i < N; i++) {
+        all = all && src[2 * i + 1] != nullptr;
+    }
+    if (all) {
+        typename L::Val w[N][U];
+        TreeLoad<L, N, U>(src + 1, off, at, w);
 #pragma unroll
-            for (uint32_t u = 0; u < kTreeVec; u++) {
-                if (FULL || live[u]) {
-                    v[i][u] = Load16<MODE>(s, pos[u]);
-                }
+        for (uint32_t i = 0; i < N; i++) {
+#pragma unroll
+            for (uint32_t u = 0; u < U; u++) {
+                v[i][u] = L::Combine(v[i][u], w[i][u]);
             }
         }
-        // second sources of the leaves (folded rank pairs), four leaves at a time: all loads of a
-        // batch first, then the combines
-        constexpr uint32_t B = G >= 4 ? 4 : G;
+    } else {
 #pragma unroll
-        for (uint32_t b0 = 0; b0 < G; b0 += B) {
-            V4 w[B][kTreeVec];
-            bool has[B];
+        for (uint32_t i = 0; i < N; i++) {
+            if (src[2 * i + 1] != nullptr) {
+                typename L::Val w[1][U];
+                TreeLoad<L, 1, U>(src + 2 * i + 1, off, at, w);
 #pragma unroll
-            for (uint32_t i = 0; i < B; i++) {
-                const void *s = gs[2 * (b0 + i) + 1];
-                has[i] = s != nullptr;
-                if (has[i]) {
-#pragma unroll
-                    for (uint32_t u = 0; u < kTreeVec; u++) {
-                        if (FULL || live[u]) {
-                            w[i][u] = Load16<MODE>(s, pos[u]);
-                        }
-                    }
-                }
-            }
-#pragma unroll
-            for (uint32_t i = 0; i < B; i++) {
-                if (has[i]) {
-#pragma unroll
-                    for (uint32_t u = 0; u < kTreeVec; u++) {
-                        if (FULL || live[u]) {
-                            v[b0 + i][u] = Combine16<T, OP>(v[b0 + i][u], w[i][u]);
-                        }
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (uint32_t w = 1; w < G; w <<= 1) {
-#pragma unroll
-            for (uint32_t i = 0; i + w < G; i += 2 * w) {
-#pragma unroll
-                for (uint32_t u = 0; u < kTreeVec; u++) {
-                    v[i][u] = Combine16<T, OP>(v[i][u], v[i + w][u]);
-                }
-            }
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < kTreeVec; u++) {
-            x[u] = v[0][u];
-        }
-        if ((gi & 1u) == 0) {
-#pragma unroll
-            for (uint32_t u = 0; u < kTreeVec; u++) {
-                l0[u] = x[u];
-            }
-        } else {
-#pragma unroll
-            for (uint32_t u = 0; u < kTreeVec; u++) {
-                x[u] = Combine16<T, OP>(l0[u], x[u]);
-            }
-            if ((gi & 2u) == 0) {
-#pragma unroll
-                for (uint32_t u = 0; u < kTreeVec; u++) {
-                    l1[u] = x[u];
-                }
-            } else {
-#pragma unroll
-                for (uint32_t u = 0; u < kTreeVec; u++) {
-                    x[u] = Combine16<T, OP>(l1[u], x[u]);
+                for (uint32_t u = 0; u < U; u++) {
+                    v[i][u] = L::Combine(v[i][u], w[0][u]);
                 }
             }
         }
     }
 }
-
-// One pass over kTreeVec * 256 vectors starting at vector vecBase of the tile.
-template <typename T, int OP, uint32_t MODE, bool FULL, uint32_t G, bool PARK = false>
-__device__ __forceinline__ void TreeVecPass(const FusedDesc &d, const void *const *__restrict__ src,
-    void *const *__restrict__ dst, uint64_t off, uint32_t vecBase, uint32_t nvec, LdsV4 *park = nullptr)
+// N leaves pairwise into x.
+template <typename L, uint32_t N, uint32_t U>
+__device__ __forceinline__ void TreeFold(typename L::Val (&v)[N][U], typename L::Val (&x)[U])
 {
-    constexpr uint32_t kTreeVec = PARK ? kTreeVecTeam : kTreeVecPlain;
-    uint64_t pos[kTreeVec];
-    bool live[kTreeVec];
 #pragma unroll
-    for (uint32_t u = 0; u < kTreeVec; u++) {
-        uint32_t i = vecBase + u * kBlockThreads + threadIdx.x;
-        live[u] = FULL || i < nvec;
-        pos[u] = off + uint64_t(i) * 16;
-    }
-    V4 r[kTreeVec];
-    TreeValue<T, OP, MODE, FULL, G, kTreeVec>(d, src, pos, live, r);
-    if (PARK) {
+    for (uint32_t w = 1; w < N; w <<= 1) {
 #pragma unroll
-        for (uint32_t u = 0; u < kTreeVec; u++) {
-            if (live[u]) {
-                park[vecBase + u * kBlockThreads + threadIdx.x] = r[u];
+        for (uint32_t i = 0; i + w < N; i += 2 * w) {
+#pragma unroll
+            for (uint32_t u = 0; u < U; u++) {
+                v[i][u] = L::Combine(v[i][u], v[i + w][u]);
             }
+        }
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) {
+        x[u] = v[0][u];
+    }
+}
+template <typename L, uint32_t U>
+__device__ __forceinline__ void TreeJoin(const typename L::Val (&a)[U], typename L::Val (&x)[U])
+{
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) {
+        x[u] = L::Combine(a[u], x[u]);
+    }
+}
+template <typename L, uint32_t N, uint32_t U>
+__device__ __forceinline__ void TreeSet(const void *const *__restrict__ src, uint64_t off, const uint32_t (&at)[U], typename L::Val (&x)[U])
+{
+    typename L::Val v[N][U];
+    TreeLoad<L, N, U>(src, off, at, v);
+    TreePairs<L, N, U>(src, off, at, v);
+    TreeFold<L, N, U>(v, x);
+}
+
+// The tree's value at U positions of a lane, `off` behind the item's pointers.
+template <typename L, uint32_t U>
+__device__ __forceinline__ void TreeValue(const FusedDesc &d, const void *const *__restrict__ src, uint64_t off, const uint32_t (&at)[U],
+    typename L::Val (&x)[U])
+{
+    if (d.nleaf < kTreeGroup) {
+        if (d.nleaf == 4) {
+            TreeSet<L, 4, U>(src, off, at, x);
+        } else if (d.nleaf == 2) {
+            TreeSet<L, 2, U>(src, off, at, x);
+        } else {
+            TreeSet<L, 1, U>(src, off, at, x);
         }
         return;
     }
-    const uint32_t ndst = d.ndst;
-    for (uint32_t k = 0; k < ndst; k++) {
-        void *o = dst[k];
+    const uint32_t ngroups = d.nleaf / kTreeGroup;   // 1, 2 or 4
+    typename L::Val l0[U], l1[U], y[U];              // pending left operands of the upper levels
+    auto count = [&](uint32_t gi) {
+        if ((gi & 1u) == 0) {
 #pragma unroll
-        for (uint32_t u = 0; u < kTreeVec; u++) {
-            if (live[u]) {
-                StoreAny16<MODE>(o, pos[u], r[u]);
+            for (uint32_t u = 0; u < U; u++) {
+                l0[u] = x[u];
+            }
+        } else {
+            TreeJoin<L, U>(l0, x);
+            if ((gi & 2u) == 0) {
+#pragma unroll
+                for (uint32_t u = 0; u < U; u++) {
+                    l1[u] = x[u];
+                }
+            } else {
+                TreeJoin<L, U>(l1, x);
             }
         }
-    }
-}
-
-// All vector passes of one tile.
-template <typename T, int OP, uint32_t G, bool PARK = false>
-__device__ __forceinline__ void TreeTileVec(const FusedDesc &d, const void *const *__restrict__ src,
-    void *const *__restrict__ dst, uint64_t off, uint32_t nvec, LdsV4 *park = nullptr)
-{
-    constexpr uint32_t kPass = (PARK ? kTreeVecTeam : kTreeVecPlain) * kBlockThreads;
-    uint32_t base = 0;
-    if (d.mode == ACC_VEC16) {
-        for (; base + kPass <= nvec; base += kPass) {
-            TreeVecPass<T, OP, ACC_VEC16, true, G, PARK>(d, src, dst, off, base, nvec, park);
+    };
+    if (d.flags & kFusedPairs) {
+#pragma nounroll
+        for (uint32_t gi = 0; gi < ngroups; gi++) {
+            const void *const *gs = src + 2 * gi * kTreeGroup;
+            TreeSet<L, 4, U>(gs, off, at, y);
+            TreeSet<L, 4, U>(gs + 8, off, at, x);
+            TreeJoin<L, U>(y, x);
+            count(gi);
         }
-        if (base < nvec) {
-            TreeVecPass<T, OP, ACC_VEC16, false, G, PARK>(d, src, dst, off, base, nvec, park);
-        }
-    } else {
-        for (; base < nvec; base += kPass) {
-            TreeVecPass<T, OP, ACC_VEC16_ANY, false, G, PARK>(d, src, dst, off, base, nvec, park);
-        }
+        return;
     }
-}
-
-// All vector passes of one tile, whatever the number of leaves.
-template <typename T, int OP, bool PARK = false>
-__device__ __forceinline__ void TreeTile(const FusedDesc &d, const void *const *__restrict__ src,
-    void *const *__restrict__ dst, uint64_t off, uint32_t nvec, LdsV4 *park = nullptr)
-{
-    if (d.nleaf >= kTreeGroup) {
-        TreeTileVec<T, OP, kTreeGroup, PARK>(d, src, dst, off, nvec, park);
-    } else if (d.nleaf == 4) {
-        TreeTileVec<T, OP, 4, PARK>(d, src, dst, off, nvec, park);
-    } else if (d.nleaf == 2) {
-        TreeTileVec<T, OP, 2, PARK>(d, src, dst, off, nvec, park);
-    } else {
-        TreeTileVec<T, OP, 1, PARK>(d, src, dst, off, nvec, park);
+    typename L::Val va[4][U], vb[4][U];
+    TreeLoad<L, 4, U>(src, off, at, va);
+    TreeLoad<L, 4, U>(src + 8, off, at, vb);
+    uint32_t gi = 0;
+#pragma nounroll
+    for (; gi + 1 < ngroups; gi++) {
+        const void *const *next = src + 2 * (gi + 1) * kTreeGroup;
+        TreeFold<L, 4, U>(va, y);
+        TreeLoad<L, 4, U>(next, off, at, va);
+        TreeFold<L, 4, U>(vb, x);
+        TreeLoad<L, 4, U>(next + 8, off, at, vb);
+        TreeJoin<L, U>(y, x);
+        count(gi);
     }
+    TreeFold<L, 4, U>(va, y);
+    TreeFold<L, 4, U>(vb, x);
+    TreeJoin<L, U>(y, x);
+    count(gi);
 }
 
 template <typename T, int OP>
-__device__ __forceinline__ void TreeElem(const FusedDesc &d, const void *const *__restrict__ src,
-    void *const *__restrict__ dst, uint64_t off, uint32_t n)
+__device__ __forceinline__ void TreeRest(const FusedDesc &d, const void *const *__restrict__ src, void *const *__restrict__ dst)
 {
-    constexpr uint32_t kMax = kTreeGroup * kTreeMaxGroups;
-    const uint32_t cnt = n / sizeof(T);
-    for (uint32_t e = threadIdx.x; e < cnt; e += kBlockThreads) {
-        const uint64_t at = off + uint64_t(e) * sizeof(T);
-        T v[kMax];
-#pragma unroll
-        for (uint32_t i = 0; i < kMax; i++) {
-            if (i < d.nleaf) {
-                v[i] = LoadElem<T>(src[2 * i], at);
-                const void *s = src[2 * i + 1];
-                if (s != nullptr) {
-                    v[i] = Elem<T, OP>::Apply(v[i], LoadElem<T>(s, at));
-                }
+    const uint32_t n = uint32_t(d.bytes);
+    if (d.mode != ACC_ELEM) {
+        uint32_t pos[kChainVec], at[kChainVec];
+        V4 x[kChainVec];
+            TilePositions(pos);
+        ReadPositions(pos, n, at);
+        TreeValue<VecLane<T, OP>, kChainVec>(d, src, 0, at, x);
+        StoreByFlags(d, dst, 0, n, pos, x);
+    } else {
+        for (uint32_t i = threadIdx.x * uint32_t(sizeof(T)); i < n; i += kBlockThreads * uint32_t(sizeof(T))) {
+            const uint32_t at[1] = {i};
+            T x[1];
+            TreeValue<ElemLane<T, OP>, 1>(d, src, 0, at, x);
+            for (uint32_t k = 0; k < d.ndst; k++) {
+                StoreElem<T>(dst[k], i, x[0]);
             }
-        }
-#pragma unroll
-        for (uint32_t w = 1; w < kMax; w <<= 1) {
-            if (w < d.nleaf) {
-#pragma unroll
-                for (uint32_t i = 0; i + w < kMax; i += 2 * w) {
-                    if (i + w < d.nleaf) {
-                        v[i] = Elem<T, OP>::Apply(v[i], v[i + w]);
-                    }
-                }
-            }
-        }
-        for (uint32_t k = 0; k < d.ndst; k++) {
-            StoreElem<T>(dst[k], at, v[0]);
         }
     }
 }
 
 template <typename T, int OP>
-__global__ void __launch_bounds__(kBlockThreads) TreeKernel(const FusedDesc *__restrict__ items, uint32_t nitems,
+__global__ void __launch_bounds__(kBlockThreads) TreeKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole,
     uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem)
 {
-    for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const FusedDesc d = items[ItemOfTile(items, nitems, tile, tilesPerItem)];
-        const uint64_t off = uint64_t(tile - d.tile0) * kTileBytes;
-        const uint64_t left = d.bytes - off;
-        const uint32_t n = left < kTileBytes ? uint32_t(left) : kTileBytes;
-        const void *const *src = srcPool + d.srcBase;
-        void *const *dst = dstPool + d.dstBase;
-        if (d.mode == ACC_ELEM) {
-            TreeElem<T, OP>(d, src, dst, off, n);
-        } else {
-            TreeTile<T, OP>(d, src, dst, off, n >> 4);
-        }
-    }
+    uint32_t pos[kChainVec];
+    TilePositions(pos);
+    WalkTiles(items, nitems, nwhole, ntiles, tilesPerItem, [](const FusedDesc &) { return 0; },
+        [&](const FusedDesc &d, int, uint64_t off) {
+            V4 x[kChainVec];
+            TreeValue<VecLane<T, OP>, kChainVec>(d, srcPool + d.srcBase, off, pos, x);
+            StoreByFlags(d, dstPool + d.dstBase, off, kTileBytes, pos, x);
+        },
+        [&](const FusedDesc &d) { TreeRest<T, OP>(d, srcPool + d.srcBase, dstPool + d.dstBase); });
 }
 
 // ---- fused general expression: a stack machine over registers -----------------------------------------
@@ -1174,18 +1226,17 @@ __global__ void __launch_bounds__(kBlockThreads) TreeKernel(const FusedDesc *__r
 // switch with constant indices.  Sources are loaded in batches like the chain kernel's.
 // Two shapes: expressions that need at most 4 values (a chain of chains, a 4-leaf tree of chains) run
 // with 4 vectors per lane like the chain kernel, deeper ones (up to 8 values) with 2.
-constexpr uint32_t kStackVecShallow = 4;
 constexpr uint32_t kStackVecDeep = 2;
 constexpr uint32_t kStackShallowDepth = 4;
-constexpr uint32_t kStackSrcBatch = 8;
+constexpr uint32_t kStackTeamBatch = 8;
 // The plain kernel issues the loads of 4 sources together: with 8 it needs every register a wave can have, one
 // workgroup fits a CU and nothing hides the table look-ups between its tiles (two-level reduce-scatter of 8 x 256 MiB
 // 426 -> 417 us, reduce 434 -> 415 us, all-reduce of 8 x 16 MiB 52 -> 47 us).  The team form, one workgroup per CU by
 // its LDS, keeps 8.
 constexpr uint32_t kStackPlainBatch = 4;
 
-template <uint32_t U> struct StackVal {
-    V4 x[U];
+template <typename V, uint32_t U> struct StackVal {
+    V x[U];
 };
 
 // The values below the top one are separate variables, not an array or a struct: a switch over
@@ -1229,177 +1280,145 @@ template <uint32_t U> struct StackVal {
         }                                 \
     }
 
-template <typename T, int OP, uint32_t MODE, bool FULL, bool DEEP, bool PARK = false, uint32_t BATCH = kStackSrcBatch>
-__device__ __forceinline__ void StackVecPass(const FusedDesc &d, const void *const *__restrict__ src,
-    const uint32_t *__restrict__ ops, void *const *__restrict__ dst, uint64_t off, uint32_t vecBase, uint32_t nvec,
-    LdsV4 *park = nullptr)
+// Pushes v and folds as its op word says.  A macro: in a function the compiler merges the cases of the switches into one
+// access through a pointer.
+#define HCCL_STACK_PUSH(v, opword)                                                          \
+    {                                                                                       \
+        const uint32_t op = (opword);                                                       \
+        if (depth > 0) {                                                                    \
+            HCCL_STACK_PUT(depth - 1, top)                                                  \
+        }                                                                                   \
+        top = (v);                                                                          \
+        depth++;                                                                            \
+        const uint32_t nfold = op & 7u;                                                     \
+        _Pragma("nounroll") for (uint32_t f = 0; f < nfold && depth >= 2; f++)              \
+        {                                                                                   \
+            StackVal<typename L::Val, U> under;                                             \
+            HCCL_STACK_GET(depth - 2, under)                                                \
+            if (!OrderMatters<T, OP>::value || ((op >> (8 + f)) & 1u)) { /* one for the whole wave */ \
+                _Pragma("unroll") for (uint32_t u = 0; u < U; u++)                          \
+                {                                                                           \
+                    top.x[u] = L::Combine(under.x[u], top.x[u]);                            \
+                }                                                                           \
+            } else {                                                                        \
+                _Pragma("unroll") for (uint32_t u = 0; u < U; u++)                          \
+                {                                                                           \
+                    top.x[u] = L::Combine(top.x[u], under.x[u]);                            \
+                }                                                                           \
+            }                                                                               \
+            depth--;                                                                        \
+        }                                                                                   \
+    }
+
+// The expression's value at U positions of a lane, `off` behind the item's pointers.  BATCH sources are loaded together; the
+// last batch loads its last source again where it has fewer.
+template <typename L, typename T, int OP, uint32_t U, bool DEEP, uint32_t BATCH>
+__device__ __forceinline__ void StackValue(const FusedDesc &d, const void *const *__restrict__ src, const uint32_t *__restrict__ ops, uint64_t off,
+    const uint32_t (&at)[U], typename L::Val (&x)[U])
 {
-    constexpr uint32_t U = DEEP ? kStackVecDeep : kStackVecShallow;
-    uint64_t pos[U];
-    bool live[U];
+    StackVal<typename L::Val, U> top;
 #pragma unroll
     for (uint32_t u = 0; u < U; u++) {
-        uint32_t i = vecBase + u * kBlockThreads + threadIdx.x;
-        live[u] = FULL || i < nvec;
-        pos[u] = off + uint64_t(i) * 16;
+        top.x[u] = typename L::Val();
     }
-    StackVal<U> top;
-#pragma unroll
-    for (uint32_t u = 0; u < U; u++) {
-        top.x[u] = V4{0, 0, 0, 0};
-    }
-    StackVal<U> b0 = top, b1 = top, b2 = top, b3 = top, b4 = top, b5 = top, b6 = top;
-    uint32_t depth = 0;                  // values on the stack, the top one included
+    StackVal<typename L::Val, U> b0 = top, b1 = top, b2 = top, b3 = top, b4 = top, b5 = top, b6 = top;
+    uint32_t depth = 0;
     const uint32_t nsrc = d.nsrc;
-    for (uint32_t j = 0; j < nsrc; j += BATCH) {
-        StackVal<U> v[BATCH];
-#pragma unroll
-        for (uint32_t jj = 0; jj < BATCH; jj++) {
-            if (j + jj < nsrc) {
-                const void *s = src[j + jj];
-#pragma unroll
-                for (uint32_t u = 0; u < U; u++) {
-                    if (live[u]) {
-                        v[jj].x[u] = Load16<MODE>(s, pos[u]);
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (uint32_t jj = 0; jj < BATCH; jj++) {
-            if (j + jj < nsrc) {
-                const uint32_t op = ops[j + jj];
-                if (depth > 0) {
-                    HCCL_STACK_PUT(depth - 1, top)
-                }
-                top = v[jj];
-                depth++;
-                const uint32_t nfold = op & 7u;
 #pragma nounroll
-                for (uint32_t f = 0; f < nfold && depth >= 2; f++) {
-                    StackVal<U> under;
-                    HCCL_STACK_GET(depth - 2, under)
-                    const bool underLeft = !OrderMatters<T, OP>::value || ((op >> (8 + f)) & 1u);
-                    if (underLeft) {           // the same for the whole wave
+    for (uint32_t j = 0; j < nsrc; j += BATCH) {
+        StackVal<typename L::Val, U> v[BATCH];
 #pragma unroll
-                        for (uint32_t u = 0; u < U; u++) {
-                            if (live[u]) {
-                                top.x[u] = Combine16<T, OP>(under.x[u], top.x[u]);
-                            }
-                        }
-                    } else {
+        for (uint32_t jj = 0; jj < BATCH; jj++) {
+            const char *s = static_cast<const char *>(src[j + jj < nsrc ? j + jj : nsrc - 1]) + off;
 #pragma unroll
-                        for (uint32_t u = 0; u < U; u++) {
-                            if (live[u]) {
-                                top.x[u] = Combine16<T, OP>(top.x[u], under.x[u]);
-                            }
-                        }
-                    }
-                    depth--;
-                }
+            for (uint32_t u = 0; u < U; u++) {
+                v[jj].x[u] = L::Load(s, at[u]);
+            }
+        }
+        PinAccesses();
+#pragma unroll
+        for (uint32_t jj = 0; jj < BATCH; jj++) {
+            if (j + jj < nsrc) {
+                HCCL_STACK_PUSH(v[jj], ops[j + jj])
             }
         }
     }
-    if (PARK) {
 #pragma unroll
-        for (uint32_t u = 0; u < U; u++) {
-            if (live[u]) {
-                park[vecBase + u * kBlockThreads + threadIdx.x] = top.x[u];
-            }
-        }
-        return;
-    }
-    const uint32_t ndst = d.ndst;
-    for (uint32_t k = 0; k < ndst; k++) {
-        void *o = dst[k];
-#pragma unroll
-        for (uint32_t u = 0; u < U; u++) {
-            if (live[u]) {
-                StoreAny16<MODE>(o, pos[u], top.x[u]);
-            }
-        }
+    for (uint32_t u = 0; u < U; u++) {
+        x[u] = top.x[u];
     }
 }
 
-// Heads, tails and unaligned buffers: the same machine element by element.
-template <typename T, int OP>
-__device__ __forceinline__ void StackElem(const FusedDesc &d, const void *const *__restrict__ src,
-    const uint32_t *__restrict__ ops, void *const *__restrict__ dst, uint64_t off, uint32_t n)
+// The values of a tile, or of a piece read at `at`, in passes as wide as the depth allows: sink(u, first vector's index, values).
+template <typename T, int OP, uint32_t BATCH, typename Sink>
+__device__ __forceinline__ void StackTile(const FusedDesc &d, const void *const *__restrict__ src, const uint32_t *__restrict__ ops, uint64_t off,
+    const uint32_t (&at)[kChainVec], Sink sink)
 {
-    const uint32_t cnt = n / sizeof(T);
-    for (uint32_t e = threadIdx.x; e < cnt; e += kBlockThreads) {
-        const uint64_t at = off + uint64_t(e) * sizeof(T);
-        constexpr bool DEEP = true;
-        T top = T();
-        T b0 = top, b1 = top, b2 = top, b3 = top, b4 = top, b5 = top, b6 = top;
-        uint32_t depth = 0;
-        for (uint32_t j = 0; j < d.nsrc; j++) {
-            const uint32_t op = ops[j];
-            if (depth > 0) {
-                HCCL_STACK_PUT(depth - 1, top)
-            }
-            top = LoadElem<T>(src[j], at);
-            depth++;
-            const uint32_t nfold = op & 7u;
-            for (uint32_t f = 0; f < nfold && depth >= 2; f++) {
-                T under;
-                HCCL_STACK_GET(depth - 2, under)
-                top = ((op >> (8 + f)) & 1u) ? Elem<T, OP>::Apply(under, top) : Elem<T, OP>::Apply(top, under);
-                depth--;
-            }
-        }
-        for (uint32_t k = 0; k < d.ndst; k++) {
-            StoreElem<T>(dst[k], at, top);
-        }
-    }
-}
-
-// All vector passes of one tile.
-template <typename T, int OP, bool PARK = false, uint32_t BATCH = kStackSrcBatch>
-__device__ __forceinline__ void StackTile(const FusedDesc &d, const void *const *__restrict__ src,
-    const uint32_t *__restrict__ ops, void *const *__restrict__ dst, uint64_t off, uint32_t nvec, LdsV4 *park = nullptr)
-{
-    constexpr uint32_t kPassShallow = kStackVecShallow * kBlockThreads, kPassDeep = kStackVecDeep * kBlockThreads;
-    uint32_t base = 0;
-    if (d.mode == ACC_VEC16) {
-        // d.nleaf: the stack depth the item needs
-        if (d.nleaf <= kStackShallowDepth) {
-            for (; base + kPassShallow <= nvec; base += kPassShallow) {
-                StackVecPass<T, OP, ACC_VEC16, true, false, PARK, BATCH>(d, src, ops, dst, off, base, nvec, park);
-            }
-        }
-        for (; base + kPassDeep <= nvec; base += kPassDeep) {
-            StackVecPass<T, OP, ACC_VEC16, true, true, PARK, BATCH>(d, src, ops, dst, off, base, nvec, park);
-        }
-        if (base < nvec) {
-            StackVecPass<T, OP, ACC_VEC16, false, true, PARK, BATCH>(d, src, ops, dst, off, base, nvec, park);
-        }
+    typedef VecLane<T, OP> L;
+    V4 x[kChainVec];
+    if (d.nleaf <= kStackShallowDepth) {      // d.nleaf: the stack depth the item needs
+        StackValue<L, T, OP, kChainVec, false, BATCH>(d, src, ops, off, at, x);
+        sink(0u, x);
     } else {
-        for (; base < nvec; base += kPassDeep) {
-            StackVecPass<T, OP, ACC_VEC16_ANY, false, true, PARK, BATCH>(d, src, ops, dst, off, base, nvec, park);
+#pragma nounroll
+        for (uint32_t h = 0; h < kChainVec; h += kStackVecDeep) {
+            const uint32_t part[kStackVecDeep] = {h == 0 ? at[0] : at[2], h == 0 ? at[1] : at[3]};
+            V4 y[kStackVecDeep];
+            StackValue<L, T, OP, kStackVecDeep, true, BATCH>(d, src, ops, off, part, y);
+            sink(h, y);
+        }
+    }
+}
+static_assert(kChainVec == 4 && kStackVecDeep == 2, "StackTile takes a tile in one pass or in two");
+
+template <typename T, int OP, uint32_t BATCH>
+__device__ __forceinline__ void StackStore(const FusedDesc &d, const void *const *__restrict__ src, const uint32_t *__restrict__ ops,
+    void *const *__restrict__ dst, uint64_t off, uint32_t nbytes, const uint32_t (&pos)[kChainVec], const uint32_t (&at)[kChainVec])
+{
+    StackTile<T, OP, BATCH>(d, src, ops, off, at, [&](uint32_t h, const auto &x) {
+        constexpr uint32_t U = sizeof(x) / sizeof(V4);
+        uint32_t where[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) {
+            where[u] = h == 0 ? pos[u] : pos[kChainVec - U + u];
+        }
+        StoreByFlags(d, dst, off, nbytes, where, x);
+    });
+}
+
+template <typename T, int OP>
+__device__ __forceinline__ void StackRest(const FusedDesc &d, const void *const *__restrict__ src, const uint32_t *__restrict__ ops, void *const *__restrict__ dst)
+{
+    const uint32_t n = uint32_t(d.bytes);
+    if (d.mode != ACC_ELEM) {
+        uint32_t pos[kChainVec], at[kChainVec];
+        TilePositions(pos);
+        ReadPositions(pos, n, at);
+        StackStore<T, OP, kStackPlainBatch>(d, src, ops, dst, 0, n, pos, at);
+    } else {
+        for (uint32_t i = threadIdx.x * uint32_t(sizeof(T)); i < n; i += kBlockThreads * uint32_t(sizeof(T))) {
+            const uint32_t at[1] = {i};
+            T x[1];
+            StackValue<ElemLane<T, OP>, T, OP, 1, true, 8>(d, src, ops, 0, at, x);
+            for (uint32_t k = 0; k < d.ndst; k++) {
+                StoreElem<T>(dst[k], i, x[0]);
+            }
         }
     }
 }
 
 template <typename T, int OP>
-__global__ void __launch_bounds__(kBlockThreads) StackKernel(const FusedDesc *__restrict__ items, uint32_t nitems,
+__global__ void __launch_bounds__(kBlockThreads) StackKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole,
     uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem)
 {
-    const uint32_t *opPool = reinterpret_cast<const uint32_t *>(items + nitems);
-    for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const FusedDesc d = items[ItemOfTile(items, nitems, tile, tilesPerItem)];
-        const uint64_t off = uint64_t(tile - d.tile0) * kTileBytes;
-        const uint64_t left = d.bytes - off;
-        const uint32_t n = left < kTileBytes ? uint32_t(left) : kTileBytes;
-        const void *const *src = srcPool + d.srcBase;
-        const uint32_t *ops = opPool + d.srcBase;
-        void *const *dst = dstPool + d.dstBase;
-        if (d.mode == ACC_ELEM) {
-            StackElem<T, OP>(d, src, ops, dst, off, n);
-        } else {
-            StackTile<T, OP, false, kStackPlainBatch>(d, src, ops, dst, off, n >> 4);
-        }
-    }
+    const uint32_t *opPool = reinterpret_cast<const uint32_t *>(items + nitems + (ntiles - nwhole));
+    uint32_t pos[kChainVec];
+    TilePositions(pos);
+    WalkTiles(items, nitems, nwhole, ntiles, tilesPerItem, [](const FusedDesc &) { return 0; },
+        [&](const FusedDesc &d, int, uint64_t off) {
+            StackStore<T, OP, kStackPlainBatch>(d, srcPool + d.srcBase, opPool + d.srcBase, dstPool + d.dstBase, off, kTileBytes, pos, pos);
+        },
+        [&](const FusedDesc &d) { StackRest<T, OP>(d, srcPool + d.srcBase, opPool + d.srcBase, dstPool + d.dstBase); });
 }
 
 }  // namespace hcclamd

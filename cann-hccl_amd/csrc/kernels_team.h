@@ -7,9 +7,9 @@
 // interleaved per workgroup, 5.9 - 6.0 TB/s when the 32 workgroups of an XCD read together and then write together;
 // 1 read : 8 writes 4.9 against 5.9 TB/s).  So here the workgroups of one XCD form a team:
 //   read phase   every workgroup evaluates up to kTeamTiles tiles (every 32nd tile of the team's region, so an XCD
-//                works on one contiguous stretch of the tile space) and parks the results in LDS.  A round of whole
-//                tiles of one item is read with all its loads issued together (a copy) or source by source with the
-//                partial results in LDS (a chain; a chain of chains), see Round() below
+//                works on one contiguous stretch of the tile space) and parks the results in LDS.  A round is
+//                read with all its loads issued together (a copy) or source by source with the
+//                partial results in LDS (a chain; a chain of chains), see BySource() below
 //   barrier      among the team's workgroups only; the other XCDs run on, in whatever phase they are
 //   write phase  every workgroup writes its parked tiles to their destinations, destination by destination
 // Workgroup b belongs to XCD b % 8 (workgroups are dealt to the XCDs round robin).  If they are not, or if the team is
@@ -71,15 +71,21 @@ __device__ __forceinline__ uint32_t TeamNextRegion(uint32_t *slot, uint32_t *tic
 
 // Arrival at the team's barrier, then (thread 0) the question for the next region while the others arrive, then the
 // wait: bounded, and given up for the rest of the launch once it has run out (kTeamGaveUpBit in the arrival word).
+// `meanwhile` runs between a workgroup's arrival and its wait.
 // Every access here is a trip to memory and back, a few microseconds under load, and whatever the last workgroup to
 // arrive does here delays its whole team: it learns from its own arrival that nobody is missing, and it has
 // normally seen the next region already (`seen`: a look at the slot taken before its last tile).
+template <typename Meanwhile>
 __device__ __forceinline__ uint32_t TeamBarrier(uint32_t *c, uint32_t target, uint32_t *slot, uint32_t *ticket, uint32_t seen,
-    uint32_t *nextShared)
+    uint32_t *nextShared, Meanwhile meanwhile)
 {
     __syncthreads();
+    uint32_t v = 0;
     if (threadIdx.x == 0) {
-        uint32_t v = TeamAdd(c + kTeamArrive, 1u) + 1u;
+        v = TeamAdd(c + kTeamArrive, 1u) + 1u;
+    }
+    meanwhile();
+    if (threadIdx.x == 0) {
         *nextShared = TeamNextRegion(slot, ticket, seen);
         if ((v & ~kTeamGaveUpBit) < target && (v & kTeamGaveUpBit) == 0u) {
             const uint64_t t0 = wall_clock64();
@@ -131,44 +137,85 @@ __device__ __forceinline__ void TeamLeave(uint32_t *teamCtr, uint32_t *ctr, uint
 }
 
 // One parked tile to one destination.
-template <uint32_t MODE, bool ORDINARY>
-__device__ __forceinline__ void TeamDrain(const LdsV4 *park, void *o, uint64_t off, uint32_t nvec)
+template <uint32_t POLICY>
+__device__ __forceinline__ void TeamDrain(const LdsV4 *park, void *o)
 {
     const uint32_t tid = threadIdx.x;
-    if (nvec == kTeamVecPerTile) {
-        V4 w[kVecPerLane];
+    const BufferRsrc r = MakeBuffer(o, kTileBytes);
+    V4 w[kVecPerLane];
 #pragma unroll
-        for (uint32_t u = 0; u < kVecPerLane; u++) {
-            w[u] = park[u * kBlockThreads + tid];
-        }
+    for (uint32_t u = 0; u < kVecPerLane; u++) {
+        w[u] = park[u * kBlockThreads + tid];
+    }
 #pragma unroll
-        for (uint32_t u = 0; u < kVecPerLane; u++) {
-            StoreAny16<MODE, ORDINARY>(o, off + (uint64_t(u) * kBlockThreads + tid) * 16, w[u]);
-        }
-    } else {
-        for (uint32_t i = tid; i < nvec; i += kBlockThreads) {
-            StoreAny16<MODE, ORDINARY>(o, off + uint64_t(i) * 16, park[i]);
-        }
+    for (uint32_t u = 0; u < kVecPerLane; u++) {
+        BufferStore16<POLICY>(r, (u * kBlockThreads + tid) * 16u, w[u]);
     }
 }
 
-// Eval: SetItem(d, srcPool) is called when the tiles move on to another item, Vec(d, srcPool, extra, off, nvec, park)
-// leaves the vectors of one tile in LDS, the static Elem(d, srcPool, extra, dstPool, off, n) handles an element-wise
-// piece (a few bytes of head or tail) there and then.
+// A workgroup's tiles of one round: every teamSize-th tile of the team's region, so that the team reads, and later writes,
+// one stretch of teamSize tiles of every stream at a time instead of teamSize stretches apart (8 ranks x 256 MiB: 1.5 %
+// faster).  They may belong to several items.
+struct TeamRound {
+    const FusedDesc *items;
+    uint32_t nitems, tilesPerItem;
+    uint32_t first, n, teamSize;
+    uint32_t *heldItem;      // LDS: the tiles' items, for the write phase
+    uint32_t *peek, *seen;   // thread 0 looks at the slot of the next round once the round's last loads are on their way
+    __device__ __forceinline__ uint32_t Tile(uint32_t q) const { return first + q * teamSize; }
+    // Item of tile q in d, which holds the item of the tile before it (q > 0).
+    __device__ __forceinline__ void Item(uint32_t q, FusedDesc &d, uint32_t &idx, uint32_t &end) const
+    {
+        const uint32_t tile = Tile(q);
+        if (q == 0 || tile >= end) {
+            idx = ItemOfTile(items, nitems, tile, tilesPerItem);
+            d = items[idx];
+            end = d.tile0 + uint32_t(d.bytes / kTileBytes);
+        }
+        if (threadIdx.x == 0) {
+            heldItem[q] = idx;
+        }
+    }
+    __device__ __forceinline__ void Peek() const
+    {
+        if (threadIdx.x == 0) {
+            *seen = TeamLoad(peek);
+        }
+    }
+};
+
+// N tiles from tile q0 of a round on, as the loads by source need them: the first entry of each one's item in the source pool,
+// and its offset from the item's pointers.
+template <uint32_t N> struct TeamPlaces {
+    uint32_t base[N];
+    uint64_t off[N];
+    uint64_t accLeft[N];
+    __device__ __forceinline__ void Find(const TeamRound &r, uint32_t q0, FusedDesc &d, uint32_t &idx, uint32_t &end)
+    {
+#pragma unroll
+        for (uint32_t q = 0; q < N; q++) {
+            r.Item(q0 + q, d, idx, end);
+            base[q] = d.srcBase;
+            off[q] = uint64_t(r.Tile(q0 + q) - d.tile0) * kTileBytes;
+            accLeft[q] = d.accLeftMask;
+        }
+    }
+};
+
+// Eval: Read(round, srcPool, extra, park) evaluates the round's tiles and leaves the vectors of tile q at
+// park[q * kTeamVecPerTile]; the static Rest(d, srcPool, extra, dstPool) handles an item behind the whole tiles there and then.
 //
-// The tile space is cut into regions (first tile, tiles per workgroup), a table the host wrote behind the counters:
-// workgroup i of a team of n takes the tiles first + i, first + i + n, ... (per of them) of the team's region.  Team x starts
+// The whole tiles are cut into regions (first tile, number of tiles), a table the host wrote behind the counters:
+// workgroup i of a team of n takes the tiles first + i, first + i + n, ... of the team's region.  Team x starts
 // with region x; the later ones are drawn from a counter as the teams get there, and the last regions are smaller,
 // so that the XCDs, which do not all move data at the same rate, finish together.
 template <typename Eval>
-__device__ __forceinline__ void TeamBody(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t ntiles,
+__device__ __forceinline__ void TeamBody(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole, uint32_t ntiles,
     const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem,
     uint32_t *__restrict__ teamCtr, const void *extra)
 {
     extern __shared__ V4 teamLds[];
     __shared__ uint32_t heldItem[kTeamTiles];
-    __shared__ uint32_t heldTile[kTeamTiles];
-    __shared__ uint32_t heldVec[kTeamTiles];      // vectors parked; 0 = nothing (no tile, or an element-wise piece)
     __shared__ uint32_t nextShared;
     LdsV4 *park = (LdsV4 *)teamLds;
 
@@ -177,111 +224,50 @@ __device__ __forceinline__ void TeamBody(const FusedDesc *__restrict__ items, ui
     const TeamRegion *regions = reinterpret_cast<const TeamRegion *>(teamCtr + kTeamHeaderWords);
     uint32_t *slots = teamCtr + kTeamHeaderWords + 2u * nregions + xcd * (nregions + 1u);
     uint32_t *ctr = teamCtr + xcd * kTeamCtrStride;
+    uint32_t nextRest = nitems + blockIdx.x;
+    auto rests = [&]() __attribute__((always_inline)) {
+        for (; nextRest < nitems + (ntiles - nwhole); nextRest += gridDim.x) {
+            const FusedDesc d = items[nextRest];
+            Eval::Rest(d, srcPool + d.srcBase, extra, dstPool + d.dstBase);
+        }
+    };
     uint32_t target = 0;
     uint32_t region = xcd;
     for (uint32_t round = 0; region < nregions; round++) {
-        // A workgroup's tiles are every teamSize-th tile of the region, not a run of consecutive ones: the team then
-        // reads, and later writes, one stretch of teamSize tiles of every stream at a time instead of teamSize
-        // stretches apart (8 ranks x 256 MiB: 1.5 % faster).
         const TeamRegion reg = regions[region];
-        const uint32_t first = reg.first + inTeam;
-        const uint32_t fit = first < ntiles ? (ntiles - 1 - first) / teamSize + 1 : 0;
-        const uint32_t n = fit < reg.per ? fit : reg.per;
+        const uint32_t n = inTeam < reg.count ? (reg.count - 1 - inTeam) / teamSize + 1 : 0;
         uint32_t seen = 0;
-        uint32_t maxDst = 0;
-        uint32_t idx = 0;
-        FusedDesc d;
-        uint32_t dEnd = 0;
-        Eval eval;
-        bool bySource = false;
-        if constexpr (Eval::kBySource) {
-            // All the round's tiles whole, vector-aligned and of one item: the team reads source by source (see
-            // TeamChainEval::Round).
-            if (n == kTeamTiles || n == kTeamTiles / 2) {
-                idx = ItemOfTile(items, nitems, first, tilesPerItem);
-                d = items[idx];
-                dEnd = d.tile0 + uint32_t((d.bytes + kTileBytes - 1) / kTileBytes);
-                const uint32_t lastTile = first + (n - 1) * teamSize;
-                bySource = d.mode == ACC_VEC16 && Eval::RoundFits(d) && lastTile < dEnd &&
-                    uint64_t(lastTile - d.tile0 + 1) * kTileBytes <= d.bytes;
-            }
-            if (bySource) {
-                const uint64_t off = uint64_t(first - d.tile0) * kTileBytes;
-                const uint64_t stride = uint64_t(teamSize) * kTileBytes;
-                if (n == kTeamTiles) {
-                    Eval::template Round<kTeamTiles>(d, srcPool + d.srcBase, extra, off, stride, park, slots + round, &seen);
-                } else {
-                    Eval::template Round<kTeamTiles / 2>(d, srcPool + d.srcBase, extra, off, stride, park, slots + round, &seen);
-                }
-                maxDst = d.ndst;
-                if (threadIdx.x < n) {
-                    heldItem[threadIdx.x] = idx;
-                    heldTile[threadIdx.x] = first + threadIdx.x * teamSize;
-                    heldVec[threadIdx.x] = kTeamVecPerTile;
-                }
-            }
-        }
-        for (uint32_t q = 0; q < n && !bySource; q++) {
-            const uint32_t tile = first + q * teamSize;
-            if (q + 1 == n && threadIdx.x == 0) {
-                // a look at the slot of the next round, in flight together with the last tile's loads: a workgroup
-                // that is behind the others finds the answer there
-                seen = TeamLoad(slots + round);
-            }
-            if (q == 0 || tile >= dEnd) {
-                idx = ItemOfTile(items, nitems, tile, tilesPerItem);
-                d = items[idx];
-                dEnd = d.tile0 + uint32_t((d.bytes + kTileBytes - 1) / kTileBytes);
-                eval.SetItem(d, srcPool);
-            }
-            const uint64_t off = uint64_t(tile - d.tile0) * kTileBytes;
-            const uint64_t rest = d.bytes - off;
-            const uint32_t bytes = rest < kTileBytes ? uint32_t(rest) : kTileBytes;
-            uint32_t nvec = 0;
-            if (d.mode == ACC_ELEM) {
-                Eval::Elem(d, srcPool, extra, dstPool, off, bytes);
-            } else {
-                nvec = bytes >> 4;
-                eval.Vec(d, srcPool, extra, off, nvec, park + q * kTeamVecPerTile);
-                maxDst = d.ndst > maxDst ? d.ndst : maxDst;
-            }
-            if (threadIdx.x == 0) {
-                heldItem[q] = idx;
-                heldTile[q] = tile;
-                heldVec[q] = nvec;
-            }
+        if (n != 0) {
+            const TeamRound r = {items, nitems, tilesPerItem, reg.first + inTeam, n, teamSize, heldItem, slots + round, &seen};
+            Eval::Read(r, srcPool, extra, park);
         }
         target += teamSize;
-        region = TeamBarrier(ctr, target, slots + round, teamCtr + kTeamTicket, seen, &nextShared);
+        // The items behind the whole tiles, a few short pieces, cost no time of their own there.  (Every team has a round: the
+        // host makes at least kTeamXcds regions.  One call: called twice, this is not inlined.)
+        region = TeamBarrier(ctr, target, slots + round, teamCtr + kTeamTicket, seen, &nextShared, rests);
         // Every lane reads back the vectors it parked itself.  A workgroup's tiles mostly belong to one item, so its
         // descriptor and the destination pointer are kept from tile to tile.
-        for (uint32_t k = 0; k < maxDst; k++) {
+        for (uint32_t k = 0, more = n; more != 0; k++) {
             uint32_t cur = ~0u;
             FusedDesc w;
-            void *o = nullptr;
+            char *o = nullptr;
+            more = 0;
             for (uint32_t q = 0; q < n; q++) {
-                const uint32_t nvec = heldVec[q];
-                if (nvec == 0) {
-                    continue;
-                }
-                if (heldItem[q] != cur) {
-                    cur = heldItem[q];
+                const uint32_t item = __builtin_amdgcn_readfirstlane(heldItem[q]);
+                if (item != cur) {
+                    cur = item;
                     w = items[cur];
-                    o = k < w.ndst ? dstPool[w.dstBase + k] : nullptr;
+                    o = k < w.ndst ? static_cast<char *>(dstPool[w.dstBase + k]) : nullptr;
+                    more |= k + 1 < w.ndst ? 1u : 0u;
                 }
                 if (o == nullptr) {
                     continue;
                 }
-                const uint64_t off = uint64_t(heldTile[q] - w.tile0) * kTileBytes;
-                const LdsV4 *from = park + q * kTeamVecPerTile;
-                if (w.mode == ACC_VEC16) {
-                    if (w.flags & kFusedOrdinaryStores) {
-                        TeamDrain<ACC_VEC16, true>(from, o, off, nvec);
-                    } else {
-                        TeamDrain<ACC_VEC16, false>(from, o, off, nvec);
-                    }
+                char *to = o + uint64_t(reg.first + inTeam + q * teamSize - w.tile0) * kTileBytes;
+                if (w.flags & kFusedOrdinaryStores) {
+                    TeamDrain<STORE_ORDINARY>(park + q * kTeamVecPerTile, to);
                 } else {
-                    TeamDrain<ACC_VEC16_ANY, false>(from, o, off, nvec);
+                    TeamDrain<STORE_STREAMED>(park + q * kTeamVecPerTile, to);
                 }
             }
         }
@@ -299,40 +285,57 @@ __device__ __forceinline__ void TeamBody(const FusedDesc *__restrict__ items, ui
 template <typename T> struct ReadsBySource { static constexpr bool value = true; };
 template <> struct ReadsBySource<Bf16Bits> { static constexpr bool value = false; };
 
-// One register set: N whole tiles of one source, `stride` bytes apart.
+// One register set: N whole tiles of their items' source j.
 template <uint32_t N>
-__device__ __forceinline__ void TeamLoadSet(V4 (&v)[N][kVecPerLane], const void *base, uint64_t off, uint64_t stride)
+__device__ __forceinline__ void TeamLoadSet(V4 (&v)[N][kVecPerLane], const TeamPlaces<N> &at, const void *const *__restrict__ srcPool, uint32_t j)
 {
-    const char *s = static_cast<const char *>(base) + off;
 #pragma unroll
     for (uint32_t q = 0; q < N; q++) {
+        const char *s = static_cast<const char *>(srcPool[at.base[q] + j]) + at.off[q];
 #pragma unroll
         for (uint32_t u = 0; u < kVecPerLane; u++) {
-            v[q][u] = Load16<ACC_VEC16>(s + q * stride + uint64_t(u) * kBlockThreads * 16, threadIdx.x * 16u);
+            v[q][u] = Load16<ACC_VEC16_ANY>(s, (u * kBlockThreads + threadIdx.x) * 16u);
         }
+    }
+}
+template <uint32_t U> __device__ __forceinline__ void TeamPark(LdsV4 *park, uint32_t first, const V4 (&x)[U])
+{
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) {
+        park[(first + u) * kBlockThreads + threadIdx.x] = x[u];
+    }
+}
+
+// Tile by tile, from tile q on: tile(d, off, where the values go) for each.
+template <typename Tile> __device__ __forceinline__ void TeamByTile(const TeamRound &r, uint32_t q, LdsV4 *park, Tile tile)
+{
+    FusedDesc d;
+    uint32_t idx = 0, end = 0;
+    for (; q < r.n; q++) {
+        if (q + 1 == r.n) {
+            // a look at the slot of the next round, in flight together with the last tile's loads: a workgroup
+            // that is behind the others finds the answer there
+            r.Peek();
+        }
+        r.Item(q, d, idx, end);
+        tile(d, uint64_t(r.Tile(q) - d.tile0) * kTileBytes, park + q * kTeamVecPerTile);
     }
 }
 
 template <typename T, int OP> struct TeamChainEval {
-    static constexpr bool kBySource = ReadsBySource<T>::value;
-    static __device__ __forceinline__ bool RoundFits(const FusedDesc &d) { return d.nsrc >= 2; }
     // Source j into the partial results: source 0 starts them.  A tile's partial results are fetched from LDS together,
     // so that their latencies overlap.
     template <uint32_t N>
-    static __device__ __forceinline__ void FoldSet(const V4 (&v)[N][kVecPerLane], const FusedDesc &d, uint32_t j, LdsV4 *park)
+    static __device__ __forceinline__ void FoldSet(const V4 (&v)[N][kVecPerLane], const TeamPlaces<N> &at, uint32_t j, LdsV4 *park)
     {
         const uint32_t tid = threadIdx.x;
         if (j == 0) {
 #pragma unroll
             for (uint32_t q = 0; q < N; q++) {
-#pragma unroll
-                for (uint32_t u = 0; u < kVecPerLane; u++) {
-                    park[q * kTeamVecPerTile + u * kBlockThreads + tid] = v[q][u];
-                }
+                TeamPark(park + q * kTeamVecPerTile, 0, v[q]);
             }
             return;
         }
-        const bool accLeft = OrderMatters<T, OP>::value && ((d.accLeftMask >> j) & 1ull);
 #pragma unroll
         for (uint32_t q = 0; q < N; q++) {
             V4 a[kVecPerLane];
@@ -340,7 +343,7 @@ template <typename T, int OP> struct TeamChainEval {
             for (uint32_t u = 0; u < kVecPerLane; u++) {
                 a[u] = park[q * kTeamVecPerTile + u * kBlockThreads + tid];
             }
-            if (accLeft) {      // the same for the whole wave
+            if (OrderMatters<T, OP>::value && ((at.accLeft[q] >> j) & 1ull)) {      // the same for the whole wave
 #pragma unroll
                 for (uint32_t u = 0; u < kVecPerLane; u++) {
                     a[u] = Combine16<T, OP>(a[u], v[q][u]);
@@ -351,186 +354,166 @@ template <typename T, int OP> struct TeamChainEval {
                     a[u] = Combine16<T, OP>(v[q][u], a[u]);
                 }
             }
-#pragma unroll
-            for (uint32_t u = 0; u < kVecPerLane; u++) {
-                park[q * kTeamVecPerTile + u * kBlockThreads + tid] = a[u];
-            }
+            TeamPark(park + q * kTeamVecPerTile, 0, a);
         }
     }
-    // A whole round at once: N whole tiles of one item, `stride` bytes apart from `off` on.  The team reads source by
-    // source -- at any moment its loads go to one stretch of N x 32 tiles of one buffer instead of 32 tiles of each of
+    // A whole round at once, whichever items its tiles belong to.  The team reads source by source -- at any moment its loads go to one stretch of N x 32 tiles of one buffer instead of 32 tiles of each of
     // the item's buffers -- and the partial results rest in LDS, folded in the chain's order, so the bits are those of
     // the tile-by-tile evaluation.  Two register sets of N x 4 vectors: while one source is folded, the next one's
     // loads are in flight, and the one after that is requested as soon as the fold has freed its set (8 ranks x
     // 256 MiB, stand-alone: 691 us this way, 770 us with one set, 705 us tile by tile).
     // Straight-line code for a source count fixed at compile time, in which every wait is for exactly the loads it
     // needs, measured the same and takes three times as long to build.
-    // `peek` is looked at (thread 0, into *seen) once the last loads are on their way.
     template <uint32_t N>
-    static __device__ __forceinline__ void Round(const FusedDesc &d, const void *const *__restrict__ src, const void *, uint64_t off,
-        uint64_t stride, LdsV4 *park, const uint32_t *peek, uint32_t *seen)
+    static __device__ __forceinline__ void BySource(const TeamRound &r, const void *const *__restrict__ srcPool, LdsV4 *park)
     {
+        FusedDesc d;
+        uint32_t idx = 0, end = 0;
+        TeamPlaces<N> at;
+        at.Find(r, 0, d, idx, end);
         const uint32_t nsrc = d.nsrc;
         V4 va[N][kVecPerLane], vb[N][kVecPerLane];
-        TeamLoadSet<N>(va, src[0], off, stride);
-        TeamLoadSet<N>(vb, src[1], off, stride);
+        TeamLoadSet<N>(va, at, srcPool, 0);
+        TeamLoadSet<N>(vb, at, srcPool, 1);
         uint32_t j = 0;
 #pragma nounroll
         for (; j + 4 <= nsrc; j += 2) {
-            FoldSet<N>(va, d, j, park);
-            TeamLoadSet<N>(va, src[j + 2], off, stride);
-            FoldSet<N>(vb, d, j + 1, park);
-            TeamLoadSet<N>(vb, src[j + 3], off, stride);
+            FoldSet<N>(va, at, j, park);
+            TeamLoadSet<N>(va, at, srcPool, j + 2);
+            FoldSet<N>(vb, at, j + 1, park);
+            TeamLoadSet<N>(vb, at, srcPool, j + 3);
         }
         // two or three sources left, the first two of them loaded or on their way
         const bool three = nsrc - j == 3;
-        FoldSet<N>(va, d, j, park);
+        FoldSet<N>(va, at, j, park);
         if (three) {
-            TeamLoadSet<N>(va, src[j + 2], off, stride);
+            TeamLoadSet<N>(va, at, srcPool, j + 2);
         }
-        if (threadIdx.x == 0) {
-            *seen = TeamLoad(peek);
-        }
-        FoldSet<N>(vb, d, j + 1, park);
+        r.Peek();
+        FoldSet<N>(vb, at, j + 1, park);
         if (three) {
-            FoldSet<N>(va, d, j + 2, park);
+            FoldSet<N>(va, at, j + 2, park);
         }
     }
-    // Up to kChainSrcBatch source pointers are kept in registers from tile to tile: fetched per tile they are a chain
-    // of dependent loads in front of the tile's data, with nothing else on the CU to hide it.
-    const void *sp[kChainSrcBatch];
-    bool few;
-    __device__ __forceinline__ void SetItem(const FusedDesc &d, const void *const *__restrict__ srcPool)
+    static __device__ __forceinline__ void Read(const TeamRound &r, const void *const *__restrict__ srcPool, const void *, LdsV4 *park)
     {
-        few = d.nsrc <= kChainSrcBatch;
+        if constexpr (ReadsBySource<T>::value) {
+            if (r.n >= kTeamTiles / 2 && (r.items[0].flags & kFusedAlike)) {
+                switch (r.n) {
+                    case 4: BySource<4>(r, srcPool, park); break;
+                    case 5: BySource<5>(r, srcPool, park); break;
+                    case 6: BySource<6>(r, srcPool, park); break;
+                    case 7: BySource<7>(r, srcPool, park); break;
+                    default: BySource<8>(r, srcPool, park); break;
+                }
+                return;
+            }
+        }
+        // Up to 8 source pointers are kept in registers from tile to tile: fetched per tile they are a chain
+        // of dependent loads in front of the tile's data, with nothing else on the CU to hide it.
+        const void *sp[8];
+        uint32_t held = ~0u;
+        uint32_t pos[kChainVec];
+        TilePositions(pos);
+        TeamByTile(r, 0, park, [&](const FusedDesc &d, uint64_t off, LdsV4 *to) {
+            V4 acc[kChainVec];
+            if (d.nsrc <= 8) {
+                if (d.srcBase != held) {
+                    held = d.srcBase;
 #pragma unroll
-        for (uint32_t j = 0; j < kChainSrcBatch; j++) {
-            sp[j] = j < d.nsrc ? srcPool[d.srcBase + j] : nullptr;
-        }
-    }
-    template <uint32_t MODE, bool ONE>
-    __device__ __forceinline__ void Passes(const FusedDesc &d, const void *const *__restrict__ src, uint64_t off, uint32_t nvec,
-        LdsV4 *park) const
-    {
-        constexpr uint32_t kPass = kChainVec * kBlockThreads;
-        uint32_t base = 0;
-        for (; base + kPass <= nvec; base += kPass) {
-            ChainVecPass<T, OP, MODE, true, false, true, ONE>(d, src, nullptr, off, base, nvec, park);
-        }
-        if (base < nvec) {
-            ChainVecPass<T, OP, MODE, false, false, true, ONE>(d, src, nullptr, off, base, nvec, park);
-        }
-    }
-    __device__ __forceinline__ void Vec(const FusedDesc &d, const void *const *__restrict__ srcPool, const void *,
-        uint64_t off, uint32_t nvec, LdsV4 *park) const
-    {
-        if (few) {
-            if (d.mode == ACC_VEC16) {
-                Passes<ACC_VEC16, true>(d, sp, off, nvec, park);
+                    for (uint32_t j = 0; j < 8; j++) {
+                        sp[j] = srcPool[d.srcBase + j];       // (the pool is padded)
+                    }
+                }
+                ChainFew<VecLane<T, OP>, T, OP, kChainVec>(d.nsrc, d.accLeftMask, sp, off, pos, acc);
             } else {
-                Passes<ACC_VEC16_ANY, true>(d, sp, off, nvec, park);
+                ChainMany<VecLane<T, OP>, T, OP, kChainVec>(d.nsrc, d.accLeftMask, srcPool + d.srcBase, off, pos, acc);
             }
-        } else {
-            if (d.mode == ACC_VEC16) {
-                Passes<ACC_VEC16, false>(d, srcPool + d.srcBase, off, nvec, park);
-            } else {
-                Passes<ACC_VEC16_ANY, false>(d, srcPool + d.srcBase, off, nvec, park);
-            }
-        }
+            TeamPark(to, 0, acc);
+        });
     }
-    static __device__ __forceinline__ void Elem(const FusedDesc &d, const void *const *__restrict__ srcPool, const void *,
-        void *const *__restrict__ dstPool, uint64_t off, uint32_t n)
+    static __device__ __forceinline__ void Rest(const FusedDesc &d, const void *const *__restrict__ src, const void *, void *const *__restrict__ dst)
     {
-        ChainElem<T, OP>(d, srcPool + d.srcBase, dstPool + d.dstBase, off, n);
+        ChainRest<T, OP>(d, src, dst);
     }
 };
 
 struct TeamCopyEval {
-    static constexpr bool kBySource = true;
-    static __device__ __forceinline__ bool RoundFits(const FusedDesc &) { return true; }
-    // A whole round at once (see TeamChainEval::Round): the loads of all N tiles are issued before the first of them is
-    // parked, instead of tile after tile with an LDS write between them.
-    template <uint32_t N>
-    static __device__ __forceinline__ void Round(const FusedDesc &, const void *const *__restrict__ src, const void *, uint64_t off,
-        uint64_t stride, LdsV4 *park, const uint32_t *peek, uint32_t *seen)
+    // The loads of all tiles are issued before the first of them is parked, instead of tile after tile with an LDS write between them.
+    // A full round whose first source lies off a word boundary is fetched in words (WordVec): all-gather of odd blocks of
+    // 2-byte elements, us, 128-bit loads / words: 8 ranks x 8 MiB 109.4 / 108.0, 16 MiB 211.7 / 207.9; 16 ranks x 8 MiB 380.7 / 371.2.
+    template <uint32_t N, typename L = MoveLane>
+    static __device__ __forceinline__ void Together(const TeamRound &r, const void *const *__restrict__ srcPool, LdsV4 *park)
     {
-        const uint32_t tid = threadIdx.x;
-        const char *s = static_cast<const char *>(src[0]) + off;
-        V4 v[N][kVecPerLane];
+        FusedDesc d;
+        uint32_t idx = 0, end = 0;
+        TeamPlaces<N> at;
+        at.Find(r, 0, d, idx, end);
+        typename L::Raw v[N][kVecPerLane];
 #pragma unroll
         for (uint32_t q = 0; q < N; q++) {
+            const char *s = static_cast<const char *>(srcPool[at.base[q]]) + at.off[q];
 #pragma unroll
             for (uint32_t u = 0; u < kVecPerLane; u++) {
-                v[q][u] = Load16<ACC_VEC16>(s + q * stride + uint64_t(u) * kBlockThreads * 16, tid * 16u);
+                v[q][u] = L::Load(s, (u * kBlockThreads + threadIdx.x) * 16u);
             }
         }
-        if (tid == 0) {
-            *seen = TeamLoad(peek);
-        }
+        r.Peek();
 #pragma unroll
         for (uint32_t q = 0; q < N; q++) {
+            V4 x[kVecPerLane];
 #pragma unroll
             for (uint32_t u = 0; u < kVecPerLane; u++) {
-                park[q * kTeamVecPerTile + u * kBlockThreads + tid] = v[q][u];
+                x[u] = L::Value(v[q][u], srcPool[at.base[q]]);
             }
+            TeamPark(park + q * kTeamVecPerTile, 0, x);
         }
     }
-    const void *s;
-    __device__ __forceinline__ void SetItem(const FusedDesc &d, const void *const *__restrict__ srcPool) { s = srcPool[d.srcBase]; }
-    __device__ __forceinline__ void Vec(const FusedDesc &d, const void *const *__restrict__, const void *, uint64_t off,
-        uint32_t nvec, LdsV4 *park) const
+    static __device__ __forceinline__ void Read(const TeamRound &r, const void *const *__restrict__ srcPool, const void *, LdsV4 *park)
     {
-        constexpr uint32_t kPass = kChainVec * kBlockThreads;
-        uint32_t base = 0;
-        if (d.mode == ACC_VEC16) {
-            for (; base + kPass <= nvec; base += kPass) {
-                CopyVecPass<ACC_VEC16, true, false, true>(s, nullptr, 0, off, base, nvec, park);
-            }
-            if (base < nvec) {
-                CopyVecPass<ACC_VEC16, false, false, true>(s, nullptr, 0, off, base, nvec, park);
-            }
-        } else {
-            for (; base + kPass <= nvec; base += kPass) {
-                CopyVecPass<ACC_VEC16_ANY, true, false, true>(s, nullptr, 0, off, base, nvec, park);
-            }
-            if (base < nvec) {
-                CopyVecPass<ACC_VEC16_ANY, false, false, true>(s, nullptr, 0, off, base, nvec, park);
-            }
+        switch (r.n) {
+            case 1: Together<1>(r, srcPool, park); break;
+            case 2: Together<2>(r, srcPool, park); break;
+            case 3: Together<3>(r, srcPool, park); break;
+            case 4: Together<4>(r, srcPool, park); break;
+            case 5: Together<5>(r, srcPool, park); break;
+            case 6: Together<6>(r, srcPool, park); break;
+            case 7: Together<7>(r, srcPool, park); break;
+            default:
+                if (r.items[ItemOfTile(r.items, r.nitems, r.first, r.tilesPerItem)].flags & kFusedWordSources) {
+                    Together<8, WordLane<uint8_t, ROP_SUM>>(r, srcPool, park);
+                } else {
+                    Together<8>(r, srcPool, park);
+                }
+                break;
         }
     }
-    static __device__ __forceinline__ void Elem(const FusedDesc &d, const void *const *__restrict__ srcPool, const void *,
-        void *const *__restrict__ dstPool, uint64_t off, uint32_t n)
+    static __device__ __forceinline__ void Rest(const FusedDesc &d, const void *const *__restrict__ src, const void *, void *const *__restrict__ dst)
     {
-        const void *s = srcPool[d.srcBase];
-        void *const *dst = dstPool + d.dstBase;
-        for (uint32_t i = threadIdx.x; i < n; i += kBlockThreads) {
-            const uint8_t b = LoadElem<uint8_t>(s, off + i);
-            for (uint32_t k = 0; k < d.ndst; k++) {
-                StoreElem<uint8_t>(dst[k], off + i, b);
-            }
-        }
+        CopyRest(d, src[0], dst);
     }
 };
 
 template <typename T, int OP> struct TeamTreeEval {
-    static constexpr bool kBySource = false;
-    __device__ __forceinline__ void SetItem(const FusedDesc &, const void *const *__restrict__) {}
-    __device__ __forceinline__ void Vec(const FusedDesc &d, const void *const *__restrict__ srcPool, const void *,
-        uint64_t off, uint32_t nvec, LdsV4 *park) const
+    static __device__ __forceinline__ void Read(const TeamRound &r, const void *const *__restrict__ srcPool, const void *, LdsV4 *park)
     {
-        TreeTile<T, OP, true>(d, srcPool + d.srcBase, nullptr, off, nvec, park);
+        uint32_t pos[kChainVec];
+        TilePositions(pos);
+        TeamByTile(r, 0, park, [&](const FusedDesc &d, uint64_t off, LdsV4 *to) {
+            V4 x[kChainVec];
+            TreeValue<VecLane<T, OP>, kChainVec>(d, srcPool + d.srcBase, off, pos, x);
+            TeamPark(to, 0, x);
+        });
     }
-    static __device__ __forceinline__ void Elem(const FusedDesc &d, const void *const *__restrict__ srcPool, const void *,
-        void *const *__restrict__ dstPool, uint64_t off, uint32_t n)
+    static __device__ __forceinline__ void Rest(const FusedDesc &d, const void *const *__restrict__ src, const void *, void *const *__restrict__ dst)
     {
-        TreeElem<T, OP>(d, srcPool + d.srcBase, dstPool + d.dstBase, off, n);
+        TreeRest<T, OP>(d, src, dst);
     }
 };
 
 // extra = the launch's op words (they follow the item table)
 template <typename T, int OP, bool ROUNDS> struct TeamStackEval {
-    static constexpr bool kBySource = ROUNDS && ReadsBySource<T>::value;
-    // A whole round source by source, as the chain's (TeamChainEval::Round), for expressions that never hold more than
+    // A whole round source by source, as the chain's (TeamChainEval::BySource), for expressions that never hold more than
     // two partial results while a source is being read (a chain of chains: the two-level all-reduce): the lower one in
     // LDS, the upper one in registers.  Three sets of eight tiles are more registers than a wave has, so the round goes
     // in halves of four tiles, through one pipeline: the second half's first sources are requested while the first
@@ -540,7 +523,6 @@ template <typename T, int OP, bool ROUNDS> struct TeamStackEval {
     // 200.6 / 183.7, int8 209.5 / 186.8, int32 199.9 / 183.9, uint64 197.4 / 177.6, fp64 194.0 / 177.4, maximum of fp32 226.4 / 191.9.
     // Its registers cost the tiles that are not read this way: 8-byte types and 8-bit products have a kernel without it
     // (ROUNDS) for launches with few such rounds (exec.cc).
-    static __device__ __forceinline__ bool RoundFits(const FusedDesc &d) { return d.nsrc >= 2 && d.nleaf <= 3; }
     static constexpr uint32_t kHalf = kTeamTiles / 2;
     typedef V4 Set[kHalf][kVecPerLane];
     static __device__ __forceinline__ void FoldUpper(Set &v, const Set &under, bool underLeft)
@@ -609,22 +591,46 @@ template <typename T, int OP, bool ROUNDS> struct TeamStackEval {
         }
         depth++;
     }
-    template <uint32_t N>
-    static __device__ __forceinline__ void Round(const FusedDesc &d, const void *const *__restrict__ src, const void *extra,
-        uint64_t off, uint64_t stride, LdsV4 *park, const uint32_t *peek, uint32_t *seen)
+    // The first four tiles of a round, or all eight: each four of one item (one program), and the same number of sources.
+    static __device__ __forceinline__ bool Fits(const TeamRound &r)
     {
-        const uint32_t *ops = static_cast<const uint32_t *>(extra) + d.srcBase;
-        const uint32_t nsrc = d.nsrc, total = nsrc * (N / kHalf);
+        uint32_t nsrc = 0;
+        for (uint32_t q = 0; q + kHalf <= r.n && (q == 0 || r.n == kTeamTiles); q += kHalf) {
+            const FusedDesc d = r.items[ItemOfTile(r.items, r.nitems, r.Tile(q), r.tilesPerItem)];
+            if (d.nsrc < 2 || d.nleaf > 3 || r.Tile(q + kHalf - 1) >= d.tile0 + uint32_t(d.bytes / kTileBytes) || (q != 0 && d.nsrc != nsrc)) {
+                return false;
+            }
+            nsrc = d.nsrc;
+        }
+        return true;
+    }
+    template <uint32_t HALVES>
+    static __device__ __forceinline__ void BySource(const TeamRound &r, const void *const *__restrict__ srcPool, const uint32_t *__restrict__ opPool,
+        LdsV4 *park)
+    {
+        FusedDesc d;
+        uint32_t idx = 0, end = 0;
+        TeamPlaces<kHalf> at[HALVES];
+        uint32_t ops[HALVES];
+#pragma unroll
+        for (uint32_t h = 0; h < HALVES; h++) {
+            at[h].Find(r, h * kHalf, d, idx, end);
+            ops[h] = d.srcBase;
+        }
+        const uint32_t nsrc = d.nsrc, total = nsrc * HALVES;
         Set va, vb, upper;
         uint32_t depth = 0;
         auto load = [&](Set &v, uint32_t j) {
-            const uint32_t half = j >= nsrc ? 1u : 0u;
-            TeamLoadSet<kHalf>(v, src[j - half * nsrc], off + half * kHalf * stride, stride);
+            if (HALVES == 2 && j >= nsrc) {
+                TeamLoadSet<kHalf>(v, at[HALVES - 1], srcPool, j - nsrc);
+            } else {
+                TeamLoadSet<kHalf>(v, at[0], srcPool, j);
+            }
         };
         auto push = [&](Set &v, uint32_t j) {
-            const uint32_t half = j >= nsrc ? 1u : 0u;
+            const uint32_t half = HALVES == 2 && j >= nsrc ? 1u : 0u;
             depth = j == half * nsrc ? 0u : depth;
-            Push(v, ops[j - half * nsrc], upper, park + half * kHalf * kTeamVecPerTile, depth);
+            Push(v, opPool[(half != 0 ? ops[HALVES - 1] : ops[0]) + j - half * nsrc], upper, park + half * kHalf * kTeamVecPerTile, depth);
         };
         load(va, 0);
         load(vb, 1);
@@ -642,26 +648,36 @@ template <typename T, int OP, bool ROUNDS> struct TeamStackEval {
         if (three) {
             load(va, j + 2);
         }
-        if (threadIdx.x == 0) {
-            *seen = TeamLoad(peek);
-        }
+        r.Peek();
         push(vb, j + 1);
         if (three) {
             push(va, j + 2);
         }
     }
-    __device__ __forceinline__ void SetItem(const FusedDesc &, const void *const *__restrict__) {}
-    __device__ __forceinline__ void Vec(const FusedDesc &d, const void *const *__restrict__ srcPool, const void *extra,
-        uint64_t off, uint32_t nvec, LdsV4 *park) const
+    static __device__ __forceinline__ void Read(const TeamRound &r, const void *const *__restrict__ srcPool, const void *extra, LdsV4 *park)
     {
-        const uint32_t *ops = static_cast<const uint32_t *>(extra) + d.srcBase;
-        StackTile<T, OP, true>(d, srcPool + d.srcBase, ops, nullptr, off, nvec, park);
+        const uint32_t *opPool = static_cast<const uint32_t *>(extra);
+        uint32_t q = 0;
+        if constexpr (ROUNDS && ReadsBySource<T>::value) {
+            if (r.n >= kHalf && Fits(r)) {
+                if (r.n == kTeamTiles) {
+                    BySource<2>(r, srcPool, opPool, park);
+                    return;
+                }
+                BySource<1>(r, srcPool, opPool, park);
+                q = kHalf;
+            }
+        }
+        uint32_t pos[kChainVec];
+        TilePositions(pos);
+        TeamByTile(r, q, park, [&](const FusedDesc &d, uint64_t off, LdsV4 *to) {
+            StackTile<T, OP, kStackTeamBatch>(d, srcPool + d.srcBase, opPool + d.srcBase, off, pos,
+                [&](uint32_t h, const auto &x) { TeamPark(to, h, x); });
+        });
     }
-    static __device__ __forceinline__ void Elem(const FusedDesc &d, const void *const *__restrict__ srcPool, const void *extra,
-        void *const *__restrict__ dstPool, uint64_t off, uint32_t n)
+    static __device__ __forceinline__ void Rest(const FusedDesc &d, const void *const *__restrict__ src, const void *extra, void *const *__restrict__ dst)
     {
-        const uint32_t *ops = static_cast<const uint32_t *>(extra) + d.srcBase;
-        StackElem<T, OP>(d, srcPool + d.srcBase, ops, dstPool + d.dstBase, off, n);
+        StackRest<T, OP>(d, src, static_cast<const uint32_t *>(extra) + d.srcBase, dst);
     }
 };
 
@@ -669,35 +685,35 @@ template <typename T, int OP, bool ROUNDS> struct TeamStackEval {
 // kernels.h).  Launched with one workgroup per CU
 // (a multiple of kTeamXcds workgroups) and kTeamDynamicLds bytes of dynamic LDS.
 template <typename T, int OP>
-__global__ void __launch_bounds__(kBlockThreads) TeamChainKernel(const FusedDesc *__restrict__ items, uint32_t nitems,
+__global__ void __launch_bounds__(kBlockThreads) TeamChainKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole,
     uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem,
     uint32_t *__restrict__ teamCtr)
 {
-    TeamBody<TeamChainEval<T, OP>>(items, nitems, ntiles, srcPool, dstPool, tilesPerItem, teamCtr, nullptr);
+    TeamBody<TeamChainEval<T, OP>>(items, nitems, nwhole, ntiles, srcPool, dstPool, tilesPerItem, teamCtr, nullptr);
 }
 
 template <int Variant>
-__global__ void __launch_bounds__(kBlockThreads) TeamCopyKernel(const FusedDesc *__restrict__ items, uint32_t nitems,
+__global__ void __launch_bounds__(kBlockThreads) TeamCopyKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole,
     uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem,
     uint32_t *__restrict__ teamCtr)
 {
-    TeamBody<TeamCopyEval>(items, nitems, ntiles, srcPool, dstPool, tilesPerItem, teamCtr, nullptr);
+    TeamBody<TeamCopyEval>(items, nitems, nwhole, ntiles, srcPool, dstPool, tilesPerItem, teamCtr, nullptr);
 }
 
 template <typename T, int OP>
-__global__ void __launch_bounds__(kBlockThreads) TeamTreeKernel(const FusedDesc *__restrict__ items, uint32_t nitems,
+__global__ void __launch_bounds__(kBlockThreads) TeamTreeKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole,
     uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem,
     uint32_t *__restrict__ teamCtr)
 {
-    TeamBody<TeamTreeEval<T, OP>>(items, nitems, ntiles, srcPool, dstPool, tilesPerItem, teamCtr, nullptr);
+    TeamBody<TeamTreeEval<T, OP>>(items, nitems, nwhole, ntiles, srcPool, dstPool, tilesPerItem, teamCtr, nullptr);
 }
 
 template <typename T, int OP, bool ROUNDS>
-__global__ void __launch_bounds__(kBlockThreads) TeamStackKernel(const FusedDesc *__restrict__ items, uint32_t nitems,
+__global__ void __launch_bounds__(kBlockThreads) TeamStackKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole,
     uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem,
     uint32_t *__restrict__ teamCtr)
 {
-    TeamBody<TeamStackEval<T, OP, ROUNDS>>(items, nitems, ntiles, srcPool, dstPool, tilesPerItem, teamCtr, items + nitems);
+    TeamBody<TeamStackEval<T, OP, ROUNDS>>(items, nitems, nwhole, ntiles, srcPool, dstPool, tilesPerItem, teamCtr, items + nitems + (ntiles - nwhole));
 }
 
 }  // namespace hcclamd

@@ -62,7 +62,7 @@ struct LaunchRec {
     uint32_t grid = 0;
     uint32_t dynamicLds = 0;      // bytes of dynamic LDS the launch asks for (team kernels)
     // kernel arguments: step kernels take (table, nitems, nwhole, ntiles, flags), fused kernels
-    // (table, nitems, ntiles, srcPool, dstPool, tilesPerItem), their team forms one more: (..., teamCtr)
+    // (table, nitems, nwhole, ntiles, srcPool, dstPool, tilesPerItem), their team forms one more: (..., teamCtr)
     const void *table = nullptr;
     uint32_t nitems = 0;
     uint32_t ntiles = 0;
@@ -70,7 +70,7 @@ struct LaunchRec {
     uint32_t flags = 0;
     const void *srcPool = nullptr;
     const void *dstPool = nullptr;
-    uint32_t tilesPerItem = 0;    // fused: every item covers this many tiles (the last at most as many); 0 = they differ
+    uint32_t tilesPerItem = 0;    // fused: every item of whole tiles covers this many (the last at most as many); 0 = they differ
     void *teamCtr = nullptr;      // team kernels: this launch's team block inside the prepared tables (counters, regions, slots)
     uint32_t roundTiles = 0;      // team kernels: tiles per workgroup in a full-size region
     bool fusedArgs = false;

@@ -53,12 +53,12 @@ extern "C" {
  *                                or all walk forwards
  *   "fused_stores"  "auto" | "nt" | "ordinary"   store kind of the fused kernels: non-temporal, or write-back, which
  *                                keeps a result of up to 256 MB in the memory-side cache for whoever reads it next; "auto"
- *                                (default): non-temporal, except write-back for pure data movement from one source to four
- *                                or more destinations with more than 512 MB of output (all-gather, broadcast)
+ *                                (default): non-temporal, and written through the L2 cache where many sources become one result
  *   "team"          "auto" | "0" | "1"   team form of the fused kernels: the workgroups of one XCD read their tiles together,
  *                                hold the results in LDS and write them together, which this memory system serves faster
- *                                than reads and writes interleaved; "auto" (default): for launches of at least two full
- *                                rounds, one where data is only moved, whose items write four or more destinations and touch
+ *                                than reads and writes interleaved; "auto" (default): for launches of at least half a
+ *                                round, a whole one where data is only moved and four where items touch fewer than twelve buffers, whose
+ *                                items write four or more destinations and touch
  *                                eight or more buffers (all-reduce, all-gather, broadcast); "1": wherever the device allows it; "0": never
  *   "team_tiles"    tiles of 16 KiB a workgroup of a team kernel takes per round, 1 ... 8 ("0", default: 8, fewer when an
  *                                item has more than 8 sources or destinations)

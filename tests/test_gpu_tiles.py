@@ -1,0 +1,115 @@
+"""Whole tiles and what is left behind them: rounds of one to eight tiles of a team, borders between items inside a round,
+pieces shorter than a tile, element-wise ends of every number of sources, blocks of which only the sources or only the
+destinations lie on a 16-byte boundary.  Against the CPU checker, bit for bit; bytes around the results untouched."""
+import numpy as np
+import pytest
+import torch
+
+import closed_forms as cf
+import gpu_harness as gh
+from closed_forms import BF16, FP16, FP32, INT8, INT64, MAX, MIN, PROD, SUM, UINT8
+
+pytestmark = pytest.mark.gpu
+H = gh.H
+TILE = 16384
+
+
+@pytest.fixture(scope="module")
+def orc():
+    from oracle import oracle
+    oracle.build()
+    return oracle
+
+
+def _ins(dt, p, n, seed):
+    rng = np.random.default_rng(seed)
+    return [cf.random_input(dt, n, rng) for _ in range(p)]
+
+
+@pytest.mark.parametrize("dt,op,algo,servers", [(FP32, SUM, "ring", 1), (FP16, MAX, "ring", 1), (INT8, PROD, "ring", 1), (BF16, SUM, "rhd", 1), (FP32, MIN, "auto", 2)])
+def test_rounds_of_one_to_eight_tiles(orc, dt, op, algo, servers):
+    # 8 ranks: n tiles for each of 256 workgroups make one round; slices of odd lengths put item borders inside it
+    p = 8
+    g = gh.Group(p, algo=algo, servers=servers, team=1)
+    try:
+        for tiles in (1, 2, 3, 4, 5, 6, 7, 8, 9):
+            n = (256 * tiles * TILE - 37 * TILE) // H.DTYPE_SIZE[dt] + 5
+            print("round of", tiles, "type", dt, "op", op, algo, flush=True)
+            ins = _ins(dt, p, n, 9800 + tiles)
+            if servers == 2:
+                want = orc.allreduce_two_level(ins, dt, op, 2, level1=orc.RHD, atomic=True, threads=8)
+            else:
+                want = orc.allreduce([x.copy() for x in ins], dt, op, algo={"ring": 0, "rhd": 2}[algo], threads=8)
+            outs, _ = gh.all_reduce(g, ins, dt, op, pad=6 if dt == FP16 else 0)
+            assert g.info()["teamLaunches"] >= 1
+            for r in range(p):
+                assert gh.same(dt, outs[r], want[r]), (tiles, r)
+    finally:
+        g.close()
+
+
+@pytest.mark.parametrize("p", [8, 3])
+def test_gathered_rounds(p):
+    # one source, many destinations: blocks that start at every byte
+    g = gh.Group(p, algo="ring", team=1)
+    try:
+        for tiles in (1, 2, 4, 7, 8, 9):
+            n = 256 * tiles * TILE // p + 1001
+            print("gathered rounds", p, tiles, n, flush=True)
+            ins = _ins(INT8, p, n, 9900 + tiles)
+            outs = gh.all_gather(g, ins, INT8)
+            assert g.info()["teamLaunches"] >= 1
+            want = np.concatenate(ins)
+            for r in range(p):
+                assert np.array_equal(outs[r], want), (tiles, r)
+    finally:
+        g.close()
+
+
+@pytest.mark.parametrize("dt,op", [(FP32, MIN), (BF16, MAX), (INT8, SUM), (UINT8, MAX), (INT64, PROD), (FP16, SUM)])
+def test_short_blocks_of_any_number_of_sources(orc, dt, op):
+    # element-wise ends, pieces of less and more than a vector per lane, both chain kernels (results with one destination and
+    # with several), trees with and without second sources
+    for p in (2, 3, 5, 7, 8, 9, 11, 12, 13, 16, 17, 24, 32):
+        for algo in ("ring", "rhd"):
+            g = gh.Group(p, algo=algo, team=0, direct=0)
+            try:
+                for n in (1, 7, 61, 1021, 5003, 20011):
+                    print("short blocks", dt, op, p, algo, n, flush=True)
+                    ins = _ins(dt, p, n * p, 9100 + n)
+                    want = orc.reducescatter(ins, dt, op, algo={"ring": 0, "rhd": 2}[algo])
+                    outs, _ = gh.reduce_scatter(g, ins, dt, op)
+                    for r in range(p):
+                        assert gh.same(dt, outs[r], want[r]), (p, algo, n, r)
+                    ins = _ins(dt, p, n, 9200 + n)
+                    want = orc.allreduce([x.copy() for x in ins], dt, op, algo={"ring": 0, "rhd": 2}[algo])
+                    outs, _ = gh.all_reduce(g, ins, dt, op)
+                    for r in range(p):
+                        assert gh.same(dt, outs[r], want[r]), (p, algo, n, r)
+            finally:
+                g.close()
+
+
+@pytest.mark.parametrize("team", [0, 1])
+@pytest.mark.parametrize("dt,op,offsets", [(FP16, MAX, (0, 2, 2, 2, 6, 0)), (INT8, SUM, (1, 1, 1, 3, 0, 5)), (FP32, SUM, (4, 0, 0, 0, 8, 12)), (BF16, SUM, (2, 4, 6, 8, 10, 12))])
+def test_buffers_at_different_offsets(orc, dt, op, offsets, team):
+    # the pointers of an item agree in part, or not at all
+    p, unit = len(offsets), H.DTYPE_SIZE[dt]
+    g = gh.Group(p, algo="ring", team=team, direct=0)
+    try:
+        for n in (3, 6 * TILE // unit + 11, 50 * TILE // unit + 3):
+            print("offsets", dt, op, team, n, flush=True)
+            ins = _ins(dt, p, n, 9300 + n)
+            want = orc.allreduce([x.copy() for x in ins], dt, op)
+            sends = [gh.to_dev(x, 16 + o) for x, o in zip(ins, offsets)]
+            whole = [torch.full((n * unit + 64,), 0xA5, dtype=torch.uint8, device="cuda") for _ in ins]
+            at = [16 + offsets[(r + 2) % p] for r in range(p)]
+            torch.cuda.synchronize()
+            H.all_reduce(g.comms, [t.data_ptr() for t in sends], [t.data_ptr() + at[r] for r, t in enumerate(whole)], n, dt, op, g.stream_ptr)
+            g.stream.synchronize()
+            for r in range(p):
+                t = whole[r]
+                assert gh.same(dt, gh.to_host(t[at[r]:at[r] + n * unit].clone(), dt), want[r]), (n, r)
+                assert bool((t[:at[r]] == 0xA5).all()) and bool((t[at[r] + n * unit:] == 0xA5).all()), (n, r)
+    finally:
+        g.close()

@@ -594,6 +594,10 @@ template <int OP> struct OrderMatters<Bf16Bits, OP> { static constexpr bool valu
 template <typename T, int OP> struct VecLane {
     typedef V4 Val;
     typedef V4 Raw;
+    typedef V4 Out;
+    typedef VecLane Exact;
+    static constexpr bool kChecked = false;      // Combine gives the same bits as Elem for every operand
+    static __device__ __forceinline__ Out Result(const Val &v) { return v; }
     static __device__ __forceinline__ Raw Load(const void *base, uint32_t pos) { return Load16<ACC_VEC16_ANY>(base, pos); }
     static __device__ __forceinline__ Val Value(const Raw &r, const void *) { return r; }
     static __device__ __forceinline__ void Store(void *base, uint32_t pos, Val v) { StoreAny16(base, pos, v); }
@@ -602,6 +606,10 @@ template <typename T, int OP> struct VecLane {
 template <typename T, int OP> struct WordLane {
     typedef V4 Val;
     typedef WordVec Raw;
+    typedef V4 Out;
+    typedef WordLane Exact;
+    static constexpr bool kChecked = false;
+    static __device__ __forceinline__ Out Result(const Val &v) { return v; }
     static __device__ __forceinline__ uint32_t Shift(const void *base) { return uint32_t(reinterpret_cast<uintptr_t>(base)) & 3u; }
     static __device__ __forceinline__ Raw Load(const void *base, uint32_t pos)
     {
@@ -615,11 +623,118 @@ template <typename T, int OP> struct WordLane {
 template <typename T, int OP> struct ElemLane {
     typedef T Val;
     typedef T Raw;
+    typedef T Out;
+    typedef ElemLane Exact;
+    static constexpr bool kChecked = false;
+    static __device__ __forceinline__ Out Result(const Val &v) { return v; }
     static __device__ __forceinline__ Raw Load(const void *base, uint32_t pos) { return LoadElem<T>(base, pos); }
     static __device__ __forceinline__ Val Value(const Raw &r, const void *) { return r; }
     static __device__ __forceinline__ void Store(void *base, uint32_t pos, Val v) { StoreElem<T>(base, pos, v); }
     static __device__ __forceinline__ Val Combine(Val a, Val b) { return Elem<T, OP>::Apply(a, b); }
 };
+
+// How a chain folds 16 bytes.  Most types: VecLane.  Where a combine takes several instructions per word because elements have
+// to be taken apart and put together again, the value is kept apart from the first source to the last (instructions per word and
+// source: 8-bit 3 instead of 6 to 11; bf16 max / min 3 or 2 instead of 9; fp16 max / min 1 or half a one instead of 5).
+template <typename T, int OP> struct FoldLane : VecLane<T, OP> {};
+
+struct SplitVec { V4 a, b; };
+
+// 8-bit: the even and the odd bytes each in 16-bit lanes.  Sum and product only look at the low byte of a lane, max and min
+// are decided by the high byte: what else a lane holds does not matter, so nothing is masked.
+template <bool SIGNED, int OP> struct ByteLane {
+    typedef SplitVec Val;
+    typedef V4 Raw;
+    typedef V4 Out;
+    typedef ByteLane Exact;
+    static constexpr bool kChecked = false;
+    static constexpr bool kHigh = OP == ROP_MAX || OP == ROP_MIN;
+    static __device__ __forceinline__ Raw Load(const void *base, uint32_t pos) { return Load16<ACC_VEC16_ANY>(base, pos); }
+    static __device__ __forceinline__ Val Value(const Raw &r, const void *) { return kHigh ? Val{r << 8, r} : Val{r, r >> 8}; }
+    static __device__ __forceinline__ V4 Each(V4 x, V4 y)
+    {
+        return V4{Pk16<SIGNED, OP>(x.x, y.x), Pk16<SIGNED, OP>(x.y, y.y), Pk16<SIGNED, OP>(x.z, y.z), Pk16<SIGNED, OP>(x.w, y.w)};
+    }
+    static __device__ __forceinline__ Val Combine(const Val &x, const Val &y) { return Val{Each(x.a, y.a), Each(x.b, y.b)}; }
+    static __device__ __forceinline__ uint32_t Join(uint32_t even, uint32_t odd)
+    {
+        // bytes of the first operand are 4 ... 7 of the selector, of the second 0 ... 3
+        return kHigh ? __builtin_amdgcn_perm(odd, even, 0x07030501u) : __builtin_amdgcn_perm(odd, even, 0x06020400u);
+    }
+    static __device__ __forceinline__ Out Result(const Val &v)
+    {
+        return V4{Join(v.a.x, v.b.x), Join(v.a.y, v.b.y), Join(v.a.z, v.b.z), Join(v.a.w, v.b.w)};
+    }
+};
+template <int OP> struct FoldLane<int8_t, OP> : ByteLane<true, OP> {};
+template <int OP> struct FoldLane<uint8_t, OP> : ByteLane<false, OP> {};
+
+// Max / min of 16-bit floats by the instructions that hand a NaN on (v_maximum3 / v_minimum3).  The selection rule
+// ((b > a) ? b : a in the schedule's order) gives the same bits unless a source is a NaN or the result is a zero, whose sign the
+// rule decides: Special(result) tells, and the sources, still in registers, are then folded by the rule.
+// `most` collects the largest of (magnitude - 1) per half: a zero or a NaN is above `limit`.
+template <uint32_t INF> struct SpecialHalves {
+    uint32_t most = 0;
+    __device__ __forceinline__ void See(uint32_t w)
+    {
+        const U2 below = BitCast<U2>(w & 0x7fff7fffu) - U2{1, 1};
+        most = BitCast<uint32_t>(__builtin_elementwise_max(BitCast<U2>(most), below));
+    }
+    __device__ __forceinline__ void See(V4 v)
+    {
+        See(v.x);
+        See(v.y);
+        See(v.z);
+        See(v.w);
+    }
+    __device__ __forceinline__ bool Any() const { return (most & 0xffffu) >= INF || (most >> 16) >= INF; }
+};
+template <int OP> struct HalfMaxLane {
+    typedef V4 Val;
+    typedef V4 Raw;
+    typedef V4 Out;
+    typedef VecLane<HalfBits, OP> Exact;
+    typedef SpecialHalves<0x7c00u> Special;
+    static constexpr bool kChecked = true;
+    static __device__ __forceinline__ Raw Load(const void *base, uint32_t pos) { return Load16<ACC_VEC16_ANY>(base, pos); }
+    static __device__ __forceinline__ Val Value(const Raw &r, const void *) { return r; }
+    static __device__ __forceinline__ uint32_t Each(uint32_t x, uint32_t y)
+    {
+        const H2 a = BitCast<H2>(x), b = BitCast<H2>(y);
+        return BitCast<uint32_t>(OP == ROP_MAX ? __builtin_elementwise_maximum(a, b) : __builtin_elementwise_minimum(a, b));
+    }
+    static __device__ __forceinline__ Val Combine(V4 x, V4 y) { return V4{Each(x.x, y.x), Each(x.y, y.y), Each(x.z, y.z), Each(x.w, y.w)}; }
+    static __device__ __forceinline__ Out Result(const Val &v) { return v; }
+};
+template <> struct FoldLane<HalfBits, ROP_MAX> : HalfMaxLane<ROP_MAX> {};
+template <> struct FoldLane<HalfBits, ROP_MIN> : HalfMaxLane<ROP_MIN> {};
+
+// bf16: the upper element as the fp32 that the whole word is (the lower element hangs on as low mantissa bits, which only
+// decide between equal upper elements; an infinity becomes a NaN by them, and is then told as one), the lower one shifted up.
+template <int OP> struct Bf16MaxLane {
+    typedef SplitVec Val;
+    typedef V4 Raw;
+    typedef V4 Out;
+    typedef VecLane<Bf16Bits, OP> Exact;
+    typedef SpecialHalves<0x7f80u> Special;
+    static constexpr bool kChecked = true;
+    static __device__ __forceinline__ Raw Load(const void *base, uint32_t pos) { return Load16<ACC_VEC16_ANY>(base, pos); }
+    static __device__ __forceinline__ Val Value(const Raw &r, const void *) { return Val{r, r << 16}; }
+    static __device__ __forceinline__ uint32_t Each(uint32_t x, uint32_t y)
+    {
+        const float a = __uint_as_float(x), b = __uint_as_float(y);
+        return __float_as_uint(OP == ROP_MAX ? __builtin_elementwise_maximum(a, b) : __builtin_elementwise_minimum(a, b));
+    }
+    static __device__ __forceinline__ V4 Each(V4 x, V4 y) { return V4{Each(x.x, y.x), Each(x.y, y.y), Each(x.z, y.z), Each(x.w, y.w)}; }
+    static __device__ __forceinline__ Val Combine(const Val &x, const Val &y) { return Val{Each(x.a, y.a), Each(x.b, y.b)}; }
+    static __device__ __forceinline__ uint32_t Join(uint32_t upper, uint32_t lower) { return __builtin_amdgcn_perm(upper, lower, 0x07060302u); }
+    static __device__ __forceinline__ Out Result(const Val &v)
+    {
+        return V4{Join(v.a.x, v.b.x), Join(v.a.y, v.b.y), Join(v.a.z, v.b.z), Join(v.a.w, v.b.w)};
+    }
+};
+template <> struct FoldLane<Bf16Bits, ROP_MAX> : Bf16MaxLane<ROP_MAX> {};
+template <> struct FoldLane<Bf16Bits, ROP_MIN> : Bf16MaxLane<ROP_MIN> {};
 
 // Keeps the compiler from moving memory accesses over this point (it sinks loads to their first use otherwise).
 __device__ __forceinline__ void PinAccesses() { asm volatile("" ::: "memory"); }
@@ -732,7 +847,7 @@ __device__ __forceinline__ void ChainFold(const void *const *__restrict__ src, c
             for (uint32_t u = 0; u < U; u++) {
                 acc[u] = L::Value(v[0][u], src[0]);
             }
-        } else if (OrderMatters<T, OP>::value && ((accLeft >> j) & 1ull)) {
+        } else if (OrderMatters<T, OP>::value && !L::kChecked && ((accLeft >> j) & 1ull)) {
             // the flag is the same for the whole wave: a branch, not both results and a select per element
 #pragma unroll
             for (uint32_t u = 0; u < U; u++) {
@@ -756,6 +871,13 @@ __device__ __forceinline__ void ChainBatch(const void *const *__restrict__ src, 
 }
 
 // Makes what comes after it wait for these values.
+template <uint32_t U> __device__ __forceinline__ void HoldBack(SplitVec (&x)[U])
+{
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) {
+        asm volatile("" : "+v"(x[u].a), "+v"(x[u].b)::"memory");
+    }
+}
 template <uint32_t U> __device__ __forceinline__ void HoldBack(V4 (&x)[U])
 {
 #pragma unroll
@@ -764,29 +886,58 @@ template <uint32_t U> __device__ __forceinline__ void HoldBack(V4 (&x)[U])
     }
 }
 
+template <typename L, uint32_t U> __device__ __forceinline__ void ChainResult(const typename L::Val (&acc)[U], typename L::Out (&x)[U])
+{
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) {
+        x[u] = L::Result(acc[u]);
+    }
+}
+template <typename L, typename T, int OP, uint32_t N, uint32_t U>
+__device__ __forceinline__ void ChainWhole(const void *const *__restrict__ src, uint64_t off, const uint32_t (&at)[U], uint64_t accLeft,
+    typename L::Out (&x)[U])
+{
+    typename L::Raw v[N][U];
+    typename L::Val acc[U];
+    ChainLoad<L, N, U>(src, off, at, v);
+    ChainFold<L, T, OP, N, U, true>(src, v, accLeft, acc);
+    ChainResult<L, U>(acc, x);
+    if constexpr (L::kChecked && N > 1) {
+        typename L::Special special;
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) {
+            special.See(x[u]);
+        }
+        if (__any(special.Any())) {
+            ChainFold<typename L::Exact, T, OP, N, U, true>(src, v, accLeft, x);
+        }
+    }
+}
+
 // The chain's value at U positions of a lane, `off` behind the item's pointers: up to 8 sources, all in flight together (src is
 // only indexed with constants: a caller may keep the pointers in registers).
 template <typename L, typename T, int OP, uint32_t U>
 __device__ __forceinline__ void ChainFew(uint32_t nsrc, uint64_t accLeft, const void *const *__restrict__ src, uint64_t off, const uint32_t (&at)[U],
-    typename L::Val (&acc)[U])
+    typename L::Out (&x)[U])
 {
     switch (nsrc) {
-        case 1: ChainBatch<L, T, OP, 1, U, true>(src, off, at, accLeft, acc); break;
-        case 2: ChainBatch<L, T, OP, 2, U, true>(src, off, at, accLeft, acc); break;
-        case 3: ChainBatch<L, T, OP, 3, U, true>(src, off, at, accLeft, acc); break;
-        case 4: ChainBatch<L, T, OP, 4, U, true>(src, off, at, accLeft, acc); break;
-        case 5: ChainBatch<L, T, OP, 5, U, true>(src, off, at, accLeft, acc); break;
-        case 6: ChainBatch<L, T, OP, 6, U, true>(src, off, at, accLeft, acc); break;
-        case 7: ChainBatch<L, T, OP, 7, U, true>(src, off, at, accLeft, acc); break;
-        default: ChainBatch<L, T, OP, 8, U, true>(src, off, at, accLeft, acc); break;
+        case 1: ChainWhole<L, T, OP, 1, U>(src, off, at, accLeft, x); break;
+        case 2: ChainWhole<L, T, OP, 2, U>(src, off, at, accLeft, x); break;
+        case 3: ChainWhole<L, T, OP, 3, U>(src, off, at, accLeft, x); break;
+        case 4: ChainWhole<L, T, OP, 4, U>(src, off, at, accLeft, x); break;
+        case 5: ChainWhole<L, T, OP, 5, U>(src, off, at, accLeft, x); break;
+        case 6: ChainWhole<L, T, OP, 6, U>(src, off, at, accLeft, x); break;
+        case 7: ChainWhole<L, T, OP, 7, U>(src, off, at, accLeft, x); break;
+        default: ChainWhole<L, T, OP, 8, U>(src, off, at, accLeft, x); break;
     }
 }
 // More than 8 sources: two sets of 4, one in flight while the other is folded.
 template <typename L, typename T, int OP, uint32_t U>
 __device__ __forceinline__ void ChainMany(uint32_t nsrc, uint64_t accLeft, const void *const *__restrict__ src, uint64_t off, const uint32_t (&at)[U],
-    typename L::Val (&acc)[U])
+    typename L::Out (&x)[U])
 {
     constexpr uint32_t N = 4;
+    typename L::Val acc[U];
     typename L::Raw va[N][U], vb[N][U];
     ChainLoad<L, N, U>(src, off, at, va);
     ChainLoad<L, N, U>(src + N, off, at, vb);
@@ -814,26 +965,29 @@ __device__ __forceinline__ void ChainMany(uint32_t nsrc, uint64_t accLeft, const
         case 3: ChainBatch<L, T, OP, 3, U, false>(src + j, off, at, accLeft >> j, acc); break;
         default: break;
     }
+    ChainResult<L, U>(acc, x);
 }
 template <typename L, typename T, int OP, uint32_t U>
 __device__ __forceinline__ void ChainValue(const FusedDesc &d, const void *const *__restrict__ src, uint64_t off, const uint32_t (&at)[U],
-    typename L::Val (&acc)[U])
+    typename L::Out (&x)[U])
 {
     if (d.nsrc <= 8) {
-        ChainFew<L, T, OP, U>(d.nsrc, d.accLeftMask, src, off, at, acc);
+        ChainFew<L, T, OP, U>(d.nsrc, d.accLeftMask, src, off, at, x);
     } else {
-        ChainMany<L, T, OP, U>(d.nsrc, d.accLeftMask, src, off, at, acc);
+        ChainMany<typename L::Exact, T, OP, U>(d.nsrc, d.accLeftMask, src, off, at, x);
     }
 }
 // The same with two sources in flight at a time: a source is requested when the one two before it is folded.
 template <typename L, typename T, int OP, uint32_t U>
 __device__ __forceinline__ void ChainSlow(const FusedDesc &d, const void *const *__restrict__ src, uint64_t off, const uint32_t (&at)[U],
-    typename L::Val (&acc)[U])
+    typename L::Out (&x)[U])
 {
     const uint32_t nsrc = d.nsrc;
     const uint64_t accLeft = d.accLeftMask;
+    typename L::Val acc[U];
     if (nsrc == 1) {
         ChainBatch<L, T, OP, 1, U, true>(src, off, at, accLeft, acc);
+        ChainResult<L, U>(acc, x);
         return;
     }
     typename L::Raw va[1][U], vb[1][U];
@@ -858,26 +1012,23 @@ __device__ __forceinline__ void ChainSlow(const FusedDesc &d, const void *const 
     } else {
         ChainFold<L, T, OP, 1, U, false>(src + j, vb, accLeft >> j, acc);
     }
+    ChainResult<L, U>(acc, x);
 }
 
 // U vectors per lane of a tile, or of a piece of `nbytes` (a multiple of 16).
 template <typename T, int OP, bool WHOLE, bool SLOW, uint32_t U>
 __device__ __forceinline__ void ChainTile(const FusedDesc &d, const void *const *__restrict__ src, void *const *__restrict__ dst, uint64_t off, uint32_t nbytes)
 {
-    typedef VecLane<T, OP> Vec;
+    typedef FoldLane<T, OP> Vec;
     typedef WordLane<T, OP> Words;
     uint32_t pos[U], at[U];
     V4 acc[U];
     TilePositions(pos);
     ReadPositions(pos, WHOLE ? kTileBytes : nbytes, at);
     if (sizeof(T) == 1 && (d.flags & kFusedWordSources)) {
-        if (SLOW) {
-            ChainSlow<Words, T, OP, U>(d, src, off, at, acc);
-        } else {
-            ChainValue<Words, T, OP, U>(d, src, off, at, acc);
-        }
+        ChainSlow<Words, T, OP, U>(d, src, off, at, acc);     // (all in flight takes more registers than there are)
     } else if (SLOW) {
-        ChainSlow<Vec, T, OP, U>(d, src, off, at, acc);
+        ChainSlow<typename Vec::Exact, T, OP, U>(d, src, off, at, acc);
     } else {
         ChainValue<Vec, T, OP, U>(d, src, off, at, acc);
     }
@@ -911,10 +1062,10 @@ __device__ __forceinline__ void ChainRest(const FusedDesc &d, const void *const 
 // ranks, fp32, 2 MiB per rank 7.3 / 7.3 / 7.5, 6 MiB 20.1 / 17.5 / 18.9, 8 MiB 23.9 / 22.2 / 23.9; reduce-scatter, 8 ranks, fp32, blocks of 8 MiB
 // 97.0 / 101.0 / 98.6, 16 MiB 192.7 / 200.1 / 190.8; 16 ranks, bf16 maximum, 512 KiB 27.6 / 25.4 / 23.7, 16 MiB 777 / 767 / 755.
 // SLOW = false has all loads of a tile in flight, the shortest way through a tile, for results with several
-// destinations.  SLOW = true has two sources' in flight and 70 registers instead of 170: many sources into one destination
+// destinations; two workgroups have to fit a CU (a launch has up to two for each).  SLOW = true has two sources' in flight and 70 registers instead of 170: many sources into one destination
 // run better on more workgroups that ask for less each.
 template <typename T, int OP, bool SLOW>
-__global__ void __launch_bounds__(kBlockThreads) ChainKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole,
+__global__ void __launch_bounds__(kBlockThreads, 2) ChainKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole,
     uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem)
 {
     WalkTiles(items, nitems, nwhole, ntiles, tilesPerItem, [](const FusedDesc &) { return 0; },

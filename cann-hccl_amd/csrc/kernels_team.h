@@ -397,7 +397,7 @@ template <typename T, int OP> struct TeamChainEval {
     }
     static __device__ __forceinline__ void Read(const TeamRound &r, const void *const *__restrict__ srcPool, const void *, LdsV4 *park)
     {
-        if constexpr (ReadsBySource<T>::value) {
+        if constexpr (ReadsBySource<T>::value && sizeof(T) != 1 && !FoldLane<T, OP>::kChecked) {    // (those fold in registers, see FoldLane)
             if (r.n >= kTeamTiles / 2 && (r.items[0].flags & kFusedAlike)) {
                 switch (r.n) {
                     case 4: BySource<4>(r, srcPool, park); break;
@@ -425,9 +425,9 @@ template <typename T, int OP> struct TeamChainEval {
                         sp[j] = srcPool[d.srcBase + j];       // (the pool is padded)
                     }
                 }
-                ChainFew<VecLane<T, OP>, T, OP, kChainVec>(d.nsrc, d.accLeftMask, sp, off, pos, acc);
+                ChainFew<FoldLane<T, OP>, T, OP, kChainVec>(d.nsrc, d.accLeftMask, sp, off, pos, acc);
             } else {
-                ChainMany<VecLane<T, OP>, T, OP, kChainVec>(d.nsrc, d.accLeftMask, srcPool + d.srcBase, off, pos, acc);
+                ChainMany<typename FoldLane<T, OP>::Exact, T, OP, kChainVec>(d.nsrc, d.accLeftMask, srcPool + d.srcBase, off, pos, acc);
             }
             TeamPark(to, 0, acc);
         });

@@ -113,3 +113,31 @@ def test_buffers_at_different_offsets(orc, dt, op, offsets, team):
                 assert bool((t[:at[r]] == 0xA5).all()) and bool((t[at[r] + n * unit:] == 0xA5).all()), (n, r)
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("dt,op", [(FP16, MAX), (FP16, MIN), (BF16, MAX), (BF16, MIN)])
+@pytest.mark.parametrize("p,team", [(8, 0), (8, 1), (5, 0), (2, 1), (12, 0)])
+def test_half_selection_over_every_bit_pattern(orc, dt, op, p, team):
+    # NaNs of every payload, both zeros, infinities, denormals: most waves see one, some results are zeros of either sign
+    g = gh.Group(p, algo="ring", team=team, direct=0)
+    try:
+        for n, kind in ((70001, "any"), (70001, "zeros"), (300007, "rare")):
+            print("selection", dt, op, p, team, n, kind, flush=True)
+            rng = np.random.default_rng(9400 + n + p)
+            ins = []
+            for r in range(p):
+                if kind == "any":
+                    x = rng.integers(0, 1 << 16, n, dtype=np.uint16)
+                elif kind == "zeros":
+                    x = rng.choice(np.array([0x0000, 0x8000, 0x0001, 0x8001, 0x3c00 if op == MIN else 0xbc00], np.uint16), n)
+                else:
+                    x = cf.random_input(dt, n, rng)
+                    x[rng.integers(0, n, 5)] = rng.choice(np.array([0x7fc1, 0xffff, 0x7c01, 0x7f81, 0x0000, 0x8000, 0x7f80, 0xff80, 0x7c00, 0xfc00], np.uint16), 5)
+                ins.append(x)
+            want = orc.allreduce([x.copy() for x in ins], dt, op)
+            for in_place in (False, True):
+                outs, _ = gh.all_reduce(g, ins, dt, op, in_place=in_place)
+                for r in range(p):
+                    assert np.array_equal(outs[r].view(np.uint16), want[r].view(np.uint16)), (kind, in_place, r)
+    finally:
+        g.close()

@@ -1,6 +1,7 @@
 // Behind the C ABI: argument checks (framework/common/src/param_check.cc), settings read from the environment and from
 // HcclCommConfig, the registry of groups, and the rendezvous of the ranks' calls -- a rank arrives, the last one issues
 // the collective; sends meet their receives.
+#include <algorithm>
 #include <chrono>
 #include <cstdlib>
 #include <cstring>
@@ -346,15 +347,25 @@ HcclResult Arrive(Comm *c, const OpSig &sig, void *send, void *recv, hipStream_t
         }
     }
     if (sig.coll == COLL_ALLTOALLV) {
-        size_t p = g->p;
-        g->pend.sendCounts.resize(p * p);
-        g->pend.sdispls.resize(p * p);
-        g->pend.recvCounts.resize(p * p);
-        g->pend.rdispls.resize(p * p);
-        std::copy(sendCounts, sendCounts + p, g->pend.sendCounts.begin() + r * p);
-        std::copy(sdispls, sdispls + p, g->pend.sdispls.begin() + r * p);
-        std::copy(recvCounts, recvCounts + p, g->pend.recvCounts.begin() + r * p);
-        std::copy(rdispls, rdispls + p, g->pend.rdispls.begin() + r * p);
+        // The tables stay from call to call.  A row that is what this rank passed the last time is compared and not copied, and
+        // if every rank's rows are, what was found out about the tables (checked, prepared) holds: a repeated call of 64 ranks then
+        // reads its 128 KiB once, instead of copying, checking, hashing and comparing them.
+        const size_t p = g->p;
+        const uint64_t *rows[4] = {sendCounts, sdispls, recvCounts, rdispls};
+        std::vector<uint64_t> *tables[4] = {&g->pend.sendCounts, &g->pend.sdispls, &g->pend.recvCounts, &g->pend.rdispls};
+        for (int k = 0; k < 4; k++) {
+            if (tables[k]->size() != p * p) {
+                tables[k]->assign(p * p, 0);
+                g->tablesChecked = false;
+                g->lastA2av = nullptr;
+            }
+            uint64_t *row = tables[k]->data() + r * p;
+            if (std::memcmp(row, rows[k], p * sizeof(uint64_t)) != 0) {
+                std::memcpy(row, rows[k], p * sizeof(uint64_t));
+                g->tablesChecked = false;
+                g->lastA2av = nullptr;
+            }
+        }
     }
     g->arrived++;
     if (g->arrived < g->p) {
@@ -384,9 +395,22 @@ HcclResult Arrive(Comm *c, const OpSig &sig, void *send, void *recv, hipStream_t
     }
     // last arrival
     HcclResult res = HCCL_SUCCESS;
-    if (sig.coll == COLL_ALLTOALLV) {
+    if (sig.coll == COLL_ALLTOALLV && !g->tablesChecked) {
         // alltoall_operator.cc:49-72: what i sends to j must be what j expects from i
-        for (uint32_t i = 0; i < g->p && res == HCCL_SUCCESS; i++) {
+        // (block by block: one of the two tables is walked across its rows)
+        constexpr uint32_t kBlock = 8;
+        const uint64_t *sent = g->pend.sendCounts.data(), *expected = g->pend.recvCounts.data();
+        uint64_t differ = 0;
+        for (uint32_t i0 = 0; i0 < g->p; i0 += kBlock) {
+            for (uint32_t j0 = 0; j0 < g->p; j0 += kBlock) {
+                for (uint32_t i = i0; i < std::min(i0 + kBlock, g->p); i++) {
+                    for (uint32_t j = j0; j < std::min(j0 + kBlock, g->p); j++) {
+                        differ |= sent[size_t(i) * g->p + j] ^ expected[size_t(j) * g->p + i];
+                    }
+                }
+            }
+        }
+        for (uint32_t i = 0; i < g->p && differ != 0 && res == HCCL_SUCCESS; i++) {
             for (uint32_t j = 0; j < g->p; j++) {
                 if (g->pend.sendCounts[size_t(i) * g->p + j] != g->pend.recvCounts[size_t(j) * g->p + i]) {
                     HCCL_LOG_ERROR("AlltoAllV: rank %u sends %llu elements to rank %u, which expects %llu", i,
@@ -397,6 +421,7 @@ HcclResult Arrive(Comm *c, const OpSig &sig, void *send, void *recv, hipStream_t
                 }
             }
         }
+        g->tablesChecked = res == HCCL_SUCCESS;
     }
     if (res == HCCL_SUCCESS) {
         g->ctx = &g->pend;

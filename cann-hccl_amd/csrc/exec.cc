@@ -634,11 +634,13 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                     block[kTeamRegionCount] = n;
                     std::memcpy(block + kTeamHeaderWords, regions.data(), regions.size() * sizeof(TeamRegion));
                 }
-                // Many sources into one destination, plain: the kernel that asks for less at a time, and stores written
-                // through (StorePolicy, kernels_impl.h).
+                // Plain chains: all loads of a tile in flight while every CU has at most one tile, two sources at a time beyond
+                // that (ChainKernel); results with one destination are written through (StorePolicy, kernels_impl.h).
+                // All-reduce, us, all in flight / two sources: 8 ranks fp32 3 MiB (192 tiles) 8.9 / 9.4, 4 MiB (256) 11.4 / 11.6, 5 MiB 17.1 / 16.2,
+                // 8 MiB 22.3 / 21.6, 12 MiB 35.9 / 34.7; bf16 maximum 8 MiB 24.8 / 21.7; 4 ranks int8 6 MiB 11.4 / 9.2; 2 ranks fp32 64 MiB 46.8 / 44.9.
                 const bool toOne = reduceColl && !team && written * 3 <= traffic;
                 const bool through = toOne && !fusedOrdinary && g->cfg.fusedStores < 0 && traffic <= 2 * kMemorySideCacheBytes;
-                if (toOne && kind == int(KK_CHAIN)) {
+                if (reduceColl && !team && kind == int(KK_CHAIN) && (toOne || tiles > g->numCu)) {
                     pl.rec.func = LookupKernel(dtype, op, KK_CHAIN_SLOW);
                 }
                 const uint32_t flags = (fusedOrdinary ? kFusedOrdinaryStores : 0u) | (through ? kFusedThroughStores : 0u) | (alike ? kFusedAlike : 0u);
@@ -873,10 +875,12 @@ bool RangesOverlap(const char *a, uint64_t al, const char *b, uint64_t bl)
     return al && bl && a < b + bl && b < a + al;
 }
 
-std::string CacheKey(const Group *g, int algo)
+// Raw bytes of everything the prepared tables depend on; the p x p tables of an all-to-all-v, which are most of it, are added by
+// CacheKeyTables.
+void CacheKey(const Group *g, int algo, std::string *into)
 {
-    // raw bytes of everything the prepared tables depend on
-    std::string key;
+    std::string &key = *into;
+    key.clear();
     auto put = [&](const void *p, size_t n) { key.append(static_cast<const char *>(p), n); };
     if (g->ctx->sig.variable) {
         put(g->ctx->vCounts.data(), g->ctx->vCounts.size() * 8);
@@ -894,13 +898,15 @@ std::string CacheKey(const Group *g, int algo)
     put(&g->cfg.teamTiles, sizeof(g->cfg.teamTiles));
     put(g->ctx->send.data(), g->ctx->send.size() * sizeof(void *));
     put(g->ctx->recv.data(), g->ctx->recv.size() * sizeof(void *));
-    if (g->ctx->sig.coll == COLL_ALLTOALLV) {
-        put(g->ctx->sendCounts.data(), g->ctx->sendCounts.size() * 8);
-        put(g->ctx->sdispls.data(), g->ctx->sdispls.size() * 8);
-        put(g->ctx->recvCounts.data(), g->ctx->recvCounts.size() * 8);
-        put(g->ctx->rdispls.data(), g->ctx->rdispls.size() * 8);
+}
+
+void CacheKeyTables(const Group *g, std::string *key)
+{
+    const std::vector<uint64_t> *tables[4] = {&g->ctx->sendCounts, &g->ctx->sdispls, &g->ctx->recvCounts, &g->ctx->rdispls};
+    key->reserve(key->size() + 4 * tables[0]->size() * sizeof(uint64_t));
+    for (const std::vector<uint64_t> *t : tables) {
+        key->append(reinterpret_cast<const char *>(t->data()), t->size() * sizeof(uint64_t));
     }
-    return key;
 }
 
 // Planning costs about a millisecond for 8 ranks and tens of milliseconds for 32; a plan depends on
@@ -1490,8 +1496,23 @@ HcclResult IssueCollective(Group *g, uint32_t launcher)
         }
         pp = uncached.get();
     }
-    const bool looked = pp != nullptr || direct != nullptr;
-    std::string key = looked ? std::string() : CacheKey(g, algo);
+    bool looked = pp != nullptr || direct != nullptr;
+    std::string &key = g->keyBuffer;      // (kept: 128 KiB at 64 ranks, which malloc would map and unmap on every call)
+    if (!looked) {
+        CacheKey(g, algo, &key);
+    }
+    std::string shortKey;
+    if (!looked && g->ctx == &g->pend && g->ctx->sig.coll == COLL_ALLTOALLV) {
+        if (g->lastA2av != nullptr && g->lastA2avKey == key && (g->lastA2av->scratchGen == g->scratchGen || g->lastA2av->info.scratchBytes == 0)) {
+            pp = g->lastA2av;       // the tables are the last call's (Arrive has compared them), and so is all else
+            hit = looked = true;
+        } else {
+            shortKey = key;
+        }
+    }
+    if (!looked && g->ctx->sig.coll == COLL_ALLTOALLV) {
+        CacheKeyTables(g, &key);
+    }
     auto it = looked ? g->cache.end() : g->cache.find(key);
     if (looked) {
         // issued below
@@ -1512,6 +1533,7 @@ HcclResult IssueCollective(Group *g, uint32_t launcher)
             // a caller's graph may replay it out of the retired buffers, so it is set aside
             (it->second->pinned ? g->pinnedStale : g->stale).push_back(std::move(it->second));
             g->cache.erase(it);
+            g->lastA2av = nullptr;
         }
         if (g->cache.size() >= g->cfg.cacheEntries && !underCapture) {
             // Full: wait once for whatever is still in flight and start over.  Dropping one entry at a
@@ -1520,6 +1542,7 @@ HcclResult IssueCollective(Group *g, uint32_t launcher)
             // Collectives recorded into a caller's graph stay, tables and all (the arena keeps their chunks).
             // (Under capture the device may not be waited for: the cache runs over until the next call outside.)
             HIP_OK(hipDeviceSynchronize());
+            g->lastA2av = nullptr;
             for (auto e = g->cache.begin(); e != g->cache.end();) {
                 e = e->second->pinned ? std::next(e) : g->cache.erase(e);
             }
@@ -1543,6 +1566,10 @@ HcclResult IssueCollective(Group *g, uint32_t launcher)
         }
         pp = fresh.get();
         g->cache[key] = std::move(fresh);
+    }
+    if (!shortKey.empty()) {
+        g->lastA2av = pp;
+        g->lastA2avKey.swap(shortKey);
     }
     hipStream_t ls = g->ctx->streams[launcher];
     bool viaGraph = false;

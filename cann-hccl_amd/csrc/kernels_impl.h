@@ -1061,9 +1061,9 @@ __device__ __forceinline__ void ChainRest(const FusedDesc &d, const void *const 
 // Two forms.  Measured, us, this kernel's loads guarded one by one (before) / all in flight / two sources in flight: all-reduce, 8
 // ranks, fp32, 2 MiB per rank 7.3 / 7.3 / 7.5, 6 MiB 20.1 / 17.5 / 18.9, 8 MiB 23.9 / 22.2 / 23.9; reduce-scatter, 8 ranks, fp32, blocks of 8 MiB
 // 97.0 / 101.0 / 98.6, 16 MiB 192.7 / 200.1 / 190.8; 16 ranks, bf16 maximum, 512 KiB 27.6 / 25.4 / 23.7, 16 MiB 777 / 767 / 755.
-// SLOW = false has all loads of a tile in flight, the shortest way through a tile, for results with several
-// destinations; two workgroups have to fit a CU (a launch has up to two for each).  SLOW = true has two sources' in flight and 70 registers instead of 170: many sources into one destination
-// run better on more workgroups that ask for less each.
+// SLOW = false has all loads of a tile in flight, the shortest way through a tile, for launches of a tile per CU or fewer.
+// SLOW = true has two sources' in flight and 70 registers instead of 170: where tiles follow one another, and for
+// many sources into one destination, workgroups that ask for less at a time move more.
 template <typename T, int OP, bool SLOW>
 __global__ void __launch_bounds__(kBlockThreads, 2) ChainKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole,
     uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem)

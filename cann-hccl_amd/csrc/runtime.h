@@ -14,6 +14,7 @@
 #include <condition_variable>
 #include <deque>
 #include <cstdint>
+#include <cstring>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -146,6 +147,34 @@ bool BuildDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLau
 // Puts the ranks' pointers in; true if they were there already (the previous call's).
 bool FillBases(DirectLaunch *d, const std::vector<void *> &send, const std::vector<void *> &recv);
 
+// Hash of a cache key: 32 bytes a step, in four chains side by side (std::hash works through one; the key of an all-to-all-v
+// of 64 ranks is 132 KiB long).
+struct KeyHash {
+    size_t operator()(const std::string &key) const
+    {
+        constexpr uint64_t kMul = 0x9E3779B97F4A7C15ull;
+        uint64_t h[4] = {key.size(), 1, 2, 3};
+        const char *p = key.data();
+        size_t left = key.size();
+        for (; left >= 32; left -= 32, p += 32) {
+            uint64_t w[4];
+            std::memcpy(w, p, 32);
+            for (int i = 0; i < 4; i++) {
+                h[i] = (h[i] ^ w[i]) * kMul;
+                h[i] ^= h[i] >> 29;
+            }
+        }
+        uint64_t w[4] = {0, 0, 0, 0};
+        std::memcpy(w, p, left);
+        uint64_t all = 0;
+        for (int i = 0; i < 4; i++) {
+            all = (all ^ h[i] ^ w[i]) * kMul;
+            all ^= all >> 32;
+        }
+        return size_t(all);
+    }
+};
+
 struct OpSig {
     int coll = -1;
     uint64_t count = 0;
@@ -168,7 +197,7 @@ struct OpCtx {
     std::vector<hipStream_t> streams;
     std::vector<uint8_t> recorded;    // per rank: the rank itself put its arrival marker on its stream (it is blocked in its call)
     bool ranksWaitThemselves = false; // the blocked ranks order their streams after the launch when they wake
-    std::vector<uint64_t> sendCounts, sdispls, recvCounts, rdispls;   // p x p (all-to-all-v)
+    std::vector<uint64_t> sendCounts, sdispls, recvCounts, rdispls;   // p x p (all-to-all-v); the rendezvous' own stay from call to call
     std::vector<uint64_t> vCounts, vDispls;                           // p (reduce-scatter-v / all-gather-v)
 };
 
@@ -224,6 +253,9 @@ struct Group {
     bool doneRecorded[8] = {};           // ... and whether its done event was recorded after it for the other streams
     std::vector<uint8_t> here;
     OpCtx pend;                      // what the ranks of the current collective passed
+    bool tablesChecked = false;      // pend's all-to-all-v tables, as they are now, were found consistent
+    Prepared *lastA2av = nullptr;    // the prepared collective of pend's tables as they are now (in `cache`), if lastA2avKey ...
+    std::string lastA2avKey;         // ... matches the rest of the key: request, settings, buffers
     OpCtx *ctx = nullptr;            // the operation being issued (the rendezvous, or a matched send / receive)
     std::map<std::pair<uint32_t, uint32_t>, std::deque<P2PPending>> p2p;
 
@@ -247,7 +279,8 @@ struct Group {
     void *noAllocBase = nullptr;      // this device's copy of the fixed workspace (noalloc.hip), looked up at set-up
     uint64_t scratchBytes = 0;
     uint64_t scratchGen = 0;
-    std::unordered_map<std::string, std::unique_ptr<Prepared>> cache;   // keyed by request, settings and buffer addresses
+    std::string keyBuffer;            // the key being looked up
+    std::unordered_map<std::string, std::unique_ptr<Prepared>, KeyHash> cache;   // keyed by request, settings and buffer addresses
     std::unordered_map<DirectKey, DirectLaunch, DirectKeyHash> direct;   // small collectives, as many as `cache` holds
     TableArena arena;
     std::unordered_map<std::string, std::shared_ptr<const Plan>> planCache;   // keyed by the plan request

@@ -5,6 +5,7 @@
 #include <cstring>
 #include <sstream>
 
+#include "launch_rules.h"
 #include "log.h"
 #include "noalloc.h"
 #include "runtime.h"
@@ -170,40 +171,6 @@ struct Builder {
         return base + r.off;
     }
 };
-
-// Cuts [0, bytes) into an element-wise head, a 16-byte vector body and an element-wise tail, given
-// the addresses involved (the first one is a destination; all are multiples of the element size).
-// The head brings most of the pointers to a 16-byte boundary (of two equal groups the one with the first destination);
-// those that are then not on one too are accessed with unaligned 128-bit loads and stores (ACC_VEC16_ANY): a reduce-scatter
-// of odd blocks reads all its sources aligned and writes its one destination unaligned.  emit(offset, bytes, mode).
-// The head of a long stretch reaches to a 128-byte boundary of those pointers:
-// a wave stores 1 KiB at a time, and when those stores straddle memory lines every line is written in
-// two pieces (measured, 8-rank fp32 all-reduce of 256 MiB per rank with all buffers 16 bytes off a
-// 128-byte boundary: 0.97 ms fused against 0.76 ms aligned).
-template <typename F> void SplitByAlignment(const std::vector<uintptr_t> &addrs, uint64_t bytes, F emit)
-{
-    size_t count[16] = {0};
-    for (uintptr_t a : addrs) {
-        count[a & 15]++;
-    }
-    uintptr_t anchor = addrs[0];
-    for (uintptr_t a : addrs) {
-        anchor = count[a & 15] > count[anchor & 15] ? a : anchor;
-    }
-    const uint64_t align = bytes >= 4 * uint64_t(kTileBytes) + 128 ? 128 : 16;
-    const uint64_t head = std::min<uint64_t>(bytes, (align - (anchor & (align - 1))) & (align - 1));
-    const uint64_t body = (bytes - head) & ~uint64_t(15);
-    const uint64_t tail = bytes - head - body;
-    if (head) {
-        emit(uint64_t(0), head, uint32_t(ACC_ELEM));
-    }
-    if (body) {
-        emit(head, body, uint32_t(count[anchor & 15] == addrs.size() ? ACC_VEC16 : ACC_VEC16_ANY));
-    }
-    if (tail) {
-        emit(head + body, tail, uint32_t(ACC_ELEM));
-    }
-}
 
 constexpr size_t kGraphMinLaunches = 12;   // fewer launches go out one by one
 // The team kernels are chosen for launches of at least this many halves of a round.  All-reduce, us, plain / team: 8 ranks,
@@ -423,7 +390,7 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                 if (bb) {
                     addrs.push_back(reinterpret_cast<uintptr_t>(bb));
                 }
-                SplitByAlignment(addrs, s.bytes, [&](uint64_t off, uint64_t n, uint32_t mode) {
+                SplitByAlignment(addrs, s.bytes, ANCHOR_FIRST, [&](uint64_t off, uint64_t n, uint32_t mode) {
                     auto add = [&](std::vector<StepDesc> &to, uint64_t at, uint64_t len) {
                         StepDesc d;
                         d.dst = dst + at;
@@ -742,7 +709,7 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                     written += n * dsts.size();
                     to.push_back(d);
                 };
-                SplitByAlignment(addrs, it.bytes, [&](uint64_t off0, uint64_t n0, uint32_t mode) {
+                SplitByAlignment(addrs, it.bytes, ANCHOR_MOST, [&](uint64_t off0, uint64_t n0, uint32_t mode) {
                     for (uint64_t at = 0; at < n0; at += piece) {
                         const uint64_t n = std::min(piece, n0 - at), whole = mode != ACC_ELEM ? n / kTileBytes * kTileBytes : 0;
                         if (whole != 0) {

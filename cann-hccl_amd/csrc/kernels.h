@@ -16,7 +16,7 @@ constexpr uint32_t kBlockThreads = 256;
 // How a step's bytes may be accessed.
 enum AccessMode : uint32_t {
     ACC_VEC16 = 0,      // every pointer 16-byte aligned, byte count a multiple of 16
-    ACC_VEC16_ANY = 1,  // multiple of 16, some pointers off a 16-byte boundary (at any element boundary)
+    ACC_VEC16_ANY = 1,  // multiple of 16, some pointers off a 16-byte boundary (at any element boundary); a step's destination on one
     ACC_ELEM = 2        // element by element (heads, tails)
 };
 

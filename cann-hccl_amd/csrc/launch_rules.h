@@ -1,0 +1,55 @@
+// How the executor cuts a stretch of bytes by the alignment of its buffers.  Pure C++: no HIP calls, so the rules can be
+// checked without a GPU.
+#pragma once
+#include <algorithm>
+#include <cstddef>
+#include <cstdint>
+#include <vector>
+
+#include "kernels.h"
+
+namespace hcclamd {
+
+// Which pointers a stretch's head brings to a 16-byte boundary.
+enum AnchorRule : int {
+    ANCHOR_FIRST = 0,   // the first one, the destination: the step kernel's vector stores are aligned ones, and what a step
+                        // stores the next one reads (ring reduce-scatter step by step, 8 ranks, bf16, sends 2 bytes off, us,
+                        // this way / the largest group: 2 MiB 25.4 / 26.3, 8 MiB 44.5 / 45.9, sends and results off 26.9 / 27.8)
+    ANCHOR_MOST = 1     // the largest group that agrees (of two equal ones the one with the first pointer): a fused
+                        // reduce-scatter of odd blocks reads all its sources aligned and writes its one destination unaligned
+};
+
+// Cuts [0, bytes) into an element-wise head, a 16-byte vector body and an element-wise tail, given
+// the addresses involved (the first one is a destination; all are multiples of the element size).
+// The head brings the anchor's pointers to a 16-byte boundary; those that are then not on one
+// too are accessed with unaligned 128-bit accesses (ACC_VEC16_ANY).  emit(offset, bytes, mode).
+// The head of a long stretch reaches to a 128-byte boundary of those pointers:
+// a wave stores 1 KiB at a time, and when those stores straddle memory lines every line is written in
+// two pieces (measured, 8-rank fp32 all-reduce of 256 MiB per rank with all buffers 16 bytes off a
+// 128-byte boundary: 0.97 ms fused against 0.76 ms aligned).
+template <typename F> void SplitByAlignment(const std::vector<uintptr_t> &addrs, uint64_t bytes, AnchorRule rule, F emit)
+{
+    size_t count[16] = {0};
+    for (uintptr_t a : addrs) {
+        count[a & 15]++;
+    }
+    uintptr_t anchor = addrs[0];
+    for (uintptr_t a : addrs) {
+        anchor = rule == ANCHOR_MOST && count[a & 15] > count[anchor & 15] ? a : anchor;
+    }
+    const uint64_t align = bytes >= 4 * uint64_t(kTileBytes) + 128 ? 128 : 16;
+    const uint64_t head = std::min<uint64_t>(bytes, (align - (anchor & (align - 1))) & (align - 1));
+    const uint64_t body = (bytes - head) & ~uint64_t(15);
+    const uint64_t tail = bytes - head - body;
+    if (head) {
+        emit(uint64_t(0), head, uint32_t(ACC_ELEM));
+    }
+    if (body) {
+        emit(head, body, uint32_t(count[anchor & 15] == addrs.size() ? ACC_VEC16 : ACC_VEC16_ANY));
+    }
+    if (tail) {
+        emit(head + body, tail, uint32_t(ACC_ELEM));
+    }
+}
+
+}  // namespace hcclamd

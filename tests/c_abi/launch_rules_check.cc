@@ -1,0 +1,75 @@
+// Host-only check of the executor's rules on sizes and alignment (cann-hccl_amd/csrc/launch_rules.h), compiled and run by
+// tests/test_launch_rules_cpu.py.
+#include <cstdio>
+#include <cstdlib>
+#include <random>
+
+#include "launch_rules.h"
+
+using namespace hcclamd;
+
+#define CHECK(c)                                              \
+    do {                                                      \
+        if (!(c)) {                                           \
+            std::printf("FAIL line %d: %s\n", __LINE__, #c);  \
+            std::exit(1);                                     \
+        }                                                     \
+    } while (0)
+
+namespace {
+
+std::mt19937_64 rng(20);
+uint64_t Draw(uint64_t n) { return rng() % n; }
+
+// Heads, bodies and tails cover the stretch in order, and a body starts where the rule says.
+void CheckSplit()
+{
+    uint64_t bodies = 0, unaligned = 0;
+    for (int round = 0; round < 40000; round++) {
+        const uint64_t unit = uint64_t(1) << Draw(4);
+        std::vector<uintptr_t> addrs(1 + Draw(9));
+        const uint64_t residues = 1 + Draw(3);     // few of them, so that groups form
+        uint64_t shift[3] = {Draw(128) / unit * unit, Draw(128) / unit * unit, Draw(128) / unit * unit};
+        for (uintptr_t &a : addrs) {
+            a = (uintptr_t(1) << 40) + Draw(1 << 20) * 128 + shift[Draw(residues)];
+        }
+        const uint64_t bytes = unit * (Draw(2) != 0 ? Draw(200) : Draw(40000));
+        for (AnchorRule rule : {ANCHOR_FIRST, ANCHOR_MOST}) {
+            uint64_t at = 0;
+            SplitByAlignment(addrs, bytes, rule, [&](uint64_t off, uint64_t n, uint32_t mode) {
+                CHECK(off == at && n != 0);
+                at += n;
+                CHECK(n % unit == 0);
+                if (mode == ACC_ELEM) {
+                    CHECK(n < 128);
+                    return;
+                }
+                CHECK(n % 16 == 0);
+                size_t agree[16] = {0}, most = 0;
+                for (uintptr_t a : addrs) {
+                    most = std::max(most, ++agree[(a + off) & 15]);
+                }
+                CHECK((agree[0] == addrs.size()) == (mode == ACC_VEC16));
+                if (rule == ANCHOR_FIRST) {
+                    CHECK(((addrs[0] + off) & 15) == 0);      // the step kernel's aligned stores
+                    CHECK(bytes < 4 * uint64_t(kTileBytes) + 128 || ((addrs[0] + off) & 127) == 0);
+                } else {
+                    CHECK(agree[0] == most);
+                }
+                bodies++;
+                unaligned += mode == ACC_VEC16_ANY ? 1 : 0;
+            });
+            CHECK(at == bytes);
+        }
+    }
+    CHECK(bodies > 30000 && unaligned > 5000);
+}
+
+}  // namespace
+
+int main()
+{
+    CheckSplit();
+    std::printf("OK\n");
+    return 0;
+}

@@ -115,6 +115,31 @@ def test_buffers_at_different_offsets(orc, dt, op, offsets, team):
         g.close()
 
 
+@pytest.mark.parametrize("dt,op", [(FP32, SUM), (BF16, MAX), (INT8, SUM)])
+@pytest.mark.parametrize("algo", ["ring", "mesh"])
+def test_steps_with_only_the_destination_off(orc, dt, op, algo):
+    # step by step, both operands at one offset from a 16-byte boundary and the destination at another
+    p, unit = 4, H.DTYPE_SIZE[dt]
+    g = gh.Group(p, algo=algo, fuse=0, deterministic=1)
+    try:
+        for n, src, dst in ((5, 0, unit), (3 * TILE // unit + 7, 0, unit), (3 * TILE // unit + 7, unit, 0), (7 * TILE // unit + 1, 8, 8 + unit)):
+            print("steps", dt, op, algo, n, src, dst, flush=True)
+            ins = _ins(dt, p, n * p, 9500 + n)
+            want = orc.reducescatter(ins, dt, op, algo={"ring": 0, "mesh": 1}[algo])
+            sends = [gh.to_dev(x, 16 + src) for x in ins]
+            whole = [torch.full((n * unit + 64,), 0xA5, dtype=torch.uint8, device="cuda") for _ in ins]
+            torch.cuda.synchronize()
+            H.reduce_scatter(g.comms, [t.data_ptr() for t in sends], [t.data_ptr() + 16 + dst for t in whole], n, dt, op, g.stream_ptr)
+            g.stream.synchronize()
+            assert g.info()["fused"] == 0
+            for r in range(p):
+                t = whole[r]
+                assert gh.same(dt, gh.to_host(t[16 + dst:16 + dst + n * unit].clone(), dt), want[r]), (n, r)
+                assert bool((t[:16 + dst] == 0xA5).all()) and bool((t[16 + dst + n * unit:] == 0xA5).all()), (n, r)
+    finally:
+        g.close()
+
+
 @pytest.mark.parametrize("dt,op", [(FP16, MAX), (FP16, MIN), (BF16, MAX), (BF16, MIN)])
 @pytest.mark.parametrize("p,team", [(8, 0), (8, 1), (5, 0), (2, 1), (12, 0)])
 def test_half_selection_over_every_bit_pattern(orc, dt, op, p, team):

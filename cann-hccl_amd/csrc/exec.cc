@@ -390,25 +390,25 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                 if (bb) {
                     addrs.push_back(reinterpret_cast<uintptr_t>(bb));
                 }
-                SplitByAlignment(addrs, s.bytes, ANCHOR_FIRST, [&](uint64_t off, uint64_t n, uint32_t mode) {
-                    auto add = [&](std::vector<StepDesc> &to, uint64_t at, uint64_t len) {
-                        StepDesc d;
-                        d.dst = dst + at;
-                        d.a = a + at;
-                        d.b = bb ? bb + at : nullptr;
-                        d.bytes = len;
-                        d.tile0 = 0;
-                        d.mode = mode;
-                        to.push_back(d);
-                    };
-                    uint64_t body = (mode == ACC_VEC16) ? n / kTileBytes * kTileBytes : 0;
-                    if (body) {
-                        add(whole, off, body);
+                auto add = [&](std::vector<StepDesc> &to, uint64_t at, uint64_t len, uint32_t mode) {
+                    if (len == 0) {
+                        return;
                     }
-                    if (n > body) {
-                        add(ragged, off + body, n - body);
-                    }
-                });
+                    StepDesc d;
+                    d.dst = dst + at;
+                    d.a = a + at;
+                    d.b = bb ? bb + at : nullptr;
+                    d.bytes = len;
+                    d.tile0 = 0;
+                    d.mode = mode;
+                    to.push_back(d);
+                };
+                const Cut cut = CutByAlignment(addrs, s.bytes, ANCHOR_FIRST);
+                const uint64_t body = cut.aligned ? cut.body / kTileBytes * kTileBytes : 0;
+                add(ragged, 0, cut.head, ACC_ELEM);
+                add(whole, cut.head, body, ACC_VEC16);
+                add(ragged, cut.head + body, cut.body - body, cut.aligned ? ACC_VEC16 : ACC_VEC16_ANY);
+                add(ragged, cut.head + cut.body, cut.tail, ACC_ELEM);
             }
             // Every other launch walks the data the other way round, so that a phase starts with what the
             // phase before it wrote last (measured, 8-rank fp32 ring all-reduce of 256 MiB per rank: 1.431 ms
@@ -512,8 +512,9 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
         // one launch per kernel kind present, or several under a launch cap: the items in their order, cut where the
         // bytes a launch moves (read and written) reach the cap
         for (int kind : {int(KK_CHAIN), int(KK_TREE), int(KK_STACK)}) {
-            std::vector<FusedDesc> descs;      // whole tiles
-            std::vector<FusedDesc> rests;      // what is left of a stretch behind them, and its element-wise ends: a tile each
+            std::vector<FusedDesc> descs;      // items that have whole tiles
+            std::vector<FusedDesc> shorts;     // items that have not
+            bool anyRest = false, anyEnds = false;
             std::vector<const void *> srcPool;
             std::vector<uint32_t> opPool;      // stack items: one word per source-pool entry
             std::vector<void *> dstPool;
@@ -523,19 +524,20 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
             std::vector<uintptr_t> addrs;
             const void *func = reduceColl ? LookupKernel(dtype, op, KernelKind(kind)) : LookupCopyKernel(KernelKind(kind));
             auto flush = [&]() {
-                if (descs.empty() && rests.empty()) {
+                if (descs.empty() && shorts.empty()) {
                     return;
                 }
                 PendingLaunch pl;
                 pl.rec.func = func;
                 pl.rec.nitems = uint32_t(descs.size());
+                pl.rec.nall = uint32_t(descs.size() + shorts.size());
                 pl.rec.nwhole = tiles;
-                pl.rec.ntiles = tiles + uint32_t(rests.size());
+                pl.rec.ntiles = tiles + (anyEnds ? 2 * pl.rec.nall : (anyRest ? pl.rec.nall : 0u));
                 // equal slices (the usual collective): the kernels find a tile's item without searching the table
-                pl.rec.tilesPerItem = descs.empty() ? 0 : TilesOf(descs[0].bytes);
+                pl.rec.tilesPerItem = descs.empty() ? 0 : uint32_t(descs[0].bytes / kTileBytes);
                 bool alike = !descs.empty() && kind == int(KK_CHAIN) && descs[0].nsrc >= 2;
                 for (size_t i = 0; i < descs.size(); i++) {
-                    const uint32_t t = TilesOf(descs[i].bytes);
+                    const uint32_t t = uint32_t(descs[i].bytes / kTileBytes);
                     if (i + 1 < descs.size() ? t != pl.rec.tilesPerItem : t > pl.rec.tilesPerItem) {
                         pl.rec.tilesPerItem = 0;
                     }
@@ -588,7 +590,7 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                     // 235 they gain: 8 ranks x 88 MiB maximum of int64 271.3 / 276.4, x 96 MiB sum of int64 264.0 / 282.0.
                     uint32_t inShort = 0;
                     for (const FusedDesc &d : descs) {
-                        const uint32_t t = TilesOf(d.bytes);
+                        const uint32_t t = uint32_t(d.bytes / kTileBytes);
                         inShort += t < pl.rec.roundTiles * perX * 3 / 4 ? t : 0u;
                     }
                     if (kind == int(KK_STACK) && inShort > tiles / 4) {
@@ -612,12 +614,9 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                 }
                 const uint32_t flags = (fusedOrdinary ? kFusedOrdinaryStores : 0u) | (through ? kFusedThroughStores : 0u) | (alike ? kFusedAlike : 0u);
                 // the op words of the stack kernel sit right behind its item table
-                pl.tableAt = b.Reserve((descs.size() + rests.size()) * sizeof(FusedDesc) + opPool.size() * sizeof(uint32_t));
+                descs.insert(descs.end(), shorts.begin(), shorts.end());
+                pl.tableAt = b.Reserve(descs.size() * sizeof(FusedDesc) + opPool.size() * sizeof(uint32_t));
                 FusedDesc *table = reinterpret_cast<FusedDesc *>(b.host.data() + pl.tableAt);
-                for (size_t i = 0; i < rests.size(); i++) {
-                    rests[i].tile0 = tiles + uint32_t(i);
-                }
-                descs.insert(descs.end(), rests.begin(), rests.end());
                 for (FusedDesc &d : descs) {
                     d.flags |= flags;
                 }
@@ -625,13 +624,14 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                 if (!opPool.empty()) {
                     std::memcpy(table + descs.size(), opPool.data(), opPool.size() * sizeof(uint32_t));
                 }
-                pl.srcAt = b.Reserve((srcPool.size() + kPoolPad) * sizeof(void *));
+                pl.srcAt = b.Reserve(srcPool.size() * sizeof(void *));
                 std::memcpy(b.host.data() + pl.srcAt, srcPool.data(), srcPool.size() * sizeof(void *));
-                pl.dstAt = b.Reserve((dstPool.size() + kPoolPad) * sizeof(void *));
+                pl.dstAt = b.Reserve(dstPool.size() * sizeof(void *));
                 std::memcpy(b.host.data() + pl.dstAt, dstPool.data(), dstPool.size() * sizeof(void *));
                 pending.push_back(pl);
                 descs.clear();
-                rests.clear();
+                shorts.clear();
+                anyRest = anyEnds = false;
                 srcPool.clear();
                 opPool.clear();
                 dstPool.clear();
@@ -658,7 +658,7 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                     dsts.push_back(t);
                     addrs.push_back(reinterpret_cast<uintptr_t>(dsts.back()));
                 }
-                if (dsts.empty()) {
+                if (dsts.empty() || it.bytes == 0) {
                     continue;
                 }
                 uint32_t streams = uint32_t(dsts.size());
@@ -681,13 +681,14 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                 for (size_t k = 0; k < srcs.size(); k++) {
                     flags |= kind == int(KK_TREE) && (k & 1u) != 0 && srcs[k] != nullptr ? kFusedPairs : 0u;
                 }
-                auto add = [&](std::vector<FusedDesc> &to, uint64_t off, uint64_t n, uint32_t mode) {
+                auto add = [&](uint64_t off, uint64_t n, uint64_t head, uint64_t tail) {
                     FusedDesc d;
                     std::memset(&d, 0, sizeof(d));
                     d.bytes = n;
                     d.accLeftMask = mask;
                     d.tile0 = tiles;
-                    d.mode = mode;
+                    d.head = uint16_t(head);
+                    d.tail = uint16_t(tail);
                     d.nsrc = uint32_t(srcs.size());
                     d.ndst = uint32_t(dsts.size());
                     d.srcBase = uint32_t(srcPool.size());
@@ -705,25 +706,26 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                     for (char *t : dsts) {
                         dstPool.push_back(t + off);
                     }
-                    traffic += n * streams;
-                    written += n * dsts.size();
-                    to.push_back(d);
+                    traffic += (n + head + tail) * streams;
+                    written += (n + head + tail) * dsts.size();
+                    tiles += uint32_t(n / kTileBytes);
+                    anyRest = anyRest || n % kTileBytes != 0;
+                    anyEnds = anyEnds || head != 0 || tail != 0;
+                    (n >= kTileBytes ? descs : shorts).push_back(d);
                 };
-                SplitByAlignment(addrs, it.bytes, ANCHOR_MOST, [&](uint64_t off0, uint64_t n0, uint32_t mode) {
-                    for (uint64_t at = 0; at < n0; at += piece) {
-                        const uint64_t n = std::min(piece, n0 - at), whole = mode != ACC_ELEM ? n / kTileBytes * kTileBytes : 0;
-                        if (whole != 0) {
-                            add(descs, off0 + at, whole, mode);
-                            tiles += uint32_t(whole / kTileBytes);
-                        }
-                        if (n != whole) {
-                            add(rests, off0 + at + whole, n - whole, mode);
-                        }
-                        if (capBytes != 0 && traffic >= capBytes) {
-                            flush();
+                const Cut cut = CutByAlignment(addrs, it.bytes, ANCHOR_MOST);
+                for (uint64_t at = 0; at == 0 || at < cut.body; at += std::min(piece, it.bytes)) {
+                    const uint64_t n = std::min(piece, cut.body - at), head = at == 0 ? cut.head : 0;
+                    const uint64_t tail = at + n == cut.body ? cut.tail : 0;
+                    const bool full = capBytes != 0 && traffic + (n + head) * streams >= capBytes;
+                    add(cut.head + at, n, head, full ? 0 : tail);
+                    if (full) {
+                        flush();
+                        if (tail != 0) {
+                            add(cut.head + cut.body, 0, 0, tail);
                         }
                     }
-                });
+                }
             }
             flush();
         }
@@ -797,17 +799,20 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
     return HCCL_SUCCESS;
 }
 
+constexpr size_t kMaxKernelArgs = 9;
+
 void KernelArgs(LaunchRec &l, void **args)
 {
     args[0] = &l.table;
     args[1] = &l.nitems;
     if (l.fusedArgs) {
-        args[2] = &l.nwhole;
-        args[3] = &l.ntiles;
-        args[4] = &l.srcPool;
-        args[5] = &l.dstPool;
-        args[6] = &l.tilesPerItem;
-        args[7] = &l.teamCtr;      // read by the team kernels only
+        args[2] = &l.nall;
+        args[3] = &l.nwhole;
+        args[4] = &l.ntiles;
+        args[5] = &l.srcPool;
+        args[6] = &l.dstPool;
+        args[7] = &l.tilesPerItem;
+        args[8] = &l.teamCtr;      // read by the team kernels only
     } else {
         args[2] = &l.nwhole;
         args[3] = &l.ntiles;
@@ -820,7 +825,7 @@ HcclResult BuildGraph(Prepared *pp)
     HIP_OK(hipGraphCreate(&pp->graph, 0));
     hipGraphNode_t prev = nullptr;
     for (LaunchRec &l : pp->launches) {
-        void *args[8];
+        void *args[kMaxKernelArgs];
         KernelArgs(l, args);
         hipKernelNodeParams kp = {};
         kp.func = const_cast<void *>(l.func);
@@ -1580,7 +1585,7 @@ HcclResult IssueCollective(Group *g, uint32_t launcher)
         HIP_OK(hipGraphLaunch(pp->exec, ls));
     } else {
         for (LaunchRec &l : pp->launches) {
-            void *args[8];
+            void *args[kMaxKernelArgs];
             KernelArgs(l, args);
             HIP_OK(hipLaunchKernel(l.func, dim3(l.grid, 1, 1), dim3(kBlockThreads, 1, 1), args, l.dynamicLds, ls));
         }

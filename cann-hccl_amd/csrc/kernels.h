@@ -16,7 +16,7 @@ constexpr uint32_t kBlockThreads = 256;
 // How a step's bytes may be accessed.
 enum AccessMode : uint32_t {
     ACC_VEC16 = 0,      // every pointer 16-byte aligned, byte count a multiple of 16
-    ACC_VEC16_ANY = 1,  // multiple of 16, some pointers off a 16-byte boundary (at any element boundary); a step's destination on one
+    ACC_VEC16_ANY = 1,  // multiple of 16, the destination 16-byte aligned, the sources at any element boundary
     ACC_ELEM = 2        // element by element (heads, tails)
 };
 
@@ -39,11 +39,15 @@ struct StepDesc {
 //           values are folded ops[j] & 7 times, bit 8 + i of ops[j] set = the lower value is the left
 //           operand of fold i.  The launch's op words (one uint32 per source-pool entry, same index)
 //           follow its item table in memory; nleaf holds the stack depth the program needs.
+// An item is one entry of the table and one list of pointers, which say where its body starts: a multiple of 16 bytes, in whole
+// tiles and a rest shorter than one.  In front of the body and behind it lie its ends, done element by element.  (The tables
+// of a collective travel to the device in front of it, and those of the call that allocates nothing have to fit 256 KiB.)
 struct FusedDesc {
-    uint64_t bytes;
+    uint64_t bytes;     // of the body
     uint64_t accLeftMask;
     uint32_t tile0;
-    uint32_t mode;
+    uint16_t head;      // bytes in front of the body, fewer than 128
+    uint16_t tail;      // bytes behind it, fewer than 16
     uint32_t nsrc;
     uint32_t ndst;
     uint32_t srcBase;   // index into the source pointer pool
@@ -55,12 +59,9 @@ struct FusedDesc {
 // flags of a fused item.  Stores: streamed past the caches unless one of the first two is set (StorePolicy, kernels_impl.h).
 constexpr uint32_t kFusedOrdinaryStores = 1u;  // write-back
 constexpr uint32_t kFusedThroughStores = 2u;   // written through to memory, without the non-temporal hint (plain kernels)
-constexpr uint32_t kFusedWordSources = 4u;     // 8-bit chains: a source starts off a 16-byte boundary
+constexpr uint32_t kFusedWordSources = 4u;     // 8-bit chains, copies: a source's body starts off a 4-byte boundary
 constexpr uint32_t kFusedPairs = 8u;           // trees: some leaf has a second source
 constexpr uint32_t kFusedAlike = 16u;          // chains: all items of the launch have the same number of sources, two or more
-
-// What the tables of a launch keep behind their pointer pools, so that eight pointers can be fetched together.
-constexpr uint32_t kPoolPad = 8;
 
 // flags of the step kernel
 constexpr uint32_t kStepOrdinaryStores = 1u;   // write-back stores instead of non-temporal ones in the fast loop
@@ -146,10 +147,13 @@ static_assert(sizeof(DirectArgs<32>) <= 4096, "kernel arguments");
 //   KK_STEP            (const StepDesc *steps, uint32_t nsteps, uint32_t nwhole, uint32_t ntiles, uint32_t flags)
 //                      steps whose tiles are all whole and ACC_VEC16 come first: tiles [0, nwhole)
 //   KK_CHAIN / KK_CHAIN_SLOW / KK_TREE / KK_STACK
-//                      (const FusedDesc *items, uint32_t nitems, uint32_t nwhole, uint32_t ntiles,
+//                      (const FusedDesc *items, uint32_t nitems, uint32_t nall, uint32_t nwhole, uint32_t ntiles,
 //                       const void *const *srcPool, void *const *dstPool, uint32_t tilesPerItem)
-//                      tiles [0, nwhole) are the whole tiles of the first nitems items, each later tile is an item of its own;
-//                      tilesPerItem: tiles of each of the first nitems items (the last one at most as many), 0 = they differ
+//                      tiles [0, nwhole) are the whole tiles of the first nitems of the nall items; tile nwhole + i is the rest of
+//                      item i's body, tile nwhole + nall + i its ends (ntiles: as many of these as any item needs, empty ones included);
+//                      tilesPerItem: whole tiles of each of the first nitems items (the last one at most as many), 0 = they differ.
+//                      Up to seven pointers behind an item's list of sources may be read (and are not used): the destinations'
+//                      pool lies behind the sources', and the tables end on a multiple of 256 bytes.
 //   KK_TEAM_*          the same and (uint32_t *teamBlock)
 //   KK_DIRECT / KK_DIRECT_WIDE   (DirectArgs<8> / DirectArgs<32>), grid (1 + chunks of the longest item, items): blockIdx.x == 0
 //                      is for the bytes behind an item's last whole vector

@@ -571,11 +571,10 @@ __global__ void __launch_bounds__(kBlockThreads) StepKernel(const StepDesc *__re
 }
 
 // ---- fused kernels: what they share ---------------------------------------------------------------------
-// The tiles of a launch come in two parts.  Tiles [0, nwhole) are whole: they belong to the first nitems items, whose
-// byte counts are multiples of kTileBytes.  Every tile from nwhole on is an item of its own (item nitems + tile - nwhole):
-// what is left of a stretch behind its last whole tile, and its element-wise ends.  The loop over whole tiles has
+// The tiles of a launch come in three parts.  Tiles [0, nwhole) are whole: they belong to the first nitems items.  Then comes a
+// tile for the rest of every item's body (of an item with less than a tile all of it), then one for every item's ends.  The loop over whole tiles has
 // nothing else in it: with the guarded paths in the same loop the compiler makes a tile's loads wait for each other and for
-// the stores of the tile before.  The pieces behind them go through the same straight-line code, all sources' loads in flight: one
+// the stores of the tile before.  Rests and ends go through the same straight-line code, all sources' loads in flight: one
 // after the other they were most of a ragged collective of a few MiB (all-reduce, 8 ranks, bf16, 2 MiB + 6 bytes per rank
 // 20.9 us, now 8.0; 32 ranks 77.6, now 27.9).
 constexpr uint32_t kChainVec = 4;      // vectors per lane per pass
@@ -782,11 +781,18 @@ template <uint32_t U> __device__ __forceinline__ void ReadPositions(const uint32
     }
 }
 
-// Walks a launch's tiles with a grid stride: whole(d, ahead(d), off) for each whole tile, rest(d) for each item behind them.
+// The rest of an item's body behind its whole tiles, and its ends, of which lane i takes the element at byte i.
+__device__ __forceinline__ uint64_t RestOffset(const FusedDesc &d) { return d.bytes / kTileBytes * kTileBytes; }
+__device__ __forceinline__ uint32_t RestBytes(const FusedDesc &d) { return uint32_t(d.bytes % kTileBytes); }
+__device__ __forceinline__ uint32_t EndBytes(const FusedDesc &d) { return uint32_t(d.head) + d.tail; }
+__device__ __forceinline__ uint64_t EndOffset(const FusedDesc &d, uint32_t i) { return (i < d.head ? 0 : d.bytes) + i - d.head; }
+static_assert(128 + 16 <= kBlockThreads, "a workgroup takes an item's ends at once");
+
+// Walks a launch's tiles with a grid stride: whole(d, ahead(d), off) for each whole tile, rest(d, ends) for each tile behind them.
 // A workgroup keeps its item while its tiles stay inside it; the next item, and what `ahead` fetches for it, is looked up
 // ahead of the current tile's loads, so that the chain of dependent loads (table, item, pointer) completes behind those.
 template <typename Ahead, typename Whole, typename Rest>
-__device__ __forceinline__ void WalkTiles(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole, uint32_t ntiles,
+__device__ __forceinline__ void WalkTiles(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nall, uint32_t nwhole, uint32_t ntiles,
     uint32_t tilesPerItem, Ahead ahead, Whole whole, Rest rest)
 {
     uint32_t tile = blockIdx.x;
@@ -815,8 +821,10 @@ __device__ __forceinline__ void WalkTiles(const FusedDesc *__restrict__ items, u
         }
     }
     for (; tile < ntiles; tile += gridDim.x) {
-        const FusedDesc d = items[nitems + (tile - nwhole)];
-        rest(d);
+        const uint32_t r = tile - nwhole;
+        const bool ends = r >= nall;
+        const FusedDesc d = items[ends ? r - nall : r];
+        rest(d, ends);
     }
 }
 
@@ -1035,24 +1043,30 @@ __device__ __forceinline__ void ChainTile(const FusedDesc &d, const void *const 
     StoreByFlags(d, dst, off, WHOLE ? kTileBytes : nbytes, pos, acc);
 }
 
-// An item behind the whole tiles.
+// An item's rest, or its ends.
 template <typename T, int OP, bool SLOW = false>
-__device__ __forceinline__ void ChainRest(const FusedDesc &d, const void *const *__restrict__ src, void *const *__restrict__ dst)
+__device__ __forceinline__ void ChainRest(const FusedDesc &d, bool ends, const void *const *__restrict__ src, void *const *__restrict__ dst)
 {
-    const uint32_t n = uint32_t(d.bytes);
-    if (d.mode != ACC_ELEM) {
+    if (!ends) {
+        const uint64_t off = RestOffset(d);
+        const uint32_t n = RestBytes(d);
+        if (n == 0) {
+            return;
+        }
         if (n <= kBlockThreads * 16u) {
-            ChainTile<T, OP, false, false, 1>(d, src, dst, 0, n);
+            ChainTile<T, OP, false, false, 1>(d, src, dst, off, n);
         } else {
-            ChainTile<T, OP, false, SLOW, kChainVec>(d, src, dst, 0, n);
+            ChainTile<T, OP, false, SLOW, kChainVec>(d, src, dst, off, n);
         }
     } else {
-        for (uint32_t i = threadIdx.x * uint32_t(sizeof(T)); i < n; i += kBlockThreads * uint32_t(sizeof(T))) {
-            const uint32_t at[1] = {i};
+        const uint32_t i = threadIdx.x * uint32_t(sizeof(T));
+        if (i < EndBytes(d)) {
+            const uint64_t off = EndOffset(d, i);
+            const uint32_t at[1] = {0};
             T acc[1];
-            ChainValue<ElemLane<T, OP>, T, OP, 1>(d, src, 0, at, acc);
+            ChainValue<ElemLane<T, OP>, T, OP, 1>(d, src, off, at, acc);
             for (uint32_t k = 0; k < d.ndst; k++) {
-                StoreElem<T>(dst[k], i, acc[0]);
+                StoreElem<T>(dst[k], off, acc[0]);
             }
         }
     }
@@ -1065,12 +1079,12 @@ __device__ __forceinline__ void ChainRest(const FusedDesc &d, const void *const 
 // SLOW = true has two sources' in flight and 70 registers instead of 170: where tiles follow one another, and for
 // many sources into one destination, workgroups that ask for less at a time move more.
 template <typename T, int OP, bool SLOW>
-__global__ void __launch_bounds__(kBlockThreads, 2) ChainKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole,
+__global__ void __launch_bounds__(kBlockThreads, 2) ChainKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nall, uint32_t nwhole,
     uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem)
 {
-    WalkTiles(items, nitems, nwhole, ntiles, tilesPerItem, [](const FusedDesc &) { return 0; },
+    WalkTiles(items, nitems, nall, nwhole, ntiles, tilesPerItem, [](const FusedDesc &) { return 0; },
         [&](const FusedDesc &d, int, uint64_t off) { ChainTile<T, OP, true, SLOW, kChainVec>(d, srcPool + d.srcBase, dstPool + d.dstBase, off, kTileBytes); },
-        [&](const FusedDesc &d) { ChainRest<T, OP, SLOW>(d, srcPool + d.srcBase, dstPool + d.dstBase); });
+        [&](const FusedDesc &d, bool ends) { ChainRest<T, OP, SLOW>(d, ends, srcPool + d.srcBase, dstPool + d.dstBase); });
 }
 
 // ---- pure data movement: one source, m destinations ------------------------------------------------------
@@ -1090,17 +1104,17 @@ __device__ __forceinline__ void CopyTile(const FusedDesc &d, const void *s, void
     ChainLoad<MoveLane, 1, kChainVec>(&s, off, at, v);
     StoreByFlags(d, dst, off, WHOLE ? kTileBytes : nbytes, pos, v[0]);
 }
-__device__ __forceinline__ void CopyRest(const FusedDesc &d, const void *s, void *const *__restrict__ dst)
+__device__ __forceinline__ void CopyRest(const FusedDesc &d, bool ends, const void *s, void *const *__restrict__ dst)
 {
-    const uint32_t n = uint32_t(d.bytes);
-    if (d.mode != ACC_ELEM) {
-        CopyTile<false>(d, s, dst, 0, n);
-    } else {
-        for (uint32_t i = threadIdx.x; i < n; i += kBlockThreads) {
-            const uint8_t b = LoadElem<uint8_t>(s, i);
-            for (uint32_t k = 0; k < d.ndst; k++) {
-                StoreElem<uint8_t>(dst[k], i, b);
-            }
+    if (!ends) {
+        if (RestBytes(d) != 0) {
+            CopyTile<false>(d, s, dst, RestOffset(d), RestBytes(d));
+        }
+    } else if (threadIdx.x < EndBytes(d)) {
+        const uint64_t off = EndOffset(d, threadIdx.x);
+        const uint8_t b = LoadElem<uint8_t>(s, off);
+        for (uint32_t k = 0; k < d.ndst; k++) {
+            StoreElem<uint8_t>(dst[k], off, b);
         }
     }
 }
@@ -1108,12 +1122,12 @@ __device__ __forceinline__ void CopyRest(const FusedDesc &d, const void *s, void
 // Same arguments and tables as the chain kernel; every item has exactly one source.  (A template only so that the
 // definition may sit in this header; Variant is unused.)
 template <int Variant>
-__global__ void __launch_bounds__(kBlockThreads) CopyKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole,
+__global__ void __launch_bounds__(kBlockThreads) CopyKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nall, uint32_t nwhole,
     uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem)
 {
-    WalkTiles(items, nitems, nwhole, ntiles, tilesPerItem, [&](const FusedDesc &d) { return srcPool[d.srcBase]; },
+    WalkTiles(items, nitems, nall, nwhole, ntiles, tilesPerItem, [&](const FusedDesc &d) { return srcPool[d.srcBase]; },
         [&](const FusedDesc &d, const void *s, uint64_t off) { CopyTile<true>(d, s, dstPool + d.dstBase, off, kTileBytes); },
-        [&](const FusedDesc &d) { CopyRest(d, srcPool[d.srcBase], dstPool + d.dstBase); });
+        [&](const FusedDesc &d, bool ends) { CopyRest(d, ends, srcPool[d.srcBase], dstPool + d.dstBase); });
 }
 
 // ---- small-segment gather: LDS staging ---------------------------------------------------------------------
@@ -1331,41 +1345,47 @@ __device__ __forceinline__ void TreeValue(const FusedDesc &d, const void *const 
 }
 
 template <typename T, int OP>
-__device__ __forceinline__ void TreeRest(const FusedDesc &d, const void *const *__restrict__ src, void *const *__restrict__ dst)
+__device__ __forceinline__ void TreeRest(const FusedDesc &d, bool ends, const void *const *__restrict__ src, void *const *__restrict__ dst)
 {
-    const uint32_t n = uint32_t(d.bytes);
-    if (d.mode != ACC_ELEM) {
+    if (!ends) {
+        const uint64_t off = RestOffset(d);
+        const uint32_t n = RestBytes(d);
+        if (n == 0) {
+            return;
+        }
         uint32_t pos[kChainVec], at[kChainVec];
         V4 x[kChainVec];
-            TilePositions(pos);
+        TilePositions(pos);
         ReadPositions(pos, n, at);
-        TreeValue<VecLane<T, OP>, kChainVec>(d, src, 0, at, x);
-        StoreByFlags(d, dst, 0, n, pos, x);
+        TreeValue<VecLane<T, OP>, kChainVec>(d, src, off, at, x);
+        StoreByFlags(d, dst, off, n, pos, x);
     } else {
-        for (uint32_t i = threadIdx.x * uint32_t(sizeof(T)); i < n; i += kBlockThreads * uint32_t(sizeof(T))) {
-            const uint32_t at[1] = {i};
+        const uint32_t i = threadIdx.x * uint32_t(sizeof(T));
+        if (i < EndBytes(d)) {
+            const uint64_t off = EndOffset(d, i);
+            const uint32_t at[1] = {0};
             T x[1];
-            TreeValue<ElemLane<T, OP>, 1>(d, src, 0, at, x);
+            TreeValue<ElemLane<T, OP>, 1>(d, src, off, at, x);
             for (uint32_t k = 0; k < d.ndst; k++) {
-                StoreElem<T>(dst[k], i, x[0]);
+                StoreElem<T>(dst[k], off, x[0]);
             }
         }
     }
 }
 
 template <typename T, int OP>
-__global__ void __launch_bounds__(kBlockThreads) TreeKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole,
+__global__ void __launch_bounds__(kBlockThreads) TreeKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nall, uint32_t nwhole,
     uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem)
 {
     uint32_t pos[kChainVec];
     TilePositions(pos);
-    WalkTiles(items, nitems, nwhole, ntiles, tilesPerItem, [](const FusedDesc &) { return 0; },
+    WalkTiles(items, nitems, nall, nwhole, ntiles, tilesPerItem, [](const FusedDesc &) { return 0; },
         [&](const FusedDesc &d, int, uint64_t off) {
             V4 x[kChainVec];
             TreeValue<VecLane<T, OP>, kChainVec>(d, srcPool + d.srcBase, off, pos, x);
             StoreByFlags(d, dstPool + d.dstBase, off, kTileBytes, pos, x);
         },
-        [&](const FusedDesc &d) { TreeRest<T, OP>(d, srcPool + d.srcBase, dstPool + d.dstBase); });
+        [&](const FusedDesc &d, bool ends) { TreeRest<T, OP>(d, ends, srcPool + d.srcBase, dstPool + d.dstBase); });
 }
 
 // ---- fused general expression: a stack machine over registers -----------------------------------------
@@ -1538,38 +1558,44 @@ __device__ __forceinline__ void StackStore(const FusedDesc &d, const void *const
 }
 
 template <typename T, int OP>
-__device__ __forceinline__ void StackRest(const FusedDesc &d, const void *const *__restrict__ src, const uint32_t *__restrict__ ops, void *const *__restrict__ dst)
+__device__ __forceinline__ void StackRest(const FusedDesc &d, bool ends, const void *const *__restrict__ src, const uint32_t *__restrict__ ops,
+    void *const *__restrict__ dst)
 {
-    const uint32_t n = uint32_t(d.bytes);
-    if (d.mode != ACC_ELEM) {
+    if (!ends) {
+        const uint32_t n = RestBytes(d);
+        if (n == 0) {
+            return;
+        }
         uint32_t pos[kChainVec], at[kChainVec];
         TilePositions(pos);
         ReadPositions(pos, n, at);
-        StackStore<T, OP, kStackPlainBatch>(d, src, ops, dst, 0, n, pos, at);
+        StackStore<T, OP, kStackPlainBatch>(d, src, ops, dst, RestOffset(d), n, pos, at);
     } else {
-        for (uint32_t i = threadIdx.x * uint32_t(sizeof(T)); i < n; i += kBlockThreads * uint32_t(sizeof(T))) {
-            const uint32_t at[1] = {i};
+        const uint32_t i = threadIdx.x * uint32_t(sizeof(T));
+        if (i < EndBytes(d)) {
+            const uint64_t off = EndOffset(d, i);
+            const uint32_t at[1] = {0};
             T x[1];
-            StackValue<ElemLane<T, OP>, T, OP, 1, true, 8>(d, src, ops, 0, at, x);
+            StackValue<ElemLane<T, OP>, T, OP, 1, true, 8>(d, src, ops, off, at, x);
             for (uint32_t k = 0; k < d.ndst; k++) {
-                StoreElem<T>(dst[k], i, x[0]);
+                StoreElem<T>(dst[k], off, x[0]);
             }
         }
     }
 }
 
 template <typename T, int OP>
-__global__ void __launch_bounds__(kBlockThreads) StackKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole,
+__global__ void __launch_bounds__(kBlockThreads) StackKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nall, uint32_t nwhole,
     uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem)
 {
-    const uint32_t *opPool = reinterpret_cast<const uint32_t *>(items + nitems + (ntiles - nwhole));
+    const uint32_t *opPool = reinterpret_cast<const uint32_t *>(items + nall);
     uint32_t pos[kChainVec];
     TilePositions(pos);
-    WalkTiles(items, nitems, nwhole, ntiles, tilesPerItem, [](const FusedDesc &) { return 0; },
+    WalkTiles(items, nitems, nall, nwhole, ntiles, tilesPerItem, [](const FusedDesc &) { return 0; },
         [&](const FusedDesc &d, int, uint64_t off) {
             StackStore<T, OP, kStackPlainBatch>(d, srcPool + d.srcBase, opPool + d.srcBase, dstPool + d.dstBase, off, kTileBytes, pos, pos);
         },
-        [&](const FusedDesc &d) { StackRest<T, OP>(d, srcPool + d.srcBase, opPool + d.srcBase, dstPool + d.dstBase); });
+        [&](const FusedDesc &d, bool ends) { StackRest<T, OP>(d, ends, srcPool + d.srcBase, opPool + d.srcBase, dstPool + d.dstBase); });
 }
 
 }  // namespace hcclamd

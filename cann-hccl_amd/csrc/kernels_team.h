@@ -203,14 +203,14 @@ template <uint32_t N> struct TeamPlaces {
 };
 
 // Eval: Read(round, srcPool, extra, park) evaluates the round's tiles and leaves the vectors of tile q at
-// park[q * kTeamVecPerTile]; the static Rest(d, srcPool, extra, dstPool) handles an item behind the whole tiles there and then.
+// park[q * kTeamVecPerTile]; the static Rest(d, ends, srcPool, extra, dstPool) handles an item's rest or its ends there and then.
 //
 // The whole tiles are cut into regions (first tile, number of tiles), a table the host wrote behind the counters:
 // workgroup i of a team of n takes the tiles first + i, first + i + n, ... of the team's region.  Team x starts
 // with region x; the later ones are drawn from a counter as the teams get there, and the last regions are smaller,
 // so that the XCDs, which do not all move data at the same rate, finish together.
 template <typename Eval>
-__device__ __forceinline__ void TeamBody(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole, uint32_t ntiles,
+__device__ __forceinline__ void TeamBody(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nall, uint32_t nwhole, uint32_t ntiles,
     const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem,
     uint32_t *__restrict__ teamCtr, const void *extra)
 {
@@ -224,11 +224,12 @@ __device__ __forceinline__ void TeamBody(const FusedDesc *__restrict__ items, ui
     const TeamRegion *regions = reinterpret_cast<const TeamRegion *>(teamCtr + kTeamHeaderWords);
     uint32_t *slots = teamCtr + kTeamHeaderWords + 2u * nregions + xcd * (nregions + 1u);
     uint32_t *ctr = teamCtr + xcd * kTeamCtrStride;
-    uint32_t nextRest = nitems + blockIdx.x;
+    uint32_t nextRest = blockIdx.x;
     auto rests = [&]() __attribute__((always_inline)) {
-        for (; nextRest < nitems + (ntiles - nwhole); nextRest += gridDim.x) {
-            const FusedDesc d = items[nextRest];
-            Eval::Rest(d, srcPool + d.srcBase, extra, dstPool + d.dstBase);
+        for (; nextRest < ntiles - nwhole; nextRest += gridDim.x) {
+            const bool ends = nextRest >= nall;
+            const FusedDesc d = items[ends ? nextRest - nall : nextRest];
+            Eval::Rest(d, ends, srcPool + d.srcBase, extra, dstPool + d.dstBase);
         }
     };
     uint32_t target = 0;
@@ -242,7 +243,7 @@ __device__ __forceinline__ void TeamBody(const FusedDesc *__restrict__ items, ui
             Eval::Read(r, srcPool, extra, park);
         }
         target += teamSize;
-        // The items behind the whole tiles, a few short pieces, cost no time of their own there.  (Every team has a round: the
+        // The items' rests and ends, a few short pieces, cost no time of their own there.  (Every team has a round: the
         // host makes at least kTeamXcds regions.  One call: called twice, this is not inlined.)
         region = TeamBarrier(ctr, target, slots + round, teamCtr + kTeamTicket, seen, &nextShared, rests);
         // Every lane reads back the vectors it parked itself.  A workgroup's tiles mostly belong to one item, so its
@@ -422,7 +423,7 @@ template <typename T, int OP> struct TeamChainEval {
                     held = d.srcBase;
 #pragma unroll
                     for (uint32_t j = 0; j < 8; j++) {
-                        sp[j] = srcPool[d.srcBase + j];       // (the pool is padded)
+                        sp[j] = srcPool[d.srcBase + j];       // (more lies behind the pool)
                     }
                 }
                 ChainFew<FoldLane<T, OP>, T, OP, kChainVec>(d.nsrc, d.accLeftMask, sp, off, pos, acc);
@@ -432,9 +433,9 @@ template <typename T, int OP> struct TeamChainEval {
             TeamPark(to, 0, acc);
         });
     }
-    static __device__ __forceinline__ void Rest(const FusedDesc &d, const void *const *__restrict__ src, const void *, void *const *__restrict__ dst)
+    static __device__ __forceinline__ void Rest(const FusedDesc &d, bool ends, const void *const *__restrict__ src, const void *, void *const *__restrict__ dst)
     {
-        ChainRest<T, OP>(d, src, dst);
+        ChainRest<T, OP>(d, ends, src, dst);
     }
 };
 
@@ -488,9 +489,9 @@ struct TeamCopyEval {
                 break;
         }
     }
-    static __device__ __forceinline__ void Rest(const FusedDesc &d, const void *const *__restrict__ src, const void *, void *const *__restrict__ dst)
+    static __device__ __forceinline__ void Rest(const FusedDesc &d, bool ends, const void *const *__restrict__ src, const void *, void *const *__restrict__ dst)
     {
-        CopyRest(d, src[0], dst);
+        CopyRest(d, ends, src[0], dst);
     }
 };
 
@@ -505,9 +506,9 @@ template <typename T, int OP> struct TeamTreeEval {
             TeamPark(to, 0, x);
         });
     }
-    static __device__ __forceinline__ void Rest(const FusedDesc &d, const void *const *__restrict__ src, const void *, void *const *__restrict__ dst)
+    static __device__ __forceinline__ void Rest(const FusedDesc &d, bool ends, const void *const *__restrict__ src, const void *, void *const *__restrict__ dst)
     {
-        TreeRest<T, OP>(d, src, dst);
+        TreeRest<T, OP>(d, ends, src, dst);
     }
 };
 
@@ -675,9 +676,9 @@ template <typename T, int OP, bool ROUNDS> struct TeamStackEval {
                 [&](uint32_t h, const auto &x) { TeamPark(to, h, x); });
         });
     }
-    static __device__ __forceinline__ void Rest(const FusedDesc &d, const void *const *__restrict__ src, const void *extra, void *const *__restrict__ dst)
+    static __device__ __forceinline__ void Rest(const FusedDesc &d, bool ends, const void *const *__restrict__ src, const void *extra, void *const *__restrict__ dst)
     {
-        StackRest<T, OP>(d, src, static_cast<const uint32_t *>(extra) + d.srcBase, dst);
+        StackRest<T, OP>(d, ends, src, static_cast<const uint32_t *>(extra) + d.srcBase, dst);
     }
 };
 
@@ -685,35 +686,35 @@ template <typename T, int OP, bool ROUNDS> struct TeamStackEval {
 // kernels.h).  Launched with one workgroup per CU
 // (a multiple of kTeamXcds workgroups) and kTeamDynamicLds bytes of dynamic LDS.
 template <typename T, int OP>
-__global__ void __launch_bounds__(kBlockThreads) TeamChainKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole,
+__global__ void __launch_bounds__(kBlockThreads) TeamChainKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nall, uint32_t nwhole,
     uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem,
     uint32_t *__restrict__ teamCtr)
 {
-    TeamBody<TeamChainEval<T, OP>>(items, nitems, nwhole, ntiles, srcPool, dstPool, tilesPerItem, teamCtr, nullptr);
+    TeamBody<TeamChainEval<T, OP>>(items, nitems, nall, nwhole, ntiles, srcPool, dstPool, tilesPerItem, teamCtr, nullptr);
 }
 
 template <int Variant>
-__global__ void __launch_bounds__(kBlockThreads) TeamCopyKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole,
+__global__ void __launch_bounds__(kBlockThreads) TeamCopyKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nall, uint32_t nwhole,
     uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem,
     uint32_t *__restrict__ teamCtr)
 {
-    TeamBody<TeamCopyEval>(items, nitems, nwhole, ntiles, srcPool, dstPool, tilesPerItem, teamCtr, nullptr);
+    TeamBody<TeamCopyEval>(items, nitems, nall, nwhole, ntiles, srcPool, dstPool, tilesPerItem, teamCtr, nullptr);
 }
 
 template <typename T, int OP>
-__global__ void __launch_bounds__(kBlockThreads) TeamTreeKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole,
+__global__ void __launch_bounds__(kBlockThreads) TeamTreeKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nall, uint32_t nwhole,
     uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem,
     uint32_t *__restrict__ teamCtr)
 {
-    TeamBody<TeamTreeEval<T, OP>>(items, nitems, nwhole, ntiles, srcPool, dstPool, tilesPerItem, teamCtr, nullptr);
+    TeamBody<TeamTreeEval<T, OP>>(items, nitems, nall, nwhole, ntiles, srcPool, dstPool, tilesPerItem, teamCtr, nullptr);
 }
 
 template <typename T, int OP, bool ROUNDS>
-__global__ void __launch_bounds__(kBlockThreads) TeamStackKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nwhole,
+__global__ void __launch_bounds__(kBlockThreads) TeamStackKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nall, uint32_t nwhole,
     uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem,
     uint32_t *__restrict__ teamCtr)
 {
-    TeamBody<TeamStackEval<T, OP, ROUNDS>>(items, nitems, nwhole, ntiles, srcPool, dstPool, tilesPerItem, teamCtr, items + nitems + (ntiles - nwhole));
+    TeamBody<TeamStackEval<T, OP, ROUNDS>>(items, nitems, nall, nwhole, ntiles, srcPool, dstPool, tilesPerItem, teamCtr, items + nall);
 }
 
 }  // namespace hcclamd

@@ -19,15 +19,20 @@ enum AnchorRule : int {
                         // reduce-scatter of odd blocks reads all its sources aligned and writes its one destination unaligned
 };
 
-// Cuts [0, bytes) into an element-wise head, a 16-byte vector body and an element-wise tail, given
-// the addresses involved (the first one is a destination; all are multiples of the element size).
+// A stretch of bytes cut into an element-wise head, a 16-byte vector body and an element-wise tail.
+struct Cut {
+    uint64_t head, body, tail;
+    bool aligned;          // every pointer is on a 16-byte boundary where the body starts
+};
+
+// Cuts [0, bytes), given the addresses involved (the first one is a destination; all are multiples of the element size).
 // The head brings the anchor's pointers to a 16-byte boundary; those that are then not on one
-// too are accessed with unaligned 128-bit accesses (ACC_VEC16_ANY).  emit(offset, bytes, mode).
+// too are accessed with unaligned 128-bit accesses.
 // The head of a long stretch reaches to a 128-byte boundary of those pointers:
 // a wave stores 1 KiB at a time, and when those stores straddle memory lines every line is written in
 // two pieces (measured, 8-rank fp32 all-reduce of 256 MiB per rank with all buffers 16 bytes off a
 // 128-byte boundary: 0.97 ms fused against 0.76 ms aligned).
-template <typename F> void SplitByAlignment(const std::vector<uintptr_t> &addrs, uint64_t bytes, AnchorRule rule, F emit)
+inline Cut CutByAlignment(const std::vector<uintptr_t> &addrs, uint64_t bytes, AnchorRule rule)
 {
     size_t count[16] = {0};
     for (uintptr_t a : addrs) {
@@ -40,16 +45,7 @@ template <typename F> void SplitByAlignment(const std::vector<uintptr_t> &addrs,
     const uint64_t align = bytes >= 4 * uint64_t(kTileBytes) + 128 ? 128 : 16;
     const uint64_t head = std::min<uint64_t>(bytes, (align - (anchor & (align - 1))) & (align - 1));
     const uint64_t body = (bytes - head) & ~uint64_t(15);
-    const uint64_t tail = bytes - head - body;
-    if (head) {
-        emit(uint64_t(0), head, uint32_t(ACC_ELEM));
-    }
-    if (body) {
-        emit(head, body, uint32_t(count[anchor & 15] == addrs.size() ? ACC_VEC16 : ACC_VEC16_ANY));
-    }
-    if (tail) {
-        emit(head + body, tail, uint32_t(ACC_ELEM));
-    }
+    return Cut{head, body, bytes - head - body, count[anchor & 15] == addrs.size()};
 }
 
 }  // namespace hcclamd

@@ -63,9 +63,10 @@ struct LaunchRec {
     uint32_t grid = 0;
     uint32_t dynamicLds = 0;      // bytes of dynamic LDS the launch asks for (team kernels)
     // kernel arguments: step kernels take (table, nitems, nwhole, ntiles, flags), fused kernels
-    // (table, nitems, nwhole, ntiles, srcPool, dstPool, tilesPerItem), their team forms one more: (..., teamCtr)
+    // (table, nitems, nall, nwhole, ntiles, srcPool, dstPool, tilesPerItem), their team forms one more: (..., teamCtr)
     const void *table = nullptr;
-    uint32_t nitems = 0;
+    uint32_t nitems = 0;          // fused: items that have whole tiles, the first ones of the table
+    uint32_t nall = 0;            // fused: all items
     uint32_t ntiles = 0;
     uint32_t nwhole = 0;
     uint32_t flags = 0;

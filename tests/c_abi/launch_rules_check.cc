@@ -35,31 +35,26 @@ void CheckSplit()
         }
         const uint64_t bytes = unit * (Draw(2) != 0 ? Draw(200) : Draw(40000));
         for (AnchorRule rule : {ANCHOR_FIRST, ANCHOR_MOST}) {
-            uint64_t at = 0;
-            SplitByAlignment(addrs, bytes, rule, [&](uint64_t off, uint64_t n, uint32_t mode) {
-                CHECK(off == at && n != 0);
-                at += n;
-                CHECK(n % unit == 0);
-                if (mode == ACC_ELEM) {
-                    CHECK(n < 128);
-                    return;
-                }
-                CHECK(n % 16 == 0);
-                size_t agree[16] = {0}, most = 0;
-                for (uintptr_t a : addrs) {
-                    most = std::max(most, ++agree[(a + off) & 15]);
-                }
-                CHECK((agree[0] == addrs.size()) == (mode == ACC_VEC16));
-                if (rule == ANCHOR_FIRST) {
-                    CHECK(((addrs[0] + off) & 15) == 0);      // the step kernel's aligned stores
-                    CHECK(bytes < 4 * uint64_t(kTileBytes) + 128 || ((addrs[0] + off) & 127) == 0);
-                } else {
-                    CHECK(agree[0] == most);
-                }
-                bodies++;
-                unaligned += mode == ACC_VEC16_ANY ? 1 : 0;
-            });
-            CHECK(at == bytes);
+            const Cut cut = CutByAlignment(addrs, bytes, rule);
+            CHECK(cut.head + cut.body + cut.tail == bytes);
+            CHECK(cut.head < 128 && cut.tail < 16 && cut.body % 16 == 0);      // (a fused item's ends are one pass of a workgroup)
+            CHECK(cut.head % unit == 0 && cut.tail % unit == 0);
+            if (cut.body == 0) {
+                continue;
+            }
+            size_t agree[16] = {0}, most = 0;
+            for (uintptr_t a : addrs) {
+                most = std::max(most, ++agree[(a + cut.head) & 15]);
+            }
+            CHECK((agree[0] == addrs.size()) == cut.aligned);
+            if (rule == ANCHOR_FIRST) {
+                CHECK(((addrs[0] + cut.head) & 15) == 0);      // the step kernel's aligned stores
+                CHECK(bytes < 4 * uint64_t(kTileBytes) + 128 || ((addrs[0] + cut.head) & 127) == 0);
+            } else {
+                CHECK(agree[0] == most);
+            }
+            bodies++;
+            unaligned += cut.aligned ? 0 : 1;
         }
     }
     CHECK(bodies > 30000 && unaligned > 5000);

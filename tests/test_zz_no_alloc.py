@@ -78,6 +78,23 @@ def test_reduce_scatter_no_alloc_rejects_what_does_not_fit(orc):
         g.close()
 
 
+@pytest.mark.parametrize("p,n", [(24, 100003), (16, 100003), (24, 40961)])
+def test_reduce_scatter_no_alloc_of_a_cut_schedule(orc, p, n):
+    # the piece-cut mesh: hundreds of items, blocks that start at every offset from a 16-byte boundary.  An item is one entry
+    # and one list of pointers whatever its ends are (24 ranks: 552 items, 140 KiB of the 256 KiB of tables)
+    g = gh.Group(p, algo="mesh", deterministic=1)
+    try:
+        ins = _ins(FP32, p, n * p, 31 * n + p)
+        ref, got, info = _both(g, ins, FP32, SUM)
+        want = orc.reducescatter(ins, FP32, SUM, algo=1, threads=8)
+        for r in range(p):
+            assert gh.same(FP32, got[r], ref[r]), r
+            assert gh.same(FP32, got[r], want[r]), r
+        assert info["fused"] == 1
+    finally:
+        g.close()
+
+
 def test_reduce_scatter_no_alloc_on_a_group_assembled_rank_by_rank(orc):
     # communicators made with HcclCommInitRootInfo: the device is set up when the last rank joins, so the first
     # collective of the group may be the one that allocates nothing

@@ -239,8 +239,6 @@ struct PendingLaunch {
 // ring reduce 886 / 840, ring broadcast 615 / 579 (every phase forwards what the previous one wrote,
 // 256 MiB or less per phase); halving-doubling all-reduce 1544 / 1685, mesh broadcast 583 / 638 (phases
 // of 1 GiB and more); uniform all-to-all 727 / 785 (nothing is read back).
-constexpr uint64_t kMemorySideCacheBytes = 256ull << 20;
-
 bool PreferOrdinaryStores(const Plan &plan, const std::vector<void *> &send, const std::vector<void *> &recv)
 {
     typedef std::pair<uint32_t, uint8_t> Where;   // (rank, buffer); a send buffer that is the receive buffer counts as it
@@ -509,6 +507,10 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                 pending.push_back(pl);
             }
         }
+        uint64_t moved = 0;       // bytes read and written, all launches
+        for (const FusedItem &it : pp->plan->fused) {
+            moved += it.bytes * (it.dst.size() + uint64_t(std::count(it.srcValid.begin(), it.srcValid.end(), 1)));
+        }
         // one launch per kernel kind present, or several under a launch cap: the items in their order, cut where the
         // bytes a launch moves (read and written) reach the cap
         for (int kind : {int(KK_CHAIN), int(KK_TREE), int(KK_STACK)}) {
@@ -612,7 +614,8 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                 if (reduceColl && !team && kind == int(KK_CHAIN) && (toOne || tiles > g->numCu)) {
                     pl.rec.func = LookupKernel(dtype, op, KK_CHAIN_SLOW);
                 }
-                const uint32_t flags = (fusedOrdinary ? kFusedOrdinaryStores : 0u) | (through ? kFusedThroughStores : 0u) | (alike ? kFusedAlike : 0u);
+                const bool copyThrough = !reduceColl && !team && !fusedOrdinary && g->cfg.fusedStores < 0 && CopiesWriteThrough(traffic, written, moved);
+                const uint32_t flags = (fusedOrdinary ? kFusedOrdinaryStores : 0u) | (through || copyThrough ? kFusedThroughStores : 0u) | (alike ? kFusedAlike : 0u);
                 // the op words of the stack kernel sit right behind its item table
                 descs.insert(descs.end(), shorts.begin(), shorts.end());
                 pl.tableAt = b.Reserve(descs.size() * sizeof(FusedDesc) + opPool.size() * sizeof(uint32_t));

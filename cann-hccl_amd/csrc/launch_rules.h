@@ -1,5 +1,5 @@
-// How the executor cuts a stretch of bytes by the alignment of its buffers.  Pure C++: no HIP calls, so the rules can be
-// checked without a GPU.
+// Rules of the executor on sizes and alignment: how a stretch of bytes is cut, how results are stored.  Pure C++: no HIP
+// calls, so the rules can be checked without a GPU.
 #pragma once
 #include <algorithm>
 #include <cstddef>
@@ -46,6 +46,20 @@ inline Cut CutByAlignment(const std::vector<uintptr_t> &addrs, uint64_t bytes, A
     const uint64_t head = std::min<uint64_t>(bytes, (align - (anchor & (align - 1))) & (align - 1));
     const uint64_t body = (bytes - head) & ~uint64_t(15);
     return Cut{head, body, bytes - head - body, count[anchor & 15] == addrs.size()};
+}
+
+constexpr uint64_t kMemorySideCacheBytes = 256ull << 20;
+
+// Whether a launch of the plain copy kernel writes its results through (StorePolicy, kernels_impl.h) instead of non-temporally:
+// `traffic` bytes read and written by the launch, `written` of them written, `moved` read and written by the whole collective, whose
+// launches all store alike.  Up to 512 MiB in all, us, non-temporal / through: all-gather 2 ranks 10 MiB 10.4 / 7.4, 64 MiB
+// (384 MiB moved) 67.7 / 60.1; 3 ranks 8 MiB 17.2 / 12.0, 32 MiB (384) 71.5 / 59.9; 8 ranks 2 MiB 28.2 / 20.1; 16 ranks 1 MiB 53.7 / 38.7;
+// uniform all-to-all 8 ranks 8 MiB 21.3 / 20.3, 32 MiB (512) 84.5 / 75.7.  Beyond, the one loses what the other
+// gains: 2 ranks 128 MiB (768) 139.5 / 143.8, 3 ranks 48 MiB (576) 107.8 / 111.7, all-to-all 64 MiB (1024) 170.0 / 172.5 -- unless every
+// block goes to four destinations or more: 5 ranks 24 MiB (720) 150.5 / 147.6, 6 ranks 24 MiB (1008) 217.8 / 210.7, 32 MiB 295 / 281.
+inline bool CopiesWriteThrough(uint64_t traffic, uint64_t written, uint64_t moved)
+{
+    return moved <= 2 * kMemorySideCacheBytes || 5 * written >= 4 * traffic;
 }
 
 }  // namespace hcclamd

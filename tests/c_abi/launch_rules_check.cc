@@ -60,11 +60,25 @@ void CheckSplit()
     CHECK(bodies > 30000 && unaligned > 5000);
 }
 
+// All launches of a collective of one shape store alike, however the cap cut it.
+void CheckCopyStores()
+{
+    for (int round = 0; round < 2000; round++) {
+        const uint64_t ndst = 1 + Draw(8), block = 1 + Draw(uint64_t(200) << 20), items = 1 + Draw(64), moved = items * block * (1 + ndst);
+        const bool whole = CopiesWriteThrough(moved, items * block * ndst, moved);
+        CHECK(whole == (ndst >= 4 || moved <= 2 * kMemorySideCacheBytes));
+        for (uint64_t n = 1; n <= items; n++) {
+            CHECK(CopiesWriteThrough(n * block * (1 + ndst), n * block * ndst, moved) == whole);
+        }
+    }
+}
+
 }  // namespace
 
 int main()
 {
     CheckSplit();
+    CheckCopyStores();
     std::printf("OK\n");
     return 0;
 }

@@ -173,58 +173,9 @@ struct Builder {
 };
 
 constexpr size_t kGraphMinLaunches = 12;   // fewer launches go out one by one
-// The team kernels are chosen for launches of at least this many halves of a round.  All-reduce, us, plain / team: 8 ranks,
-// fp32, 12 MiB (768 tiles) 36.0 / 36.6, 16 MiB (1024, half a round) 49.5 / 46.2, 24 MiB 72.4 / 68.2, 32 MiB 96.3 / 88.0, 48 MiB 145.4 /
-// 137.3; 32 ranks, bf16 halving-doubling (a round is 1024 tiles), 4 MiB (256) 45.3 / 46.6, 8 MiB (512) 95.1 / 87.8, 16 MiB 209 / 172.5.
-constexpr uint32_t kTeamMinHalfRounds = 1;
-// Items with fewer than 12 sources and destinations (4 ranks, fp32): 16 MiB 24.3 / 26.1, 32 MiB (a round) 48.0 / 47.4, 48 MiB 70.5 / 74.8,
-// 64 MiB 93.6 / 95.1, 128 MiB (4 rounds) 188.5 / 183.3.
-constexpr uint32_t kTeamMinHalfRoundsFew = 8;
-// One source and many destinations: 8-rank all-gather, blocks of 2 MiB (1024 tiles) 25.9 / 30.0, 4 MiB (2048, a round) 60.0 / 54.2,
-// 8 MiB 122.9 / 105.4; 16 ranks 1 MiB (1024) 54.8 / 53.4, 2 MiB 121.2 / 100.9.
-constexpr uint32_t kTeamMinHalfRoundsCopy = 2;
 constexpr size_t kAsyncUploadBytes = 4 * kNoAllocUploadBytes;   // tables up to this size are uploaded by launches
 
 uint32_t TilesOf(uint64_t bytes) { return uint32_t((bytes + kTileBytes - 1) / kTileBytes); }
-
-// The regions the teams of a launch draw (kernels_team.h): roundTiles tiles per workgroup; over the last quarter of the
-// tiles the size is halved whenever fewer than 8 regions of the current size are left.  The XCDs do not all move data at
-// the same rate, and with regions that get smaller towards the end they finish together (measured, 8 x 256 MiB fp32
-// all-reduce: 727 us with 64 equal regions dealt out in order, 714 us with the shrinking tail
-// drawn from the counter; shrinking earlier costs more than it brings, small regions run slower --
-// the more so since rounds of many whole tiles are read in one piece: with "fewer than 16"
-// all-gather and broadcast took 2 % longer, the all-reduces 1 %).
-// Less than two rounds: a full one and what is left dealt out evenly, or one round of what there is.  All-reduce of 8 ranks, fp32,
-// us, this way / two equal rounds / the rule above: 40 MiB 113.5 / 118.6 / 111.7, 48 MiB 136.6 / 140.2 / 147.4, 56 MiB 161.9 / 161.8 / 158.4;
-// all-gather 8 x 6 MiB 80.7 / - / 92.0.
-std::vector<TeamRegion> TeamRegions(uint32_t tiles, uint32_t ntiles, uint32_t roundTiles, uint32_t perTeam)
-{
-    std::vector<TeamRegion> regions;
-    const uint32_t round = roundTiles * perTeam * kTeamXcds;
-    uint32_t per = roundTiles;
-    for (uint32_t at = 0; at < tiles;) {
-        const uint32_t left = tiles - at;
-        if (ntiles < 2 * round) {
-            const uint32_t teamsLeft = kTeamXcds - uint32_t(regions.size()) % kTeamXcds;
-            const uint32_t n = std::min(roundTiles * perTeam, (left + teamsLeft - 1) / teamsLeft);
-            regions.push_back(TeamRegion{at, n});
-            at += n;
-            continue;
-        }
-        if (uint64_t(at) * 4 >= uint64_t(tiles) * 3) {
-            while (per > 1 && uint64_t(per) * perTeam * 8 > left) {
-                per /= 2;
-            }
-        }
-        const uint32_t n = std::min(left, per * perTeam);
-        regions.push_back(TeamRegion{at, n});
-        at += n;
-    }
-    while (regions.size() < kTeamXcds) {
-        regions.push_back(TeamRegion{tiles, 0});     // every team has a round (the items behind the whole tiles are handled there)
-    }
-    return regions;
-}
 
 struct PendingLaunch {
     LaunchRec rec;
@@ -556,6 +507,7 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                 const bool teamFits = teamFunc != nullptr && g->numCu >= kTeamXcds && g->numCu % kTeamXcds == 0 && g->cfg.blocksPerCu == 0;
                 bool team = teamFits && g->cfg.team == 1;
                 double storeStreams = 0, allStreams = 0, bytes = 0;
+                uint64_t whole = 0;       // bytes of the items that have whole tiles
                 if (teamFits && g->cfg.team != 0) {
                     for (const FusedDesc &d : descs) {
                         uint32_t nsrc = 0;
@@ -565,6 +517,7 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                         storeStreams += double(d.ndst) * double(d.bytes);
                         allStreams += double(d.ndst + nsrc) * double(d.bytes);
                         bytes += double(d.bytes);
+                        whole += d.bytes + d.head + d.tail;
                     }
                     // A round should keep a workgroup busy for a mebibyte or two per phase (8 tiles of 8 streams): fewer
                     // tiles per round when a tile has many more sources or destinations than that (measured, 32-rank
@@ -576,7 +529,7 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                     if (g->cfg.team < 0) {
                         const uint32_t halfRounds = !reduceColl ? kTeamMinHalfRoundsCopy : (allStreams < 12.0 * bytes ? kTeamMinHalfRoundsFew : kTeamMinHalfRounds);
                         team = bytes > 0 && storeStreams >= 4.0 * bytes && allStreams >= 8.0 * bytes &&
-                            2 * pl.rec.ntiles >= halfRounds * pl.rec.roundTiles * g->numCu;
+                            TeamRounds(whole, halfRounds, pl.rec.roundTiles, g->numCu);
                     }
                 }
                 if (team) {
@@ -598,7 +551,7 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                     if (kind == int(KK_STACK) && inShort > tiles / 4) {
                         pl.rec.func = LookupKernel(dtype, op, KK_TEAM_STACK_TILES);
                     }
-                    const std::vector<TeamRegion> regions = TeamRegions(tiles, pl.rec.ntiles, pl.rec.roundTiles, perX);
+                    const std::vector<TeamRegion> regions = TeamRegions(tiles, whole, pl.rec.roundTiles, perX);
                     const uint32_t n = uint32_t(regions.size());
                     pl.ctrAt = b.Reserve(size_t(TeamBlockWords(n)) * 4);     // zero in the image, and zero again after every launch
                     uint32_t *block = reinterpret_cast<uint32_t *>(b.host.data() + pl.ctrAt);

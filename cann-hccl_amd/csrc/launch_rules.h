@@ -1,5 +1,5 @@
-// Rules of the executor on sizes and alignment: how a stretch of bytes is cut, how results are stored.  Pure C++: no HIP
-// calls, so the rules can be checked without a GPU.
+// Rules of the executor on sizes and alignment: how a stretch of bytes is cut, which tiles the teams take, how results
+// are stored.  Pure C++: no HIP calls, so the rules can be checked without a GPU.
 #pragma once
 #include <algorithm>
 #include <cstddef>
@@ -46,6 +46,64 @@ inline Cut CutByAlignment(const std::vector<uintptr_t> &addrs, uint64_t bytes, A
     const uint64_t head = std::min<uint64_t>(bytes, (align - (anchor & (align - 1))) & (align - 1));
     const uint64_t body = (bytes - head) & ~uint64_t(15);
     return Cut{head, body, bytes - head - body, count[anchor & 15] == addrs.size()};
+}
+
+// The team kernels are chosen for launches of at least this many halves of a round of whole tiles.  All-reduce, us, plain / team: 8 ranks,
+// fp32, 12 MiB (768 tiles) 36.0 / 36.6, 16 MiB (1024, half a round) 49.5 / 46.2, 24 MiB 72.4 / 68.2, 32 MiB 96.3 / 88.0, 48 MiB 145.4 /
+// 137.3; 32 ranks, bf16 halving-doubling (a round is 1024 tiles), 4 MiB (256) 45.3 / 46.6, 8 MiB (512) 95.1 / 87.8, 16 MiB 209 / 172.5.
+constexpr uint32_t kTeamMinHalfRounds = 1;
+// Items with fewer than 12 sources and destinations (4 ranks, fp32): 16 MiB 24.3 / 26.1, 32 MiB (a round) 48.0 / 47.4, 48 MiB 70.5 / 74.8,
+// 64 MiB 93.6 / 95.1, 128 MiB (4 rounds) 188.5 / 183.3.
+constexpr uint32_t kTeamMinHalfRoundsFew = 8;
+// One source and many destinations: 8-rank all-gather, blocks of 2 MiB (1024 tiles) 25.9 / 30.0, 4 MiB (2048, a round) 60.0 / 54.2,
+// 8 MiB 122.9 / 105.4; 16 ranks 1 MiB (1024) 54.8 / 53.4, 2 MiB 121.2 / 100.9.
+constexpr uint32_t kTeamMinHalfRoundsCopy = 2;
+
+// Whether a launch whose items with whole tiles have `bytes` in all runs that long.  (By bytes, not by tiles: a buffer that starts
+// off a boundary leaves every item a tile short, and many short pieces are no round.)
+inline bool TeamRounds(uint64_t bytes, uint32_t halfRounds, uint32_t roundTiles, uint32_t workgroups)
+{
+    return 2 * bytes >= uint64_t(halfRounds) * roundTiles * workgroups * kTileBytes;
+}
+
+// The regions the teams of a launch draw (kernels_team.h): roundTiles tiles per workgroup; over the last quarter of the
+// tiles the size is halved whenever fewer than 8 regions of the current size are left.  The XCDs do not all move data at
+// the same rate, and with regions that get smaller towards the end they finish together (measured, 8 x 256 MiB fp32
+// all-reduce: 727 us with 64 equal regions dealt out in order, 714 us with the shrinking tail
+// drawn from the counter; shrinking earlier costs more than it brings, small regions run slower --
+// the more so since rounds of many whole tiles are read in one piece: with "fewer than 16"
+// all-gather and broadcast took 2 % longer, the all-reduces 1 %).
+// Less than two rounds (by `bytes`, see TeamRounds: a buffer off a boundary by a few bytes is dealt out like one on it; 8 ranks
+// x 64 MiB 12 bytes off a boundary 177.9 us, by whole tiles 186.4): a full one and what is left dealt out evenly, or one round of
+// what there is.  All-reduce of 8 ranks, fp32, us, this way / two equal rounds / the rule above: 40 MiB 113.5 / 118.6 / 111.7,
+// 48 MiB 136.6 / 140.2 / 147.4, 56 MiB 161.9 / 161.8 / 158.4; all-gather 8 x 6 MiB 80.7 / - / 92.0.
+inline std::vector<TeamRegion> TeamRegions(uint32_t tiles, uint64_t bytes, uint32_t roundTiles, uint32_t perTeam)
+{
+    std::vector<TeamRegion> regions;
+    const bool even = !TeamRounds(bytes, 4, roundTiles, perTeam * kTeamXcds);
+    uint32_t per = roundTiles;
+    for (uint32_t at = 0; at < tiles;) {
+        const uint32_t left = tiles - at;
+        if (even) {
+            const uint32_t teamsLeft = kTeamXcds - uint32_t(regions.size()) % kTeamXcds;
+            const uint32_t n = std::min(roundTiles * perTeam, (left + teamsLeft - 1) / teamsLeft);
+            regions.push_back(TeamRegion{at, n});
+            at += n;
+            continue;
+        }
+        if (uint64_t(at) * 4 >= uint64_t(tiles) * 3) {
+            while (per > 1 && uint64_t(per) * perTeam * 8 > left) {
+                per /= 2;
+            }
+        }
+        const uint32_t n = std::min(left, per * perTeam);
+        regions.push_back(TeamRegion{at, n});
+        at += n;
+    }
+    while (regions.size() < kTeamXcds) {
+        regions.push_back(TeamRegion{tiles, 0});     // every team has a round (the items behind the whole tiles are handled there)
+    }
+    return regions;
 }
 
 constexpr uint64_t kMemorySideCacheBytes = 256ull << 20;

@@ -60,6 +60,39 @@ void CheckSplit()
     CHECK(bodies > 30000 && unaligned > 5000);
 }
 
+// The regions cover the whole tiles in order, none holds more than its team can park, and every team has one; short of a round
+// every team gets as many tiles as the others.
+void CheckTeamRegions()
+{
+    for (int round = 0; round < 20000; round++) {
+        const uint32_t roundTiles = 1 + uint32_t(Draw(kTeamTiles)), perTeam = 1 + uint32_t(Draw(40)), all = roundTiles * perTeam * kTeamXcds;
+        const uint32_t tiles = uint32_t(Draw(2) != 0 ? Draw(all) : Draw(8 * uint64_t(all)));
+        const uint64_t pieces = Draw(uint64_t(tiles) + 1) * Draw(kTileBytes);      // behind the whole tiles: less than a tile for each item
+        const std::vector<TeamRegion> regions = TeamRegions(tiles, uint64_t(tiles) * kTileBytes + pieces, roundTiles, perTeam);
+        CHECK(regions.size() >= kTeamXcds);
+        uint32_t at = 0, least = tiles, most = 0;
+        for (const TeamRegion &r : regions) {
+            CHECK((r.first == at || r.count == 0) && r.count <= roundTiles * perTeam);
+            at += r.count;
+            least = std::min(least, r.count);
+            most = std::max(most, r.count);
+        }
+        CHECK(at == tiles && (tiles >= all || most - least <= 1));
+    }
+}
+
+// The line does not move with a buffer's start or with the number of pieces: the same bytes, cut anywhere.
+void CheckTeamRounds()
+{
+    for (int round = 0; round < 20000; round++) {
+        const uint32_t halfRounds = 1 + uint32_t(Draw(8)), roundTiles = 1 + uint32_t(Draw(kTeamTiles)), cus = 8 * (1 + uint32_t(Draw(40))), items = 1 + uint32_t(Draw(64));
+        const uint64_t line = uint64_t(halfRounds) * roundTiles * cus * kTileBytes / 2, each = (line + items - 1) / items + kTileBytes;
+        const Cut cut = CutByAlignment({(uintptr_t(1) << 40) + Draw(128)}, each, ANCHOR_MOST);
+        CHECK(TeamRounds(items * (cut.head + cut.body + cut.tail), halfRounds, roundTiles, cus));
+        CHECK(!TeamRounds(line - 1, halfRounds, roundTiles, cus));
+    }
+}
+
 // All launches of a collective of one shape store alike, however the cap cut it.
 void CheckCopyStores()
 {
@@ -78,6 +111,8 @@ void CheckCopyStores()
 int main()
 {
     CheckSplit();
+    CheckTeamRegions();
+    CheckTeamRounds();
     CheckCopyStores();
     std::printf("OK\n");
     return 0;

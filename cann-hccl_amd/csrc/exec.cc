@@ -403,11 +403,10 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
             launchNo++;
         }
     } else {
-        // Fused results are streamed past the caches (non-temporal stores) unless the caller asks for
-        // write-back stores.  Measured, 8-rank fp32 all-reduce replayed on the same buffers: write-back is
+        // Fused results are not written back unless the caller asks for it (StoreFlags).  Measured, 8-rank fp32
+        // all-reduce replayed on the same buffers, against non-temporal stores: write-back is
         // 5 % and 12 % faster at 16 and 32 MiB per rank (the output then stays in the 256 MB memory-side
         // cache), 20 % slower at 4 MiB and 7 % slower from 64 MiB per rank up.
-        const bool fusedOrdinary = g->cfg.fusedStores == 1;
         // Pure data movement in many short segments (an all-to-all-v of a few hundred bytes per pair): those go to
         // the gather kernel, a wave per segment through LDS, instead of a tile, a table search and up to three
         // descriptors each (measured, 64 ranks, 4096 segments of 430 bytes on average: 32 us with the tile kernel).
@@ -559,16 +558,13 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
                     std::memcpy(block + kTeamHeaderWords, regions.data(), regions.size() * sizeof(TeamRegion));
                 }
                 // Plain chains: all loads of a tile in flight while every CU has at most one tile, two sources at a time beyond
-                // that (ChainKernel); results with one destination are written through (StorePolicy, kernels_impl.h).
+                // that (ChainKernel), as where many sources become one result.
                 // All-reduce, us, all in flight / two sources: 8 ranks fp32 3 MiB (192 tiles) 8.9 / 9.4, 4 MiB (256) 11.4 / 11.6, 5 MiB 17.1 / 16.2,
                 // 8 MiB 22.3 / 21.6, 12 MiB 35.9 / 34.7; bf16 maximum 8 MiB 24.8 / 21.7; 4 ranks int8 6 MiB 11.4 / 9.2; 2 ranks fp32 64 MiB 46.8 / 44.9.
-                const bool toOne = reduceColl && !team && written * 3 <= traffic;
-                const bool through = toOne && !fusedOrdinary && g->cfg.fusedStores < 0 && traffic <= 2 * kMemorySideCacheBytes;
-                if (reduceColl && !team && kind == int(KK_CHAIN) && (toOne || tiles > g->numCu)) {
+                if (reduceColl && !team && kind == int(KK_CHAIN) && (written * 3 <= traffic || tiles > g->numCu)) {
                     pl.rec.func = LookupKernel(dtype, op, KK_CHAIN_SLOW);
                 }
-                const bool copyThrough = !reduceColl && !team && !fusedOrdinary && g->cfg.fusedStores < 0 && CopiesWriteThrough(traffic, written, moved);
-                const uint32_t flags = (fusedOrdinary ? kFusedOrdinaryStores : 0u) | (through || copyThrough ? kFusedThroughStores : 0u) | (alike ? kFusedAlike : 0u);
+                const uint32_t flags = StoreFlags(g->cfg.fusedStores, reduceColl, team, traffic, written, moved) | (alike ? kFusedAlike : 0u);
                 // the op words of the stack kernel sit right behind its item table
                 descs.insert(descs.end(), shorts.begin(), shorts.end());
                 pl.tableAt = b.Reserve(descs.size() * sizeof(FusedDesc) + opPool.size() * sizeof(uint32_t));

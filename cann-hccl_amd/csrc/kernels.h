@@ -53,14 +53,15 @@ struct FusedDesc {
     uint32_t srcBase;   // index into the source pointer pool
     uint32_t dstBase;   // index into the destination pointer pool
     uint32_t nleaf;
-    uint32_t flags;     // kFusedOrdinaryStores
+    uint32_t flags;     // kFused...
 };
 
-// flags of a fused item.  Stores: streamed past the caches unless one of the first two is set (StorePolicy, kernels_impl.h).
+// flags of a fused item.  Stores: one of the first two and kFusedNtStores (StorePolicy, kernels_impl.h), or, in the team kernels, none.
 constexpr uint32_t kFusedOrdinaryStores = 1u;  // write-back
 constexpr uint32_t kFusedThroughStores = 2u;   // written through to memory, without the non-temporal hint (plain kernels)
 constexpr uint32_t kFusedWordSources = 4u;     // 8-bit chains, copies: a source's body starts off a 4-byte boundary
 constexpr uint32_t kFusedPairs = 8u;           // trees: some leaf has a second source
+constexpr uint32_t kFusedNtStores = 32u;       // non-temporal
 constexpr uint32_t kFusedAlike = 16u;          // chains: all items of the launch have the same number of sources, two or more
 
 // flags of the step kernel

@@ -345,6 +345,7 @@ __device__ __forceinline__ void StoreAny16(void *base, uint64_t pos, V4 v)
 //   1 source, 8 destinations of 4, 24, 96 MiB        5.2 / 4.8 / 6.1 / 5.9   5.4 / 5.1 / 5.5 / 5.5   5.2 / 5.1 / 5.3 / 5.2
 //   8 sources, 1 destination of 8, 32, 48, 96 MiB    6.1 / - / 6.2 / 6.1   6.3 / - / 6.5 / 6.1   6.3 / - / 6.5 / 6.2   6.1 / - / 6.1 / 6.1
 //   one to one, 32, 96 MiB                           5.3 / - / 5.9 / 5.5   6.0 / - / 6.2 / 6.1
+// Which one: StoreFlags (launch_rules.h) for the plain kernels; the team kernels stream unless the caller has set otherwise.
 enum StorePolicy : uint32_t {
     STORE_ORDINARY = 0,      // write-back
     STORE_NT = 2,            // non-temporal
@@ -387,7 +388,7 @@ template <typename T> __device__ __forceinline__ void StoreElem(void *base, uint
 // one phase writes the next phase reads, and part of it is still in the memory-side cache then
 // (measured, 8-rank fp32 ring all-reduce of 256 MiB per rank, 14 phases: 1.478 ms with non-temporal
 // stores, 1.433 ms with ordinary ones; ordinary loads instead cost 9 %).  The fused kernels write
-// results nobody reads back and keep non-temporal stores (ordinary ones cost 7 % at 256 MiB per rank).
+// results nobody reads back (StorePolicy; ordinary stores cost them 7 % at 256 MiB per rank).
 __device__ __forceinline__ V4 StepLoad(const void *base, uint64_t byteOff)
 {
     return Load16<ACC_VEC16>(base, byteOff);

@@ -267,6 +267,8 @@ __device__ __forceinline__ void TeamBody(const FusedDesc *__restrict__ items, ui
                 char *to = o + uint64_t(reg.first + inTeam + q * teamSize - w.tile0) * kTileBytes;
                 if (w.flags & kFusedOrdinaryStores) {
                     TeamDrain<STORE_ORDINARY>(park + q * kTeamVecPerTile, to);
+                } else if (w.flags & kFusedNtStores) {
+                    TeamDrain<STORE_NT>(park + q * kTeamVecPerTile, to);
                 } else {
                     TeamDrain<STORE_STREAMED>(park + q * kTeamVecPerTile, to);
                 }

@@ -120,4 +120,22 @@ inline bool CopiesWriteThrough(uint64_t traffic, uint64_t written, uint64_t move
     return moved <= 2 * kMemorySideCacheBytes || 5 * written >= 4 * traffic;
 }
 
+// The same for a launch of the plain reducing kernels: many sources into one destination, up to 512 MiB in all.
+inline bool ResultsWriteThrough(uint64_t traffic, uint64_t written, uint64_t moved)
+{
+    return 3 * written <= traffic && moved <= 2 * kMemorySideCacheBytes;
+}
+
+// How a launch of a fused collective stores (flags of its items).  setting: "fused_stores", -1 "auto", 0 "nt", 1 "ordinary".
+inline uint32_t StoreFlags(int setting, bool reduces, bool team, uint64_t traffic, uint64_t written, uint64_t moved)
+{
+    if (setting >= 0) {
+        return setting == 1 ? kFusedOrdinaryStores : kFusedNtStores;
+    }
+    if (team) {
+        return 0;
+    }
+    return (reduces ? ResultsWriteThrough(traffic, written, moved) : CopiesWriteThrough(traffic, written, moved)) ? kFusedThroughStores : kFusedNtStores;
+}
+
 }  // namespace hcclamd

@@ -93,15 +93,24 @@ void CheckTeamRounds()
     }
 }
 
-// All launches of a collective of one shape store alike, however the cap cut it.
-void CheckCopyStores()
+// All launches of a collective of one shape store alike, however the cap cut it; what the caller has set holds everywhere.
+void CheckStores()
 {
     for (int round = 0; round < 2000; round++) {
-        const uint64_t ndst = 1 + Draw(8), block = 1 + Draw(uint64_t(200) << 20), items = 1 + Draw(64), moved = items * block * (1 + ndst);
-        const bool whole = CopiesWriteThrough(moved, items * block * ndst, moved);
-        CHECK(whole == (ndst >= 4 || moved <= 2 * kMemorySideCacheBytes));
+        const bool reduces = Draw(2) != 0;
+        const uint64_t nsrc = reduces ? 2 + Draw(16) : 1, ndst = 1 + Draw(8), block = 1 + Draw(uint64_t(200) << 20), items = 1 + Draw(64);
+        const uint64_t moved = items * block * (nsrc + ndst);
+        const uint32_t whole = StoreFlags(-1, reduces, false, moved, items * block * ndst, moved);
+        const bool small = moved <= 2 * kMemorySideCacheBytes;
+        CHECK(whole == ((reduces ? small && nsrc >= 2 * ndst : small || ndst >= 4) ? kFusedThroughStores : kFusedNtStores));
         for (uint64_t n = 1; n <= items; n++) {
-            CHECK(CopiesWriteThrough(n * block * (1 + ndst), n * block * ndst, moved) == whole);
+            const uint64_t traffic = n * block * (nsrc + ndst), written = n * block * ndst;
+            CHECK(StoreFlags(-1, reduces, false, traffic, written, moved) == whole);
+            CHECK(StoreFlags(-1, reduces, true, traffic, written, moved) == 0);
+            for (bool team : {false, true}) {
+                CHECK(StoreFlags(0, reduces, team, traffic, written, moved) == kFusedNtStores);
+                CHECK(StoreFlags(1, reduces, team, traffic, written, moved) == kFusedOrdinaryStores);
+            }
         }
     }
 }
@@ -113,7 +122,7 @@ int main()
     CheckSplit();
     CheckTeamRegions();
     CheckTeamRounds();
-    CheckCopyStores();
+    CheckStores();
     std::printf("OK\n");
     return 0;
 }

@@ -633,7 +633,8 @@ template <typename T, int OP> struct ElemLane {
     static __device__ __forceinline__ Val Combine(Val a, Val b) { return Elem<T, OP>::Apply(a, b); }
 };
 
-// How a chain folds 16 bytes.  Most types: VecLane.  Where a combine takes several instructions per word because elements have
+// How a chain folds 16 bytes: 8-bit types always, 16-bit max / min where all loads of up to 8 sources are in flight (with more
+// sources, or two sources at a time, they take Exact).  Most types: VecLane.  Where a combine takes several instructions per word because elements have
 // to be taken apart and put together again, the value is kept apart from the first source to the last (instructions per word and
 // source: 8-bit 3 instead of 6 to 11; bf16 max / min 3 or 2 instead of 9; fp16 max / min 1 or half a one instead of 5).
 template <typename T, int OP> struct FoldLane : VecLane<T, OP> {};
@@ -670,31 +671,63 @@ template <int OP> struct FoldLane<int8_t, OP> : ByteLane<true, OP> {};
 template <int OP> struct FoldLane<uint8_t, OP> : ByteLane<false, OP> {};
 
 // Max / min of 16-bit floats by the instructions that hand a NaN on (v_maximum3 / v_minimum3).  The selection rule
-// ((b > a) ? b : a in the schedule's order) gives the same bits unless a source is a NaN or the result is a zero, whose sign the
-// rule decides: Special(result) tells, and the sources, still in registers, are then folded by the rule.
-// `most` collects the largest of (magnitude - 1) per half: a zero or a NaN is above `limit`.
-template <uint32_t INF> struct SpecialHalves {
-    uint32_t most = 0;
-    __device__ __forceinline__ void See(uint32_t w)
+// ((b > a) ? b : a in the schedule's order) gives the same bits unless a source is a NaN, and the result then is one, or the result
+// is a zero and sources are zeros of both signs, between which the rule goes by the order.  Of these the instructions take +0 for a
+// maximum and -0 for a minimum: a zero result of the other sign is right as it is, and this one where no source holds the other.
+// ChainWhole looks at the first source, then at the result, then at all sources, still in registers, and folds by the rule where it has to.
+// All-reduce, 8 ranks, bf16 maximum, us, always by the rule / folded again for every zero or NaN / this way: 64 MiB normal data
+// 196 / 177 / 177, 1 % zeros 198 / 199 / 182, negative values as zeros 197 / 202 / 183, zeros of both signs 196 / 203 / 188, 1 % NaNs 197 / 202 / 188, one
+// NaN in 1200 results 197 / 199 / 200; 2 MiB 8.7 / 6.3 / 6.3, 8.8 / 8.8 / 7.0, 8.9 / 9.1 / 7.3, 8.6 / 9.0 / 8.7, 8.6 / 8.9 / 8.3, 8.6 / 8.7 / 9.0; fp16 64 MiB 187 / 173 /
+// 176, 188 / 185 / 181, 189 / 193 / 182, 188 / 192 / 182, 189 / 192 / 183, 189 / 187 / 191.
+template <uint32_t INF, int OP> struct SpecialHalves {
+    uint32_t most = 0, least = ~0u, leastSigned = 0x7fff7fffu;
+    // NaNs, and zeros of either sign: the largest of (magnitude - 1) per half is not below INF then
+    __device__ __forceinline__ void SeeAny(V4 v)
     {
-        const U2 below = BitCast<U2>(w & 0x7fff7fffu) - U2{1, 1};
-        most = BitCast<uint32_t>(__builtin_elementwise_max(BitCast<U2>(most), below));
-    }
-    __device__ __forceinline__ void See(V4 v)
-    {
-        See(v.x);
-        See(v.y);
-        See(v.z);
-        See(v.w);
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+            most = BitCast<uint32_t>(__builtin_elementwise_max(BitCast<U2>(most), BitCast<U2>(v[i] & 0x7fff7fffu) - U2{1, 1}));
+        }
     }
     __device__ __forceinline__ bool Any() const { return (most & 0xffffu) >= INF || (most >> 16) >= INF; }
+    // NaNs: the largest magnitude is above INF
+    __device__ __forceinline__ void SeeNan(V4 v)
+    {
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+            most = BitCast<uint32_t>(__builtin_elementwise_max(BitCast<U2>(most), BitCast<U2>(v[i] & 0x7fff7fffu)));
+        }
+    }
+    __device__ __forceinline__ bool Nan() const { return (most & 0xffffu) > INF || (most >> 16) > INF; }
+    // +0 is the least number without sign, -0 the least with one
+    __device__ __forceinline__ void SeePlus(V4 v)
+    {
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+            least = BitCast<uint32_t>(__builtin_elementwise_min(BitCast<U2>(least), BitCast<U2>(v[i])));
+        }
+    }
+    __device__ __forceinline__ bool Plus() const { return (least & 0xffffu) == 0 || (least >> 16) == 0; }
+    __device__ __forceinline__ void SeeMinus(V4 v)
+    {
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+            leastSigned = BitCast<uint32_t>(__builtin_elementwise_min(BitCast<S2>(leastSigned), BitCast<S2>(v[i])));
+        }
+    }
+    __device__ __forceinline__ bool Minus() const { return (leastSigned & 0xffffu) == 0x8000u || (leastSigned >> 16) == 0x8000u; }
+    // the zero that the instructions take, and the one that they pass over
+    __device__ __forceinline__ void SeeTaken(V4 v) { OP == ROP_MAX ? SeePlus(v) : SeeMinus(v); }
+    __device__ __forceinline__ bool Taken() const { return OP == ROP_MAX ? Plus() : Minus(); }
+    __device__ __forceinline__ void SeePassed(V4 v) { OP == ROP_MAX ? SeeMinus(v) : SeePlus(v); }
+    __device__ __forceinline__ bool Passed() const { return OP == ROP_MAX ? Minus() : Plus(); }
 };
 template <int OP> struct HalfMaxLane {
     typedef V4 Val;
     typedef V4 Raw;
     typedef V4 Out;
     typedef VecLane<HalfBits, OP> Exact;
-    typedef SpecialHalves<0x7c00u> Special;
+    typedef SpecialHalves<0x7c00u, OP> Special;
     static constexpr bool kChecked = true;
     static __device__ __forceinline__ Raw Load(const void *base, uint32_t pos) { return Load16<ACC_VEC16_ANY>(base, pos); }
     static __device__ __forceinline__ Val Value(const Raw &r, const void *) { return r; }
@@ -716,7 +749,7 @@ template <int OP> struct Bf16MaxLane {
     typedef V4 Raw;
     typedef V4 Out;
     typedef VecLane<Bf16Bits, OP> Exact;
-    typedef SpecialHalves<0x7f80u> Special;
+    typedef SpecialHalves<0x7f80u, OP> Special;
     static constexpr bool kChecked = true;
     static __device__ __forceinline__ Raw Load(const void *base, uint32_t pos) { return Load16<ACC_VEC16_ANY>(base, pos); }
     static __device__ __forceinline__ Val Value(const Raw &r, const void *) { return Val{r, r << 16}; }
@@ -909,17 +942,48 @@ __device__ __forceinline__ void ChainWhole(const void *const *__restrict__ src, 
     typename L::Raw v[N][U];
     typename L::Val acc[U];
     ChainLoad<L, N, U>(src, off, at, v);
-    ChainFold<L, T, OP, N, U, true>(src, v, accLeft, acc);
-    ChainResult<L, U>(acc, x);
     if constexpr (L::kChecked && N > 1) {
-        typename L::Special special;
+        // Each question is asked of a wave.  A first vector that holds a NaN or zeros of both signs: by the rule at once.
+        typename L::Special first;
+        first.SeeNan(v[0][0]);
+        first.SeePlus(v[0][0]);
+        first.SeeMinus(v[0][0]);
+        bool byRule = __any(first.Nan()) || (__any(first.Plus()) && __any(first.Minus()));
+        if (!byRule) {
+            ChainFold<L, T, OP, N, U, true>(src, v, accLeft, acc);
+            ChainResult<L, U>(acc, x);
+            typename L::Special any;
 #pragma unroll
-        for (uint32_t u = 0; u < U; u++) {
-            special.See(x[u]);
+            for (uint32_t u = 0; u < U; u++) {
+                any.SeeAny(x[u]);
+            }
+            if (__builtin_expect(__any(any.Any()), 0)) {
+                typename L::Special result;
+#pragma unroll
+                for (uint32_t u = 0; u < U; u++) {
+                    result.SeeNan(x[u]);
+                    result.SeeTaken(x[u]);
+                }
+                byRule = __any(result.Nan());
+                if (!byRule && __any(result.Taken())) {
+                    typename L::Special sources;
+#pragma unroll
+                    for (uint32_t j = 0; j < N; j++) {
+#pragma unroll
+                        for (uint32_t u = 0; u < U; u++) {
+                            sources.SeePassed(v[j][u]);
+                        }
+                    }
+                    byRule = __any(sources.Passed());
+                }
+            }
         }
-        if (__any(special.Any())) {
+        if (__builtin_expect(byRule, 0)) {
             ChainFold<typename L::Exact, T, OP, N, U, true>(src, v, accLeft, x);
         }
+    } else {
+        ChainFold<L, T, OP, N, U, true>(src, v, accLeft, acc);
+        ChainResult<L, U>(acc, x);
     }
 }
 
@@ -1077,8 +1141,9 @@ __device__ __forceinline__ void ChainRest(const FusedDesc &d, bool ends, const v
 // ranks, fp32, 2 MiB per rank 7.3 / 7.3 / 7.5, 6 MiB 20.1 / 17.5 / 18.9, 8 MiB 23.9 / 22.2 / 23.9; reduce-scatter, 8 ranks, fp32, blocks of 8 MiB
 // 97.0 / 101.0 / 98.6, 16 MiB 192.7 / 200.1 / 190.8; 16 ranks, bf16 maximum, 512 KiB 27.6 / 25.4 / 23.7, 16 MiB 777 / 767 / 755.
 // SLOW = false has all loads of a tile in flight, the shortest way through a tile, for launches of a tile per CU or fewer.
-// SLOW = true has two sources' in flight and 70 registers instead of 170: where tiles follow one another, and for
-// many sources into one destination, workgroups that ask for less at a time move more.
+// SLOW = true has two sources' in flight and 70 registers instead of 161 (fp32, fp16 sum; bf16 120 instead of 254, int8 102 - 115
+// instead of 253 - 256): where tiles follow one another, and for many sources into one destination, workgroups that ask for
+// less at a time move more.
 template <typename T, int OP, bool SLOW>
 __global__ void __launch_bounds__(kBlockThreads, 2) ChainKernel(const FusedDesc *__restrict__ items, uint32_t nitems, uint32_t nall, uint32_t nwhole,
     uint32_t ntiles, const void *const *__restrict__ srcPool, void *const *__restrict__ dstPool, uint32_t tilesPerItem)

@@ -7,7 +7,7 @@ import torch
 
 import closed_forms as cf
 import gpu_harness as gh
-from closed_forms import BF16, FP16, FP32, INT8, INT64, MAX, MIN, PROD, SUM, UINT8
+from closed_forms import BF16, FP16, FP32, FP64, INT8, INT64, MAX, MIN, PROD, SUM, UINT8
 
 pytestmark = pytest.mark.gpu
 H = gh.H
@@ -164,5 +164,68 @@ def test_half_selection_over_every_bit_pattern(orc, dt, op, p, team):
                 outs, _ = gh.all_reduce(g, ins, dt, op, in_place=in_place)
                 for r in range(p):
                     assert np.array_equal(outs[r].view(np.uint16), want[r].view(np.uint16)), (kind, in_place, r)
+    finally:
+        g.close()
+
+
+def _placed_specials(dt, op, p, rng):
+    """Ordinary values, and every 2600 elements (a wave reads 2048 of a tile) one place where up to two sources hold a special
+    one, in each half of a word, in the first, a middle and the last source."""
+    inf = 0x7f80 if dt == BF16 else 0x7c00
+    singles = [inf, 0x8000 | inf, inf | 0x40 if dt == BF16 else inf | 0x200, 0x8000 | inf | 1, inf | 1, 0x0000, 0x8000, 0x0001, 0x8001]
+    places = sorted({0, p // 2, p - 1})
+    kinds = [[(v, r)] for v in singles for r in places]
+    kinds += [[(a, r), (b, q)] for a, b in ((0x0000, 0x8000), (0x8000, 0x0000)) for r in places for q in places if r < q]
+    step = 2600
+    n = 2 * step * len(kinds)
+    # losing values: a zero placed among them is the result
+    lose = rng.integers(1, 0x30, n).astype(np.uint16) * 0x100 + rng.integers(0, 256, n).astype(np.uint16)
+    ins = [np.roll(lose, 17 * r) | np.uint16(0x8000 if op == MAX else 0) for r in range(p)]
+    for i, kind in enumerate(kinds):
+        for half in (0, 1):
+            at = (2 * i + half) * step + int(rng.integers(0, step // 2)) * 2 + half
+            for v, r in kind:
+                ins[r][at] = v
+    return ins
+
+
+@pytest.mark.parametrize("dt,op", [(FP16, MAX), (FP16, MIN), (BF16, MAX), (BF16, MIN)])
+@pytest.mark.parametrize("team", [0, 1])
+def test_half_selection_with_one_special_in_a_wave(orc, dt, op, team):
+    # the result of the fast fold stands in most waves: it may be a zero of either sign, an infinity, a denormal
+    for p in range(2, 10):
+        g = gh.Group(p, algo="ring", team=team, direct=0)
+        try:
+            print("placed specials", dt, op, p, team, flush=True)
+            ins = _placed_specials(dt, op, p, np.random.default_rng(9600 + p))
+            want = orc.allreduce([x.copy() for x in ins], dt, op)
+            outs, _ = gh.all_reduce(g, ins, dt, op)
+            for r in range(p):
+                assert np.array_equal(outs[r].view(np.uint16), want[r].view(np.uint16)), (p, r)
+        finally:
+            g.close()
+
+
+@pytest.mark.parametrize("dt,op", [(FP32, MAX), (FP32, MIN), (FP64, MAX)])
+@pytest.mark.parametrize("algo", ["ring", "mesh"])
+def test_rounds_keep_the_operand_order(orc, dt, op, algo):
+    # rounds read source by source whose tiles belong to two items, on values that tell the order: zeros of both signs, NaNs
+    p, unit = 8, H.DTYPE_SIZE[dt]
+    bits = np.uint32 if unit == 4 else np.uint64
+    top = 32 if unit == 4 else 64
+    exp = 0x7f800000 if unit == 4 else 0x7ff0000000000000
+    values = np.array([0, 1 << (top - 1), 0, 1 << (top - 1), exp | 1, exp | (1 << (top - 1)) | 77, 1, exp], bits)
+    g = gh.Group(p, algo=algo, team=1)
+    try:
+        for tiles in (4, 5, 6, 7, 8):
+            n = (256 * tiles * TILE - 37 * TILE) // unit + 5
+            print("order in rounds of", tiles, "type", dt, "op", op, algo, flush=True)
+            rng = np.random.default_rng(9700 + tiles)
+            ins = [values[rng.integers(0, len(values), n)].view(np.float32 if unit == 4 else np.float64) for _ in range(p)]
+            want = orc.allreduce([x.copy() for x in ins], dt, op, algo={"ring": orc.RING, "mesh": orc.MESH_ATOMIC}[algo], threads=8)
+            outs, _ = gh.all_reduce(g, ins, dt, op)
+            assert g.info()["teamLaunches"] >= 1
+            for r in range(p):
+                assert np.array_equal(outs[r].view(bits), want[r].view(bits)), (tiles, r)
     finally:
         g.close()

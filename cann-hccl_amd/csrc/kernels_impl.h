@@ -597,6 +597,7 @@ template <typename T, int OP> struct VecLane {
     typedef V4 Out;
     typedef VecLane Exact;
     static constexpr bool kChecked = false;      // Combine gives the same bits as Elem for every operand
+    static constexpr bool kHoldBack = sizeof(T) == 1 && OP == ROP_SUM;      // see TreeFold
     static __device__ __forceinline__ Out Result(const Val &v) { return v; }
     static __device__ __forceinline__ Raw Load(const void *base, uint32_t pos) { return Load16<ACC_VEC16_ANY>(base, pos); }
     static __device__ __forceinline__ Val Value(const Raw &r, const void *) { return r; }
@@ -626,6 +627,7 @@ template <typename T, int OP> struct ElemLane {
     typedef T Out;
     typedef ElemLane Exact;
     static constexpr bool kChecked = false;
+    static constexpr bool kHoldBack = false;
     static __device__ __forceinline__ Out Result(const Val &v) { return v; }
     static __device__ __forceinline__ Raw Load(const void *base, uint32_t pos) { return LoadElem<T>(base, pos); }
     static __device__ __forceinline__ Val Value(const Raw &r, const void *) { return r; }
@@ -1312,7 +1314,11 @@ __device__ __forceinline__ void TreePairs(const void *const *__restrict__ src, u
         }
     }
 }
-// N leaves pairwise into x.
+// N leaves pairwise into x.  8-bit sums: the compiler keeps them apart as even and odd bytes from one level to the next and past the
+// set's end, which takes 312 registers in the plain kernel and leaves a CU one workgroup; put together at a set's end it takes 223,
+// and two fit.  Halving-doubling reduce-scatter, 8 ranks, us, 8 leaves in one set (before) / kept apart / put together: blocks of 1 MiB
+// 12.2 / 12.9 / 10.8, 2 MiB 23.7 / 26.1 / 21.5, 8 MiB 101.5 / 99.5 / 99.8; all-reduce 8 ranks 8 MiB 24.7 / 20.8 / 21.3; reduce 16 ranks 64 MiB
+// 193 / 182 / 189.  (Other types take 253 to 292 and lose by it: all-reduce 16 ranks fp32 4 MiB 19.6 / 20.2, int64 19.7 / 20.2.)
 template <typename L, uint32_t N, uint32_t U>
 __device__ __forceinline__ void TreeFold(typename L::Val (&v)[N][U], typename L::Val (&x)[U])
 {
@@ -1329,6 +1335,9 @@ __device__ __forceinline__ void TreeFold(typename L::Val (&v)[N][U], typename L:
 #pragma unroll
     for (uint32_t u = 0; u < U; u++) {
         x[u] = v[0][u];
+    }
+    if constexpr (L::kHoldBack) {
+        HoldBack(x);
     }
 }
 template <typename L, uint32_t U>

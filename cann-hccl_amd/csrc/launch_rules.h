@@ -55,8 +55,10 @@ constexpr uint32_t kTeamMinHalfRounds = 1;
 // Items with fewer than 12 sources and destinations (4 ranks, fp32): 16 MiB 24.3 / 26.1, 32 MiB (a round) 48.0 / 47.4, 48 MiB 70.5 / 74.8,
 // 64 MiB 93.6 / 95.1, 128 MiB (4 rounds) 188.5 / 183.3.
 constexpr uint32_t kTeamMinHalfRoundsFew = 8;
-// One source and many destinations: 8-rank all-gather, blocks of 2 MiB (1024 tiles) 25.9 / 30.0, 4 MiB (2048, a round) 60.0 / 54.2,
-// 8 MiB 122.9 / 105.4; 16 ranks 1 MiB (1024) 54.8 / 53.4, 2 MiB 121.2 / 100.9.
+// One source and many destinations, all-gather: 8 ranks 3 MiB (1536 tiles) 29.2 / 39.4, 4 MiB (2048, a round) 41.6 / 52.0, 5 MiB 64.5 / 68.4,
+// 2 bytes off a boundary 71.7 / 69.9, 6 MiB 86.4 / 79.8, 8 MiB 120.9 / 105.5; 16 ranks 1 MiB (1024) 38.5 / 52.5, 2 MiB 104.6 / 99.0; 9 ranks 4 MiB 66.8 /
+// 67.6.  (The line was drawn when the plain kernel's results were not written through, 4 MiB 60.0 / 54.2; between a round and
+// the memory-side cache's size the plain form is now the faster one.)
 constexpr uint32_t kTeamMinHalfRoundsCopy = 2;
 
 // Whether a launch whose items with whole tiles have `bytes` in all runs that long.  (By bytes, not by tiles: a buffer that starts
@@ -110,14 +112,16 @@ constexpr uint64_t kMemorySideCacheBytes = 256ull << 20;
 
 // Whether a launch of the plain copy kernel writes its results through (StorePolicy, kernels_impl.h) instead of non-temporally:
 // `traffic` bytes read and written by the launch, `written` of them written, `moved` read and written by the whole collective, whose
-// launches all store alike.  Up to 512 MiB in all, us, non-temporal / through: all-gather 2 ranks 10 MiB 10.4 / 7.4, 64 MiB
-// (384 MiB moved) 67.7 / 60.1; 3 ranks 8 MiB 17.2 / 12.0, 32 MiB (384) 71.5 / 59.9; 8 ranks 2 MiB 28.2 / 20.1; 16 ranks 1 MiB 53.7 / 38.7;
-// uniform all-to-all 8 ranks 8 MiB 21.3 / 20.3, 32 MiB (512) 84.5 / 75.7.  Beyond, the one loses what the other
-// gains: 2 ranks 128 MiB (768) 139.5 / 143.8, 3 ranks 48 MiB (576) 107.8 / 111.7, all-to-all 64 MiB (1024) 170.0 / 172.5 -- unless every
-// block goes to four destinations or more: 5 ranks 24 MiB (720) 150.5 / 147.6, 6 ranks 24 MiB (1008) 217.8 / 210.7, 32 MiB 295 / 281.
+// launches all store alike.  One destination: never.  On the same buffers again and again it pays (all-to-all-v of 16 ranks, 210 MiB,
+// non-temporal / through, us, 37.1 / 36.6; uniform all-to-all 8 ranks 32 MiB 84.5 / 75.7), on four sets of buffers in turn it does not: 16 ranks
+// 210 MiB 39.1 / 45.9, 480 MiB 85.0 / 91.8, 8 ranks 314 MiB 55.8 / 59.3, 64 ranks 412 MiB 90.9 / 102.4.  Several, up to 512 MiB in all (all-gather,
+// same buffers; four sets in turn): 2 ranks 10 MiB 10.4 / 7.4; 11.8 / 12.0, 64 MiB (384 MiB moved) 67.7 / 60.1; 79.4 / 78.8, 3 ranks 8 MiB 17.2 / 12.0; 18.7 /
+// 18.0, 8 ranks 2 MiB 28.2 / 20.1; 27.4 / 26.9, 16 ranks 1 MiB 53.7 / 38.7; 54.6 / 53.8.  Beyond, the one loses what the other
+// gains: 2 ranks 128 MiB (768) 139.5 / 143.8, 3 ranks 48 MiB (576) 107.8 / 111.7 -- unless every
+// block goes to four destinations or more: 5 ranks 24 MiB (720) 150.5 / 147.6, 6 ranks 24 MiB (1008) 217.8 / 210.7; 219.9 / 213.1.
 inline bool CopiesWriteThrough(uint64_t traffic, uint64_t written, uint64_t moved)
 {
-    return moved <= 2 * kMemorySideCacheBytes || 5 * written >= 4 * traffic;
+    return 2 * written > traffic && (moved <= 2 * kMemorySideCacheBytes || 5 * written >= 4 * traffic);
 }
 
 // The same for a launch of the plain reducing kernels: many sources into one destination, up to 512 MiB in all.

@@ -54,8 +54,8 @@ extern "C" {
  *   "fused_stores"  "auto" | "nt" | "ordinary"   store kind of the fused kernels: non-temporal, or write-back, which
  *                                keeps a result of up to 256 MB in the memory-side cache for whoever reads it next; "auto"
  *                                (default): written through the L2 cache where many sources become one result and where
- *                                data is only moved, if the collective reads and writes up to 512 MiB in all (a move to
- *                                four destinations and more: of any size); non-temporal beyond; both in the team form
+ *                                data is moved to several destinations, if the collective reads and writes up to 512 MiB in
+ *                                all (four destinations and more: of any size); non-temporal beyond; both in the team form
  *   "team"          "auto" | "0" | "1"   team form of the fused kernels: the workgroups of one XCD read their tiles together,
  *                                hold the results in LDS and write them together, which this memory system serves faster
  *                                than reads and writes interleaved; "auto" (default): for launches of at least half a

@@ -102,7 +102,7 @@ void CheckStores()
         const uint64_t moved = items * block * (nsrc + ndst);
         const uint32_t whole = StoreFlags(-1, reduces, false, moved, items * block * ndst, moved);
         const bool small = moved <= 2 * kMemorySideCacheBytes;
-        CHECK(whole == ((reduces ? small && nsrc >= 2 * ndst : small || ndst >= 4) ? kFusedThroughStores : kFusedNtStores));
+        CHECK(whole == ((reduces ? small && nsrc >= 2 * ndst : ndst >= 2 && (small || ndst >= 4)) ? kFusedThroughStores : kFusedNtStores));
         for (uint64_t n = 1; n <= items; n++) {
             const uint64_t traffic = n * block * (nsrc + ndst), written = n * block * ndst;
             CHECK(StoreFlags(-1, reduces, false, traffic, written, moved) == whole);

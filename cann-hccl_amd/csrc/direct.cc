@@ -136,6 +136,25 @@ bool DirectFits(int coll, uint32_t p, uint64_t bytes, int dtype)
     }
 }
 
+// Beyond those limits, where the items are alike (PackDirect): a wave per KiB keeps every CU equally busy when there are few tiles of
+// 16 KiB, or tiles of few sources and destinations.  Three sets of buffers in turn, us, tile kernels / packed:
+//   all-reduce, fp32: 2 ranks 4 MiB 4.7 / 3.5, 16 MiB 12.6 / 11.9, 32 MiB 23.2 / 21.1, 64 MiB 44.3 / 43.7; 4 ranks 2 MiB 4.9 / 3.7, 3 MiB 5.6 / 4.6, 4 MiB
+//     6.0 / 6.5; 8 ranks 1.5 MiB 6.5 / 4.6, 2 MiB 7.2 / 6.0, 2.25 MiB 7.4 / 6.7, 2.5 MiB 7.6 / 7.7; 16 ranks 1.25 MiB 10.4 / 7.7, 1.5 MiB 11.0 / 9.6,
+//     2 MiB 12.6 / 14.9; 32 ranks 1.25 MiB 20 / 14, 1.5 MiB 21.3 / 17.7; bf16 and int8 alike
+//   reduce-scatter (bytes received by all ranks), fp32: 2 ranks 6 MiB 4.5 / 3.9, 12 MiB 7.2 / 6.4, 16 MiB 9.0 / 9.0; 4 ranks 4 MiB 5.0 / 4.3, 6 MiB 6.4 / 5.9, 8 MiB
+//     7.4 / 7.5; 8 ranks 3 MiB 6.3 / 5.4, 4 MiB 7.4 / 7.0, 6 MiB 10.1 / 9.9; 16 ranks 2.5 MiB 9.1 / 8.4, 3 MiB 9.8 / 10.0
+bool PackedFits(int coll, uint32_t p, uint64_t bytes)
+{
+    constexpr uint64_t kQuarter = uint64_t(1) << 18;      // of a MiB
+    if (coll == COLL_ALLREDUCE) {
+        return p > 1 && p <= 32 && bytes <= (p == 2 ? 128 : p <= 4 ? 14 : p <= 8 ? 9 : 6) * kQuarter;
+    }
+    if (coll == COLL_REDUCESCATTER) {
+        return p > 1 && p <= 8 && bytes * p <= (p == 2 ? 56 : p <= 4 ? 24 : bytes % 16 == 0 ? 18 : 14) * kQuarter;
+    }
+    return false;
+}
+
 bool BuildDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaunch *d)
 {
     d->func = nullptr;
@@ -157,6 +176,152 @@ bool BuildDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLau
     return d->func != nullptr;
 }
 
+namespace {
+
+// Arguments of `P` ranks out of items of `nsrc` sources each, already found alike.
+template <uint32_t P> void FillPacked(const Plan &plan, const std::vector<uint32_t> &order, uint32_t info, DirectLaunch *d)
+{
+    d->packed.assign(sizeof(PackedArgs<P>), 0);
+    PackedArgs<P> *args = reinterpret_cast<PackedArgs<P> *>(d->packed.data());
+    const FusedItem &f = plan.fused[0], &last = plan.fused[plan.fused.size() - 1];
+    args->first = uint32_t(f.bytes);
+    args->last = uint32_t(last.bytes);
+    if (plan.fused.size() > 1) {
+        args->srcStep = uint32_t(plan.fused[1].src[0].off);
+        args->dstStep = uint32_t(plan.fused[1].dst[0].off);
+    }
+    args->info = info;
+    for (size_t j = 0; j < order.size(); j++) {
+        args->order[P > 16 ? j / 4 : j / 8] |= order[j] << (P > 16 ? 8 * (j % 4) : 4 * (j % 8));
+    }
+    d->packedRanks = P;
+}
+
+// base + (offset << shift) for every rank's pointer; false where the offsets do not fit 32 bits.
+template <uint32_t P> bool FillOffsets(DirectLaunch *d, uint32_t ranks, const std::vector<void *> &send, const std::vector<void *> &recv)
+{
+    PackedArgs<P> *args = reinterpret_cast<PackedArgs<P> *>(d->packed.data());
+    uint64_t least = ~uint64_t(0), most = 0, bits = 0;
+    for (uint32_t r = 0; r < ranks; r++) {
+        for (const void *v : {send[r], recv[r]}) {
+            const uint64_t at = reinterpret_cast<uint64_t>(v);
+            least = std::min(least, at);
+            most = std::max(most, at);
+            bits |= at;
+        }
+    }
+    // (an alignment of the addresses themselves is one of their differences; beyond 4 KiB a larger shift brings nothing)
+    const uint32_t shift = uint32_t(__builtin_ctzll(bits | 4096));
+    least &= ~uint64_t(4095);
+    if (((most - least) >> shift) > 0xffffffffull) {
+        return false;
+    }
+    args->base = least;
+    args->info = (args->info & ~(63u << kPackedShift)) | (shift << kPackedShift);
+    for (uint32_t r = 0; r < ranks; r++) {
+        args->off[r] = uint32_t((reinterpret_cast<uint64_t>(send[r]) - least) >> shift);
+        args->off[P + r] = uint32_t((reinterpret_cast<uint64_t>(recv[r]) - least) >> shift);
+    }
+    return true;
+}
+
+}  // namespace
+
+void PackDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaunch *d)
+{
+    const uint32_t p = plan.p, n = uint32_t(plan.fused.size());
+    if (p > 32 || n == 0 || n > p) {
+        return;
+    }
+    const FusedItem &f = plan.fused[0];
+    const bool tree = f.kind == FK_TREE;
+    if (f.kind == FK_STACK) {
+        return;
+    }
+    // the sources of an item: a tree's leaves one behind the other, all of them pairs or none
+    auto sources = [&](const FusedItem &it, std::vector<uint32_t> *ranks) {
+        ranks->clear();
+        const bool pairs = tree && it.srcValid[1] != 0;
+        for (size_t k = 0; k < it.src.size(); k++) {
+            const bool here = !tree || (k & 1u) == 0 || pairs;
+            if ((it.srcValid[k] != 0) != here) {
+                return false;
+            }
+            if (here) {
+                if (it.src[k].buf != BUF_SEND) {
+                    return false;
+                }
+                ranks->push_back(it.src[k].rank);
+            }
+        }
+        return true;
+    };
+    std::vector<uint32_t> order, ranks;
+    if (!sources(f, &order) || order.empty() || order.size() > 32 || (tree && ((order.size() & (order.size() - 1)) != 0 || order.size() < 2))) {
+        return;
+    }
+    const bool toOne = f.dst.size() == 1 && p > 1;
+    bool left = true, ring = true, ends = false;      // chain: every source behind the first is the right operand; all but the second the left one
+    const uint64_t srcStep = n > 1 ? plan.fused[1].src[0].off : 0, dstStep = n > 1 ? plan.fused[1].dst[0].off : 0;
+    uint64_t longest = 0;
+    for (uint32_t i = 0; i < n; i++) {
+        const FusedItem &it = plan.fused[i];
+        if (it.kind != f.kind || (i + 1 < n && it.bytes != f.bytes) || it.bytes > 0x7fffffffull || !sources(it, &ranks) || ranks.size() != order.size() ||
+            it.dst.size() != (toOne ? 1 : p)) {
+            return;
+        }
+        for (size_t j = 0; j < ranks.size(); j++) {
+            const uint32_t want = tree ? order[j] ^ i : (order[j] + i) % p;
+            if (ranks[j] != want) {
+                return;
+            }
+        }
+        for (size_t k = 0; k < it.src.size(); k++) {
+            if (it.srcValid[k] != 0 && it.src[k].off != i * srcStep) {
+                return;
+            }
+        }
+        uint64_t seen = 0;
+        for (size_t k = 0; k < it.dst.size(); k++) {
+            if (it.dst[k].buf != BUF_RECV || it.dst[k].off != i * dstStep || (toOne && it.dst[k].rank != i)) {
+                return;
+            }
+            seen |= uint64_t(1) << it.dst[k].rank;
+        }
+        if (!toOne && seen != (uint64_t(1) << p) - 1) {
+            return;
+        }
+        for (size_t j = 1; !tree && j < it.accLeft.size(); j++) {
+            left = left && it.accLeft[j] != 0;
+            ring = ring && (it.accLeft[j] != 0) == (j == 1);
+        }
+        ends = ends || it.bytes % 16 != 0;
+        longest = std::max(longest, it.bytes);
+    }
+    // (the offsets of the last item and its length are 32-bit numbers of the plan's, which BuildDirect has looked at)
+    if (!tree && order.size() > 1 && !left && !ring) {
+        return;
+    }
+    const uint32_t info = uint32_t(order.size()) << kPackedSources | n << kPackedItems | p << kPackedModulus | (tree ? kPackedTree : 0u) |
+        (toOne ? kPackedToOne : 0u) | (ends ? kPackedEnds : 0u) | (!tree && !left ? kPackedRing : 0u);
+    KernelKind kind = KK_PACKED_8;
+    if (p <= 8) {
+        FillPacked<8>(plan, order, info, d);
+    } else if (p <= 16) {
+        FillPacked<16>(plan, order, info, d);
+        kind = KK_PACKED_16;
+    } else {
+        FillPacked<32>(plan, order, info, d);
+        kind = KK_PACKED_32;
+    }
+    const uint32_t shape = PackedShape(uint32_t(order.size()));
+    if (reduceColl && shape < kPackedShapes && order.size() == p) {       // (of two sources, added and exclusive-ored are the same)
+        kind = KernelKind((tree ? KK_PACKED_TREE : (left ? KK_PACKED_CHAIN : KK_PACKED_RING)) + shape);
+    }
+    d->packedGridX = uint32_t(longest / kDirectChunk + (longest % kDirectChunk >= 16 ? 1 : 0)) + (ends ? 1u : 0u);
+    d->packedFunc = reduceColl ? LookupKernel(dtype, op, kind) : LookupCopyKernel(kind);
+}
+
 bool FillBases(DirectLaunch *d, const std::vector<void *> &send, const std::vector<void *> &recv)
 {
     uint64_t *base = reinterpret_cast<uint64_t *>(d->image.data());     // DirectArgs<>::base comes first
@@ -165,6 +330,11 @@ bool FillBases(DirectLaunch *d, const std::vector<void *> &send, const std::vect
         const uint64_t p = reinterpret_cast<uint64_t>((d->bases[i].second == BUF_SEND ? send : recv)[d->bases[i].first]);
         same = same && base[i] == p;
         base[i] = p;
+    }
+    if (d->packedFunc != nullptr && !same) {
+        const uint32_t ranks = uint32_t(send.size());
+        d->usePacked = d->packedRanks == 8 ? FillOffsets<8>(d, ranks, send, recv)
+                                           : (d->packedRanks == 16 ? FillOffsets<16>(d, ranks, send, recv) : FillOffsets<32>(d, ranks, send, recv));
     }
     return same;
 }

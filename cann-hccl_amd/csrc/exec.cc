@@ -1250,7 +1250,12 @@ DirectLaunch *FindDirect(Group *g, int algo)
     const OpSig &sig = g->ctx->sig;
     const GroupConfig &cfg = g->cfg;
     if (sig.noAlloc || sig.variable || sig.coll == COLL_ALLTOALLV || !cfg.fuse || !cfg.direct || cfg.team == 1 || cfg.blocksPerCu != 0 ||
-        cfg.launchCapMiB >= 0 || cfg.fusedStores >= 0 || !DirectFits(sig.coll, g->p, sig.count * DtypeSize(sig.dtype), sig.dtype)) {
+        cfg.launchCapMiB >= 0 || cfg.fusedStores >= 0) {
+        return nullptr;
+    }
+    const uint64_t bytes = sig.count * DtypeSize(sig.dtype);
+    const bool small = DirectFits(sig.coll, g->p, bytes, sig.dtype);
+    if (!small && !PackedFits(sig.coll, g->p, bytes)) {
         return nullptr;
     }
     uint64_t inPlace = 0;
@@ -1273,10 +1278,12 @@ DirectLaunch *FindDirect(Group *g, int algo)
             return nullptr;             // the general path reports it
         }
         if (BuildDirect(*plan, ReduceColl(sig.coll), sig.dtype, sig.op, &d)) {
+            PackDirect(*plan, ReduceColl(sig.coll), sig.dtype, sig.op, &d);
             d.info = MakeInfo(g, algo, *plan, true);
             d.info.launches = 1;
-            d.info.direct = 1;
-        } else {
+            d.info.direct = small ? 1 : 0;
+        }
+        if (d.func == nullptr || (!small && d.packedFunc == nullptr)) {
             d = DirectLaunch();
         }
         it = g->direct.emplace(key, std::move(d)).first;
@@ -1287,7 +1294,7 @@ DirectLaunch *FindDirect(Group *g, int algo)
         return nullptr;
     }
     d->info.cacheHit = FillBases(d, g->ctx->send, g->ctx->recv) ? 1 : 0;
-    return d;
+    return small || d->usePacked ? d : nullptr;
 }
 
 }  // namespace
@@ -1531,8 +1538,9 @@ HcclResult IssueCollective(Group *g, uint32_t launcher)
         others = true;
     }
     if (direct != nullptr) {
-        void *args[1] = {direct->image.data()};
-        HIP_OK(hipLaunchKernel(direct->func, dim3(direct->gridX, direct->gridY, 1), dim3(kBlockThreads, 1, 1), args, 0, ls));
+        void *args[1] = {direct->usePacked ? direct->packed.data() : direct->image.data()};
+        HIP_OK(hipLaunchKernel(direct->usePacked ? direct->packedFunc : direct->func,
+            dim3(direct->usePacked ? direct->packedGridX : direct->gridX, direct->gridY, 1), dim3(kDirectThreads, 1, 1), args, 0, ls));
     } else if (viaGraph) {
         HIP_OK(hipGraphLaunch(pp->exec, ls));
     } else {

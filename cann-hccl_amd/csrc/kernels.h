@@ -84,9 +84,17 @@ enum KernelKind : int {
     KK_DIRECT = 7, KK_DIRECT_WIDE = 8,                         // small collectives, see below
     KK_TEAM_STACK_TILES = 9,                                   // the team's stack kernel without its rounds read source by source
     KK_CHAIN_SLOW = 10,                                        // the chain kernel with two sources in flight
-    KK_COUNT = 11,
-    KK_GATHER = 11                                             // copy kernel table only
+    KK_PACKED_8 = 11, KK_PACKED_16 = 12, KK_PACKED_32 = 13,    // small collectives whose items are alike, by the most ranks they take
+    KK_PACKED_CHAIN = 14,                                      // the same for 2, 4, 8, 16 sources (kinds 14 ... 17): chains whose sources
+                                                               // are the right operands,
+    KK_PACKED_RING = 18,                                       // chains whose sources behind the second one are the left operands,
+    KK_PACKED_TREE = 22,                                       // trees
+    KK_COUNT = 26,
+    KK_GATHER = 26                                             // copy kernel table only
 };
+constexpr uint32_t kPackedShapes = 4;
+// Index of a number of sources among those that have a kernel of their own, kPackedShapes where it has none.
+constexpr uint32_t PackedShape(uint32_t nsrc) { return nsrc == 2 ? 0 : nsrc == 4 ? 1 : nsrc == 8 ? 2 : nsrc == 16 ? 3 : kPackedShapes; }
 
 // Team form of a fused kernel: the workgroups of one XCD read their tiles together, park the results in LDS, and write
 // them together (kernels_team.h).  Launched with a multiple of kTeamXcds workgroups (one per CU) and kTeamDynamicLds
@@ -116,7 +124,8 @@ inline uint32_t TeamBlockWords(uint32_t nregions) { return kTeamHeaderWords + 2u
 
 // Small collectives (kernels_direct.h): the whole description of a launch rides in its kernel arguments.  All sources of
 // an item lie at the same offset of their buffers and all destinations at the same offset of theirs.
-constexpr uint32_t kDirectChunk = kBlockThreads * 16;    // bytes of an item per workgroup
+constexpr uint32_t kDirectThreads = 64;                  // a workgroup is one wave,
+constexpr uint32_t kDirectChunk = kDirectThreads * 16;   // of an item it takes these bytes
 enum DirectKind : uint32_t { DIRECT_CHAIN = 0, DIRECT_TREE = 1, DIRECT_STACK = 2 };
 
 // CAP = 8: up to 8 sources and destinations per item; CAP = 32: up to 32 (no stack programs).
@@ -143,6 +152,27 @@ template <uint32_t CAP> struct DirectArgs {
 };
 static_assert(sizeof(DirectArgs<32>) <= 4096, "kernel arguments");
 
+// The same for items that are alike, the usual collective: item i reads the send buffers at i * srcStep and writes the receive
+// buffers at i * dstStep, all of them or the one of rank i, and its list of sources is item 0's with i added to every rank (chains:
+// ring, mesh) or exclusive-ored (trees: halving-doubling).  P: the most ranks.  A rank's pointer is base + (off << shift).
+template <uint32_t P> struct PackedArgs {
+    uint64_t base;
+    uint32_t first, last;              // bytes of an item, of the last one
+    uint32_t srcStep, dstStep;
+    uint32_t info;                     // kPacked... fields
+    uint32_t order[P > 16 ? 8 : P / 8];   // item 0's sources: a byte each, four bits up to 16 ranks
+    uint32_t off[2 * P];               // send buffers, then receive buffers
+};
+// A launch costs the host more with every line of arguments, most of all beyond the second one (8 ranks, 128 bytes and up).  Empty
+// kernels one after the other, us, 64, 104, 136, 264, 1352 bytes of arguments: 2.6, 2.8, 3.4, 3.5, 4.1 (2.2, 2.2, 2.35, 2.35, 2.4 while the
+// calling thread happens to run where the arguments' memory is near).
+static_assert(sizeof(PackedArgs<8>) <= 104, "two lines of kernel arguments");
+constexpr uint32_t kPackedSources = 0, kPackedItems = 6, kPackedModulus = 12, kPackedShift = 18;   // lowest bits of the fields of six bits
+constexpr uint32_t kPackedTree = 1u << 24;      // pairwise bottom-up over the sources; else a chain
+constexpr uint32_t kPackedToOne = 1u << 25;     // one destination, the item's rank; else one to every rank of the modulus
+constexpr uint32_t kPackedEnds = 1u << 26;      // some item ends in a part of a vector
+constexpr uint32_t kPackedRing = 1u << 27;      // chain: sources behind the second one are the left operands; else the right ones
+
 // Kernel entry for (data type, reduce op, kind); nullptr if the combination is not built.
 // Signatures:
 //   KK_STEP            (const StepDesc *steps, uint32_t nsteps, uint32_t nwhole, uint32_t ntiles, uint32_t flags)
@@ -156,6 +186,8 @@ static_assert(sizeof(DirectArgs<32>) <= 4096, "kernel arguments");
 //                      Up to seven pointers behind an item's list of sources may be read (and are not used): the destinations'
 //                      pool lies behind the sources', and the tables end on a multiple of 256 bytes.
 //   KK_TEAM_*          the same and (uint32_t *teamBlock)
+//   KK_PACKED_n        (PackedArgs<n>; those of 2, 4 and 8 sources PackedArgs<8>, of 16 PackedArgs<16>), grid (chunks of the longest item, items), with kPackedEnds one more in x, the first one, for the bytes
+//                      behind an item's last whole vector
 //   KK_DIRECT / KK_DIRECT_WIDE   (DirectArgs<8> / DirectArgs<32>), grid (1 + chunks of the longest item, items): blockIdx.x == 0
 //                      is for the bytes behind an item's last whole vector
 const void *LookupKernel(int hcclDataType, int hcclReduceOp, KernelKind kind);
@@ -163,7 +195,7 @@ const void *LookupKernel(int hcclDataType, int hcclReduceOp, KernelKind kind);
 //   KK_GATHER          (const SegDesc *segs, uint32_t nsegs)
 //                      copy kernel table only
 // Byte-wise variants for pure data movement (all-gather, all-to-all-v): KK_STEP, KK_CHAIN, KK_TEAM_CHAIN, KK_GATHER,
-// KK_DIRECT and KK_DIRECT_WIDE.
+// KK_DIRECT, KK_DIRECT_WIDE and KK_PACKED_n.
 const void *LookupCopyKernel(KernelKind kind);
 
 }  // namespace hcclamd

@@ -5,15 +5,17 @@
 // their tables have to be in device memory first.  Here an item's record lies at a place that follows from the block
 // index, all of its pointers are fetched together, and the data loads of up to 16 sources are issued back to back
 // without a branch between them (the number of sources picks straight-line code; a guard per source makes the compiler
-// wait for each load).  Measured on MI355X, time of the kernel, tile form / this form: 8 ranks, ring all-reduce, fp32
-// 8 KiB per rank 4.5 / 3.5 us, bf16 8 KiB 5.8 / 3.2, bf16 512 KiB 6.1 / 3.6; 24 ranks, halving-doubling, bf16 256 KiB
-// 19.7 / 7.6.  An empty kernel takes 2; what is left is two trips to the arguments, one to the data, and the stores.
-// No table is uploaded or kept, so a call with new buffers costs what a repeated one does (8 ranks x 8 KiB through ctypes,
-// 200 sets of buffers used once each: 6.1 us per call, 5.9 repeated; through tables 11.1 and 6.0).
+// wait for each load).  What a launch takes on the device, us, first in first out, 8 ranks: an empty kernel 1.6, all-reduce of fp32 8 KiB per
+// rank 3.5 with a branch per destination, a trip per pointer, and all shapes in one kernel, 2.2 this way; bf16 64 KiB 3.6 / 2.5, 1 MiB 5.9 / 3.4.
+// No table is uploaded or kept, so a call with new buffers costs what a repeated one does.
 //
-// A workgroup handles 4 KiB of one item (blockIdx.y), one 16-byte vector per lane: four times as many workgroups as the
-// tile kernels use.  Accesses are unaligned 128-bit ones (the instruction is the same one), so one form serves every
-// alignment; the bytes behind the last whole vector go element by element to a workgroup of their own (blockIdx.x == 0), side by side with the others.
+// A workgroup is one wave and handles 1 KiB of one item (blockIdx.y), one 16-byte vector per lane: what a CU has in flight limits it, so
+// the work has to spread evenly over the CUs.  8 ranks, fp32, workgroups of 4 KiB / 2 KiB / 1 KiB: 64 KiB 2.5 / 2.2 / 2.2, 1.25 MiB 4.4 / 3.9 / 3.3,
+// 2.25 MiB 7.6 / 7.1 / 6.5 (2 MiB, a whole number of 4 KiB to a CU: 5.6 / 5.9 / 5.8).  Accesses are unaligned 128-bit ones (the instruction is the same
+// one), so one form serves every alignment; the bytes behind the last whole vector go element by element to a workgroup of their own
+// (blockIdx.x == 0), side by side with the others.
+//
+// Two kinds of arguments: a record per item, and for items that are alike, the usual collective, one record for all (PackedArgs).
 #pragma once
 #include "kernels_impl.h"
 
@@ -22,7 +24,27 @@ namespace hcclamd {
 // The kernel arguments where they lie (constant memory): read through the parameter itself, the wide form is copied to
 // private memory first.
 #define HCCL_CONSTANT __attribute__((address_space(4)))
+// All of these, fetched before anything behind it: on its own the compiler waits for one before it asks for the next.
+template <uint32_t N, typename W> __device__ __forceinline__ void Fetched(const W (&w)[N])
+{
+    if constexpr (N == 1) {
+        asm volatile("" ::"s"(w[0]));
+    } else if constexpr (N < 4) {
+        asm volatile("" ::"s"(w[0]), "s"(w[1]), "s"(w[N - 1]));
+    } else if constexpr (N < 8) {
+        asm volatile("" ::"s"(w[0]), "s"(w[1]), "s"(w[2]), "s"(w[3]), "s"(w[N > 4 ? 4 : 0]), "s"(w[N > 5 ? 5 : 0]), "s"(w[N > 6 ? 6 : 0]));
+    } else if constexpr (N == 8) {
+        asm volatile("" ::"s"(w[0]), "s"(w[1]), "s"(w[2]), "s"(w[3]), "s"(w[4]), "s"(w[5]), "s"(w[6]), "s"(w[7]));
+    } else {
+        static_assert(N == 16, "how many are fetched together");
+        asm volatile("" ::"s"(w[0]), "s"(w[1]), "s"(w[2]), "s"(w[3]), "s"(w[4]), "s"(w[5]), "s"(w[6]), "s"(w[7]), "s"(w[8]), "s"(w[9]),
+            "s"(w[10]), "s"(w[11]), "s"(w[12]), "s"(w[13]), "s"(w[14]), "s"(w[15]));
+    }
+}
+
 template <uint32_t CAP> struct DirectView {
+    typedef uint64_t Word;       // what there is of a pointer in the arguments
+    static constexpr bool kMany = CAP > 8;
     const DirectArgs<CAP> HCCL_CONSTANT *args;
     const DirectItem<CAP> HCCL_CONSTANT *it;
     __device__ __forceinline__ DirectView()
@@ -33,31 +55,73 @@ template <uint32_t CAP> struct DirectView {
         asm volatile("" ::"s"(it->bytes), "s"(it->srcOff), "s"(it->dstOff), "s"(it->nsrc), "s"(it->ndst), "s"(it->kind), "s"(it->src[0]),
             "s"(it->src[1]), "s"(it->dst[0]), "s"(it->dst[1]));
     }
+    __device__ __forceinline__ uint32_t Bytes() const { return it->bytes; }
+    __device__ __forceinline__ uint32_t SrcOff() const { return it->srcOff; }
+    __device__ __forceinline__ uint32_t DstOff() const { return it->dstOff; }
+    __device__ __forceinline__ uint32_t Sources() const { return it->nsrc; }
+    __device__ __forceinline__ uint32_t Destinations() const { return it->ndst; }
     // base pointer of entry j of the list of sources / destinations (base indexes, four to a word)
-    __device__ __forceinline__ uint64_t Src(uint32_t j) const { return args->base[(it->src[j >> 2] >> (8u * (j & 3u))) & 0xffu]; }
-    __device__ __forceinline__ uint64_t Dst(uint32_t k) const { return args->base[(it->dst[k >> 2] >> (8u * (k & 3u))) & 0xffu]; }
+    __device__ __forceinline__ Word Src(uint32_t j) const { return args->base[(it->src[j >> 2] >> (8u * (j & 3u))) & 0xffu]; }
+    __device__ __forceinline__ Word Dst(uint32_t k) const { return args->base[(it->dst[k >> 2] >> (8u * (k & 3u))) & 0xffu]; }
+    __device__ __forceinline__ uint64_t Pointer(Word w) const { return w; }
+};
+template <uint32_t P> struct PackedView {
+    typedef uint32_t Word;
+    static constexpr bool kMany = P > 8;
+    static constexpr uint32_t kRanks = P;
+    const PackedArgs<P> HCCL_CONSTANT *k;
+    __device__ __forceinline__ PackedView()
+    {
+        k = (const PackedArgs<P> HCCL_CONSTANT *)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" ::"s"(k->base), "s"(k->first), "s"(k->last), "s"(k->srcStep), "s"(k->dstStep), "s"(k->info), "s"(k->order[0]));
+    }
+    __device__ __forceinline__ uint32_t Field(uint32_t at) const { return (k->info >> at) & 63u; }
+    __device__ __forceinline__ uint32_t Bytes() const
+    {
+        // (a choice between the two is turned into one between their addresses, another trip)
+        const uint32_t f = k->first, l = k->last;
+        return l ^ ((f ^ l) & (blockIdx.y + 1 == Field(kPackedItems) ? 0u : ~0u));
+    }
+    __device__ __forceinline__ uint32_t SrcOff() const { return blockIdx.y * k->srcStep; }
+    __device__ __forceinline__ uint32_t DstOff() const { return blockIdx.y * k->dstStep; }
+    __device__ __forceinline__ uint32_t Sources() const { return Field(kPackedSources); }
+    __device__ __forceinline__ uint32_t Destinations() const { return k->info & kPackedToOne ? 1u : Field(kPackedModulus); }
+    __device__ __forceinline__ uint64_t Pointer(Word w) const { return k->base + (uint64_t(w) << Field(kPackedShift)); }
+    __device__ __forceinline__ uint32_t Order(uint32_t j) const
+    {
+        return P > 16 ? (k->order[(j >> 2) & 7u] >> (8u * (j & 3u))) & 0xffu : (k->order[(j >> 3) & (P / 8 - 1)] >> (4u * (j & 7u))) & 15u;
+    }
+    // source j of a chain, of a tree
+    __device__ __forceinline__ Word Src(uint32_t j) const
+    {
+        const uint32_t sum = Order(j) + blockIdx.y, mod = Field(kPackedModulus);
+        return k->off[min(sum, sum - mod)];       // (below the modulus the difference wraps around)
+    }
+    __device__ __forceinline__ Word Leaf(uint32_t j) const { return k->off[Order(j) ^ blockIdx.y]; }
+    __device__ __forceinline__ Word Dst(uint32_t n) const { return k->off[P + (k->info & kPackedToOne ? blockIdx.y : n)]; }
 };
 
-// N sources from source j0 on into acc.
-template <typename L, typename T, int OP, uint32_t CAP, uint32_t N>
-__device__ __forceinline__ void DirectBatch(const DirectView<CAP> &view, uint32_t j0, uint32_t off,
-    typename L::Val &acc)
+// N sources from source j0 on into acc; FIRST: the first of them starts it.  left(j): the value so far is the left operand.
+template <typename L, typename T, int OP, uint32_t N, bool FIRST, typename View, typename Left>
+__device__ __forceinline__ void DirectBatch(const View &view, uint32_t j0, uint32_t off, typename L::Val &acc, Left left)
 {
-    uint64_t p[N];
+    typename View::Word p[N];
 #pragma unroll
     for (uint32_t j = 0; j < N; j++) {
         p[j] = view.Src(j0 + j);
     }
+    Fetched(p);
     typename L::Val v[N];
 #pragma unroll
     for (uint32_t j = 0; j < N; j++) {
-        v[j] = L::Load(reinterpret_cast<const void *>(p[j]), off);
+        v[j] = L::Load(reinterpret_cast<const void *>(view.Pointer(p[j])), off);
     }
     PinAccesses();
-    acc = j0 == 0 ? v[0] : ((OrderMatters<T, OP>::value && !((view.it->accLeft >> j0) & 1u)) ? L::Combine(v[0], acc) : L::Combine(acc, v[0]));
 #pragma unroll
-    for (uint32_t j = 1; j < N; j++) {
-        if (OrderMatters<T, OP>::value && !((view.it->accLeft >> (j0 + j)) & 1u)) {
+    for (uint32_t j = 0; j < N; j++) {
+        if (FIRST && j == 0) {
+            acc = v[0];
+        } else if (OrderMatters<T, OP>::value && !left(j0 + j)) {
             acc = L::Combine(v[j], acc);
         } else {
             acc = L::Combine(acc, v[j]);
@@ -65,33 +129,66 @@ __device__ __forceinline__ void DirectBatch(const DirectView<CAP> &view, uint32_
     }
 }
 
-template <typename L, typename T, int OP, uint32_t CAP>
-__device__ __forceinline__ typename L::Val DirectChain(const DirectView<CAP> &view, uint32_t off)
+// first(j), later(j): whether the value so far is the left operand, for the sources loaded first and for those behind them.
+template <typename L, typename T, int OP, typename View, typename First, typename Later>
+__device__ __forceinline__ typename L::Val DirectChain(const View &view, uint32_t off, First first, Later later)
 {
     typename L::Val acc;
-    const uint32_t nsrc = view.it->nsrc;
-    uint32_t j = 0;
-    if (CAP > 8) {
-#pragma nounroll
-        for (; j + 16 <= nsrc; j += 16) {
-            DirectBatch<L, T, OP, CAP, 16>(view, j, off, acc);
-        }
+    const uint32_t nsrc = view.Sources();
+    if (__builtin_expect(nsrc == 8, 1)) {
+        DirectBatch<L, T, OP, 8, true>(view, 0, off, acc, first);
+        return acc;
     }
-    if (j + 8 <= nsrc) {
-        DirectBatch<L, T, OP, CAP, 8>(view, j, off, acc);
-        j += 8;
-    }
-    switch (nsrc - j) {
-        case 1: DirectBatch<L, T, OP, CAP, 1>(view, j, off, acc); break;
-        case 2: DirectBatch<L, T, OP, CAP, 2>(view, j, off, acc); break;
-        case 3: DirectBatch<L, T, OP, CAP, 3>(view, j, off, acc); break;
-        case 4: DirectBatch<L, T, OP, CAP, 4>(view, j, off, acc); break;
-        case 5: DirectBatch<L, T, OP, CAP, 5>(view, j, off, acc); break;
-        case 6: DirectBatch<L, T, OP, CAP, 6>(view, j, off, acc); break;
-        case 7: DirectBatch<L, T, OP, CAP, 7>(view, j, off, acc); break;
+    switch (nsrc) {
+        case 1: DirectBatch<L, T, OP, 1, true>(view, 0, off, acc, first); return acc;
+        case 2: DirectBatch<L, T, OP, 2, true>(view, 0, off, acc, first); return acc;
+        case 3: DirectBatch<L, T, OP, 3, true>(view, 0, off, acc, first); return acc;
+        case 4: DirectBatch<L, T, OP, 4, true>(view, 0, off, acc, first); return acc;
+        case 5: DirectBatch<L, T, OP, 5, true>(view, 0, off, acc, first); return acc;
+        case 6: DirectBatch<L, T, OP, 6, true>(view, 0, off, acc, first); return acc;
+        case 7: DirectBatch<L, T, OP, 7, true>(view, 0, off, acc, first); return acc;
         default: break;
     }
+    if constexpr (View::kMany) {
+        uint32_t j = 8;
+        if (nsrc >= 16) {
+            DirectBatch<L, T, OP, 16, true>(view, 0, off, acc, first);
+            j = 16;
+        } else {
+            DirectBatch<L, T, OP, 8, true>(view, 0, off, acc, first);
+        }
+#pragma nounroll
+        for (; j + 16 <= nsrc; j += 16) {
+            DirectBatch<L, T, OP, 16, false>(view, j, off, acc, later);
+        }
+        if (j + 8 <= nsrc) {
+            DirectBatch<L, T, OP, 8, false>(view, j, off, acc, later);
+            j += 8;
+        }
+        switch (nsrc - j) {
+            case 1: DirectBatch<L, T, OP, 1, false>(view, j, off, acc, later); break;
+            case 2: DirectBatch<L, T, OP, 2, false>(view, j, off, acc, later); break;
+            case 3: DirectBatch<L, T, OP, 3, false>(view, j, off, acc, later); break;
+            case 4: DirectBatch<L, T, OP, 4, false>(view, j, off, acc, later); break;
+            case 5: DirectBatch<L, T, OP, 5, false>(view, j, off, acc, later); break;
+            case 6: DirectBatch<L, T, OP, 6, false>(view, j, off, acc, later); break;
+            case 7: DirectBatch<L, T, OP, 7, false>(view, j, off, acc, later); break;
+            default: break;
+        }
+    }
     return acc;
+}
+
+// N values pairwise, bottom-up, into the first of them.
+template <typename L, uint32_t N> __device__ __forceinline__ void DirectPairwise(typename L::Val (&v)[N])
+{
+#pragma unroll
+    for (uint32_t w = 1; w < N; w <<= 1) {
+#pragma unroll
+        for (uint32_t i = 0; i + w < N; i += 2 * w) {
+            v[i] = L::Combine(v[i], v[i + w]);
+        }
+    }
 }
 
 // G leaves from leaf i0 on, folded pairwise.  `second` of the item: the leaves that are two sources combined; the list of second
@@ -99,16 +196,27 @@ __device__ __forceinline__ typename L::Val DirectChain(const DirectView<CAP> &vi
 template <typename L, uint32_t CAP, uint32_t G>
 __device__ __forceinline__ typename L::Val DirectLeaves(const DirectView<CAP> &view, uint32_t i0, uint32_t off)
 {
+    uint64_t p[G];
+#pragma unroll
+    for (uint32_t i = 0; i < G; i++) {
+        p[i] = view.Src(i0 + i);
+    }
+    Fetched(p);
     typename L::Val v[G];
 #pragma unroll
     for (uint32_t i = 0; i < G; i++) {
-        v[i] = L::Load(reinterpret_cast<const void *>(view.Src(i0 + i)), off);
+        v[i] = L::Load(reinterpret_cast<const void *>(p[i]), off);
     }
     if (view.it->second != 0) {
         typename L::Val w[G];
 #pragma unroll
         for (uint32_t i = 0; i < G; i++) {
-            w[i] = L::Load(reinterpret_cast<const void *>(view.Src(kDirectSecond<CAP> + i0 + i)), off);
+            p[i] = view.Src(kDirectSecond<CAP> + i0 + i);
+        }
+        Fetched(p);
+#pragma unroll
+        for (uint32_t i = 0; i < G; i++) {
+            w[i] = L::Load(reinterpret_cast<const void *>(p[i]), off);
         }
         PinAccesses();
 #pragma unroll
@@ -119,13 +227,7 @@ __device__ __forceinline__ typename L::Val DirectLeaves(const DirectView<CAP> &v
         }
     }
     PinAccesses();
-#pragma unroll
-    for (uint32_t w = 1; w < G; w <<= 1) {
-#pragma unroll
-        for (uint32_t i = 0; i + w < G; i += 2 * w) {
-            v[i] = L::Combine(v[i], v[i + w]);
-        }
-    }
+    DirectPairwise<L, G>(v);
     return v[0];
 }
 
@@ -156,10 +258,16 @@ template <typename L, typename T, int OP, uint32_t CAP>
 __device__ __forceinline__ typename L::Val DirectStack(const DirectView<CAP> &view, uint32_t off)
 {
     constexpr bool DEEP = false;
-    typename L::Val v[8];
+    uint64_t p[8];
 #pragma unroll
     for (uint32_t j = 0; j < 8; j++) {      // the list repeats its last source up to 8
-        v[j] = L::Load(reinterpret_cast<const void *>(view.Src(j)), off);
+        p[j] = view.Src(j);
+    }
+    Fetched(p);
+    typename L::Val v[8];
+#pragma unroll
+    for (uint32_t j = 0; j < 8; j++) {
+        v[j] = L::Load(reinterpret_cast<const void *>(p[j]), off);
     }
     PinAccesses();
     typename L::Val top = v[0], b0 = top, b1 = top, b2 = top, b3 = top, b4 = top, b5 = top, b6 = top;   // (b3 ... b6 only named)
@@ -191,94 +299,206 @@ __device__ __forceinline__ typename L::Val DirectStack(const DirectView<CAP> &vi
     return top;
 }
 
-// The first 8 destinations, fetched before the data (the list is padded: no guards).
-template <uint32_t CAP>
-__device__ __forceinline__ void DirectFetchDst(const DirectView<CAP> &view, uint32_t k0, uint64_t (&o)[8])
+template <typename L, typename T, int OP, uint32_t CAP>
+__device__ __forceinline__ typename L::Val DirectValue(const DirectView<CAP> &view, uint32_t off)
 {
-#pragma unroll
-    for (uint32_t k = 0; k < 8; k++) {
-        o[k] = view.Dst(k0 + k);
+    if (view.it->kind == DIRECT_CHAIN) {
+        auto left = [&](uint32_t j) { return ((view.it->accLeft >> j) & 1u) != 0; };
+        return DirectChain<L, T, OP>(view, off, left, left);
     }
+    if (CAP > 8 || view.it->kind == DIRECT_TREE) {
+        return DirectTree<L, CAP>(view, off);
+    }
+    return DirectStack<L, T, OP, CAP>(view, off);
 }
 
-template <typename L, uint32_t CAP>
-__device__ __forceinline__ void DirectStore(const DirectView<CAP> &view, uint64_t (&o)[8], uint32_t at, typename L::Val r)
+// G sources from source j0 on, pairwise.
+template <typename L, uint32_t P, uint32_t G>
+__device__ __forceinline__ typename L::Val PackedLeaves(const PackedView<P> &view, uint32_t j0, uint32_t off)
 {
-    const uint32_t ndst = view.it->ndst, to = view.it->dstOff + at;
-    for (uint32_t k0 = 0;;) {
+    uint32_t p[G];
 #pragma unroll
-        for (uint32_t k = 0; k < 8; k++) {
-            if (k0 + k < ndst) {
-                L::Store(reinterpret_cast<void *>(o[k]), to, r);
+    for (uint32_t i = 0; i < G; i++) {
+        p[i] = view.Leaf(j0 + i);
+    }
+    Fetched(p);
+    typename L::Val v[G];
+#pragma unroll
+    for (uint32_t i = 0; i < G; i++) {
+        v[i] = L::Load(reinterpret_cast<const void *>(view.Pointer(p[i])), off);
+    }
+    PinAccesses();
+    DirectPairwise<L, G>(v);
+    return v[0];
+}
+template <typename L, typename T, int OP, uint32_t P>
+__device__ __forceinline__ typename L::Val DirectValue(const PackedView<P> &view, uint32_t off)
+{
+    if (__builtin_expect((view.k->info & kPackedTree) != 0, 0)) {
+        switch (view.Sources()) {
+            case 2: return PackedLeaves<L, P, 2>(view, 0, off);
+            case 4: return PackedLeaves<L, P, 4>(view, 0, off);
+            case 8: return PackedLeaves<L, P, 8>(view, 0, off);
+            default: break;
+        }
+        if constexpr (P > 8) {
+            typename L::Val v = PackedLeaves<L, P, 16>(view, 0, off);
+            if (P > 16 && view.Sources() == 32) {
+                v = L::Combine(v, PackedLeaves<L, P, 16>(view, 16, off));
+            }
+            return v;
+        } else {
+            return typename L::Val();
+        }
+    }
+    auto yes = [](uint32_t) { return true; };
+    if (OrderMatters<T, OP>::value && (view.k->info & kPackedRing) != 0) {
+        return DirectChain<L, T, OP>(view, off, [](uint32_t j) { return j < 2; }, [](uint32_t) { return false; });
+    }
+    return DirectChain<L, T, OP>(view, off, yes, yes);
+}
+
+// A lane's vector to every destination: N at a time without a branch between them, those behind the last one dropped by the
+// range check of their buffers.  A branch per destination is a jump to a line of code that has to be fetched, and a pointer fetched
+// where it is used a trip to the arguments.  Written through: plain non-temporal stores take half as long again at 1 MiB per rank.
+template <uint32_t N, typename View>
+__device__ __forceinline__ void DirectStoreTo(const View &view, uint32_t k0, uint32_t ndst, uint32_t at, V4 r)
+{
+    const uint32_t bytes = view.Bytes() & ~15u, to = view.DstOff();
+    typename View::Word o[N];
+#pragma unroll
+    for (uint32_t k = 0; k < N; k++) {
+        o[k] = view.Dst(k0 + k);      // (the lists are padded)
+    }
+    Fetched(o);
+#pragma unroll
+    for (uint32_t k = 0; k < N; k++) {
+        BufferStore16<STORE_THROUGH>(MakeBuffer(reinterpret_cast<void *>(view.Pointer(o[k]) + to), k0 + k < ndst ? bytes : 0u), at, r);
+    }
+}
+template <typename View>
+__device__ __forceinline__ void DirectStore(const View &view, uint32_t at, V4 r)
+{
+    const uint32_t ndst = view.Destinations();
+    if (__builtin_expect(ndst > 4, 1)) {
+        DirectStoreTo<8>(view, 0, ndst, at, r);
+        if constexpr (View::kMany) {
+#pragma nounroll
+            for (uint32_t k0 = 8; k0 < ndst; k0 += 8) {
+                DirectStoreTo<8>(view, k0, ndst, at, r);
             }
         }
-        k0 += 8;
-        if (CAP <= 8 || k0 >= ndst) {
-            break;
-        }
-        DirectFetchDst<CAP>(view, k0, o);
-    }
-}
-
-// One lane's position: its value, and where that goes.
-template <typename L, typename T, int OP, uint32_t CAP>
-__device__ __forceinline__ void DirectLane(const DirectView<CAP> &view, uint32_t at)
-{
-    const uint32_t off = view.it->srcOff + at;
-    uint64_t o[8];
-    DirectFetchDst<CAP>(view, 0, o);
-    typename L::Val r;
-    if (view.it->kind == DIRECT_CHAIN) {
-        r = DirectChain<L, T, OP, CAP>(view, off);
-    } else if (CAP > 8 || view.it->kind == DIRECT_TREE) {
-        r = DirectTree<L, CAP>(view, off);
+    } else if (ndst == 1) {
+        DirectStoreTo<1>(view, 0, ndst, at, r);
     } else {
-        r = DirectStack<L, T, OP, CAP>(view, off);
+        DirectStoreTo<4>(view, 0, ndst, at, r);
     }
-    DirectStore<L, CAP>(view, o, at, r);
 }
 
-template <typename L, uint32_t CAP>
-__device__ __forceinline__ void DirectMove(const DirectView<CAP> &view, uint32_t at)
+// The item's whole vectors, a lane's at byte `at`, or the element behind them that is this lane's.
+template <typename T, int OP, typename View> __device__ __forceinline__ void DirectVector(const View &view, uint32_t at)
 {
-    uint64_t o[8];
-    DirectFetchDst<CAP>(view, 0, o);
-    const typename L::Val r = L::Load(reinterpret_cast<const void *>(view.Src(0)), view.it->srcOff + at);
-    DirectStore<L, CAP>(view, o, at, r);
+    if (at + 16u <= view.Bytes()) {
+        DirectStore(view, at, DirectValue<VecLane<T, OP>, T, OP>(view, view.SrcOff() + at));
+    }
+}
+template <typename View, typename Value> __device__ __forceinline__ void DirectEnd(const View &view, Value value)
+{
+    typedef decltype(value(0u)) T;
+    const uint32_t rest = view.Bytes() & 15u, mine = threadIdx.x * uint32_t(sizeof(T));
+    if (mine < rest) {
+        const uint32_t at = view.Bytes() - rest + mine, ndst = view.Destinations();
+        const T r = value(view.SrcOff() + at);
+#pragma nounroll
+        for (uint32_t k = 0; k < ndst; k++) {
+            StoreElem<T>(reinterpret_cast<void *>(view.Pointer(view.Dst(k))), view.DstOff() + at, r);
+        }
+    }
 }
 
 template <typename T, int OP, uint32_t CAP>
-__global__ void __launch_bounds__(kBlockThreads) DirectKernel(const DirectArgs<CAP>)
+__global__ void __launch_bounds__(kDirectThreads) DirectKernel(const DirectArgs<CAP>)
 {
     const DirectView<CAP> view;
     if (blockIdx.x != 0) {
-        const uint32_t at = (blockIdx.x - 1) * kDirectChunk + threadIdx.x * 16u;
-        if (at + 16u <= view.it->bytes) {
-            DirectLane<VecLane<T, OP>, T, OP, CAP>(view, at);
+        DirectVector<T, OP>(view, (blockIdx.x - 1) * kDirectChunk + threadIdx.x * 16u);
+    } else {
+        DirectEnd(view, [&](uint32_t off) { return DirectValue<ElemLane<T, OP>, T, OP>(view, off); });
+    }
+}
+template <typename T, int OP, uint32_t P>
+__global__ void __launch_bounds__(kDirectThreads) PackedKernel(const PackedArgs<P>)
+{
+    const PackedView<P> view;
+    const uint32_t ends = view.k->info & kPackedEnds ? 1u : 0u;
+    if (blockIdx.x >= ends) {
+        DirectVector<T, OP>(view, (blockIdx.x - ends) * kDirectChunk + threadIdx.x * 16u);
+    } else {
+        DirectEnd(view, [&](uint32_t off) { return DirectValue<ElemLane<T, OP>, T, OP>(view, off); });
+    }
+}
+
+// The usual numbers of sources, each with a kernel of its own, in which the way of a vector is one stretch of code: with all numbers
+// and shapes in one kernel the way leads over half a dozen jumps to lines that have to be fetched.  8 ranks, device time per launch, us,
+// one kernel / this way: fp32 8 KiB 2.5 / 2.1, 64 KiB 2.9 / 2.4, 1 MiB 3.4 / 3.0; bf16 2.8 / 2.4, 3.2 / 2.7, 3.7 / 3.3.
+// (Two sources have one order for every shape: the first is the left operand.)
+enum PackedOrder : int { PACKED_LEFT = 0, PACKED_RING = 1, PACKED_TREE = 2 };
+template <typename L, typename T, int OP, uint32_t N, int SHAPE, typename View>
+__device__ __forceinline__ typename L::Val PackedValue(const View &view, uint32_t off)
+{
+    if constexpr (SHAPE == PACKED_TREE) {
+        return PackedLeaves<L, View::kRanks, N>(view, 0, off);
+    } else {
+        typename L::Val acc;
+        DirectBatch<L, T, OP, N, true>(view, 0, off, acc, [](uint32_t j) { return SHAPE == PACKED_LEFT || j < 2; });
+        return acc;
+    }
+}
+template <typename T, int OP, uint32_t P, uint32_t N, int SHAPE>
+__global__ void __launch_bounds__(kDirectThreads) PackedShapeKernel(const PackedArgs<P>)
+{
+    const PackedView<P> view;
+    const uint32_t ends = view.k->info & kPackedEnds ? 1u : 0u;
+    if (blockIdx.x >= ends) {
+        const uint32_t at = (blockIdx.x - ends) * kDirectChunk + threadIdx.x * 16u;
+        if (at + 16u <= view.Bytes()) {
+            DirectStore(view, at, PackedValue<VecLane<T, OP>, T, OP, N, SHAPE>(view, view.SrcOff() + at));
         }
     } else {
-        const uint32_t rest = view.it->bytes & 15u;
-        if (threadIdx.x * uint32_t(sizeof(T)) < rest) {
-            DirectLane<ElemLane<T, OP>, T, OP, CAP>(view, view.it->bytes - rest + threadIdx.x * uint32_t(sizeof(T)));
-        }
+        DirectEnd(view, [&](uint32_t off) { return PackedValue<ElemLane<T, OP>, T, OP, N, SHAPE>(view, off); });
     }
 }
 
 // Pure data movement: one source per item.
+template <typename View> __device__ __forceinline__ void DirectMove(const View &view, uint32_t at)
+{
+    if (at + 16u <= view.Bytes()) {
+        DirectStore(view, at, MoveLane::Load(reinterpret_cast<const void *>(view.Pointer(view.Src(0))), view.SrcOff() + at));
+    }
+}
+template <typename View> __device__ __forceinline__ void DirectMoveEnd(const View &view)
+{
+    DirectEnd(view, [&](uint32_t off) { return LoadElem<uint8_t>(reinterpret_cast<const void *>(view.Pointer(view.Src(0))), off); });
+}
 template <uint32_t CAP>
-__global__ void __launch_bounds__(kBlockThreads) DirectCopyKernel(const DirectArgs<CAP>)
+__global__ void __launch_bounds__(kDirectThreads) DirectCopyKernel(const DirectArgs<CAP>)
 {
     const DirectView<CAP> view;
     if (blockIdx.x != 0) {
-        const uint32_t at = (blockIdx.x - 1) * kDirectChunk + threadIdx.x * 16u;
-        if (at + 16u <= view.it->bytes) {
-            DirectMove<VecLane<uint8_t, ROP_SUM>, CAP>(view, at);
-        }
+        DirectMove(view, (blockIdx.x - 1) * kDirectChunk + threadIdx.x * 16u);
     } else {
-        const uint32_t rest = view.it->bytes & 15u;
-        if (threadIdx.x < rest) {
-            DirectMove<ElemLane<uint8_t, ROP_SUM>, CAP>(view, view.it->bytes - rest + threadIdx.x);
-        }
+        DirectMoveEnd(view);
+    }
+}
+template <uint32_t P>
+__global__ void __launch_bounds__(kDirectThreads) PackedCopyKernel(const PackedArgs<P>)
+{
+    const PackedView<P> view;
+    const uint32_t ends = view.k->info & kPackedEnds ? 1u : 0u;
+    if (blockIdx.x >= ends) {
+        DirectMove(view, (blockIdx.x - ends) * kDirectChunk + threadIdx.x * 16u);
+    } else {
+        DirectMoveEnd(view);
     }
 }
 

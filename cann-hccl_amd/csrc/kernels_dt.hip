@@ -53,15 +53,23 @@ using DT = uint8_t;
 
 #if HCCL_DT == 255
 // pure data movement: the step kernel's copy path and the copy kernel
-extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[6] = {
+extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[9] = {
     reinterpret_cast<const void *>(&StepKernel<DT, ROP_SUM>),
     reinterpret_cast<const void *>(&CopyKernel<0>),
     reinterpret_cast<const void *>(&GatherKernel<0>),
     reinterpret_cast<const void *>(&TeamCopyKernel<0>),
     reinterpret_cast<const void *>(&DirectCopyKernel<8>),
     reinterpret_cast<const void *>(&DirectCopyKernel<32>),
+    reinterpret_cast<const void *>(&PackedCopyKernel<8>),
+    reinterpret_cast<const void *>(&PackedCopyKernel<16>),
+    reinterpret_cast<const void *>(&PackedCopyKernel<32>),
 };
 #else
+#define HCCL_SHAPES(OP, SHAPE)                                                                                                   \
+    reinterpret_cast<const void *>(&PackedShapeKernel<DT, OP, 8, 2, SHAPE == PACKED_LEFT ? SHAPE : PACKED_LEFT>),                 \
+        reinterpret_cast<const void *>(&PackedShapeKernel<DT, OP, 8, 4, SHAPE>),                                                  \
+        reinterpret_cast<const void *>(&PackedShapeKernel<DT, OP, 8, 8, SHAPE>),                                                  \
+        reinterpret_cast<const void *>(&PackedShapeKernel<DT, OP, 16, 16, SHAPE>)
 #define HCCL_ROW(OP)                                                     \
     {                                                                    \
         reinterpret_cast<const void *>(&StepKernel<DT, OP>),             \
@@ -75,6 +83,10 @@ extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[6] = {
         reinterpret_cast<const void *>(&DirectKernel<DT, OP, 32>),       \
         reinterpret_cast<const void *>(&TeamStackKernel<DT, OP, sizeof(DT) != 8 && (sizeof(DT) != 1 || OP != ROP_PROD)>),   \
         reinterpret_cast<const void *>(&ChainKernel<DT, OP, true>),      \
+        reinterpret_cast<const void *>(&PackedKernel<DT, OP, 8>),        \
+        reinterpret_cast<const void *>(&PackedKernel<DT, OP, 16>),       \
+        reinterpret_cast<const void *>(&PackedKernel<DT, OP, 32>),       \
+        HCCL_SHAPES(OP, PACKED_LEFT), HCCL_SHAPES(OP, (OrderMatters<DT, OP>::value ? PACKED_RING : PACKED_LEFT)), HCCL_SHAPES(OP, PACKED_TREE),   \
     }
 extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[4][KK_COUNT] = {
     HCCL_ROW(ROP_SUM), HCCL_ROW(ROP_PROD), HCCL_ROW(ROP_MAX), HCCL_ROW(ROP_MIN),

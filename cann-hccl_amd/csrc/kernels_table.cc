@@ -6,7 +6,7 @@ namespace hcclamd {
 #define HCCL_DECL(name) extern const void *const kKernels_##name[4][KK_COUNT];
 HCCL_DECL(int8) HCCL_DECL(int16) HCCL_DECL(int32) HCCL_DECL(fp16) HCCL_DECL(fp32) HCCL_DECL(int64)
 HCCL_DECL(uint64) HCCL_DECL(uint8) HCCL_DECL(uint16) HCCL_DECL(uint32) HCCL_DECL(fp64) HCCL_DECL(bf16)
-extern const void *const kKernels_bytes[6];
+extern const void *const kKernels_bytes[9];
 
 const void *LookupKernel(int dt, int op, KernelKind kind)
 {
@@ -46,6 +46,9 @@ const void *LookupCopyKernel(KernelKind kind)
     }
     if (kind == KK_DIRECT || kind == KK_DIRECT_WIDE) {
         return kKernels_bytes[kind == KK_DIRECT ? 4 : 5];
+    }
+    if (kind == KK_PACKED_8 || kind == KK_PACKED_16 || kind == KK_PACKED_32) {
+        return kKernels_bytes[6 + kind - KK_PACKED_8];
     }
     return nullptr;
 }

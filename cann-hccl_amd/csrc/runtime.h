@@ -138,13 +138,21 @@ struct DirectLaunch {
     std::vector<std::pair<uint32_t, uint8_t>> bases;   // (rank, buffer) of every base pointer
     std::vector<uint8_t> image;                        // the kernel's arguments, a DirectArgs
     std::vector<uint64_t> sendBytes, recvBytes;        // per rank, as the plan's
+    const void *packedFunc = nullptr;                  // the same collective with a PackedArgs, nullptr: its items are not alike
+    uint32_t packedRanks = 0, packedGridX = 0;         // ranks that its arguments have room for
+    std::vector<uint8_t> packed;
+    bool usePacked = false;                            // this call's buffers fit it
     OpInfo info;
 };
 
 // Whether a collective is small enough for this form, whatever its schedule (bytes: of the call's count).
 bool DirectFits(int coll, uint32_t p, uint64_t bytes, int dtype);
+// Whether a larger one goes out in the packed form if its items are alike.
+bool PackedFits(int coll, uint32_t p, uint64_t bytes);
 // The launch of `plan`; false (func == nullptr) where the kernels' records cannot hold it.
 bool BuildDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaunch *d);
+// The packed form of a launch that BuildDirect has made, where the plan's items are alike.
+void PackDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaunch *d);
 // Puts the ranks' pointers in; true if they were there already (the previous call's).
 bool FillBases(DirectLaunch *d, const std::vector<void *> &send, const std::vector<void *> &recv);
 

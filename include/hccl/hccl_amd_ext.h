@@ -98,7 +98,7 @@ typedef struct HcclAmdOpInfoDef {
     uint64_t schedWritten;
     uint64_t scratchBytes;   /* per-rank scratch in use */
     uint32_t teamLaunches;   /* how many of the launches are team kernels (setting "team") */
-    uint32_t direct;         /* 1: one launch whose descriptors ride in its arguments (setting "direct") */
+    uint32_t direct;         /* 1: a small collective, one launch whose descriptors ride in its arguments (setting "direct") */
 } HcclAmdOpInfo;
 
 /* What the most recent collective of this communicator's group issued. */

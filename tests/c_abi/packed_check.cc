@@ -1,0 +1,216 @@
+// The packed arguments of small collectives (cann-hccl_amd/csrc/direct.cc, PackDirect) against the planner, on the host: a seeded
+// walk over requests and buffers.  The arguments are read back as the kernels of kernels_direct.h read them, to addresses, and
+// every item has to be the plan's: the same expression over the same addresses, the same destinations.  A usual collective
+// (ring, uncut mesh, halving-doubling over a power of two) has to be taken.  argv[1] = requests.  Prints how many went which way.
+#include <algorithm>
+#include <cstdio>
+#include <cstdlib>
+#include <set>
+#include <string>
+#include <vector>
+
+#include "runtime.h"
+
+namespace hcclamd {
+static const char g_kernels[KK_COUNT] = {};
+const void *LookupKernel(int, int, KernelKind kind) { return &g_kernels[kind]; }
+const void *LookupCopyKernel(KernelKind kind) { return &g_kernels[kind]; }
+}  // namespace hcclamd
+
+using namespace hcclamd;
+
+namespace {
+
+uint64_t g_state = 0x9E3779B97F4A7C15ull;
+uint64_t Below(uint64_t n)
+{
+    g_state = g_state * 6364136223846793005ull + 1442695040888963407ull;
+    return n == 0 ? 0 : (g_state >> 29) % n;
+}
+
+std::string At(uint64_t a) { return std::to_string(a); }
+std::string Both(const std::string &a, const std::string &b) { return "(" + a + "+" + b + ")"; }
+std::string Pairwise(std::vector<std::string> v)
+{
+    for (size_t w = 1; w < v.size(); w <<= 1) {
+        for (size_t i = 0; i + w < v.size(); i += 2 * w) {
+            v[i] = Both(v[i], v[i + w]);
+        }
+    }
+    return v[0];
+}
+
+struct Item {
+    uint64_t bytes = 0;
+    std::string value;
+    std::set<uint64_t> dst;
+};
+
+Item OfPlan(const FusedItem &f, const std::vector<void *> &send, const std::vector<void *> &recv)
+{
+    auto where = [&](const Ref &r) { return reinterpret_cast<uint64_t>((r.buf == BUF_SEND ? send : recv)[r.rank]) + r.off; };
+    Item it;
+    it.bytes = f.bytes;
+    for (const Ref &d : f.dst) {
+        it.dst.insert(where(d));
+    }
+    if (f.kind == FK_TREE) {
+        std::vector<std::string> leaf;
+        for (uint32_t i = 0; i < f.nleaf; i++) {
+            leaf.push_back(f.srcValid[2 * i + 1] ? Both(At(where(f.src[2 * i])), At(where(f.src[2 * i + 1]))) : At(where(f.src[2 * i])));
+        }
+        it.value = Pairwise(leaf);
+        return it;
+    }
+    it.value = At(where(f.src[0]));
+    for (size_t j = 1; j < f.src.size(); j++) {
+        it.value = f.accLeft[j] ? Both(it.value, At(where(f.src[j]))) : Both(At(where(f.src[j])), it.value);
+    }
+    return it;
+}
+
+template <uint32_t P> Item OfArguments(const PackedArgs<P> &k, uint32_t i, bool *ok)
+{
+    auto field = [&](uint32_t at) { return (k.info >> at) & 63u; };
+    auto pointer = [&](uint32_t n) {
+        *ok = *ok && n < 2 * P;
+        return k.base + (uint64_t(k.off[n % (2 * P)]) << field(kPackedShift));
+    };
+    const uint32_t nsrc = field(kPackedSources), mod = field(kPackedModulus);
+    *ok = *ok && nsrc >= 1 && nsrc <= P && mod <= P && i < mod;
+    std::vector<std::string> src;
+    for (uint32_t j = 0; j < nsrc; j++) {
+        const uint32_t o = P > 16 ? (k.order[j / 4] >> (8 * (j % 4))) & 0xff : (k.order[j / 8] >> (4 * (j % 8))) & 15;
+        const uint32_t r = (k.info & kPackedTree) ? o ^ i : (o + i >= mod ? o + i - mod : o + i);
+        *ok = *ok && r < mod;
+        src.push_back(At(pointer(r) + uint64_t(i) * k.srcStep));
+    }
+    Item it;
+    it.bytes = i + 1 == field(kPackedItems) ? k.last : k.first;
+    if (k.info & kPackedTree) {
+        *ok = *ok && (nsrc & (nsrc - 1)) == 0 && nsrc >= 2;
+        it.value = Pairwise(src);
+    } else {
+        it.value = src[0];
+        for (uint32_t j = 1; j < nsrc; j++) {
+            const bool left = !(k.info & kPackedRing) || j < 2;
+            it.value = left ? Both(it.value, src[j]) : Both(src[j], it.value);
+        }
+    }
+    for (uint32_t n = 0; n < ((k.info & kPackedToOne) ? 1 : mod); n++) {
+        it.dst.insert(pointer(P + ((k.info & kPackedToOne) ? i : n)) + uint64_t(i) * k.dstStep);
+    }
+    return it;
+}
+
+template <uint32_t P> bool Same(const Plan &plan, const DirectLaunch &d, const std::vector<void *> &send, const std::vector<void *> &recv)
+{
+    if (d.packed.size() != sizeof(PackedArgs<P>)) {
+        return false;
+    }
+    const PackedArgs<P> &k = *reinterpret_cast<const PackedArgs<P> *>(d.packed.data());
+    // the kernel: one of its own for 2, 4, 8 or 16 sources of as many ranks, else the one for the arguments
+    const uint32_t nsrc = (k.info >> kPackedSources) & 63u, mod = (k.info >> kPackedModulus) & 63u, shape = PackedShape(nsrc);
+    int kind = P == 8 ? KK_PACKED_8 : P == 16 ? KK_PACKED_16 : KK_PACKED_32;
+    if (shape < kPackedShapes && nsrc == mod) {
+        kind = int(shape) + ((k.info & kPackedTree) ? KK_PACKED_TREE : (k.info & kPackedRing) ? KK_PACKED_RING : KK_PACKED_CHAIN);
+        if (P != (nsrc == 16 ? 16 : 8)) {
+            return false;
+        }
+    }
+    if (d.packedFunc != LookupKernel(0, 0, KernelKind(kind))) {
+        return false;
+    }
+    const uint32_t ends = (k.info & kPackedEnds) ? 1 : 0;
+    bool ok = ((k.info >> kPackedItems) & 63u) == plan.fused.size() && d.gridY == plan.fused.size();
+    for (uint32_t i = 0; ok && i < plan.fused.size(); i++) {
+        const Item a = OfPlan(plan.fused[i], send, recv), b = OfArguments<P>(k, i, &ok);
+        ok = ok && a.bytes == b.bytes && a.value == b.value && a.dst == b.dst && (a.bytes % 16 == 0 || ends) &&
+            uint64_t(d.packedGridX - ends) * kDirectChunk >= a.bytes / 16 * 16;
+    }
+    return ok;
+}
+
+}  // namespace
+
+int main(int argc, char **argv)
+{
+    const long want = argc > 1 ? std::atol(argv[1]) : 3000;
+    long taken[3] = {0, 0, 0}, unlike = 0, apart = 0, trees = 0, inPlace = 0;
+    for (long n = 0; n < want;) {
+        PlanRequest rq;
+        const int colls[] = {COLL_ALLREDUCE, COLL_ALLREDUCE, COLL_REDUCESCATTER, COLL_ALLGATHER, COLL_BROADCAST, COLL_REDUCE, COLL_SCATTER};
+        rq.coll = CollKind(colls[Below(Below(4) ? 4 : 7)]);
+        const Algo algos[] = {ALGO_RING, ALGO_RING, ALGO_MESH, ALGO_MESH_ATOMIC, ALGO_RHD};
+        rq.algo = algos[Below(5)];
+        rq.p = uint32_t(Below(3) ? 1 + Below(8) : 1 + Below(40));
+        if (rq.algo == ALGO_MESH && rq.p > 12) {
+            rq.p = uint32_t(2 + Below(11));
+        }
+        if (rq.coll == COLL_SCATTER) {
+            rq.algo = ALGO_MESH;
+        }
+        if (Below(8) == 0 && rq.p % 2 == 0 && rq.p > 2) {
+            rq.servers = 2;
+        }
+        const uint32_t units[] = {1, 2, 4, 8};
+        rq.unit = units[Below(4)];
+        rq.root = uint32_t(Below(rq.p));
+        const bool same = rq.coll == COLL_BROADCAST || (rq.coll == COLL_ALLREDUCE && Below(2));
+        rq.alias.assign(rq.p, same ? 1 : 0);
+        rq.count = 1 + Below(Below(2) ? 300 : 40000 / rq.p);
+        Plan plan;
+        std::string err;
+        DirectLaunch d;
+        if (BuildPlan(rq, &plan, &err) != 0 || !BuildDirect(plan, true, 4, 0, &d)) {
+            continue;
+        }
+        n++;
+        PackDirect(plan, true, 4, 0, &d);
+        const bool usual = rq.p <= 32 && rq.servers == 1 &&
+            ((rq.coll == COLL_ALLGATHER) || ((rq.coll == COLL_ALLREDUCE || rq.coll == COLL_REDUCESCATTER) &&
+                (rq.algo == ALGO_RING || rq.algo == ALGO_MESH_ATOMIC || (rq.algo == ALGO_RHD && (rq.p & (rq.p - 1)) == 0))));
+        if (usual && rq.p > 1 && d.packedFunc == nullptr) {
+            std::printf("coll %d algo %d p %u count %llu unit %u: not taken\n", int(rq.coll), int(rq.algo), rq.p, (unsigned long long)rq.count, rq.unit);
+            return 1;
+        }
+        // several sets of buffers: near one another, at odd addresses, and, now and then, too far apart for 32 bits
+        for (int set = 0; set < 3; set++) {
+            const uint64_t align[] = {512, 1, 4096, 2, 16, 256};
+            const uint64_t grain = align[Below(6)], reach = set == 2 ? uint64_t(1) << (33 + Below(13)) : uint64_t(1) << (24 + Below(8));
+            std::vector<void *> send(rq.p), recv(rq.p);
+            for (uint32_t r = 0; r < rq.p; r++) {
+                send[r] = reinterpret_cast<void *>(0x7f0000000000ull + Below(reach) / grain * grain);
+                recv[r] = same ? send[r] : reinterpret_cast<void *>(0x7f0000000000ull + Below(reach) / grain * grain);
+            }
+            const bool hit = FillBases(&d, send, recv);
+            if (hit && set == 0) {
+                std::printf("a first call's buffers counted as seen\n");
+                return 1;
+            }
+            if (!d.usePacked) {
+                apart += d.packedFunc != nullptr;
+                if (d.packedFunc != nullptr && set < 2) {
+                    std::printf("buffers within 2 GiB not taken\n");
+                    return 1;
+                }
+                continue;
+            }
+            const bool ok = d.packedRanks == 8 ? Same<8>(plan, d, send, recv) : d.packedRanks == 16 ? Same<16>(plan, d, send, recv) : Same<32>(plan, d, send, recv);
+            if (!ok || rq.p > d.packedRanks) {
+                std::printf("coll %d algo %d p %u servers %u count %llu unit %u: the arguments are not the plan's items\n", int(rq.coll), int(rq.algo), rq.p,
+                    rq.servers, (unsigned long long)rq.count, rq.unit);
+                return 1;
+            }
+            inPlace += same;
+        }
+        unlike += d.packedFunc == nullptr;
+        trees += d.packedFunc != nullptr && plan.fused[0].kind == FK_TREE;
+        if (d.packedFunc != nullptr) {
+            taken[d.packedRanks == 8 ? 0 : d.packedRanks == 16 ? 1 : 2]++;
+        }
+    }
+    std::printf("OK up to 8 ranks %ld 16 ranks %ld 32 ranks %ld trees %ld in place %ld unlike %ld too far apart %ld\n", taken[0], taken[1], taken[2], trees,
+        inPlace, unlike, apart);
+    return 0;
+}

@@ -1,0 +1,74 @@
+"""Small collectives with packed arguments (a wave per KiB of an item), against the CPU checker bit for bit: every shape that has a kernel of
+its own (2, 4, 8, 16 sources; chains of either operand order, trees), other numbers of sources, the edges of a wave's KiB and of a
+vector, in place, off a boundary, up to and beyond the sizes where the tile kernels take over."""
+import numpy as np
+import pytest
+
+import closed_forms as cf
+import gpu_harness as gh
+from closed_forms import BF16, FP16, FP32, INT8, INT64, MAX, MIN, PROD, SUM
+
+pytestmark = pytest.mark.gpu
+RING, MESH, RHD = 0, 4, 2      # (4: the mesh without the piece cut, which these types and operations run)
+MIB = 1 << 20
+LIMIT = {2: 32 * MIB, 3: 7 * MIB // 2, 4: 7 * MIB // 2, 8: 9 * MIB // 4}     # of an all-reduce; more ranks: 1.5 MiB
+
+
+def _ins(dt, p, n, seed, special):
+    rng = np.random.default_rng(seed)
+    ins = [cf.random_input(dt, n, rng) for _ in range(p)]
+    if special:
+        odd = np.array([np.nan, 0.0, -0.0, np.inf, -np.inf, 1.0], np.float32)
+        for x in ins:
+            at = rng.random(n) < 0.5
+            x[at] = cf.narrow(dt, odd[rng.integers(0, odd.size, int(at.sum()))])
+    return ins
+
+
+@pytest.mark.parametrize("p,algo", [(2, RING), (3, RING), (4, RING), (4, MESH), (4, RHD), (7, MESH), (8, RING), (8, MESH), (8, RHD), (11, RING), (16, RING),
+                                    (16, MESH), (16, RHD), (24, RING), (32, MESH), (32, RHD)])
+def test_all_reduce(orc, p, algo):
+    g = gh.Group(p, algo={RING: "ring", MESH: "mesh", RHD: "rhd"}[algo])
+    try:
+        for k, (dt, op, pad, in_place, special) in enumerate([(FP32, SUM, 0, False, False), (BF16, MAX, 2, True, True), (FP16, MIN, 6, False, True), (INT8, SUM, 1, True, False)]):
+            unit = gh.H.DTYPE_SIZE[dt]
+            sizes = {1, 1024 * p // unit, 1024 * p // unit + 1, (2048 * p - 128) // unit - 1, 8 * 1024 * p // unit + 3}
+            if k % 2 == (algo == RING):
+                limit = min(LIMIT.get(p, 3 * MIB // 2), 4 * MIB)
+                sizes |= {limit // unit - 1, limit // unit, limit // unit + 1}
+            for n in sorted(sizes):
+                print("packed all-reduce", p, algo, "type", dt, "op", op, "n", n, flush=True)
+                ins = _ins(dt, p, n, 13 * p + n % 1013 + k, special)
+                want = orc.allreduce(ins, dt, op, algo=algo)
+                outs, keep = gh.all_reduce(g, ins, dt, op, in_place=in_place, pad=pad)
+                assert g.info()["launches"] == 1 and g.info()["fused"] == 1
+                assert g.info()["direct"] == int(n * unit <= MIB)
+                for r in range(p):
+                    assert gh.same(dt, outs[r], want[r]), (dt, op, n, r)
+                    assert keep is None or np.array_equal(keep[r].view(np.uint8), ins[r].view(np.uint8))
+    finally:
+        g.close()
+
+
+@pytest.mark.parametrize("p", [2, 4, 5, 8, 16])
+def test_blocks(orc, p):
+    g = gh.Group(p)
+    limit = {2: 14 * MIB, 4: 6 * MIB}.get(p, 9 * MIB // 2)
+    try:
+        for dt, op, pad in ((INT8, PROD, 1), (BF16, SUM, 2), (FP32, MIN, 0), (INT64, SUM, 8)):
+            unit = gh.H.DTYPE_SIZE[dt]
+            even = limit // p // unit // 16 * 16
+            for n in (1, 1024 // unit, 1024 // unit + 1, 3 * 1024 // unit - 1) + ((even, even + 16) if dt in (BF16, FP32) else (7 * MIB // 2 // p // unit // 16 * 16 - 1,)):
+                print("packed blocks", p, "type", dt, "n", n, flush=True)
+                ins = _ins(dt, p, n * p, 71 * p + n, False)
+                want = orc.reducescatter(ins, dt, op)
+                outs, _ = gh.reduce_scatter(g, ins, dt, op, pad=pad)
+                for r in range(p):
+                    assert gh.same(dt, outs[r], want[r]), ("reduce-scatter", dt, n, r)
+                if n < 5000:
+                    parts = [x[:n] for x in ins]
+                    outs = gh.all_gather(g, parts, dt, pad=pad)
+                    for r in range(p):
+                        assert np.array_equal(outs[r].view(np.uint8), np.concatenate(parts).view(np.uint8)), ("all-gather", dt, n, r)
+    finally:
+        g.close()

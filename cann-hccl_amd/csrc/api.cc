@@ -410,19 +410,21 @@ HcclResult HcclAlltoAllV(const void *sendBuf, const void *sendCounts, const void
     }
     const uint64_t *sc = static_cast<const uint64_t *>(sendCounts);
     const uint64_t *rc = static_cast<const uint64_t *>(recvCounts);
-    bool hasSend = false, hasRecv = false;
+    // (the largest count is all ones: no branch per entry, of which a call of 64 ranks has 8192)
+    static_assert((kSysMaxCount & (kSysMaxCount + 1)) == 0, "one bit beyond it is enough");
+    uint64_t sent = 0, received = 0;
     for (uint32_t i = 0; i < p; i++) {
-        if (sc[i] > kSysMaxCount || rc[i] > kSysMaxCount) {
-            HCCL_LOG_ERROR("HcclAlltoAllV: a count exceeds the maximum");
-            return HCCL_E_PARA;
-        }
-        hasSend = hasSend || sc[i] != 0;
-        hasRecv = hasRecv || rc[i] != 0;
+        sent |= sc[i];
+        received |= rc[i];
     }
-    if (hasSend) {
+    if ((sent | received) > kSysMaxCount) {
+        HCCL_LOG_ERROR("HcclAlltoAllV: a count exceeds the maximum");
+        return HCCL_E_PARA;
+    }
+    if (sent != 0) {
         CHK_PTR(sendBuf);
     }
-    if (hasRecv) {
+    if (received != 0) {
         CHK_PTR(recvBuf);
     }
     HcclResult r = CheckOpParam("HcclAlltoAllV", 0, sendType, stream);

@@ -347,6 +347,15 @@ HcclResult Arrive(Comm *c, const OpSig &sig, void *send, void *recv, hipStream_t
         }
     }
     if (sig.coll == COLL_ALLTOALLV) {
+        const uint64_t *rows[4] = {sendCounts, sdispls, recvCounts, rdispls};
+        if (g->arrived == 0) {
+            A2avBegin(g, ElemSize(sig.dtype));
+        }
+        if (g->a2avOpen && !A2avRow(g, r, send, recv, rows)) {
+            A2avExpand(g, r);
+        }
+    }
+    if (sig.coll == COLL_ALLTOALLV && !g->a2avOpen) {
         // The tables stay from call to call.  A row that is what this rank passed the last time is compared and not copied, and
         // if every rank's rows are, what was found out about the tables (checked, prepared) holds: a repeated call of 64 ranks then
         // reads its 128 KiB once, instead of copying, checking, hashing and comparing them.
@@ -395,7 +404,15 @@ HcclResult Arrive(Comm *c, const OpSig &sig, void *send, void *recv, hipStream_t
     }
     // last arrival
     HcclResult res = HCCL_SUCCESS;
-    if (sig.coll == COLL_ALLTOALLV && !g->tablesChecked) {
+    g->a2avReady = nullptr;
+    if (sig.coll == COLL_ALLTOALLV && g->a2avOpen) {
+        g->ctx = &g->pend;
+        res = A2avFinish(g, stream, &g->a2avReady);
+        if (res == HCCL_SUCCESS && g->a2avReady == nullptr) {
+            A2avExpand(g, g->p);
+        }
+    }
+    if (sig.coll == COLL_ALLTOALLV && res == HCCL_SUCCESS && g->a2avReady == nullptr && !g->tablesChecked) {
         // alltoall_operator.cc:49-72: what i sends to j must be what j expects from i
         // (block by block: one of the two tables is walked across its rows)
         constexpr uint32_t kBlock = 8;

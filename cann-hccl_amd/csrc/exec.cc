@@ -1046,6 +1046,8 @@ PlanRequest MakeRequest(const Group *g, int algo)
 
 bool ReduceColl(int coll) { return coll == COLL_ALLREDUCE || coll == COLL_REDUCESCATTER || coll == COLL_REDUCE; }
 
+}  // namespace
+
 // Buffers of different ranks must not overlap where one of them is written (HCCL_E_PARA); a send buffer that
 // overlaps a receive buffer other than as an exact in-place pair is staged through scratch (*needStage).
 // An all-gather in place -- rank r sends its own block of its receive buffer -- is none of that for the fused form, in
@@ -1106,6 +1108,8 @@ HcclResult CheckOverlap(const Group *g, const std::vector<uint64_t> &sendBytes, 
     }
     return HCCL_SUCCESS;
 }
+
+namespace {
 
 OpInfo MakeInfo(const Group *g, int algo, const Plan &plan, bool fused)
 {
@@ -1361,6 +1365,9 @@ Group::~Group()
     if (barrierMem) {
         (void)hipFree(barrierMem);
     }
+    if (a2avTables) {
+        (void)hipFree(a2avTables);
+    }
 }
 
 const char *CollName(int coll)
@@ -1408,7 +1415,8 @@ HcclResult IssueCollective(Group *g, uint32_t launcher)
         (g->ctx->sig.coll == COLL_ALLREDUCE || g->ctx->sig.coll == COLL_REDUCESCATTER || g->ctx->sig.coll == COLL_REDUCE)) {
         algo = ALGO_MESH_ATOMIC;
     }
-    DirectLaunch *direct = FindDirect(g, algo);
+    A2avSet *a2av = g->ctx == &g->pend && g->ctx->sig.coll == COLL_ALLTOALLV ? g->a2avReady : nullptr;
+    DirectLaunch *direct = a2av != nullptr ? nullptr : FindDirect(g, algo);
     Prepared *pp = nullptr;
     std::unique_ptr<Prepared> uncached;   // the collective of a call that allocates nothing: built, launched, dropped
     bool hit = false;
@@ -1427,7 +1435,7 @@ HcclResult IssueCollective(Group *g, uint32_t launcher)
         }
         pp = uncached.get();
     }
-    bool looked = pp != nullptr || direct != nullptr;
+    bool looked = pp != nullptr || direct != nullptr || a2av != nullptr;
     std::string &key = g->keyBuffer;      // (kept: 128 KiB at 64 ranks, which malloc would map and unmap on every call)
     if (!looked) {
         CacheKey(g, algo, &key);
@@ -1498,7 +1506,7 @@ HcclResult IssueCollective(Group *g, uint32_t launcher)
         pp = fresh.get();
         g->cache[key] = std::move(fresh);
     }
-    if (!shortKey.empty()) {
+    if (!shortKey.empty() && pp != nullptr) {
         g->lastA2av = pp;
         g->lastA2avKey.swap(shortKey);
     }
@@ -1506,6 +1514,16 @@ HcclResult IssueCollective(Group *g, uint32_t launcher)
     bool viaGraph = false;
     if (direct != nullptr) {
         g->lastInfo = direct->info;
+    } else if (a2av != nullptr) {
+        OpInfo info;
+        info.coll = COLL_ALLTOALLV;
+        info.algo = algo;
+        info.fused = 1;
+        info.cacheHit = a2av->hit ? 1 : 0;
+        info.launches = a2av->launches;
+        info.bytesRead = info.bytesWritten = a2av->moved;
+        info.stepRead = info.stepWritten = a2av->moved * (g->cfg.servers > 1 && g->cfg.algo != ALGO_PAIRWISE ? 2 : 1);   // (staged: every byte twice)
+        g->lastInfo = info;
     } else {
         HcclResult ready = ReadyToLaunch(g, pp, ls, hit, &viaGraph);
         if (ready != HCCL_SUCCESS) {
@@ -1541,6 +1559,11 @@ HcclResult IssueCollective(Group *g, uint32_t launcher)
         void *args[1] = {direct->usePacked ? direct->packed.data() : direct->image.data()};
         HIP_OK(hipLaunchKernel(direct->usePacked ? direct->packedFunc : direct->func,
             dim3(direct->usePacked ? direct->packedGridX : direct->gridX, direct->gridY, 1), dim3(kDirectThreads, 1, 1), args, 0, ls));
+    } else if (a2av != nullptr) {
+        HcclResult launched = A2avLaunch(g, a2av, ls);
+        if (launched != HCCL_SUCCESS) {
+            return launched;
+        }
     } else if (viaGraph) {
         HIP_OK(hipGraphLaunch(pp->exec, ls));
     } else {

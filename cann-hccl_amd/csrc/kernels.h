@@ -78,6 +78,28 @@ struct SegDesc {
 };
 constexpr uint32_t kGatherMaxBytes = 8192;
 
+// An all-to-all-v as its callers describe it (kernels_a2av.h): up to P ranks, counts and displacements in elements.
+template <uint32_t P> struct A2avTable {
+    uint64_t send[P], recv[P];
+    uint32_t rowStart[P];      // first piece of receiver j's blocks; behind the last receiver the number of pieces
+    uint32_t count[P * P];     // [receiver][sender]
+    uint32_t to[P * P];        // [receiver][sender]: displacement in the receive buffer
+    uint32_t from[P * P];      // [receiver][sender]: displacement in the send buffer
+};
+// A block goes in pieces of (1 << shift) bytes, counted from the memory line of 128 bytes that its place in the receive buffer begins
+// in; the pieces are numbered receiver by receiver, sender by sender.  A launch takes pieces [first, end).
+struct A2avRange {
+    uint32_t first, end;
+    uint32_t unitShift, shift;
+};
+template <uint32_t P> struct A2avArgs {
+    A2avTable<P> table;
+    A2avRange range;
+};
+static_assert(sizeof(A2avArgs<16>) <= 4096, "kernel arguments");
+constexpr uint32_t kA2avLine = 128;
+constexpr uint32_t kA2avShift = 12;      // pieces of 4 KiB, four vectors per lane
+
 enum KernelKind : int {
     KK_STEP = 0, KK_CHAIN = 1, KK_TREE = 2, KK_STACK = 3,
     KK_TEAM_CHAIN = 4, KK_TEAM_TREE = 5, KK_TEAM_STACK = 6,   // team forms of the fused kernels, see below
@@ -90,7 +112,9 @@ enum KernelKind : int {
     KK_PACKED_RING = 18,                                       // chains whose sources behind the second one are the left operands,
     KK_PACKED_TREE = 22,                                       // trees
     KK_COUNT = 26,
-    KK_GATHER = 26                                             // copy kernel table only
+    KK_GATHER = 26,                                            // copy kernel table only, like these:
+    KK_A2AV = 27                                               // all-to-all-v from the callers' tables, of 8, 16, 32, 64 ranks: workgroups of
+                                                               // one wave (kinds 27 ... 30), of four (31 ... 34)
 };
 constexpr uint32_t kPackedShapes = 4;
 // Index of a number of sources among those that have a kernel of their own, kPackedShapes where it has none.
@@ -193,6 +217,8 @@ constexpr uint32_t kPackedRing = 1u << 27;      // chain: sources behind the sec
 const void *LookupKernel(int hcclDataType, int hcclReduceOp, KernelKind kind);
 
 //   KK_GATHER          (const SegDesc *segs, uint32_t nsegs)
+//                      copy kernel table only
+//   KK_A2AV            up to 16 ranks (A2avArgs<P>), else (const A2avTable<P> *table, A2avRange); any number of workgroups
 //                      copy kernel table only
 // Byte-wise variants for pure data movement (all-gather, all-to-all-v): KK_STEP, KK_CHAIN, KK_TEAM_CHAIN, KK_GATHER,
 // KK_DIRECT, KK_DIRECT_WIDE and KK_PACKED_n.

@@ -1,5 +1,6 @@
 // Instantiates the kernels for one HcclDataType (selected with -DHCCL_DT=<enum value>), so that the
 // twelve element types build in parallel, plus the byte-wise copy variants (-DHCCL_DT=255).
+#include "kernels_a2av.h"
 #include "kernels_direct.h"
 #include "kernels_team.h"
 
@@ -53,7 +54,7 @@ using DT = uint8_t;
 
 #if HCCL_DT == 255
 // pure data movement: the step kernel's copy path and the copy kernel
-extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[9] = {
+extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[17] = {
     reinterpret_cast<const void *>(&StepKernel<DT, ROP_SUM>),
     reinterpret_cast<const void *>(&CopyKernel<0>),
     reinterpret_cast<const void *>(&GatherKernel<0>),
@@ -63,6 +64,14 @@ extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[9] = {
     reinterpret_cast<const void *>(&PackedCopyKernel<8>),
     reinterpret_cast<const void *>(&PackedCopyKernel<16>),
     reinterpret_cast<const void *>(&PackedCopyKernel<32>),
+    reinterpret_cast<const void *>(&A2avArgsKernel<8, 64, STORE_THROUGH>),
+    reinterpret_cast<const void *>(&A2avArgsKernel<16, 64, STORE_THROUGH>),
+    reinterpret_cast<const void *>(&A2avTableKernel<32, 64, STORE_THROUGH>),
+    reinterpret_cast<const void *>(&A2avTableKernel<64, 64, STORE_THROUGH>),
+    reinterpret_cast<const void *>(&A2avArgsKernel<8, kBlockThreads, STORE_NT>),
+    reinterpret_cast<const void *>(&A2avArgsKernel<16, kBlockThreads, STORE_NT>),
+    reinterpret_cast<const void *>(&A2avTableKernel<32, kBlockThreads, STORE_NT>),
+    reinterpret_cast<const void *>(&A2avTableKernel<64, kBlockThreads, STORE_NT>),
 };
 #else
 #define HCCL_SHAPES(OP, SHAPE)                                                                                                   \

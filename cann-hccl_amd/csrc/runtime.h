@@ -232,6 +232,22 @@ struct StageSlot {
     bool used = false;
 };
 
+// An all-to-all-v as its ranks called it, in the form that the device takes it (a2av.cc).
+constexpr uint32_t kA2avSets = 8;
+struct A2avSet {
+    bool valid = false;               // a call that was issued: what follows belongs together
+    bool hit = false;                 // the call under way is this one
+    std::vector<uint8_t> image;       // an A2avTable; up to 16 ranks an A2avArgs
+    std::vector<uint32_t> sent, place;   // [sender][receiver]: the senders' counts and displacements (the image holds the receivers' counts)
+    std::vector<uint64_t> sendBytes, recvBytes;
+    uint64_t lastUse = 0;
+    uint64_t moved = 0;
+    uint32_t unitShift = 0, pieces = 0, launches = 0;
+    uint32_t width = 0;               // workgroups of four waves per CU, results non-temporal; 0: of one wave, written through
+    void *table = nullptr;            // more than 16 ranks: the image in device memory, written and read on `stream` alone
+    hipStream_t stream = nullptr;
+};
+
 struct Group;
 
 struct Comm {
@@ -265,6 +281,15 @@ struct Group {
     bool tablesChecked = false;      // pend's all-to-all-v tables, as they are now, were found consistent
     Prepared *lastA2av = nullptr;    // the prepared collective of pend's tables as they are now (in `cache`), if lastA2avKey ...
     std::string lastA2avKey;         // ... matches the rest of the key: request, settings, buffers
+    // the all-to-all-v whose ranks are arriving
+    bool a2avOpen = false;           // its rows are taken over as they come (else they go to pend's tables)
+    uint32_t a2avAlive = 0;          // the sets that agree with every row so far, a bit each
+    int a2avBuilding = -1;           // the set it is written down in, as soon as it agrees with none
+    uint32_t a2avUnit = 0;
+    uint64_t a2avClock = 0;
+    std::vector<A2avSet> a2avSets;   // the latest calls, kA2avSets of them
+    void *a2avTables = nullptr;      // their tables in device memory (more than 16 ranks)
+    A2avSet *a2avReady = nullptr;    // complete and checked, for IssueCollective
     OpCtx *ctx = nullptr;            // the operation being issued (the rendezvous, or a matched send / receive)
     std::map<std::pair<uint32_t, uint32_t>, std::deque<P2PPending>> p2p;
 
@@ -301,6 +326,20 @@ struct Group {
 
 // Creates the group's events on first use of the device.  HCCL_E_RUNTIME when there is no GPU.
 HcclResult EnsureDevice(Group *g, bool quiet);
+
+// All-to-all-v from the callers' tables.  The first rank to arrive: whether this call goes that way as far as the settings tell.
+void A2avBegin(Group *g, uint32_t unit);
+// A rank's rows (send counts, send displacements, receive counts, receive displacements); false: a value of 2^32 or more.
+bool A2avRow(Group *g, uint32_t r, void *send, void *recv, const uint64_t *const rows[4]);
+// The rows of the ranks that have arrived, but for `except`, into pend's tables: the call goes the general way.
+void A2avExpand(Group *g, uint32_t except);
+// The last rank has arrived.  *ready: what to launch, nullptr where the call goes the general way.
+HcclResult A2avFinish(Group *g, hipStream_t stream, A2avSet **ready);
+HcclResult A2avLaunch(Group *g, A2avSet *s, hipStream_t stream);
+
+// Whether the ranks' buffers may share memory as they do (exec.cc).
+HcclResult CheckOverlap(const Group *g, const std::vector<uint64_t> &sendBytes, const std::vector<uint64_t> &recvBytes, bool *needStage,
+    bool *gatherInPlace);
 
 // Called with the group mutex held, by the last rank to arrive.
 HcclResult IssueCollective(Group *g, uint32_t launcherRank);

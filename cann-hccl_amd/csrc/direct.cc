@@ -136,21 +136,49 @@ bool DirectFits(int coll, uint32_t p, uint64_t bytes, int dtype)
     }
 }
 
-// Beyond those limits, where the items are alike (PackDirect): a wave per KiB keeps every CU equally busy when there are few tiles of
-// 16 KiB, or tiles of few sources and destinations.  Three sets of buffers in turn, us, tile kernels / packed:
-//   all-reduce, fp32: 2 ranks 4 MiB 4.7 / 3.5, 16 MiB 12.6 / 11.9, 32 MiB 23.2 / 21.1, 64 MiB 44.3 / 43.7; 4 ranks 2 MiB 4.9 / 3.7, 3 MiB 5.6 / 4.6, 4 MiB
-//     6.0 / 6.5; 8 ranks 1.5 MiB 6.5 / 4.6, 2 MiB 7.2 / 6.0, 2.25 MiB 7.4 / 6.7, 2.5 MiB 7.6 / 7.7; 16 ranks 1.25 MiB 10.4 / 7.7, 1.5 MiB 11.0 / 9.6,
-//     2 MiB 12.6 / 14.9; 32 ranks 1.25 MiB 20 / 14, 1.5 MiB 21.3 / 17.7; bf16 and int8 alike
-//   reduce-scatter (bytes received by all ranks), fp32: 2 ranks 6 MiB 4.5 / 3.9, 12 MiB 7.2 / 6.4, 16 MiB 9.0 / 9.0; 4 ranks 4 MiB 5.0 / 4.3, 6 MiB 6.4 / 5.9, 8 MiB
-//     7.4 / 7.5; 8 ranks 3 MiB 6.3 / 5.4, 4 MiB 7.4 / 7.0, 6 MiB 10.1 / 9.9; 16 ranks 2.5 MiB 9.1 / 8.4, 3 MiB 9.8 / 10.0
-bool PackedFits(int coll, uint32_t p, uint64_t bytes)
+// Beyond those limits, where the items are alike (PackDirect): waves of 1 or 4 KiB keep every CU equally busy where the tile kernels' tiles of
+// 16 KiB do not, that is where there are few of them, or a few more than one (4 MiB) or two (8 MiB) for each CU: a CU takes some 4 us for a tile
+// that is read from 8 buffers and stored to 8.  Three sets of buffers in turn, us, tile kernels / packed with KiB / packed with 4 KiB:
+//   all-reduce, 2 ranks: 4 MiB 4.5 / 3.6 / 3.6, 6 MiB 5.7 / 5.1 / 4.5, 8 MiB 6.0 / 6.0 / 5.8, 24 MiB 18.0 / 16.6 / 17.1, 48 MiB 33.8 / 31.9 / 33.5
+//     4 ranks: 3 MiB 5.2 / 4.5 / 4.6, 4.25 MiB 8.0 / 6.9 / 6.0, 6 MiB 8.7 / 9.4 / 7.6, 7 MiB 9.5 / 10.4 / 9.8, 8 MiB 10.6 / 12.2 / 12.0, 9 MiB
+//       14.1 / 13.9 / 13.8, 14 MiB 21.7 / 19.9 / 20.1, 24 MiB 35.9 / 32.1 / 31.6, 28 MiB 40.7 / 41.1 / 40.9
+//     8 ranks: 1.5 MiB 6.4 / 4.6 / 5.5, 2 MiB 7.0 / 6.0 / 6.1, 2.5 MiB 7.5 / 7.7 / 7.0, 3 MiB 8.3 / 9.7 / 7.8 (bf16 maximum 8.6 / - / 9.5), 4 MiB 10.7 / 12.5 / 10.5,
+//       4.25 MiB 14.3 / 13.2 / 11.5, 5 MiB 15.8 / 15.1 / 12.8, 6 MiB 16.7 / 17.6 / 16.5, 8 MiB 21.1 / 22.4 / 22.0, 8.5 MiB 26.4 / 24.2 / 24.5, 12 MiB
+//       34.7 / 33.7 / 33.2, 14 MiB 41.7 / 44.0 / 42.8
+//     16 ranks: 1.5 MiB 11.0 / 9.5 / 10.2, 2 MiB 12.3 / 13.3 / 11.1, 3 MiB 16.0 / 18.1 / 15.6 (bf16 17.5 / - / 17.7), 4.25 MiB 27.7 / 24.6 / 22.9, 5 MiB
+//       29.6 / 27.5 / 25.7, 6 MiB 33.3 / 35.3 / 31.2 (fp16, bf16 up to 33), 8.5 MiB 54.5 / 57.3 / 53.1; 32 ranks 1.5 MiB 21.3 / 17.7 / -
+//   reduce-scatter (bytes received by all ranks), blocks of whole vectors: 2 ranks 6 MiB 4.5 / 4.0, 14 MiB 8.5 / 7.9, 16 MiB 9.1 / 9.0, 20 MiB 11.7 / 11.1, 64 MiB
+//     32.2 / 30.1; 4 ranks 5 MiB 6.1 / 5.1, 7 MiB 7.0 / 6.6, 8 MiB 7.6 / 7.7, 9 MiB 9.8 / 8.1, 11 MiB 10.5 / 10.2, 12 MiB 11.0 / 11.4; 8 ranks 3 MiB
+//     6.3 / 5.3, 4 MiB 7.3 / 7.0, 5 MiB 9.4 / 8.2, 6 MiB 10.1 / 9.7, 7 MiB 11.2 / 10.9, 8 MiB 12.1 / 13.5; 16 ranks 1 MiB 7.7 / 5.1, 2 MiB 8.6 / 8.3 (bf16
+//     10.1 / 8.4), 3 MiB 9.8 / 9.7, 4.25 MiB 15.5 / 13.5, 5 MiB 16.4 / 15.3, 6 MiB 17.8 / 20.4
+//   other blocks: 2 ranks 14 MiB 8.9 / 8.8, 4 ranks 6 MiB 6.9 / 6.8, 8 ranks 3 MiB 6.7 / 5.9, 4 MiB 8.5 / 7.8, 5 MiB 9.8 / 9.0, 16 ranks 2 MiB 9.2 / 7.9,
+//     3 MiB 10.3 / 10.7.  Waves of 4 KiB bring nothing where every block has one destination (8 ranks bf16 pairwise, 4 MiB 6.9 / 7.7).
+// Two kinds of calls gain less and stay out: 16 ranks' all-reduce of a 16-bit floating-point type from 1.5 MiB, whose waves of 4 KiB wait for their own
+// arithmetic (1.75 MiB bf16 sum 12.4 / 12.1, fp16 minimum of the uncut mesh 12.2 / 16.1), and bytes off a vector boundary (8 ranks 4.75 MiB 9.3 / 10.1).
+bool PackedFits(int coll, uint32_t p, uint64_t bytes, int dtype)
 {
     constexpr uint64_t kQuarter = uint64_t(1) << 18;      // of a MiB
+    if (p < 2 || p > 32) {
+        return false;
+    }
+    const bool shaped = PackedShape(p) < kPackedShapes, bytesOnly = dtype == HCCL_DATA_TYPE_INT8 || dtype == HCCL_DATA_TYPE_UINT8;
+    auto within = [](uint64_t total, uint64_t above, uint64_t upTo) { return total > above * kQuarter && total <= upTo * kQuarter; };
     if (coll == COLL_ALLREDUCE) {
-        return p > 1 && p <= 32 && bytes <= (p == 2 ? 128 : p <= 4 ? 14 : p <= 8 ? 9 : 6) * kQuarter;
+        if (!shaped) {
+            return bytes <= (p <= 4 ? 14 : p <= 8 ? 9 : 6) * kQuarter;
+        }
+        const bool busy = p == 16 && (dtype == HCCL_DATA_TYPE_FP16 || dtype == HCCL_DATA_TYPE_BFP16);
+        return p == 2 ? bytes <= 192 * kQuarter : p == 4 ? bytes <= 24 * kQuarter || within(bytes, 32, 96) :
+            bytes <= (busy ? 6 : 11) * kQuarter || within(bytes, 16, 22) || (p == 8 && within(bytes, 32, 48));
     }
     if (coll == COLL_REDUCESCATTER) {
-        return p > 1 && p <= 8 && bytes * p <= (p == 2 ? 56 : p <= 4 ? 24 : bytes % 16 == 0 ? 18 : 14) * kQuarter;
+        const uint64_t total = bytes * p;
+        if (bytes % 16 == 0) {
+            return p == 2 ? total <= 60 * kQuarter || within(total, 64, 256) : p <= 4 ? total <= (shaped ? 30 : 24) * kQuarter || (shaped && within(total, 32, 44)) :
+                p <= 8 ? total <= (shaped ? 24 : 18) * kQuarter : p == 16 && (total <= 11 * kQuarter || within(total, 16, 20));
+        }
+        return p == 2 ? total <= 56 * kQuarter : p <= 4 ? total <= 24 * kQuarter : p <= 8 ? total <= 14 * kQuarter || (p == 8 && !bytesOnly && within(total, 16, 20)) :
+            p == 16 && total <= 10 * kQuarter;
     }
     return false;
 }
@@ -314,11 +342,20 @@ void PackDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaun
         FillPacked<32>(plan, order, info, d);
         kind = KK_PACKED_32;
     }
+    uint64_t total = 0;
+    for (const FusedItem &it : plan.fused) {
+        total += it.bytes;
+    }
     const uint32_t shape = PackedShape(uint32_t(order.size()));
+    bool wide = false;
     if (reduceColl && shape < kPackedShapes && order.size() == p) {       // (of two sources, added and exclusive-ored are the same)
         kind = KernelKind((tree ? KK_PACKED_TREE : (left ? KK_PACKED_CHAIN : KK_PACKED_RING)) + shape);
+        // waves of 4 KiB where PackedFits' figures say so
+        wide = !toOne && total > (p <= 8 ? kPackedNarrowBytes : kPackedNarrowBytes / 4 * 3) && total <= 4 * kPackedNarrowBytes;
     }
-    d->packedGridX = uint32_t(longest / kDirectChunk + (longest % kDirectChunk >= 16 ? 1 : 0)) + (ends ? 1u : 0u);
+    const uint32_t chunk = wide ? kPackedWideChunk : kDirectChunk;
+    kind = wide ? KernelKind(kind + KK_PACKED_WIDE) : kind;
+    d->packedGridX = uint32_t(longest / chunk + (longest % chunk >= 16 ? 1 : 0)) + (ends ? 1u : 0u);
     d->packedFunc = reduceColl ? LookupKernel(dtype, op, kind) : LookupCopyKernel(kind);
 }
 

@@ -1259,7 +1259,7 @@ DirectLaunch *FindDirect(Group *g, int algo)
     }
     const uint64_t bytes = sig.count * DtypeSize(sig.dtype);
     const bool small = DirectFits(sig.coll, g->p, bytes, sig.dtype);
-    if (!small && !PackedFits(sig.coll, g->p, bytes)) {
+    if (!small && !PackedFits(sig.coll, g->p, bytes, sig.dtype)) {
         return nullptr;
     }
     uint64_t inPlace = 0;

@@ -110,11 +110,12 @@ enum KernelKind : int {
     KK_PACKED_CHAIN = 14,                                      // the same for 2, 4, 8, 16 sources (kinds 14 ... 17): chains whose sources
                                                                // are the right operands,
     KK_PACKED_RING = 18,                                       // chains whose sources behind the second one are the left operands,
-    KK_PACKED_TREE = 22,                                       // trees
-    KK_COUNT = 26,
-    KK_GATHER = 26,                                            // copy kernel table only, like these:
-    KK_A2AV = 27                                               // all-to-all-v from the callers' tables, of 8, 16, 32, 64 ranks: workgroups of
-                                                               // one wave (kinds 27 ... 30), of four (31 ... 34)
+    KK_PACKED_TREE = 22,                                       // trees;
+    KK_PACKED_WIDE = 12,                                       // added to one of the last 12 kinds: four vectors per lane
+    KK_COUNT = 38,
+    KK_GATHER = 38,                                            // copy kernel table only, like these:
+    KK_A2AV = 39                                               // all-to-all-v from the callers' tables, of 8, 16, 32, 64 ranks: workgroups of
+                                                               // one wave (kinds 39 ... 42), of four (43 ... 46)
 };
 constexpr uint32_t kPackedShapes = 4;
 // Index of a number of sources among those that have a kernel of their own, kPackedShapes where it has none.
@@ -149,7 +150,9 @@ inline uint32_t TeamBlockWords(uint32_t nregions) { return kTeamHeaderWords + 2u
 // Small collectives (kernels_direct.h): the whole description of a launch rides in its kernel arguments.  All sources of
 // an item lie at the same offset of their buffers and all destinations at the same offset of theirs.
 constexpr uint32_t kDirectThreads = 64;                  // a workgroup is one wave,
-constexpr uint32_t kDirectChunk = kDirectThreads * 16;   // of an item it takes these bytes
+constexpr uint32_t kDirectChunk = kDirectThreads * 16;   // of an item it takes these bytes,
+constexpr uint32_t kPackedWideChunk = 4 * kDirectChunk;  // or these
+constexpr uint64_t kPackedNarrowBytes = uint64_t(2) << 20;   // (collectives beyond these, direct.cc)
 enum DirectKind : uint32_t { DIRECT_CHAIN = 0, DIRECT_TREE = 1, DIRECT_STACK = 2 };
 
 // CAP = 8: up to 8 sources and destinations per item; CAP = 32: up to 32 (no stack programs).
@@ -210,7 +213,7 @@ constexpr uint32_t kPackedRing = 1u << 27;      // chain: sources behind the sec
 //                      Up to seven pointers behind an item's list of sources may be read (and are not used): the destinations'
 //                      pool lies behind the sources', and the tables end on a multiple of 256 bytes.
 //   KK_TEAM_*          the same and (uint32_t *teamBlock)
-//   KK_PACKED_n        (PackedArgs<n>; those of 2, 4 and 8 sources PackedArgs<8>, of 16 PackedArgs<16>), grid (chunks of the longest item, items), with kPackedEnds one more in x, the first one, for the bytes
+//   KK_PACKED_n        (PackedArgs<n>; those of 2, 4 and 8 sources PackedArgs<8>, of 16 PackedArgs<16>), grid (chunks of the longest item's whole vectors, items), with kPackedEnds one more in x, the first one, for the bytes
 //                      behind an item's last whole vector
 //   KK_DIRECT / KK_DIRECT_WIDE   (DirectArgs<8> / DirectArgs<32>), grid (1 + chunks of the longest item, items): blockIdx.x == 0
 //                      is for the bytes behind an item's last whole vector

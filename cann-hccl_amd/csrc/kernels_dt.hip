@@ -74,11 +74,14 @@ extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[17] = {
     reinterpret_cast<const void *>(&A2avTableKernel<64, kBlockThreads, STORE_NT>),
 };
 #else
-#define HCCL_SHAPES(OP, SHAPE)                                                                                                   \
-    reinterpret_cast<const void *>(&PackedShapeKernel<DT, OP, 8, 2, SHAPE == PACKED_LEFT ? SHAPE : PACKED_LEFT>),                 \
-        reinterpret_cast<const void *>(&PackedShapeKernel<DT, OP, 8, 4, SHAPE>),                                                  \
-        reinterpret_cast<const void *>(&PackedShapeKernel<DT, OP, 8, 8, SHAPE>),                                                  \
-        reinterpret_cast<const void *>(&PackedShapeKernel<DT, OP, 16, 16, SHAPE>)
+#define HCCL_SHAPES(KERNEL, OP, SHAPE)                                                                                           \
+    reinterpret_cast<const void *>(&KERNEL<DT, OP, 8, 2, SHAPE == PACKED_LEFT ? SHAPE : PACKED_LEFT>),                            \
+        reinterpret_cast<const void *>(&KERNEL<DT, OP, 8, 4, SHAPE>),                                                             \
+        reinterpret_cast<const void *>(&KERNEL<DT, OP, 8, 8, SHAPE>),                                                             \
+        reinterpret_cast<const void *>(&KERNEL<DT, OP, 16, 16, SHAPE>)
+#define HCCL_ORDERS(KERNEL, OP)                                                                                                  \
+    HCCL_SHAPES(KERNEL, OP, PACKED_LEFT), HCCL_SHAPES(KERNEL, OP, (OrderMatters<DT, OP>::value ? PACKED_RING : PACKED_LEFT)),     \
+        HCCL_SHAPES(KERNEL, OP, PACKED_TREE)
 #define HCCL_ROW(OP)                                                     \
     {                                                                    \
         reinterpret_cast<const void *>(&StepKernel<DT, OP>),             \
@@ -95,7 +98,7 @@ extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[17] = {
         reinterpret_cast<const void *>(&PackedKernel<DT, OP, 8>),        \
         reinterpret_cast<const void *>(&PackedKernel<DT, OP, 16>),       \
         reinterpret_cast<const void *>(&PackedKernel<DT, OP, 32>),       \
-        HCCL_SHAPES(OP, PACKED_LEFT), HCCL_SHAPES(OP, (OrderMatters<DT, OP>::value ? PACKED_RING : PACKED_LEFT)), HCCL_SHAPES(OP, PACKED_TREE),   \
+        HCCL_ORDERS(PackedShapeKernel, OP), HCCL_ORDERS(PackedWideKernel, OP),                                                    \
     }
 extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[4][KK_COUNT] = {
     HCCL_ROW(ROP_SUM), HCCL_ROW(ROP_PROD), HCCL_ROW(ROP_MAX), HCCL_ROW(ROP_MIN),

@@ -148,7 +148,7 @@ struct DirectLaunch {
 // Whether a collective is small enough for this form, whatever its schedule (bytes: of the call's count).
 bool DirectFits(int coll, uint32_t p, uint64_t bytes, int dtype);
 // Whether a larger one goes out in the packed form if its items are alike.
-bool PackedFits(int coll, uint32_t p, uint64_t bytes);
+bool PackedFits(int coll, uint32_t p, uint64_t bytes, int dtype);
 // The launch of `plan`; false (func == nullptr) where the kernels' records cannot hold it.
 bool BuildDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaunch *d);
 // The packed form of a launch that BuildDirect has made, where the plan's items are alike.

@@ -21,6 +21,7 @@ using namespace hcclamd;
 
 namespace {
 
+long g_wide = 0;
 uint64_t g_state = 0x9E3779B97F4A7C15ull;
 uint64_t Below(uint64_t n)
 {
@@ -117,7 +118,17 @@ template <uint32_t P> bool Same(const Plan &plan, const DirectLaunch &d, const s
         if (P != (nsrc == 16 ? 16 : 8)) {
             return false;
         }
+        // of several MiB to many destinations: four vectors per lane
+        uint64_t total = 0;
+        for (const FusedItem &f : plan.fused) {
+            total += f.bytes;
+        }
+        if (!(k.info & kPackedToOne) && total > (nsrc == 16 ? 3u << 19 : 2u << 20) && total <= 8u << 20) {
+            kind += KK_PACKED_WIDE;
+            g_wide++;
+        }
     }
+    const uint32_t chunk = kind >= KK_PACKED_CHAIN + KK_PACKED_WIDE ? 4096 : 1024;
     if (d.packedFunc != LookupKernel(0, 0, KernelKind(kind))) {
         return false;
     }
@@ -126,7 +137,7 @@ template <uint32_t P> bool Same(const Plan &plan, const DirectLaunch &d, const s
     for (uint32_t i = 0; ok && i < plan.fused.size(); i++) {
         const Item a = OfPlan(plan.fused[i], send, recv), b = OfArguments<P>(k, i, &ok);
         ok = ok && a.bytes == b.bytes && a.value == b.value && a.dst == b.dst && (a.bytes % 16 == 0 || ends) &&
-            uint64_t(d.packedGridX - ends) * kDirectChunk >= a.bytes / 16 * 16;
+            uint64_t(d.packedGridX - ends) * chunk >= a.bytes / 16 * 16;
     }
     return ok;
 }
@@ -158,7 +169,7 @@ int main(int argc, char **argv)
         rq.root = uint32_t(Below(rq.p));
         const bool same = rq.coll == COLL_BROADCAST || (rq.coll == COLL_ALLREDUCE && Below(2));
         rq.alias.assign(rq.p, same ? 1 : 0);
-        rq.count = 1 + Below(Below(2) ? 300 : 40000 / rq.p);
+        rq.count = 1 + Below(Below(2) ? 300 : Below(4) ? 40000 / rq.p : 12000000 / rq.unit);
         Plan plan;
         std::string err;
         DirectLaunch d;
@@ -210,7 +221,7 @@ int main(int argc, char **argv)
             taken[d.packedRanks == 8 ? 0 : d.packedRanks == 16 ? 1 : 2]++;
         }
     }
-    std::printf("OK up to 8 ranks %ld 16 ranks %ld 32 ranks %ld trees %ld in place %ld unlike %ld too far apart %ld\n", taken[0], taken[1], taken[2], trees,
-        inPlace, unlike, apart);
+    std::printf("OK up to 8 ranks %ld 16 ranks %ld 32 ranks %ld trees %ld in place %ld unlike %ld too far apart %ld wide %ld\n", taken[0], taken[1], taken[2], trees,
+        inPlace, unlike, apart, g_wide);
     return 0;
 }

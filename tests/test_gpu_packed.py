@@ -11,7 +11,7 @@ from closed_forms import BF16, FP16, FP32, INT8, INT64, MAX, MIN, PROD, SUM
 pytestmark = pytest.mark.gpu
 RING, MESH, RHD = 0, 4, 2      # (4: the mesh without the piece cut, which these types and operations run)
 MIB = 1 << 20
-LIMIT = {2: 32 * MIB, 3: 7 * MIB // 2, 4: 7 * MIB // 2, 8: 9 * MIB // 4}     # of an all-reduce; more ranks: 1.5 MiB
+LIMIT = {2: 48 * MIB, 3: 7 * MIB // 2, 4: 6 * MIB, 7: 9 * MIB // 4, 8: 11 * MIB // 4, 16: 11 * MIB // 4}     # of an all-reduce; more ranks: 1.5 MiB
 
 
 def _ins(dt, p, n, seed, special):
@@ -50,10 +50,36 @@ def test_all_reduce(orc, p, algo):
         g.close()
 
 
+@pytest.mark.parametrize("p,algo", [(p, a) for p in (2, 4, 8, 16) for a in ("ring", "mesh", "rhd")])
+def test_four_vectors_per_lane(orc, p, algo):
+    """Between 2 and 8 MiB (16 ranks: from 1.5 MiB): whole waves of 4 KiB, one vector and one element more or less, either end of the range."""
+    g = gh.Group(p, algo=algo)
+    first = (3 if p == 16 else 4) * MIB // 2
+    try:
+        for k, (dt, op, pad, in_place, special) in enumerate([(FP32, MAX, 4, True, True), (BF16, SUM, 0, False, False), (INT8, PROD, 1, False, False), (INT64, SUM, 0, True, False)]):
+            unit = gh.H.DTYPE_SIZE[dt]
+            whole = (first // p + 4096) // 4096 * 4096 * p
+            sizes = {whole, whole + 16 * p, whole - 16 * p} if k % 2 else {first + unit, whole + unit, whole - unit}
+            if k == ("ring", "mesh", "rhd").index(algo):
+                sizes |= {11 * MIB // 2 // unit * unit} if p > 4 else {6 * MIB}
+            for size in sorted(sizes):
+                n = size // unit
+                print("packed, four vectors per lane", p, algo, "type", dt, "op", op, "n", n, flush=True)
+                ins = _ins(dt, p, n, 17 * p + n % 1013 + k, special)
+                want = orc.allreduce(ins, dt, op, algo={"ring": RING, "mesh": MESH, "rhd": RHD}[algo])
+                outs, keep = gh.all_reduce(g, ins, dt, op, in_place=in_place, pad=pad)
+                assert g.info()["launches"] == 1 and g.info()["fused"] == 1
+                for r in range(p):
+                    assert gh.same(dt, outs[r], want[r]), (dt, op, n, r)
+                    assert keep is None or np.array_equal(keep[r].view(np.uint8), ins[r].view(np.uint8))
+    finally:
+        g.close()
+
+
 @pytest.mark.parametrize("p", [2, 4, 5, 8, 16])
 def test_blocks(orc, p):
     g = gh.Group(p)
-    limit = {2: 14 * MIB, 4: 6 * MIB}.get(p, 9 * MIB // 2)
+    limit = {2: 15 * MIB, 4: 15 * MIB // 2, 8: 6 * MIB, 16: 11 * MIB // 4}.get(p, 9 * MIB // 2)
     try:
         for dt, op, pad in ((INT8, PROD, 1), (BF16, SUM, 2), (FP32, MIN, 0), (INT64, SUM, 8)):
             unit = gh.H.DTYPE_SIZE[dt]

@@ -280,6 +280,7 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
     const uint32_t stepGrid = std::max(1u, g->numCu * (g->cfg.blocksPerCu ? g->cfg.blocksPerCu : 2u));
     uint32_t fusedPerCu = g->cfg.blocksPerCu;
     if (fusedPerCu == 0) {
+        constexpr double kMiB = 1024.0 * 1024.0;
         double streamBytes = 0, storeBytes = 0, bytes = 0;
         for (const FusedItem &it : pp->plan->fused) {
             uint32_t nsrc = 0;
@@ -292,16 +293,22 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
         }
         double streams = bytes > 0 ? streamBytes / bytes : 2.0;   // loads + stores per lane and vector
         fusedPerCu = streams >= 8.0 ? 1u : (streams >= 3.0 ? 2u : 4u);
-        // That holds for shapes that write as much as they read or more, and for everything much larger than the
-        // memory-side cache.  Many sources into one destination (reduce-scatter, reduce) of 8- and 16-bit elements,
-        // where a combine costs several instructions, run better wide up to about a gigabyte in all (measured, bf16
-        // sum: 8 ranks x 64 MiB 104 us at 1 per CU, 99 at 8; 16 ranks x 64 MiB 196 / 189; a reduce of 8 x 256 MiB in one
-        // launch 416 / 423, so not there, but a reduce-scatter of that size, which goes out in launches of 512 MiB, 413 /
-        // 396; fp32 within a percent either way at every size).
-        const double launchBytes = capBytes != 0 ? std::min(streamBytes, double(capBytes)) : streamBytes;
-        if (fusedPerCu == 1 && reduceColl && DtypeSize(dtype) <= 2 && storeBytes * 5.0 <= streamBytes &&
-            launchBytes <= 1.25 * 1024.0 * 1024.0 * 1024.0) {
-            fusedPerCu = 8;
+        // Many sources into one destination (reduce-scatter, reduce).  Beyond the memory-side cache few workgroups keep the
+        // sources' streams apart, below it many hide the latency of a combine, which for elements of one and two bytes takes
+        // several instructions.  Three sets of buffers in turn, us, 1 / 2 / 8 per CU: 8 ranks in a ring bf16 sum of 64 MiB 93.2 / 98 / 99.3,
+        // 256 MiB 376 / - / 401, fp32 93.0 / 97.3 / 96.5, int8 96.8 / 95.6 / 98.7; 16 ranks x 32 MiB fp16 87 / - / 94; bf16 of 48 MiB 73.3 / 70.1 / 72.0, of 32
+        // MiB 49.5 / 49.0 / 47.5; 4 ranks x 128 MiB bf16 105.6 / 108.9 / -, fp32 105.4 / 110.1 / -, but 5 ranks x 100 MiB 110.3 / 101.3 / -; trees alike.
+        const bool toOne = reduceColl && storeBytes * 5.0 <= streamBytes && (fusedPerCu == 1 || (streams <= 5.0 && streamBytes > 512.0 * kMiB));
+        if (toOne) {
+            const bool bytewise = DtypeSize(dtype) == 1;
+            fusedPerCu = streamBytes > 512.0 * kMiB ? (bytewise ? 2u : 1u) : streamBytes > 320.0 * kMiB ? 2u : DtypeSize(dtype) <= 2 ? 8u : 2u;
+        }
+        // One source into two or more destinations (all-gather, broadcast) without the teams: many workgroups as long as the results stay in
+        // the memory-side cache (three sets in turn, us, 1 or 2 / 8 per CU: 8 ranks 256 KiB 4.6 / 4.1, 2 MiB 26.4 / 25.6, 3 MiB 42.7 / 40.5; 4 ranks
+        // 4 MiB (80 MiB moved) 13.7 / 13.0, 8 MiB (160) 30.9 / 30.1, 16 MiB (320) 61.5 / 63; 3 ranks 8 MiB (96) 17.2 / 16.3, 13 MiB (156) 30.3 / 31.2; 5 ranks
+        // 7 MiB (210) 43.0 / 43.5; 2 ranks 64 MiB (384) 73 / 70.5, 128 MiB (768) 145 / 145).
+        if (!reduceColl && streams >= 3.0 && streamBytes <= (streams <= 3.0 ? 512.0 : streams >= 8.0 ? 256.0 : 128.0) * kMiB) {
+            fusedPerCu = 8u;
         }
         // Plain copies (one source, one destination) go through the copy kernel, which really gets the
         // occupancy it is launched with; with non-temporal stores more workgroups only widen the range
@@ -312,9 +319,12 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
             fusedPerCu = 2u;
         }
         // few tiles per workgroup: a second workgroup per CU evens out the tail (measured: 16-rank
-        // ring all-reduce of 32 MiB per rank 241 us at 1 per CU, 220 us at 2)
-        if (fusedPerCu == 1 && bytes / kTileBytes < 32.0 * g->numCu) {
-            fusedPerCu = 2;
+        // ring all-reduce of 32 MiB per rank 241 us at 1 per CU, 220 us at 2), eight do so better between 3 and 16 tiles per CU
+        // (at 2 / 8: 4 ranks 32 MiB 47.1 / 44.5, 48 MiB 70.1 / 69.0; 8 ranks 15.9 MiB bf16 maximum 46.4 / 43.8; 16 ranks 12 MiB 71.1 / 67.2;
+        // 8 ranks 10 MiB, 2.5 tiles, 29.0 / 30.8; 4 ranks 64 MiB equal, int8 26 MiB 37.3 / 39.0)
+        if (fusedPerCu == 1 && !toOne && bytes / kTileBytes < 32.0 * g->numCu) {
+            const double tilesPerCu = bytes / kTileBytes / g->numCu;
+            fusedPerCu = reduceColl && DtypeSize(dtype) > 1 && tilesPerCu >= 3.0 && tilesPerCu < 16.0 ? 8 : 2;
         }
     }
     const uint32_t treeGrid = std::max(1u, g->numCu * fusedPerCu);

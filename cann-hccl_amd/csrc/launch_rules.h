@@ -60,6 +60,13 @@ constexpr uint32_t kTeamMinHalfRoundsFew = 8;
 // 67.6.  (The line was drawn when the plain kernel's results were not written through, 4 MiB 60.0 / 54.2; between a round and
 // the memory-side cache's size the plain form is now the faster one.)
 constexpr uint32_t kTeamMinHalfRoundsCopy = 2;
+// One source and 4 to 6 destinations: items on whole 128-byte lines (they have neither head nor tail) / others.  Few streams suffer less from one another, so the team's order pays
+// later; but its time hardly depends on where the buffers lie, while the plain form's does (three sets of buffers in turn, plain with eight workgroups per CU /
+// team, several placements; rounds): 4 ranks 16 MiB (2) 62 / 65, 32 MiB (4) 122 ... 131 / 118, 40 MiB 144 / 144, 48 MiB 166 ... 191 / 171 ... 173, 64 MiB (8) 255 / 226,
+// 128 MiB (16) 487 / 440; 5 ranks 16 MiB (2.5) 86.9 / 89.3, 27 MiB (4.2) 150 ... 166 / 145, 60 MiB 329 ... 339 / 307; 6 ranks 16 MiB (3) 115 ... 121 / 120, 22 MiB
+// (4.1) 166 / 159, 55 MiB 404 / 382.  Off a boundary: 4 ranks 26 MiB 91 ... 94 / 102, 40 MiB (5) 147 / 154, 64 MiB (8) 245 ... 255 / 243, 80 MiB 287 / 299, 100 MiB
+// 389 / 374; 5 ranks 40 MiB (6.25) 206 ... 231 / 217 ... 220, 60 MiB (9.4) 314 / 320; 6 ranks 24 MiB (4.5) 183 / 184, 30 MiB 215 / 225, 40 MiB (7.5) 311 / 301.
+constexpr uint32_t kTeamMinHalfRoundsCopyFew = 8, kTeamMinHalfRoundsCopyFewUneven = 16;
 
 // Whether a launch whose items with whole tiles have `bytes` in all runs that long.  (By bytes, not by tiles: a buffer that starts
 // off a boundary leaves every item a tile short, and many short pieces are no round.)

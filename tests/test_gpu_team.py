@@ -263,3 +263,28 @@ def test_library_picks_the_team_form_for_large_write_heavy_collectives(orc):
             assert np.array_equal(outs[r], want[r]), r
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("p,off", [(4, 0), (5, 0), (6, 0), (4, 1), (5, 1), (6, 1), (3, 0), (7, 0)])
+def test_gathers_of_four_to_six_blocks_take_the_team_form_beyond_their_line(p, off):
+    # with rounds of one tile per workgroup: 4 rounds of 4 MiB where every block lies on whole 128-byte lines, 8 elsewhere; 3 destinations stay plain, 7
+    # change at one round
+    g = gh.Group(p, team="auto", team_tiles=1)
+    line = (8 if off else 1 if p > 6 else 4) * torch.cuda.get_device_properties(0).multi_processor_count * 16384
+    try:
+        for step, team in ((-128, 0), (128, int(p > 3))):
+            n = line // p // 128 * 128 + step + off
+            print("gather", p, "off", off, "n", n, flush=True)
+            gen = torch.Generator(device="cuda").manual_seed(n)
+            sends = [torch.randint(-128, 128, (n,), dtype=torch.int8, device="cuda", generator=gen) for _ in range(p)]
+            recvs = [torch.zeros(n * p + off + 16, dtype=torch.int8, device="cuda") for _ in range(p)]
+            torch.cuda.synchronize()
+            H.all_gather(g.comms, [t.data_ptr() for t in sends], [t.data_ptr() + off for t in recvs], n, INT8, g.stream_ptr)
+            assert g.info()["teamLaunches"] == team and g.info()["launches"] == 1, (n, g.info())
+            torch.cuda.synchronize()
+            want = torch.cat(sends)
+            for r in range(p):
+                assert torch.equal(recvs[r][off:off + n * p], want), r
+                assert int(recvs[r][:off].count_nonzero()) == 0 and int(recvs[r][off + n * p:].count_nonzero()) == 0, r
+    finally:
+        g.close()

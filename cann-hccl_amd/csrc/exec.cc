@@ -303,14 +303,15 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
             const bool bytewise = DtypeSize(dtype) == 1;
             fusedPerCu = streamBytes > 512.0 * kMiB ? (bytewise ? 2u : 1u) : streamBytes > 320.0 * kMiB ? 2u : DtypeSize(dtype) <= 2 ? 8u : 2u;
         }
-        // One source into two or more destinations (all-gather, broadcast) without the teams: many workgroups as long as the results stay in
+        // Blocks of several sources into two or more destinations each (all-gather) without the teams: many workgroups as long as the results stay in
         // the memory-side cache, and again far beyond it where there are fewer than 7 destinations (three sets in turn, us, 1 or 2 / 8 per CU,
         // bytes moved in parentheses: 8 ranks 256 KiB 4.6 / 4.1, 2 MiB 26.4 / 25.6, 3 MiB 42.7 / 40.5; 4 ranks 4 MiB (80 MiB) 13.7 / 13.0, 8 MiB (160)
         // 30.9 / 30.1, 16 MiB (320) 61.5 / 63, 40 MiB (800) 150 / 144; 3 ranks 8 MiB (96) 17.2 / 16.3, 13 MiB (156) 30.3 / 31.2, 24 MiB (288) 54.6 / 55.7,
         // 64 MiB (768) 145 / 138, 96 MiB 213 ... 239 / 217 ... 229; 5 ranks 7 MiB (210) 43.0 / 43.5, 40 MiB (1200) 215 / 206; 2 ranks 64 MiB (384) 73 / 70.5, 112 MiB
-        // (672) 129 / 121, 128 MiB 139 / 140).
+        // (672) 129 / 121, 128 MiB 139 / 140).  A broadcast sweeps one source and is left at two: 3 ranks 32 MiB 14.3 / 15.2, 4 ranks 256 MiB 176 / 185, 6 ranks 100
+        // MiB 110 / 113.
         const double cached = (streams >= 8.0 ? 256.0 : 128.0) * kMiB;
-        if (!reduceColl && streams >= 3.0 && (streams <= 3.0 || streamBytes <= cached || (streams < 8.0 && streamBytes > 512.0 * kMiB))) {
+        if (g->ctx->sig.coll == COLL_ALLGATHER && streams >= 3.0 && (streams <= 3.0 || streamBytes <= cached || (streams < 8.0 && streamBytes > 512.0 * kMiB))) {
             fusedPerCu = 8u;
         }
         // Plain copies (one source, one destination) go through the copy kernel, which really gets the

@@ -297,11 +297,18 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
         // sources' streams apart, below it many hide the latency of a combine, which for elements of one and two bytes takes
         // several instructions.  Three sets of buffers in turn, us, 1 / 2 / 8 per CU: 8 ranks in a ring bf16 sum of 64 MiB 93.2 / 98 / 99.3,
         // 256 MiB 376 / - / 401, fp32 93.0 / 97.3 / 96.5, int8 96.8 / 95.6 / 98.7; 16 ranks x 32 MiB fp16 87 / - / 94; bf16 of 48 MiB 73.3 / 70.1 / 72.0, of 32
-        // MiB 49.5 / 49.0 / 47.5; 4 ranks x 128 MiB bf16 105.6 / 108.9 / -, fp32 105.4 / 110.1 / -, but 5 ranks x 100 MiB 110.3 / 101.3 / -; trees alike.
-        const bool toOne = reduceColl && storeBytes * 5.0 <= streamBytes && (fusedPerCu == 1 || (streams <= 5.0 && streamBytes > 512.0 * kMiB));
+        // MiB 49.5 / 49.0 / 47.5; 4 ranks x 128 MiB bf16 105.6 / 108.9 / -, fp32 105.4 / 110.1 / -, but 5 ranks x 100 MiB 110.3 / 101.3 / -.
+        const bool manyToOne = reduceColl && storeBytes * 5.0 <= streamBytes;
+        const bool toOne = manyToOne && !pp->plan->fused.empty() && pp->plan->fused[0].kind == FK_CHAIN && (fusedPerCu == 1 || (streams <= 5.0 && streamBytes > 512.0 * kMiB));
         if (toOne) {
             const bool bytewise = DtypeSize(dtype) == 1;
             fusedPerCu = streamBytes > 512.0 * kMiB ? (bytewise ? 2u : 1u) : streamBytes > 320.0 * kMiB ? 2u : DtypeSize(dtype) <= 2 ? 8u : 2u;
+        }
+        // Trees and stack programs, whose combines are more of the work, gain nothing from few (fp32 tree of 8 x 64 MiB 1 / 2 per CU 101 / 99) and keep many for
+        // elements of one and two bytes up to about a gigabyte (two servers, 8 ranks, bf16 40 MiB 2 / 8 per CU 63.8 / 62.2).
+        const double launchBytes = capBytes != 0 ? std::min(streamBytes, double(capBytes)) : streamBytes;
+        if (manyToOne && !toOne && fusedPerCu == 1 && DtypeSize(dtype) <= 2 && launchBytes <= 1280.0 * kMiB) {
+            fusedPerCu = 8;
         }
         // Blocks of several sources into two or more destinations each (all-gather) without the teams: many workgroups as long as the results stay in
         // the memory-side cache, and again far beyond it where there are fewer than 7 destinations (three sets in turn, us, 1 or 2 / 8 per CU,

@@ -1,4 +1,4 @@
-"""Small collectives with packed arguments (a wave per KiB of an item), against the CPU checker bit for bit: every shape that has a kernel of
+"""Small collectives with packed arguments (a wave per KiB of an item), against the oracle bit for bit: every shape that has a kernel of
 its own (2, 4, 8, 16 sources; chains of either operand order, trees), other numbers of sources, the edges of a wave's KiB and of a
 vector, in place, off a boundary, up to and beyond the sizes where the tile kernels take over."""
 import numpy as np

@@ -360,26 +360,12 @@ HcclResult A2avFinish(Group *g, hipStream_t stream, A2avSet **ready)
         (void)hipGetLastError();
         return HCCL_SUCCESS;
     }
-    const bool onDevice = g->p > 16;
     if (g->a2avBuilding < 0) {
-        for (uint32_t k = 0; k < kA2avSets; k++) {
-            A2avSet *s = &g->a2avSets[k];
-            // (tables in device memory belong to the stream that they were written on)
-            if (((g->a2avAlive >> k) & 1u) && (!onDevice || s->stream == stream)) {
-                s->hit = true;
-                s->lastUse = ++g->a2avClock;
-                *ready = s;
-                return HCCL_SUCCESS;
-            }
-        }
-        // the same call on another stream: written down once more
-        const uint32_t to = Victim(g);
-        A2avSet *s = &g->a2avSets[to], *from = &g->a2avSets[uint32_t(__builtin_ctz(g->a2avAlive))];
-        s->valid = false;
-        s->image = from->image;
-        s->sent = from->sent;
-        s->place = from->place;
-        g->a2avBuilding = int(to);
+        A2avSet *s = &g->a2avSets[uint32_t(__builtin_ctz(g->a2avAlive))];
+        s->hit = true;
+        s->lastUse = ++g->a2avClock;
+        *ready = s;
+        return HCCL_SUCCESS;
     }
     A2avSet *s = &g->a2avSets[uint32_t(g->a2avBuilding)];
     bool general = false;
@@ -392,17 +378,43 @@ HcclResult A2avFinish(Group *g, hipStream_t stream, A2avSet **ready)
     return HCCL_SUCCESS;
 }
 
-HcclResult A2avUpload(Group *g, A2avSet *s, hipStream_t stream)
+namespace {
+
+// Puts the set's tables into device memory, if they are not there, for a launch on `stream`; nothing here waits on the host for other streams' work.
+// A set that another call takes over is written anew, behind the launches that read it.  As long as all of a group's calls come on one
+// stream, its order sees to that and a call pays for no event.  From the first call on a second stream on, every launch leaves an event behind,
+// and sets are written to the other half of the memory: what launches that left no event may still read is never written again.
+HcclResult OnDevice(Group *g, A2avSet *s, hipStream_t stream)
 {
     const size_t bytes = (TableBytes(g->p) + 255) & ~size_t(255);
     if (g->a2avTables == nullptr) {
-        HIP_OK(hipMalloc(&g->a2avTables, kA2avSets * bytes));
+        HIP_OK(hipMalloc(&g->a2avTables, 2 * kA2avSets * bytes));
+        g->a2avStream = stream;
     }
-    s->table = static_cast<char *>(g->a2avTables) + size_t(s - g->a2avSets.data()) * bytes;
-    if (s->stream != nullptr && s->stream != stream) {
-        HIP_OK(hipDeviceSynchronize());      // another stream's call may still be reading these tables
+    g->a2avStreams = g->a2avStreams || g->a2avStream != stream;
+    if (s->onDevice) {
+        if (s->stream != stream && !s->arrived) {
+            if (hipEventQuery(s->uploaded) == hipSuccess) {
+                s->arrived = true;
+            } else {
+                (void)hipGetLastError();
+                HIP_OK(hipStreamWaitEvent(stream, s->uploaded, 0));
+            }
+        }
+        return HCCL_SUCCESS;
     }
-    s->stream = stream;
+    if (s->uploaded == nullptr) {
+        HIP_OK(hipEventCreateWithFlags(&s->uploaded, hipEventDisableTiming));
+    } else if (g->a2avStreams) {
+        HIP_OK(hipStreamWaitEvent(stream, s->uploaded, 0));
+        for (A2avReader &r : s->readers) {
+            if (r.reading) {
+                HIP_OK(hipStreamWaitEvent(stream, r.done, 0));
+                r.reading = false;
+            }
+        }
+    }
+    s->table = static_cast<char *>(g->a2avTables) + (2 * size_t(s - g->a2avSets.data()) + (g->a2avStreams ? 1 : 0)) * bytes;
     StageSlot &slot = g->stageSlots[g->stageNext++ % g->stageSlots.size()];
     if (slot.used) {
         HIP_OK(hipEventSynchronize(slot.done));
@@ -411,20 +423,52 @@ HcclResult A2avUpload(Group *g, A2avSet *s, hipStream_t stream)
     HIP_OK(UploadFromPinned(s->table, slot.host, TableBytes(g->p), stream));
     HIP_OK(hipEventRecord(slot.done, stream));
     slot.used = true;
+    HIP_OK(hipEventRecord(s->uploaded, stream));
+    s->stream = stream;
+    s->arrived = false;
+    s->onDevice = true;
     return HCCL_SUCCESS;
 }
 
+// What a launch on `stream` leaves its event in.  A set remembers a few streams; beyond those a launch goes behind the one whose place it takes.
+HcclResult Reader(A2avSet *s, hipStream_t stream, A2avReader **reader)
+{
+    for (A2avReader &r : s->readers) {
+        if (r.stream == stream) {
+            *reader = &r;
+            return HCCL_SUCCESS;
+        }
+    }
+    if (s->readers.size() < kA2avReaders) {
+        A2avReader fresh;
+        HIP_OK(hipEventCreateWithFlags(&fresh.done, hipEventDisableTiming));
+        s->readers.push_back(fresh);
+        *reader = &s->readers.back();
+    } else {
+        *reader = &s->readers[s->nextReader++ % kA2avReaders];
+        HIP_OK(hipStreamWaitEvent(stream, (*reader)->done, 0));
+    }
+    (*reader)->stream = stream;
+    return HCCL_SUCCESS;
+}
+
+}  // namespace
+
 HcclResult A2avLaunch(Group *g, A2avSet *s, hipStream_t stream)
 {
+    const bool inArguments = g->p <= 16;
+    A2avReader *reader = nullptr;
     if (!s->hit) {
-        if (g->p > 16) {
-            HcclResult r = A2avUpload(g, s, stream);
-            if (r != HCCL_SUCCESS) {
-                return r;
-            }
+        s->onDevice = false;
+    }
+    if (!inArguments) {
+        HcclResult r = OnDevice(g, s, stream);
+        if (r == HCCL_SUCCESS && g->a2avStreams) {
+            r = Reader(s, stream, &reader);
         }
-        s->valid = true;
-        s->lastUse = ++g->a2avClock;
+        if (r != HCCL_SUCCESS) {
+            return r;
+        }
     }
     const uint32_t ranks = RanksOf(g->p), which = uint32_t(__builtin_ctz(ranks)) - 3;
     const void *func = LookupCopyKernel(KernelKind(KK_A2AV + which + (s->width == 0 ? 0 : 4)));
@@ -439,11 +483,19 @@ HcclResult A2avLaunch(Group *g, A2avSet *s, hipStream_t stream)
             continue;
         }
         void *args[2] = {&s->table, &range};
-        if (g->p <= 16) {
+        if (inArguments) {
             std::memcpy(s->image.data() + TableBytes(g->p), &range, sizeof(range));
             args[0] = s->image.data();
         }
         HIP_OK(hipLaunchKernel(func, dim3(grid, 1, 1), dim3(64 * waves, 1, 1), args, 0, stream));
+    }
+    if (reader != nullptr) {
+        HIP_OK(hipEventRecord(reader->done, stream));
+        reader->reading = true;
+    }
+    if (!s->hit) {
+        s->valid = true;
+        s->lastUse = ++g->a2avClock;
     }
     return HCCL_SUCCESS;
 }

@@ -1390,6 +1390,14 @@ Group::~Group()
     if (barrierMem) {
         (void)hipFree(barrierMem);
     }
+    for (A2avSet &s : a2avSets) {
+        if (s.uploaded) {
+            (void)hipEventDestroy(s.uploaded);
+        }
+        for (A2avReader &r : s.readers) {
+            (void)hipEventDestroy(r.done);
+        }
+    }
     if (a2avTables) {
         (void)hipFree(a2avTables);
     }

@@ -234,6 +234,12 @@ struct StageSlot {
 
 // An all-to-all-v as its ranks called it, in the form that the device takes it (a2av.cc).
 constexpr uint32_t kA2avSets = 8;
+constexpr uint32_t kA2avReaders = 8;
+struct A2avReader {
+    hipStream_t stream = nullptr;
+    hipEvent_t done = nullptr;        // behind the latest launch there that reads the set's tables
+    bool reading = false;             // there was one since they were written
+};
 struct A2avSet {
     bool valid = false;               // a call that was issued: what follows belongs together
     bool hit = false;                 // the call under way is this one
@@ -244,8 +250,13 @@ struct A2avSet {
     uint64_t moved = 0;
     uint32_t unitShift = 0, pieces = 0, launches = 0;
     uint32_t width = 0;               // workgroups of four waves per CU, results non-temporal; 0: of one wave, written through
-    void *table = nullptr;            // more than 16 ranks: the image in device memory, written and read on `stream` alone
+    // the image in device memory (OnDevice, a2av.cc)
+    bool onDevice = false, arrived = false;   // it was written, on `stream`; that is known to have been done
+    void *table = nullptr;
     hipStream_t stream = nullptr;
+    hipEvent_t uploaded = nullptr;
+    std::vector<A2avReader> readers;  // once the group's calls come on several streams
+    uint32_t nextReader = 0;
 };
 
 struct Group;
@@ -288,7 +299,9 @@ struct Group {
     uint32_t a2avUnit = 0;
     uint64_t a2avClock = 0;
     std::vector<A2avSet> a2avSets;   // the latest calls, kA2avSets of them
-    void *a2avTables = nullptr;      // their tables in device memory (more than 16 ranks)
+    void *a2avTables = nullptr;      // their tables in device memory, two places for each
+    hipStream_t a2avStream = nullptr;   // the stream of the first call that read them ...
+    bool a2avStreams = false;        // ... and whether one came on another
     A2avSet *a2avReady = nullptr;    // complete and checked, for IssueCollective
     OpCtx *ctx = nullptr;            // the operation being issued (the rendezvous, or a matched send / receive)
     std::map<std::pair<uint32_t, uint32_t>, std::deque<P2PPending>> p2p;

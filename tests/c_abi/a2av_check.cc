@@ -1,0 +1,273 @@
+// The tables of all-to-all-v calls in device memory (cann-hccl_amd/csrc/a2av.cc), on the host: a seeded walk over calls of one group on a
+// model of streams and events (the first quarter of them on one stream), in which work is done as late as the orders allow, in any order they leave open.  Whenever a launch is done, the
+// tables it reads have to be those of its call.  The calls may not wait for the device, and a call known by its numbers counts as known on whatever
+// stream it comes.  argv[1] = ranks, argv[2] = calls, argv[3] = streams, argv[4] = sets of tables in turn.
+#include <algorithm>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <deque>
+#include <map>
+#include <memory>
+#include <string>
+#include <vector>
+
+#include "noalloc.h"
+#include "runtime.h"
+
+namespace {
+
+uint64_t g_state = 0x2545F4914F6CDD1Dull;
+uint64_t Below(uint64_t n)
+{
+    g_state = g_state * 6364136223846793005ull + 1442695040888963407ull;
+    return n == 0 ? 0 : (g_state >> 29) % n;
+}
+
+struct Op {
+    enum { UPLOAD, LAUNCH, RECORD, WAIT } kind;
+    const uint8_t *from = nullptr;      // upload
+    uint8_t *to = nullptr;              // upload, launch
+    size_t bytes = 0;
+    std::vector<uint8_t> want;          // launch: the tables it has to find
+    uint32_t event = 0;
+    uint64_t serial = 0;                // of a record: which one; of a wait: for which one
+};
+std::map<uintptr_t, std::deque<Op>> g_streams;
+struct Event {
+    uint64_t recorded = 0, done = 0;
+};
+std::vector<Event> g_events(1);
+long g_deviceWaits = 0, g_hostWaits = 0, g_launches = 0, g_wrong = 0, g_records = 0, g_order = 0;
+const hcclamd::A2avSet *g_ready = nullptr;      // the call being launched
+std::vector<uint8_t> g_expected;                // its tables
+
+Event &Of(hipEvent_t e) { return g_events[reinterpret_cast<uintptr_t>(e)]; }
+std::deque<Op> &Of(hipStream_t s) { return g_streams[reinterpret_cast<uintptr_t>(s)]; }
+
+bool Step(std::deque<Op> &q)
+{
+    if (q.empty() || (q.front().kind == Op::WAIT && g_events[q.front().event].done < q.front().serial)) {
+        return false;
+    }
+    const Op &op = q.front();
+    if (op.kind == Op::UPLOAD) {
+        std::memcpy(op.to, op.from, op.bytes);
+    } else if (op.kind == Op::LAUNCH) {
+        g_wrong += std::memcmp(op.to, op.want.data(), op.want.size()) != 0;
+    } else if (op.kind == Op::RECORD) {
+        g_events[op.event].done = std::max(g_events[op.event].done, op.serial);
+    }
+    q.pop_front();
+    return true;
+}
+// Some work of some streams.
+void Progress(uint64_t steps)
+{
+    for (uint64_t n = 0; n < steps && !g_streams.empty(); n++) {
+        auto it = g_streams.begin();
+        std::advance(it, Below(g_streams.size()));
+        Step(it->second);
+    }
+}
+void Until(const Event &e, uint64_t serial)
+{
+    for (long n = 0; e.done < serial; n++) {
+        Progress(1);
+        if (n > 100000000) {
+            std::printf("a wait that never ends\n");
+            std::exit(1);
+        }
+    }
+}
+
+}  // namespace
+
+extern "C" {
+hipError_t hipMalloc(void **p, size_t n) { *p = std::calloc(1, n); return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned)
+{
+    g_events.emplace_back();
+    *e = reinterpret_cast<hipEvent_t>(g_events.size() - 1);
+    return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s)
+{
+    Op op;
+    op.kind = Op::RECORD;
+    op.event = uint32_t(reinterpret_cast<uintptr_t>(e));
+    op.serial = ++Of(e).recorded;
+    Of(s).push_back(op);
+    g_records++;
+    return hipSuccess;
+}
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned)
+{
+    Op op;
+    op.kind = Op::WAIT;
+    op.event = uint32_t(reinterpret_cast<uintptr_t>(e));
+    op.serial = Of(e).recorded;
+    Of(s).push_back(op);
+    g_order++;
+    return hipSuccess;
+}
+hipError_t hipEventQuery(hipEvent_t e) { return Of(e).done == Of(e).recorded ? hipSuccess : hipErrorNotReady; }
+hipError_t hipEventSynchronize(hipEvent_t e)
+{
+    g_hostWaits += Of(e).done != Of(e).recorded;
+    Until(Of(e), Of(e).recorded);
+    return hipSuccess;
+}
+hipError_t hipDeviceSynchronize()
+{
+    g_deviceWaits++;
+    for (bool any = true; any;) {
+        any = false;
+        for (auto &s : g_streams) {
+            while (Step(s.second)) {
+                any = true;
+            }
+        }
+    }
+    return hipSuccess;
+}
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *st) { *st = hipStreamCaptureStatusNone; return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+const char *hipGetErrorString(hipError_t) { return "?"; }
+hipError_t hipLaunchKernel(const void *, dim3, dim3, void **args, size_t, hipStream_t s)
+{
+    g_launches++;
+    if (args[0] != &g_ready->table) {       // the tables themselves, which a launch copies at once
+        g_wrong += std::memcmp(args[0], g_expected.data(), g_expected.size()) != 0;
+        return hipSuccess;
+    }
+    Op op;
+    op.kind = Op::LAUNCH;
+    op.to = static_cast<uint8_t *>(g_ready->table);
+    op.want = g_expected;
+    Of(s).push_back(op);
+    return hipSuccess;
+}
+}
+
+namespace hcclamd {
+hipError_t UploadFromPinned(void *dst, const void *pinned, size_t bytes, hipStream_t stream)
+{
+    Op op;
+    op.kind = Op::UPLOAD;
+    op.to = static_cast<uint8_t *>(dst);
+    op.from = static_cast<const uint8_t *>(pinned);
+    op.bytes = bytes;
+    Of(stream).push_back(op);
+    return hipSuccess;
+}
+const void *LookupCopyKernel(KernelKind) { return &g_state; }
+HcclResult CheckOverlap(const Group *, const std::vector<uint64_t> &, const std::vector<uint64_t> &, bool *stage, bool *own)
+{
+    *stage = *own = false;
+    return HCCL_SUCCESS;
+}
+Prepared::~Prepared() = default;
+Group::~Group() = default;
+}  // namespace hcclamd
+
+using namespace hcclamd;
+
+int main(int argc, char **argv)
+{
+    const uint32_t p = uint32_t(argc > 1 ? std::atoi(argv[1]) : 20);
+    const long calls = argc > 2 ? std::atol(argv[2]) : 1000;
+    const uint64_t streams = uint64_t(argc > 3 ? std::atoi(argv[3]) : 3), sets = uint64_t(argc > 4 ? std::atoi(argv[4]) : 5);
+    std::unique_ptr<Group> owner(new Group);
+    Group *g = owner.get();
+    g->p = p;
+    g->deviceReady = true;
+    g->here.assign(p, 0);
+    g->stageSlots.resize(8);
+    for (StageSlot &slot : g->stageSlots) {
+        slot.host = std::calloc(1, 128 << 10);
+        (void)hipEventCreateWithFlags(&slot.done, 0);
+    }
+    const size_t tableBytes = p <= 8 ? sizeof(A2avTable<8>) : p <= 16 ? sizeof(A2avTable<16>) : p <= 32 ? sizeof(A2avTable<32>) : sizeof(A2avTable<64>);
+    // calls: counts of set c, blocks one behind the other
+    std::vector<std::vector<uint64_t>> cnt(sets), back(sets), sd(sets), rd(sets);
+    for (uint64_t c = 0; c < sets; c++) {
+        cnt[c].resize(p * p);
+        back[c].resize(p * p);
+        sd[c].resize(p * p);
+        rd[c].resize(p * p);
+        for (uint64_t &n : cnt[c]) {
+            n = Below(5000);
+        }
+        for (uint32_t i = 0; i < p; i++) {
+            uint64_t at = 0, to = 0;
+            for (uint32_t j = 0; j < p; j++) {
+                sd[c][i * p + j] = at;
+                rd[c][i * p + j] = to;
+                back[c][i * p + j] = cnt[c][j * p + i];
+                at += cnt[c][i * p + j];
+                to += cnt[c][j * p + i];
+            }
+        }
+    }
+    long known = 0, shouldKnow = 0;
+    std::deque<uint64_t> latest;        // the last distinct calls
+    for (long n = 0; n < calls; n++) {
+        const uint64_t c = Below(3) ? Below(sets) : uint64_t(n) % sets, stream = n < calls / 4 ? 1 : 1 + (Below(2) ? Below(streams) : uint64_t(n) % streams);
+        g->arrived = 0;
+        std::fill(g->here.begin(), g->here.end(), 0);
+        A2avBegin(g, 4);
+        for (uint32_t r = 0; r < p; r++) {
+            g->here[r] = 1;
+            const uint64_t *rows[4] = {&cnt[c][r * p], &sd[c][r * p], &back[c][r * p], &rd[c][r * p]};
+            if (!A2avRow(g, r, reinterpret_cast<void *>(0x10000000ull + (uint64_t(r) << 24)), reinterpret_cast<void *>(0x7f0000000000ull + (uint64_t(r) << 24)), rows)) {
+                std::printf("a row not taken\n");
+                return 1;
+            }
+            g->arrived++;
+        }
+        A2avSet *ready = nullptr;
+        if (A2avFinish(g, reinterpret_cast<hipStream_t>(stream), &ready) != HCCL_SUCCESS || ready == nullptr) {
+            std::printf("call %ld: not taken\n", n);
+            return 1;
+        }
+        g_ready = ready;
+        g_expected.assign(ready->image.begin(), ready->image.begin() + long(tableBytes));
+        const auto seen = std::find(latest.begin(), latest.end(), c);
+        shouldKnow += seen != latest.end();
+        known += ready->hit;
+        if (seen != latest.end()) {
+            latest.erase(seen);
+        }
+        latest.push_back(c);
+        if (latest.size() > kA2avSets) {
+            latest.pop_front();
+        }
+        if (A2avLaunch(g, ready, reinterpret_cast<hipStream_t>(stream)) != HCCL_SUCCESS) {
+            std::printf("call %ld: not launched\n", n);
+            return 1;
+        }
+        if (Below(6) == 0) {
+            Progress(Below(16));
+        }
+    }
+    const long records = g_records;
+    for (auto &s : g_streams) {
+        if (!s.second.empty()) {
+            hipEvent_t e;
+            (void)hipEventCreateWithFlags(&e, 0);
+            (void)hipEventRecord(e, reinterpret_cast<hipStream_t>(s.first));
+        }
+    }
+    const long waits = g_deviceWaits;
+    (void)hipDeviceSynchronize();
+    for (auto &s : g_streams) {
+        if (!s.second.empty()) {
+            std::printf("a wait that never ends\n");
+            return 1;
+        }
+    }
+    std::printf("%s launches %ld wrong %ld device waits %ld known %ld of %ld records %ld orders %ld\n",
+        g_wrong == 0 && waits == 0 && known == shouldKnow ? "OK" : "BAD", g_launches, g_wrong, waits, known, shouldKnow, records, g_order);
+    return g_wrong == 0 && waits == 0 && known == shouldKnow ? 0 : 1;
+}

@@ -131,6 +131,43 @@ def test_sets_and_streams_in_turn(p):
         g.close()
 
 
+@pytest.mark.parametrize("p", [10, 24])
+def test_no_stream_waits_for_another(p):
+    """A call known by its numbers is known on every stream; new tables on streams in turn are queued while another stream is at work."""
+    rng = np.random.default_rng(83 + p)
+    g = gh.Group(p)
+    try:
+        runs = [Run(rng, p, 4, lambda n: rng.integers(0, 300, (n, n)), "any", 4) for _ in range(16)]
+        streams = [torch.cuda.Stream() for _ in range(3)]
+        for r in runs:
+            r.clear()
+        for k, r in enumerate(runs[:10]):       # (more than are kept, on all of the streams)
+            r.call(g, streams[k % 3])
+        torch.cuda.synchronize()
+        for r in runs[:10]:
+            r.check()
+        for r in runs[4:10]:
+            r.clear()
+        for r in runs[4:10]:
+            for s in streams:
+                r.call(g, s)
+                assert g.info()["cacheHit"] == 1
+        for r in runs[4:10]:
+            r.check()
+        busy, there = torch.cuda.Stream(), torch.cuda.Event()
+        with torch.cuda.stream(busy):
+            torch.cuda._sleep(200_000_000)
+            there.record()
+        for k, r in enumerate(runs[10:16]):     # (no more than there are pinned buffers for them)
+            r.call(g, streams[(2 * k) % 3])
+            assert g.info()["cacheHit"] == 0
+        assert not there.query(), "a call waited for work on another stream"
+        for r in runs[10:16]:
+            r.check()
+    finally:
+        g.close()
+
+
 @pytest.mark.parametrize("p", [6, 18])
 def test_the_general_way_gives_the_same(p):
     rng = np.random.default_rng(59 + p)

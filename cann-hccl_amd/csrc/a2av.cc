@@ -456,7 +456,9 @@ HcclResult Reader(A2avSet *s, hipStream_t stream, A2avReader **reader)
 
 HcclResult A2avLaunch(Group *g, A2avSet *s, hipStream_t stream)
 {
-    const bool inArguments = g->p <= 16;
+    // Up to 16 ranks a new call's tables travel in the arguments; from its second time on it reads them from device memory: the launch call writes 944
+    // bytes of arguments to 8 ranks, 3.4 KB to 16, of 24 otherwise.
+    const bool inArguments = g->p <= 16 && !s->hit;
     A2avReader *reader = nullptr;
     if (!s->hit) {
         s->onDevice = false;
@@ -471,7 +473,7 @@ HcclResult A2avLaunch(Group *g, A2avSet *s, hipStream_t stream)
         }
     }
     const uint32_t ranks = RanksOf(g->p), which = uint32_t(__builtin_ctz(ranks)) - 3;
-    const void *func = LookupCopyKernel(KernelKind(KK_A2AV + which + (s->width == 0 ? 0 : 4)));
+    const void *func = LookupCopyKernel(KernelKind(inArguments ? KK_A2AV_ARGS + which + (s->width == 0 ? 0 : 2) : KK_A2AV + which + (s->width == 0 ? 0 : 4)));
     if (func == nullptr) {
         return HCCL_E_NOT_SUPPORT;
     }

@@ -114,8 +114,9 @@ enum KernelKind : int {
     KK_PACKED_WIDE = 12,                                       // added to one of the last 12 kinds: four vectors per lane
     KK_COUNT = 38,
     KK_GATHER = 38,                                            // copy kernel table only, like these:
-    KK_A2AV = 39                                               // all-to-all-v from the callers' tables, of 8, 16, 32, 64 ranks: workgroups of
-                                                               // one wave (kinds 39 ... 42), of four (43 ... 46)
+    KK_A2AV = 39,                                              // all-to-all-v from the callers' tables in device memory, of 8, 16, 32, 64
+                                                               // ranks: workgroups of one wave (kinds 39 ... 42), of four (43 ... 46);
+    KK_A2AV_ARGS = 47                                          // in the kernel arguments, of 8, 16 ranks: one wave (47, 48), four (49, 50)
 };
 constexpr uint32_t kPackedShapes = 4;
 // Index of a number of sources among those that have a kernel of their own, kPackedShapes where it has none.
@@ -221,7 +222,7 @@ const void *LookupKernel(int hcclDataType, int hcclReduceOp, KernelKind kind);
 
 //   KK_GATHER          (const SegDesc *segs, uint32_t nsegs)
 //                      copy kernel table only
-//   KK_A2AV            up to 16 ranks (A2avArgs<P>), else (const A2avTable<P> *table, A2avRange); any number of workgroups
+//   KK_A2AV            (const A2avTable<P> *table, A2avRange); KK_A2AV_ARGS (A2avArgs<P>); any number of workgroups
 //                      copy kernel table only
 // Byte-wise variants for pure data movement (all-gather, all-to-all-v): KK_STEP, KK_CHAIN, KK_TEAM_CHAIN, KK_GATHER,
 // KK_DIRECT, KK_DIRECT_WIDE and KK_PACKED_n.

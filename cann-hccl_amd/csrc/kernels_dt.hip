@@ -54,7 +54,7 @@ using DT = uint8_t;
 
 #if HCCL_DT == 255
 // pure data movement: the step kernel's copy path and the copy kernel
-extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[17] = {
+extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[21] = {
     reinterpret_cast<const void *>(&StepKernel<DT, ROP_SUM>),
     reinterpret_cast<const void *>(&CopyKernel<0>),
     reinterpret_cast<const void *>(&GatherKernel<0>),
@@ -64,14 +64,18 @@ extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[17] = {
     reinterpret_cast<const void *>(&PackedCopyKernel<8>),
     reinterpret_cast<const void *>(&PackedCopyKernel<16>),
     reinterpret_cast<const void *>(&PackedCopyKernel<32>),
-    reinterpret_cast<const void *>(&A2avArgsKernel<8, 64, STORE_THROUGH>),
-    reinterpret_cast<const void *>(&A2avArgsKernel<16, 64, STORE_THROUGH>),
+    reinterpret_cast<const void *>(&A2avTableKernel<8, 64, STORE_THROUGH>),
+    reinterpret_cast<const void *>(&A2avTableKernel<16, 64, STORE_THROUGH>),
     reinterpret_cast<const void *>(&A2avTableKernel<32, 64, STORE_THROUGH>),
     reinterpret_cast<const void *>(&A2avTableKernel<64, 64, STORE_THROUGH>),
-    reinterpret_cast<const void *>(&A2avArgsKernel<8, kBlockThreads, STORE_NT>),
-    reinterpret_cast<const void *>(&A2avArgsKernel<16, kBlockThreads, STORE_NT>),
+    reinterpret_cast<const void *>(&A2avTableKernel<8, kBlockThreads, STORE_NT>),
+    reinterpret_cast<const void *>(&A2avTableKernel<16, kBlockThreads, STORE_NT>),
     reinterpret_cast<const void *>(&A2avTableKernel<32, kBlockThreads, STORE_NT>),
     reinterpret_cast<const void *>(&A2avTableKernel<64, kBlockThreads, STORE_NT>),
+    reinterpret_cast<const void *>(&A2avArgsKernel<8, 64, STORE_THROUGH>),
+    reinterpret_cast<const void *>(&A2avArgsKernel<16, 64, STORE_THROUGH>),
+    reinterpret_cast<const void *>(&A2avArgsKernel<8, kBlockThreads, STORE_NT>),
+    reinterpret_cast<const void *>(&A2avArgsKernel<16, kBlockThreads, STORE_NT>),
 };
 #else
 #define HCCL_SHAPES(KERNEL, OP, SHAPE)                                                                                           \

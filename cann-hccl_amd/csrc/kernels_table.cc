@@ -6,7 +6,7 @@ namespace hcclamd {
 #define HCCL_DECL(name) extern const void *const kKernels_##name[4][KK_COUNT];
 HCCL_DECL(int8) HCCL_DECL(int16) HCCL_DECL(int32) HCCL_DECL(fp16) HCCL_DECL(fp32) HCCL_DECL(int64)
 HCCL_DECL(uint64) HCCL_DECL(uint8) HCCL_DECL(uint16) HCCL_DECL(uint32) HCCL_DECL(fp64) HCCL_DECL(bf16)
-extern const void *const kKernels_bytes[17];
+extern const void *const kKernels_bytes[21];
 
 const void *LookupKernel(int dt, int op, KernelKind kind)
 {
@@ -50,7 +50,7 @@ const void *LookupCopyKernel(KernelKind kind)
     if (kind == KK_PACKED_8 || kind == KK_PACKED_16 || kind == KK_PACKED_32) {
         return kKernels_bytes[6 + kind - KK_PACKED_8];
     }
-    if (kind >= KK_A2AV && kind < KK_A2AV + 8) {
+    if (kind >= KK_A2AV && kind < KK_A2AV_ARGS + 4) {
         return kKernels_bytes[9 + kind - KK_A2AV];
     }
     return nullptr;

@@ -201,7 +201,8 @@ uint64_t Extent(const uint32_t *at, const uint32_t *count, uint32_t p)
 HcclResult Complete(Group *g, A2avSet *s, uint32_t unit, bool *general)
 {
     const View v = ViewOf(s, g->p);
-    const uint32_t p = g->p;
+    const uint32_t p = g->p, unitShift = uint32_t(__builtin_ctz(unit));
+    s->unitShift = unitShift;
     HcclResult r = SidesAgree(g, *s, v);
     if (r != HCCL_SUCCESS) {
         return r;
@@ -246,7 +247,7 @@ HcclResult Complete(Group *g, A2avSet *s, uint32_t unit, bool *general)
             }
         }
     }
-    const uint32_t unitShift = uint32_t(__builtin_ctz(unit)), size = 1u << kA2avShift;
+    const uint32_t size = 1u << kA2avShift;
     uint64_t pieces = 0;
     for (uint32_t j = 0; j < v.stride; j++) {
         v.rowStart[j] = uint32_t(pieces);
@@ -262,7 +263,6 @@ HcclResult Complete(Group *g, A2avSet *s, uint32_t unit, bool *general)
     }
     total *= unit;
     s->pieces = uint32_t(pieces);
-    s->unitShift = unitShift;
     s->width = total <= kOneWaveTotal ? 0 : (total <= kTwoPerCuTotal ? 2 : 1);
     s->launches = uint32_t((total + kLaunchTotal - 1) / kLaunchTotal);
     s->moved = total;
@@ -311,7 +311,7 @@ bool A2avRow(Group *g, uint32_t r, void *send, void *recv, const uint64_t *const
         }
         const uint32_t to = Victim(g);
         A2avSet *s = &g->a2avSets[to];
-        s->valid = false;
+        s->valid = s->general = false;
         s->image.resize(ImageBytes(g->p));
         s->sent.resize(size_t(g->p) * g->p);
         s->place.resize(size_t(g->p) * g->p);
@@ -330,8 +330,11 @@ void A2avExpand(Group *g, uint32_t except)
 {
     const uint32_t p = g->p;
     A2avSet *s = g->a2avBuilding >= 0 ? &g->a2avSets[uint32_t(g->a2avBuilding)] : (g->a2avAlive != 0 ? &g->a2avSets[uint32_t(__builtin_ctz(g->a2avAlive))] : nullptr);
+    // (rows that are in pend's tables already leave what was found out about those as it is)
     std::vector<uint64_t> *tables[4] = {&g->pend.sendCounts, &g->pend.sdispls, &g->pend.recvCounts, &g->pend.rdispls};
+    bool same = true;
     for (std::vector<uint64_t> *t : tables) {
+        same = same && t->size() == size_t(p) * p;
         t->resize(size_t(p) * p);
     }
     for (uint32_t r = 0; s != nullptr && r < p; r++) {
@@ -341,11 +344,17 @@ void A2avExpand(Group *g, uint32_t except)
         const View v = ViewOf(s, p);
         const uint32_t *rows[4] = {s->sent.data() + size_t(r) * p, s->place.data() + size_t(r) * p, v.count + size_t(r) * v.stride, v.to + size_t(r) * v.stride};
         for (int k = 0; k < 4; k++) {
-            std::copy(rows[k], rows[k] + p, tables[k]->data() + size_t(r) * p);
+            uint64_t *to = tables[k]->data() + size_t(r) * p;
+            if (Differ(to, rows[k], p) != 0) {
+                std::copy(rows[k], rows[k] + p, to);
+                same = false;
+            }
         }
     }
-    g->tablesChecked = false;
-    g->lastA2av = nullptr;
+    if (!same) {
+        g->tablesChecked = false;
+        g->lastA2av = nullptr;
+    }
     g->a2avOpen = false;
 }
 
@@ -364,14 +373,20 @@ HcclResult A2avFinish(Group *g, hipStream_t stream, A2avSet **ready)
         A2avSet *s = &g->a2avSets[uint32_t(__builtin_ctz(g->a2avAlive))];
         s->hit = true;
         s->lastUse = ++g->a2avClock;
-        *ready = s;
+        *ready = s->general ? nullptr : s;
         return HCCL_SUCCESS;
     }
     A2avSet *s = &g->a2avSets[uint32_t(g->a2avBuilding)];
     bool general = false;
     HcclResult r = Complete(g, s, g->a2avUnit, &general);
-    if (r != HCCL_SUCCESS || general) {
+    if (r != HCCL_SUCCESS) {
         return r;
+    }
+    if (general) {
+        // (its tables and buffers say so: it will go that way whenever it comes back)
+        s->valid = s->general = true;
+        s->lastUse = ++g->a2avClock;
+        return HCCL_SUCCESS;
     }
     s->hit = false;
     *ready = s;

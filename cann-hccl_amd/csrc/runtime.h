@@ -242,6 +242,7 @@ struct A2avReader {
 };
 struct A2avSet {
     bool valid = false;               // a call that was issued: what follows belongs together
+    bool general = false;             // it goes the general way
     bool hit = false;                 // the call under way is this one
     std::vector<uint8_t> image;       // an A2avTable; up to 16 ranks an A2avArgs
     std::vector<uint32_t> sent, place;   // [sender][receiver]: the senders' counts and displacements (the image holds the receivers' counts)

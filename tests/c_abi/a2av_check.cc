@@ -1,7 +1,8 @@
 // The tables of all-to-all-v calls in device memory (cann-hccl_amd/csrc/a2av.cc), on the host: a seeded walk over calls of one group on a
 // model of streams and events (the first quarter of them on one stream), in which work is done as late as the orders allow, in any order they leave open.  Whenever a launch is done, the
 // tables it reads have to be those of its call.  The calls may not wait for the device, and a call known by its numbers counts as known on whatever
-// stream it comes.  argv[1] = ranks, argv[2] = calls, argv[3] = streams, argv[4] = sets of tables in turn.
+// stream it comes.  argv[1] = ranks, argv[2] = calls, argv[3] = streams, argv[4] = sets of tables in turn.  argv[2] = 0: calls that go the general
+// way instead.  Their tables have to come out as the ranks passed them, and what was found out about those has to hold as long as they are the last ones.
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
@@ -39,6 +40,8 @@ struct Event {
 };
 std::vector<Event> g_events(1);
 long g_deviceWaits = 0, g_hostWaits = 0, g_launches = 0, g_wrong = 0, g_records = 0, g_order = 0, g_inArguments = 0;
+bool g_stage = false;                           // the call's buffers overlap
+long g_overlapChecks = 0;
 const hcclamd::A2avSet *g_ready = nullptr;      // the call being launched
 std::vector<uint8_t> g_expected;                // its tables
 
@@ -165,7 +168,9 @@ hipError_t UploadFromPinned(void *dst, const void *pinned, size_t bytes, hipStre
 const void *LookupCopyKernel(KernelKind) { return &g_state; }
 HcclResult CheckOverlap(const Group *, const std::vector<uint64_t> &, const std::vector<uint64_t> &, bool *stage, bool *own)
 {
-    *stage = *own = false;
+    g_overlapChecks++;
+    *stage = g_stage;
+    *own = false;
     return HCCL_SUCCESS;
 }
 Prepared::~Prepared() = default;
@@ -173,6 +178,125 @@ Group::~Group() = default;
 }  // namespace hcclamd
 
 using namespace hcclamd;
+
+namespace {
+
+struct Tables {
+    std::vector<uint64_t> t[4];      // counts and displacements of the senders, of the receivers
+};
+Tables Draw(uint32_t p)
+{
+    Tables c;
+    for (std::vector<uint64_t> &t : c.t) {
+        t.resize(p * p);
+    }
+    for (uint64_t &n : c.t[0]) {
+        n = Below(5000);
+    }
+    for (uint32_t i = 0; i < p; i++) {
+        uint64_t at = 0, to = 0;
+        for (uint32_t j = 0; j < p; j++) {
+            c.t[1][i * p + j] = at;
+            c.t[3][i * p + j] = to;
+            c.t[2][i * p + j] = c.t[0][j * p + i];
+            at += c.t[0][i * p + j];
+            to += c.t[0][j * p + i];
+        }
+    }
+    return c;
+}
+
+// The ranks arrive; false as soon as one's row does not fit.  What Arrive does then, and for the ranks behind it, is done here too.
+bool Rows(Group *g, const Tables &c)
+{
+    const uint32_t p = g->p;
+    bool taken = true;
+    g->arrived = 0;
+    std::fill(g->here.begin(), g->here.end(), 0);
+    A2avBegin(g, 4);
+    for (uint32_t r = 0; r < p; r++) {
+        g->here[r] = 1;
+        const uint64_t *rows[4] = {&c.t[0][r * p], &c.t[1][r * p], &c.t[2][r * p], &c.t[3][r * p]};
+        if (taken && !A2avRow(g, r, reinterpret_cast<void *>(0x10000000ull + (uint64_t(r) << 24)), reinterpret_cast<void *>(0x7f0000000000ull + (uint64_t(r) << 24)), rows)) {
+            A2avExpand(g, r);
+            taken = false;
+        }
+        std::vector<uint64_t> *pend[4] = {&g->pend.sendCounts, &g->pend.sdispls, &g->pend.recvCounts, &g->pend.rdispls};
+        for (int k = 0; k < 4 && !taken; k++) {
+            uint64_t *row = pend[k]->data() + r * p;
+            if (!std::equal(rows[k], rows[k] + p, row)) {
+                std::copy(rows[k], rows[k] + p, row);
+                g->tablesChecked = false;
+                g->lastA2av = nullptr;
+            }
+        }
+        g->arrived++;
+    }
+    return taken;
+}
+
+int General(Group *g)
+{
+    const uint32_t p = g->p;
+    Tables a = Draw(p), b = Draw(p), far = Draw(p);
+    far.t[1][(p / 2) * p + 1] = uint64_t(1) << 40;      // (of a block that is empty)
+    far.t[0][(p / 2) * p + 1] = far.t[2][1 * p + p / 2] = 0;
+    Prepared *const prepared = reinterpret_cast<Prepared *>(uintptr_t(64));
+    // which tables, whether their buffers overlap, whether what is known of the last general call's tables has to hold
+    const struct {
+        const Tables *t;
+        bool stage, holds;
+    } calls[] = {{&a, true, false}, {&a, true, true}, {&b, false, true}, {&a, true, true}, {&far, false, false}, {&far, false, true}, {&b, false, true}, {&far, false, true},
+        {&a, true, false}, {&a, true, true}};
+    long checks = 0;
+    for (size_t n = 0; n < sizeof(calls) / sizeof(calls[0]); n++) {
+        g_stage = calls[n].stage;
+        const long before = g_overlapChecks;
+        A2avSet *ready = nullptr;
+        const bool rows = Rows(g, *calls[n].t);
+        if (rows && A2avFinish(g, reinterpret_cast<hipStream_t>(uintptr_t(1)), &ready) != HCCL_SUCCESS) {
+            std::printf("general call %zu: refused\n", n);
+            return 1;
+        }
+        checks += g_overlapChecks - before;
+        if (calls[n].t == &b) {
+            g_ready = ready;
+            if (ready != nullptr) {
+                g_expected.assign(ready->image.begin(), ready->image.begin() + 16);
+            }
+            if (ready == nullptr || A2avLaunch(g, ready, reinterpret_cast<hipStream_t>(uintptr_t(1))) != HCCL_SUCCESS) {
+                std::printf("general call %zu: an ordinary one not launched\n", n);
+                return 1;
+            }
+            continue;
+        }
+        if (ready != nullptr || rows != (calls[n].t == &a)) {
+            std::printf("general call %zu: taken\n", n);
+            return 1;
+        }
+        if (rows) {
+            A2avExpand(g, p);
+        }
+        const std::vector<uint64_t> *pend[4] = {&g->pend.sendCounts, &g->pend.sdispls, &g->pend.recvCounts, &g->pend.rdispls};
+        for (int k = 0; k < 4; k++) {
+            if (*pend[k] != calls[n].t->t[k]) {
+                std::printf("general call %zu: table %d is not what the ranks passed\n", n, k);
+                return 1;
+            }
+        }
+        if ((g->tablesChecked && g->lastA2av == prepared) != calls[n].holds) {
+            std::printf("general call %zu: what was known of its tables %s\n", n, calls[n].holds ? "is lost" : "was kept for others");
+            return 1;
+        }
+        g->tablesChecked = true;
+        g->lastA2av = prepared;
+    }
+    // (one look at each of the two sets of tables that fit: a's, b's)
+    std::printf("%s looked over %ld\n", checks == 2 ? "OK" : "BAD", checks);
+    return checks == 2 ? 0 : 1;
+}
+
+}  // namespace
 
 int main(int argc, char **argv)
 {
@@ -189,43 +313,21 @@ int main(int argc, char **argv)
         slot.host = std::calloc(1, 128 << 10);
         (void)hipEventCreateWithFlags(&slot.done, 0);
     }
+    if (calls == 0) {
+        return General(g);
+    }
     const size_t tableBytes = p <= 8 ? sizeof(A2avTable<8>) : p <= 16 ? sizeof(A2avTable<16>) : p <= 32 ? sizeof(A2avTable<32>) : sizeof(A2avTable<64>);
-    // calls: counts of set c, blocks one behind the other
-    std::vector<std::vector<uint64_t>> cnt(sets), back(sets), sd(sets), rd(sets);
+    std::vector<Tables> tables;
     for (uint64_t c = 0; c < sets; c++) {
-        cnt[c].resize(p * p);
-        back[c].resize(p * p);
-        sd[c].resize(p * p);
-        rd[c].resize(p * p);
-        for (uint64_t &n : cnt[c]) {
-            n = Below(5000);
-        }
-        for (uint32_t i = 0; i < p; i++) {
-            uint64_t at = 0, to = 0;
-            for (uint32_t j = 0; j < p; j++) {
-                sd[c][i * p + j] = at;
-                rd[c][i * p + j] = to;
-                back[c][i * p + j] = cnt[c][j * p + i];
-                at += cnt[c][i * p + j];
-                to += cnt[c][j * p + i];
-            }
-        }
+        tables.push_back(Draw(p));
     }
     long known = 0, shouldKnow = 0;
     std::deque<uint64_t> latest;        // the last distinct calls
     for (long n = 0; n < calls; n++) {
         const uint64_t c = Below(3) ? Below(sets) : uint64_t(n) % sets, stream = n < calls / 4 ? 1 : 1 + (Below(2) ? Below(streams) : uint64_t(n) % streams);
-        g->arrived = 0;
-        std::fill(g->here.begin(), g->here.end(), 0);
-        A2avBegin(g, 4);
-        for (uint32_t r = 0; r < p; r++) {
-            g->here[r] = 1;
-            const uint64_t *rows[4] = {&cnt[c][r * p], &sd[c][r * p], &back[c][r * p], &rd[c][r * p]};
-            if (!A2avRow(g, r, reinterpret_cast<void *>(0x10000000ull + (uint64_t(r) << 24)), reinterpret_cast<void *>(0x7f0000000000ull + (uint64_t(r) << 24)), rows)) {
-                std::printf("a row not taken\n");
-                return 1;
-            }
-            g->arrived++;
+        if (!Rows(g, tables[c])) {
+            std::printf("a row not taken\n");
+            return 1;
         }
         A2avSet *ready = nullptr;
         if (A2avFinish(g, reinterpret_cast<hipStream_t>(stream), &ready) != HCCL_SUCCESS || ready == nullptr) {

@@ -29,3 +29,9 @@ def check(tmp_path_factory):
 def test_tables_of_several_streams(check, ranks, calls, streams, sets):
     out = subprocess.run([check, str(ranks), str(calls), str(streams), str(sets)], stdout=subprocess.PIPE, text=True, timeout=120)
     assert out.returncode == 0 and out.stdout.startswith("OK"), out.stdout
+
+
+@pytest.mark.parametrize("ranks", [2, 8, 13, 40, 64])
+def test_calls_that_go_the_general_way(check, ranks):
+    out = subprocess.run([check, str(ranks), "0"], stdout=subprocess.PIPE, text=True, timeout=120)
+    assert out.returncode == 0 and out.stdout.startswith("OK"), out.stdout

@@ -206,6 +206,21 @@ bool BuildDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLau
 
 namespace {
 
+// Whether the KiB of an item go to the XCDs in fours (KiBOf, kernels_direct.h): `total` bytes in `items` items of more than 8 ranks.  Us, workgroups of 4 KiB / of
+// KiB one by one / in fours: reduce of 2 MiB, fp32, 16 ranks 7.4 / 7.7 / 6.9, 24 ranks 9.9 / 10.8 / 9.8, 32 ranks 12.8 / 13.9 / 12.7, bf16, 16 ranks 7.1 / 8.0 / 7.5; but 12 ranks,
+// whose buffers of 1.5 and 2 MiB stay apart, 5.1 / 4.6 / 4.8 and 5.5 / 5.3 / 5.6.  Reduce-scatter (results in all), fp32, 12 ranks 2 MiB 6.5 / 6.3 / 5.8, 2.5 MiB 7.0 / 7.3 /
+// 6.8, 16 ranks 2 MiB 8.1 / 7.7 / 6.9, 24 ranks 2.5 MiB 12.5 / 12.8 / 11.8; bf16, 12 ranks 3.5 MiB 10.0 / 10.0 / 9.4, but 16 ranks 2.5 MiB 8.5 / 8.7 / 8.8, 3.5 MiB 11.4 / 11.7 /
+// 12.1.  All-reduce, 32 ranks 512 KiB 8.1 / 7.7 / 6.8 (with both batches of sources in flight); 16 ranks 768 KiB 6.3 / 5.0 / 5.2.  Up to 8 sources it makes no difference;
+// copies lose (20 MiB read and written 4.2 / 4.6).
+bool PackedInFours(uint32_t p, uint32_t items, bool toOne, uint64_t total, int dtype)
+{
+    if (p > 16 || !toOne) {
+        return p > 16;
+    }
+    const bool halves = dtype == HCCL_DATA_TYPE_FP16 || dtype == HCCL_DATA_TYPE_BFP16;
+    return items > 1 ? p < 16 || !halves || total <= uint64_t(9) << 18 : p == 16;
+}
+
 // Arguments of `P` ranks out of items of `nsrc` sources each, already found alike.
 template <uint32_t P> void FillPacked(const Plan &plan, const std::vector<uint32_t> &order, uint32_t info, DirectLaunch *d)
 {
@@ -330,8 +345,13 @@ void PackDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaun
     if (!tree && order.size() > 1 && !left && !ring) {
         return;
     }
+    uint64_t total = 0;
+    for (const FusedItem &it : plan.fused) {
+        total += it.bytes;
+    }
+    const bool fours = reduceColl && p > 8 && PackedInFours(p, n, toOne, total, dtype);
     const uint32_t info = uint32_t(order.size()) << kPackedSources | n << kPackedItems | p << kPackedModulus | (tree ? kPackedTree : 0u) |
-        (toOne ? kPackedToOne : 0u) | (ends ? kPackedEnds : 0u) | (!tree && !left ? kPackedRing : 0u);
+        (toOne ? kPackedToOne : 0u) | (fours ? kPackedFours : 0u) | (ends ? kPackedEnds : 0u) | (!tree && !left ? kPackedRing : 0u);
     KernelKind kind = KK_PACKED_8;
     if (p <= 8) {
         FillPacked<8>(plan, order, info, d);
@@ -341,10 +361,6 @@ void PackDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaun
     } else {
         FillPacked<32>(plan, order, info, d);
         kind = KK_PACKED_32;
-    }
-    uint64_t total = 0;
-    for (const FusedItem &it : plan.fused) {
-        total += it.bytes;
     }
     const uint32_t shape = PackedShape(uint32_t(order.size()));
     bool wide = false;

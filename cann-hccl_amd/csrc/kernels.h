@@ -199,6 +199,7 @@ constexpr uint32_t kPackedSources = 0, kPackedItems = 6, kPackedModulus = 12, kP
 constexpr uint32_t kPackedTree = 1u << 24;      // pairwise bottom-up over the sources; else a chain
 constexpr uint32_t kPackedToOne = 1u << 25;     // one destination, the item's rank; else one to every rank of the modulus
 constexpr uint32_t kPackedEnds = 1u << 26;      // some item ends in a part of a vector
+constexpr uint32_t kPackedFours = 1u << 28;     // KiB in fours to the XCDs (more than 8 ranks)
 constexpr uint32_t kPackedRing = 1u << 27;      // chain: sources behind the second one are the left operands; else the right ones
 
 // Kernel entry for (data type, reduce op, kind); nullptr if the combination is not built.

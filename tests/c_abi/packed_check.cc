@@ -21,7 +21,7 @@ using namespace hcclamd;
 
 namespace {
 
-long g_wide = 0;
+long g_wide = 0, g_fours = 0;
 uint64_t g_state = 0x9E3779B97F4A7C15ull;
 uint64_t Below(uint64_t n)
 {
@@ -133,7 +133,8 @@ template <uint32_t P> bool Same(const Plan &plan, const DirectLaunch &d, const s
         return false;
     }
     const uint32_t ends = (k.info & kPackedEnds) ? 1 : 0;
-    bool ok = ((k.info >> kPackedItems) & 63u) == plan.fused.size() && d.gridY == plan.fused.size();
+    g_fours += (k.info & kPackedFours) != 0;
+    bool ok = (P > 8 || !(k.info & kPackedFours)) && ((k.info >> kPackedItems) & 63u) == plan.fused.size() && d.gridY == plan.fused.size();
     for (uint32_t i = 0; ok && i < plan.fused.size(); i++) {
         const Item a = OfPlan(plan.fused[i], send, recv), b = OfArguments<P>(k, i, &ok);
         ok = ok && a.bytes == b.bytes && a.value == b.value && a.dst == b.dst && (a.bytes % 16 == 0 || ends) &&
@@ -221,7 +222,7 @@ int main(int argc, char **argv)
             taken[d.packedRanks == 8 ? 0 : d.packedRanks == 16 ? 1 : 2]++;
         }
     }
-    std::printf("OK up to 8 ranks %ld 16 ranks %ld 32 ranks %ld trees %ld in place %ld unlike %ld too far apart %ld wide %ld\n", taken[0], taken[1], taken[2], trees,
-        inPlace, unlike, apart, g_wide);
+    std::printf("OK up to 8 ranks %ld 16 ranks %ld 32 ranks %ld trees %ld in place %ld unlike %ld too far apart %ld wide %ld in fours %ld\n", taken[0], taken[1], taken[2], trees,
+        inPlace, unlike, apart, g_wide, g_fours);
     return 0;
 }

@@ -3,6 +3,7 @@ its own (2, 4, 8, 16 sources; chains of either operand order, trees), other numb
 vector, in place, off a boundary, up to and beyond the sizes where the tile kernels take over."""
 import numpy as np
 import pytest
+import torch
 
 import closed_forms as cf
 import gpu_harness as gh
@@ -98,3 +99,42 @@ def test_blocks(orc, p):
                         assert np.array_equal(outs[r].view(np.uint8), np.concatenate(parts).view(np.uint8)), ("all-gather", dt, n, r)
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("p", [9, 15, 16, 17, 24, 25, 31, 32])
+def test_many_sources(orc, p):
+    """More than 8 sources: KiB that go to the XCDs in fours (whole groups of 32, and what is left of one), two batches of sources in flight."""
+    groups = {a: gh.Group(p, algo=a) for a in ("ring", "mesh")}
+    if p in (16, 24):
+        groups["rhd"] = gh.Group(p, algo="rhd")
+    try:
+        for k, (dt, op, pad, special) in enumerate([(FP32, SUM, 0, False), (BF16, MIN, 2, True), (FP16, MAX, 6, True), (INT8, SUM, 1, False)]):
+            unit = gh.H.DTYPE_SIZE[dt]
+            for size in (32 * 1024 - 16, 32 * 1024, 32 * 1024 + 16 * (k % 2) + unit, 65 * 1024 + 48 + unit):
+                n = size // unit
+                for name, g in groups.items():
+                    algo = {"ring": RING, "mesh": MESH, "rhd": RHD}[name]
+                    print("many sources", p, name, "type", dt, "n", n, flush=True)
+                    ins = _ins(dt, p, n * p, 5 * p + n % 811 + k, special)
+                    want = orc.reducescatter(ins, dt, op, algo=algo)
+                    outs, _ = gh.reduce_scatter(g, ins, dt, op, pad=pad)
+                    assert g.info()["direct"] == 1 and g.info()["launches"] == 1
+                    for r in range(p):
+                        assert gh.same(dt, outs[r], want[r]), ("reduce-scatter", name, dt, n, r)
+                    parts = [x[:n] for x in ins]
+                    root = n % p
+                    src, dst = [gh.to_dev(x, pad) for x in parts], [gh.empty_dev(n * unit, pad) for _ in range(p)]
+                    torch.cuda.synchronize()
+                    gh.H.reduce(g.comms, [t.data_ptr() for t in src], [t.data_ptr() for t in dst], n, dt, op, root, g.stream_ptr)
+                    g.stream.synchronize()
+                    assert g.info()["direct"] == 1 and g.info()["launches"] == 1
+                    assert gh.same(dt, gh.to_host(dst[root], dt), orc.reduce_to_root(parts, dt, op, root, algo=algo)), ("reduce", name, dt, n)
+                    if size < 33 * 1024 and name == "ring":
+                        whole = [x[:min(n * p, MIB // unit)] for x in ins]     # (an item of every rank's, as in the others)
+                        want = orc.allreduce(whole, dt, op, algo=algo)
+                        outs, _ = gh.all_reduce(g, whole, dt, op, pad=pad)
+                        for r in range(p):
+                            assert gh.same(dt, outs[r], want[r]), ("all-reduce", dt, n, r)
+    finally:
+        for g in groups.values():
+            g.close()

@@ -32,10 +32,13 @@ namespace {
         }                                                                                             \
     } while (0)
 
-// How wide (bytes moved in all).  Three sets of tables in turn, us, workgroups of one wave, written through / two of four waves per CU / one of them:
-// 16 ranks 7 MB 4.5 / 5.0 / 5.3, 22 MB 9.1 / 9.8 / 10.4; 98 MB 34.5 / 35.1 / 35.1; 64 ranks 103 MB - / 38.6 / 39.2; 8 ranks 112 MB 43.5 / 40.7 / 41.0, 377 MB
-// 142.9 / 134.9 / 131.7; 16 ranks 392 MB 141 / 135.3 / 132.2; 32 ranks 426 MB 155 / 146.8 / 142.7.
-constexpr uint64_t kOneWaveTotal = uint64_t(32) << 20, kTwoPerCuTotal = uint64_t(128) << 20;
+// How wide (bytes moved in all).  Three sets of buffers and tables in turn, us, 16 workgroups of one wave per CU, written through / two of four waves, non-temporal / one of
+// them.  While what is read and written stays in the memory-side cache, the first: lognormal blocks, 16 ranks 26 MiB 10.7 / 11.8 / 12.1, 60 MiB 21.7 / 23.3 / 23.7, 90 MiB 31.0 / 33.5
+// / 33.7, 95 MiB 33.1 / 35.1 / -, 100 MiB 36.7 / 37.0 / -, 105 MiB 39.3 / 38.3 / -; 64 ranks 90 MiB 32.8 / 36.6 / 36.9, 100 MiB 39.9 / 40.7 / -, 110 MiB 44.7 / 44.3 / -; uniform,
+// 8 ranks 60 MiB 20.3 / 22.1 / 22.5, 95 MiB 31.9 / 33.5 / -, 100 MiB 34.5 / 35.3 / -, 105 MiB 37.9 / 37.0 / -.  Beyond, two; one for more than 16 ranks from 128 MiB on: uniform, 4 ranks
+// 512 MiB 182 / 173.5 / 175.3, 8 ranks 512 MiB 182 / 172.8 / 174.7, 2 GiB 723 / 696 / 700, 16 ranks 2 GiB 730 / 704 / 711, but 32 ranks 512 MiB 192 / 188 / 179, 2 GiB 742 / 712 / 699;
+// lognormal, 16 ranks 424 MiB - / 148.7 / 148.1, 32 ranks - / 154.8 / 152.4, 64 ranks 310 MiB - / 119.0 / 117.0.
+constexpr uint64_t kOneWaveTotal = uint64_t(96) << 20, kTwoPerCuTotal = uint64_t(128) << 20;
 constexpr uint64_t kLaunchTotal = uint64_t(256) << 20;    // in one launch (as other collectives that hop from buffer to buffer)
 
 // The image's tables, wherever they lie for the group's number of ranks.
@@ -263,7 +266,7 @@ HcclResult Complete(Group *g, A2avSet *s, uint32_t unit, bool *general)
     }
     total *= unit;
     s->pieces = uint32_t(pieces);
-    s->width = total <= kOneWaveTotal ? 0 : (total <= kTwoPerCuTotal ? 2 : 1);
+    s->width = total <= kOneWaveTotal ? 0 : (p <= 16 || total <= kTwoPerCuTotal ? 2 : 1);
     s->launches = uint32_t((total + kLaunchTotal - 1) / kLaunchTotal);
     s->moved = total;
     return HCCL_SUCCESS;

@@ -85,9 +85,9 @@ def test_shapes(p):
         g.close()
 
 
-@pytest.mark.parametrize("p,mib", [(8, 40), (16, 40), (4, 600), (32, 48)])
+@pytest.mark.parametrize("p,mib", [(8, 40), (16, 40), (4, 600), (32, 48), (8, 100), (16, 100), (32, 100), (48, 140)])
 def test_large(p, mib):
-    # beyond 32 MiB in all workgroups of four waves, beyond 256 MiB several launches
+    # beyond 96 MiB in all workgroups of four waves, beyond 256 MiB several launches
     rng = np.random.default_rng(77)
     g = gh.Group(p)
     try:

@@ -273,70 +273,28 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
             (coll == COLL_REDUCESCATTER && g->cfg.servers <= 1);
         capBytes = hops ? uint64_t(512) << 20 : 0;
     }
-    // Launch width.  Streaming kernels on this part run best with few, fat workgroups as long as a
-    // lane keeps enough memory operations in flight: 1 workgroup per CU when an item touches 8 or
-    // more streams (sources + destinations), more when it touches fewer (measured on MI355X: 8 -> 8
-    // all-reduce and 1 -> 8 all-gather best at 1 per CU, the 2 -> 1 step kernel at 2 per CU).
     const uint32_t stepGrid = std::max(1u, g->numCu * (g->cfg.blocksPerCu ? g->cfg.blocksPerCu : 2u));
     uint32_t fusedPerCu = g->cfg.blocksPerCu;
     if (fusedPerCu == 0) {
-        constexpr double kMiB = 1024.0 * 1024.0;
-        double streamBytes = 0, storeBytes = 0, bytes = 0;
+        FusedShape shape;
         for (const FusedItem &it : pp->plan->fused) {
             uint32_t nsrc = 0;
             for (uint8_t v : it.srcValid) {
                 nsrc += v;
             }
-            streamBytes += double(nsrc + it.dst.size()) * double(it.bytes);
-            storeBytes += double(it.dst.size()) * double(it.bytes);
-            bytes += double(it.bytes);
+            shape.streamBytes += double(nsrc + it.dst.size()) * double(it.bytes);
+            shape.storeBytes += double(it.dst.size()) * double(it.bytes);
+            shape.bytes += double(it.bytes);
+            shape.sources = std::max(shape.sources, nsrc);
         }
-        double streams = bytes > 0 ? streamBytes / bytes : 2.0;   // loads + stores per lane and vector
-        fusedPerCu = streams >= 8.0 ? 1u : (streams >= 3.0 ? 2u : 4u);
-        // Many sources into one destination (reduce-scatter, reduce).  Beyond the memory-side cache few workgroups keep the
-        // sources' streams apart, below it many hide the latency of a combine, which for elements of one and two bytes takes
-        // several instructions.  Three sets of buffers in turn, us, 1 / 2 / 8 per CU: 8 ranks in a ring bf16 sum of 64 MiB 93.2 / 98 / 99.3,
-        // 256 MiB 376 / - / 401, fp32 93.0 / 97.3 / 96.5, int8 96.8 / 95.6 / 98.7; 16 ranks x 32 MiB fp16 87 / - / 94; bf16 of 48 MiB 73.3 / 70.1 / 72.0, of 32
-        // MiB 49.5 / 49.0 / 47.5; 4 ranks x 128 MiB bf16 105.6 / 108.9 / -, fp32 105.4 / 110.1 / -, but 5 ranks x 100 MiB 110.3 / 101.3 / -.
-        const bool manyToOne = reduceColl && storeBytes * 5.0 <= streamBytes;
-        const bool toOne = manyToOne && !pp->plan->fused.empty() && pp->plan->fused[0].kind == FK_CHAIN && (fusedPerCu == 1 || (streams <= 5.0 && streamBytes > 512.0 * kMiB));
-        if (toOne) {
-            const bool bytewise = DtypeSize(dtype) == 1;
-            fusedPerCu = streamBytes > 512.0 * kMiB ? (bytewise ? 2u : 1u) : streamBytes > 320.0 * kMiB ? 2u : DtypeSize(dtype) <= 2 ? 8u : 2u;
-        }
-        // Trees and stack programs, whose combines are more of the work, gain nothing from few (fp32 tree of 8 x 64 MiB 1 / 2 per CU 101 / 99) and keep many for
-        // elements of one and two bytes up to about a gigabyte (two servers, 8 ranks, bf16 40 MiB 2 / 8 per CU 63.8 / 62.2).
-        const double launchBytes = capBytes != 0 ? std::min(streamBytes, double(capBytes)) : streamBytes;
-        if (manyToOne && !toOne && fusedPerCu == 1 && DtypeSize(dtype) <= 2 && launchBytes <= 1280.0 * kMiB) {
-            fusedPerCu = 8;
-        }
-        // Blocks of several sources into two or more destinations each (all-gather) without the teams: many workgroups as long as the results stay in
-        // the memory-side cache, and again far beyond it where there are fewer than 7 destinations (three sets in turn, us, 1 or 2 / 8 per CU,
-        // bytes moved in parentheses: 8 ranks 256 KiB 4.6 / 4.1, 2 MiB 26.4 / 25.6, 3 MiB 42.7 / 40.5; 4 ranks 4 MiB (80 MiB) 13.7 / 13.0, 8 MiB (160)
-        // 30.9 / 30.1, 16 MiB (320) 61.5 / 63, 40 MiB (800) 150 / 144; 3 ranks 8 MiB (96) 17.2 / 16.3, 13 MiB (156) 30.3 / 31.2, 24 MiB (288) 54.6 / 55.7,
-        // 64 MiB (768) 145 / 138, 96 MiB 213 ... 239 / 217 ... 229; 5 ranks 7 MiB (210) 43.0 / 43.5, 40 MiB (1200) 215 / 206; 2 ranks 64 MiB (384) 73 / 70.5, 112 MiB
-        // (672) 129 / 121, 128 MiB 139 / 140).  A broadcast sweeps one source and is left at two: 3 ranks 32 MiB 14.3 / 15.2, 4 ranks 256 MiB 176 / 185, 6 ranks 100
-        // MiB 110 / 113.
-        const double cached = (streams >= 8.0 ? 256.0 : 128.0) * kMiB;
-        if (g->ctx->sig.coll == COLL_ALLGATHER && streams >= 3.0 && (streams <= 3.0 || streamBytes <= cached || (streams < 8.0 && streamBytes > 512.0 * kMiB))) {
-            fusedPerCu = 8u;
-        }
-        // Plain copies (one source, one destination) go through the copy kernel, which really gets the
-        // occupancy it is launched with; with non-temporal stores more workgroups only widen the range
-        // of addresses written at a time, which this memory system likes less (measured, 8 ranks:
-        // uniform all-to-all of 32 MiB per pair 752 us at 1 or 2 per CU, 835 us at 4, 850 us at 8;
-        // 16-rank all-to-all-v, 106 MB of ragged segments: 55.6 / 40.5 / 42.5 / 41.3 us at 1 / 2 / 4 / 8).
-        if (!reduceColl && streams < 3.0) {
-            fusedPerCu = 2u;
-        }
-        // few tiles per workgroup: a second workgroup per CU evens out the tail (measured: 16-rank
-        // ring all-reduce of 32 MiB per rank 241 us at 1 per CU, 220 us at 2), eight do so better between 3 and 16 tiles per CU
-        // (at 2 / 8: 4 ranks 32 MiB 47.1 / 44.5, 48 MiB 70.1 / 69.0; 8 ranks 15.9 MiB bf16 maximum 46.4 / 43.8; 16 ranks 12 MiB 71.1 / 67.2;
-        // 8 ranks 10 MiB, 2.5 tiles, 29.0 / 30.8; 4 ranks 64 MiB equal, int8 26 MiB 37.3 / 39.0)
-        if (fusedPerCu == 1 && !toOne && bytes / kTileBytes < 32.0 * g->numCu) {
-            const double tilesPerCu = bytes / kTileBytes / g->numCu;
-            fusedPerCu = reduceColl && DtypeSize(dtype) > 1 && tilesPerCu >= 3.0 && tilesPerCu < 16.0 ? 8 : 2;
-        }
+        shape.reduces = reduceColl;
+        shape.chains = !pp->plan->fused.empty() && pp->plan->fused[0].kind == FK_CHAIN;
+        shape.allGather = g->ctx->sig.coll == COLL_ALLGATHER;
+        shape.reduceScatter = g->ctx->sig.coll == COLL_REDUCESCATTER;
+        shape.unit = DtypeSize(dtype);
+        shape.capBytes = capBytes;
+        shape.numCu = g->numCu;
+        fusedPerCu = FusedPerCu(shape);
     }
     const uint32_t treeGrid = std::max(1u, g->numCu * fusedPerCu);
     const uint32_t fusedGrid = std::max(1u, g->numCu * fusedPerCu);

@@ -149,4 +149,85 @@ inline uint32_t StoreFlags(int setting, bool reduces, bool team, uint64_t traffi
     return (reduces ? ResultsWriteThrough(traffic, written, moved) : CopiesWriteThrough(traffic, written, moved)) ? kFusedThroughStores : kFusedNtStores;
 }
 
+// What the width of a launch of the plain fused kernels goes by, summed over a collective's items.
+struct FusedShape {
+    double streamBytes = 0;     // read and written
+    double storeBytes = 0;      // written
+    double bytes = 0;           // of the items themselves
+    bool reduces = false, chains = false;          // a reduction; of chains (else of trees or stack programs)
+    bool allGather = false, reduceScatter = false;
+    uint32_t sources = 0;       // of an item
+    uint32_t unit = 1;          // bytes of an element
+    uint64_t capBytes = 0;      // read and written by one launch, 0: by all
+    uint32_t numCu = 256;
+};
+
+// Workgroups per CU.  Streaming kernels on this part run best with few, fat workgroups as long as a
+// lane keeps enough memory operations in flight: 1 workgroup per CU when an item touches 8 or
+// more streams (sources + destinations), more when it touches fewer (measured on MI355X: 8 -> 8
+// all-reduce and 1 -> 8 all-gather best at 1 per CU, the 2 -> 1 step kernel at 2 per CU).
+inline uint32_t FusedPerCu(const FusedShape &f)
+{
+    constexpr double kMiB = 1024.0 * 1024.0;
+    const double streams = f.bytes > 0 ? f.streamBytes / f.bytes : 2.0;   // loads + stores per lane and vector
+    uint32_t perCu = streams >= 8.0 ? 1u : (streams >= 3.0 ? 2u : 4u);
+    // Many sources into one destination (reduce-scatter, reduce).  Beyond the memory-side cache few workgroups keep the
+    // sources' streams apart, below it many hide the latency of a combine, which for elements of one and two bytes takes
+    // several instructions.  Three sets of buffers in turn, us, 1 / 2 / 8 per CU: 8 ranks in a ring bf16 sum of 64 MiB 93.2 / 98 / 99.3,
+    // 256 MiB 376 / - / 401, fp32 93.0 / 97.3 / 96.5, int8 96.8 / 95.6 / 98.7; 16 ranks x 32 MiB fp16 87 / - / 94; bf16 of 48 MiB 73.3 / 70.1 / 72.0, of 32
+    // MiB 49.5 / 49.0 / 47.5; 4 ranks x 128 MiB bf16 105.6 / 108.9 / -, fp32 105.4 / 110.1 / -, but 5 ranks x 100 MiB 110.3 / 101.3 / -.
+    // Many more sources (MiB read in all): fp32 reduce, 24 ranks 600 MiB 103.8 / 103.5, 32 ranks 2400 MiB 413.6 / 408.6, 48 ranks 408.2 / 391.1, 64 ranks 402.8 / 386.4,
+    // reduce-scatter, 24 ranks 441.2 / 435.3, 40 ranks 2600 MiB 454.9 / 448.8, 60 ranks 496.7 / 482.7 (16 ranks 436.0 / 435.1).  Reduce-scatters, whose many items are short
+    // then: bf16, 28 ranks 2600 MiB 434 / 458 / 494, 48 ranks 440 / 458 / 470, 52 ranks 439 / 452 / 463, 56 ranks 512 / 521 / 509, 60 ranks 514 / 517 / 500, 64 ranks 560
+    // MiB 143 / 142 / 134, 2600 MiB 500 / 513 / 487; int8, 36 ranks 537 / 449 / 469, 40 ranks 539 / 427 / 454, 44 ranks 900 MiB 189 / 173 / 158, 1500 MiB 288 / 262 / 247, 48 ranks
+    // 400 MiB 98 / 87 / 76, 2600 MiB 520 / 472 / 438, 64 ranks 593 / 533 / 465.
+    const bool manyToOne = f.reduces && f.storeBytes * 5.0 <= f.streamBytes;
+    const bool toOne = manyToOne && f.chains && (perCu == 1 || (streams <= 5.0 && f.streamBytes > 512.0 * kMiB));
+    if (toOne) {
+        if (f.unit == 1 && f.reduceScatter && f.sources > 40 && f.streamBytes > 320.0 * kMiB) {
+            perCu = 8u;
+        } else if (f.streamBytes > 512.0 * kMiB) {
+            perCu = f.unit == 1 ? 2u : f.unit == 2 ? (f.reduceScatter && f.sources > 52 ? 8u : 1u) : (f.sources >= 24 ? 2u : 1u);
+        } else {
+            perCu = f.streamBytes > 320.0 * kMiB ? 2u : f.unit <= 2 ? 8u : 2u;
+        }
+    }
+    // Trees and stack programs, whose combines are more of the work, gain nothing from few (fp32 tree of 8 x 64 MiB 1 / 2 per CU 101 / 99) and keep many for
+    // elements of one and two bytes up to about a gigabyte (two servers, 8 ranks, bf16 40 MiB 2 / 8 per CU 63.8 / 62.2).
+    const double launchBytes = f.capBytes != 0 ? std::min(f.streamBytes, double(f.capBytes)) : f.streamBytes;
+    if (manyToOne && !toOne && perCu == 1 && f.unit <= 2 && launchBytes <= 1280.0 * kMiB) {
+        perCu = 8;
+    }
+    // Blocks of several sources into two or more destinations each (all-gather) without the teams: many workgroups as long as the results stay in
+    // the memory-side cache, and again far beyond it where there are fewer than 7 destinations (three sets in turn, us, 1 or 2 / 8 per CU,
+    // bytes moved in parentheses: 8 ranks 256 KiB 4.6 / 4.1, 2 MiB 26.4 / 25.6, 3 MiB 42.7 / 40.5; 4 ranks 4 MiB (80 MiB) 13.7 / 13.0, 8 MiB (160)
+    // 30.9 / 30.1, 16 MiB (320) 61.5 / 63, 40 MiB (800) 150 / 144; 3 ranks 8 MiB (96) 17.2 / 16.3, 13 MiB (156) 30.3 / 31.2, 24 MiB (288) 54.6 / 55.7,
+    // 64 MiB (768) 145 / 138, 96 MiB 213 ... 239 / 217 ... 229; 5 ranks 7 MiB (210) 43.0 / 43.5, 40 MiB (1200) 215 / 206; 2 ranks 64 MiB (384) 73 / 70.5, 112 MiB
+    // (672) 129 / 121, 128 MiB 139 / 140).  A broadcast sweeps one source and is left at two: 3 ranks 32 MiB 14.3 / 15.2, 4 ranks 256 MiB 176 / 185, 6 ranks 100
+    // MiB 110 / 113.
+    const double cached = (streams >= 8.0 ? 256.0 : 128.0) * kMiB;
+    if (f.allGather && streams >= 3.0 && (streams <= 3.0 || f.streamBytes <= cached || (streams < 8.0 && f.streamBytes > 512.0 * kMiB))) {
+        perCu = 8u;
+    }
+    // Plain copies (one source, one destination) go through the copy kernel, which really gets the
+    // occupancy it is launched with; with non-temporal stores more workgroups only widen the range
+    // of addresses written at a time, which this memory system likes less (measured, 8 ranks:
+    // uniform all-to-all of 32 MiB per pair 752 us at 1 or 2 per CU, 835 us at 4, 850 us at 8;
+    // 16-rank all-to-all-v, 106 MB of ragged segments: 55.6 / 40.5 / 42.5 / 41.3 us at 1 / 2 / 4 / 8).
+    if (!f.reduces && streams < 3.0) {
+        perCu = 2u;
+    }
+    // few tiles per workgroup: a second workgroup per CU evens out the tail (measured: 16-rank
+    // ring all-reduce of 32 MiB per rank 241 us at 1 per CU, 220 us at 2), eight do so better between 3 and 16 tiles per CU
+    // (at 2 / 8: 4 ranks 32 MiB 47.1 / 44.5, 48 MiB 70.1 / 69.0; 8 ranks 15.9 MiB bf16 maximum 46.4 / 43.8; 16 ranks 12 MiB 71.1 / 67.2;
+    // 8 ranks 10 MiB, 2.5 tiles, 29.0 / 30.8; 4 ranks 64 MiB equal, int8 26 MiB 37.3 / 39.0), trees and stack programs only up to 4 (halving-doubling: 4 ranks
+    // bf16 12.8 MiB 21.0 / 20.1, 16 MiB 23.5 / 24.2, 24 MiB 35.8 / 36.4, 32 MiB 47.5 / 48.5, 16 ranks 12.8 MiB 85.0 / 84.4; two servers: 4 ranks 12.8 MiB
+    // 21.0 / 20.1, 16 MiB 23.5 / 24.1, 32 MiB 47.4 / 48.5).
+    if (perCu == 1 && !toOne && f.bytes / kTileBytes < 32.0 * f.numCu) {
+        const double tilesPerCu = f.bytes / kTileBytes / f.numCu;
+        perCu = f.reduces && f.unit > 1 && tilesPerCu >= 3.0 && tilesPerCu < (f.chains ? 16.0 : 4.0) ? 8 : 2;
+    }
+    return perCu;
+}
+
 }  // namespace hcclamd

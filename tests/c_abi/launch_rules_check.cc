@@ -115,6 +115,42 @@ void CheckStores()
     }
 }
 
+// Workgroups per CU on either side of the lines.
+void CheckWidth()
+{
+    auto width = [](bool scatter, uint32_t ranks, uint32_t unit, double mibRead) {
+        FusedShape f;
+        f.reduces = f.chains = true;
+        f.reduceScatter = scatter;
+        f.sources = ranks;
+        f.unit = unit;
+        f.bytes = mibRead * 1048576.0 / ranks;
+        f.storeBytes = f.bytes;
+        f.streamBytes = f.bytes * (ranks + 1);
+        f.capBytes = scatter ? uint64_t(512) << 20 : 0;
+        return FusedPerCu(f);
+    };
+    for (bool scatter : {false, true}) {
+        CHECK(width(scatter, 8, 4, 512) == 1 && width(scatter, 23, 4, 2400) == 1 && width(scatter, 24, 4, 600) == 2 && width(scatter, 64, 8, 2400) == 2);
+        CHECK(width(scatter, 8, 2, 512) == 1 && width(scatter, 52, 2, 2400) == 1 && width(scatter, 53, 2, 2400) == (scatter ? 8u : 1u));
+        CHECK(width(scatter, 8, 1, 600) == 2 && width(scatter, 40, 1, 2400) == 2 && width(scatter, 41, 1, 2400) == (scatter ? 8u : 2u));
+        CHECK(width(scatter, 48, 1, 330) == (scatter ? 8u : 2u) && width(scatter, 48, 1, 300) == 8 && width(scatter, 48, 2, 300) == 8 && width(scatter, 48, 4, 300) == 2);
+    }
+    auto mid = [](bool chains, uint32_t unit, double tilesPerCu) {
+        FusedShape f;
+        f.reduces = true;
+        f.chains = chains;
+        f.sources = 4;
+        f.unit = unit;
+        f.bytes = tilesPerCu * 256 * kTileBytes;
+        f.storeBytes = f.bytes * 4;
+        f.streamBytes = f.bytes * 8;
+        return FusedPerCu(f);
+    };
+    CHECK(mid(true, 4, 2.9) == 2 && mid(true, 4, 3.1) == 8 && mid(true, 2, 15.9) == 8 && mid(true, 2, 16.1) == 2 && mid(true, 1, 8) == 2 && mid(true, 4, 33) == 1);
+    CHECK(mid(false, 4, 2.9) == 2 && mid(false, 4, 3.1) == 8 && mid(false, 2, 3.9) == 8 && mid(false, 2, 4.1) == 2 && mid(false, 4, 15.9) == 2 && mid(false, 1, 3.5) == 2);
+}
+
 }  // namespace
 
 int main()
@@ -123,6 +159,7 @@ int main()
     CheckTeamRegions();
     CheckTeamRounds();
     CheckStores();
+    CheckWidth();
     std::printf("OK\n");
     return 0;
 }

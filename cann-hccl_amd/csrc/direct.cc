@@ -9,24 +9,26 @@ namespace hcclamd {
 namespace {
 
 // Where the tile kernels become the better form: they keep four times as much in flight per lane, which pays once every
-// CU has work.  Measured (us per collective among others, tile kernels / this form):
-//   all-reduce, 8 ranks, bf16 ring: 512 KiB 5.9 / 3.6, 1 MiB 7.1 / 5.3, 2 MiB 8.2 / 8.0, 4 MiB 12.1 / 13.9;
-//     fp32 ring 1 MiB 6.0 / 5.7, 2 MiB 7.0 / 7.9; 16 ranks 1 MiB 10.7 / 8.7, 2 MiB 12.9 / 14.8;
-//     halving-doubling, bf16, 24 ranks 256 KiB 16.9 / 6.5, 1 MiB 20.8 / 13.7
-//   reduce-scatter, 8 ranks, bf16 (bytes received by all ranks): 2 MiB 6.8 / 4.9, 4 MiB 8.2 / 7.7, 8 MiB 13.5 / 13.5
-//   all-gather (bytes sent by all ranks): 8 ranks 2 MiB 4.3 / 4.1, 4 MiB 6.9 / 6.9, 8 MiB 12.6 / 14.3;
-//     16 ranks 1 MiB 5.1 / 4.2, 2 MiB 6.7 / 6.8
+// CU has work.  Three sets of buffers in turn, us, tile kernels / this form (the usual ones packed):
+//   all-reduce, 8 ranks, ring, bf16 512 KiB 5.7 / 3.6, 1 MiB 6.3 / 3.7, fp32 5.3 / 3.7, 5.9 / 3.6; 16 ranks, fp32 9.1 / 4.5, 10.3 / 6.2; halving-doubling, bf16, 12
+//     ranks 256 KiB 9.3 / 4.5, 1 MiB 10.6 / 6.5, 24 ranks 17.3 / 5.5, 19.8 / 9.7
+//   reduce-scatter, 8 ranks, bf16 (bytes received by all ranks): 1 MiB 5.3 / 3.5, 2 MiB 6.2 / 4.1, 4 MiB 7.8 / 7.2
+//   all-gather (read and written): 8 ranks 5 MiB 4.2 / 3.4, 20 MiB 4.3 / 4.4; 16 ranks 5.1 / 4.4, 5.3 / 4.5
 constexpr uint64_t kDirectMaxBytes = uint64_t(1) << 20;       // of a reduction's results
 constexpr uint64_t kDirectMaxToOne = uint64_t(4) << 20;       // the same where each has one destination
-// Blocks of whole 16-byte vectors of more than three sources, in types that combine in an instruction or two: the tile
-// kernels get ahead sooner there.  Tile kernels / this form, us, new data for every call, one destination per result:
-//   reduce-scatter, fp32: 4 ranks 2.5 MiB 5.1 / 5.1, 4 MiB 6.1 / 6.2; 16 ranks 2.5 MiB 10.4 / 9.7, 3 MiB 11.3 / 11.9;
-//     32 ranks 2.5 MiB 17.6 / 16.5, 4 MiB 23.5 / 24.8; int64 32 ranks 3 MiB 18.5 / 20.5
-//   reduce, fp32: 8 ranks 2.5 MiB 6.8 / 6.3, 4 MiB 8.5 / 8.8; 32 ranks 2.5 MiB 17.2 / 16.3, 4 MiB 22.8 / 25.4
-// Up to the larger limit this form stays ahead for bf16 and 8-bit elements (32 ranks, 4 MiB: bf16 27.6 / 25.1, int8 26.3 / 25.1)
-// and for ragged blocks, whose ends the tile kernels take element by element (fp32, 32 ranks, 4 MiB 62.9 / 27.6), and for three sources or fewer (3 ranks, 4 MiB 6.2 / 5.4).
-// Copies, also from one to one, are ahead up to their limit for 2 to 32 ranks (scatter of 10 MiB 6.4 / 6.0).
+// Blocks of whole 16-byte vectors of more than three sources, in types that combine in an instruction or two: beyond this line the
+// packed form alone goes on (PackedFits).  Tile kernels / this form, us, one destination per result:
+//   reduce-scatter, 2.5 MiB: fp32, 4 ranks 4.2 / 3.3, 16 ranks 9.2 / 8.2, 32 ranks 15.9 / 14.7; int64, 32 ranks 15.7 / 14.7
+//   reduce, fp32, 2.5 MiB: 8 ranks 5.9 / 4.7, 32 ranks 15.6 / 14.9
+// Up to the larger limit this form stays ahead for bf16 of up to 8 ranks and for 8-bit elements (4 MiB: bf16, 4 ranks 5.2 / 4.3, 8 ranks 7.6 / 7.5; int8, 8 ranks 7.9 / 7.6, 12
+// ranks 3.5 MiB 10.2 / 9.9, 4 MiB 10.6 / 11.4, 32 ranks 23.3 / 21.7, 24.4 / 27.8), for ragged blocks of few ranks (int8, 8 ranks 3.5 MiB 8.0 / 7.9, 32 ranks 3 MiB 23.7 / 23.3, 3.5
+// MiB 25.0 / 26.8) and for three sources or fewer (3 ranks, 4 MiB 4.7 / 3.9).  bf16 of more than 8 ranks stops where its combining is what the waves wait for: 16 ranks 3 MiB
+// 11.2 / 10.0, 3.25 MiB 11.6 / 11.2, 3.5 MiB 11.6 / 12.1, 4 MiB 12.5 / 14.5, 32 ranks 20.1 / 19.0, 3.5 MiB 19.9 / 21.1, 4 MiB 21.7 / 26.2; ragged, 16 ranks 2.5 MiB 10.9 / 10.3, 3 MiB 11.5 /
+// 12.1, 24 ranks 15.2 / 13.8, 15.7 / 18.7.
+// Copies, also from one to one, are ahead up to their limit (20 MiB read and written: broadcast, 2 ranks 5.3 / 5.1, 32 ranks 7.7 / 5.6, send 5.0 / 4.6, scatter 5.1 / 5.0 ... 5.3), and a
+// call with new buffers uploads nothing; with known buffers a small one costs 0.2 more than with tables (its arguments are 1.3 KB).
 constexpr uint64_t kDirectMaxToOneEven = uint64_t(5) << 19;
+constexpr uint64_t kDirectMaxToOneBf16 = uint64_t(13) << 18, kDirectMaxToOneBf16Ragged = uint64_t(11) << 18;
 constexpr uint64_t kDirectMaxTraffic = uint64_t(20) << 20;    // read and written by a collective that only moves data
 // The rule looks at the call alone: a collective that is too large is told apart before anything is looked up or planned
 // for it (with a look into the plan, a caller with more distinct requests than this form's table holds paid for a plan on
@@ -123,7 +125,8 @@ template <uint32_t CAP> bool FillDirect(const Plan &plan, DirectLaunch *d)
 bool DirectFits(int coll, uint32_t p, uint64_t bytes, int dtype)
 {
     const bool even = bytes % 16 == 0 && p > 3 && dtype != HCCL_DATA_TYPE_INT8 && dtype != HCCL_DATA_TYPE_UINT8 && dtype != HCCL_DATA_TYPE_BFP16;
-    const uint64_t toOne = even ? kDirectMaxToOneEven : kDirectMaxToOne;
+    const bool bf16 = p > 8 && dtype == HCCL_DATA_TYPE_BFP16;
+    const uint64_t toOne = even ? kDirectMaxToOneEven : !bf16 ? kDirectMaxToOne : bytes % 16 == 0 ? kDirectMaxToOneBf16 : kDirectMaxToOneBf16Ragged;
     switch (coll) {
         case COLL_ALLREDUCE: return bytes <= (p > 1 ? kDirectMaxBytes : toOne);
         case COLL_REDUCESCATTER: return bytes <= toOne / p;

@@ -143,10 +143,34 @@ template <uint32_t P> bool Same(const Plan &plan, const DirectLaunch &d, const s
     return ok;
 }
 
+#define CHECK(c)                                             \
+    do {                                                     \
+        if (!(c)) {                                          \
+            std::printf("line %d: not so: %s\n", __LINE__, #c); \
+            std::exit(1);                                    \
+        }                                                    \
+    } while (0)
+
+// Both sides of the lines up to which a call goes out with its records in the arguments.
+void CheckLimits()
+{
+    const uint64_t mib = uint64_t(1) << 20;
+    for (uint32_t p : {2u, 8u, 9u, 16u, 32u}) {
+        for (int dtype : {HCCL_DATA_TYPE_BFP16, HCCL_DATA_TYPE_INT8, HCCL_DATA_TYPE_FP32}) {
+            const bool bf16 = dtype == HCCL_DATA_TYPE_BFP16 && p > 8, even = dtype == HCCL_DATA_TYPE_FP32 && p > 3;
+            const uint64_t whole = even ? 5 * mib / 2 : bf16 ? 13 * mib / 4 : 4 * mib, ragged = bf16 ? 11 * mib / 4 : 4 * mib;
+            CHECK(DirectFits(COLL_REDUCE, p, whole, dtype) && !DirectFits(COLL_REDUCE, p, whole + 16, dtype));
+            CHECK(DirectFits(COLL_REDUCE, p, ragged - 4, dtype) && !DirectFits(COLL_REDUCE, p, ragged + 4, dtype));
+            CHECK(DirectFits(COLL_REDUCESCATTER, p, whole / p / 16 * 16, dtype) && !DirectFits(COLL_REDUCESCATTER, p, whole / p / 16 * 16 + 16, dtype));
+        }
+    }
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
 {
+    CheckLimits();
     const long want = argc > 1 ? std::atol(argv[1]) : 3000;
     long taken[3] = {0, 0, 0}, unlike = 0, apart = 0, trees = 0, inPlace = 0;
     for (long n = 0; n < want;) {

@@ -22,7 +22,7 @@ constexpr uint64_t kDirectMaxToOne = uint64_t(4) << 20;       // the same where 
 //   reduce, fp32, 2.5 MiB: 8 ranks 5.9 / 4.7, 32 ranks 15.6 / 14.9
 // Up to the larger limit this form stays ahead for bf16 of up to 8 ranks and for 8-bit elements (4 MiB: bf16, 4 ranks 5.2 / 4.3, 8 ranks 7.6 / 7.5; int8, 8 ranks 7.9 / 7.6, 12
 // ranks 3.5 MiB 10.2 / 9.9, 4 MiB 10.6 / 11.4, 32 ranks 23.3 / 21.7, 24.4 / 27.8), for ragged blocks of few ranks (int8, 8 ranks 3.5 MiB 8.0 / 7.9, 32 ranks 3 MiB 23.7 / 23.3, 3.5
-// MiB 25.0 / 26.8) and for three sources or fewer (3 ranks, 4 MiB 4.7 / 3.9).  bf16 of more than 8 ranks stops where its combining is what the waves wait for: 16 ranks 3 MiB
+// MiB 25.0 / 26.8) and for three sources or fewer (3 ranks, 4 MiB 4.7 / 3.9).  bf16 of more than 8 ranks stops before (CombiningBound) where its combining is what the waves wait for: 16 ranks 3 MiB
 // 11.2 / 10.0, 3.25 MiB 11.6 / 11.2, 3.5 MiB 11.6 / 12.1, 4 MiB 12.5 / 14.5, 32 ranks 20.1 / 19.0, 3.5 MiB 19.9 / 21.1, 4 MiB 21.7 / 26.2; ragged, 16 ranks 2.5 MiB 10.9 / 10.3, 3 MiB 11.5 /
 // 12.1, 24 ranks 15.2 / 13.8, 15.7 / 18.7.
 // Copies, also from one to one, are ahead up to their limit (20 MiB read and written: broadcast, 2 ranks 5.3 / 5.1, 32 ranks 7.7 / 5.6, send 5.0 / 4.6, scatter 5.1 / 5.0 ... 5.3), and a
@@ -125,8 +125,7 @@ template <uint32_t CAP> bool FillDirect(const Plan &plan, DirectLaunch *d)
 bool DirectFits(int coll, uint32_t p, uint64_t bytes, int dtype)
 {
     const bool even = bytes % 16 == 0 && p > 3 && dtype != HCCL_DATA_TYPE_INT8 && dtype != HCCL_DATA_TYPE_UINT8 && dtype != HCCL_DATA_TYPE_BFP16;
-    const bool bf16 = p > 8 && dtype == HCCL_DATA_TYPE_BFP16;
-    const uint64_t toOne = even ? kDirectMaxToOneEven : !bf16 ? kDirectMaxToOne : bytes % 16 == 0 ? kDirectMaxToOneBf16 : kDirectMaxToOneBf16Ragged;
+    const uint64_t toOne = even ? kDirectMaxToOneEven : kDirectMaxToOne;
     switch (coll) {
         case COLL_ALLREDUCE: return bytes <= (p > 1 ? kDirectMaxBytes : toOne);
         case COLL_REDUCESCATTER: return bytes <= toOne / p;
@@ -137,6 +136,13 @@ bool DirectFits(int coll, uint32_t p, uint64_t bytes, int dtype)
         case COLL_SENDRECV: return bytes <= kDirectMaxTraffic / 2;
         default: return false;
     }
+}
+
+bool CombiningBound(int coll, uint32_t p, uint64_t bytes, int dtype)
+{
+    const uint64_t total = coll == COLL_REDUCESCATTER ? bytes * p : bytes;
+    return (coll == COLL_REDUCESCATTER || coll == COLL_REDUCE) && p > 8 && dtype == HCCL_DATA_TYPE_BFP16 &&
+        total > (bytes % 16 == 0 ? kDirectMaxToOneBf16 : kDirectMaxToOneBf16Ragged);
 }
 
 // Beyond those limits, where the items are alike (PackDirect): waves of 1 or 4 KiB keep every CU equally busy where the tile kernels' tiles of

@@ -1241,7 +1241,7 @@ DirectLaunch *FindDirect(Group *g, int algo)
         return nullptr;
     }
     const uint64_t bytes = sig.count * DtypeSize(sig.dtype);
-    const bool small = DirectFits(sig.coll, g->p, bytes, sig.dtype);
+    const bool small = DirectFits(sig.coll, g->p, bytes, sig.dtype) && !CombiningBound(sig.coll, g->p, bytes, sig.dtype);
     if (!small && !PackedFits(sig.coll, g->p, bytes, sig.dtype)) {
         return nullptr;
     }

@@ -147,6 +147,8 @@ struct DirectLaunch {
 
 // Whether a collective is small enough for this form, whatever its schedule (bytes: of the call's count).
 bool DirectFits(int coll, uint32_t p, uint64_t bytes, int dtype);
+// Whether it is left to the tile kernels all the same: reductions to one destination whose combining the waves wait for.
+bool CombiningBound(int coll, uint32_t p, uint64_t bytes, int dtype);
 // Whether a larger one goes out in the packed form if its items are alike.
 bool PackedFits(int coll, uint32_t p, uint64_t bytes, int dtype);
 // The launch of `plan`; false (func == nullptr) where the kernels' records cannot hold it.

@@ -159,9 +159,11 @@ void CheckLimits()
         for (int dtype : {HCCL_DATA_TYPE_BFP16, HCCL_DATA_TYPE_INT8, HCCL_DATA_TYPE_FP32}) {
             const bool bf16 = dtype == HCCL_DATA_TYPE_BFP16 && p > 8, even = dtype == HCCL_DATA_TYPE_FP32 && p > 3;
             const uint64_t whole = even ? 5 * mib / 2 : bf16 ? 13 * mib / 4 : 4 * mib, ragged = bf16 ? 11 * mib / 4 : 4 * mib;
-            CHECK(DirectFits(COLL_REDUCE, p, whole, dtype) && !DirectFits(COLL_REDUCE, p, whole + 16, dtype));
-            CHECK(DirectFits(COLL_REDUCE, p, ragged - 4, dtype) && !DirectFits(COLL_REDUCE, p, ragged + 4, dtype));
-            CHECK(DirectFits(COLL_REDUCESCATTER, p, whole / p / 16 * 16, dtype) && !DirectFits(COLL_REDUCESCATTER, p, whole / p / 16 * 16 + 16, dtype));
+            auto fits = [&](int coll, uint64_t bytes) { return DirectFits(coll, p, bytes, dtype) && !CombiningBound(coll, p, bytes, dtype); };
+            CHECK(fits(COLL_REDUCE, whole) && !fits(COLL_REDUCE, whole + 16));
+            CHECK(fits(COLL_REDUCE, ragged - 4) && !fits(COLL_REDUCE, ragged + 4));
+            CHECK(fits(COLL_REDUCESCATTER, whole / p / 16 * 16) && !fits(COLL_REDUCESCATTER, whole / p / 16 * 16 + 16));
+            CHECK(!CombiningBound(COLL_ALLREDUCE, p, 8 * mib, dtype));
         }
     }
 }

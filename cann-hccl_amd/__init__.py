@@ -41,7 +41,7 @@ EXPORTS = [
     "HcclCommInitClusterInfoConfig", "HcclCreateSubCommConfig", "HcclGetRootInfo", "HcclCommInitRootInfo",
     "HcclCommInitRootInfoConfig", "HcclBroadcast", "HcclScatter", "HcclSend", "HcclRecv", "HcclReduce",
     "HcclBatchSendRecv", "HcclCommSetMemoryRange", "HcclCommUnsetMemoryRange", "HcclCommActivateCommMemory",
-    "HcclCommDeactivateCommMemory", "HcclAmdSetParam", "HcclAmdGetLastOpInfo", "HcclAmdDescribePlan", "HcclAmdReduceScatterNoAlloc",
+    "HcclCommDeactivateCommMemory", "HcclAmdSetParam", "HcclAmdGetLastOpInfo", "HcclAmdGetLastOpForm", "HcclAmdDescribePlan", "HcclAmdReduceScatterNoAlloc",
 ]
 
 
@@ -189,6 +189,7 @@ def lib():
     L.HcclCommResume.argtypes = [vp]
     L.HcclAmdSetParam.argtypes = [vp, ctypes.c_char_p, ctypes.c_char_p]
     L.HcclAmdGetLastOpInfo.argtypes = [vp, ctypes.POINTER(HcclAmdOpInfo)]
+    L.HcclAmdGetLastOpForm.argtypes = [vp, ctypes.POINTER(ctypes.c_int32)]
     L.HcclAmdDescribePlan.argtypes = [i32, i32, u32, u64, i32, u64, u64, u64, ctypes.POINTER(u64), ctypes.c_char_p,
                                       ctypes.c_size_t, ctypes.POINTER(ctypes.c_size_t)]
     _call = _native_call(L) or _through_ctypes
@@ -262,6 +263,13 @@ def last_op_info(comm):
     info = HcclAmdOpInfo()
     _check("HcclAmdGetLastOpInfo", lib().HcclAmdGetLastOpInfo(comm, ctypes.byref(info)))
     return {f[0]: getattr(info, f[0]) for f in HcclAmdOpInfo._fields_}
+
+
+def last_op_form(comm):
+    """What the kernels of the last collective worked from (HcclAmdOpForm)."""
+    form = ctypes.c_int32()
+    _check("HcclAmdGetLastOpForm", lib().HcclAmdGetLastOpForm(comm, ctypes.byref(form)))
+    return form.value
 
 
 def all_reduce(comms, sends, recvs, count, dtype, op, stream):

@@ -472,11 +472,13 @@ HcclResult Reader(A2avSet *s, hipStream_t stream, A2avReader **reader)
 
 }  // namespace
 
+// Up to 16 ranks a new call's tables travel in the arguments; from its second time on it reads them from device memory: the launch call writes 944
+// bytes of arguments to 8 ranks, 3.4 KB to 16, of 24 otherwise.
+bool A2avInArguments(const Group *g, const A2avSet *s) { return g->p <= 16 && !s->hit; }
+
 HcclResult A2avLaunch(Group *g, A2avSet *s, hipStream_t stream)
 {
-    // Up to 16 ranks a new call's tables travel in the arguments; from its second time on it reads them from device memory: the launch call writes 944
-    // bytes of arguments to 8 ranks, 3.4 KB to 16, of 24 otherwise.
-    const bool inArguments = g->p <= 16 && !s->hit;
+    const bool inArguments = A2avInArguments(g, s);
     A2avReader *reader = nullptr;
     if (!s->hit) {
         s->onDevice = false;

@@ -224,6 +224,19 @@ HcclResult HcclAmdGetLastOpInfo(HcclComm comm, HcclAmdOpInfo *info)
     return HCCL_SUCCESS;
 }
 
+HcclResult HcclAmdGetLastOpForm(HcclComm comm, int32_t *form)
+{
+    CHK_PTR(comm);
+    CHK_PTR(form);
+    Comm *c = AsComm(comm);
+    if (c == nullptr) {
+        return HCCL_E_PARA;
+    }
+    std::lock_guard<std::mutex> lock(c->group->m);
+    *form = c->group->lastInfo.form;
+    return HCCL_SUCCESS;
+}
+
 HcclResult HcclAmdDescribePlan(int32_t coll, int32_t algo, uint32_t nRanks, uint64_t count, HcclDataType dataType,
     uint64_t cclBytes, uint64_t align, uint64_t inPlaceMask, const uint64_t *tables, char *out, size_t cap, size_t *needed)
 {

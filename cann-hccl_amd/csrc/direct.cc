@@ -378,6 +378,7 @@ void PackDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaun
         // waves of 4 KiB where PackedFits' figures say so
         wide = !toOne && total > (p <= 8 ? kPackedNarrowBytes : kPackedNarrowBytes / 4 * 3) && total <= 4 * kPackedNarrowBytes;
     }
+    d->packedWide = wide;
     const uint32_t chunk = wide ? kPackedWideChunk : kDirectChunk;
     kind = wide ? KernelKind(kind + KK_PACKED_WIDE) : kind;
     d->packedGridX = uint32_t(longest / chunk + (longest % chunk >= 16 ? 1 : 0)) + (ends ? 1u : 0u);

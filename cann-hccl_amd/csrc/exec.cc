@@ -1505,6 +1505,7 @@ HcclResult IssueCollective(Group *g, uint32_t launcher)
     bool viaGraph = false;
     if (direct != nullptr) {
         g->lastInfo = direct->info;
+        g->lastInfo.form = !direct->usePacked ? HCCL_AMD_FORM_RECORDS : (direct->packedWide ? HCCL_AMD_FORM_PACKED_WIDE : HCCL_AMD_FORM_PACKED);
     } else if (a2av != nullptr) {
         OpInfo info;
         info.coll = COLL_ALLTOALLV;
@@ -1512,6 +1513,7 @@ HcclResult IssueCollective(Group *g, uint32_t launcher)
         info.fused = 1;
         info.cacheHit = a2av->hit ? 1 : 0;
         info.launches = a2av->launches;
+        info.form = A2avInArguments(g, a2av) ? HCCL_AMD_FORM_A2AV_ARGUMENTS : HCCL_AMD_FORM_A2AV_DEVICE;
         info.bytesRead = info.bytesWritten = a2av->moved;
         info.stepRead = info.stepWritten = a2av->moved * (g->cfg.servers > 1 && g->cfg.algo != ALGO_PAIRWISE ? 2 : 1);   // (staged: every byte twice)
         g->lastInfo = info;

@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "arena.h"
+#include "hccl/hccl_amd_ext.h"
 #include "hccl/hccl_types.h"
 #include "kernels.h"
 #include "plan.h"
@@ -83,7 +84,8 @@ struct OpInfo {
     int coll = 0, algo = 0, fused = 0, graph = 0, cacheHit = 0;
     uint32_t launches = 0;
     uint32_t teamLaunches = 0;
-    uint32_t direct = 0;                          // 1: one launch whose descriptors ride in its arguments
+    uint32_t direct = 0;                          // 1: a small collective, one launch whose descriptors ride in its arguments
+    int form = HCCL_AMD_FORM_TABLES;              // what its kernels work from
     uint64_t bytesRead = 0, bytesWritten = 0;     // what the issued kernels move in HBM, all ranks
     uint64_t stepRead = 0, stepWritten = 0;       // the step-by-step schedule's figure
     uint64_t scratchBytes = 0;
@@ -141,6 +143,7 @@ struct DirectLaunch {
     const void *packedFunc = nullptr;                  // the same collective with a PackedArgs, nullptr: its items are not alike
     uint32_t packedRanks = 0, packedGridX = 0;         // ranks that its arguments have room for
     std::vector<uint8_t> packed;
+    bool packedWide = false;                           // four vectors per lane
     bool usePacked = false;                            // this call's buffers fit it
     OpInfo info;
 };
@@ -351,6 +354,8 @@ bool A2avRow(Group *g, uint32_t r, void *send, void *recv, const uint64_t *const
 void A2avExpand(Group *g, uint32_t except);
 // The last rank has arrived.  *ready: what to launch, nullptr where the call goes the general way.
 HcclResult A2avFinish(Group *g, hipStream_t stream, A2avSet **ready);
+// Whether that launch carries the tables in its arguments.
+bool A2avInArguments(const Group *g, const A2avSet *s);
 HcclResult A2avLaunch(Group *g, A2avSet *s, hipStream_t stream);
 
 // Whether the ranks' buffers may share memory as they do (exec.cc).

@@ -104,6 +104,17 @@ typedef struct HcclAmdOpInfoDef {
 /* What the most recent collective of this communicator's group issued. */
 extern HcclResult HcclAmdGetLastOpInfo(HcclComm comm, HcclAmdOpInfo *info);
 
+/* What the kernels of the most recent collective of this communicator's group worked from. */
+typedef enum HcclAmdOpFormDef {
+    HCCL_AMD_FORM_TABLES = 0,          /* tables in device memory, made for the call's buffers (tile and step kernels) */
+    HCCL_AMD_FORM_RECORDS = 1,         /* a record per item in the kernel arguments */
+    HCCL_AMD_FORM_PACKED = 2,          /* one record for all items, which are alike, in the arguments; a wave per KiB */
+    HCCL_AMD_FORM_PACKED_WIDE = 3,     /* the same, a wave per 4 KiB */
+    HCCL_AMD_FORM_A2AV_ARGUMENTS = 4,  /* an all-to-all-v's own tables, in the arguments */
+    HCCL_AMD_FORM_A2AV_DEVICE = 5      /* an all-to-all-v's own tables, in device memory */
+} HcclAmdOpForm;
+extern HcclResult HcclAmdGetLastOpForm(HcclComm comm, int32_t *form);
+
 /* Plans a collective without a device and writes the plan as JSON (phases of copy / reduce steps,
  * fused items, byte counts) into out[0..cap).  coll / algo as in HcclAmdOpInfo; for the rooted
  * collectives (coll 4 broadcast, 5 reduce, 6 scatter) the algo argument carries the root rank in its low 16 bits and the

@@ -2,6 +2,7 @@
 with what lies between the blocks: rank counts around the kernels' 8, 16, 32, 64, element sizes, empty blocks, blocks at any byte, blocks in
 any order with gaps, pieces at the edges of 4 KiB, several sets of tables and streams in turn, and the calls that go the general way."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -243,6 +244,66 @@ def test_new_tables_under_load():
             r.clear()
         for r in runs:
             r.call(g)
+        for r in runs:
+            r.check()
+    finally:
+        g.close()
+
+
+@pytest.mark.parametrize("p", [2, 8, 9, 16, 17, 32, 33, 64])
+def test_which_form(p):
+    """A new call, a known one, the general way (HcclAmdOpForm: 4 in the arguments, 5 in device memory, 0 planned)."""
+    rng = np.random.default_rng(7 * p)
+    g = gh.Group(p)
+    try:
+        run = Run(rng, p, 4, lambda n: rng.integers(0, 300, (n, n)), "packed", 4)
+        for params, want in (({}, 4 if p <= 16 else 5), ({}, 5), ({}, 5), ({"direct": 0}, 0), ({"direct": "auto"}, 5)):
+            g.set(**params)
+            run.clear()
+            run.call(g)
+            assert H.last_op_form(g.comms[0]) == want, params
+            run.check()
+        n = 1000
+        send, recv = [torch.randint(0, 256, (p * n,), dtype=torch.uint8, device="cuda") for _ in range(p)], [torch.empty(p * n, dtype=torch.uint8, device="cuda") for _ in range(p)]
+        torch.cuda.synchronize()
+        for want in (4 if p <= 16 else 5, 5):
+            H.all_to_all(g.comms, [t.data_ptr() for t in send], [t.data_ptr() for t in recv], n, TYPES[1], g.stream_ptr)
+            assert H.last_op_form(g.comms[0]) == want
+        g.stream.synchronize()
+        for j in range(p):
+            assert torch.equal(recv[j], torch.cat([send[i][j * n:(j + 1) * n] for i in range(p)])), j
+    finally:
+        g.close()
+
+
+@pytest.mark.parametrize("p", [12, 20])
+def test_one_thread_and_stream_per_rank(p):
+    """Whichever rank comes last, on whichever stream: a known call is known."""
+    rng = np.random.default_rng(11 * p)
+    g = gh.Group(p, blocking_arrive=1, arrive_timeout_ms=20000)
+    try:
+        runs = [Run(rng, p, 4, lambda n: rng.integers(0, 300, (n, n)), "any", 4) for _ in range(4)]
+        streams = [torch.cuda.Stream() for _ in range(p)]
+        for r in runs:
+            r.clear()
+        codes, seen = [[] for _ in range(p)], []
+
+        def work(r):
+            for turn in range(4):
+                for run in runs:
+                    rows = [t[r].ctypes.data for t in run.t]
+                    codes[r].append(H.lib().HcclAlltoAllV(run.dev[r].data_ptr() + run.pad, rows[0], rows[1], TYPES[4], run.out[r].data_ptr() + run.pad, rows[2], rows[3],
+                                                          TYPES[4], g.comms[r], streams[r].cuda_stream))
+                    if r == 0 and turn:
+                        seen.append(H.last_op_info(g.comms[0])["cacheHit"])
+            streams[r].synchronize()
+
+        threads = [threading.Thread(target=work, args=(r,)) for r in range(p)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join(60)
+        assert codes == [[0] * 16] * p and seen == [1] * 12
         for r in runs:
             r.check()
     finally:

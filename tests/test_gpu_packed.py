@@ -138,3 +138,74 @@ def test_many_sources(orc, p):
     finally:
         for g in groups.values():
             g.close()
+
+
+# What a call's kernels work from (HcclAmdOpForm), by quarters of a MiB on 256 CUs: up to (the first), then beyond it.
+TABLES, RECORDS, PACKED, WIDE = 0, 1, 2, 3
+ALL_REDUCE = {2: [(8, PACKED), (32, WIDE), (192, PACKED)], 4: [(8, PACKED), (24, WIDE), (32, TABLES), (96, PACKED)],
+              8: [(8, PACKED), (11, WIDE), (16, TABLES), (22, WIDE), (32, TABLES), (48, PACKED)], 16: [(6, PACKED), (11, WIDE), (16, TABLES), (22, WIDE)]}
+ALL_REDUCE_HALVES = {**ALL_REDUCE, 16: [(6, PACKED), (16, TABLES), (22, WIDE)]}
+WHOLE_BLOCKS = {2: [(60, PACKED), (64, TABLES), (256, PACKED)], 3: [(24, PACKED)], 4: [(30, PACKED), (32, TABLES), (44, PACKED)], 6: [(18, PACKED)],
+                8: [(24, PACKED)], 16: [(11, PACKED), (16, TABLES), (20, PACKED)]}
+RAGGED_BLOCKS = {2: [(56, PACKED)], 3: [(24, PACKED)], 4: [(24, PACKED)], 6: [(16, PACKED)], 8: [(20, PACKED)], 16: [(16, PACKED)]}
+
+
+def _as_the_tiles(g, call, form, what):
+    """`call` takes this form and gives the bits of the tile kernels."""
+    print("form", *what, "expected", form, flush=True)
+    outs = call()
+    assert gh.H.last_op_form(g.comms[0]) == form, what
+    g.set(direct=0)
+    tiles = call()
+    assert gh.H.last_op_form(g.comms[0]) == TABLES
+    g.set(direct="auto")
+    for a, b in zip(outs, tiles):
+        assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), what
+
+
+def _lines(edges):
+    return [(upto, form, beyond) for (upto, form), (_, beyond) in zip(edges, edges[1:] + [(None, TABLES)])]
+
+
+@pytest.mark.parametrize("p,algo", [(p, a) for p in (2, 4, 8, 16) for a in ("ring", "mesh", "rhd")])
+def test_form_of_all_reduce(p, algo):
+    assert torch.cuda.get_device_properties(0).multi_processor_count == 256
+    g = gh.Group(p, algo=algo)
+    try:
+        for dt, op in ((FP32, SUM), (BF16, MAX), (INT8, MIN)):
+            unit = gh.H.DTYPE_SIZE[dt]
+            for upto, form, beyond in _lines((ALL_REDUCE_HALVES if dt == BF16 else ALL_REDUCE)[p]):
+                if upto > 100 and dt != FP32:
+                    continue
+                for n, want in ((upto * MIB // 4 // unit, form), (upto * MIB // 4 // unit + 1, beyond)):
+                    ins = _ins(dt, p, n, 19 * p + unit, False)
+                    _as_the_tiles(g, lambda: gh.all_reduce(g, ins, dt, op)[0], want, (p, algo, dt, n))
+    finally:
+        g.close()
+
+
+@pytest.mark.parametrize("p", [2, 3, 4, 6, 8, 16])
+def test_form_of_reduce_scatter(p):
+    assert torch.cuda.get_device_properties(0).multi_processor_count == 256
+    g = gh.Group(p)
+    try:
+        for edges, ragged in ((WHOLE_BLOCKS[p], 0), (RAGGED_BLOCKS[p], 1)):
+            for upto, form, beyond in _lines(edges):
+                last = upto * MIB // 4 // p // 16 * 4 - 3 * ragged
+                for n, want in ((last, form), (last + 4 + 12 * ragged, beyond)):
+                    ins = _ins(FP32, p, n * p, 23 * p + ragged, False)
+                    _as_the_tiles(g, lambda: gh.reduce_scatter(g, ins, FP32, SUM)[0], want, (p, n))
+    finally:
+        g.close()
+
+
+def test_form_of_others():
+    g = gh.Group(8, servers=2)
+    try:
+        ins = _ins(FP32, 8, 5000, 3, False)
+        _as_the_tiles(g, lambda: gh.all_reduce(g, ins, FP32, SUM)[0], RECORDS, ("two servers",))
+        g.set(servers=1)
+        _as_the_tiles(g, lambda: gh.all_gather(g, ins, FP32), PACKED, ("all-gather",))
+        _as_the_tiles(g, lambda: gh.all_reduce(g, ins, FP32, SUM)[0], PACKED, ("one server",))
+    finally:
+        g.close()

@@ -146,8 +146,8 @@ bool CombiningBound(int coll, uint32_t p, uint64_t bytes, int dtype)
 }
 
 // Beyond those limits, where the items are alike (PackDirect): waves of 1 or 4 KiB keep every CU equally busy where the tile kernels' tiles of
-// 16 KiB do not, that is where there are few of them, or a few more than one (4 MiB) or two (8 MiB) for each CU: a CU takes some 4 us for a tile
-// that is read from 8 buffers and stored to 8.  Three sets of buffers in turn, us, tile kernels / packed with KiB / packed with 4 KiB:
+// 16 KiB do not, that is where there are few of them, or a few more than one, two or three for each CU (on 256 CUs 4, 8, 12 MiB): a CU takes some 4 us for a tile
+// that is read from 8 buffers and stored to 8.  So the windows are in sixteenths of a tile for each CU, 256 KiB on 256 CUs.  Measured there, three sets of buffers in turn, us, tile kernels / packed with KiB / packed with 4 KiB:
 //   all-reduce, 2 ranks: 4 MiB 4.5 / 3.6 / 3.6, 6 MiB 5.7 / 5.1 / 4.5, 8 MiB 6.0 / 6.0 / 5.8, 24 MiB 18.0 / 16.6 / 17.1, 48 MiB 33.8 / 31.9 / 33.5
 //     4 ranks: 3 MiB 5.2 / 4.5 / 4.6, 4.25 MiB 8.0 / 6.9 / 6.0, 6 MiB 8.7 / 9.4 / 7.6, 7 MiB 9.5 / 10.4 / 9.8, 8 MiB 10.6 / 12.2 / 12.0, 9 MiB
 //       14.1 / 13.9 / 13.8, 14 MiB 21.7 / 19.9 / 20.1, 24 MiB 35.9 / 32.1 / 31.6, 28 MiB 40.7 / 41.1 / 40.9
@@ -162,32 +162,57 @@ bool CombiningBound(int coll, uint32_t p, uint64_t bytes, int dtype)
 //     10.1 / 8.4), 3 MiB 9.8 / 9.7, 4.25 MiB 15.5 / 13.5, 5 MiB 16.4 / 15.3, 6 MiB 17.8 / 20.4
 //   other blocks: 2 ranks 14 MiB 8.9 / 8.8, 4 ranks 6 MiB 6.9 / 6.8, 8 ranks 3 MiB 6.7 / 5.9, 4 MiB 8.5 / 7.8, 5 MiB 9.8 / 9.0, 16 ranks 2 MiB 9.2 / 7.9,
 //     3 MiB 10.3 / 10.7.  Waves of 4 KiB bring nothing where every block has one destination (8 ranks bf16 pairwise, 4 MiB 6.9 / 7.7).
-// Two kinds of calls gain less and stay out: 16 ranks' all-reduce of a 16-bit floating-point type from 1.5 MiB, whose waves of 4 KiB wait for their own
-// arithmetic (1.75 MiB bf16 sum 12.4 / 12.1, fp16 minimum of the uncut mesh 12.2 / 16.1), and bytes off a vector boundary (8 ranks 4.75 MiB 9.3 / 10.1).
-bool PackedFits(int coll, uint32_t p, uint64_t bytes, int dtype)
+// Two kinds of calls gain less and stay out: 16 ranks' all-reduce of a 16-bit floating-point type between 1.5 and 4 MiB, whose waves of 4 KiB wait for their own
+// arithmetic (1.75 MiB bf16 sum 12.4 / 12.1, fp16 minimum of the uncut mesh 12.2 / 16.1; beyond 4 MiB the tiles wait longer: 4.25 MiB bf16 sum 27.1 / 23.2, maximum
+// 25.8 / 22.9, halving-doubling 30.8 / 24.2, 5.44 MiB 31.5 / 29.3, 31.3 / 30.5, 33.6 / 30.8), and bytes off a vector boundary (8 ranks 4.75 MiB 9.3 / 10.1).
+namespace {
+
+enum PackedCalls : uint8_t {
+    ALL_REDUCE_HALVES = 1, ALL_REDUCE_OTHERS = 2, ALL_REDUCE = 3,     // of fp16 and bf16; of other types
+    BLOCKS_WHOLE = 4,                                                 // reduce-scatter, blocks of whole 16-byte vectors
+    BLOCKS_BYTES = 8, BLOCKS_OTHERS = 16, BLOCKS_RAGGED = 24          // other blocks, of 8-bit elements; of other types
+};
+struct PackedWindow {
+    uint8_t calls, least, most;      // ranks
+    uint16_t above, upTo;            // bytes of an all-reduce, received by all ranks of a reduce-scatter
+};
+constexpr PackedWindow kPackedWindows[] = {
+    {ALL_REDUCE, 2, 2, 0, 192},
+    {ALL_REDUCE, 3, 3, 0, 14},
+    {ALL_REDUCE, 4, 4, 0, 24}, {ALL_REDUCE, 4, 4, 32, 96},
+    {ALL_REDUCE, 5, 7, 0, 9},
+    {ALL_REDUCE, 8, 8, 0, 11}, {ALL_REDUCE, 8, 8, 16, 22}, {ALL_REDUCE, 8, 8, 32, 48},
+    {ALL_REDUCE, 9, 32, 0, 6}, {ALL_REDUCE_OTHERS, 16, 16, 6, 11}, {ALL_REDUCE, 16, 16, 16, 22},
+    {BLOCKS_WHOLE, 2, 2, 0, 60}, {BLOCKS_WHOLE, 2, 2, 64, 256},
+    {BLOCKS_WHOLE, 3, 3, 0, 24},
+    {BLOCKS_WHOLE, 4, 4, 0, 30}, {BLOCKS_WHOLE, 4, 4, 32, 44},
+    {BLOCKS_WHOLE, 5, 7, 0, 18},
+    {BLOCKS_WHOLE, 8, 8, 0, 24},
+    {BLOCKS_WHOLE, 16, 16, 0, 11}, {BLOCKS_WHOLE, 16, 16, 16, 20},
+    {BLOCKS_RAGGED, 2, 2, 0, 56},
+    {BLOCKS_RAGGED, 3, 4, 0, 24},
+    {BLOCKS_RAGGED, 5, 8, 0, 14}, {BLOCKS_OTHERS, 8, 8, 16, 20},
+    {BLOCKS_RAGGED, 16, 16, 0, 10},
+};
+uint64_t SixteenthTiles(uint32_t numCu) { return uint64_t(numCu) * kTileBytes / 16; }
+
+}  // namespace
+
+bool PackedFits(int coll, uint32_t p, uint64_t bytes, int dtype, uint32_t numCu)
 {
-    constexpr uint64_t kQuarter = uint64_t(1) << 18;      // of a MiB
-    if (p < 2 || p > 32) {
-        return false;
-    }
-    const bool shaped = PackedShape(p) < kPackedShapes, bytesOnly = dtype == HCCL_DATA_TYPE_INT8 || dtype == HCCL_DATA_TYPE_UINT8;
-    auto within = [](uint64_t total, uint64_t above, uint64_t upTo) { return total > above * kQuarter && total <= upTo * kQuarter; };
+    uint8_t call = 0;
+    uint64_t total = bytes;
     if (coll == COLL_ALLREDUCE) {
-        if (!shaped) {
-            return bytes <= (p <= 4 ? 14 : p <= 8 ? 9 : 6) * kQuarter;
-        }
-        const bool busy = p == 16 && (dtype == HCCL_DATA_TYPE_FP16 || dtype == HCCL_DATA_TYPE_BFP16);
-        return p == 2 ? bytes <= 192 * kQuarter : p == 4 ? bytes <= 24 * kQuarter || within(bytes, 32, 96) :
-            bytes <= (busy ? 6 : 11) * kQuarter || within(bytes, 16, 22) || (p == 8 && within(bytes, 32, 48));
+        call = dtype == HCCL_DATA_TYPE_FP16 || dtype == HCCL_DATA_TYPE_BFP16 ? ALL_REDUCE_HALVES : ALL_REDUCE_OTHERS;
+    } else if (coll == COLL_REDUCESCATTER) {
+        call = bytes % 16 == 0 ? BLOCKS_WHOLE : (dtype == HCCL_DATA_TYPE_INT8 || dtype == HCCL_DATA_TYPE_UINT8 ? BLOCKS_BYTES : BLOCKS_OTHERS);
+        total *= p;
     }
-    if (coll == COLL_REDUCESCATTER) {
-        const uint64_t total = bytes * p;
-        if (bytes % 16 == 0) {
-            return p == 2 ? total <= 60 * kQuarter || within(total, 64, 256) : p <= 4 ? total <= (shaped ? 30 : 24) * kQuarter || (shaped && within(total, 32, 44)) :
-                p <= 8 ? total <= (shaped ? 24 : 18) * kQuarter : p == 16 && (total <= 11 * kQuarter || within(total, 16, 20));
+    const uint64_t unit = SixteenthTiles(numCu);
+    for (const PackedWindow &w : kPackedWindows) {
+        if ((w.calls & call) != 0 && p >= w.least && p <= w.most && total > w.above * unit && total <= w.upTo * unit) {
+            return true;
         }
-        return p == 2 ? total <= 56 * kQuarter : p <= 4 ? total <= 24 * kQuarter : p <= 8 ? total <= 14 * kQuarter || (p == 8 && !bytesOnly && within(total, 16, 20)) :
-            p == 16 && total <= 10 * kQuarter;
     }
     return false;
 }
@@ -279,7 +304,7 @@ template <uint32_t P> bool FillOffsets(DirectLaunch *d, uint32_t ranks, const st
 
 }  // namespace
 
-void PackDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaunch *d)
+void PackDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaunch *d, uint32_t numCu)
 {
     const uint32_t p = plan.p, n = uint32_t(plan.fused.size());
     if (p > 32 || n == 0 || n > p) {
@@ -376,7 +401,7 @@ void PackDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaun
     if (reduceColl && shape < kPackedShapes && order.size() == p) {       // (of two sources, added and exclusive-ored are the same)
         kind = KernelKind((tree ? KK_PACKED_TREE : (left ? KK_PACKED_CHAIN : KK_PACKED_RING)) + shape);
         // waves of 4 KiB where PackedFits' figures say so
-        wide = !toOne && total > (p <= 8 ? kPackedNarrowBytes : kPackedNarrowBytes / 4 * 3) && total <= 4 * kPackedNarrowBytes;
+        wide = !toOne && total > (p <= 8 ? 8 : 6) * SixteenthTiles(numCu) && total <= 32 * SixteenthTiles(numCu);
     }
     d->packedWide = wide;
     const uint32_t chunk = wide ? kPackedWideChunk : kDirectChunk;

@@ -1242,7 +1242,7 @@ DirectLaunch *FindDirect(Group *g, int algo)
     }
     const uint64_t bytes = sig.count * DtypeSize(sig.dtype);
     const bool small = DirectFits(sig.coll, g->p, bytes, sig.dtype) && !CombiningBound(sig.coll, g->p, bytes, sig.dtype);
-    if (!small && !PackedFits(sig.coll, g->p, bytes, sig.dtype)) {
+    if (!small && !PackedFits(sig.coll, g->p, bytes, sig.dtype, g->numCu)) {
         return nullptr;
     }
     uint64_t inPlace = 0;
@@ -1265,7 +1265,7 @@ DirectLaunch *FindDirect(Group *g, int algo)
             return nullptr;             // the general path reports it
         }
         if (BuildDirect(*plan, ReduceColl(sig.coll), sig.dtype, sig.op, &d)) {
-            PackDirect(*plan, ReduceColl(sig.coll), sig.dtype, sig.op, &d);
+            PackDirect(*plan, ReduceColl(sig.coll), sig.dtype, sig.op, &d, g->numCu);
             d.info = MakeInfo(g, algo, *plan, true);
             d.info.launches = 1;
             d.info.direct = small ? 1 : 0;

@@ -153,7 +153,6 @@ inline uint32_t TeamBlockWords(uint32_t nregions) { return kTeamHeaderWords + 2u
 constexpr uint32_t kDirectThreads = 64;                  // a workgroup is one wave,
 constexpr uint32_t kDirectChunk = kDirectThreads * 16;   // of an item it takes these bytes,
 constexpr uint32_t kPackedWideChunk = 4 * kDirectChunk;  // or these
-constexpr uint64_t kPackedNarrowBytes = uint64_t(2) << 20;   // (collectives beyond these, direct.cc)
 enum DirectKind : uint32_t { DIRECT_CHAIN = 0, DIRECT_TREE = 1, DIRECT_STACK = 2 };
 
 // CAP = 8: up to 8 sources and destinations per item; CAP = 32: up to 32 (no stack programs).

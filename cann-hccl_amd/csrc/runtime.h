@@ -153,11 +153,11 @@ bool DirectFits(int coll, uint32_t p, uint64_t bytes, int dtype);
 // Whether it is left to the tile kernels all the same: reductions to one destination whose combining the waves wait for.
 bool CombiningBound(int coll, uint32_t p, uint64_t bytes, int dtype);
 // Whether a larger one goes out in the packed form if its items are alike.
-bool PackedFits(int coll, uint32_t p, uint64_t bytes, int dtype);
+bool PackedFits(int coll, uint32_t p, uint64_t bytes, int dtype, uint32_t numCu);
 // The launch of `plan`; false (func == nullptr) where the kernels' records cannot hold it.
 bool BuildDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaunch *d);
 // The packed form of a launch that BuildDirect has made, where the plan's items are alike.
-void PackDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaunch *d);
+void PackDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaunch *d, uint32_t numCu = 256);
 // Puts the ranks' pointers in; true if they were there already (the previous call's).
 bool FillBases(DirectLaunch *d, const std::vector<void *> &send, const std::vector<void *> &recv);
 

@@ -168,11 +168,53 @@ void CheckLimits()
     }
 }
 
+// Both sides of the windows in which the packed form goes on, by sixteenths of a tile for each CU.
+void CheckWindows()
+{
+    struct Line {
+        int coll;
+        uint32_t least, most;
+        int dtype;
+        bool ragged;
+        std::vector<uint32_t> edges;      // out, in, out, ...
+    };
+    const int ar = COLL_ALLREDUCE, rs = COLL_REDUCESCATTER, fp32 = HCCL_DATA_TYPE_FP32, int8 = HCCL_DATA_TYPE_INT8;
+    const std::vector<Line> lines = {
+        {ar, 2, 2, fp32, false, {192}}, {ar, 3, 3, fp32, false, {14}}, {ar, 4, 4, fp32, false, {24, 32, 96}}, {ar, 5, 7, fp32, false, {9}},
+        {ar, 8, 8, int8, false, {11, 16, 22, 32, 48}}, {ar, 9, 15, fp32, false, {6}}, {ar, 16, 16, fp32, false, {11, 16, 22}},
+        {ar, 16, 16, HCCL_DATA_TYPE_BFP16, false, {6, 16, 22}}, {ar, 16, 16, HCCL_DATA_TYPE_FP16, false, {6, 16, 22}}, {ar, 17, 32, fp32, false, {6}},
+        {rs, 2, 2, fp32, false, {60, 64, 256}}, {rs, 3, 3, fp32, false, {24}}, {rs, 4, 4, fp32, false, {30, 32, 44}}, {rs, 5, 7, fp32, false, {18}},
+        {rs, 8, 8, int8, false, {24}}, {rs, 9, 15, fp32, false, {}}, {rs, 16, 16, fp32, false, {11, 16, 20}}, {rs, 17, 32, fp32, false, {}},
+        {rs, 2, 2, fp32, true, {56}}, {rs, 3, 4, int8, true, {24}}, {rs, 5, 7, fp32, true, {14}}, {rs, 8, 8, fp32, true, {14, 16, 20}},
+        {rs, 8, 8, int8, true, {14}}, {rs, 9, 15, fp32, true, {}}, {rs, 16, 16, fp32, true, {10}}, {rs, 17, 32, fp32, true, {}},
+    };
+    for (uint32_t numCu : {256u, 128u, 32u}) {
+        const uint64_t sixteenth = uint64_t(numCu) * 1024;
+        for (const Line &l : lines) {
+            for (uint32_t p = l.least; p <= l.most; p++) {
+                const uint64_t share = l.coll == rs ? p : 1;
+                auto in = [&](uint64_t bytes) { return PackedFits(l.coll, p, bytes - (l.ragged ? 12 : 0), l.dtype, numCu); };
+                bool inside = !l.edges.empty();
+                CHECK(in(4096) == inside);
+                for (uint32_t e : l.edges) {
+                    const uint64_t upTo = e * sixteenth / share / 16 * 16;
+                    CHECK(in(upTo) == inside);
+                    inside = !inside;
+                    CHECK(in(upTo + (l.ragged ? 32 : 16)) == inside);
+                }
+                CHECK(!in(uint64_t(1) << 32));
+            }
+        }
+        CHECK(!PackedFits(COLL_ALLREDUCE, 1, 4096, fp32, numCu) && !PackedFits(COLL_ALLREDUCE, 33, 4096, fp32, numCu) && !PackedFits(COLL_REDUCE, 8, 4096, fp32, numCu));
+    }
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
 {
     CheckLimits();
+    CheckWindows();
     const long want = argc > 1 ? std::atol(argv[1]) : 3000;
     long taken[3] = {0, 0, 0}, unlike = 0, apart = 0, trees = 0, inPlace = 0;
     for (long n = 0; n < want;) {

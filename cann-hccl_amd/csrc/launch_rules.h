@@ -66,6 +66,9 @@ constexpr uint32_t kTeamMinHalfRoundsCopy = 2;
 // 128 MiB (16) 487 / 440; 5 ranks 16 MiB (2.5) 86.9 / 89.3, 27 MiB (4.2) 150 ... 166 / 145, 60 MiB 329 ... 339 / 307; 6 ranks 16 MiB (3) 115 ... 121 / 120, 22 MiB
 // (4.1) 166 / 159, 55 MiB 404 / 382.  Off a boundary: 4 ranks 26 MiB 91 ... 94 / 102, 40 MiB (5) 147 / 154, 64 MiB (8) 245 ... 255 / 243, 80 MiB 287 / 299, 100 MiB
 // 389 / 374; 5 ranks 40 MiB (6.25) 206 ... 231 / 217 ... 220, 60 MiB (9.4) 314 / 320; 6 ranks 24 MiB (4.5) 183 / 184, 30 MiB 215 / 225, 40 MiB (7.5) 311 / 301.
+// Broadcasts, whose one item is read from one buffer, gain more from the same lines on (plain / team, three sets of buffers and every rank as the root in turn): 5 ranks 128 MiB
+// (4) 129.2 / 116.2, 256 MiB 267 / 219, 600 MiB 635 / 497; 6 ranks 160.0 / 135.2, 322 / 259, 760 / 588; 7 ranks 188.2 / 154.8, 382 / 298, 893 / 684; off a boundary, 256 MiB (8)
+// 5 ranks 267 / 221, 6 ranks 321 / 261, 7 ranks 384 / 301.
 constexpr uint32_t kTeamMinHalfRoundsCopyFew = 8, kTeamMinHalfRoundsCopyFewUneven = 16;
 
 // Whether a launch whose items with whole tiles have `bytes` in all runs that long.  (By bytes, not by tiles: a buffer that starts

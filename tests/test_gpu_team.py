@@ -288,3 +288,29 @@ def test_gathers_of_four_to_six_blocks_take_the_team_form_beyond_their_line(p, o
                 assert int(recvs[r][:off].count_nonzero()) == 0 and int(recvs[r][off + n * p:].count_nonzero()) == 0, r
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("p,off", [(5, 0), (6, 0), (7, 0), (5, 1), (7, 1), (4, 0), (8, 0)])
+def test_broadcasts_to_four_to_six_ranks_take_the_team_form_beyond_their_line(p, off):
+    # the same lines as the gathers': 3 destinations stay plain, 7 change at one round
+    g = gh.Group(p, team="auto", team_tiles=1)
+    line = (8 if off else 1 if p > 7 else 4) * torch.cuda.get_device_properties(0).multi_processor_count * 16384
+    try:
+        for step, team in ((-128, 0), (128, int(p > 4))):
+            n, root = line + step + off, p - 2
+            if n * p <= 20 << 20:
+                continue        # (goes out with its records in the arguments)
+            print("broadcast", p, "off", off, "n", n, flush=True)
+            gen = torch.Generator(device="cuda").manual_seed(n)
+            bufs = [torch.zeros(n + off + 16, dtype=torch.int8, device="cuda") for _ in range(p)]
+            want = torch.randint(-128, 128, (n,), dtype=torch.int8, device="cuda", generator=gen)
+            bufs[root][off:off + n] = want
+            torch.cuda.synchronize()
+            H.broadcast(g.comms, [t.data_ptr() + off for t in bufs], n, INT8, root, g.stream_ptr)
+            assert g.info()["teamLaunches"] == team and g.info()["launches"] == 1, (n, g.info())
+            torch.cuda.synchronize()
+            for r in range(p):
+                assert torch.equal(bufs[r][off:off + n], want), r
+                assert int(bufs[r][:off].count_nonzero()) == 0 and int(bufs[r][off + n:].count_nonzero()) == 0, r
+    finally:
+        g.close()

@@ -157,9 +157,9 @@ bool CombiningBound(int coll, uint32_t p, uint64_t bytes, int dtype)
 //     16 ranks: 1.5 MiB 11.0 / 9.5 / 10.2, 2 MiB 12.3 / 13.3 / 11.1, 3 MiB 16.0 / 18.1 / 15.6 (bf16 17.5 / - / 17.7), 4.25 MiB 27.7 / 24.6 / 22.9, 5 MiB
 //       29.6 / 27.5 / 25.7, 6 MiB 33.3 / 35.3 / 31.2 (fp16, bf16 up to 33), 8.5 MiB 54.5 / 57.3 / 53.1; 32 ranks 1.5 MiB 21.3 / 17.7 / -
 //   reduce-scatter (bytes received by all ranks), blocks of whole vectors: 2 ranks 6 MiB 4.5 / 4.0, 14 MiB 8.5 / 7.9, 16 MiB 9.1 / 9.0, 20 MiB 11.7 / 11.1, 64 MiB
-//     32.2 / 30.1; 4 ranks 5 MiB 6.1 / 5.1, 7 MiB 7.0 / 6.6, 8 MiB 7.6 / 7.7, 9 MiB 9.8 / 8.1, 11 MiB 10.5 / 10.2, 12 MiB 11.0 / 11.4; 8 ranks 3 MiB
-//     6.3 / 5.3, 4 MiB 7.3 / 7.0, 5 MiB 9.4 / 8.2, 6 MiB 10.1 / 9.7, 7 MiB 11.2 / 10.9, 8 MiB 12.1 / 13.5; 16 ranks 1 MiB 7.7 / 5.1, 2 MiB 8.6 / 8.3 (bf16
-//     10.1 / 8.4), 3 MiB 9.8 / 9.7, 4.25 MiB 15.5 / 13.5, 5 MiB 16.4 / 15.3, 6 MiB 17.8 / 20.4
+//     32.2 / 30.1; 4 ranks 5 MiB 6.1 / 5.1, 7 MiB 7.0 / 6.6 (int8 6.4 MiB 6.5 / 6.9), 8 MiB 7.6 / 7.7, 9 MiB 9.8 / 8.1, 11 MiB 10.5 / 10.2, 12 MiB 11.0 / 11.4; 8 ranks 3 MiB
+//     6.3 / 5.3, 4 MiB 7.3 / 7.0, 5 MiB 9.4 / 8.2, 6 MiB 10.1 / 9.7 (int8 5.7 MiB 9.8 / 10.6), 7 MiB 11.2 / 10.9, 8 MiB 12.1 / 13.5; 16 ranks 1 MiB 7.7 / 5.1, 2 MiB 8.6 / 8.3 (bf16
+//     10.1 / 8.4), 3 MiB 9.8 / 9.7, 4.05 MiB (fp16) 12.4 / 14.0, 4.25 MiB 15.5 / 13.5, 5 MiB 16.4 / 15.3, 6 MiB 17.8 / 20.4
 //   other blocks: 2 ranks 14 MiB 8.9 / 8.8, 4 ranks 6 MiB 6.9 / 6.8, 8 ranks 3 MiB 6.7 / 5.9, 4 MiB 8.5 / 7.8, 5 MiB 9.8 / 9.0, 16 ranks 2 MiB 9.2 / 7.9,
 //     3 MiB 10.3 / 10.7.  Waves of 4 KiB bring nothing where every block has one destination (8 ranks bf16 pairwise, 4 MiB 6.9 / 7.7).
 // Two kinds of calls gain less and stay out: 16 ranks' all-reduce of a 16-bit floating-point type between 1.5 and 4 MiB, whose waves of 4 KiB wait for their own
@@ -169,48 +169,72 @@ namespace {
 
 enum PackedCalls : uint8_t {
     ALL_REDUCE_HALVES = 1, ALL_REDUCE_OTHERS = 2, ALL_REDUCE = 3,     // of fp16 and bf16; of other types
-    BLOCKS_WHOLE = 4,                                                 // reduce-scatter, blocks of whole 16-byte vectors
+    BLOCKS_WHOLE = 4, BLOCKS_WHOLE_BYTES = 32, BLOCKS = 36,           // reduce-scatter, blocks of whole 16-byte vectors; of 8-bit elements
     BLOCKS_BYTES = 8, BLOCKS_OTHERS = 16, BLOCKS_RAGGED = 24          // other blocks, of 8-bit elements; of other types
 };
 struct PackedWindow {
     uint8_t calls, least, most;      // ranks
     uint16_t above, upTo;            // bytes of an all-reduce, received by all ranks of a reduce-scatter
+    uint16_t upToOff;                // where sends and results lie off half a memory line
 };
 constexpr PackedWindow kPackedWindows[] = {
-    {ALL_REDUCE, 2, 2, 0, 192},
-    {ALL_REDUCE, 3, 3, 0, 14},
-    {ALL_REDUCE, 4, 4, 0, 24}, {ALL_REDUCE, 4, 4, 32, 96},
-    {ALL_REDUCE, 5, 7, 0, 9},
-    {ALL_REDUCE, 8, 8, 0, 11}, {ALL_REDUCE, 8, 8, 16, 22}, {ALL_REDUCE, 8, 8, 32, 48},
-    {ALL_REDUCE, 9, 32, 0, 6}, {ALL_REDUCE_OTHERS, 16, 16, 6, 11}, {ALL_REDUCE, 16, 16, 16, 22},
-    {BLOCKS_WHOLE, 2, 2, 0, 60}, {BLOCKS_WHOLE, 2, 2, 64, 256},
-    {BLOCKS_WHOLE, 3, 3, 0, 24},
-    {BLOCKS_WHOLE, 4, 4, 0, 30}, {BLOCKS_WHOLE, 4, 4, 32, 44},
-    {BLOCKS_WHOLE, 5, 7, 0, 18},
-    {BLOCKS_WHOLE, 8, 8, 0, 24},
-    {BLOCKS_WHOLE, 16, 16, 0, 11}, {BLOCKS_WHOLE, 16, 16, 16, 20},
-    {BLOCKS_RAGGED, 2, 2, 0, 56},
-    {BLOCKS_RAGGED, 3, 4, 0, 24},
-    {BLOCKS_RAGGED, 5, 8, 0, 14}, {BLOCKS_OTHERS, 8, 8, 16, 20},
-    {BLOCKS_RAGGED, 16, 16, 0, 10},
+    {ALL_REDUCE, 2, 2, 0, 192, 64},
+    {ALL_REDUCE, 3, 3, 0, 14, 14},
+    {ALL_REDUCE, 4, 4, 0, 24, 21}, {ALL_REDUCE, 4, 4, 32, 96, 32},
+    {ALL_REDUCE, 5, 7, 0, 9, 9},
+    {ALL_REDUCE, 8, 8, 0, 11, 11}, {ALL_REDUCE, 8, 8, 16, 22, 21}, {ALL_REDUCE, 8, 8, 32, 48, 42},
+    {ALL_REDUCE, 9, 32, 0, 6, 6}, {ALL_REDUCE_OTHERS, 16, 16, 6, 11, 11}, {ALL_REDUCE, 16, 16, 16, 22, 21},
+    {BLOCKS, 2, 2, 0, 60, 60}, {BLOCKS, 2, 2, 64, 256, 64},
+    {BLOCKS, 3, 3, 0, 24, 24},
+    {BLOCKS, 4, 4, 0, 24, 24}, {BLOCKS_WHOLE, 4, 4, 24, 30, 26}, {BLOCKS, 4, 4, 32, 44, 41},
+    {BLOCKS, 5, 7, 0, 18, 18},
+    {BLOCKS, 8, 8, 0, 21, 21}, {BLOCKS_WHOLE, 8, 8, 21, 24, 21},
+    {BLOCKS, 16, 16, 0, 11, 11}, {BLOCKS, 16, 16, 17, 20, 20},
+    {BLOCKS_RAGGED, 2, 2, 0, 56, 56},
+    {BLOCKS_RAGGED, 3, 4, 0, 24, 24},
+    {BLOCKS_RAGGED, 5, 8, 0, 14, 14}, {BLOCKS_OTHERS, 8, 8, 16, 20, 20},
+    {BLOCKS_RAGGED, 16, 16, 0, 10, 10},
 };
 uint64_t SixteenthTiles(uint32_t numCu) { return uint64_t(numCu) * kTileBytes / 16; }
 
 }  // namespace
 
-bool PackedFits(int coll, uint32_t p, uint64_t bytes, int dtype, uint32_t numCu)
+// Buffers off a boundary.  The tile kernels bring their vectors to one, the packed ones access them as they come, which costs little as long as they lie on
+// 4 bytes: tiles / packed, all-reduce, bf16, 8 ranks 2.5 MiB on 512 bytes 7.8 / 7.4, 4 bytes off 7.9 / 7.8, 2 bytes off 7.9 / 11.7, 5 MiB 15.6 / 13.3, 15.7 / 14.0, 15.7 / 19.0.  Of an
+// all-reduce it takes sends and results off 4 bytes for packed to fall behind (8 ranks 2.5 MiB, only sends 7.9 / 7.6, only results 7.9 / 6.4), and then not below some size: 2 ranks
+// 3 MiB 0.87 of the tiles' time, 4 MiB 1.02 ... 1.10; 3 ranks 2.25 MiB 0.95 ... 1.00, 3.25 MiB 1.2; 4 ranks 1.75 MiB 0.75 ... 0.94, 2.25 MiB 1.12 ... 1.19; 6 and 8 ranks 1.5 MiB 0.94 ... 1.00,
+// 8 ranks 1.75 MiB 1.06 ... 1.10; 12 to 32 ranks 1.25 MiB 0.82 ... 1.02, 16 ranks 1.5 MiB 0.99 ... 1.12.  A reduce-scatter of whole vectors reads its sources off 4 bytes whatever its results: 2 ranks
+// 3 MiB 0.88 ... 1.00, 5 MiB 0.94 ... 1.05; 3 ranks 2 MiB 0.80 ... 0.95, 2.5 MiB 1.09, 5 MiB 0.98 ... 1.11; 4 to 16 ranks 3 MiB 0.90 ... 1.04, 4 ranks 4 MiB 1.03 ... 1.19, 8 ranks 3.5 MiB 1.06 ... 1.11,
+// 5.5 MiB 1.16 ... 1.22.  Blocks of parts of vectors lie off by themselves, and their windows hold wherever the buffers lie.
+// Stores that straddle memory lines cost something at any size: sends and results off half a line leave the upper ends of the larger windows to the tiles (packed as a share of the tiles' time, random sizes,
+// types and placements; all-reduce, 4 ranks 20 ... 24 quarters of a MiB on / off lines 0.91 / 1.00, 32 ... 96 0.92 / 1.02, 8 ranks 45 ... 48 0.93 / 1.06, 16 ranks 21 and 22 0.94 / 1.04, 2 ranks 190 0.90 / 1.02;
+// reduce-scatter, 4 ranks 26 ... 30 1.02 / 1.07, 41 ... 44 0.99 / 1.07, 8 ranks 21 ... 24 1.00 / 1.06, 2 ranks 200 0.96 / 1.04).  In place, where reads and stores of one line are by different waves, more: 2 ranks 9 ... 19 1.04, 3 ranks 8 ... 10
+// 1.03, 12 ... 14 1.08, 4 ranks 8 ... 16 1.03 ... 1.20, 6 ranks 8 and 9 1.03, 8 ranks 8 ... 11 1.07, 16 ranks 6 ... 11 1.06 ... 1.17, 16 ... 22 0.98 ... 1.17.
+bool PackedFits(int coll, uint32_t p, uint64_t bytes, int dtype, uint32_t numCu, uint64_t sends, uint64_t recvs, bool inPlace)
 {
     uint8_t call = 0;
     uint64_t total = bytes;
     if (coll == COLL_ALLREDUCE) {
         call = dtype == HCCL_DATA_TYPE_FP16 || dtype == HCCL_DATA_TYPE_BFP16 ? ALL_REDUCE_HALVES : ALL_REDUCE_OTHERS;
     } else if (coll == COLL_REDUCESCATTER) {
-        call = bytes % 16 == 0 ? BLOCKS_WHOLE : (dtype == HCCL_DATA_TYPE_INT8 || dtype == HCCL_DATA_TYPE_UINT8 ? BLOCKS_BYTES : BLOCKS_OTHERS);
+        const bool bytesOnly = dtype == HCCL_DATA_TYPE_INT8 || dtype == HCCL_DATA_TYPE_UINT8;
+        call = bytes % 16 == 0 ? (bytesOnly ? BLOCKS_WHOLE_BYTES : BLOCKS_WHOLE) : (bytesOnly ? BLOCKS_BYTES : BLOCKS_OTHERS);
         total *= p;
     }
     const uint64_t unit = SixteenthTiles(numCu);
+    const bool off = (sends & 3u) != 0 && (coll == COLL_ALLREDUCE ? (recvs & 3u) != 0 : call == BLOCKS_WHOLE || call == BLOCKS_WHOLE_BYTES);
+    const bool offLine = (sends & 63u) != 0 && (recvs & 63u) != 0;
+    uint64_t most = 0;
+    if (off) {
+        most = coll != COLL_ALLREDUCE ? (p == 3 ? 8 : 12) : (p == 2 ? 12 : p <= 4 ? 7 : p <= 8 ? 6 : 5);
+    } else if (offLine && inPlace && coll == COLL_ALLREDUCE) {
+        most = p == 2 ? 12 : p == 3 ? 8 : p == 4 ? 7 : p <= 7 ? 8 : p == 8 ? 7 : p == 16 ? 5 : 0;
+    }
+    if (most != 0 && total > most * unit) {
+        return false;
+    }
     for (const PackedWindow &w : kPackedWindows) {
-        if ((w.calls & call) != 0 && p >= w.least && p <= w.most && total > w.above * unit && total <= w.upTo * unit) {
+        if ((w.calls & call) != 0 && p >= w.least && p <= w.most && total > w.above * unit && total <= (offLine ? w.upToOff : w.upTo) * unit) {
             return true;
         }
     }

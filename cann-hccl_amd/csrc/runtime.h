@@ -152,8 +152,9 @@ struct DirectLaunch {
 bool DirectFits(int coll, uint32_t p, uint64_t bytes, int dtype);
 // Whether it is left to the tile kernels all the same: reductions to one destination whose combining the waves wait for.
 bool CombiningBound(int coll, uint32_t p, uint64_t bytes, int dtype);
-// Whether a larger one goes out in the packed form if its items are alike.
-bool PackedFits(int coll, uint32_t p, uint64_t bytes, int dtype, uint32_t numCu);
+// Whether a larger one goes out in the packed form if its items are alike.  sends, recvs: the ranks' buffers' addresses, or-ed;
+// inPlace: an all-reduce that is.
+bool PackedFits(int coll, uint32_t p, uint64_t bytes, int dtype, uint32_t numCu, uint64_t sends = 0, uint64_t recvs = 0, bool inPlace = false);
 // The launch of `plan`; false (func == nullptr) where the kernels' records cannot hold it.
 bool BuildDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaunch *d);
 // The packed form of a launch that BuildDirect has made, where the plan's items are alike.

@@ -183,8 +183,8 @@ void CheckWindows()
         {ar, 2, 2, fp32, false, {192}}, {ar, 3, 3, fp32, false, {14}}, {ar, 4, 4, fp32, false, {24, 32, 96}}, {ar, 5, 7, fp32, false, {9}},
         {ar, 8, 8, int8, false, {11, 16, 22, 32, 48}}, {ar, 9, 15, fp32, false, {6}}, {ar, 16, 16, fp32, false, {11, 16, 22}},
         {ar, 16, 16, HCCL_DATA_TYPE_BFP16, false, {6, 16, 22}}, {ar, 16, 16, HCCL_DATA_TYPE_FP16, false, {6, 16, 22}}, {ar, 17, 32, fp32, false, {6}},
-        {rs, 2, 2, fp32, false, {60, 64, 256}}, {rs, 3, 3, fp32, false, {24}}, {rs, 4, 4, fp32, false, {30, 32, 44}}, {rs, 5, 7, fp32, false, {18}},
-        {rs, 8, 8, int8, false, {24}}, {rs, 9, 15, fp32, false, {}}, {rs, 16, 16, fp32, false, {11, 16, 20}}, {rs, 17, 32, fp32, false, {}},
+        {rs, 2, 2, fp32, false, {60, 64, 256}}, {rs, 3, 3, fp32, false, {24}}, {rs, 4, 4, fp32, false, {30, 32, 44}}, {rs, 4, 4, int8, false, {24, 32, 44}}, {rs, 5, 7, fp32, false, {18}},
+        {rs, 8, 8, fp32, false, {24}}, {rs, 8, 8, int8, false, {21}}, {rs, 9, 15, fp32, false, {}}, {rs, 16, 16, fp32, false, {11, 17, 20}}, {rs, 17, 32, fp32, false, {}},
         {rs, 2, 2, fp32, true, {56}}, {rs, 3, 4, int8, true, {24}}, {rs, 5, 7, fp32, true, {14}}, {rs, 8, 8, fp32, true, {14, 16, 20}},
         {rs, 8, 8, int8, true, {14}}, {rs, 9, 15, fp32, true, {}}, {rs, 16, 16, fp32, true, {10}}, {rs, 17, 32, fp32, true, {}},
     };
@@ -209,12 +209,50 @@ void CheckWindows()
     }
 }
 
+// Buffers off a boundary, both sides of the lines that hold for them.
+void CheckOffBoundary()
+{
+    const uint64_t q = 256 * 1024;
+    const int ar = COLL_ALLREDUCE, rs = COLL_REDUCESCATTER, type = HCCL_DATA_TYPE_BFP16;
+    auto in = [&](int coll, uint32_t p, uint64_t quarters, uint64_t more, uint64_t sends, uint64_t recvs) {
+        return PackedFits(coll, p, (quarters * q / (coll == rs ? p : 1)) / 16 * 16 + more, type, 256, 0x7f0000000000ull | sends, 0x7f0000000000ull | recvs);
+    };
+    const uint32_t allReduce[][2] = {{2, 12}, {3, 7}, {4, 7}, {6, 6}, {8, 6}, {12, 5}, {16, 5}, {32, 5}};
+    for (const auto &l : allReduce) {
+        CHECK(in(ar, l[0], l[1], 0, 2, 2) && !in(ar, l[0], l[1], 16, 2, 2) && !in(ar, l[0], l[1], 16, 3, 1));
+        CHECK(in(ar, l[0], l[1], 16, 4, 4) && in(ar, l[0], l[1], 16, 2, 4) && in(ar, l[0], l[1], 16, 8, 1));
+    }
+    CHECK(!in(ar, 4, 20, 0, 6, 2) && in(ar, 4, 20, 0, 4, 4) && !in(ar, 8, 20, 0, 1, 1) && in(ar, 8, 20, 0, 1, 0) && !in(ar, 8, 40, 0, 2, 2) && in(ar, 8, 40, 0, 4, 4));
+    const uint32_t blocks[][2] = {{2, 12}, {3, 8}, {4, 12}, {6, 12}, {8, 12}};
+    for (const auto &l : blocks) {
+        CHECK(in(rs, l[0], l[1], 0, 2, 0) && !in(rs, l[0], l[1], 16, 2, 0) && in(rs, l[0], l[1], 16, 0, 2) && in(rs, l[0], l[1], 16, 4, 4) && in(rs, l[0], l[1], 2, 2, 2));
+    }
+    CHECK(!in(rs, 16, 18, 0, 6, 0) && in(rs, 16, 18, 0, 4, 0) && !in(rs, 8, 20, 0, 2, 0));
+    // off half a memory line the upper ends go, in place more
+    CHECK(in(ar, 2, 64, 0, 4, 4) && !in(ar, 2, 64, 16, 4, 4) && in(ar, 2, 64, 16, 64, 4) && in(ar, 2, 64, 16, 4, 0) && !in(ar, 4, 80, 0, 16, 16) && in(ar, 4, 80, 0, 64, 64));
+    CHECK(in(rs, 2, 200, 0, 0, 16) && !in(rs, 2, 200, 0, 8, 16) && in(rs, 2, 200, 0, 64, 16));
+    const uint32_t ends[][5] = {{uint32_t(ar), 4, 24, 21, 0}, {uint32_t(ar), 8, 22, 21, 0}, {uint32_t(ar), 8, 48, 42, 0}, {uint32_t(ar), 16, 22, 21, 0}, {uint32_t(rs), 4, 30, 26, 0},
+                                {uint32_t(rs), 4, 44, 41, 0}, {uint32_t(rs), 8, 24, 21, 0}};
+    for (const auto &l : ends) {
+        CHECK(in(l[0], l[1], l[2], 0, 0, 0) && !in(l[0], l[1], l[2], 16, 0, 0) && in(l[0], l[1], l[3], 0, 4, 4) && !in(l[0], l[1], l[3], 16, 4, 4) && in(l[0], l[1], l[3], 16, 64, 4));
+    }
+    auto inPlace = [&](uint32_t p, uint64_t quarters, uint64_t more, uint64_t at) {
+        return PackedFits(ar, p, quarters * q + more, type, 256, 0x7f0000000000ull | at, 0x7f0000000000ull | at, true);
+    };
+    const uint32_t same[][2] = {{2, 12}, {3, 8}, {4, 7}, {6, 8}, {8, 7}, {16, 5}};
+    for (const auto &l : same) {
+        CHECK(inPlace(l[0], l[1], 0, 4) && !inPlace(l[0], l[1], 16, 4) && !inPlace(l[0], l[1], 16, 16) && inPlace(l[0], l[1], 16, 64));
+    }
+    CHECK(inPlace(12, 6, 0, 4) && inPlace(32, 6, 0, 16) && !inPlace(4, 15, 0, 4) && !inPlace(8, 20, 0, 4) && in(ar, 8, 20, 0, 4, 4));
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
 {
     CheckLimits();
     CheckWindows();
+    CheckOffBoundary();
     const long want = argc > 1 ? std::atol(argv[1]) : 3000;
     long taken[3] = {0, 0, 0}, unlike = 0, apart = 0, trees = 0, inPlace = 0;
     for (long n = 0; n < want;) {

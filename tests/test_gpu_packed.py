@@ -146,7 +146,7 @@ ALL_REDUCE = {2: [(8, PACKED), (32, WIDE), (192, PACKED)], 4: [(8, PACKED), (24,
               8: [(8, PACKED), (11, WIDE), (16, TABLES), (22, WIDE), (32, TABLES), (48, PACKED)], 16: [(6, PACKED), (11, WIDE), (16, TABLES), (22, WIDE)]}
 ALL_REDUCE_HALVES = {**ALL_REDUCE, 16: [(6, PACKED), (16, TABLES), (22, WIDE)]}
 WHOLE_BLOCKS = {2: [(60, PACKED), (64, TABLES), (256, PACKED)], 3: [(24, PACKED)], 4: [(30, PACKED), (32, TABLES), (44, PACKED)], 6: [(18, PACKED)],
-                8: [(24, PACKED)], 16: [(11, PACKED), (16, TABLES), (20, PACKED)]}
+                8: [(24, PACKED)], 16: [(11, PACKED), (17, TABLES), (20, PACKED)]}
 RAGGED_BLOCKS = {2: [(56, PACKED)], 3: [(24, PACKED)], 4: [(24, PACKED)], 6: [(16, PACKED)], 8: [(20, PACKED)], 16: [(16, PACKED)]}
 
 
@@ -207,5 +207,29 @@ def test_form_of_others():
         g.set(servers=1)
         _as_the_tiles(g, lambda: gh.all_gather(g, ins, FP32), PACKED, ("all-gather",))
         _as_the_tiles(g, lambda: gh.all_reduce(g, ins, FP32, SUM)[0], PACKED, ("one server",))
+    finally:
+        g.close()
+
+
+@pytest.mark.parametrize("p,quarters,up", [(2, 12, 40), (4, 7, 20), (8, 6, 20), (16, 5, 18), (6, 6, 8), (4, 7, 80)])
+def test_form_off_a_boundary(p, quarters, up):
+    """All-reduces whose buffers lie off 4 bytes are packed up to a size only; those off 4 or 16 bytes stop at four tiles per CU."""
+    g = gh.Group(p)
+    try:
+        for dt, op, pad in ((BF16, MAX, 2), (INT8, SUM, 3), (FP32, SUM, 4)):
+            unit = gh.H.DTYPE_SIZE[dt]
+            for q in (quarters, up):
+                n = q * MIB // 4 // unit
+                want = TABLES if q == up and (pad != 4 or q > 64) else None
+                ins = _ins(dt, p, n, 29 * p + pad, False)
+                print("off a boundary", p, "type", dt, "n", n, "pad", pad, flush=True)
+                outs, _ = gh.all_reduce(g, ins, dt, op, pad=pad)
+                form = gh.H.last_op_form(g.comms[0])
+                assert form == TABLES if want == TABLES else form in (PACKED, WIDE), (dt, n, pad, form)
+                g.set(direct=0)
+                tiles, _ = gh.all_reduce(g, ins, dt, op, pad=pad)
+                g.set(direct="auto")
+                for r in range(p):
+                    assert np.array_equal(outs[r].view(np.uint8), tiles[r].view(np.uint8)), (dt, n, r)
     finally:
         g.close()

@@ -22,9 +22,7 @@ constexpr uint64_t kDirectMaxToOne = uint64_t(4) << 20;       // the same where 
 //   reduce, fp32, 2.5 MiB: 8 ranks 5.9 / 4.7, 32 ranks 15.6 / 14.9
 // Up to the larger limit this form stays ahead for bf16 of up to 8 ranks and for 8-bit elements (4 MiB: bf16, 4 ranks 5.2 / 4.3, 8 ranks 7.6 / 7.5; int8, 8 ranks 7.9 / 7.6, 12
 // ranks 3.5 MiB 10.2 / 9.9, 4 MiB 10.6 / 11.4, 32 ranks 23.3 / 21.7, 24.4 / 27.8), for ragged blocks of few ranks (int8, 8 ranks 3.5 MiB 8.0 / 7.9, 32 ranks 3 MiB 23.7 / 23.3, 3.5
-// MiB 25.0 / 26.8) and for three sources or fewer (3 ranks, 4 MiB 4.7 / 3.9).  bf16 of more than 8 ranks stops before (CombiningBound) where its combining is what the waves wait for: 16 ranks 3 MiB
-// 11.2 / 10.0, 3.25 MiB 11.6 / 11.2, 3.5 MiB 11.6 / 12.1, 4 MiB 12.5 / 14.5, 32 ranks 20.1 / 19.0, 3.5 MiB 19.9 / 21.1, 4 MiB 21.7 / 26.2; ragged, 16 ranks 2.5 MiB 10.9 / 10.3, 3 MiB 11.5 /
-// 12.1, 24 ranks 15.2 / 13.8, 15.7 / 18.7.
+// MiB 25.0 / 26.8) and for three sources or fewer (3 ranks, 4 MiB 4.7 / 3.9).
 // Copies, also from one to one, are ahead up to their limit (20 MiB read and written: broadcast, 2 ranks 5.3 / 5.1, 32 ranks 7.7 / 5.6, send 5.0 / 4.6, scatter 5.1 / 5.0 ... 5.3), and a
 // call with new buffers uploads nothing; with known buffers a small one costs 0.2 more than with tables (its arguments are 1.3 KB).
 constexpr uint64_t kDirectMaxToOneEven = uint64_t(5) << 19;
@@ -138,11 +136,21 @@ bool DirectFits(int coll, uint32_t p, uint64_t bytes, int dtype)
     }
 }
 
-bool CombiningBound(int coll, uint32_t p, uint64_t bytes, int dtype)
+// bf16, of which every combining rounds: with 16 and more sources the waves of this form come to wait for it where the tile kernels' larger ones still have loads in flight.  This form's
+// time as a share of the tiles', reduce-scatter of whole vectors / of others / reduce, sum: 16 ranks 3 MiB 0.92 / 1.03 / 0.92, 3.25 MiB 0.97 / 1.05 / 1.01, 3.75 MiB 1.07 / 1.21 / 1.10; 24 ranks 2.75 MiB
+// 0.87 / 0.99 / 0.85, 3 MiB 0.90 / 1.15 / 0.91, 3.5 MiB 1.02 / 1.14 / 1.04; 32 ranks 3 MiB 0.90 / 1.05 / 0.92, 3.25 MiB 0.97 / 1.09 / 1.00, 4 MiB 1.11 / 1.44 / 1.07.  Fewer ranks stay ahead up to 4 MiB (9 ranks
+// 3.5 MiB 0.93 / 0.97 / 0.91, 12 ranks 3.25 MiB 0.91 / 0.93 / 0.94, 4 MiB 0.99 / 1.02 / 1.02, 14 ranks 1.01 / 1.00 / 1.04), and so do maxima and minima, which round nothing (16 ranks 3.5 MiB 0.88 / 0.98 /
+// 0.90, 32 ranks 0.92 / 1.03 / 0.91), but for blocks of parts of vectors of 28 and more (28 ranks 3.25 MiB 0.98, 3.5 MiB 1.17, 32 ranks 3.25 MiB 0.96, 4 MiB 1.33).
+bool CombiningBound(int coll, uint32_t p, uint64_t bytes, int dtype, int op)
 {
-    const uint64_t total = coll == COLL_REDUCESCATTER ? bytes * p : bytes;
-    return (coll == COLL_REDUCESCATTER || coll == COLL_REDUCE) && p > 8 && dtype == HCCL_DATA_TYPE_BFP16 &&
-        total > (bytes % 16 == 0 ? kDirectMaxToOneBf16 : kDirectMaxToOneBf16Ragged);
+    if ((coll != COLL_REDUCESCATTER && coll != COLL_REDUCE) || p < 16 || dtype != HCCL_DATA_TYPE_BFP16) {
+        return false;
+    }
+    const bool selects = op == HCCL_REDUCE_MAX || op == HCCL_REDUCE_MIN, ragged = coll == COLL_REDUCESCATTER && bytes % 16 != 0;
+    if (selects && (!ragged || p < 28)) {
+        return false;
+    }
+    return (coll == COLL_REDUCESCATTER ? bytes * p : bytes) > (ragged && !selects ? kDirectMaxToOneBf16Ragged : kDirectMaxToOneBf16);
 }
 
 // Beyond those limits, where the items are alike (PackDirect): waves of 1 or 4 KiB keep every CU equally busy where the tile kernels' tiles of

@@ -1247,7 +1247,7 @@ DirectLaunch *FindDirect(Group *g, int algo)
         sends |= reinterpret_cast<uint64_t>(g->ctx->send[r]);
         recvs |= reinterpret_cast<uint64_t>(g->ctx->recv[r]);
     }
-    const bool small = DirectFits(sig.coll, g->p, bytes, sig.dtype) && !CombiningBound(sig.coll, g->p, bytes, sig.dtype);
+    const bool small = DirectFits(sig.coll, g->p, bytes, sig.dtype) && !CombiningBound(sig.coll, g->p, bytes, sig.dtype, sig.op);
     if (!small && !PackedFits(sig.coll, g->p, bytes, sig.dtype, g->numCu, sends, recvs, inPlace != 0)) {
         return nullptr;
     }

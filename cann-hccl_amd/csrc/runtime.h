@@ -151,7 +151,7 @@ struct DirectLaunch {
 // Whether a collective is small enough for this form, whatever its schedule (bytes: of the call's count).
 bool DirectFits(int coll, uint32_t p, uint64_t bytes, int dtype);
 // Whether it is left to the tile kernels all the same: reductions to one destination whose combining the waves wait for.
-bool CombiningBound(int coll, uint32_t p, uint64_t bytes, int dtype);
+bool CombiningBound(int coll, uint32_t p, uint64_t bytes, int dtype, int op);
 // Whether a larger one goes out in the packed form if its items are alike.  sends, recvs: the ranks' buffers' addresses, or-ed;
 // inPlace: an all-reduce that is.
 bool PackedFits(int coll, uint32_t p, uint64_t bytes, int dtype, uint32_t numCu, uint64_t sends = 0, uint64_t recvs = 0, bool inPlace = false);

@@ -155,15 +155,19 @@ template <uint32_t P> bool Same(const Plan &plan, const DirectLaunch &d, const s
 void CheckLimits()
 {
     const uint64_t mib = uint64_t(1) << 20;
-    for (uint32_t p : {2u, 8u, 9u, 16u, 32u}) {
+    for (uint32_t p : {2u, 8u, 9u, 14u, 16u, 27u, 28u, 32u}) {
         for (int dtype : {HCCL_DATA_TYPE_BFP16, HCCL_DATA_TYPE_INT8, HCCL_DATA_TYPE_FP32}) {
-            const bool bf16 = dtype == HCCL_DATA_TYPE_BFP16 && p > 8, even = dtype == HCCL_DATA_TYPE_FP32 && p > 3;
-            const uint64_t whole = even ? 5 * mib / 2 : bf16 ? 13 * mib / 4 : 4 * mib, ragged = bf16 ? 11 * mib / 4 : 4 * mib;
-            auto fits = [&](int coll, uint64_t bytes) { return DirectFits(coll, p, bytes, dtype) && !CombiningBound(coll, p, bytes, dtype); };
-            CHECK(fits(COLL_REDUCE, whole) && !fits(COLL_REDUCE, whole + 16));
-            CHECK(fits(COLL_REDUCE, ragged - 4) && !fits(COLL_REDUCE, ragged + 4));
-            CHECK(fits(COLL_REDUCESCATTER, whole / p / 16 * 16) && !fits(COLL_REDUCESCATTER, whole / p / 16 * 16 + 16));
-            CHECK(!CombiningBound(COLL_ALLREDUCE, p, 8 * mib, dtype));
+            for (int op : {HCCL_REDUCE_SUM, HCCL_REDUCE_PROD, HCCL_REDUCE_MAX, HCCL_REDUCE_MIN}) {
+                const bool bf16 = dtype == HCCL_DATA_TYPE_BFP16 && p >= 16, even = dtype == HCCL_DATA_TYPE_FP32 && p > 3;
+                const bool selects = op == HCCL_REDUCE_MAX || op == HCCL_REDUCE_MIN;
+                const uint64_t whole = even ? 5 * mib / 2 : bf16 && !selects ? 13 * mib / 4 : 4 * mib;
+                const uint64_t ragged = !bf16 ? 4 * mib : !selects ? 11 * mib / 4 : p >= 28 ? 13 * mib / 4 : 4 * mib;
+                auto fits = [&](int coll, uint64_t bytes) { return DirectFits(coll, p, bytes, dtype) && !CombiningBound(coll, p, bytes, dtype, op); };
+                CHECK(fits(COLL_REDUCE, whole) && !fits(COLL_REDUCE, whole + 16));
+                CHECK(fits(COLL_REDUCESCATTER, whole / p / 16 * 16) && !fits(COLL_REDUCESCATTER, whole / p / 16 * 16 + 16));
+                CHECK(fits(COLL_REDUCESCATTER, ragged / p / 16 * 16 - 4) && !fits(COLL_REDUCESCATTER, ragged / p / 16 * 16 + 20));
+                CHECK(!CombiningBound(COLL_ALLREDUCE, p, 8 * mib, dtype, op));
+            }
         }
     }
 }

@@ -291,6 +291,7 @@ HcclResult BuildTables(Group *g, Prepared *pp, bool reduceColl, int dtype, int o
         shape.chains = !pp->plan->fused.empty() && pp->plan->fused[0].kind == FK_CHAIN;
         shape.allGather = g->ctx->sig.coll == COLL_ALLGATHER;
         shape.reduceScatter = g->ctx->sig.coll == COLL_REDUCESCATTER;
+        shape.bf16Selects = reduceColl && dtype == HCCL_DATA_TYPE_BFP16 && (op == HCCL_REDUCE_MAX || op == HCCL_REDUCE_MIN);
         shape.unit = DtypeSize(dtype);
         shape.capBytes = capBytes;
         shape.numCu = g->numCu;

@@ -159,6 +159,7 @@ struct FusedShape {
     double bytes = 0;           // of the items themselves
     bool reduces = false, chains = false;          // a reduction; of chains (else of trees or stack programs)
     bool allGather = false, reduceScatter = false;
+    bool bf16Selects = false;   // maximum or minimum of bf16
     uint32_t sources = 0;       // of an item
     uint32_t unit = 1;          // bytes of an element
     uint64_t capBytes = 0;      // read and written by one launch, 0: by all
@@ -184,13 +185,22 @@ inline uint32_t FusedPerCu(const FusedShape &f)
     // then: bf16, 28 ranks 2600 MiB 434 / 458 / 494, 48 ranks 440 / 458 / 470, 52 ranks 439 / 452 / 463, 56 ranks 512 / 521 / 509, 60 ranks 514 / 517 / 500, 64 ranks 560
     // MiB 143 / 142 / 134, 2600 MiB 500 / 513 / 487; int8, 36 ranks 537 / 449 / 469, 40 ranks 539 / 427 / 454, 44 ranks 900 MiB 189 / 173 / 158, 1500 MiB 288 / 262 / 247, 48 ranks
     // 400 MiB 98 / 87 / 76, 2600 MiB 520 / 472 / 438, 64 ranks 593 / 533 / 465.
+    // Seven sources are streams enough for two (bf16 540 MiB 103.1 / 96.2 / 98.3, 1500 MiB 291.8 / 268.7 / 274.7, 2600 MiB 502 / 477 / 489, fp32 900 MiB 167.0 / 157.5 / 160.4, reduce, fp32 540 MiB 97.7 / 93.0 / 96.2).
+    // Maxima and minima of bf16 go by a rule of several instructions beyond 8 sources: 10 ranks 900 MiB 175.6 / 164.4 / 168.4, 24 ranks 2600 MiB 488 / 460 / 471, 40 ranks 900 MiB 186 / 167 / 169, 48 ranks
+    // 165.7 / 159.0 / 157.4, 2600 MiB 489 / 473 / 466, 52 ranks 900 MiB 174.6 / 157.4 / 152.7, 8 ranks 163.9 / 158.0 / 159.2, but a reduce of 8 155.1 / 156.9 / 160.5, of 16 167.9 / 159.3 / 161.5, of 48 160.2 / 156.6 / 154.1.
+    // Such elements, and those of one byte, do best with eight somewhat longer the more sources there are (2 / 8 per CU): int8 28 ranks 400 MiB 67.7 / 72.1, 32 ranks 330 MiB 59.7 / 54.4, 400 MiB 66.2 / 64.0,
+    // 430 MiB 72.1 / 77.9, 36 ranks 400 MiB 70.5 / 66.3, 460 MiB 76.9 / 81.8, 40 ranks 400 MiB 74.1 / 67.1, 500 MiB 84.8 / 87.0; bf16 maximum 32 ranks 330 MiB 60.1 / 57.6, 430 MiB 75.3 / 80.7, 40 ranks 74.3 / 70.9, 500
+    // MiB 86.3 / 94.2; reduce, int8, 48 ranks 400 MiB 83.1 / 72.1, 540 MiB 92.5 / 85.7, 64 ranks 112.7 / 96.4, bf16 maximum 48 ranks 450 MiB 86.8 / 82.1, 64 ranks 540 MiB 111.7 / 103.3.
     const bool manyToOne = f.reduces && f.storeBytes * 5.0 <= f.streamBytes;
     const bool toOne = manyToOne && f.chains && (perCu == 1 || (streams <= 5.0 && f.streamBytes > 512.0 * kMiB));
     if (toOne) {
-        if (f.unit == 1 && f.reduceScatter && f.sources > 40 && f.streamBytes > 320.0 * kMiB) {
+        const bool costly = f.unit == 1 || f.bf16Selects;
+        if (costly && ((f.sources >= 32 && f.streamBytes <= 416.0 * kMiB) || (f.sources > 40 && f.streamBytes <= 640.0 * kMiB) ||
+            (f.reduceScatter && f.sources > (f.unit == 1 ? 40u : 44u)))) {
             perCu = 8u;
         } else if (f.streamBytes > 512.0 * kMiB) {
-            perCu = f.unit == 1 ? 2u : f.unit == 2 ? (f.reduceScatter && f.sources > 52 ? 8u : 1u) : (f.sources >= 24 ? 2u : 1u);
+            const bool two = f.sources == 7 || (costly && (f.unit == 1 || f.sources > (f.reduceScatter ? 7u : 8u))) || (f.unit > 2 && f.sources >= 24);
+            perCu = two ? 2u : f.unit == 2 && f.reduceScatter && f.sources > 52 ? 8u : 1u;
         } else {
             perCu = f.streamBytes > 320.0 * kMiB ? 2u : f.unit <= 2 ? 8u : 2u;
         }

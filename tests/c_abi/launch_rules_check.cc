@@ -118,10 +118,11 @@ void CheckStores()
 // Workgroups per CU on either side of the lines.
 void CheckWidth()
 {
-    auto width = [](bool scatter, uint32_t ranks, uint32_t unit, double mibRead) {
+    auto width = [](bool scatter, uint32_t ranks, uint32_t unit, double mibRead, bool bf16Selects = false) {
         FusedShape f;
         f.reduces = f.chains = true;
         f.reduceScatter = scatter;
+        f.bf16Selects = bf16Selects;
         f.sources = ranks;
         f.unit = unit;
         f.bytes = mibRead * 1048576.0 / ranks;
@@ -134,7 +135,17 @@ void CheckWidth()
         CHECK(width(scatter, 8, 4, 512) == 1 && width(scatter, 23, 4, 2400) == 1 && width(scatter, 24, 4, 600) == 2 && width(scatter, 64, 8, 2400) == 2);
         CHECK(width(scatter, 8, 2, 512) == 1 && width(scatter, 52, 2, 2400) == 1 && width(scatter, 53, 2, 2400) == (scatter ? 8u : 1u));
         CHECK(width(scatter, 8, 1, 600) == 2 && width(scatter, 40, 1, 2400) == 2 && width(scatter, 41, 1, 2400) == (scatter ? 8u : 2u));
-        CHECK(width(scatter, 48, 1, 330) == (scatter ? 8u : 2u) && width(scatter, 48, 1, 300) == 8 && width(scatter, 48, 2, 300) == 8 && width(scatter, 48, 4, 300) == 2);
+        CHECK(width(scatter, 48, 1, 300) == 8 && width(scatter, 48, 2, 300) == 8 && width(scatter, 48, 4, 300) == 2);
+        CHECK(width(scatter, 7, 4, 600) == 2 && width(scatter, 7, 2, 2400) == 2 && width(scatter, 7, 1, 600) == 2 && width(scatter, 7, 2, 200) == 8);
+        CHECK(width(scatter, 7, 2, 600, true) == 2 && width(scatter, 8, 2, 600, true) == (scatter ? 2u : 1u) && width(scatter, 9, 2, 600, true) == 2);
+        CHECK(width(scatter, 44, 2, 2400, true) == 2 && width(scatter, 45, 2, 2400, true) == (scatter ? 8u : 2u));
+        for (bool selects : {false, true}) {
+            const uint32_t unit = selects ? 2 : 1;
+            CHECK(width(scatter, 31, unit, 330, selects) == 2 && width(scatter, 32, unit, 330, selects) == 8 && width(scatter, 32, unit, 420, selects) == 2);
+            CHECK(width(scatter, 40, unit, 450, selects) == 2 && width(scatter, 48, unit, 450, selects) == 8 && width(scatter, 64, unit, 600, selects) == 8);
+            CHECK(width(scatter, 64, unit, 700, selects) == (scatter ? 8u : 2u));
+        }
+        CHECK(width(scatter, 32, 2, 330) == 2 && width(scatter, 48, 2, 450) == 2);
     }
     auto mid = [](bool chains, uint32_t unit, double tilesPerCu) {
         FusedShape f;

@@ -35,9 +35,10 @@ namespace {
 // How wide (bytes moved in all).  Three sets of buffers and tables in turn, us, 16 workgroups of one wave per CU, written through / two of four waves, non-temporal / one of
 // them.  While what is read and written stays in the memory-side cache, the first: lognormal blocks, 16 ranks 26 MiB 10.7 / 11.8 / 12.1, 60 MiB 21.7 / 23.3 / 23.7, 90 MiB 31.0 / 33.5
 // / 33.7, 95 MiB 33.1 / 35.1 / -, 100 MiB 36.7 / 37.0 / -, 105 MiB 39.3 / 38.3 / -; 64 ranks 90 MiB 32.8 / 36.6 / 36.9, 100 MiB 39.9 / 40.7 / -, 110 MiB 44.7 / 44.3 / -; uniform,
-// 8 ranks 60 MiB 20.3 / 22.1 / 22.5, 95 MiB 31.9 / 33.5 / -, 100 MiB 34.5 / 35.3 / -, 105 MiB 37.9 / 37.0 / -.  Beyond, two; one for more than 16 ranks from 128 MiB on: uniform, 4 ranks
-// 512 MiB 182 / 173.5 / 175.3, 8 ranks 512 MiB 182 / 172.8 / 174.7, 2 GiB 723 / 696 / 700, 16 ranks 2 GiB 730 / 704 / 711, but 32 ranks 512 MiB 192 / 188 / 179, 2 GiB 742 / 712 / 699;
-// lognormal, 16 ranks 424 MiB - / 148.7 / 148.1, 32 ranks - / 154.8 / 152.4, 64 ranks 310 MiB - / 119.0 / 117.0.
+// 8 ranks 60 MiB 20.3 / 22.1 / 22.5, 95 MiB 31.9 / 33.5 / -, 100 MiB 34.5 / 35.3 / -, 105 MiB 37.9 / 37.0 / -.  Beyond, two up to 128 MiB.
+// From there on two for uniform blocks of up to 16 ranks, which the workgroups then take in step, one for others (planned copies / two / one): uniform, 4 ranks 512 MiB 86.1 / 87.4 / 88.0 (one way), 1000 MiB
+// 168.3 / 172.1 / 173.5, 8 ranks 512 MiB 86.2 / 87.3 / 88.7, 16 ranks 92.6 / 91.7 / 94.4, 32 ranks 1000 MiB 175.1 / 179.4 / 177.8; lognormal, 2 ranks 95.0 / 97.7 / 96.2 and 183.4 / 187.4 / 185.0, 4 ranks 100.2 / 102.1 /
+// 100.1, 196.3 / 199.7 / 196.2, 8 ranks 99.8 / 101.1 / 98.4, 192.3 / 196.8 / 191.4, 16 ranks 98.3 / 98.9 / 96.2, 187.8 / 190.9 / 185.1, 32 ranks 103.1 / 103.0 / 100.1, 194.9 / 197.5 / 190.1, 64 ranks 214 / 206 / 199.
 constexpr uint64_t kOneWaveTotal = uint64_t(96) << 20, kTwoPerCuTotal = uint64_t(128) << 20;
 constexpr uint64_t kLaunchTotal = uint64_t(256) << 20;    // in one launch (as other collectives that hop from buffer to buffer)
 
@@ -264,9 +265,10 @@ HcclResult Complete(Group *g, A2avSet *s, uint32_t unit, bool *general)
         *general = true;
         return HCCL_SUCCESS;
     }
+    const bool alike = total == uint64_t(longest) * p * p;
     total *= unit;
     s->pieces = uint32_t(pieces);
-    s->width = total <= kOneWaveTotal ? 0 : (p <= 16 || total <= kTwoPerCuTotal ? 2 : 1);
+    s->width = total <= kOneWaveTotal ? 0 : ((p <= 16 && alike) || total <= kTwoPerCuTotal ? 2 : 1);
     s->launches = uint32_t((total + kLaunchTotal - 1) / kLaunchTotal);
     s->moved = total;
     return HCCL_SUCCESS;

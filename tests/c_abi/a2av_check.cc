@@ -3,6 +3,7 @@
 // tables it reads have to be those of its call.  The calls may not wait for the device, and a call known by its numbers counts as known on whatever
 // stream it comes.  argv[1] = ranks, argv[2] = calls, argv[3] = streams, argv[4] = sets of tables in turn.  argv[2] = 0: calls that go the general
 // way instead.  Their tables have to come out as the ranks passed them, and what was found out about those has to hold as long as they are the last ones.
+// argv[2] = -1: how wide launches are.
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
@@ -296,6 +297,44 @@ int General(Group *g)
     return checks == 2 ? 0 : 1;
 }
 
+// Workgroups per CU on both sides of the lines, 0: sixteen of one wave.  One block longer by four bytes and one shorter: no longer uniform.
+int Widths(Group *g)
+{
+    const uint32_t p = g->p;
+    for (uint64_t kib : {uint64_t(90) << 10, uint64_t(100) << 10, uint64_t(124) << 10, uint64_t(140) << 10, uint64_t(500) << 10}) {
+        for (bool uniform : {true, false}) {
+            Tables c;
+            for (std::vector<uint64_t> &t : c.t) {
+                t.resize(p * p);
+            }
+            for (uint64_t &n : c.t[0]) {
+                n = kib * 256 / p / p;
+            }
+            c.t[0][1] += uniform ? 0 : 1;
+            c.t[0][p] -= uniform ? 0 : 1;
+            for (uint32_t i = 0; i < p; i++) {
+                for (uint32_t j = 0; j < p; j++) {
+                    c.t[2][i * p + j] = c.t[0][j * p + i];
+                    c.t[1][i * p + j] = j == 0 ? 0 : c.t[1][i * p + j - 1] + c.t[0][i * p + j - 1];
+                    c.t[3][i * p + j] = j == 0 ? 0 : c.t[3][i * p + j - 1] + c.t[2][i * p + j - 1];
+                }
+            }
+            A2avSet *ready = nullptr;
+            if (!Rows(g, c) || A2avFinish(g, reinterpret_cast<hipStream_t>(uintptr_t(1)), &ready) != HCCL_SUCCESS || ready == nullptr) {
+                std::printf("%llu KiB: not taken\n", (unsigned long long)kib);
+                return 1;
+            }
+            const uint32_t mib = uint32_t(kib >> 10), want = mib < 96 ? 0 : mib < 128 || (uniform && p <= 16) ? 2 : 1;
+            if (ready->width != want) {
+                std::printf("%u MiB, uniform %d: %u workgroups per CU\n", mib, int(uniform), ready->width);
+                return 1;
+            }
+        }
+    }
+    std::printf("OK\n");
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -313,8 +352,8 @@ int main(int argc, char **argv)
         slot.host = std::calloc(1, 128 << 10);
         (void)hipEventCreateWithFlags(&slot.done, 0);
     }
-    if (calls == 0) {
-        return General(g);
+    if (calls <= 0) {
+        return calls == 0 ? General(g) : Widths(g);
     }
     const size_t tableBytes = p <= 8 ? sizeof(A2avTable<8>) : p <= 16 ? sizeof(A2avTable<16>) : p <= 32 ? sizeof(A2avTable<32>) : sizeof(A2avTable<64>);
     std::vector<Tables> tables;

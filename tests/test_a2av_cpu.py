@@ -35,3 +35,9 @@ def test_tables_of_several_streams(check, ranks, calls, streams, sets):
 def test_calls_that_go_the_general_way(check, ranks):
     out = subprocess.run([check, str(ranks), "0"], stdout=subprocess.PIPE, text=True, timeout=120)
     assert out.returncode == 0 and out.stdout.startswith("OK"), out.stdout
+
+
+@pytest.mark.parametrize("ranks", [2, 16, 17, 64])
+def test_widths(check, ranks):
+    out = subprocess.run([check, str(ranks), "-1"], stdout=subprocess.PIPE, text=True, timeout=120)
+    assert out.returncode == 0 and out.stdout.startswith("OK"), out.stdout

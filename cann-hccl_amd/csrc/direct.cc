@@ -440,6 +440,14 @@ void PackDirect(const Plan &plan, bool reduceColl, int dtype, int op, DirectLaun
     kind = wide ? KernelKind(kind + KK_PACKED_WIDE) : kind;
     d->packedGridX = uint32_t(longest / chunk + (longest % chunk >= 16 ? 1 : 0)) + (ends ? 1u : 0u);
     d->packedFunc = reduceColl ? LookupKernel(dtype, op, kind) : LookupCopyKernel(kind);
+    // Both batches of many sources in flight, but for large all-reduces whose combining takes an instruction or two, where the waves a CU holds count for more (share of the time batch after
+    // batch: fp32, 32 ranks 1 MiB 0.94, 1.12 MiB 1.09, 1.5 MiB 1.17, 24 ranks 1.5 MiB 1.04; bf16 sum, 32 ranks 1.5 MiB 0.93, int8 0.89), and for maxima and minima of 32 halves, whose registers leave no
+    // room for it (all-reduce of bf16, 512 KiB 1.26, fp16 1.13).
+    const bool halves = dtype == HCCL_DATA_TYPE_FP16 || dtype == HCCL_DATA_TYPE_BFP16, selects = op == HCCL_REDUCE_MAX || op == HCCL_REDUCE_MIN;
+    const bool costly = dtype == HCCL_DATA_TYPE_INT8 || dtype == HCCL_DATA_TYPE_UINT8 || (dtype == HCCL_DATA_TYPE_BFP16 && !selects);
+    if (reduceColl && !tree && order.size() >= 24 && !(order.size() == 32 && halves && selects) && (toOne || costly || total <= 4 * SixteenthTiles(numCu))) {
+        d->packedTwoFunc = LookupKernel(dtype, op, KernelKind(KK_PACKED_TWO + (order.size() == 32 ? 1 : 0)));
+    }
 }
 
 bool FillBases(DirectLaunch *d, const std::vector<void *> &send, const std::vector<void *> &recv)

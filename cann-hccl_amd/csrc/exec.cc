@@ -1553,7 +1553,8 @@ HcclResult IssueCollective(Group *g, uint32_t launcher)
     }
     if (direct != nullptr) {
         void *args[1] = {direct->usePacked ? direct->packed.data() : direct->image.data()};
-        HIP_OK(hipLaunchKernel(direct->usePacked ? direct->packedFunc : direct->func,
+        const void *packedFunc = direct->packedTwoFunc != nullptr ? direct->packedTwoFunc : direct->packedFunc;
+        HIP_OK(hipLaunchKernel(direct->usePacked ? packedFunc : direct->func,
             dim3(direct->usePacked ? direct->packedGridX : direct->gridX, direct->gridY, 1), dim3(kDirectThreads, 1, 1), args, 0, ls));
     } else if (a2av != nullptr) {
         HcclResult launched = A2avLaunch(g, a2av, ls);

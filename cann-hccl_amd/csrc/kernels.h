@@ -112,11 +112,12 @@ enum KernelKind : int {
     KK_PACKED_RING = 18,                                       // chains whose sources behind the second one are the left operands,
     KK_PACKED_TREE = 22,                                       // trees;
     KK_PACKED_WIDE = 12,                                       // added to one of the last 12 kinds: four vectors per lane
-    KK_COUNT = 38,
-    KK_GATHER = 38,                                            // copy kernel table only, like these:
-    KK_A2AV = 39,                                              // all-to-all-v from the callers' tables in device memory, of 8, 16, 32, 64
-                                                               // ranks: workgroups of one wave (kinds 39 ... 42), of four (43 ... 46);
-    KK_A2AV_ARGS = 47                                          // in the kernel arguments, of 8, 16 ranks: one wave (47, 48), four (49, 50)
+    KK_PACKED_TWO = 38,                                        // chains of 24 ... 31 sources, both batches of them in flight; of 32 (39)
+    KK_COUNT = 40,
+    KK_GATHER = 40,                                            // copy kernel table only, like these:
+    KK_A2AV = 41,                                              // all-to-all-v from the callers' tables in device memory, of 8, 16, 32, 64
+                                                               // ranks: workgroups of one wave (kinds 41 ... 44), of four (45 ... 48);
+    KK_A2AV_ARGS = 49                                          // in the kernel arguments, of 8, 16 ranks: one wave (49, 50), four (51, 52)
 };
 constexpr uint32_t kPackedShapes = 4;
 // Index of a number of sources among those that have a kernel of their own, kPackedShapes where it has none.
@@ -214,7 +215,7 @@ constexpr uint32_t kPackedRing = 1u << 27;      // chain: sources behind the sec
 //                      Up to seven pointers behind an item's list of sources may be read (and are not used): the destinations'
 //                      pool lies behind the sources', and the tables end on a multiple of 256 bytes.
 //   KK_TEAM_*          the same and (uint32_t *teamBlock)
-//   KK_PACKED_n        (PackedArgs<n>; those of 2, 4 and 8 sources PackedArgs<8>, of 16 PackedArgs<16>), grid (chunks of the longest item's whole vectors, items), with kPackedEnds one more in x, the first one, for the bytes
+//   KK_PACKED_n        (PackedArgs<n>; those of 2, 4 and 8 sources PackedArgs<8>, of 16 PackedArgs<16>; KK_PACKED_TWO PackedArgs<32>), grid (chunks of the longest item's whole vectors, items), with kPackedEnds one more in x, the first one, for the bytes
 //                      behind an item's last whole vector
 //   KK_DIRECT / KK_DIRECT_WIDE   (DirectArgs<8> / DirectArgs<32>), grid (1 + chunks of the longest item, items): blockIdx.x == 0
 //                      is for the bytes behind an item's last whole vector

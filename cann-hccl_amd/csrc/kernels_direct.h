@@ -176,8 +176,25 @@ __device__ __forceinline__ void DirectTwoBatches(const View &view, uint32_t off,
     }
 }
 
-// first(j), later(j): whether the value so far is the left operand, for the sources loaded first and for those behind them.
-template <typename L, typename T, int OP, typename View, typename First, typename Later>
+// The sources from j on, fewer than 8.
+template <typename L, typename T, int OP, typename View, typename Later>
+__device__ __forceinline__ void DirectRest(const View &view, uint32_t j, uint32_t off, typename L::Val &acc, Later later)
+{
+    switch (view.Sources() - j) {
+        case 1: DirectBatch<L, T, OP, 1, false>(view, j, off, acc, later); break;
+        case 2: DirectBatch<L, T, OP, 2, false>(view, j, off, acc, later); break;
+        case 3: DirectBatch<L, T, OP, 3, false>(view, j, off, acc, later); break;
+        case 4: DirectBatch<L, T, OP, 4, false>(view, j, off, acc, later); break;
+        case 5: DirectBatch<L, T, OP, 5, false>(view, j, off, acc, later); break;
+        case 6: DirectBatch<L, T, OP, 6, false>(view, j, off, acc, later); break;
+        case 7: DirectBatch<L, T, OP, 7, false>(view, j, off, acc, later); break;
+        default: break;
+    }
+}
+
+// first(j), later(j): whether the value so far is the left operand, for the sources loaded first and for those behind them.  TWO: of 24 sources and more both batches in flight; else one after
+// the other.
+template <typename L, typename T, int OP, bool TWO, typename View, typename First, typename Later>
 __device__ __forceinline__ typename L::Val DirectChain(const View &view, uint32_t off, First first, Later later)
 {
     typename L::Val acc;
@@ -198,10 +215,10 @@ __device__ __forceinline__ typename L::Val DirectChain(const View &view, uint32_
     }
     if constexpr (View::kMany) {
         uint32_t j = 8;
-        if (nsrc >= 32) {
+        if (TWO && nsrc >= 32) {
             DirectTwoBatches<L, T, OP, 16, 16>(view, off, acc, first, later);
             j = 32;
-        } else if (nsrc >= 24) {
+        } else if (TWO && nsrc >= 24) {
             DirectTwoBatches<L, T, OP, 16, 8>(view, off, acc, first, later);
             j = 24;
         } else if (nsrc >= 16) {
@@ -210,20 +227,17 @@ __device__ __forceinline__ typename L::Val DirectChain(const View &view, uint32_
         } else {
             DirectBatch<L, T, OP, 8, true>(view, 0, off, acc, first);
         }
+        if constexpr (!TWO) {
+#pragma nounroll
+            for (; j + 16 <= nsrc; j += 16) {
+                DirectBatch<L, T, OP, 16, false>(view, j, off, acc, later);
+            }
+        }
         if (j + 8 <= nsrc) {
             DirectBatch<L, T, OP, 8, false>(view, j, off, acc, later);
             j += 8;
         }
-        switch (nsrc - j) {
-            case 1: DirectBatch<L, T, OP, 1, false>(view, j, off, acc, later); break;
-            case 2: DirectBatch<L, T, OP, 2, false>(view, j, off, acc, later); break;
-            case 3: DirectBatch<L, T, OP, 3, false>(view, j, off, acc, later); break;
-            case 4: DirectBatch<L, T, OP, 4, false>(view, j, off, acc, later); break;
-            case 5: DirectBatch<L, T, OP, 5, false>(view, j, off, acc, later); break;
-            case 6: DirectBatch<L, T, OP, 6, false>(view, j, off, acc, later); break;
-            case 7: DirectBatch<L, T, OP, 7, false>(view, j, off, acc, later); break;
-            default: break;
-        }
+        DirectRest<L, T, OP>(view, j, off, acc, later);
     }
     return acc;
 }
@@ -353,7 +367,7 @@ __device__ __forceinline__ typename L::Val DirectValue(const DirectView<CAP> &vi
 {
     if (view.it->kind == DIRECT_CHAIN) {
         auto left = [&](uint32_t j) { return ((view.it->accLeft >> j) & 1u) != 0; };
-        return DirectChain<L, T, OP>(view, off, left, left);
+        return DirectChain<L, T, OP, true>(view, off, left, left);
     }
     if (CAP > 8 || view.it->kind == DIRECT_TREE) {
         return DirectTree<L, CAP>(view, off);
@@ -402,9 +416,9 @@ __device__ __forceinline__ typename L::Val DirectValue(const PackedView<P> &view
     }
     auto yes = [](uint32_t) { return true; };
     if (OrderMatters<T, OP>::value && (view.k->info & kPackedRing) != 0) {
-        return DirectChain<L, T, OP>(view, off, [](uint32_t j) { return j < 2; }, [](uint32_t) { return false; });
+        return DirectChain<L, T, OP, false>(view, off, [](uint32_t j) { return j < 2; }, [](uint32_t) { return false; });
     }
-    return DirectChain<L, T, OP>(view, off, yes, yes);
+    return DirectChain<L, T, OP, false>(view, off, yes, yes);
 }
 
 // A lane's vector to every destination: N at a time without a branch between them, those behind the last one dropped by the
@@ -484,6 +498,45 @@ __global__ void __launch_bounds__(kDirectThreads) PackedKernel(const PackedArgs<
         DirectVector<T, OP>(view, KiBOf(blockIdx.x - ends, view.Bytes(), P > 8 && (view.k->info & kPackedFours) != 0) * kDirectChunk + threadIdx.x * 16u);
     } else {
         DirectEnd(view, [&](uint32_t off) { return DirectValue<ElemLane<T, OP>, T, OP>(view, off); });
+    }
+}
+
+// Chains of 24 ... 32 sources with both batches in flight, in a kernel of their own: in one with the others its registers and its code, which the way of fewer sources leads
+// around, cost those more than it gains here.  as a share of the time batch after batch, apart / in one kernel: 17
+// ranks' bf16 sum 768 KiB reduce-scatter 1.01 / 1.09, reduce 1.03 / 1.10, all-reduce 1.01 / 1.07, 20 ranks' all-reduce of 512 KiB 0.99 / 1.13; what it brings 24 to 32: reduce-scatter
+// of 512 KiB to 1 MiB bf16 0.78 ... 0.88, int8 0.83 ... 0.97, fp32 0.89 ... 0.97, reduce 0.76 ... 0.85, 0.82 ... 0.97, 0.87 ... 1.00.
+template <typename L, typename T, int OP, bool ALL, typename First, typename Later>
+__device__ __forceinline__ typename L::Val PackedTwoChain(const PackedView<32> &view, uint32_t off, First first, Later later)
+{
+    typename L::Val acc;
+    if constexpr (ALL) {
+        DirectTwoBatches<L, T, OP, 16, 16>(view, off, acc, first, later);
+    } else {
+        DirectTwoBatches<L, T, OP, 16, 8>(view, off, acc, first, later);
+        DirectRest<L, T, OP>(view, 24, off, acc, later);
+    }
+    return acc;
+}
+template <typename L, typename T, int OP, bool ALL> __device__ __forceinline__ typename L::Val PackedTwoValue(const PackedView<32> &view, uint32_t off)
+{
+    if (OrderMatters<T, OP>::value && (view.k->info & kPackedRing) != 0) {
+        return PackedTwoChain<L, T, OP, ALL>(view, off, [](uint32_t j) { return j < 2; }, [](uint32_t) { return false; });
+    }
+    auto yes = [](uint32_t) { return true; };
+    return PackedTwoChain<L, T, OP, ALL>(view, off, yes, yes);
+}
+// ALL: 32 sources, else 24 ... 31.
+template <typename T, int OP, bool ALL> __global__ void __launch_bounds__(kDirectThreads) PackedTwoKernel(const PackedArgs<32>)
+{
+    const PackedView<32> view;
+    const uint32_t ends = view.k->info & kPackedEnds ? 1u : 0u;
+    if (blockIdx.x >= ends) {
+        const uint32_t at = KiBOf(blockIdx.x - ends, view.Bytes(), (view.k->info & kPackedFours) != 0) * kDirectChunk + threadIdx.x * 16u;
+        if (at + 16u <= view.Bytes()) {
+            DirectStore(view, at, PackedTwoValue<VecLane<T, OP>, T, OP, ALL>(view, view.SrcOff() + at));
+        }
+    } else {
+        DirectEnd(view, [&](uint32_t off) { return PackedTwoValue<ElemLane<T, OP>, T, OP, ALL>(view, off); });
     }
 }
 

@@ -103,6 +103,8 @@ extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[21] = {
         reinterpret_cast<const void *>(&PackedKernel<DT, OP, 16>),       \
         reinterpret_cast<const void *>(&PackedKernel<DT, OP, 32>),       \
         HCCL_ORDERS(PackedShapeKernel, OP), HCCL_ORDERS(PackedWideKernel, OP),                                                    \
+        reinterpret_cast<const void *>(&PackedTwoKernel<DT, OP, false>), \
+        reinterpret_cast<const void *>(&PackedTwoKernel<DT, OP, true>),  \
     }
 extern const void *const HCCL_CAT(kKernels_, HCCL_DT_NAME)[4][KK_COUNT] = {
     HCCL_ROW(ROP_SUM), HCCL_ROW(ROP_PROD), HCCL_ROW(ROP_MAX), HCCL_ROW(ROP_MIN),

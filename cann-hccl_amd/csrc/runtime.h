@@ -141,6 +141,7 @@ struct DirectLaunch {
     std::vector<uint8_t> image;                        // the kernel's arguments, a DirectArgs
     std::vector<uint64_t> sendBytes, recvBytes;        // per rank, as the plan's
     const void *packedFunc = nullptr;                  // the same collective with a PackedArgs, nullptr: its items are not alike
+    const void *packedTwoFunc = nullptr;               // a kernel that does it sooner, nullptr: none
     uint32_t packedRanks = 0, packedGridX = 0;         // ranks that its arguments have room for
     std::vector<uint8_t> packed;
     bool packedWide = false;                           // four vectors per lane

@@ -289,6 +289,17 @@ int main(int argc, char **argv)
         }
         n++;
         PackDirect(plan, true, 4, 0, &d);
+        // (sums of fp32: both batches of many sources in flight, up to 1 MiB where there is more than one destination)
+        uint64_t total = 0;
+        for (const FusedItem &f : plan.fused) {
+            total += f.bytes;
+        }
+        const FusedItem &item = plan.fused[0];
+        const bool two = d.packedFunc != nullptr && item.kind == FK_CHAIN && item.src.size() >= 24 && (item.dst.size() == 1 || total <= 1u << 20);
+        if (d.packedTwoFunc != (two ? LookupKernel(0, 0, KernelKind(item.src.size() == 32 ? KK_PACKED_TWO + 1 : KK_PACKED_TWO)) : nullptr)) {
+            std::printf("coll %d p %u total %llu: the kernel for %zu sources\n", int(rq.coll), rq.p, (unsigned long long)total, item.src.size());
+            return 1;
+        }
         const bool usual = rq.p <= 32 && rq.servers == 1 &&
             ((rq.coll == COLL_ALLGATHER) || ((rq.coll == COLL_ALLREDUCE || rq.coll == COLL_REDUCESCATTER) &&
                 (rq.algo == ALGO_RING || rq.algo == ALGO_MESH_ATOMIC || (rq.algo == ALGO_RHD && (rq.p & (rq.p - 1)) == 0))));

@@ -297,7 +297,7 @@ int main(int argc, char **argv)
         const FusedItem &item = plan.fused[0];
         const bool two = d.packedFunc != nullptr && item.kind == FK_CHAIN && item.src.size() >= 24 && (item.dst.size() == 1 || total <= 1u << 20);
         if (d.packedTwoFunc != (two ? LookupKernel(0, 0, KernelKind(item.src.size() == 32 ? KK_PACKED_TWO + 1 : KK_PACKED_TWO)) : nullptr)) {
-            std::printf("coll %d p %u total %llu: the kernel for %zu sources\n", int(rq.coll), rq.p, (unsigned long long)total, item.src.size());
+            std::printf("coll %d p %u total %llu: the kernel for %u sources\n", int(rq.coll), rq.p, (unsigned long long)total, item.src.size());
             return 1;
         }
         const bool usual = rq.p <= 32 && rq.servers == 1 &&

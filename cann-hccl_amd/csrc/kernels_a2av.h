@@ -1,6 +1,6 @@
 // All-to-all-v straight from the tables of its callers: a block's source, destination and length follow from three numbers of
-// theirs, so nothing is planned, cut or laid out for the device; 12 bytes per pair of ranks travel to it, up to 16 ranks in the kernel
-// arguments.
+// theirs, so nothing is planned, cut or laid out for the device; 12 bytes per pair of ranks travel to it, a new call's of up to 16 ranks in the
+// kernel arguments.
 //
 // A wave takes a piece of 4 KiB of a block at a time.  It finds it by itself: the lanes
 // hold the first piece of every receiver's blocks (at most 64 receivers, one per lane), then that receiver's row of the tables, whose

@@ -1242,15 +1242,20 @@ DirectLaunch *FindDirect(Group *g, int algo)
         return nullptr;
     }
     const uint64_t bytes = sig.count * DtypeSize(sig.dtype);
-    uint64_t inPlace = 0, sends = 0, recvs = 0;
+    uint64_t inPlace = 0;
     for (uint32_t r = 0; r < g->p; r++) {
         inPlace |= uint64_t(g->ctx->send[r] == g->ctx->recv[r] ? 1 : 0) << r;
-        sends |= reinterpret_cast<uint64_t>(g->ctx->send[r]);
-        recvs |= reinterpret_cast<uint64_t>(g->ctx->recv[r]);
     }
     const bool small = DirectFits(sig.coll, g->p, bytes, sig.dtype) && !CombiningBound(sig.coll, g->p, bytes, sig.dtype, sig.op);
-    if (!small && !PackedFits(sig.coll, g->p, bytes, sig.dtype, g->numCu, sends, recvs, inPlace != 0)) {
-        return nullptr;
+    if (!small) {
+        uint64_t sends = 0, recvs = 0;
+        for (uint32_t r = 0; r < g->p; r++) {
+            sends |= reinterpret_cast<uint64_t>(g->ctx->send[r]);
+            recvs |= reinterpret_cast<uint64_t>(g->ctx->recv[r]);
+        }
+        if (!PackedFits(sig.coll, g->p, bytes, sig.dtype, g->numCu, sends, recvs, inPlace != 0)) {
+            return nullptr;
+        }
     }
     const DirectKey key = {{uint64_t(sig.coll) | (uint64_t(algo) << 8) | (uint64_t(sig.dtype) << 16) | (uint64_t(sig.op) << 24) | (uint64_t(sig.root) << 32) |
             (uint64_t(sig.peer) << 48), sig.count, inPlace, cfg.cclBytes, cfg.align,
